@@ -1,93 +1,285 @@
-// Plain tiled matrix product  Y[t,n] = sum_k X[t,k] W[n,k] (+bias) (+resid).
+// The float32 matrix product  Y[t,n] = sum_k X[t,k] W[n,k] (+bias) (+resid): the true 32-bit path
+// of every projection, and the fallback of the bf16 path for sizes its kernels refuse.
 //
-// The true 32-bit path of every projection, and the fallback of the bf16 path
-// for sizes the MFMA kernels refuse.  Every output element is accumulated by
-// one thread with fmaf in ascending k starting from zero, so its value does
-// not depend on how many rows share the launch or where its tile lies: the
-// same (row, column) gives the same bits in a whole prompt, in a single-token
-// step and in any batch.  W is [out, in] row-major, the memory of a
+// It runs on the float32 matrix cores.  v_mfma_f32_16x16x4_f32 adds its four products to the
+// accumulator one after the other in ascending k, each with one rounding: the bits of a chain of
+// fmaf (checked against fmaf over 1,000 k, denormals among them).  An element is the sum of its
+// segments of kSegment k, each such a chain from zero, added in ascending order: a function of k
+// alone, so its value does not depend on how many rows share the launch, on the tile or on the
+// waves that made it.  The same (row, column) gives the same bits in a whole prompt, in a
+// single-token step and in any batch.  W is [out, in] row-major, the memory of a
 // projection weight (/root/reference/core/include/sonicboom/quant/quantized_matmul.h:74-77);
 // the bias is added after the product and the residual after the bias
 // (/root/reference/core/src/model/emit.cpp:260-261, :447).
-#include "common.h"
+//
+// A block owns 16 CT columns of 16 TT rows.  Its WAVES waves take the segments of K between them
+// (segment s goes to wave s % WAVES), straight from memory and without a barrier on the way; the
+// segments' sums meet in LDS.  A lane loads four consecutive k of one row, the four lane groups of
+// a row 64 bytes side by side; four lane swaps turn the 4 x 4 of lane groups and registers over,
+// after which register s holds k = 4 s + lane group, what step s of the matrix instruction takes.
+// W that a projection keeps is packed (FORM kPacked): blocks of 16 rows x 16 k in the order that
+// the lanes take, 1 KB each, consecutive in k, so that a wave reads one stream and swaps nothing.
+// The loads run kAhead steps of 16 k ahead in a ring of registers.  Gated (G = 2): a column tile
+// is a tile of W's first half and the same tile of the second, and Y = act(first) * second.
+//
+// What bounds it: with few rows the read of W (each wave must have enough of it in flight) and the
+// chain's latency, with many the matrix cores.  Measured on MI355X at the 0.5B layer sizes, 3 rows, against the
+// kernel with one fmaf chain a thread that stood here before: 896 x 896 107 us then, 9.2 now; 896 x 4,864
+// 597 and 16.7; the gated 9,728 x 896 110 + 4.8 (its activation) and 16.2.  520 rows: the gated product 179 + 7 and
+// 150 (61 TFLOP/s), 896 x 4,864 666 and 78.  From row-major W with swaps the 3-row products took 13.6, 19.4 and 15 us.
+#include "mfma.h"
 
 namespace {
 
-constexpr int kTile = 64;   // rows and columns of a block's tile
-constexpr int kStep = 16;   // k per stage
-constexpr int kThreads = 256;
+constexpr int kSegment = 1024;          // k of one chain; part of what the result's bits are
+constexpr int kSteps = kSegment / 16;   // loads of a row in a segment
 
-template <typename TX, typename TW, typename TO>
-__global__ void __launch_bounds__(kThreads)
-gemm_plain_kernel(TO *y, const TX *__restrict__ x, const TW *__restrict__ w,
-                  const void *__restrict__ bias, int bias_dtype, const float *resid, int n_rows,
-                  int n_out, int n_in) {
-  __shared__ float xs[kStep][kTile + 4];
-  __shared__ float ws[kStep][kTile + 4];
-  const int t0 = blockIdx.y * kTile;
-  const int n0 = blockIdx.x * kTile;
-  const int tid = threadIdx.x;
-  const int ty = tid / 16, tx = tid % 16;
+enum Form { kAny, kPacked, kPackedAny };   // W row-major; W packed, X by 16-byte loads; W packed, X element by element
 
-  float acc[4][4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
+__device__ __forceinline__ void swap_halves(float &a, float &b) {
+  const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  const uint32_t p0 = p[0], p1 = p[1];
+  a = __uint_as_float(p0);
+  b = __uint_as_float(p1);
+}
+__device__ __forceinline__ void swap_rows(float &a, float &b) {
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  const uint32_t p0 = p[0], p1 = p[1];
+  a = __uint_as_float(p0);
+  b = __uint_as_float(p1);
+}
 
-  for (int k0 = 0; k0 < n_in; k0 += kStep) {
+// In: register s of lane group g holds k = 4 g + s.  Out: k = 4 s + g.
+__device__ __forceinline__ void by_step(const floatx4_t &raw, float (&f)[4]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int e = tid + i * kThreads;
-      const int r = e / kStep, k = e % kStep;
-      const int gk = k0 + k;
-      const int gt = t0 + r, gn = n0 + r;
-      xs[k][r] = (gt < n_rows && gk < n_in) ? ld_f(x, size_t(gt) * n_in + gk) : 0.0f;
-      ws[k][r] = (gn < n_out && gk < n_in) ? ld_f(w, size_t(gn) * n_in + gk) : 0.0f;
-    }
-    __syncthreads();
+  for (int e = 0; e < 4; ++e) f[e] = raw[e];
+  swap_rows(f[0], f[1]);
+  swap_rows(f[2], f[3]);
+  swap_halves(f[0], f[2]);
+  swap_halves(f[1], f[3]);
+}
+
+constexpr uint32_t kPastEnd = 0x80000000u;      // an offset past every descriptor's end: reads as zeros
+
+// Four consecutive k of a row of T that starts at `row`; zeros where k lies at or past `end`.
+template <typename T>
+__device__ __forceinline__ floatx4_t load4_any(const T *row, int k, int end) {
+  floatx4_t v;
 #pragma unroll
-    for (int k = 0; k < kStep; ++k) {
-      float a[4], b[4];
+  for (int e = 0; e < 4; ++e) v[e] = k + e < end ? ld_f(row, size_t(k) + e) : 0.0f;
+  return v;
+}
+
+struct PlainArgs {
+  void *y;
+  int y_dtype;
+  const void *bias;
+  int bias_dtype;
+  const float *resid;
+  int n_rows, n_out, n_in;
+  int gate;        // the activation (an sb_gate) of the gated form
+};
+
+template <typename TX, typename TW, int FORM, int TT, int CT, int G, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
+gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a) {
+  constexpr int kStreams = CT * G, kTiles = TT * CT;
+  // steps in flight: as many as 192 registers hold (128 or less beside the accumulators of larger tiles
+  // and the addresses of loads element by element)
+  constexpr int kRegs = 4 * (kStreams + TT);
+  constexpr int kAhead = FORM != kPacked ? 4 : kRegs == 8 ? 24 : kRegs <= 12 ? 16 : kRegs <= 16 ? 8 : 4;
+  constexpr int kUnits = (kTiles * 64 + 64 * WAVES - 1) / (64 * WAVES);   // groups of four outputs a thread
+  extern __shared__ floatx4_t part[];            // [WAVES][TT * kStreams][64]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, g = lane >> 4;
+  const unsigned tiles_n = (a.n_out + 16 * CT - 1) / (16 * CT);
+  const int n0 = int(blockIdx.x % tiles_n) * (16 * CT), t0 = int(blockIdx.x / tiles_n) * (16 * TT);
+  const int w_tiles = (a.n_out + 15) / 16, w_steps = (a.n_in + 15) / 16;      // packed: of one half
+
+  // Rows past the last one read the last one again (their outputs are not stored).
+  const TX *x0 = x + size_t(t0) * a.n_in;
+  const int x_rows = min(16 * TT, a.n_rows - t0);
+  const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<TX *>(x0), 0, uint32_t(size_t(x_rows) * a.n_in * sizeof(TX)), 0x00020000);
+  size_t x_at[TT];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) a[i] = xs[k][ty * 4 + i];
+  for (int j = 0; j < TT; ++j) x_at[j] = size_t(min(16 * j + r, x_rows - 1)) * a.n_in;
+  const TW *w_row[kStreams];
+  int w_tile[kStreams];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) b[j] = ws[k][tx * 4 + j];
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-    }
-    __syncthreads();
+  for (int i = 0; i < kStreams; ++i) {           // stream i: column tile i / G, half i % G
+    w_tile[i] = (i % G) * w_tiles + min(n0 / 16 + i / G, w_tiles - 1);
+    if (FORM == kAny) w_row[i] = w + (size_t(i % G) * a.n_out + min(n0 + 16 * (i / G) + r, a.n_out - 1)) * a.n_in;
   }
 
+  floatx4_t total[kUnits][G];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int gt = t0 + ty * 4 + i;
-    if (gt >= n_rows) continue;
+  for (int u = 0; u < kUnits; ++u)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int gn = n0 + tx * 4 + j;
-      if (gn >= n_out) continue;
-      float v = acc[i][j];
-      if (bias) v = v + ld_dyn(bias, bias_dtype, gn);
-      if (resid) v = v + resid[size_t(gt) * n_out + gn];
-      st_f(y, size_t(gt) * n_out + gn, v);
+    for (int q = 0; q < G; ++q) total[u][q] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  const int n_seg = (a.n_in + kSegment - 1) / kSegment;
+  for (int s0 = 0; s0 < n_seg; s0 += WAVES) {
+    const int seg = s0 + wave;
+    if (seg < n_seg) {                           // uniform over the wave
+      const int k_end = min((seg + 1) * kSegment, a.n_in);
+      const int steps = (k_end - seg * kSegment + 15) / 16;
+      // packed: a descriptor a stream, of its tile's blocks up to the segment's end
+      __amdgpu_buffer_rsrc_t rsrc_w[kStreams];
+      if constexpr (FORM != kAny) {
+#pragma unroll
+        for (int i = 0; i < kStreams; ++i)
+          rsrc_w[i] = __builtin_amdgcn_make_buffer_rsrc(
+              const_cast<TW *>(w) + (size_t(w_tile[i]) * w_steps + size_t(seg) * kSteps) * 256, 0, uint32_t(steps) * 1024u, 0x00020000);
+      }
+      floatx4_t acc[kStreams][TT];
+#pragma unroll
+      for (int i = 0; i < kStreams; ++i)
+#pragma unroll
+        for (int j = 0; j < TT; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+      floatx4_t rw[kAhead][kStreams], rx[kAhead][TT];
+      const int k_lane = seg * kSegment + 4 * g;
+      auto ask = [&](int slot, int step) {
+        const int k = k_lane + 16 * step;
+#pragma unroll
+        for (int i = 0; i < kStreams; ++i) {
+          if constexpr (FORM == kAny) rw[slot][i] = load4_any(w_row[i], k, k_end);
+          else rw[slot][i] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[i], lane * 16 + step * 1024, 0, 0));
+        }
+#pragma unroll
+        for (int j = 0; j < TT; ++j) {
+          if constexpr (FORM == kPacked)
+            rx[slot][j] = __builtin_bit_cast(floatx4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                rsrc_x, int(k < k_end ? uint32_t((x_at[j] + k) * 4) : kPastEnd), 0, 0));
+          else rx[slot][j] = load4_any(x0 + x_at[j], k, k_end);
+        }
+      };
+      auto multiply = [&](int slot, auto then) {
+        float fw[kStreams][4], fx[TT][4];
+#pragma unroll
+        for (int i = 0; i < kStreams; ++i) {
+          if constexpr (FORM == kAny) {
+            by_step(rw[slot][i], fw[i]);
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) fw[i][e] = rw[slot][i][e];
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < TT; ++j) by_step(rx[slot][j], fx[j]);
+        then();
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+          for (int i = 0; i < kStreams; ++i)
+#pragma unroll
+            for (int j = 0; j < TT; ++j)
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[i][s], fx[j][s], acc[i][j], 0, 0, 0);
+      };
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) ask(u, u);
+      int step = 0;
+      for (; step + kAhead <= steps; step += kAhead) {       // whole rounds of the ring
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) multiply(u, [&]() { ask(u, step + kAhead + u); });
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u)
+        if (step + u < steps) multiply(u, []() {});
+#pragma unroll
+      for (int i = 0; i < kStreams; ++i)
+#pragma unroll
+        for (int j = 0; j < TT; ++j) {
+          if constexpr (WAVES == 1) total[(i / G) * TT + j][i % G] = total[(i / G) * TT + j][i % G] + acc[i][j];
+          else part[((wave * G + i % G) * kTiles + (i / G) * TT + j) * 64 + lane] = acc[i][j];
+        }
+    }
+    if constexpr (WAVES > 1) {
+      __syncthreads();
+      const int here = min(WAVES, n_seg - s0);
+#pragma unroll
+      for (int u = 0; u < kUnits; ++u) {
+        const int unit = tid + u * 64 * WAVES;
+        if (unit < kTiles * 64)
+          for (int v = 0; v < here; ++v)
+#pragma unroll
+            for (int q = 0; q < G; ++q) total[u][q] = total[u][q] + part[(v * G + q) * kTiles * 64 + unit];
+      }
+      __syncthreads();
+    }
+  }
+
+  // unit (tile (i, j), lane (g, r)): columns 16 i + 4 g + 0..3 of row 16 j + r
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u) {
+    const int unit = tid + u * 64 * WAVES;
+    if (unit >= kTiles * 64) continue;
+    const int tile = unit >> 6, l = unit & 63;
+    const int t = t0 + 16 * (tile % TT) + (l & 15), nb = n0 + 16 * (tile / TT) + 4 * (l >> 4);
+    if (t >= a.n_rows) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int n = nb + e;
+      if (n >= a.n_out) continue;
+      float v = total[u][0][e];
+      if constexpr (G == 2) v = gate_act(v, a.gate) * total[u][G - 1][e];
+      if (a.bias) v = v + ld_dyn(a.bias, a.bias_dtype, n);
+      const size_t idx = size_t(t) * a.n_out + n;
+      if (a.resid) v = v + a.resid[idx];
+      if (a.y_dtype == SB_F32) ((float *)a.y)[idx] = v;
+      else ((bf16_t *)a.y)[idx] = f32_to_bf16(v);
     }
   }
 }
 
-template <typename TX, typename TW>
-int launch_y(void *y, int y_dtype, const TX *x, const TW *w, const void *bias, int bias_dtype,
-             const float *resid, int n_rows, int n_out, int n_in, hipStream_t s) {
-  dim3 grid((n_out + kTile - 1) / kTile, (n_rows + kTile - 1) / kTile);
-  if (y_dtype == SB_F32)
-    gemm_plain_kernel<TX, TW, float><<<grid, kThreads, 0, s>>>((float *)y, x, w, bias, bias_dtype,
-                                                              resid, n_rows, n_out, n_in);
-  else
-    gemm_plain_kernel<TX, TW, bf16_t><<<grid, kThreads, 0, s>>>((bf16_t *)y, x, w, bias, bias_dtype,
-                                                               resid, n_rows, n_out, n_in);
+template <typename TX, typename TW, int FORM, int TT, int CT, int G, int WAVES>
+int launch_one(const TX *x, const TW *w, const PlainArgs &a, hipStream_t s) {
+  constexpr int lds_bytes = WAVES == 1 ? 0 : WAVES * TT * CT * G * 1024;
+  auto kern = gemm_f32_kernel<TX, TW, FORM, TT, CT, G, WAVES>;
+  static bool raised = false;     // per instantiation; harmless if repeated
+  if (lds_bytes > 48 * 1024 && !raised) {
+    const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    SB_REQUIRE(e == hipSuccess, "sb_gemm: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    raised = true;
+  }
+  const long long blocks = (long long)((a.n_out + 16 * CT - 1) / (16 * CT)) * ((a.n_rows + 16 * TT - 1) / (16 * TT));
+  SB_SUPPORT(blocks <= 0x7fffffffLL, "sb_gemm: too many tiles");
+  kern<<<unsigned(blocks), 64 * WAVES, lds_bytes, s>>>(x, w, a);
   return sb::check_launch("sb_gemm");
+}
+
+template <int TT, int CT, int G>
+int launch_packed(const float *x, const float *w, const PlainArgs &a, int n_seg, hipStream_t s) {
+  if (n_seg == 1) return launch_one<float, float, kPacked, TT, CT, G, 1>(x, w, a, s);
+  if (n_seg == 2) return launch_one<float, float, kPacked, TT, CT, G, 2>(x, w, a, s);
+  if (n_seg <= 4) return launch_one<float, float, kPacked, TT, CT, G, 4>(x, w, a, s);
+  return launch_one<float, float, kPacked, TT, CT, G, 8>(x, w, a, s);
+}
+
+// The largest tile whose waves still give most of the 1,024 SIMDs one: larger tiles read X and W fewer
+// times (a wave of a 16 x 16 tile asks for 64 bytes a cycle and CU, what the cache gives; 64 x 64 for 16),
+// smaller ones leave no SIMD idle.
+template <int G>
+int launch_packed_tiles(const float *x, const float *w, const PlainArgs &a, int n_seg, hipStream_t s) {
+  const auto waves = [&](int tt, int ct) {
+    return (long long)((a.n_rows + 16 * tt - 1) / (16 * tt)) * ((a.n_out + 16 * ct - 1) / (16 * ct)) * (n_seg < 8 ? n_seg : 8);
+  };
+  constexpr long long kEnough = 768;
+  if (a.n_rows <= 16) {
+    if (G == 1 && waves(1, 2) >= 4 * kEnough) return launch_packed<1, 2, G>(x, w, a, n_seg, s);
+    return launch_packed<1, 1, G>(x, w, a, n_seg, s);
+  }
+  if (a.n_rows > 32 && waves(4, 4 / G) >= kEnough) return launch_packed<4, 4 / G, G>(x, w, a, n_seg, s);
+  if (a.n_rows > 32 && waves(4, 2 / G) >= kEnough) return launch_packed<4, 2 / G, G>(x, w, a, n_seg, s);
+  if (G == 1 && waves(2, 2) >= kEnough) return launch_packed<2, 2, G>(x, w, a, n_seg, s);
+  return launch_packed<2, 1, G>(x, w, a, n_seg, s);
+}
+
+// Every type, any inner size and alignment: loads element by element.
+template <typename TX, typename TW>
+int launch_any(const TX *x, const TW *w, const PlainArgs &a, int n_seg, hipStream_t s) {
+  if (n_seg == 1) return launch_one<TX, TW, kAny, 2, 1, 1, 1>(x, w, a, s);
+  return launch_one<TX, TW, kAny, 2, 1, 1, 8>(x, w, a, s);
 }
 
 }  // namespace
@@ -103,19 +295,42 @@ extern "C" int sb_gemm(void *y, int y_dtype, const void *x, int x_dtype, const v
              "sb_gemm: unknown dtype");
   SB_REQUIRE(!(resid && y_dtype != SB_F32 && (const void *)resid == y),
              "sb_gemm: a residual that aliases the output must be f32");
-  SB_SUPPORT((n_rows + kTile - 1) / kTile <= 65535, "sb_gemm: more than %d rows in one call",
-             65535 * kTile);
+  SB_SUPPORT((n_rows + 63) / 64 <= 65535, "sb_gemm: more than %d rows in one call", 65535 * 64);
   if (n_rows == 0) return SB_OK;
   hipStream_t s = (hipStream_t)stream;
-  if (x_dtype == SB_F32 && w_dtype == SB_F32)
-    return launch_y(y, y_dtype, (const float *)x, (const float *)w, bias, bias_dtype, resid, n_rows,
-                    n_out, n_in, s);
-  if (x_dtype == SB_BF16 && w_dtype == SB_BF16)
-    return launch_y(y, y_dtype, (const bf16_t *)x, (const bf16_t *)w, bias, bias_dtype, resid, n_rows,
-                    n_out, n_in, s);
-  if (x_dtype == SB_F32 && w_dtype == SB_BF16)
-    return launch_y(y, y_dtype, (const float *)x, (const bf16_t *)w, bias, bias_dtype, resid, n_rows,
-                    n_out, n_in, s);
-  return launch_y(y, y_dtype, (const bf16_t *)x, (const float *)w, bias, bias_dtype, resid, n_rows,
-                  n_out, n_in, s);
+  const PlainArgs a{y, y_dtype, bias, bias_dtype, resid, n_rows, n_out, n_in, SB_GATE_NONE};
+  const int n_seg = (n_in + kSegment - 1) / kSegment;
+  if (x_dtype == SB_F32 && w_dtype == SB_F32) return launch_any((const float *)x, (const float *)w, a, n_seg, s);
+  if (x_dtype == SB_F32) return launch_any((const float *)x, (const bf16_t *)w, a, n_seg, s);
+  if (w_dtype == SB_F32) return launch_any((const bf16_t *)x, (const float *)w, a, n_seg, s);
+  return launch_any((const bf16_t *)x, (const bf16_t *)w, a, n_seg, s);
+}
+
+// The same for float32 X and packed float32 W (blocks of 16 rows x 16 k, consecutive in k, zero padded: the
+// element of row r, k = 4 s + g of a block lies at (16 g + r) * 4 + s; gated: the two halves one after the
+// other, each padded), with gated != 0: Y = act(X Wg^T) * (X Wu^T).  The bits of sb_gemm.
+extern "C" int sb_gemm_f32_packed(void *y, int y_dtype, const float *x, const float *w, const void *bias, int bias_dtype,
+                                  const float *resid, int n_rows, int n_out, int n_in, int gated, void *stream) {
+  SB_REQUIRE(y && x && w, "sb_gemm_f32_packed: null pointer");
+  SB_REQUIRE(n_rows >= 0 && n_out > 0 && n_in > 0, "sb_gemm_f32_packed: bad sizes rows=%d out=%d in=%d", n_rows, n_out, n_in);
+  SB_REQUIRE(sb::valid_dtype(y_dtype) && (!bias || sb::valid_dtype(bias_dtype)), "sb_gemm_f32_packed: unknown dtype");
+  SB_REQUIRE(!(resid && y_dtype != SB_F32 && (const void *)resid == y),
+             "sb_gemm_f32_packed: a residual that aliases the output must be f32");
+  SB_REQUIRE(!(gated && (bias || resid)), "sb_gemm_f32_packed: the gated form takes no bias or residual");
+  SB_SUPPORT(gated >= SB_GATE_NONE && gated <= SB_GATE_RELU, "sb_gemm_f32_packed: unknown gate activation %d", gated);
+  SB_SUPPORT((n_rows + 63) / 64 <= 65535, "sb_gemm_f32_packed: more than %d rows in one call", 65535 * 64);
+  SB_SUPPORT(reinterpret_cast<uintptr_t>(w) % 16 == 0, "sb_gemm_f32_packed: the packed weights must be 16-byte aligned");
+  if (n_rows == 0) return SB_OK;
+  hipStream_t s = (hipStream_t)stream;
+  const PlainArgs a{y, y_dtype, bias, bias_dtype, resid, n_rows, n_out, n_in, gated};
+  const int n_seg = (n_in + kSegment - 1) / kSegment;
+  // 16-byte loads need rows of X that start on 16 bytes; offsets inside a block's rows fit 31 bits
+  const bool vec = n_in % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && size_t(n_in) * 64 * 4 < (size_t(1) << 31);
+  if (!vec) {
+    if (gated) return n_seg == 1 ? launch_one<float, float, kPackedAny, 2, 1, 2, 1>(x, w, a, s)
+                                 : launch_one<float, float, kPackedAny, 2, 1, 2, 8>(x, w, a, s);
+    return n_seg == 1 ? launch_one<float, float, kPackedAny, 2, 1, 1, 1>(x, w, a, s)
+                      : launch_one<float, float, kPackedAny, 2, 1, 1, 8>(x, w, a, s);
+  }
+  return gated ? launch_packed_tiles<2>(x, w, a, n_seg, s) : launch_packed_tiles<1>(x, w, a, n_seg, s);
 }

@@ -109,12 +109,17 @@ int sb_reduce_resid_norm(void *y, int y_dtype, float *x, const float *partial, i
                          const void *bias, int bias_dtype, const void *w, int w_dtype, int n_rows,
                          int width, float eps, int do_norm, void *stream);
 
-/* Y[t,n] = sum_k X[t,k] W[n,k] (+ bias[n]) (+ resid[t,n]).   Plain tiled kernel,
- * float accumulation in ascending k for every element whatever the batch.
+/* Y[t,n] = sum_k X[t,k] W[n,k] (+ bias[n]) (+ resid[t,n]) in float32: chains of fused
+ * multiply-adds over 1024 k each, added in ascending order, for every element whatever the batch.
  * resid is f32 [t,n] and may be the same buffer as Y (when Y is f32). */
 int sb_gemm(void *y, int y_dtype, const void *x, int x_dtype, const void *w, int w_dtype,
             const void *bias, int bias_dtype, const float *resid,
             int n_rows, int n_out, int n_in, void *stream);
+/* The same bits from packed float32 weights (blocks of 16 rows x 16 k, 1 KB each, consecutive in k, rows and k
+ * zero padded: row r, k = 4 s + g of a block at (16 g + r) * 4 + s); gated (an sb_gate): W holds two
+ * halves of n_out rows, each packed by itself, and Y = act(X Wg^T) * (X Wu^T). */
+int sb_gemm_f32_packed(void *y, int y_dtype, const float *x, const float *w, const void *bias, int bias_dtype,
+                       const float *resid, int n_rows, int n_out, int n_in, int gated, void *stream);
 
 /* out[t,i] = act(gu[t,i]) * gu[t,width+i];  gu is [t, 2*width]; gate: SB_GATE_SILU or
  * SB_GATE_GELU_TANH. */

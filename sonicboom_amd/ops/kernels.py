@@ -129,7 +129,7 @@ def rmsnorm(x: torch.Tensor, weight: Optional[torch.Tensor], eps: float, out_dty
 
 def gemm_plain(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], resid: Optional[torch.Tensor],
                out_dtype: torch.dtype, out: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """y = x w^T (+bias) (+resid) by the plain tiled kernel; any sizes, f32 or bf16 operands."""
+    """y = x w^T (+bias) (+resid) in float32, ``w`` row-major; any sizes, f32 or bf16 operands."""
     _dev(x, w, bias, resid, out)
     if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
         raise KernelLibraryError(f"gemm shapes do not match: x {tuple(x.shape)}, w {tuple(w.shape)}")
@@ -146,6 +146,50 @@ def gemm_plain(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], r
     lib = library.core()
     check(lib.sb_gemm(_p(out), _dt(out), _p(x), _dt(x), _p(w), _dt(w), _p(bias),
                       _dt(bias) if bias is not None else 0, _p(resid), t, n, k, _stream()))
+    return out
+
+
+def pack_weight_f32(w: torch.Tensor, gated: bool = False) -> torch.Tensor:
+    """A float32 projection weight [out, in] in the order the float32 matrix cores take it: rows and k
+    padded to 16, every 16 x 16 tile one 1 KB block, lane l = 16 g + r of a wave owning the elements
+    [row r][k = g, 4 + g, 8 + g, 12 + g] at offset 4 l, tiles of one row block consecutive in k.  With
+    ``gated`` the two halves [gate; up] are packed one after the other.  Returns a flat float32 tensor."""
+    if w.dim() != 2 or w.dtype != torch.float32:
+        raise KernelLibraryError("pack_weight_f32 takes a float32 matrix [out, in]")
+    out = []
+    for h in (w.chunk(2, dim=0) if gated else (w,)):
+        n, k = h.shape
+        n16, k16 = (n + 15) // 16 * 16, (k + 15) // 16 * 16
+        if (n16, k16) != (n, k):
+            h = torch.nn.functional.pad(h, (0, k16 - k, 0, n16 - n))
+        out.append(h.reshape(n16 // 16, 16, k16 // 16, 4, 4).permute(0, 2, 4, 1, 3).reshape(-1))
+    return torch.cat(out).contiguous() if len(out) > 1 else out[0].contiguous()
+
+
+def gemm_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], resid: Optional[torch.Tensor],
+             out_dtype: torch.dtype, packed_shape, out: Optional[torch.Tensor] = None, gated=False) -> torch.Tensor:
+    """The bits of :func:`gemm_plain` for float32 rows and a weight that :func:`pack_weight_f32` has laid out;
+    ``packed_shape`` = (rows of w, inner size).  With ``gated`` (an activation's name) y = act(x wg^T) * (x wu^T)
+    for w = [wg; wu]."""
+    _dev(x, w, bias, resid, out)
+    rows, k = packed_shape
+    if x.dtype != torch.float32 or w.dtype != torch.float32 or x.dim() != 2 or x.shape[1] != k:
+        raise KernelLibraryError(f"gemm_f32 takes float32 rows of {k} and packed float32 weights, not {tuple(x.shape)} {x.dtype}")
+    gate = gate_code(gated)
+    halves = 2 if gate else 1
+    t, n = x.shape[0], rows // halves
+    if rows % halves or w.numel() != halves * ((n + 15) // 16 * 16) * ((k + 15) // 16 * 16):
+        raise KernelLibraryError(f"{w.numel()} packed elements are not a weight of {packed_shape}")
+    if bias is not None and bias.numel() != n:
+        raise KernelLibraryError(f"bias has {bias.numel()} elements, the product has {n} columns")
+    if resid is not None and (resid.dtype != torch.float32 or tuple(resid.shape) != (t, n)):
+        raise KernelLibraryError("the residual must be float32 and shaped like the product")
+    if out is None:
+        out = torch.empty((t, n), dtype=out_dtype, device=x.device)
+    elif out.dtype != out_dtype or tuple(out.shape) != (t, n):
+        raise KernelLibraryError("gemm output buffer has the wrong shape or type")
+    check(library.core().sb_gemm_f32_packed(_p(out), _dt(out), _p(x), _p(w), _p(bias), _dt(bias) if bias is not None else 0,
+                                            _p(resid), t, n, k, gate, _stream()))
     return out
 
 

@@ -22,6 +22,7 @@ _CORE_SIGNATURES = {
     "sb_embed": [_P, _P, _I, _P, _I, _I, _I, _P],
     "sb_rmsnorm": [_P, _I, _P, _P, _I, _P, _I, _I, _F, _P],
     "sb_gemm": [_P, _I, _P, _I, _P, _I, _P, _I, _P, _I, _I, _I, _P],
+    "sb_gemm_f32_packed": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
     "sb_silu_mul": [_P, _I, _P, _I, _I, _I, _P],
     "sb_gate_mul": [_P, _I, _P, _I, _I, _I, _I, _P],
     "sb_add_into": [_P, _P, _I, _Z, _P],

@@ -4,7 +4,8 @@ Not a part of its own: mixers and feed-forwards own their projections and
 call this helper, which picks the kernel from the types and sizes at hand:
 
 * float32 weights (the 32-bit path, or a tensor the file stores in 32-bit):
-  the plain kernel, true float32 throughout;
+  the float32 matrix cores, true float32 throughout, from a weight laid out once in
+  their order (:func:`sonicboom_amd.ops.pack_weight_f32`);
 * bfloat16 weights and activations: the matrix-core kernels (two that stream
   the weights once for few rows, a tiled one for more).  For them the weight is
   re-laid once, when the projection is built, into the tile order the matrix
@@ -39,10 +40,13 @@ class Linear:
         if bias is not None and bias.numel() != self.n_out:
             raise ValueError(f"bias has {bias.numel()} elements, the projection has {self.n_out} outputs")
         self.bias = None if bias is None else bias.contiguous()
-        self.packed = None
+        self.packed = self.packed_f32 = None
         self.weight = weight.contiguous()
         if fast and weight.is_cuda and weight.dtype == torch.bfloat16 and self.n_in % 8 == 0:
             self.packed = ops.pack_weight(self.weight, gated)
+            self.weight = None
+        elif fast and weight.is_cuda and weight.dtype == torch.float32:
+            self.packed_f32 = ops.pack_weight_f32(self.weight, gated)
             self.weight = None
 
     def _row_major(self) -> torch.Tensor:
@@ -59,6 +63,9 @@ class Linear:
                 x = ops.cast(x, torch.bfloat16)
             return ops.gemm_bf16(x, self.packed, self.bias, resid, out_dtype, out,
                                  packed_shape=(self.rows, self.n_in))
+        if self.packed_f32 is not None:
+            return ops.gemm_f32(ops.cast(x, torch.float32), self.packed_f32, self.bias, resid, out_dtype,
+                                (self.rows, self.n_in), out)
         w = self._row_major()
         if w.dtype == torch.float32 and x.dtype != torch.float32:
             x = ops.cast(x, torch.float32)
@@ -117,6 +124,9 @@ class Linear:
                 x = ops.cast(x, torch.bfloat16)
             return ops.gemm_bf16(x, self.packed, None, None, out_dtype, gated=self.activation,
                                  packed_shape=(self.rows, self.n_in))
+        if self.packed_f32 is not None:
+            return ops.gemm_f32(ops.cast(x, torch.float32), self.packed_f32, None, None, out_dtype,
+                                (self.rows, self.n_in), gated=self.activation)
         w = self._row_major()
         if w.dtype == torch.float32 and x.dtype != torch.float32:
             x = ops.cast(x, torch.float32)

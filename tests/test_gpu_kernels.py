@@ -131,6 +131,27 @@ def test_gemm_plain_does_not_depend_on_the_batch():
         assert torch.equal(alone[0], whole[r])
 
 
+@pytest.mark.parametrize("t, n, k", [(1, 16, 16), (3, 70, 33), (16, 33, 1020), (17, 300, 1024), (33, 130, 1025), (64, 257, 2052),
+                                     (65, 64, 4864), (2, 12300, 48), (700, 272, 9000)])
+def test_gemm_f32_packed_gives_the_bits_of_the_plain_product(t, n, k):
+    """Tile edges, remainders of 4, 16 and 1,024 k, every tile shape of the launcher, rows off 16 bytes."""
+    from sonicboom_amd import ops
+    x, w = randn(t, k).to(DEV), randn(n, k, scale=0.05).to(DEV)
+    bias, resid = randn(n, scale=0.1).to(DEV), randn(t, n).to(DEV)
+    want = ops.gemm_plain(x, w, bias, resid, F32)
+    # the sum of a row of k products, each side within k half-ulps of its chains
+    close(want, ref_gemm(x.cpu(), w.cpu(), bias.cpu(), resid.cpu()), atol=2e-5 * math.sqrt(k), rtol=1e-5, what="gemm_plain")
+    packed = ops.pack_weight_f32(w)
+    assert torch.equal(ops.gemm_f32(x, packed, bias, resid, F32, (n, k)), want)
+    assert torch.equal(ops.gemm_f32(x[t - 1:], packed, bias, resid[t - 1:].contiguous(), F32, (n, k)), want[t - 1:])
+    off = torch.empty(t * k + 1, device=DEV)[1:].view(t, k).copy_(x)
+    assert torch.equal(ops.gemm_f32(off, packed, bias, resid, F32, (n, k)), want)
+    if n % 2 == 0:
+        both = ops.gemm_plain(x, w, None, None, F32)
+        gated = ops.gemm_f32(x, ops.pack_weight_f32(w, True), None, None, F32, (n, k), gated="silu")
+        assert torch.equal(gated, ops.silu_mul(both, F32))
+
+
 @pytest.mark.parametrize("t", [1, 5, 16, 17, 33, 64, 65, 128, 300])
 @pytest.mark.parametrize("n, k", [(96, 64), (100, 96), (224, 200), (3584, 512), (1000, 3584), (72, 18944 // 8)])
 def test_gemm_bf16_matrix_cores(t, n, k):
