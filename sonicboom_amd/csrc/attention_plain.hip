@@ -1,4 +1,4 @@
-// Attention over the paged cache, one wave per (row, query head): the true
+// Attention over the paged cache, one block per (row, query head): the true
 // 32-bit path, and the path of the bf16 engine for sizes its MFMA kernels
 // refuse.
 //
@@ -13,19 +13,38 @@
 // [page][kv head][d][position].
 //
 // Keys are taken 64 at a time in chunks at absolute positions [64c, 64c+64),
-// lane l owning key 64c+l.  The running maximum, the running sum and the
-// output accumulate chunk after chunk in ascending c, and inside a chunk in
-// ascending key, so the arithmetic of a row is a function of its position and
+// lane l owning key 64c+l.  A chunk's maximum, sum and mix are made by one wave from
+// nothing, in ascending key; the chunks' results are joined one after the other in
+// ascending c, so the arithmetic of a row is a function of its position and
 // window alone: it does not change with the batch, with the cut of the prompt
-// into steps or with the physical pages.
+// into steps, with the physical pages or with the waves that share the chunks.
+//
+// It is bound by latency: a chunk is two dependent reads (the page's number, then its
+// keys and values).  The block's waves take a chunk each, and a wave asks for a chunk's values
+// before it reads its keys, sixteen bytes a load.  Measured with 14 heads of 64 in float32: one token of 3
+// sequences of 40 to 260 keys 37.7 us with one wave a row and head and an element a load, 10.7 now; their
+// prompts' 520 rows 116 and 74.
 #include "common.h"
 
 namespace {
 
 constexpr int kMaxHeadDim = 256;
 
-template <typename TA, typename TC>
-__global__ void __launch_bounds__(64)
+// Eight consecutive elements (the caches keep groups of eight together).
+__device__ __forceinline__ void ld_eight(const float *p, float (&v)[8]) {
+  const float4 a = *reinterpret_cast<const float4 *>(p), b = *reinterpret_cast<const float4 *>(p + 4);
+  v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+}
+__device__ __forceinline__ void ld_eight(const bf16_t *p, float (&v)[8]) {
+  const uint4 a = *reinterpret_cast<const uint4 *>(p);
+  const uint32_t w[4] = {a.x, a.y, a.z, a.w};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[2 * i] = __uint_as_float(w[i] << 16), v[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+}
+
+// EIGHTS: head_dim % 8 == 0, and keys are read a group of eight at a time.
+template <typename TA, typename TC, int WAVES, bool EIGHTS>
+__global__ void __launch_bounds__(64 * WAVES)
 attention_plain_kernel(TA *__restrict__ out, const TA *__restrict__ q, int q_stride,
                        const TC *__restrict__ k_cache, const TC *__restrict__ v_cache,
                        const int32_t *__restrict__ page_table, int max_pages, int n_pages_total,
@@ -33,12 +52,16 @@ attention_plain_kernel(TA *__restrict__ out, const TA *__restrict__ q, int q_str
                        int heads_q, int heads_kv, int head_dim, float scale, int window, int v_dim,
                        float softcap, int sink, const float *__restrict__ sink_scores,
                        const float *__restrict__ gate, int gate_stride, int gate_per_head, int chunk) {
+  constexpr int kThreads = 64 * WAVES, kDims = (kMaxHeadDim + kThreads - 1) / kThreads;
   __shared__ float qs[kMaxHeadDim];
-  __shared__ float ps[64];
-  const int row = blockIdx.x, h = blockIdx.y, lane = threadIdx.x;
+  __shared__ float ps[WAVES][64];
+  __shared__ float part_m[WAVES], part_l[WAVES];
+  __shared__ float part_o[WAVES][kMaxHeadDim];
+  const int row = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int pos = row_pos[row], seq = row_seq[row];
   const int kvh = h / (heads_q / heads_kv);
-  for (int d = lane; d < head_dim; d += 64) qs[d] = ld_f(q, size_t(row) * q_stride + size_t(h) * head_dim + d);
+  for (int d = tid; d < head_dim; d += kThreads) qs[d] = ld_f(q, size_t(row) * q_stride + size_t(h) * head_dim + d);
   __syncthreads();
 
   const int lo = chunk > 0 ? pos - pos % chunk : (window > 0 && pos >= window) ? pos - window + 1 : 0;
@@ -47,52 +70,105 @@ attention_plain_kernel(TA *__restrict__ out, const TA *__restrict__ q, int q_str
   // number (as it is: no scale, no cap): the running maximum starts at its score and the running
   // sum at its weight
   float m = sink ? (sink_scores ? sink_scores[h] : 0.0f) : neg_inf, l = sink ? 1.0f : 0.0f;
-  float o[kMaxHeadDim / 64] = {0.0f, 0.0f, 0.0f, 0.0f};
-
-  for (int c = lo / SB_PAGE; c <= pos / SB_PAGE; ++c) {
-    const int page = c < max_pages ? page_table[size_t(seq) * max_pages + c] : -1;
-    if (page < 0 || page >= n_pages_total) continue;  // uniform over the wave
-    const TC *kp = k_cache + (size_t(page) * heads_kv + kvh) * SB_PAGE * head_dim;
-    const TC *vp = v_cache + (size_t(page) * heads_kv + kvh) * SB_PAGE * v_dim;
-    const int j = c * SB_PAGE + lane;
-    const bool visible = j >= lo && j <= pos;
-    float s = neg_inf;
-    if (visible) {
-      float dot = 0.0f;
-      for (int d = 0; d < head_dim; ++d) dot = fmaf(qs[d], ld_f(kp, sb_key_index(lane, d, head_dim)), dot);
-      s = dot * scale;
-      if (softcap > 0.0f) s = softcap * tanhf(s / softcap);
-    }
-    const float cm = wave_max(s);
-    const float m_new = fmaxf(m, cm);
-    const float p = visible ? expf(s - m_new) : 0.0f;
-    const float alpha = expf(m - m_new);  // 0 for the first chunk
-    l = l * alpha + wave_sum(p);
-    ps[lane] = p;
-    __syncthreads();
-    const int j0 = max(lo - c * SB_PAGE, 0), j1 = min(pos - c * SB_PAGE, SB_PAGE - 1);
+  float o[kDims];
 #pragma unroll
-    for (int i = 0; i < kMaxHeadDim / 64; ++i) {
-      const int d = lane + 64 * i;
-      if (d < v_dim) {
-        float acc = o[i] * alpha;
-        for (int jj = j0; jj <= j1; ++jj) acc = fmaf(ps[jj], ld_f(vp, sb_value_index(d, jj)), acc);
-        o[i] = acc;
+  for (int i = 0; i < kDims; ++i) o[i] = 0.0f;
+
+  const int c_end = pos / SB_PAGE + 1;
+  for (int c0 = lo / SB_PAGE; c0 < c_end; c0 += WAVES) {
+    const int c = c0 + wave;
+    const int page = c < c_end && c < max_pages ? page_table[size_t(seq) * max_pages + c] : -1;
+    const bool live = page >= 0 && page < n_pages_total;      // uniform over the wave
+    if (live) {
+      const TC *kp = k_cache + (size_t(page) * heads_kv + kvh) * SB_PAGE * head_dim;
+      const TC *vp = v_cache + (size_t(page) * heads_kv + kvh) * SB_PAGE * v_dim;
+      const int j = c * SB_PAGE + lane;
+      const bool visible = j >= lo && j <= pos;
+      // the values of this lane's first dimension, asked for ahead of the keys
+      float v[8][8];
+      if (lane < v_dim) {
+#pragma unroll
+        for (int jg = 0; jg < 8; ++jg) ld_eight(vp + sb_value_index(lane, 8 * jg), v[jg]);
       }
+      float s = neg_inf;
+      if (visible) {
+        float dot = 0.0f;
+        if constexpr (EIGHTS) {
+#pragma unroll 8
+          for (int d = 0; d < head_dim; d += 8) {
+            float k8[8];
+            ld_eight(kp + sb_key_index(lane, d, head_dim), k8);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) dot = fmaf(qs[d + e], k8[e], dot);
+          }
+        } else {
+          for (int d = 0; d < head_dim; ++d) dot = fmaf(qs[d], ld_f(kp, sb_key_index(lane, d, head_dim)), dot);
+        }
+        s = dot * scale;
+        if (softcap > 0.0f) s = softcap * tanhf(s / softcap);
+      }
+      const float cm = wave_max(s);
+      const float p = visible ? expf(s - cm) : 0.0f;
+      const float cl = wave_sum(p);
+      ps[wave][lane] = p;
+      if (lane == 0) part_m[wave] = cm, part_l[wave] = cl;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      // (keys outside the window are left out by their place, not by a weight of zero: what the
+      // cache holds there is anything)
+      const int j0 = max(lo - c * SB_PAGE, 0), j1 = min(pos - c * SB_PAGE, SB_PAGE - 1);
+      for (int d = lane; d < v_dim; d += 64) {
+        if (d >= 64) {
+#pragma unroll
+          for (int jg = 0; jg < 8; ++jg) ld_eight(vp + sb_value_index(d, 8 * jg), v[jg]);
+        }
+        float acc = 0.0f;
+#pragma unroll
+        for (int jj = 0; jj < SB_PAGE; ++jj) acc = fmaf(ps[wave][jj], jj >= j0 && jj <= j1 ? v[jj >> 3][jj & 7] : 0.0f, acc);
+        part_o[wave][d] = acc;
+      }
+    } else if (lane == 0) {
+      part_l[wave] = -1.0f;                      // no such chunk
     }
     __syncthreads();
-    m = m_new;
+    for (int w = 0; w < WAVES; ++w) {
+      const float cl = part_l[w];
+      if (cl < 0.0f) continue;                   // (a sum that is not a number goes on)
+      const float cm = part_m[w], m_new = fmaxf(m, cm);
+      const float alpha = expf(m - m_new), beta = expf(cm - m_new);      // alpha 0 for the first chunk
+      l = l * alpha + cl * beta;
+#pragma unroll
+      for (int i = 0; i < kDims; ++i) {
+        const int d = tid + kThreads * i;
+        if (d < v_dim) o[i] = o[i] * alpha + part_o[w][d] * beta;
+      }
+      m = m_new;
+    }
+    __syncthreads();
   }
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
-  for (int i = 0; i < kMaxHeadDim / 64; ++i) {
-    const int d = lane + 64 * i;
+  for (int i = 0; i < kDims; ++i) {
+    const int d = tid + kThreads * i;
     if (d < v_dim) {
       float r = o[i] * inv;
       // an output gate: the result times the sigmoid of the gate's number at the same place of the row, or of the head's one
       if (gate) r = r * (1.0f / (1.0f + expf(-gate[size_t(row) * gate_stride + (gate_per_head ? size_t(h) : size_t(h) * v_dim + d)])));
       st_f(out, size_t(row) * heads_q * v_dim + size_t(h) * v_dim + d, r);
     }
+  }
+}
+
+// Waves of a block: four, each a chunk of 64 keys at a time; eight where the blocks alone leave SIMDs idle.
+template <typename TA, typename TC, typename... A>
+void launch_attention(dim3 grid, int head_dim, hipStream_t s, A... a) {
+  const bool few = (long long)grid.x * grid.y <= 512;
+  if (head_dim % 8 == 0) {
+    if (few) attention_plain_kernel<TA, TC, 8, true><<<grid, 512, 0, s>>>(a...);
+    else attention_plain_kernel<TA, TC, 4, true><<<grid, 256, 0, s>>>(a...);
+  } else {
+    attention_plain_kernel<TA, TC, 4, false><<<grid, 256, 0, s>>>(a...);
   }
 }
 
@@ -190,7 +266,7 @@ extern "C" int sb_attention_chunked(void *out, const void *q, int act_dtype, int
   hipStream_t s = (hipStream_t)stream;
   dim3 grid(n_rows, heads_q);
 #define SB_GO(TA, TC)                                                                           \
-  attention_plain_kernel<TA, TC><<<grid, 64, 0, s>>>(                                            \
+  launch_attention<TA, TC>(grid, head_dim, s,                                                    \
       (TA *)out, (const TA *)q, q_stride, (const TC *)k_cache, (const TC *)v_cache, page_table,  \
       max_pages, n_pages_total, row_pos, row_seq, heads_q, heads_kv, head_dim, scale, window, v_dim,  \
       softcap, sink, sink_scores, gate, gate_stride, gate_per_head, chunk)
