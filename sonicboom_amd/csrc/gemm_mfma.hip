@@ -23,6 +23,22 @@
 namespace {
 
 constexpr int kXcds = 8;
+
+// The gate's activation in the epilogue of a tile: gate_act, with SiLU's exponential and division on the
+// vector units' own exp2 and reciprocal.  exp(-g) = 2^(h + l), the product with log2(e) carried in two
+// parts, and one Newton step on the quotient keep it within two units of the last of 24 bits (the result is
+// rounded to 8 of them next).  expf and the full division cost a 256 x 256 tile's epilogue 8.5 us of
+// vector instructions, 9 % of the tile at 3,584 k.
+template <int GATE>
+__device__ __forceinline__ float tile_gate(float g) {
+  if constexpr (GATE != SB_GATE_SILU) return gate_act(g, GATE);
+  const bool inside = fabsf(g) < 80.0f;          // outside, the corrections may meet infinities
+  const float h = g * -1.44269502f, l = fmaf(g, -1.44269502f, -h) + g * -1.92596303e-8f;
+  const float e = __builtin_amdgcn_exp2f(h);
+  const float d = 1.0f + (inside ? fmaf(e, l * 0.693147182f, e) : e), r = __builtin_amdgcn_rcpf(d);
+  const float q = g * r;
+  return inside ? fmaf(fmaf(-d, q, g), r, q) : q;
+}
 typedef uint16_t u16x4_t __attribute__((ext_vector_type(4)));
 
 struct Args {
@@ -90,7 +106,8 @@ __device__ __forceinline__ bool tile_of_block(const Args &a, int block, int &tm,
 // program order, so a fence for the compiler is all the ordering it needs.
 // SLABS groups of SLAB rows (32 or 16) make a wave's rows, NW: waves along N, NC: output columns
 // of a wave; `lds_f`: at least (waves of the block) * SLAB * PITCH floats.
-template <int SLABS, int SLAB, int NW, int NC, int PITCH, class Fill>
+// SWZ (PITCH = NC = 64, SLAB 16): no padding, the four quarters of row r turned round by r / 4.
+template <int SLABS, int SLAB, int NW, int NC, int PITCH, bool SWZ = false, class Fill>
 __device__ __forceinline__ void store_tile(const Args &a, float *lds_f, int t0, int n0, bool raw_allowed, Fill fill) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int wm = wave / NW, wn = wave % NW;
@@ -115,7 +132,7 @@ __device__ __forceinline__ void store_tile(const Args &a, float *lds_f, int t0, 
     for (int p = 0; p < kPasses; ++p) {
       const int r = p * kRowsPerPass + r_in;
       const int t = t0 + wm * (SLABS * SLAB) + i * SLAB + r;
-      floatx4_t v = *reinterpret_cast<const floatx4_t *>(turn + r * PITCH + c4);
+      floatx4_t v = *reinterpret_cast<const floatx4_t *>(turn + r * PITCH + (SWZ ? c4 ^ (((r >> 2) & 3) * 16) : c4));
       if (t >= a.n_rows || n_first >= a.n_out) continue;
       const size_t idx = size_t(t) * a.n_out + n_first;
       if (a.vec4) {
@@ -170,7 +187,7 @@ __device__ __forceinline__ void fill_from_32(floatx16_t (&acc)[MT][2], int i, fl
   for (int e = 0; e < 16; ++e) {
     const int row = 8 * (e >> 2) + row_base + (e & 3);
     if (GATED) {
-      turn[row * kPitch + col] = gate_act(acc[i][0][e], GATED) * acc[i][1][e];   // GATED: the sb_gate, fixed at compile time
+      turn[row * kPitch + col] = tile_gate<GATED>(acc[i][0][e]) * acc[i][1][e];   // GATED: the sb_gate, fixed at compile time
     } else {
       turn[row * kPitch + col] = acc[i][0][e];
       turn[row * kPitch + 32 + col] = acc[i][1][e];
@@ -456,13 +473,16 @@ gemm_mfma_kernel(Args a) {
 // bank conflicts without a swizzle.  Fragments: B for a whole k-step in two sets of registers, A
 // in a ring of four tiles that runs two tiles ahead of the MFMAs.
 //
+// (Two waves a SIMD are asked for also where LDS holds one block of four: with 512 registers to a wave the
+// compiler kept half of the accumulators in the other register file and moved 96 of them a stage.)
+//
 // PERSIST: the grid is one round of blocks, and a block goes on to the tile one grid further
 // until the tiles end.  The last stage of a tile then loads the first stage of the next tile (not
 // itself once more), so the next tile's loop starts right after the epilogue with its operands in
 // LDS, the epilogue's stores drain behind the next tile's products instead of holding the CU
 // until the block has left, and no block has to be started for a tile.
 template <int MT16, int NW, int BK, int NBUF, int GATED, bool PERSIST>
-__global__ void __launch_bounds__(128 * NW)
+__global__ void __launch_bounds__(128 * NW, 2)
 gemm_direct16_kernel(Args a) {
   constexpr int BM = 32 * MT16, BN = 64 * NW, kThreads = 128 * NW, kWaves = kThreads / 64;
   constexpr int CPR = BK / 8;                       // 16-byte chunks in an LDS row of A
@@ -577,7 +597,11 @@ gemm_direct16_kernel(Args a) {
         acc[i][f] = mfma16(fa[tile & 3], fb[j & 1][f], acc[i][f]);
         if (f == 0 && tile + 2 < kTiles) read_a(tile + 2);
         // the next k-step's B fragments, one with each of the first A tiles of this one
-        if (f == 1 && i < 4 && j + 1 < kSteps32) read_b(j + 1, i);
+        // (two tiles a k-step: two with each)
+        if (f == 1 && i < 4 && j + 1 < kSteps32) {
+#pragma unroll
+          for (int ff = i; ff < 4; ff += MT16) read_b(j + 1, ff);
+        }
         if (f >= 2 && tile * 2 + (f - 2) < kLoads) issue_load(tile * 2 + (f - 2), kt_load, buf_load);
         // keep this order: left alone, the scheduler gathers the memory operations into lumps
         // and reads each fragment right before its MFMA, and the matrix pipe waits on both
@@ -603,7 +627,7 @@ gemm_direct16_kernel(Args a) {
             if (GATED) {
 #pragma unroll
               for (int f = 0; f < 2; ++f)
-                turn[row * kPitch + f * 16 + fr] = gate_act(acc[i][f][e], GATED) * acc[i][f + 2][e];
+                turn[row * kPitch + f * 16 + fr] = tile_gate<GATED>(acc[i][f][e]) * acc[i][f + 2][e];
             } else {
 #pragma unroll
               for (int f = 0; f < 4; ++f) turn[row * kPitch + f * 16 + fr] = acc[i][f][e];
@@ -644,6 +668,176 @@ gemm_direct16_kernel(Args a) {
     epilogue(tm, tn, NBUF == 2 ? (buf ^ 1) : 0);
     if (!PERSIST || !more) break;
     // the next stage's loads go into the buffer that the epilogue has turned its rows through
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    vblock += int(gridDim.x);
+    tm = tm_next;
+    tn = tn_next;
+  }
+}
+
+
+// ---------------------------------------------------------------------------------------------
+// The same, 256 x 256 tiles, in stages of 32 k through four buffers.  In the kernel above every wave
+// comes out of a stage's barrier with empty hands: it reads six fragments and waits for them before its first
+// product, both waves of a SIMD at once.  Here the barrier that ends stage s promises stage s + 2 (the wait
+// before it leaves only the newest stage's loads in flight), so the first fragments of stage s + 1 are read
+// in stage s, with its last tiles, and the products go on right behind the barrier.
+// A's rows are 64 bytes a stage: two 16-row tiles lie side by side in the 128-byte lines of LDS whose
+// swizzle the fragment reads take without conflicts.  The epilogue turns its rows through the one buffer that
+// holds nothing (swizzled instead of padded: it is exactly as large).
+// Measured, kernel above against this one: 3.6 % faster on the gate/up product of 2,048 x 37,888 x 3,584 (469 and 451 us),
+// 8 % on 6,398 x 2,048 x 11,008 (257 and 236), 3 % on 16,384 x 3,584 x 18,944 (1.87 and 1.81 ms), each by itself; in whole
+// prompt steps, back to back, 1 to 2.5 %.  What bounds it: with the loads left out 1.6 to 1.8 PFLOP/s, with the products left
+// out 0.55 of the time; the two together run at the clock that the chip's power allows.
+template <int GATED, bool PERSIST>
+__global__ void __launch_bounds__(512)
+gemm_pipe_kernel(Args a) {
+  constexpr int MT16 = 8, NW = 4, BM = 256, BN = 256, kWaves = 8, NBUF = 4;
+  constexpr int kLoads = 4;                          // of a wave and stage: two of A, two of W
+  constexpr int kBufChunks = (BM + BN) * 4;          // 16-byte chunks of a stage buffer: A, then W
+  extern __shared__ bf16x8_t lds[];
+  typedef __attribute__((address_space(3))) bf16x8_t *lds_ptr_t;
+
+  int vblock = blockIdx.x, tm, tn;
+  if (!tile_of_block(a, vblock, tm, tn)) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / NW, wn = wave % NW;
+
+  const size_t w_rows_total = size_t(GATED ? 2 : 1) * size_t(a.w_tiles) * 16;
+  const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t *>(a.x), 0, uint32_t(size_t(a.n_rows) * a.n_in * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t *>(a.w), 0, uint32_t(w_rows_total * size_t(a.w_steps) * 64), 0x00020000);
+  // sources of the loads at stage 0 of tile (m, n): as in the kernel above but for A's lines: line l of a
+  // buffer holds, in the places p ^ (l / 2) % 8, chunks p % 4 of row l % 16 of tiles 2 (l / 16) (p < 4) and the next
+  uint32_t off[kLoads];
+  auto aim_at = [&](int m, int n) {
+    const int t0 = m * BM, n0 = n * (GATED ? BN / 2 : BN);
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+      if (i < 2) {
+        const int place = (i * kWaves + wave) * 64 + lane;
+        const int line = place / 8, c8 = (place % 8) ^ ((line / 2) & 7);
+        const int row = (line / 16) * 32 + (c8 >> 2) * 16 + line % 16;
+        off[i] = uint32_t((size_t(t0 + row) * a.n_in + (c8 & 3) * 8) * 2);
+      } else {
+        const int rt = (i - 2) * kWaves + wave;
+        const int tile = GATED ? ((rt & 3) >> 1) * a.w_tiles + n0 / 16 + (rt >> 2) * 2 + (rt & 1) : n0 / 16 + rt;
+        off[i] = uint32_t((size_t(tile) * a.w_steps * 512 + size_t(lane) * 8) * 2);
+      }
+    }
+  };
+  auto issue_load = [&](int i, int kt, int buf) {
+    const bool is_a = i < 2;
+    const int chunk = buf * kBufChunks + (is_a ? (i * kWaves + wave) * 64 : BM * 4 + ((i - 2) * kWaves + wave) * 64);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(is_a ? rsrc_x : rsrc_w, (lds_ptr_t)(lds) + chunk, 16, int(off[i]),
+                                             is_a ? kt * 64 : kt * 1024, 0, 0);
+  };
+  // everything but the loads of the newest stage has landed, for this wave and after the barrier for all
+  auto wait_and_meet = [&]() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+
+  // stages of 32 k, an even count (the host: an inner size in 64s, slices of whole 64s)
+  const int n_k_all = a.n_in / 32;
+  const int kt_begin = a.partial ? int(blockIdx.y) * a.stages_per_slice * 2 : 0;
+  const int n_k = a.partial ? min(kt_begin + a.stages_per_slice * 2, n_k_all) : n_k_all;
+  // A stage past the end (of the last tile, when the block goes on) is the last stage once more, into a
+  // buffer that nobody reads again, so that the count of loads in flight stays the same.
+  aim_at(tm, tn);
+#pragma unroll
+  for (int s = 0; s < NBUF - 1; ++s)
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) issue_load(i, min(kt_begin + s, n_k - 1), s);
+  wait_and_meet();
+
+  const int fr = lane & 15, fg = lane >> 4;
+  int a_lane[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) a_lane[j] = wm * (16 * MT16) * 4 + fr * 8 + ((4 * j + fg) ^ ((fr / 2) & 7));
+  auto a_at = [&](int i) { return a_lane[i & 1] + (i >> 1) * 128; };
+  const int b_lane = BM * 4 + wn * 4 * 64 + lane;
+
+  floatx4_t acc[MT16][4];
+  bf16x8_t fa[4], fb[2][4];       // A in a ring of four tiles, W in a set for even and one for odd stages
+  auto stage = [&](auto PAR, int buf, int kt_load) {
+    constexpr int par = decltype(PAR)::value;
+    const bf16x8_t *ls = lds + buf * kBufChunks, *ls_next = lds + ((buf + 1) & (NBUF - 1)) * kBufChunks;
+    const int buf_load = (buf + NBUF - 1) & (NBUF - 1);
+#pragma unroll
+    for (int i = 0; i < MT16; ++i) {
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        acc[i][f] = mfma16(fa[i & 3], fb[par][f], acc[i][f]);
+        // two tiles ahead; the next stage's first two with the last two of this one, its W with the last four
+        if (f == 0) fa[(i + 2) & 3] = i + 2 < MT16 ? ls[a_at(i + 2)] : ls_next[a_at(i + 2 - MT16)];
+        if (f == 1 && i >= MT16 - 4) fb[par ^ 1][i - (MT16 - 4)] = ls_next[b_lane + (i - (MT16 - 4)) * 64];
+        if (f >= 2 && i < 2) issue_load(i * 2 + f - 2, kt_load, buf_load);
+        __builtin_amdgcn_sched_barrier(0);       // keep this order (see above)
+      }
+    }
+    wait_and_meet();
+  };
+
+  constexpr int NC = GATED ? 32 : 64, kPitch = GATED ? NC + 4 : NC;
+  static_assert(kBufChunks * 16 >= kWaves * 16 * kPitch * 4, "the turning areas must fit a stage buffer");
+  auto epilogue = [&](int m, int n, int buf_free) {
+    store_tile<MT16, 16, NW, NC, kPitch, !GATED>(
+        a, reinterpret_cast<float *>(lds + buf_free * kBufChunks), m * BM, n * (GATED ? BN / 2 : BN), !GATED,
+        [&](int i, float *turn) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int row = 4 * fg + e;
+            if (GATED) {
+#pragma unroll
+              for (int f = 0; f < 2; ++f)
+                turn[row * kPitch + f * 16 + fr] = tile_gate<GATED>(acc[i][f][e]) * acc[i][f + 2][e];
+            } else {
+#pragma unroll
+              for (int f = 0; f < 4; ++f) turn[row * kPitch + (f ^ fg) * 16 + fr] = acc[i][f][e];
+            }
+          }
+        });
+  };
+
+  int buf = 0;
+#pragma unroll
+  for (int f = 0; f < 4; ++f) fb[0][f] = lds[b_lane + f * 64];
+  fa[0] = lds[a_at(0)];
+  fa[1] = lds[a_at(1)];
+  for (;;) {
+#pragma unroll
+    for (int i = 0; i < MT16; ++i)
+#pragma unroll
+      for (int f = 0; f < 4; ++f) acc[i][f] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    int tm_next = 0, tn_next = 0;
+    const bool more = PERSIST && tile_of_block(a, vblock + int(gridDim.x), tm_next, tn_next);
+    auto stage_to_load = [&](int kt) {
+      const int l = kt + NBUF - 1;
+      if (l < n_k) return l;
+      if (!PERSIST || !more) return n_k - 1;
+      if (l == n_k) aim_at(tm_next, tn_next);    // from here on the loads are the next tile's
+      return l - n_k + kt_begin;
+    };
+    for (int kt = kt_begin; kt < n_k; kt += 2) {
+      stage(std::integral_constant<int, 0>{}, buf, stage_to_load(kt));
+      buf = (buf + 1) & (NBUF - 1);
+      stage(std::integral_constant<int, 1>{}, buf, stage_to_load(kt + 1));
+      buf = (buf + 1) & (NBUF - 1);
+    }
+    if (!PERSIST || !more) {
+      // the last loads (of the last stage again) are still writing LDS
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    epilogue(tm, tn, (buf + NBUF - 1) & (NBUF - 1));       // the other three hold the next tile's first stages
+    if (!PERSIST || !more) break;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -735,9 +929,45 @@ int launch_direct(const Args &a, long long blocks, int round_blocks, hipStream_t
   }
 }
 
+template <int GATED, bool PERSIST>
+int launch_pipe_one(const Args &a, long long blocks, hipStream_t s) {
+  constexpr int lds_bytes = 4 * (256 + 256) * 4 * 16;
+  static bool raised = false;     // per instantiation; harmless if repeated
+  if (!raised) {
+    const hipError_t e = hipFuncSetAttribute((const void *)gemm_pipe_kernel<GATED, PERSIST>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             lds_bytes);
+    SB_REQUIRE(e == hipSuccess, "sb_gemm_mfma_bf16: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    raised = true;
+  }
+  const int n_k = a.n_in / 64;
+  const unsigned slices = a.partial ? unsigned((n_k + a.stages_per_slice - 1) / a.stages_per_slice) : 1u;
+  long long grid = (blocks + kXcds - 1) / kXcds * kXcds;
+  if (PERSIST && grid > sb::cu_count()) grid = sb::cu_count();        // 128 KB of LDS: a block a CU
+  gemm_pipe_kernel<GATED, PERSIST><<<dim3(unsigned(grid), slices), 512, lds_bytes, s>>>(a);
+  return SB_OK;
+}
+
+int launch_pipe(const Args &a, long long blocks, bool a_block_a_tile, hipStream_t s) {
+  // (going on to the next tile, whose first three stages are loaded in the last of this one, takes four stages)
+  if (a_block_a_tile || a.n_in < 128) {
+    switch (a.gated) {
+      case 3: return launch_pipe_one<3, false>(a, blocks, s);
+      case 2: return launch_pipe_one<2, false>(a, blocks, s);
+      case 1: return launch_pipe_one<1, false>(a, blocks, s);
+      default: return launch_pipe_one<0, false>(a, blocks, s);
+    }
+  }
+  switch (a.gated) {
+    case 3: return launch_pipe_one<3, true>(a, blocks, s);
+    case 2: return launch_pipe_one<2, true>(a, blocks, s);
+    case 1: return launch_pipe_one<1, true>(a, blocks, s);
+    default: return launch_pipe_one<0, true>(a, blocks, s);
+  }
+}
+
 // Tile shapes the launcher chooses from: rows x columns of Y per block.
 struct Shape { int bm, bn; };
-constexpr Shape kShapes[5] = {{128, 128}, {256, 128}, {256, 256}, {128, 256}, {192, 256}};
+constexpr Shape kShapes[6] = {{128, 128}, {256, 128}, {256, 256}, {128, 256}, {192, 256}, {64, 128}};
 
 // The tile shape for a problem: the one with the best product of three factors.  How fast the
 // shape's kernel runs on a full grid, relative to 128 x 128 (measured on MI355X at 2,048 to 16,384
@@ -825,15 +1055,23 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
   a.vec4 = n_out % 4 == 0 && (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(resid)) % 16 == 0;
   const bool direct_ok = packed && n_in % 64 == 0;
   int variant = pick_shape(n_rows, n_out, n_in, a.gated, direct_ok);
-  // a test's or a measurement's choice: the shape (0..3) + 16 * the path (0: the launcher's, 1:
-  // through registers, 2: straight into LDS)
+  // Gated products of a few hundred rows (K cannot be cut over the grid): 128 x 128 tiles straight into LDS
+  // where they make one round over the CUs (288 rows against 9,728 x 896: 14.2 us, through registers 15.1); a
+  // little over one round, 64 x 128 tiles, three to a CU (183 rows against 17,920 x 1,536, 280 tiles of 128: 26.4 and 31.5).
   int path = 0;
+  if (gated && direct_ok && variant == 0 && n_rows <= 384) {
+    const long long tiles = (long long)((n_rows + 127) / 128) * ((n_out + 63) / 64);
+    if (tiles <= sb::cu_count()) path = 2;
+    else if (tiles <= sb::cu_count() * 3 / 2 && (n_rows + 63) / 64 * 64 < (n_rows + 127) / 128 * 128) variant = 5, path = 2;
+  }
+  // a test's or a measurement's choice: the shape (0..5) + 16 * the path (0: the launcher's, 1:
+  // through registers, 2: straight into LDS)
   if (tile_shape >= 0) {
-    SB_REQUIRE((tile_shape & 15) < 5 && (tile_shape >> 4) < 4, "sb_gemm_mfma_bf16: unknown tile shape %d", tile_shape);
+    SB_REQUIRE((tile_shape & 15) < 6 && (tile_shape >> 4) < 4, "sb_gemm_mfma_bf16: unknown tile shape %d", tile_shape);
     variant = tile_shape & 15;
     path = tile_shape >> 4;
   }
-  if (!packed) variant = 0;       // the bigger tiles are built for packed weights only
+  if (!packed) variant = 0, path = 0;       // the bigger tiles are built for packed weights only
   const int bm = kShapes[variant].bm, bn = gated ? kShapes[variant].bn / 2 : kShapes[variant].bn;
   a.tiles_m = (n_rows + bm - 1) / bm;
   a.tiles_n = (n_out + bn - 1) / bn;
@@ -852,19 +1090,21 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
   a.w_steps = (n_in + 31) / 32;
   int rc;
   SB_SUPPORT(path < 2 || direct_ok, "sb_gemm_mfma_bf16: the direct path takes packed weights and an inner size in 64s");
-  // left to itself only the 256 x 256 shape goes straight into LDS: the smaller tiles' stages are too
+  // left to themselves the shapes of 256 columns go straight into LDS; the smaller tiles' stages are too
   // short for loads that run one stage ahead, and the register path, which runs two ahead, is
-  // faster there (128 x 128, QKV product at 2,048 rows: 92 against 128 us)
+  // faster there unless the tiles make one round and LDS holds four stages of each
   const bool direct = path >= 2 || (path == 0 && direct_ok && (variant == 2 || variant == 4));
-  SB_SUPPORT(variant < 3 || direct, "sb_gemm_mfma_bf16: the shapes 128 x 256 and 192 x 256 exist on the direct path only");
+  SB_SUPPORT(variant < 3 || direct, "sb_gemm_mfma_bf16: the shapes 128 x 256, 192 x 256 and 64 x 128 exist on the direct path only");
   if (direct) {
-    // path 3 (a measurement's): the 256 x 256 shape with a block for every tile
-    if (variant == 0) rc = launch_direct<4, 2, 64, 2, false>(a, blocks, 0, s);
+    // the shapes of four waves take as many buffers as the tiles' count leaves LDS for: four (a block a CU, three
+    // stages in flight) in one round over the CUs, else two (two or three blocks a CU)
+    const bool one_round = (blocks + kXcds - 1) / kXcds * kXcds <= sb::cu_count();
+    if (variant == 0) rc = one_round ? launch_direct<4, 2, 64, 4, false>(a, blocks, 0, s) : launch_direct<4, 2, 64, 2, false>(a, blocks, 0, s);
     else if (variant == 1) rc = launch_direct<8, 2, 64, 2, false>(a, blocks, 0, s);
-    else if (variant == 2 && path == 3) rc = launch_direct<8, 4, 64, 2, false>(a, blocks, 0, s);
-    else if (variant == 2) rc = launch_direct<8, 4, 64, 2, true>(a, blocks, sb::cu_count(), s);     // 128 KB of LDS: a block a CU
+    else if (variant == 2) rc = launch_pipe(a, blocks, path == 3, s);      // (path 3: a measurement's)
     else if (variant == 3) rc = launch_direct<4, 4, 64, 2, false>(a, blocks, 0, s);
-    else rc = launch_direct<6, 4, 64, 2, true>(a, blocks, sb::cu_count(), s);
+    else if (variant == 4) rc = launch_direct<6, 4, 64, 2, true>(a, blocks, sb::cu_count(), s);
+    else rc = one_round ? launch_direct<2, 2, 64, 4, false>(a, blocks, 0, s) : launch_direct<2, 2, 64, 2, false>(a, blocks, 0, s);
   } else {
     if (variant == 0) rc = launch<2, 2, 64, 2, true>(a, blocks, packed, s);
     else if (variant == 1) rc = launch<4, 2, 64, 2, false>(a, blocks, packed, s);
@@ -892,7 +1132,15 @@ namespace {
 // round as it is, a cut priced at 0.9 to 0.97 measured 0.99 to 1.04).  Measured, whole + norm against cut + the pass that adds the slices, the
 // residual and the norm: down (3,584 x 18,944) at 1,280 rows 237 against 152 us, at 2,048 rows 272
 // against 247; output (3,584 x 3,584) at 1,280 rows 69 against 52.
-struct PartialPlan { int slices; bool big; };
+//
+// A few hundred rows: the same tiles of 128 x 128, or of 64 x 128, loaded straight into LDS with four
+// stages' buffers, a block a CU, where tiles x slices make one round over each die's 32 CUs.  A launch costs
+// 3.5 us and a stage of 64 k, measured at 183 to 500 rows of the 0.5B to 7B products, 0.33 us (64 rows), 0.55 (128 rows)
+// and 0.65 (128 x 128 through registers); the consumer reads and the product writes a slice at 4 TB/s.
+// 183 rows against 1,536 x 1,536: 8.5 us through registers, 6.2; 288 against 896 x 4,864: 14.9 and 9.8; 183 against
+// 3,584 x 18,944: 50.9 and 45.5.
+enum PartialTile { kRegisters128, kBig, kDirect128, kDirect64 };
+struct PartialPlan { int slices; PartialTile tile; };
 double load_factor(long long blocks) { return blocks <= 170 ? 0.72 : 0.72 + 0.28 * double(blocks - 170) / 86.0; }
 PartialPlan partial_plan(int n_rows, int n_out, int n_in, bool direct_ok) {
   const long long tiles = (long long)((n_rows + 127) / 128) * ((n_out + 127) / 128);
@@ -925,11 +1173,28 @@ PartialPlan partial_plan(int n_rows, int n_out, int n_in, bool direct_ok) {
     }
     if (s_best && t_best < 0.9 * t_whole) {
       const int per = int((n_k + s_best - 1) / s_best);
-      return {(n_k + per - 1) / per, true};
+      return {(n_k + per - 1) / per, kBig};
     }
   }
+  if (s > 1 && direct_ok && n_rows <= 512) {
+    const auto cost = [&](double stage_us, long long slices) {
+      return stage_us * double((n_k + slices - 1) / slices) + 2.0 * slices * n_rows * double(n_out) * 4.0 / 4e6;
+    };
+    double best = cost(0.65, s);
+    PartialTile tile = kRegisters128;
+    for (int half = 0; half < 2; ++half) {
+      const int bm = half ? 64 : 128;
+      const long long n_tiles = (long long)((n_rows + bm - 1) / bm) * ((n_out + 127) / 128);
+      for (long long s2 = 2; s2 <= 8 && (n_tiles + kXcds - 1) / kXcds * s2 <= sb::cu_count() / kXcds && s2 * 3 <= n_k; ++s2) {
+        const double t = cost(half ? 0.33 : 0.55, s2);
+        if (t < best) best = t, tile = half ? kDirect64 : kDirect128, s = s2;
+      }
+    }
+    const int per = int((n_k + s - 1) / s);
+    return {(n_k + per - 1) / per, tile};
+  }
   const int per = int((n_k + s - 1) / s);
-  return {(n_k + per - 1) / per, false};
+  return {(n_k + per - 1) / per, kRegisters128};
 }
 }  // namespace
 
@@ -955,9 +1220,9 @@ extern "C" int sb_gemm_mfma_partial_bf16(float *partial, const void *x, const vo
   a.bias = nullptr; a.bias_dtype = 0; a.resid = nullptr; a.resid_scale = 1.0f;
   a.n_rows = n_rows; a.n_out = n_out; a.n_in = n_in; a.gated = 0; a.relu_sq = 0;
   const PartialPlan plan = partial_plan(n_rows, n_out, n_in, packed && n_in % 64 == 0);
-  const int tile = plan.big ? 256 : 128;
-  a.tiles_m = (n_rows + tile - 1) / tile;
-  a.tiles_n = (n_out + tile - 1) / tile;
+  const int bm = plan.tile == kBig ? 256 : plan.tile == kDirect64 ? 64 : 128, bn = plan.tile == kBig ? 256 : 128;
+  a.tiles_m = (n_rows + bm - 1) / bm;
+  a.tiles_n = (n_out + bn - 1) / bn;
   const long long blocks = (long long)a.tiles_m * a.tiles_n;
   SB_SUPPORT(blocks <= 0x7fffffffLL, "sb_gemm_mfma_partial_bf16: too many tiles");
   const unsigned long long w_rows = (unsigned long long)((n_out + 15) / 16 * 16);
@@ -973,8 +1238,11 @@ extern "C" int sb_gemm_mfma_partial_bf16(float *partial, const void *x, const vo
   a.partial = partial;
   a.vec4 = n_out % 4 == 0 && reinterpret_cast<uintptr_t>(partial) % 16 == 0;
   a.stages_per_slice = (n_k + slices - 1) / slices;
-  const int rc = plan.big ? launch_direct_one<8, 4, 64, 2, 0, false>(a, blocks, 0, (hipStream_t)stream)
-                          : launch<2, 2, 64, 2, true>(a, blocks, packed, (hipStream_t)stream);
+  hipStream_t st = (hipStream_t)stream;
+  const int rc = plan.tile == kBig         ? launch_pipe_one<0, false>(a, blocks, st)
+                 : plan.tile == kDirect128 ? launch_direct_one<4, 2, 64, 4, 0, false>(a, blocks, 0, st)
+                 : plan.tile == kDirect64  ? launch_direct_one<2, 2, 64, 4, 0, false>(a, blocks, 0, st)
+                                           : launch<2, 2, 64, 2, true>(a, blocks, packed, st);
   if (rc != SB_OK) return rc;
   return sb::check_launch("sb_gemm_mfma_partial_bf16");
 }

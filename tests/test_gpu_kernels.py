@@ -265,6 +265,57 @@ def test_gemm_bf16_every_path(shape, path, t, n, k):
             close(got, want, atol=1e-4 * math.sqrt(k), rtol=1e-4, what=f"gated {act} shape {shape} {path}")
 
 
+@pytest.mark.parametrize("t, n, k", [(65, 100, 64), (183, 226, 192), (288, 264, 128), (300, 1001, 448), (65, 72, 2368)])
+@pytest.mark.parametrize("big", [False, True])
+def test_gemm_bf16_tiles_of_64_rows(t, n, k, big):
+    """Straight into LDS in one round over the CUs (four stages in flight) and in more (two): rows, columns and
+    stage counts that end inside a tile or a round of the buffers."""
+    from sonicboom_amd import ops
+    t, n = (t * 9, n * 9) if big else (t, n)
+    x, w = randn(t, k, dtype=BF16), randn(n, k, dtype=BF16, scale=0.05)
+    wd, inner = w.to(DEV), n // 2
+    want = ref_gemm(x, w, None, None)
+    for shape in (5, 0):
+        with ops.gemm_tile_shape(shape, "direct"):
+            got = ops.gemm_bf16(x.to(DEV), ops.pack_weight(wd), None, None, F32, packed_shape=(n, k))
+            close(got, want, atol=3e-5 * math.sqrt(k), rtol=1e-5, what=f"shape {shape}")
+            g, u = want[:, :inner].double(), want[:, inner:2 * inner].double()
+            got = ops.gemm_bf16(x.to(DEV), ops.pack_weight(wd[:2 * inner].contiguous(), True), None, None, F32,
+                                gated=True, packed_shape=(2 * inner, k))
+            close(got, g / (1.0 + torch.exp(-g)) * u, atol=1e-4 * math.sqrt(k), rtol=1e-4, what=f"gated shape {shape}")
+
+
+@pytest.mark.parametrize("t, n, k", [(65, 896, 896), (183, 1536, 8960), (288, 900, 4864), (183, 3584, 1280), (512, 1100, 640),
+                                     (1500, 3584, 4096), (100, 64, 192)])
+def test_gemm_bf16_k_slices_of_tiled_products(t, n, k):
+    """The raw product in K slices, at sizes that take each of its tiles."""
+    from sonicboom_amd import ops
+    x, w = randn(t, k, dtype=BF16), randn(n, k, dtype=BF16, scale=0.05)
+    part = ops.gemm_bf16_partial(x.to(DEV), ops.pack_weight(w.to(DEV)), packed_shape=(n, k))
+    got = part.sum(0) if part is not None else ops.gemm_bf16(x.to(DEV), ops.pack_weight(w.to(DEV)), None, None, F32, packed_shape=(n, k))
+    close(got, ref_gemm(x, w, None, None), atol=3e-5 * math.sqrt(k), rtol=1e-5, what="slices")
+
+
+def test_silu_of_the_tiled_product_over_its_range():
+    """A product that hands the gate its numbers as they are, over the float32 range: against 64-bit arithmetic to
+    two units of the last of 24 bits, and where e^-g runs out of the range to what is as good as zero."""
+    from sonicboom_amd import ops
+    g = torch.cat([torch.linspace(-120, 120, 4001), torch.logspace(-30, 38, 400), -torch.logspace(-30, 38, 400),
+                   torch.zeros(1)]).to(BF16)
+    x = torch.zeros(g.numel(), 32, dtype=BF16)
+    x[:, 0] = g
+    x[:, 1] = 1.0
+    w = torch.zeros(2, 32, dtype=BF16)
+    w[0, 0] = 1.0
+    w[1, 1] = 1.0
+    got = ops.gemm_bf16(x.to(DEV), ops.pack_weight(w.to(DEV), True), None, None, F32, gated=True, packed_shape=(2, 32)).cpu()[:, 0].double()
+    z = x[:, 0].double()
+    want = z / (1.0 + torch.exp(-z))
+    ok = z > -80.0
+    assert ((got - want).abs()[ok] <= 2.5e-7 * want.abs()[ok]).all()
+    assert (got[~ok].abs() <= 1e-30).all()
+
+
 def test_gemm_bf16_blocks_that_go_from_tile_to_tile():
     """More 256 x 256 tiles than the GPU has CUs: the blocks of the kernel that loads straight into
     LDS go on to a second tile, whose first stage the first tile's last stage has loaded; in
