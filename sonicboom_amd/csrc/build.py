@@ -42,6 +42,7 @@ CORE_SOURCES = [
     "random_fill.hip", "recurrent.hip", "attention_latent.hip", "attention_latent_mfma.hip",
     "outnorm.hip", "headnorm_kv.hip", "moe.hip", "moe_mfma.hip", "timeconv.hip", "state_space.hip",
     "attention_mixed.hip", "join.hip", "decay_scan.hip", "decay_chunks.hip", "streams.hip", "rownorm.hip", "gated_lru.hip",
+    "dense_layers.hip",
 ]
 HEADERS = ["common.h", "sb_hip.h", "mfma.h"]
 ATTN_SOURCES = ["attention_mfma.hip"]

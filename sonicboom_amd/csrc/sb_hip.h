@@ -645,6 +645,37 @@ int sb_gated_lru(void *out, int out_dtype, const float *x, const float *y, int r
                  const int32_t *row_pos, const int32_t *row_seq, const int32_t *cu_rows, const int32_t *slots, int n_rows, int n_seqs,
                  int width, int block, float *ab, const int32_t *chunks, int n_chunks, float *folded, void *stream);
 
+/* The kernel that a whole bf16 product of these sizes takes: 0 the weight-streaming one whose waves split the output
+ * features, 1 the one whose waves split K, 2 the tiled one. */
+int sb_gemm_bf16_kernel(int n_rows, int n_out, int gated, int packed);
+
+/* A run of like decoder layers (pre-norm; grouped-query attention with rotation and biases on q, k, v; gated dense
+ * feed-forward; packed bf16 weights) over the rows of a step, in one call: the launches that the layers' parts make.
+ * x += attention(h); h = rmsnorm(x) * norm_w; x += down(gate_up(h)); h = rmsnorm(x) * next_w (NULL: left undefined). */
+typedef struct sb_dense_layer {
+  const void *qkv_w, *out_w, *gate_up_w, *down_w;
+  const float *qkv_bias;                    /* or NULL */
+  const void *norm_w, *next_w;
+  const float *inv_freq, *freq_factors;     /* as sb_rope_kv_store */
+  void *k_cache, *v_cache;                  /* bf16 */
+  float norm_eps, next_eps, scale;
+  int norm_dtype, next_dtype, rot_dims, window, gate;      /* gate: an sb_gate */
+} sb_dense_layer;
+typedef struct sb_dense_step {
+  float *x;                                 /* [n_rows][width], in place */
+  void *h, *q, *att, *mid;                  /* bf16 [n_rows][width], [.][heads_q * head_dim] twice, [.][inner]; h: the first norm of x */
+  float *part;                              /* sb_dense_layers_floats(...) */
+  size_t part_floats;
+  int (*attention)(void *, const void *, const void *, const void *, const int32_t *, int, int, const int32_t *, const int32_t *, int,
+                   int, int, float, int, int, void *);            /* sb_attn_prefill_bf16 of the head size's library */
+  const char *(*attention_error)(void);
+  const int32_t *row_pos, *row_seq, *page_table, *tiles;
+  int n_rows, width, inner, heads_q, heads_kv, head_dim, max_pages, n_pages, n_tiles, tile_rows;
+} sb_dense_step;
+int sb_reduce_resid_norm_max_width(void);
+size_t sb_dense_layers_floats(int n_rows, int width, int qkv_width, int q_width, int inner);
+int sb_dense_layers(const sb_dense_step *step, const sb_dense_layer *layers, int n_layers, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

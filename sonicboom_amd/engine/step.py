@@ -17,6 +17,7 @@ import numpy as np
 import torch
 
 from ..cache.paged import CacheError, PagedCache
+from . import dense
 from .model import DecoderModel
 
 
@@ -197,6 +198,8 @@ class Engine:
         self.bindings = model.bindings(self.cache)
         self.use_graphs = True
         self._loop = None
+        # a model that is a run of like dense layers launches all of a short prompt step's layers in one call
+        self.one_call_layers = True
         # set to a callable (name, tensor) to receive a step's named intermediates, in the order of
         # the computation: "embedding", "entry<i>.after_mixer", "entry<i>.after_ffn", "logits"
         self.tracer = None
@@ -314,6 +317,11 @@ class Engine:
         x = model.embedding.forward(ctx.ids, ctx)
         if tracer is not None:
             tracer("embedding", x)
+        if tracer is None and self.one_call_layers and dense.takes_step(ctx):
+            run = dense.DenseLayers.of(model, self.bindings)
+            if run is not None:
+                run(x, ctx)
+                return self._finish(x, ctx)
         h = None
         for junction in model.junctions:
             h = junction.begin(x, ctx)
@@ -330,6 +338,11 @@ class Engine:
             ctx.trace = (lambda what, t, _i=i: tracer(f"entry{_i}.{what}", t)) if tracer is not None else None
             h = model.blocks[e.block].forward(x, ctx, self.bindings[i], h=h, next_norm=next_norm)
         ctx.trace = None
+        return self._finish(x, ctx)
+
+    def _finish(self, x: torch.Tensor, ctx) -> torch.Tensor:
+        """The final norm and the head on the wanted rows of the stream."""
+        model, tracer = self.model, self.tracer
         ctx.shared = None
         if ctx.n_wanted == 0:
             return torch.empty((0, model.vocab), dtype=torch.float32, device=self.device)

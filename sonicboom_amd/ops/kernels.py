@@ -636,6 +636,59 @@ def reduce_resid_norm(partial: torch.Tensor, bias: Optional[torch.Tensor], x: to
     return y
 
 
+class DenseLayer(ctypes.Structure):
+    """sb_dense_layer of the kernel library."""
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("qkv_w", "out_w", "gate_up_w", "down_w", "qkv_bias", "norm_w", "next_w", "inv_freq",
+                                                "freq_factors", "k_cache", "v_cache")]
+                + [(n, ctypes.c_float) for n in ("norm_eps", "next_eps", "scale")]
+                + [(n, ctypes.c_int) for n in ("norm_dtype", "next_dtype", "rot_dims", "window", "gate")])
+
+
+class _DenseStep(ctypes.Structure):
+    """sb_dense_step of the kernel library."""
+    _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "h", "q", "att", "mid", "part")] + [("part_floats", ctypes.c_size_t)]
+                + [(n, ctypes.c_void_p) for n in ("attention", "attention_error", "row_pos", "row_seq", "page_table", "tiles")]
+                + [(n, ctypes.c_int) for n in ("n_rows", "width", "inner", "heads_q", "heads_kv", "head_dim", "max_pages", "n_pages",
+                                               "n_tiles", "tile_rows")])
+
+
+def dense_layers(x: torch.Tensor, h: torch.Tensor, layers, inner: int, heads_q: int, heads_kv: int, head_dim: int,
+                 page_table: torch.Tensor, n_pages: int, row_pos: torch.Tensor, row_seq: torch.Tensor, tiles: torch.Tensor,
+                 tile_rows: int) -> None:
+    """Decoder layers (a ctypes array of :class:`DenseLayer`) over a step's rows in one call of the library: ``x`` float32
+    [rows, width] in place, ``h`` bfloat16 the first layer's norm of it (overwritten)."""
+    _dev(x, h, page_table, row_pos, row_seq, tiles)
+    t, width = x.shape
+    if x.dtype != torch.float32 or h.dtype != torch.bfloat16 or tuple(h.shape) != (t, width):
+        raise KernelLibraryError("dense_layers takes the float32 stream and its first norm in bfloat16")
+    _check_rows(row_pos, row_seq, page_table, t)
+    if tiles.dtype != torch.int32 or tiles.dim() != 2 or tiles.shape[1] != 4:
+        raise KernelLibraryError("tiles must be int32 [n, 4]")
+    lib, attn = library.core(), library.attention_library(head_dim)
+    q_width = heads_q * head_dim
+    floats = lib.sb_dense_layers_floats(t, width, q_width + 2 * heads_kv * head_dim, q_width, inner)
+    # one allocation for what the layers hand from kernel to kernel, each part on 256 bytes
+    sizes = [4 * floats, 2 * t * q_width, 2 * t * q_width, 2 * t * inner]
+    offsets = [0]
+    for n in sizes:
+        offsets.append(offsets[-1] + (n + 255) // 256 * 256)
+    work = torch.empty((offsets[-1],), dtype=torch.uint8, device=x.device)
+    base = work.data_ptr()
+    step = _DenseStep(x=x.data_ptr(), h=h.data_ptr(), part=base, part_floats=floats, q=base + offsets[1], att=base + offsets[2],
+                      mid=base + offsets[3],
+                      attention=ctypes.cast(attn.sb_attn_prefill_bf16, ctypes.c_void_p),
+                      attention_error=ctypes.cast(attn.sb_attn_last_error, ctypes.c_void_p),
+                      row_pos=row_pos.data_ptr(), row_seq=row_seq.data_ptr(), page_table=page_table.data_ptr(), tiles=tiles.data_ptr(),
+                      n_rows=t, width=width, inner=inner, heads_q=heads_q, heads_kv=heads_kv, head_dim=head_dim,
+                      max_pages=page_table.shape[1], n_pages=n_pages, n_tiles=tiles.shape[0], tile_rows=int(tile_rows))
+    check(lib.sb_dense_layers(ctypes.addressof(step), ctypes.addressof(layers), len(layers), _stream()))
+
+
+def launchers_choose() -> bool:
+    """Whether this thread imposes no choice on the launchers (see :class:`_Hints`)."""
+    return _hints.few_rows_kernel is None and not _hints.stream and _hints.tile_shape < 0 and not _hints.decode_pages
+
+
 def reduce_resid_norm_ok(width: int, scale: float = 1.0, groups: int = 1) -> bool:
     if scale != 1.0 or groups != 1:
         return groups >= 1 and width % groups == 0       # the kernel for scaled sums and grouped norms: any width
@@ -692,21 +745,9 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], re
     lib = library.core()
     bdt = _dt(bias) if bias is not None else 0
     packed = 1 if packed_shape is not None else 0
-    # A wide packed matrix (enough 16-row tiles, or gate/up pairs of them, for STREAM_MIN_BLOCKS
-    # blocks of four waves) and up to 128 rows: the kernel whose waves split the output features
-    # and share the rows through LDS.  Other products of up to 64 rows: the kernel whose waves
-    # split K and which can cut K over the grid as well.  The rest: the tiled kernel.
     which = _hints.few_rows_kernel
     if which is None:
-        wave_units = -(-n // 16) if gated else -(-n // 32)
-        which = "stream" if packed and wave_units >= 4 * STREAM_MIN_BLOCKS else "skinny"
-        if t > SKINNY_MAX_ROWS and which == "stream":
-            # 65 to 128 rows: the tiled kernel's 128 x 128 tiles do as well or better unless the
-            # matrix is wide and their count leaves the last round over the 256 CUs nearly empty
-            # (8,960 x 1,536 and 11,008 x 2,048 at 96 rows: 21 and 26 us tiled, 25 and 34 streamed)
-            rounds = -(-n // (64 if gated else 128)) / 256.0
-            if wave_units < 4 * STREAM_MIN_BLOCKS_MORE_ROWS or math.ceil(rounds) / rounds < 1.4:
-                which = "tiled"
+        which = ("stream", "skinny", "tiled")[lib.sb_gemm_bf16_kernel(t, n, gate, packed)]
     if t <= STREAM_MAX_ROWS and which == "stream" and packed:
         check(lib.sb_gemm_stream_bf16(_p(out), _dt(out), _p(x), _p(w), _p(bias), bdt, _p(resid), t, n, k,
                                       gate, _hints.stream, _stream()))
@@ -797,14 +838,6 @@ def gemm_few_rows_kernel(which: Optional[str], waves: int = 0, slices: int = 0):
 
 
 MFMA_MAX_HEAD_DIM = 256
-# Blocks of four waves that a matrix must give the stream kernel.  A block streams its share of W at
-# what one CU pulls, whatever the count of blocks, so fewer blocks than CUs only pay while the
-# other kernel, which spreads K over the whole GPU, has more bytes to move than a block's share
-# takes: gate/up pairs of 8,960 x 1,536 (140 blocks) 13 to 18 us against 18 to 29 at up to 64 rows,
-# 11,008 x 2,048 (172 blocks) 19 to 25 against 25 to 34; 8,192 x 2,048 (128 blocks) 18 against 16,
-# and 4,864 x 896 (76 blocks) 4 % slower in a whole decode step.
-STREAM_MIN_BLOCKS = 136
-STREAM_MIN_BLOCKS_MORE_ROWS = 192        # for 65 to 128 rows
 STREAM_MAX_ROWS = 128
 
 
@@ -977,6 +1010,16 @@ def attention_row_tiles(heads_q: int, heads_kv: int, head_dim: int, dtype=torch.
     return (base,)
 
 
+def attention_tile_height(ctx, heads_q: int, heads_kv: int, row_tile) -> int:
+    """The height of the row tiles that a prompt step's attention takes, of those its mixer has asked for."""
+    heights = (row_tile,) if isinstance(row_tile, int) else tuple(row_tile)
+    if TALL_ROW_TILE in heights[1:]:
+        blocks = ctx.row_tiles(TALL_ROW_TILE).shape[0] * heads_kv * ((heads_q // heads_kv + 7) // 8)
+        if blocks >= TALL_MIN_BLOCKS:
+            return TALL_ROW_TILE
+    return heights[0]
+
+
 def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, page_table: torch.Tensor, ctx,
               heads_q: int, heads_kv: int, head_dim: int, scale: float, window: int,
               fast: bool = True, row_tile=ATTENTION_ROW_TILE) -> torch.Tensor:
@@ -989,12 +1032,7 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pag
         if ctx.is_decode:
             return attention_decode_mfma(q, k_cache, v_cache, page_table, ctx.row_pos, heads_q, heads_kv,
                                          head_dim, scale, window)
-        heights = (row_tile,) if isinstance(row_tile, int) else tuple(row_tile)
-        height = heights[0]
-        if TALL_ROW_TILE in heights[1:]:
-            blocks = ctx.row_tiles(TALL_ROW_TILE).shape[0] * heads_kv * ((heads_q // heads_kv + 7) // 8)
-            if blocks >= TALL_MIN_BLOCKS:
-                height = TALL_ROW_TILE
+        height = attention_tile_height(ctx, heads_q, heads_kv, row_tile)
         return attention_prefill_mfma(q, k_cache, v_cache, page_table, ctx.row_pos, ctx.row_tiles(height),
                                       heads_q, heads_kv, head_dim, scale, window, tile_rows=height)
     return attention_plain(q, k_cache, v_cache, page_table, ctx.row_pos, ctx.row_seq, heads_q, heads_kv,

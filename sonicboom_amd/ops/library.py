@@ -23,6 +23,8 @@ _CORE_SIGNATURES = {
     "sb_rmsnorm": [_P, _I, _P, _P, _I, _P, _I, _I, _F, _P],
     "sb_gemm": [_P, _I, _P, _I, _P, _I, _P, _I, _P, _I, _I, _I, _P],
     "sb_gemm_f32_packed": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
+    "sb_gemm_bf16_kernel": [_I, _I, _I, _I],
+    "sb_dense_layers": [_P, _P, _I, _P],
     "sb_silu_mul": [_P, _I, _P, _I, _I, _I, _P],
     "sb_gate_mul": [_P, _I, _P, _I, _I, _I, _I, _P],
     "sb_add_into": [_P, _P, _I, _Z, _P],
@@ -210,6 +212,8 @@ def core():
                 _declare(lib, _OPTIONAL_SIGNATURES, optional=True)
                 lib.sb_gemm_skinny_scratch.argtypes = [_I, _I, _I, _I]
                 lib.sb_gemm_skinny_scratch.restype = c_size_t
+                lib.sb_dense_layers_floats.argtypes = [_I, _I, _I, _I, _I]
+                lib.sb_dense_layers_floats.restype = c_size_t
                 lib.sb_top_candidates_scratch.argtypes = [_I, _I]
                 lib.sb_top_candidates_scratch.restype = c_size_t
                 lib.sb_read_probe.argtypes = [_P, _P, _Z, _I, _P]

@@ -1,0 +1,56 @@
+"""Prompt steps whose layers are launched by one call give the bits of the same steps launched part by part."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def config(width, heads, kv, inner, vocab=500, layers=3, tied=True):
+    return {"architectures": ["Qwen2ForCausalLM"], "num_hidden_layers": layers, "hidden_size": width, "num_attention_heads": heads,
+            "num_key_value_heads": kv, "intermediate_size": inner, "vocab_size": vocab, "rope_theta": 10000.0, "rms_norm_eps": 1e-6,
+            "max_position_embeddings": 4096, "tie_word_embeddings": tied}
+
+
+# (sizes whose products go to every kernel; head sizes with tiles of 16, 32 and 64 rows; widths off the stages' 64)
+SIZES = [config(128, 2, 2, 320), config(896, 14, 2, 4864), config(256, 4, 1, 712), config(2048, 16, 2, 11008, layers=2), config(160, 10, 2, 96)]
+STEPS = [[1, 3], [64], [65], [7, 1, 200, 33], [129], [700, 500], [1536], [1537]]
+
+
+@pytest.mark.parametrize("cfg", SIZES, ids=lambda c: f"{c['hidden_size']}")
+def test_one_call_gives_the_same_bits(cfg):
+    from sonicboom_amd.engine import DecoderModel, Engine, StepEntry
+    model = DecoderModel.from_random(cfg, 3, "bfloat16", "cuda:0")
+    engines = [Engine(model, 64 * 80, max_slots=4) for _ in range(2)]
+    engines[1].one_call_layers = False
+    rng = np.random.default_rng(5)
+    for lengths in STEPS:
+        slots = [[e.alloc_slot() for _ in lengths] for e in engines]
+        for more in (lengths, [5 for _ in lengths], [1 for _ in lengths]):       # a prompt, a continuation, a token each
+            tokens = [rng.integers(0, cfg["vocab_size"], size=n).tolist() for n in more]
+            got, want = (e.step([StepEntry(s, t, (0, len(t) - 1)) for s, t in zip(ss, tokens)]) for e, ss in zip(engines, slots))
+            assert torch.equal(got, want), (lengths, more)
+        for e, ss in zip(engines, slots):
+            for s in ss:
+                e.free_slot(s)
+    from sonicboom_amd.engine.dense import DenseLayers
+    assert DenseLayers.of(model, engines[0].bindings) is not None
+
+
+def test_other_models_and_choices_keep_their_parts():
+    from sonicboom_amd import ops
+    from sonicboom_amd.engine import DecoderModel, Engine, StepEntry
+    from sonicboom_amd.engine.dense import DenseLayers
+    model = DecoderModel.from_random(SIZES[0], 3, "float32", "cuda:0")
+    e = Engine(model, 64 * 4)
+    assert DenseLayers.of(model, e.bindings) is None
+    model = DecoderModel.from_random(SIZES[0], 3, "bfloat16", "cuda:0")
+    e = Engine(model, 64 * 4)
+    seen = []
+    e.tracer = lambda name, t: seen.append(name)
+    s = e.alloc_slot()
+    e.step([StepEntry(s, [1, 2, 3], (2,))])
+    assert "entry2.after_ffn" in seen
+    with ops.gemm_tile_shape(0):
+        assert not ops.launchers_choose()
+    assert ops.launchers_choose()
