@@ -937,6 +937,98 @@ attn_prefill_tall_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ q,
 }
 
 // ---------------------------------------------------------------------------------------------
+// Prefill with few rows against many keys: a block takes sixteen rows of ONE query head, and its eight waves take the
+// pages in turn (wave w the pages first + w, first + w + 8, ..), straight from the cache; their sums meet in LDS.  What
+// bounds such a step in the form above is the chain of pages that a block walks, some 1.8 us a page with a block a CU or less;
+// here a block reads its pages alone and holds eight of them in flight, some 0.5 us a page (head size 128) or 0.2 (64), the
+// rate at which a CU gets them.  Measured, that form -> this one (us):
+//   12 heads on 2, size 128: 288 rows 13.2 -> 7.0; 183 rows of three sequences on 461 to 961 keys 27.7 -> 13.4;
+//   256 rows on 4,256 keys 88 -> 36; 16 rows on 16,000 keys 311 -> 124.  14 on 2, size 64: 10.3 -> 5.8, 21.0 -> 7.5, 68 -> 20,
+//   238 -> 52.  4 on 4, size 64 (tiles of 64 rows): 8.4 -> 5.2, 19.1 -> 7.3, 78 -> 18, 258 -> 64.
+constexpr bool kKeysOk = HD <= 128;      // (beyond, a page's fragments no longer fit the registers at once)
+constexpr int kKeyWaves = 8;
+constexpr int kKeyStride = HD + 4;       // floats of a column's sums in LDS: lanes of a store four banks apart
+constexpr int kKeyLds = (kKeyWaves * 16 * kKeyStride + kKeyWaves * 32) * 4;
+
+template <bool OK>
+__global__ void __launch_bounds__(64 * kKeyWaves, 2)
+attn_prefill_keys_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k_cache,
+                         const bf16_t *__restrict__ v_cache, const int32_t *__restrict__ page_table, int max_pages,
+                         int n_pages_total, const int32_t *__restrict__ row_pos, const int32_t *__restrict__ tiles,
+                         int n_tiles, int heads_q, int heads_kv, int row_groups, float scale_log2, int window) {
+  if constexpr (OK) {
+    extern __shared__ uint4 lds_pages[];
+    float *lds_o = reinterpret_cast<float *>(lds_pages);             // [wave][column][kKeyStride]
+    float *lds_m = lds_o + kKeyWaves * 16 * kKeyStride, *lds_l = lds_m + kKeyWaves * 16;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, g = lane >> 4;
+    // The heads of a group read the same pages: they get block numbers eight apart, which one die runs.
+    const int group = heads_q / heads_kv;
+    const int xcd = int(blockIdx.x) & 7, j = int(blockIdx.x) >> 3;
+    const int unit = xcd + 8 * (j / group), hg = j % group;
+    const int per_tile = heads_kv * row_groups;
+    if (unit >= n_tiles * per_tile) return;
+    const int tile = n_tiles - 1 - unit / per_tile, rem = unit % per_tile;
+    const int kvh = rem % heads_kv, rg = rem / heads_kv;
+    const int head = kvh * group + hg;
+    const int n_rows = min(tiles[tile * 4 + 1] - 16 * rg, 16), seq = tiles[tile * 4 + 2];
+    if (n_rows <= 0) return;
+    const int row0 = tiles[tile * 4] + 16 * rg;
+    const bool col_ok = r < n_rows;
+    const int row = row0 + (col_ok ? r : 0);
+    const int pos = row_pos[row];
+    const int col_pos = col_ok ? pos : -1;
+    const int col_lo = (window > 0 && pos >= window) ? pos - window + 1 : 0;
+    const int pos_first = row_pos[row0], key_hi = row_pos[row0 + n_rows - 1];
+    const int key_lo = (window > 0 && pos_first >= window) ? pos_first - window + 1 : 0;
+    bf16x8_t qf[1][KS];
+    load_q(qf[0], q + (size_t(row) * heads_q + head) * HD, col_ok, lane);
+    WaveState<1> st;
+    init_state<1>(st);
+    const int32_t *pt = page_table + size_t(seq) * max_pages;
+    const int pg_hi = min(key_hi / SB_PAGE, max_pages - 1);
+    for (int pg = key_lo / SB_PAGE + wave; pg <= pg_hi; pg += kKeyWaves) {
+      const int page = pt[pg];
+      if (page < 0 || page >= n_pages_total) continue;
+      const size_t off = (size_t(page) * heads_kv + kvh) * SB_PAGE * HD;
+      attend_page<1>(st, qf, k_cache + off, v_cache + off, pg * SB_PAGE, col_pos, col_lo, key_lo, key_hi, scale_log2, lane);
+    }
+    float l = st.l[0];
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+      *reinterpret_cast<floatx4_t *>(lds_o + (wave * 16 + r) * kKeyStride + dt * 16 + 4 * g) = st.o[0][dt];
+    if (g == 0) {
+      lds_m[wave * 16 + r] = st.m[0];
+      lds_l[wave * 16 + r] = l;
+    }
+    __syncthreads();
+    // four neighbouring elements of a column a thread, the waves in ascending order
+    for (int e = threadIdx.x; e < 16 * (HD / 4); e += 64 * kKeyWaves) {
+      const int c = e / (HD / 4), d = (e % (HD / 4)) * 4;
+      if (c >= n_rows) continue;
+      float m = -__builtin_inff();
+#pragma unroll
+      for (int w = 0; w < kKeyWaves; ++w) m = fmaxf(m, lds_m[w * 16 + c]);
+      const float m_use = m == -__builtin_inff() ? 0.f : m;
+      floatx4_t o = floatx4_t{0.f, 0.f, 0.f, 0.f};
+      float sum = 0.f;
+#pragma unroll
+      for (int w = 0; w < kKeyWaves; ++w) {
+        const float f = __builtin_amdgcn_exp2f(lds_m[w * 16 + c] - m_use);
+        const floatx4_t ow = *reinterpret_cast<const floatx4_t *>(lds_o + (w * 16 + c) * kKeyStride + d);
+        o[0] += ow[0] * f; o[1] += ow[1] * f; o[2] += ow[2] * f; o[3] += ow[3] * f;
+        sum += lds_l[w * 16 + c] * f;
+      }
+      const float inv = sum > 0.f ? 1.f / sum : 0.f;
+      *reinterpret_cast<uint2 *>(out + (size_t(row0 + c) * heads_q + head) * HD + d) =
+          make_uint2(pack_bf16(o[0] * inv, o[1] * inv), pack_bf16(o[2] * inv, o[3] * inv));
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------------------------
 // Decode: one row per sequence.  Block (chunk, kv head x head tile, sequence); wave w of the
 // block takes page 4 * chunk + w; columns are the query heads of the kv head.
 //
@@ -1832,10 +1924,11 @@ extern "C" int sb_attn_prefill_tile_rows(int heads_q, int heads_kv) {
 // q, out: bf16 [n_rows, heads_q * HD]; tiles int32 [n_tiles][4] = (first row, rows <= tile_rows,
 // sequence, 0), every tile inside one sequence and its rows at consecutive positions.  tile_rows:
 // 16, or what sb_attn_prefill_tile_rows gives for these heads.
+// form: 0, or a test's or a measurement's choice: 1 pages through the block one by one, 2 pages over the block's waves.
 extern "C" int sb_attn_prefill_bf16(void *out, const void *q, const void *k_cache, const void *v_cache,
                                     const int32_t *page_table, int max_pages, int n_pages_total,
                                     const int32_t *row_pos, const int32_t *tiles, int n_tiles, int heads_q,
-                                    int heads_kv, float scale, int window, int tile_rows, void *stream) {
+                                    int heads_kv, float scale, int window, int tile_rows, int form, void *stream) {
   int rc = check_common(out, q, k_cache, v_cache, page_table, row_pos, max_pages, n_pages_total, heads_q,
                         heads_kv, window, "sb_attn_prefill_bf16");
   if (rc != SB_OK) return rc;
@@ -1854,7 +1947,32 @@ extern "C" int sb_attn_prefill_bf16(void *out, const void *q, const void *k_cach
   if (nc > nc_max) nc = nc_max;
   const int head_tiles = (group + nc - 1) / nc;
   const int y_per_kv = (head_tiles + waves - 1) / waves;
-  if (tile_rows == 32 && sb_attn_prefill_tall_ok(heads_q, heads_kv)) {
+  const bool tall = tile_rows == 32 && sb_attn_prefill_tall_ok(heads_q, heads_kv);
+  SB_REQUIRE(tall || tile_rows == 16 || tile_rows == sb_attn_prefill_tile_rows(heads_q, heads_kv),
+             "sb_attn_prefill_bf16: tiles of %d rows do not suit %d heads on %d kv heads", tile_rows, heads_q, heads_kv);
+  if constexpr (kKeysOk) {
+    const long long units = (long long)n_tiles * (tile_rows / 16) * heads_kv;
+    const long long blocks = (units + 7) / 8 * 8 * group;
+    // Every head reads the pages for itself here, which pays while the blocks come in a round or two.  Two rounds at head
+    // sizes above 64: up to 512 blocks it is ahead or level (504: 14.2 -> 11.0 us; 24 sequences of 16 rows on 2,000 keys, 384
+    // blocks: 56.5 -> 55.1), at 560 behind (9.8 -> 12.0) or, with eight heads a kv head, still ahead (1,024: 32.3 -> 31.3).
+    // Up to 64 a page is half as long: 896 blocks 21.0 -> 13.8, 1,792 37.3 -> 34.4.
+    if (form == 2 || (form == 0 && blocks <= (HD <= 64 ? 1024 : 512))) {
+      SB_SUPPORT(blocks <= 0x7fffffffLL, "sb_attn_prefill_bf16: too many blocks");
+      static bool raised_keys = false;
+      if (kKeyLds > 48 * 1024 && !raised_keys) {
+        const hipError_t e = hipFuncSetAttribute((const void *)attn_prefill_keys_kernel<kKeysOk>,
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, kKeyLds);
+        SB_REQUIRE(e == hipSuccess, "sb_attn_prefill_bf16: cannot reserve %d bytes of LDS: %s", kKeyLds, hipGetErrorString(e));
+        raised_keys = true;
+      }
+      attn_prefill_keys_kernel<kKeysOk><<<dim3(unsigned(blocks)), 64 * kKeyWaves, kKeyLds, s>>>(
+          (bf16_t *)out, (const bf16_t *)q, (const bf16_t *)k_cache, (const bf16_t *)v_cache, page_table, max_pages,
+          n_pages_total, row_pos, tiles, n_tiles, heads_q, heads_kv, tile_rows / 16, scale * kLog2e, window);
+      return sb::check_launch("sb_attn_prefill_bf16");
+    }
+  }
+  if (tall) {
     const int y_tall = (group + 7) / 8;
     SB_SUPPORT((long long)n_tiles * heads_kv * y_tall <= 0x7fffffffLL, "sb_attn_prefill_bf16: too many blocks");
     constexpr int lds_tall = 2 * 2 * kPageChunks * 16;
@@ -1871,8 +1989,6 @@ extern "C" int sb_attn_prefill_bf16(void *out, const void *q, const void *k_cach
         n_pages_total, row_pos, tiles, n_tiles, heads_q, heads_kv, y_tall, scale * kLog2e, window);
     return sb::check_launch("sb_attn_prefill_bf16");
   }
-  SB_REQUIRE(tile_rows == 16 || tile_rows == sb_attn_prefill_tile_rows(heads_q, heads_kv),
-             "sb_attn_prefill_bf16: tiles of %d rows do not suit %d heads on %d kv heads", tile_rows, heads_q, heads_kv);
   const int row_groups = tile_rows / 16;       // more than one: waves == 4, nc == 1, head_tiles * row_groups == 4
   SB_SUPPORT((long long)n_tiles * heads_kv * y_per_kv <= 0x7fffffffLL, "sb_attn_prefill_bf16: too many blocks");
   dim3 grid(unsigned(n_tiles) * unsigned(heads_kv * y_per_kv));

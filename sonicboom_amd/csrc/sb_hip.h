@@ -667,7 +667,7 @@ typedef struct sb_dense_step {
   float *part;                              /* sb_dense_layers_floats(...) */
   size_t part_floats;
   int (*attention)(void *, const void *, const void *, const void *, const int32_t *, int, int, const int32_t *, const int32_t *, int,
-                   int, int, float, int, int, void *);            /* sb_attn_prefill_bf16 of the head size's library */
+                   int, int, float, int, int, int, void *);       /* sb_attn_prefill_bf16 of the head size's library */
   const char *(*attention_error)(void);
   const int32_t *row_pos, *row_seq, *page_table, *tiles;
   int n_rows, width, inner, heads_q, heads_kv, head_dim, max_pages, n_pages, n_tiles, tile_rows;

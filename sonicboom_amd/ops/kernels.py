@@ -29,6 +29,7 @@ class _Hints(threading.local):
     stream = 0                  # waves | slices << 8 of the weight-streaming product
     tile_shape = -1             # of the tiled product
     decode_pages = 0            # pages per wave of decode attention
+    prefill_form = 0            # of prefill attention
 
 
 _hints = _Hints()
@@ -686,7 +687,8 @@ def dense_layers(x: torch.Tensor, h: torch.Tensor, layers, inner: int, heads_q: 
 
 def launchers_choose() -> bool:
     """Whether this thread imposes no choice on the launchers (see :class:`_Hints`)."""
-    return _hints.few_rows_kernel is None and not _hints.stream and _hints.tile_shape < 0 and not _hints.decode_pages
+    return _hints.few_rows_kernel is None and not _hints.stream and _hints.tile_shape < 0 and not _hints.decode_pages \
+        and not _hints.prefill_form
 
 
 def reduce_resid_norm_ok(width: int, scale: float = 1.0, groups: int = 1) -> bool:
@@ -968,8 +970,21 @@ def attention_prefill_mfma(q, k_cache, v_cache, page_table, row_pos, tiles, head
     out = torch.empty_like(q)
     check(lib.sb_attn_prefill_bf16(_p(out), _p(q), _p(k_cache), _p(v_cache), _p(page_table), page_table.shape[1],
                                    k_cache.shape[0], _p(row_pos), _p(tiles), tiles.shape[0], heads_q, heads_kv,
-                                   float(scale), int(window), int(tile_rows), _stream()), lib, "sb_attn_last_error")
+                                   float(scale), int(window), int(tile_rows), _hints.prefill_form, _stream()), lib,
+          "sb_attn_last_error")
     return out
+
+
+@contextlib.contextmanager
+def attention_prefill_form(form: int):
+    """For tests and measurements: inside the block this thread's prefill attention walks a tile's pages one by one
+    (1) or cuts them over a block's waves (2, head sizes up to 128) instead of choosing from the sizes; 0: its choice."""
+    before = _hints.prefill_form
+    _hints.prefill_form = int(form)
+    try:
+        yield
+    finally:
+        _hints.prefill_form = before
 
 
 # rows of one sequence that a block of the prefill attention kernels takes together; a mixer that

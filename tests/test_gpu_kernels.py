@@ -1047,6 +1047,19 @@ def test_attention_prefill_window_edge(hq, hkv, hd, window):
             close(got, want, atol=2e-2, rtol=1e-2, what=f"window {window}, dominant key {d}, tiles of {height}")
 
 
+@pytest.mark.parametrize("hq, hkv, hd", [(4, 4, 16), (6, 2, 64), (2, 1, 96), (5, 1, 112), (28, 4, 128), (12, 2, 128)])
+@pytest.mark.parametrize("window", [0, 70, 300])
+@pytest.mark.parametrize("form", [1, 2])
+def test_attention_prefill_forms(hq, hkv, hd, window, form):
+    """Pages one by one through a block and pages cut over a block's waves, whichever the sizes would choose: whole
+    prompts and a continuation in tiles of every height, and the edges of a window over more pages than a block has waves."""
+    from sonicboom_amd import ops
+    with ops.attention_prefill_form(form):
+        test_attention_prefill_matrix_cores(hq, hkv, hd, min(window, 70))
+        if window:
+            test_attention_prefill_window_edge(hq, hkv, hd, window)
+
+
 FOLDED_SHAPES = [(4, 2, 16, 16), (3, 1, 32, 32), (5, 5, 48, 16), (6, 2, 80, 64), (28, 4, 128, 128), (16, 1, 64, 0),
                  (2, 1, 256, 256)]
 
