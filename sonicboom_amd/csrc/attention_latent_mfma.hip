@@ -7,16 +7,19 @@
 // lands as four consecutive outputs of one row per lane.
 //
 // sb_latent_attention_bf16: all query heads read the same cached rows [c | r], so a block stages
-// a page of 64 rows once in LDS, twice over: as it lies (a key's numbers consecutive: the A
-// operand of S^T = K Q^T) and with the latent part turned (a number's keys consecutive: the A
-// operand of O^T = C^T P^T), half a page at a time in two buffers that take turns, and its eight
-// waves run four tiles of 16 query columns against it, two waves a tile.
-// In a prompt step a wave's 16 columns are 16 consecutive rows of one head; in a decode step they
-// are 16 heads of the one row.  The next half's rows are asked of memory before the current
-// half's products start, wait in registers and go into the other buffer afterwards.  Softmax runs
-// in the result layout of S^T (a lane holds 8 keys of one column; column maximum and sum over the four lane groups), P goes
+// them once in LDS for 64 query columns.
+// A decode step (a column is a head of the one row): half a page, 32 rows, at a time in two buffers that take turns,
+// twice over: as it lies (a key's numbers consecutive: the A operand of S^T = K Q^T) and with the latent part turned (a
+// number's keys consecutive: the A operand of O^T = C^T P^T).  Its eight waves run four tiles of 16 columns against it,
+// two waves a tile.  The next half's rows are asked of memory before the current half's products start, wait in
+// registers and go into the other buffer afterwards.  Softmax runs in the result layout of S^T (a lane holds 8 keys of
+// one column; column maximum and sum over the four lane groups), P goes
 // back in as the B operand of the second product without leaving registers: the keys of a
 // 32-key step are taken in the order the first product left them, by V's fragment reads.
+// A prompt step (a column is one of up to 16 consecutive rows of a head, four heads a block) has a kernel of its own below:
+// measured against the form above on prompt rows, 16 heads, rows of 512 + 64 (us): 300 rows 66 -> 41, 1,000 223 -> 109,
+// 4,001 1,129 -> 406 (690 TFLOP/s of the products it cannot do without), with a window of 512 327 -> 140; 20 heads of 256 + 32 at 4,001 rows
+// 823 -> 340; 3 heads of 128 + 64 114 -> 64.
 #include "mfma.h"
 
 namespace {
@@ -101,8 +104,8 @@ __global__ void __launch_bounds__(kAttnThreads)
 latent_attention_mfma_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ q, const bf16_t *__restrict__ cache,
                              const int32_t *__restrict__ page_table, int max_pages, int n_pages_total,
                              const int32_t *__restrict__ row_pos, const int32_t *__restrict__ tiles, int heads, int rank,
-                             int rot_dim, float scale, int window, int tile_rows, int n_splits,
-                             float *__restrict__ part_o, float *__restrict__ part_ml, int n_rows) {
+                             int rot_dim, float scale, int window, int n_splits, float *__restrict__ part_o,
+                             float *__restrict__ part_ml, int n_rows) {
   extern __shared__ __align__(16) unsigned char lds[];
   const int latent = rank + rot_dim;
   const int kq = (latent + 31) / 32, nv = (rank + 15) / 16;
@@ -112,22 +115,15 @@ latent_attention_mfma_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict_
   bf16_t *vt_base = ks_base + 2 * ks_size;           // [2][nv * 16][kVtStride]
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int col = lane & 15, g = lane >> 4;
-  // the last tiles of a prompt see the most keys: they go first, so that the short ones fill the end
   const int tile = int(gridDim.x) - 1 - int(blockIdx.x);
-  const int r0 = tiles[4 * tile], n_tile = tiles[4 * tile + 1], seq = tiles[4 * tile + 2];
-  const int heads_per_wave = 16 / tile_rows;
+  const int row = tiles[4 * tile], seq = tiles[4 * tile + 2];
   const int group = wave / kParts, part = wave % kParts;       // the wave's tile of columns, and its share of the latent part
   const int nv_part = (nv + kParts - 1) / kParts;
-  const int head = (blockIdx.y * kColGroups + group) * heads_per_wave + col / tile_rows;
-  const int r = col % tile_rows;
-  const bool wave_works = (blockIdx.y * kColGroups + group) * heads_per_wave < heads;
-  const bool valid = r < n_tile && head < heads;
-  const int row = r0 + min(r, n_tile - 1);
-  const int pos0 = row_pos[r0];
-  const int pos = pos0 + min(r, n_tile - 1);         // a tile's rows are consecutive positions of one sequence
+  const int head = (blockIdx.y * kColGroups + group) * 16 + col;
+  const bool wave_works = (blockIdx.y * kColGroups + group) * 16 < heads;
+  const bool valid = head < heads;
+  const int pos = row_pos[row];
   const int lo = (window > 0 && pos >= window) ? pos - window + 1 : 0;
-  const int lo_blk = (window > 0 && pos0 >= window) ? pos0 - window + 1 : 0;
-  const int hi_blk = pos0 + n_tile - 1;
 
   // the pads that staging never writes must not hold what multiplies to NaN
   for (int i = tid; i < 2 * kHalf * (lk - latent); i += kAttnThreads) {
@@ -137,7 +133,7 @@ latent_attention_mfma_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict_
   for (int b = 0; b < 2; ++b)
     for (int i = tid; i < (nv * 16 - rank) * kVtStride; i += kAttnThreads) vt_base[b * vt_size + rank * kVtStride + i] = 0;
 
-  // this lane's query fragments: column (row, head), k = 32 kk + 8 g .. + 7
+  // this lane's query fragments: column (head), k = 32 kk + 8 g .. + 7
   uint4 qf[KQ];
   const bf16_t *qrow = q + (size_t(row) * heads + min(head, heads - 1)) * latent;
 #pragma unroll
@@ -158,7 +154,7 @@ latent_attention_mfma_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict_
   const int chunks = latent / 8;
   constexpr int kMaxStage = (KQ * 32 / 8 * kHalf + kAttnThreads - 1) / kAttnThreads;
   uint4 set_a[kMaxStage], set_b[kMaxStage];      // two halves on their way from memory to LDS
-  int h_first = lo_blk / kHalf, h_last = hi_blk / kHalf;                // halves count from the sequence's start
+  int h_first = lo / kHalf, h_last = pos / kHalf;                       // halves count from the sequence's start
   if (n_splits > 1) {                                                   // this block's share of them
     const int per = (h_last - h_first + n_splits) / n_splits;
     h_first += int(blockIdx.z) * per;
@@ -343,6 +339,244 @@ latent_attention_mfma_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict_
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Prompt steps: a block takes a tile of up to 16 rows and four heads, 64 query columns, and a page of 64 keys a step.
+// LDS is what bounds it: with 16 columns a wave every 1 KB that a wave reads of it feeds one product.  Here a wave has 32:
+//   scores:  wave (cg, kt, kh) multiplies half kh of the numbers of keys 32 kt .. with the 32 columns of half cg of the
+//            block, and hands half of the partial scores to the wave with the other numbers, whose sums it gets;
+//   sums:    it adds up a quarter of the latent part, all 64 keys, for those 32 columns.
+// The weights pass between the four waves of a half through LDS, relative to a maximum that they share.  Every page
+// lies in LDS once, as it comes (a key's chunks of 16 bytes in an order in which neither reading meets a bank twice,
+// loaded straight into LDS): the second product's operand, numbers by keys, is read with ds_read_b64_tr_b16, which hands a
+// group of 16 lanes a block of four keys by 16 numbers turned.  Two pages take turns in two buffers.
+// (The wave split by numbers, not by keys, keeps the queries in 72 registers instead of 144.  LDS is read through a
+// vector type: reads of a struct type make the compiler wait for the next page's loads before the first of them.)
+typedef short shortx4_t __attribute__((ext_vector_type(4)));
+constexpr int kPageThreads = 512;
+
+// The order of a key's chunks within each run of eight: bits 1, 2 and 3 of the key choose among the eight places, bit 0
+// the half of the banks (a key is an odd number of runs long).  Sixteen keys read at one chunk, and four keys read at
+// four neighbouring ones, all lie in different banks.
+__device__ __forceinline__ int key_turn(int key) { return ((key & 2) << 1) | ((key & 4) >> 1) | ((key & 8) >> 3); }
+
+// What the four waves of a half exchange lies in four regions of 2 KB (one a wave): first the partial scores a wave hands
+// over, all of its region; then the column maxima of the wave that has read them, in its second half; then the weights of
+// columns 8 w .. 8 w + 7 in its first (64 keys of a column, the chunks of eight keys turned by the column).
+constexpr int kRegion = 2048;
+template <int KQ>
+constexpr int latent_pages_lds() { return 2 * SB_PAGE * KQ * 64 + 8 * kRegion; }
+
+template <int KQ, int ND>
+__global__ void __launch_bounds__(kPageThreads, 2)
+latent_attention_pages_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ q, const bf16_t *__restrict__ cache,
+                              const int32_t *__restrict__ page_table, int max_pages, int n_pages_total,
+                              const int32_t *__restrict__ row_pos, const int32_t *__restrict__ tiles, int heads, int rank,
+                              int rot_dim, float scale, int window, int n_splits, float *__restrict__ part_o,
+                              float *__restrict__ part_ml, int n_rows) {
+  typedef __attribute__((address_space(3))) bf16x8_t *lds_ptr_t;
+  typedef __attribute__((address_space(3))) shortx4_t *lds_tr_t;
+  constexpr int CH = 4 * KQ;                          // chunks of a key in LDS (those past the row's end hold zeros)
+  constexpr int kBuf = SB_PAGE * CH;
+  extern __shared__ bf16x8_t lds_latent[];            // [2][SB_PAGE][CH], then the eight regions
+  const int latent = rank + rot_dim;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int cg = wave >> 2, kw = wave & 3, kt = kw & 1, kh = kw >> 1;
+  const int c32 = lane & 31, r16 = lane & 15, h = lane >> 5;
+  unsigned char *regions = reinterpret_cast<unsigned char *>(lds_latent + 2 * kBuf) + cg * 4 * kRegion;
+  // the last tiles of a prompt see the most keys: they go first, so that the short ones fill the end
+  const int tile = int(gridDim.x) - 1 - int(blockIdx.x);
+  const int r0 = tiles[4 * tile], n_tile = tiles[4 * tile + 1], seq = tiles[4 * tile + 2];
+  const int head = blockIdx.y * 4 + cg * 2 + (c32 >> 4);       // this lane's column: a head, and row r16 of the tile
+  const bool valid = r16 < n_tile && head < heads;
+  const int row = r0 + min(r16, n_tile - 1);
+  const int pos0 = row_pos[r0];
+  const int pos = pos0 + min(r16, n_tile - 1);        // a tile's rows are consecutive positions of one sequence
+  const int lo = (window > 0 && pos >= window) ? pos - window + 1 : 0;
+  const int lo_blk = (window > 0 && pos0 >= window) ? pos0 - window + 1 : 0;
+  const int hi_blk = pos0 + n_tile - 1;
+  const int lo_last = (window > 0 && hi_blk >= window) ? hi_blk - window + 1 : 0;      // the first key that every row sees
+
+  bf16x8_t qf[KQ];
+  const bf16_t *qrow = q + (size_t(row) * heads + min(head, heads - 1)) * latent;
+#pragma unroll
+  for (int i = 0; i < KQ; ++i) {
+    const int k = 16 * (kh * KQ + i) + 8 * h;
+    qf[i] = as_bf16x8(ld16(qrow + (k < latent ? k : 0), valid && k < latent));      // latent is a multiple of 8
+  }
+  const float neg_inf = -__builtin_inff();
+  const float scale2 = scale * 1.4426950408889634f;
+  float m_run = neg_inf, l_run = 0.f;
+  floatx16_t o[ND];
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
+
+  int pg_first = lo_blk / SB_PAGE, pg_last = min(hi_blk / SB_PAGE, max_pages - 1);
+  if (n_splits > 1) {
+    const int per = (pg_last - pg_first + n_splits) / n_splits;
+    pg_first += int(blockIdx.z) * per;
+    pg_last = min(pg_last, pg_first + per - 1);
+  }
+  const int32_t *pt = page_table + size_t(seq) * max_pages;
+  auto next_page = [&](int pg) {
+    while (pg <= pg_last) {
+      const int page = pt[pg];
+      if (page >= 0 && page < n_pages_total) break;
+      ++pg;
+    }
+    return pg;
+  };
+  const uint32_t page_bytes = uint32_t(SB_PAGE) * latent * 2;
+  auto bring = [&](int pg, int buf) {
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t *>(cache + size_t(pt[pg]) * SB_PAGE * latent), 0, page_bytes, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < CH / 8; ++i) {
+      const int at = (wave * (CH / 8) + i) * 64;
+      const int slot = at + lane, key = slot / CH, place = slot - key * CH;
+      const int chunk = place ^ key_turn(key);                   // CH is a multiple of 8: the exchange stays in its run
+      const uint32_t off = 8 * chunk < latent ? uint32_t(key * latent + 8 * chunk) * 2 : page_bytes;      // past the end: zeros
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(lds_latent) + buf * kBuf + at, 16, int(off), 0, 0, 0);
+    }
+  };
+  auto met = [&]() {                     // what the waves have written to LDS is there for all of them, what they read is read
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto landed = [&]() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    met();
+  };
+
+  // where this lane reads: a key's chunk 2 (kh KQ + i) + h for the scores, four keys' halves of chunks for the sums (eight
+  // chunks on a key's place repeats, so a few places do for all of them)
+  const int key_s = 32 * kt + c32, key_v = 8 * h + ((lane >> 2) & 3);                 // of the first four of a group's eight keys
+  const int chunk_v = 4 * ND * kw + 2 * ((lane >> 4) & 1) + ((lane >> 1) & 1);
+  int at_s[4], at_v[2][2];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) at_s[p] = key_s * CH + ((2 * (kh * KQ + p) + h) ^ key_turn(key_s));
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+      at_v[t][p] = 2 * ((key_v + 4 * t) * CH + ((chunk_v + 4 * p) ^ key_turn(key_v + 4 * t))) + (lane & 1);
+  float *give = reinterpret_cast<float *>(regions + kw * kRegion) + 4 * lane;
+  float *take = reinterpret_cast<float *>(regions + (kw ^ 2) * kRegion) + 4 * lane;
+  float *max_out = reinterpret_cast<float *>(regions + (kw ^ 2) * kRegion + 1024) + c32;
+  const float *max_in = reinterpret_cast<float *>(regions + 1024) + c32;
+  unsigned char *column = regions + (c32 >> 3) * kRegion + (c32 & 7) * 128;           // this lane's column of weights
+
+  int pg = next_page(pg_first), buf = 0;
+  if (pg <= pg_last) bring(pg, 0);
+  landed();
+  while (pg <= pg_last) {
+    const int pg_next = next_page(pg + 1);
+    if (pg_next <= pg_last) bring(pg_next, buf ^ 1);
+    const bf16x8_t *page = lds_latent + buf * kBuf;
+
+    floatx16_t part;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) part[i] = 0.f;
+#pragma unroll
+    for (int i = 0; i < KQ; ++i) part = mfma32(page[at_s[i & 3] + 8 * (i >> 2)], qf[i], part);
+    // part[i]: half the numbers of key 32 kt + 8 (i / 4) + 4 h + i % 4; of its 16 a lane keeps eight, keys 16 kh .. + 15
+    floatx4_t keep[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const floatx4_t first = {part[4 * u], part[4 * u + 1], part[4 * u + 2], part[4 * u + 3]};
+      const floatx4_t second = {part[8 + 4 * u], part[9 + 4 * u], part[10 + 4 * u], part[11 + 4 * u]};
+      keep[u] = kh ? second : first;
+      *reinterpret_cast<floatx4_t *>(give + 256 * u) = kh ? first : second;
+    }
+    met();
+    float s[8];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const floatx4_t other = *reinterpret_cast<const floatx4_t *>(take + 256 * u);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[4 * u + i] = (keep[u][i] + other[i]) * scale2;
+    }
+    if (!(pg * SB_PAGE + SB_PAGE - 1 <= pos0 && pg * SB_PAGE >= lo_last)) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int j = pg * SB_PAGE + 32 * kt + 16 * kh + 8 * (i >> 2) + 4 * h + (i & 3);
+        s[i] = j >= lo && j <= pos ? s[i] : neg_inf;
+      }
+    }
+    float mx = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    *max_out = mx;                       // both halves of the wave write the same
+    met();
+    mx = fmaxf(fmaxf(max_in[0], max_in[kRegion / 4]), fmaxf(max_in[2 * kRegion / 4], max_in[3 * kRegion / 4]));
+    // the maximum the sums are relative to moves only when a score passes it by kLazy (2^kLazy in the weights, which
+    // float32 sums and bfloat16 weights carry easily); the four waves of a half see the same numbers
+    const bool move = mx > m_run + kLazy;
+    if (__any(move)) {
+      const float alpha = move ? __builtin_amdgcn_exp2f(m_run - mx) : 1.f;      // 0 while nothing has been seen
+      m_run = move ? mx : m_run;
+      l_run *= alpha;
+#pragma unroll
+      for (int d = 0; d < ND; ++d)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
+    }
+    const float m_safe = m_run == neg_inf ? 0.f : m_run;
+    float p[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] = __builtin_amdgcn_exp2f(s[i] - m_safe);
+    l_run += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      *reinterpret_cast<shortx4_t *>(column + (((4 * kt + 2 * kh + u) ^ ((c32 >> 1) & 7)) * 16 + 8 * h)) =
+          __builtin_bit_cast(shortx4_t, make_uint2(pack_bf16(p[4 * u], p[4 * u + 1]), pack_bf16(p[4 * u + 2], p[4 * u + 3])));
+    met();
+#pragma unroll
+    for (int ks = 0; ks < SB_PAGE / 16; ++ks) {
+      const bf16x8_t w = *reinterpret_cast<const bf16x8_t *>(column + ((2 * ks + h) ^ ((c32 >> 1) & 7)) * 16);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        shortx4_t v[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+          v[t] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_tr_t)(reinterpret_cast<shortx4_t *>(lds_latent) + 2 * buf * kBuf + at_v[t][d & 1] + 32 * ks * CH + 16 * (d >> 1)));
+        const uint2 v0 = __builtin_bit_cast(uint2, v[0]), v1 = __builtin_bit_cast(uint2, v[1]);
+        o[d] = mfma32(as_bf16x8(make_uint4(v0.x, v0.y, v1.x, v1.y)), w, o[d]);
+      }
+    }
+    landed();
+    pg = pg_next;
+    buf ^= 1;
+  }
+
+  // the columns' sums of weights, over the halves of a wave and the four waves
+  l_run += __shfl_xor(l_run, 32, 64);
+  reinterpret_cast<float *>(regions + kw * kRegion)[c32] = l_run;
+  met();
+  const float *l4 = reinterpret_cast<float *>(regions) + c32;
+  const float l_tot = (l4[0] + l4[kRegion / 4]) + (l4[2 * kRegion / 4] + l4[3 * kRegion / 4]);
+  if (!valid) return;
+  const float inv = n_splits > 1 ? 1.0f : l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+  const size_t to = size_t(row) * heads + head;
+  const size_t split_to = size_t(blockIdx.z) * n_rows * heads + to;
+#pragma unroll
+  for (int d = 0; d < ND; ++d)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int at = 32 * (ND * kw + d) + 8 * u + 4 * h;       // four consecutive numbers; rank is a multiple of 8
+      if (at >= rank) continue;
+      const float v0 = o[d][4 * u] * inv, v1 = o[d][4 * u + 1] * inv, v2 = o[d][4 * u + 2] * inv, v3 = o[d][4 * u + 3] * inv;
+      if (n_splits > 1) *reinterpret_cast<float4 *>(part_o + split_to * rank + at) = make_float4(v0, v1, v2, v3);
+      else *reinterpret_cast<uint2 *>(out + to * rank + at) = make_uint2(pack_bf16(v0, v1), pack_bf16(v2, v3));
+    }
+  if (n_splits > 1 && kw == 0 && h == 0) {
+    part_ml[2 * split_to] = m_run;
+    part_ml[2 * split_to + 1] = l_tot;
+  }
+}
+
 // out[column, :] = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), M the largest m_s: the shares of
 // a column's keys that n_splits blocks worked on, put together.  A block a column; the shares'
 // weights 2^(m_s - M) wait in LDS, and a thread asks for eight shares of its numbers at a time.
@@ -395,6 +629,23 @@ int launch_attention(bf16_t *out, const bf16_t *q, const bf16_t *cache, const in
                      int rot_dim, float scale, int window, int tile_rows, int n_splits, float *part_o, float *part_ml,
                      int n_rows, hipStream_t s) {
   const int latent = rank + rot_dim;
+  if (tile_rows == 16) {
+    constexpr int ND = NV / 8, lds_pages = latent_pages_lds<KQ>();
+    static bool raised_pages = false;
+    if (!raised_pages) {
+      if (hipFuncSetAttribute((const void *)latent_attention_pages_kernel<KQ, ND>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                              lds_pages) != hipSuccess)
+        (void)hipGetLastError();
+      raised_pages = true;
+    }
+    latent_attention_pages_kernel<KQ, ND><<<dim3(n_tiles, (heads + 3) / 4, n_splits), kPageThreads, lds_pages, s>>>(
+        out, q, cache, page_table, max_pages, n_pages_total, row_pos, tiles, heads, rank, rot_dim, scale, window, n_splits,
+        part_o, part_ml, n_rows);
+    if (n_splits > 1)
+      latent_merge_kernel<<<unsigned(size_t(n_rows) * heads), 256, 0, s>>>(out, part_o, part_ml, n_splits,
+                                                                           size_t(n_rows) * heads, rank);
+    return sb::check_launch("sb_latent_attention_bf16");
+  }
   const int kq = (latent + 31) / 32, nv = (rank + 15) / 16;
   const size_t lds = 2 * (size_t(kHalf) * (kq * 32 + kPadK) + size_t(nv) * 16 * kVtStride) * sizeof(bf16_t);
   static bool raised = false;              // once per kernel of this shape: more dynamic LDS than the default allows
@@ -404,11 +655,10 @@ int launch_attention(bf16_t *out, const bf16_t *q, const bf16_t *cache, const in
       (void)hipGetLastError();
     raised = true;
   }
-  const int heads_per_block = kColGroups * (16 / tile_rows);
-  dim3 grid(n_tiles, (heads + heads_per_block - 1) / heads_per_block, n_splits);
+  dim3 grid(n_tiles, (heads + kColGroups * 16 - 1) / (kColGroups * 16), n_splits);
   latent_attention_mfma_kernel<KQ, NV><<<grid, kAttnThreads, lds, s>>>(out, q, cache, page_table, max_pages, n_pages_total,
                                                                    row_pos, tiles, heads, rank, rot_dim, scale, window,
-                                                                   tile_rows, n_splits, part_o, part_ml, n_rows);
+                                                                   n_splits, part_o, part_ml, n_rows);
   if (n_splits > 1)
     latent_merge_kernel<<<unsigned(size_t(n_rows) * heads), 256, 0, s>>>(out, part_o, part_ml, n_splits,
                                                                          size_t(n_rows) * heads, rank);

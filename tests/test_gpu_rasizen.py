@@ -592,6 +592,37 @@ def test_matrix_core_latent_attention_equals_the_plain_kernel(heads, dim, rot_di
     part_close(outs[True][1], outs[True][0].float().cpu().numpy(), "bfloat16", "portions and single rows against whole")
 
 
+@pytest.mark.parametrize("heads, rank, rot_dim", [(5, 40, 8), (3, 64, 32), (4, 128, 64), (7, 200, 24), (2, 256, 64), (1, 264, 8), (6, 512, 64)])
+@pytest.mark.parametrize("window", [0, 64, 129])
+def test_matrix_core_latent_attention_of_prompt_rows(heads, rank, rot_dim, window):
+    """Every compiled shape at its largest and at sizes that leave chunks, tiles and heads over; tiles cut short, rows
+    that end on a page's first and last slot, a page that is not there, keys shared out over blocks or not."""
+    from sonicboom_amd import ops
+    latent = rank + rot_dim
+    seqs = [(0, 1), (0, 64), (63, 17), (190, 66), (511, 40), (1000, 25)]           # (cached keys, rows)
+    n_pages = [(a + n + 63) // 64 for a, n in seqs]
+    table = torch.full((len(seqs), max(n_pages) + 1), -1, dtype=torch.int32)
+    order, at = torch.randperm(sum(n_pages), generator=torch.Generator().manual_seed(2)), 0
+    for i, n in enumerate(n_pages):
+        table[i, :n] = order[at:at + n].int()
+        at += n
+    table[4, 3] = -1                                                                # its keys are seen by nobody
+    cache = rand(sum(n_pages), 64, latent, seed=3).to(BF16).to(DEV)
+    pos = torch.tensor([a + i for a, n in seqs for i in range(n)], dtype=torch.int32, device=DEV)
+    seq = torch.tensor([i for i, (_, n) in enumerate(seqs) for _ in range(n)], dtype=torch.int32, device=DEV)
+    q = rand(len(pos), heads, latent, seed=4).to(BF16).to(DEV)
+    tiles, row0 = [], 0
+    for i, (_, n) in enumerate(seqs):
+        tiles += [(row0 + r, min(16, n - r), i, 0) for r in range(0, n, 16)]
+        row0 += n
+    tiles, table = torch.tensor(tiles, dtype=torch.int32, device=DEV), table.to(DEV)
+    want = ops.latent_attention_plain(q, cache, table, pos, seq, rank, latent ** -0.5, window).float().cpu().numpy()
+    for max_keys in (0, 1025):          # whole, and in shares
+        got = ops.latent_attention_mfma(q, cache, table, pos, tiles, rank, latent ** -0.5, window, False, max_keys)
+        # both round weights or results to bfloat16 (2^-9 of values up to about 4)
+        assert np.abs(got.float().cpu().numpy() - want).max() <= 2.0 ** -6 + 2.0 ** -8 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("rows, n_out, n_in", [(300, 96, 64), (1000, 520, 256), (129, 40, 72)])
 def test_tiled_product_adds_into_the_stream_with_a_multiplier(rows, n_out, n_in):
     """resid += scale * (x W^T + b) in the tiled product's epilogue, against the product followed by the scaled add."""
