@@ -601,6 +601,52 @@ def gemm_bf16_partial(x: torch.Tensor, w: torch.Tensor, packed_shape=None) -> Op
     return partial
 
 
+# Rows of a decode step up to which the norm between attention and the feed-forward rides in the products around it
+SPLIT_MAX_ROWS = 8
+
+
+class ScaledRows:
+    """An RMS norm of a residual stream that is not finished: ``values`` bfloat16 [rows, width] are x * weight, and a
+    row's factor 1 / sqrt(mean of x^2 + eps) follows from ``ssq`` float32 [parts, rows], sums of squares over the
+    row's parts.  :func:`gemm_split_gated`, which reads it, multiplies the factor into its result."""
+
+    def __init__(self, values: torch.Tensor, ssq: torch.Tensor, eps: float):
+        self.values, self.ssq, self.eps = values, ssq, float(eps)
+
+
+def gemm_split_join(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], resid: torch.Tensor, packed_shape,
+                    norm_weight: Optional[torch.Tensor], eps: float) -> ScaledRows:
+    """resid += x w^T (+ bias) for up to 16 bfloat16 rows and packed weights; returns the unfinished RMS norm of the new
+    residual, which the same pass leaves."""
+    _dev(x, w, bias, resid, norm_weight)
+    n, k = packed_shape
+    t = x.shape[0]
+    if x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or x.dim() != 2 or x.shape[1] != k:
+        raise KernelLibraryError(f"gemm shapes do not match: x {tuple(x.shape)}, w {(n, k)}")
+    if resid.dtype != torch.float32 or tuple(resid.shape) != (t, n) or (bias is not None and bias.numel() != n) \
+            or (norm_weight is not None and norm_weight.numel() != n):
+        raise KernelLibraryError("the residual must be float32 and shaped like the product, bias and norm weight as long as a row")
+    xw = torch.empty((t, n), dtype=torch.bfloat16, device=x.device)
+    ssq = torch.empty(((n + 15) // 16, t), dtype=torch.float32, device=x.device)
+    check(library.core().sb_gemm_split_join_bf16(
+        _p(resid), _p(xw), _p(ssq), _p(norm_weight), _dt(norm_weight) if norm_weight is not None else 0, _p(x), _p(w), _p(bias),
+        _dt(bias) if bias is not None else 0, t, n, k, _stream()))
+    return ScaledRows(xw, ssq, eps)
+
+
+def gemm_split_gated(x: ScaledRows, w: torch.Tensor, packed_shape, gated) -> torch.Tensor:
+    """act(x wg^T) * (x wu^T) in bfloat16 for up to 16 rows and packed weights."""
+    rows, ssq = x.values, x.ssq
+    _dev(rows, ssq, w)
+    n, k, t = packed_shape[0] // 2, packed_shape[1], rows.shape[0]
+    if w.dtype != torch.bfloat16 or rows.dim() != 2 or rows.shape[1] != k or packed_shape[0] % 2:
+        raise KernelLibraryError(f"gemm shapes do not match: x {tuple(rows.shape)}, w {tuple(packed_shape)}")
+    out = torch.empty((t, n), dtype=torch.bfloat16, device=rows.device)
+    check(library.core().sb_gemm_split_gated_bf16(_p(out), _p(rows), _p(ssq), ssq.shape[0], x.eps, _p(w), t, n, k,
+                                                  gate_code(gated), _stream()))
+    return out
+
+
 def reduce_resid_norm(partial: torch.Tensor, bias: Optional[torch.Tensor], x: torch.Tensor,
                       norm_weight: Optional[torch.Tensor], eps: float, out_dtype: Optional[torch.dtype],
                       scale: float = 1.0, groups: int = 1) -> Optional[torch.Tensor]:

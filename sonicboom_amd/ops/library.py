@@ -22,6 +22,8 @@ _CORE_SIGNATURES = {
     "sb_embed": [_P, _P, _I, _P, _I, _I, _I, _P],
     "sb_rmsnorm": [_P, _I, _P, _P, _I, _P, _I, _I, _F, _P],
     "sb_gemm": [_P, _I, _P, _I, _P, _I, _P, _I, _P, _I, _I, _I, _P],
+    "sb_gemm_split_join_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P],
+    "sb_gemm_split_gated_bf16": [_P, _P, _P, _I, _F, _P, _I, _I, _I, _I, _P],
     "sb_gemm_f32_packed": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
     "sb_gemm_bf16_kernel": [_I, _I, _I, _I],
     "sb_dense_layers": [_P, _P, _I, _P],

@@ -208,10 +208,13 @@ class Attention(Mixer):
     graph_safe = True     # its launches depend on device buffers only
     fold_rotation = True  # decode steps: rotate and store inside the attention kernel where it takes the sizes
 
-    def forward(self, h, x, ctx, binding, then_norm=None):
+    def forward(self, h, x, ctx, binding, then_norm=None, unfinished=False):
         """x += attention(h).  Returns then_norm(x) when the output projection could apply the
-        norm in its last pass, else None."""
+        norm in its last pass, else None.  ``unfinished``: the reader also takes the norm without its
+        rows' factors (Linear.join)."""
         a = self._attend(h, ctx, binding)
+        if unfinished and self.out_scale == 1.0 and self.out.joins(a, then_norm):
+            return self.out.join(a, x, then_norm)
         return self.out.add_into(a, x, then_norm, self.rt.act_dtype, scale=self.out_scale)
 
     def from_rows(self, rows, ctx, binding):

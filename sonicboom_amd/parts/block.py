@@ -33,6 +33,8 @@ from __future__ import annotations
 import torch
 
 from .. import ops
+from .attention import Attention
+from .ffn import GatedDenseFFN
 from .base import Branch, Joined, Part, StateSpec, register_part
 from .spec import PartSpec, TensorSpec
 
@@ -90,7 +92,9 @@ class PreNormBlock(Part):
             h = ops.time_conv(h, self.input_conv, None, binding.states["block.input_conv"], ctx, act, residual=True)
         f = None
         after = self.ffn_norm if self.ffn is not None else next_norm     # the norm that follows the mixer
-        if getattr(self.mixer, "fuses_norm", False):
+        if type(self.mixer) is Attention and type(self.ffn) is GatedDenseFFN and self.ffn.takes_unfinished(ctx):
+            f = self.mixer.forward(h, x, ctx, binding, then_norm=after, unfinished=True)
+        elif getattr(self.mixer, "fuses_norm", False):
             f = self.mixer.forward(h, x, ctx, binding, then_norm=after)
         else:
             self.mixer.forward(h, x, ctx, binding)

@@ -64,6 +64,11 @@ class GatedDenseFFN(Part):
     fuses_norm = True
     graph_safe = True     # its launches depend on device buffers only
 
+    def takes_unfinished(self, ctx) -> bool:
+        """Whether forward() also takes what Linear.join() returns: in decode steps (what a prompt step launches is
+        written down a second time for steps made in one call)."""
+        return ctx.is_decode and self.gate_up.packed is not None and self.rt.act_dtype == torch.bfloat16 and self.gate_up.n_in % 8 == 0
+
     def forward(self, h, x, ctx, then_norm=None):
         """x += out_scale * ffn(h).  Returns then_norm(x) when the down projection could apply the
         norm in its last pass, else None."""

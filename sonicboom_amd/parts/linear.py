@@ -103,6 +103,15 @@ class Linear:
             ops.add_scaled(resid, self(x, torch.float32), scale)      # a pass of its own over the stream
         return None
 
+    def joins(self, x: torch.Tensor, then_norm) -> bool:
+        """Whether join() takes the call."""
+        return self.packed is not None and not self.gated and x.dtype == torch.bfloat16 and x.shape[0] <= ops.SPLIT_MAX_ROWS \
+            and self.n_in % 8 == 0 and ops.launchers_choose() and getattr(then_norm, "fusable", False) and int(then_norm.groups) == 1
+
+    def join(self, x: torch.Tensor, resid: torch.Tensor, then_norm) -> "ops.ScaledRows":
+        """resid += x W^T (+ b); returns then_norm(resid) but for the rows' factors, for gated_product() to finish."""
+        return ops.gemm_split_join(x, self.packed, self.bias, resid, (self.rows, self.n_in), then_norm.weight, then_norm.eps)
+
     def activated(self, x: torch.Tensor, out_dtype: torch.dtype, activation: str, params: Optional[torch.Tensor] = None) -> torch.Tensor:
         """act(x W^T (+ b)): in the tiled product's epilogue where it knows the activation; in the pass that adds a product's K
         slices where there are any; else in a pass of its own over the float32 product."""
@@ -118,7 +127,9 @@ class Linear:
 
     def gated_product(self, x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
         """act(x Wg^T) * (x Wu^T): one fused kernel on the matrix cores, or the product in
-        float32 followed by the activation kernel."""
+        float32 followed by the activation kernel.  ``x``: rows, or what join() has returned."""
+        if isinstance(x, ops.ScaledRows):
+            return ops.gemm_split_gated(x, self.packed, (self.rows, self.n_in), self.activation)
         if self.packed is not None:
             if x.dtype != torch.bfloat16:
                 x = ops.cast(x, torch.bfloat16)

@@ -1060,6 +1060,39 @@ def test_attention_prefill_forms(hq, hkv, hd, window, form):
             test_attention_prefill_window_edge(hq, hkv, hd, window)
 
 
+@pytest.mark.parametrize("rows, width, n_in, inner", [(1, 16, 8, 16), (3, 104, 96, 40), (8, 896, 896, 200), (16, 72, 1032, 17), (5, 1536, 2048, 33)])
+@pytest.mark.parametrize("gate", ["silu", "gelu_tanh", "relu"])
+def test_products_that_carry_the_norm_between_them(rows, width, n_in, inner, gate):
+    """The product that joins the stream and leaves an unfinished norm, and the gated one that finishes it, against 64 bits:
+    one step of 32 k and less, waves without any, features and rows that fill no tile, with and without bias and weight."""
+    from sonicboom_amd import ops
+    x, w, b = randn(rows, n_in).to(BF16), randn(width, n_in, scale=0.1, seed=1).to(BF16), randn(width, seed=2)
+    resid, nw = randn(rows, width, seed=3), randn(width, seed=4).to(BF16)
+    wg = randn(2 * inner, width, scale=0.1, seed=5).to(BF16)
+    for bias, weight in ((b, nw), (None, None)):
+        want = resid.double() + x.double() @ w.double().T + (0.0 if bias is None else bias.double())
+        stream = resid.to(DEV).clone()
+        h = ops.gemm_split_join(x.to(DEV), ops.pack_weight(w.to(DEV)), None if bias is None else bias.to(DEV), stream, (width, n_in),
+                                None if weight is None else weight.to(DEV), 1e-6)
+        # float32 sums of n_in products of size 0.1: n_in 2^-24 of the sum of their magnitudes at most
+        bound = (x.abs().double() @ w.abs().double().T + resid.abs().double() + 1.0) * (n_in + 4) * 2.0 ** -24
+        assert ((stream.cpu().double() - want).abs() <= bound).all()
+        now = stream.cpu().double()
+        assert torch.allclose(h.ssq.cpu().double().sum(0), now.square().sum(1), rtol=1e-5)
+        scaled = now * (1.0 if weight is None else weight.double())
+        assert ((h.values.cpu().double() - scaled).abs() <= scaled.abs() * 2.0 ** -8 + 1e-30).all()
+        got = ops.gemm_split_gated(h, ops.pack_weight(wg.to(DEV), True), (2 * inner, width), gate).cpu().double()
+        # from the same bfloat16 rows: float32 sums, then one rounding to bfloat16
+        f = (now.square().mean(1, keepdim=True) + 1e-6).rsqrt()
+        e = f * (h.values.cpu().double() @ wg.double().T)
+        g, u = e[:, :inner], e[:, inner:]
+        act = {"silu": torch.nn.functional.silu, "relu": torch.relu,
+               "gelu_tanh": lambda v: torch.nn.functional.gelu(v, approximate="tanh")}[gate]
+        ref = act(g) * u
+        slack = (f * (h.values.cpu().double().abs() @ wg.double().abs().T)) * (width + 40) * 2.0 ** -24
+        assert ((got - ref).abs() <= ref.abs() * 2.0 ** -8 + 1.2 * (slack[:, :inner] * u.abs() + slack[:, inner:] * g.abs()) + 1e-5).all()
+
+
 FOLDED_SHAPES = [(4, 2, 16, 16), (3, 1, 32, 32), (5, 5, 48, 16), (6, 2, 80, 64), (28, 4, 128, 128), (16, 1, 64, 0),
                  (2, 1, 256, 256)]
 
