@@ -601,6 +601,9 @@ def gemm_bf16_partial(x: torch.Tensor, w: torch.Tensor, packed_shape=None) -> Op
     return partial
 
 
+# Blocks of four waves that a matrix must give the weight-streaming product: kStreamMinBlocks of csrc/dense_layers.hip
+STREAM_MIN_BLOCKS = 136
+
 # Rows of a decode step up to which the norm between attention and the feed-forward rides in the products around it
 SPLIT_MAX_ROWS = 8
 
