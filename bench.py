@@ -172,7 +172,7 @@ class OpTimer:
     ``sonicboom_amd.ops`` that launches is wrapped between two events on the stream, and the
     times are summed by (function, what it worked on)."""
 
-    NAMES = ("embed", "rmsnorm", "gemm_bf16", "gemm_bf16_partial", "reduce_resid_norm", "rope_kv_store",
+    NAMES = ("embed", "rmsnorm", "gemm_bf16", "gemm_bf16_partial", "gemm_split_join", "gemm_split_gated", "reduce_resid_norm", "rope_kv_store",
              "attention", "attention_decode_rope", "argmax", "gemm_plain", "silu_mul", "add_into", "cast")
 
     def __init__(self, m):
@@ -180,7 +180,7 @@ class OpTimer:
 
     def _label(self, name, args, kw):
         m = self.m
-        if name in ("gemm_bf16", "gemm_bf16_partial"):
+        if name.startswith(("gemm_bf16", "gemm_split")):
             n, k = kw.get("packed_shape") or (args[1].shape[0], args[1].shape[-1])
             if kw.get("gated"):
                 return "gate_up"
@@ -358,7 +358,7 @@ def main() -> int:
         d, ff = m["d"], m["ff"]
         targets = {"qkv": ((m["hq"] + 2 * m["hkv"]) * m["hd"], d), "out": (d, m["hq"] * m["hd"]), "down": (d, ff)}
         forced = {"shape": None, "form": (0, 0)}
-        launcher_partial = ops.gemm_bf16_partial
+        launcher_partial, join_rows = ops.gemm_bf16_partial, ops.SPLIT_MAX_ROWS
 
         def partial(x, w, packed_shape=None):
             if packed_shape is not None and tuple(packed_shape) == forced["shape"]:
@@ -375,6 +375,8 @@ def main() -> int:
 
             def step_ms(shape, form):
                 forced["shape"], forced["form"] = shape, form
+                # (the output product of few rows joins the stream itself unless it is the one that is forced)
+                ops.SPLIT_MAX_ROWS = 0 if shape == targets["out"] else join_rows
                 loop = DecodeLoop(eng, use_graph=not a.no_graph)
                 loop.start(slots, [1] * batch)
                 for _ in range(4):
@@ -398,7 +400,7 @@ def main() -> int:
             for s in slots:
                 eng.free_slot(s)
             del eng
-        ops.gemm_bf16_partial = launcher_partial
+        ops.gemm_bf16_partial, ops.SPLIT_MAX_ROWS = launcher_partial, join_rows
         return 0
 
     if a.workload == "mixed":
@@ -797,7 +799,7 @@ class AllOpsTimer:
 
     SKIP = ("pack_weight", "read_bandwidth", "random_normal", "attention_row_tile", "attention_row_tiles",
             "attention_tall_ok", "attention_tile_height", "launchers_choose", "pack_weight_f32", "attention_mfma_ok", "attention_decode_rope_ok", "gate_code", "reduce_resid_norm_ok",
-            "attention_decode_pages_per_wave", "attention_prefill_form", "ScaledRows", "gemm_tile_shape", "gemm_few_rows_kernel", "mingru_chunk_rows",
+            "attention_decode_pages_per_wave", "attention_prefill_form", "gemm_tile_shape", "gemm_few_rows_kernel", "mingru_chunk_rows",
             "loaded_paths", "check", "latent_attention_mfma_ok", "capped_attention_mfma_ok", "moe_max_top", "moe_plan",
             "time_conv_max_taps", "state_scan_limits", "state_scan_chunk_rows", "shared_attention_mfma_ok", "decay_scan_max_side", "decay_scan_max_rank", "decay_chunk_rows",
             "streams_max", "gated_lru_chunk_rows", "gated_lru_limits", "gated_lru_chunked_ok")

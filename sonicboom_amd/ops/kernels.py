@@ -617,8 +617,8 @@ class ScaledRows:
         self.values, self.ssq, self.eps = values, ssq, float(eps)
 
 
-def gemm_split_join(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], resid: torch.Tensor, packed_shape,
-                    norm_weight: Optional[torch.Tensor], eps: float) -> ScaledRows:
+def gemm_split_join(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], resid: torch.Tensor,
+                    norm_weight: Optional[torch.Tensor], eps: float, packed_shape) -> ScaledRows:
     """resid += x w^T (+ bias) for up to 16 bfloat16 rows and packed weights; returns the unfinished RMS norm of the new
     residual, which the same pass leaves."""
     _dev(x, w, bias, resid, norm_weight)
@@ -637,7 +637,7 @@ def gemm_split_join(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tenso
     return ScaledRows(xw, ssq, eps)
 
 
-def gemm_split_gated(x: ScaledRows, w: torch.Tensor, packed_shape, gated) -> torch.Tensor:
+def gemm_split_gated(x: ScaledRows, w: torch.Tensor, gated, packed_shape) -> torch.Tensor:
     """act(x wg^T) * (x wu^T) in bfloat16 for up to 16 rows and packed weights."""
     rows, ssq = x.values, x.ssq
     _dev(rows, ssq, w)

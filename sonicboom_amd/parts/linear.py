@@ -110,7 +110,8 @@ class Linear:
 
     def join(self, x: torch.Tensor, resid: torch.Tensor, then_norm) -> "ops.ScaledRows":
         """resid += x W^T (+ b); returns then_norm(resid) but for the rows' factors, for gated_product() to finish."""
-        return ops.gemm_split_join(x, self.packed, self.bias, resid, (self.rows, self.n_in), then_norm.weight, then_norm.eps)
+        return ops.gemm_split_join(x, self.packed, self.bias, resid, then_norm.weight, then_norm.eps,
+                                   packed_shape=(self.rows, self.n_in))
 
     def activated(self, x: torch.Tensor, out_dtype: torch.dtype, activation: str, params: Optional[torch.Tensor] = None) -> torch.Tensor:
         """act(x W^T (+ b)): in the tiled product's epilogue where it knows the activation; in the pass that adds a product's K
@@ -129,7 +130,7 @@ class Linear:
         """act(x Wg^T) * (x Wu^T): one fused kernel on the matrix cores, or the product in
         float32 followed by the activation kernel.  ``x``: rows, or what join() has returned."""
         if isinstance(x, ops.ScaledRows):
-            return ops.gemm_split_gated(x, self.packed, (self.rows, self.n_in), self.activation)
+            return ops.gemm_split_gated(x, self.packed, gated=self.activation, packed_shape=(self.rows, self.n_in))
         if self.packed is not None:
             if x.dtype != torch.bfloat16:
                 x = ops.cast(x, torch.bfloat16)

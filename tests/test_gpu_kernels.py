@@ -1072,8 +1072,8 @@ def test_products_that_carry_the_norm_between_them(rows, width, n_in, inner, gat
     for bias, weight in ((b, nw), (None, None)):
         want = resid.double() + x.double() @ w.double().T + (0.0 if bias is None else bias.double())
         stream = resid.to(DEV).clone()
-        h = ops.gemm_split_join(x.to(DEV), ops.pack_weight(w.to(DEV)), None if bias is None else bias.to(DEV), stream, (width, n_in),
-                                None if weight is None else weight.to(DEV), 1e-6)
+        h = ops.gemm_split_join(x.to(DEV), ops.pack_weight(w.to(DEV)), None if bias is None else bias.to(DEV), stream,
+                                None if weight is None else weight.to(DEV), 1e-6, packed_shape=(width, n_in))
         # float32 sums of n_in products of size 0.1: n_in 2^-24 of the sum of their magnitudes at most
         bound = (x.abs().double() @ w.abs().double().T + resid.abs().double() + 1.0) * (n_in + 4) * 2.0 ** -24
         assert ((stream.cpu().double() - want).abs() <= bound).all()
@@ -1081,7 +1081,7 @@ def test_products_that_carry_the_norm_between_them(rows, width, n_in, inner, gat
         assert torch.allclose(h.ssq.cpu().double().sum(0), now.square().sum(1), rtol=1e-5)
         scaled = now * (1.0 if weight is None else weight.double())
         assert ((h.values.cpu().double() - scaled).abs() <= scaled.abs() * 2.0 ** -8 + 1e-30).all()
-        got = ops.gemm_split_gated(h, ops.pack_weight(wg.to(DEV), True), (2 * inner, width), gate).cpu().double()
+        got = ops.gemm_split_gated(h, ops.pack_weight(wg.to(DEV), True), gate, packed_shape=(2 * inner, width)).cpu().double()
         # from the same bfloat16 rows: float32 sums, then one rounding to bfloat16
         f = (now.square().mean(1, keepdim=True) + 1e-6).rsqrt()
         e = f * (h.values.cpu().double() @ wg.double().T)
