@@ -108,7 +108,9 @@ attention_plain_kernel(TA *__restrict__ out, const TA *__restrict__ q, int q_str
         if (softcap > 0.0f) s = softcap * tanhf(s / softcap);
       }
       const float cm = wave_max(s);
-      const float p = visible ? expf(s - cm) : 0.0f;
+      // (a score that ran out of the range weighs nothing, also in a chunk that holds no other: the join goes by the
+      // maximum over all chunks)
+      const float p = visible && s != neg_inf ? expf(s - cm) : 0.0f;
       const float cl = wave_sum(p);
       ps[wave][lane] = p;
       if (lane == 0) part_m[wave] = cm, part_l[wave] = cl;

@@ -695,6 +695,32 @@ def test_attention_plain_kernel(hq, hkv, hd, dtype, window):
         close(got[r:r + 1], want, what=f"row {r} (seq {s}, pos {p})", **tol)
 
 
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("hd", [20, 64])
+@pytest.mark.parametrize("gone", [[64], [70], [64, 130], list(range(64, 128)), list(range(128, 140))])
+def test_attention_plain_scores_out_of_range(hd, dtype, gone):
+    """Keys whose score is minus infinity weigh nothing, alone in a chunk of keys or all of it, in the last chunk or before."""
+    from sonicboom_amd import ops
+    hq, hkv, n = 4, 2, 140
+    rows = [64, 70, 127, 128, 139]
+    q, k, v = randn(len(rows), hq, hd), randn(n, hkv, hd, seed=1), randn(n, hkv, hd, seed=2)
+    q[..., 3], k[..., 3] = 1e25, 0.0
+    k[gone, :, 3] = -1e25                      # the product of the two lies below the float32 range
+    q, k, v = q.to(dtype), k.to(dtype), v.to(dtype)
+    table = torch.tensor([[2, 0, 1]], dtype=torch.int32)
+    kc, vc = fill_cache_from([k], [v], table, dtype)
+    got = ops.attention_plain(q.reshape(len(rows), hq * hd).to(DEV), kc, vc, table.to(DEV), torch.tensor(rows, dtype=torch.int32).to(DEV),
+                              torch.zeros(len(rows), dtype=torch.int32).to(DEV), hq, hkv, hd, hd ** -0.5, 0)
+    kept = [j for j in range(n) if j not in gone]
+    want = torch.zeros(len(rows), hq, hd, dtype=torch.float64)
+    for i, pos in enumerate(rows):
+        js = [j for j in kept if j <= pos]
+        for h in range(hq):
+            p = torch.softmax(k[js, h // 2].double() @ q[i, h].double() * hd ** -0.5, 0)
+            want[i, h] = p @ v[js, h // 2].double()
+    close(got, want.reshape(len(rows), hq * hd), atol=2e-5 if dtype == F32 else 2e-2, rtol=1e-5 if dtype == F32 else 1e-2)
+
+
 def attention_case(hq, hkv, hd, lens, rows_per_seq, window, seed=0):
     """Random bf16 keys, values and queries for sequences of ``lens`` tokens on scattered pages;
     ``rows_per_seq[s]`` lists the positions of sequence s that ask.  Returns device operands and the
