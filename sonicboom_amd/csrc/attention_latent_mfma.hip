@@ -172,7 +172,10 @@ latent_attention_mfma_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict_
     for (int it = 0; it < kMaxStage; ++it) {
       const int idx = tid + it * kAttnThreads;
       const int key = idx % kHalf, chunk = idx / kHalf;
-      staged[it] = ld16(src + size_t(key) * latent + 8 * min(chunk, chunks - 1), page >= 0 && chunk < chunks);
+      // (keys that the row does not see are staged as zeros: their slots may hold what another sequence left there, and a
+      // weight of zero does not keep a NaN out of the sums)
+      const int j = h * kHalf + key;
+      staged[it] = ld16(src + size_t(key) * latent + 8 * min(chunk, chunks - 1), page >= 0 && chunk < chunks && j >= lo && j <= pos);
     }
   };
   // A thread holds eight numbers of one key; the turned copy wants a number's keys side by side.
@@ -429,6 +432,9 @@ latent_attention_pages_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict
   };
   const uint32_t page_bytes = uint32_t(SB_PAGE) * latent * 2;
   auto bring = [&](int pg, int buf) {
+    // keys that no row of the tile sees come as zeros: their slots may hold what another sequence left there, and a weight
+    // of zero does not keep a NaN out of the sums
+    const int first_key = lo_blk - pg * SB_PAGE, last_key = hi_blk - pg * SB_PAGE;
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<bf16_t *>(cache + size_t(pt[pg]) * SB_PAGE * latent), 0, page_bytes, 0x00020000);
 #pragma unroll
@@ -436,7 +442,8 @@ latent_attention_pages_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict
       const int at = (wave * (CH / 8) + i) * 64;
       const int slot = at + lane, key = slot / CH, place = slot - key * CH;
       const int chunk = place ^ key_turn(key);                   // CH is a multiple of 8: the exchange stays in its run
-      const uint32_t off = 8 * chunk < latent ? uint32_t(key * latent + 8 * chunk) * 2 : page_bytes;      // past the end: zeros
+      const bool in = 8 * chunk < latent && key >= first_key && key <= last_key;
+      const uint32_t off = in ? uint32_t(key * latent + 8 * chunk) * 2 : page_bytes;      // past the end: zeros
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)(lds_latent) + buf * kBuf + at, 16, int(off), 0, 0, 0);
     }
   };

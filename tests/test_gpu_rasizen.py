@@ -623,6 +623,41 @@ def test_matrix_core_latent_attention_of_prompt_rows(heads, rank, rot_dim, windo
         assert np.abs(got.float().cpu().numpy() - want).max() <= 2.0 ** -6 + 2.0 ** -8 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("heads, rank, rot_dim", [(5, 40, 8), (3, 128, 64), (2, 256, 64), (17, 512, 64)])
+@pytest.mark.parametrize("window", [0, 100])
+@pytest.mark.parametrize("single", [False, True])
+def test_matrix_core_latent_attention_leaves_unseen_slots_out(heads, rank, rot_dim, window, single):
+    """Slots that no row of a sequence sees (past its end, before its window) may hold anything, a NaN among it: the
+    results have the bits that they have over zeros.  Prompt rows and single rows, whole and with the keys shared out."""
+    from sonicboom_amd import ops
+    latent = rank + rot_dim
+    seqs = [(0, 1), (70, 1), (131, 1), (959, 1), (500, 1)] if single else [(0, 5), (40, 30), (131, 16), (900, 40)]
+    n_pages = [(a + n + 63) // 64 for a, n in seqs]
+    table = torch.full((len(seqs), max(n_pages)), -1, dtype=torch.int32)
+    cache, at = rand(sum(n_pages), 64, latent, seed=3).to(BF16), 0
+    unseen = torch.zeros(sum(n_pages) * 64, dtype=torch.bool)
+    for i, (a, n) in enumerate(seqs):
+        table[i, :n_pages[i]] = torch.arange(at, at + n_pages[i]).int()
+        unseen[at * 64 + a + n:(at + n_pages[i]) * 64] = True
+        if window:
+            unseen[at * 64:at * 64 + max(a - window + 1, 0)] = True
+        at += n_pages[i]
+    pos = torch.tensor([a + i for a, n in seqs for i in range(n)], dtype=torch.int32, device=DEV)
+    q = rand(len(pos), heads, latent, seed=4).to(BF16).to(DEV)
+    tiles, row0 = [], 0
+    for i, (_, n) in enumerate(seqs):
+        tiles += [(row0 + r, min(16, n - r), i, 0) for r in range(0, n, 16)]
+        row0 += n
+    tiles, table = torch.tensor(tiles, dtype=torch.int32, device=DEV), table.to(DEV)
+    for max_keys in (0, 960):
+        out = []
+        for fill in (0.0, float("nan"), float("inf")):
+            c = cache.clone()
+            c.view(-1, latent)[unseen] = fill
+            out.append(ops.latent_attention_mfma(q, c.to(DEV), table, pos, tiles, rank, latent ** -0.5, window, single, max_keys))
+        assert torch.isfinite(out[0].float()).all() and torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
 @pytest.mark.parametrize("rows, n_out, n_in", [(300, 96, 64), (1000, 520, 256), (129, 40, 72)])
 def test_tiled_product_adds_into_the_stream_with_a_multiplier(rows, n_out, n_in):
     """resid += scale * (x W^T + b) in the tiled product's epilogue, against the product followed by the scaled add."""
