@@ -9,6 +9,8 @@
 //          columns, so it can be multiplied in after the next product: (x w inv) W^T = inv (x w) W^T.
 //   gated: act(inv g) * (inv u), the factor made by every block from the sums of squares that the joining product's blocks
 //          left, parts added in a fixed order.
+// The squares are float products added up in double, and the mean is rounded once, as every RMS norm here does it
+// (embed_norm.hip).  The weighted rows are rounded to bfloat16 before the factor and not after it: the same relative error.
 // Measured (us, replayed graphs, weights cold; one and eight rows): the joining product with its norm against K slices and
 // the pass, width 896 6.2 -> 3.7 and 6.6 -> 4.0, 1,536 7.4 -> 4.6 and 7.8 -> 5.1, 2,048 8.6 -> 6.1 and 8.9 -> 6.5, 3,584
 // 11.1 -> 8.1 and 11.5 -> 8.4; the gated one against the kernel that streams weights, 9,728 x 896 7.3 -> 7.6 and 7.7 -> 7.8,
@@ -27,7 +29,7 @@ namespace {
 struct SplitArgs {
   int n_rows, n_out, n_in;
   // gated: the row's factor of X, an unfinished norm: ssq [ssq_parts][n_rows]
-  const float *ssq;
+  const double *ssq;
   int ssq_parts;
   float eps;
   bf16_t *y;            // gated: [n_rows][n_out]
@@ -36,7 +38,7 @@ struct SplitArgs {
   int bias_dtype;
   float *resid;         // join: [n_rows][n_out], added to in place
   bf16_t *xw;           // join: x * norm_w, and
-  float *ssq_out;       // [tiles][n_rows]
+  double *ssq_out;      // [tiles][n_rows]
   const void *norm_w;   // (NULL: ones)
   int norm_dtype;
 };
@@ -50,7 +52,7 @@ gemm_split_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, Sp
   constexpr int kAhead = 8;
   constexpr int kGroups = 64 * W / kMaxRows;     // threads a row that add its sums of squares
   __shared__ floatx4_t red[W * G * 64];
-  __shared__ float row_part[kGroups * kMaxRows];
+  __shared__ double row_part[kGroups * kMaxRows];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
@@ -87,7 +89,7 @@ gemm_split_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, Sp
   float old[4] = {0.f, 0.f, 0.f, 0.f}, nw[4] = {1.f, 1.f, 1.f, 1.f}, bias[4] = {0.f, 0.f, 0.f, 0.f};
   if constexpr (GATED) {
     const int row = tid % kMaxRows, grp = tid / kMaxRows;
-    float s = 0.f;
+    double s = 0.0;
     if (row < a.n_rows) {
 #pragma unroll 4
       for (int p = grp; p < a.ssq_parts; p += kGroups) s += a.ssq[size_t(p) * a.n_rows + row];
@@ -134,21 +136,22 @@ gemm_split_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, Sp
     for (int k = 0; k < W; ++k) v[g] = v[g] + red[(k * G + g) * 64 + lane];
   }
   if constexpr (GATED) {
-    float s = 0.f;
+    double s = 0.0;
 #pragma unroll
     for (int k = 0; k < kGroups; ++k) s += row_part[k * kMaxRows + r];
-    const float inv = 1.0f / sqrtf(s / float(a.n_in) + a.eps);
+    const float inv = 1.0f / sqrtf(float(s / double(a.n_in)) + a.eps);
     if (!unit_live) return;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
       if (unit_n + e < a.n_out)
         a.y[size_t(r) * a.n_out + unit_n + e] = f32_to_bf16(gate_act(v[0][e] * inv, a.gate) * (v[G - 1][e] * inv));
   } else {
-    float sq = 0.f, now[4];
+    float now[4];
+    double sq = 0.0;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       now[e] = old[e] + (v[0][e] + bias[e]);
-      sq = fmaf(now[e], now[e], sq);             // (columns and rows past the last one are zeros)
+      sq += double(now[e] * now[e]);             // (columns and rows past the last one are zeros)
     }
     if (unit_live) {
 #pragma unroll
@@ -179,7 +182,7 @@ int check(const char *what, const void *x, const void *w, int n_rows, int n_out,
 
 }  // namespace
 
-extern "C" int sb_gemm_split_join_bf16(float *resid, void *xw, float *ssq, const void *norm_w, int norm_dtype, const void *x,
+extern "C" int sb_gemm_split_join_bf16(float *resid, void *xw, double *ssq, const void *norm_w, int norm_dtype, const void *x,
                                        const void *w, const void *bias, int bias_dtype, int n_rows, int n_out, int n_in,
                                        void *stream) {
   const int rc = check("sb_gemm_split_join_bf16", x, w, n_rows, n_out, n_in);
@@ -201,7 +204,7 @@ extern "C" int sb_gemm_split_join_bf16(float *resid, void *xw, float *ssq, const
   return sb::check_launch("sb_gemm_split_join_bf16");
 }
 
-extern "C" int sb_gemm_split_gated_bf16(void *y, const void *x, const float *ssq, int ssq_parts, float eps, const void *w,
+extern "C" int sb_gemm_split_gated_bf16(void *y, const void *x, const double *ssq, int ssq_parts, float eps, const void *w,
                                         int n_rows, int n_out, int n_in, int gate, void *stream) {
   const int rc = check("sb_gemm_split_gated_bf16", x, w, n_rows, n_out, n_in);
   if (rc != SB_OK) return rc;

@@ -124,12 +124,12 @@ int sb_gemm_f32_packed(void *y, int y_dtype, const float *x, const float *w, con
 /* bf16 products of up to 16 rows against packed weights whose blocks own their output features whole.
  * join: resid[t,n] += sum_k X[t,k] W[n,k] (+ bias[n]), resid f32 [n_rows][n_out] in place, and an RMS norm of it whose factor
  * of a row is still to be multiplied in: xw[t,n] = bf16(resid[t,n] * norm_w[n]) (norm_w NULL: ones), ssq
- * [ceil(n_out / 16)][n_rows] the sums of the squares of resid over sixteen columns each. */
-int sb_gemm_split_join_bf16(float *resid, void *xw, float *ssq, const void *norm_w, int norm_dtype, const void *x, const void *w,
+ * f64 [ceil(n_out / 16)][n_rows] the sums of the squares of resid over sixteen columns each. */
+int sb_gemm_split_join_bf16(float *resid, void *xw, double *ssq, const void *norm_w, int norm_dtype, const void *x, const void *w,
                             const void *bias, int bias_dtype, int n_rows, int n_out, int n_in, void *stream);
 /* Y = act(f X Wg^T) * (f X Wu^T), bf16 [n_rows][n_out]: f[t] = 1 / sqrt(sum of ssq[.][t] / n_in + eps) the factor of such a
- * norm X, ssq f32 [ssq_parts][n_rows]; gate: an sb_gate. */
-int sb_gemm_split_gated_bf16(void *y, const void *x, const float *ssq, int ssq_parts, float eps, const void *w, int n_rows,
+ * norm X, ssq f64 [ssq_parts][n_rows]; gate: an sb_gate. */
+int sb_gemm_split_gated_bf16(void *y, const void *x, const double *ssq, int ssq_parts, float eps, const void *w, int n_rows,
                              int n_out, int n_in, int gate, void *stream);
 
 /* out[t,i] = act(gu[t,i]) * gu[t,width+i];  gu is [t, 2*width]; gate: SB_GATE_SILU or

@@ -610,7 +610,7 @@ SPLIT_MAX_ROWS = 8
 
 class ScaledRows:
     """An RMS norm of a residual stream that is not finished: ``values`` bfloat16 [rows, width] are x * weight, and a
-    row's factor 1 / sqrt(mean of x^2 + eps) follows from ``ssq`` float32 [parts, rows], sums of squares over the
+    row's factor 1 / sqrt(mean of x^2 + eps) follows from ``ssq`` float64 [parts, rows], sums of squares over the
     row's parts.  :func:`gemm_split_gated`, which reads it, multiplies the factor into its result."""
 
     def __init__(self, values: torch.Tensor, ssq: torch.Tensor, eps: float):
@@ -630,7 +630,7 @@ def gemm_split_join(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tenso
             or (norm_weight is not None and norm_weight.numel() != n):
         raise KernelLibraryError("the residual must be float32 and shaped like the product, bias and norm weight as long as a row")
     xw = torch.empty((t, n), dtype=torch.bfloat16, device=x.device)
-    ssq = torch.empty(((n + 15) // 16, t), dtype=torch.float32, device=x.device)
+    ssq = torch.empty(((n + 15) // 16, t), dtype=torch.float64, device=x.device)
     check(library.core().sb_gemm_split_join_bf16(
         _p(resid), _p(xw), _p(ssq), _p(norm_weight), _dt(norm_weight) if norm_weight is not None else 0, _p(x), _p(w), _p(bias),
         _dt(bias) if bias is not None else 0, t, n, k, _stream()))
@@ -662,6 +662,8 @@ def reduce_resid_norm(partial: torch.Tensor, bias: Optional[torch.Tensor], x: to
         raise KernelLibraryError("reduce_resid_norm needs float32 slices [s, rows, width] and a residual [rows, width]")
     s_, t, width = partial.shape
     if bias is not None and bias.numel() != width:
+    if ssq.dtype != torch.float64 or ssq.dim() != 2 or ssq.shape[1] != t:
+        raise KernelLibraryError("the sums of squares must be float64 [parts, rows]")
         raise KernelLibraryError("bias does not match the row width")
     if norm_weight is not None and norm_weight.numel() != width:
         raise KernelLibraryError("norm weight does not match the row width")

@@ -1119,6 +1119,30 @@ def test_products_that_carry_the_norm_between_them(rows, width, n_in, inner, gat
         assert ((got - ref).abs() <= ref.abs() * 2.0 ** -8 + 1.2 * (slack[:, :inner] * u.abs() + slack[:, inner:] * g.abs()) + 1e-5).all()
 
 
+def test_the_norm_between_two_products_sums_in_double():
+    """Rows whose squares are float numbers but whose sum of squares over the width is none, and rows of many small numbers
+    beside a large one: the factor follows from the sum in double, as of every RMS norm."""
+    from sonicboom_amd import ops
+    rows, width, n_in, inner = 4, 3584, 64, 48
+    x, w = torch.zeros(rows, n_in, dtype=BF16).to(DEV), randn(width, n_in, seed=1).to(BF16).to(DEV)
+    resid = randn(rows, width, seed=2)
+    resid[0] = 1.5e19 * torch.sign(resid[0])               # 2.25e38 each, 8.1e41 in all
+    resid[1, 0], resid[1, 1:] = 3e4, 1.0                   # every square of 1 lies below half a unit of the last place of 9e8
+    resid[2] *= 1e-18
+    wg = randn(2 * inner, width, scale=0.1, seed=5).to(BF16)
+    h = ops.gemm_split_join(x, ops.pack_weight(w), None, resid.to(DEV), None, 1e-6, packed_shape=(width, n_in))
+    squares = (resid * resid).double().sum(1)
+    # sums of 3,584 squares in double: exact to 2^-40
+    assert h.ssq.dtype == torch.float64 and ((h.ssq.cpu().sum(0) - squares).abs() <= squares * 2.0 ** -40).all()
+    got = ops.gemm_split_gated(h, ops.pack_weight(wg.to(DEV), True), "relu", packed_shape=(2 * inner, width)).cpu().double()
+    f = (squares / width + 1e-6).rsqrt()[:, None]
+    e = f * (h.values.cpu().double() @ wg.double().T)
+    slack = (f * (h.values.cpu().double().abs() @ wg.double().abs().T)) * (width + 40) * 2.0 ** -24
+    g, u, sg, su = e[:, :inner], e[:, inner:], slack[:, :inner], slack[:, inner:]
+    assert torch.isfinite(got).all() and got[0].abs().max() > 0.1
+    assert ((got - torch.relu(g) * u).abs() <= (torch.relu(g) * u).abs() * 2.0 ** -8 + 1.2 * (sg * u.abs() + su * g.abs()) + 1e-5).all()
+
+
 FOLDED_SHAPES = [(4, 2, 16, 16), (3, 1, 32, 32), (5, 5, 48, 16), (6, 2, 80, 64), (28, 4, 128, 128), (16, 1, 64, 0),
                  (2, 1, 256, 256)]
 
