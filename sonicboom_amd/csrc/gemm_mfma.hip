@@ -24,20 +24,45 @@ namespace {
 
 constexpr int kXcds = 8;
 
-// The gate's activation in the epilogue of a tile: gate_act, with SiLU's exponential and division on the
-// vector units' own exp2 and reciprocal.  exp(-g) = 2^(h + l), the product with log2(e) carried in two
-// parts, and one Newton step on the quotient keep it within two units of the last of 24 bits (the result is
-// rounded to 8 of them next).  expf and the full division cost a 256 x 256 tile's epilogue 8.5 us of
-// vector instructions, 9 % of the tile at 3,584 k.
-template <int GATE>
+// The gate's activation in the epilogue of a tile: gate_act, with SiLU's exponential and division put together from the
+// vector units' own exp2 and reciprocal for |g| < 87, where neither runs out of the range.  exp(-g) = 2^n 2^a, n the whole
+// number nearest to the product with log2(e) and a what is left of it, log2(e) in two parts; one Newton step on the quotient
+// rounds it like a division.  Against 64 bits, 2^24 numbers each of [-88.7, -80], [-80, -20], [-20, -1], [-1, 1] and [0, 120]:
+// the errors are those of expf and the full division (at most 2.1, 2.3, 3.1, 2.5 and 2.0 units of 2^-24, root mean squares
+// 0.61, 0.61, 0.64, 0.67 and 0.26), from which 20 of the numbers differ at all.  The compiler's expf and division cost a
+// 256 x 256 tile's epilogue 8.5 us of vector instructions, 9 % of the tile at 3,584 k; this form is level with one that reduces
+// nothing and was up to 4.3 units off (2,048 x 37,888 x 3,584 448 and 447 us, 16,384 rows 3.32 and 3.32 ms, 6,398 x 22,016 x
+// 2,048 484 and 483 us).
+// FAR: some number of the wave's tile lies outside; those take gate_act.
+constexpr float kSiluRange = 87.0f;
+template <int GATE, bool FAR>
 __device__ __forceinline__ float tile_gate(float g) {
-  if constexpr (GATE != SB_GATE_SILU) return gate_act(g, GATE);
-  const bool inside = fabsf(g) < 80.0f;          // outside, the corrections may meet infinities
-  const float h = g * -1.44269502f, l = fmaf(g, -1.44269502f, -h) + g * -1.92596303e-8f;
-  const float e = __builtin_amdgcn_exp2f(h);
-  const float d = 1.0f + (inside ? fmaf(e, l * 0.693147182f, e) : e), r = __builtin_amdgcn_rcpf(d);
-  const float q = g * r;
-  return inside ? fmaf(fmaf(-d, q, g), r, q) : q;
+  if constexpr (GATE != SB_GATE_SILU) {
+    return gate_act(g, GATE);
+  } else {
+#pragma clang fp contract(off)                   // (h - n fused into one operation would count h's rounding twice)
+    constexpr float kMagic = 12582912.0f;        // 1.5 * 2^23: adding it rounds to whole numbers, n in the sum's low bits
+    const float h = g * -1.44269502f, t = h + kMagic;
+    const float l = fmaf(g, -1.92596303e-8f, fmaf(g, -1.44269502f, -h));
+    const uint32_t e = __float_as_uint(__builtin_amdgcn_exp2f((h - (t - kMagic)) + l));
+    const float d = 1.0f + __uint_as_float((__float_as_uint(t) << 23) + e);
+    const float r = __builtin_amdgcn_rcpf(d), q = g * r;
+    const float y = fmaf(fmaf(-d, q, g), r, q);
+    if constexpr (FAR) {
+      const float full = gate_act(g, SB_GATE_SILU);
+      return fabsf(g) >= kSiluRange ? full : y;
+    }
+    return y;
+  }
+}
+// Whether FAR holds; COUNT numbers a lane, the i-th of them number(i).  (Passes a NaN over: it is one in y already.)
+template <int GATE, int COUNT, class Number>
+__device__ __forceinline__ bool silu_far(Number number) {
+  if constexpr (GATE != SB_GATE_SILU) return false;
+  float largest = 0.0f;
+#pragma unroll
+  for (int i = 0; i < COUNT; ++i) largest = fmaxf(largest, fabsf(number(i)));
+  return __any(largest >= kSiluRange);
 }
 typedef uint16_t u16x4_t __attribute__((ext_vector_type(4)));
 
@@ -179,7 +204,7 @@ __device__ __forceinline__ void store_tile(const Args &a, float *lds_f, int t0, 
 // The filling of the turning area from 32 x 32 tiles: acc[i][j][e] is row 8 * (e / 4) +
 // 4 * (lane / 32) + e % 4, column lane % 32 of tile (i, j).  PITCH = NC + 8: rows four apart fall on
 // the other half of the banks.
-template <int MT, int GATED>
+template <int MT, int GATED, bool FAR>
 __device__ __forceinline__ void fill_from_32(floatx16_t (&acc)[MT][2], int i, float *turn) {
   constexpr int kPitch = (GATED ? 32 : 64) + 8;
   const int lane = threadIdx.x & 63, col = lane & 31, row_base = (lane >> 5) * 4;
@@ -187,7 +212,7 @@ __device__ __forceinline__ void fill_from_32(floatx16_t (&acc)[MT][2], int i, fl
   for (int e = 0; e < 16; ++e) {
     const int row = 8 * (e >> 2) + row_base + (e & 3);
     if (GATED) {
-      turn[row * kPitch + col] = tile_gate<GATED>(acc[i][0][e]) * acc[i][1][e];   // GATED: the sb_gate, fixed at compile time
+      turn[row * kPitch + col] = tile_gate<GATED, FAR>(acc[i][0][e]) * acc[i][1][e];   // GATED: the sb_gate, fixed at compile time
     } else {
       turn[row * kPitch + col] = acc[i][0][e];
       turn[row * kPitch + 32 + col] = acc[i][1][e];
@@ -446,9 +471,13 @@ gemm_mfma_kernel(Args a) {
 
   static_assert(2 * (BM + BN) * CPR * 16 >= (kThreads / 64) * 32 * ((GATED ? 32 : 64) + 8) * 4,
                 "the turning areas of the epilogue must fit the stage buffers");
+  const bool far = silu_far<GATED, 16 * MT>([&](int i) { return acc[i / 16][0][i % 16]; });
   store_tile<MT, 32, NW, (GATED ? 32 : 64), (GATED ? 32 : 64) + 8>(
       a, reinterpret_cast<float *>(lds), t0, n0, !GATED,
-      [&](int i, float *turn) { fill_from_32<MT, GATED>(acc, i, turn); });
+      [&](int i, float *turn) {
+        if (GATED == SB_GATE_SILU && far) fill_from_32<MT, GATED, true>(acc, i, turn);
+        else fill_from_32<MT, GATED, false>(acc, i, turn);
+      });
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -618,21 +647,26 @@ gemm_direct16_kernel(Args a) {
   static_assert((NBUF == 2 ? 1 : NBUF) * kBufChunks * 16 >= kWaves * 16 * kPitch * 4,
                 "the turning areas must fit a stage buffer (two buffers: the other one may hold the next tile)");
   auto epilogue = [&](int m, int n, int buf_free) {
+    const bool far = silu_far<GATED, 8 * MT16>([&](int i) { return acc[i / 8][i % 8 / 4][i % 4]; });
     store_tile<MT16, 16, NW, NC, kPitch>(
         a, reinterpret_cast<float *>(lds + buf_free * kBufChunks), m * BM, n * (GATED ? BN / 2 : BN), !GATED,
         [&](int i, float *turn) {
+          const auto fill = [&](auto FAR) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int row = 4 * fg + e;
-            if (GATED) {
+            for (int e = 0; e < 4; ++e) {
+              const int row = 4 * fg + e;
+              if constexpr (GATED != 0) {
 #pragma unroll
-              for (int f = 0; f < 2; ++f)
-                turn[row * kPitch + f * 16 + fr] = tile_gate<GATED>(acc[i][f][e]) * acc[i][f + 2][e];
-            } else {
+                for (int f = 0; f < 2; ++f)
+                  turn[row * kPitch + f * 16 + fr] = tile_gate<GATED, decltype(FAR)::value>(acc[i][f][e]) * acc[i][f + 2][e];
+              } else {
 #pragma unroll
-              for (int f = 0; f < 4; ++f) turn[row * kPitch + f * 16 + fr] = acc[i][f][e];
+                for (int f = 0; f < 4; ++f) turn[row * kPitch + f * 16 + fr] = acc[i][f][e];
+              }
             }
-          }
+          };
+          if (GATED == SB_GATE_SILU && far) fill(std::true_type{});
+          else fill(std::false_type{});
         });
   };
 
@@ -787,21 +821,26 @@ gemm_pipe_kernel(Args a) {
   constexpr int NC = GATED ? 32 : 64, kPitch = GATED ? NC + 4 : NC;
   static_assert(kBufChunks * 16 >= kWaves * 16 * kPitch * 4, "the turning areas must fit a stage buffer");
   auto epilogue = [&](int m, int n, int buf_free) {
+    const bool far = silu_far<GATED, 8 * MT16>([&](int i) { return acc[i / 8][i % 8 / 4][i % 4]; });
     store_tile<MT16, 16, NW, NC, kPitch, !GATED>(
         a, reinterpret_cast<float *>(lds + buf_free * kBufChunks), m * BM, n * (GATED ? BN / 2 : BN), !GATED,
         [&](int i, float *turn) {
+          const auto fill = [&](auto FAR) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int row = 4 * fg + e;
-            if (GATED) {
+            for (int e = 0; e < 4; ++e) {
+              const int row = 4 * fg + e;
+              if constexpr (GATED != 0) {
 #pragma unroll
-              for (int f = 0; f < 2; ++f)
-                turn[row * kPitch + f * 16 + fr] = tile_gate<GATED>(acc[i][f][e]) * acc[i][f + 2][e];
-            } else {
+                for (int f = 0; f < 2; ++f)
+                  turn[row * kPitch + f * 16 + fr] = tile_gate<GATED, decltype(FAR)::value>(acc[i][f][e]) * acc[i][f + 2][e];
+              } else {
 #pragma unroll
-              for (int f = 0; f < 4; ++f) turn[row * kPitch + (f ^ fg) * 16 + fr] = acc[i][f][e];
+                for (int f = 0; f < 4; ++f) turn[row * kPitch + (f ^ fg) * 16 + fr] = acc[i][f][e];
+              }
             }
-          }
+          };
+          if (GATED == SB_GATE_SILU && far) fill(std::true_type{});
+          else fill(std::false_type{});
         });
   };
 

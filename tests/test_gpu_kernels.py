@@ -316,6 +316,37 @@ def test_silu_of_the_tiled_product_over_its_range():
     assert (got[~ok].abs() <= 1e-30).all()
 
 
+@pytest.mark.parametrize("shape, path", [(None, None), (0, "registers"), (2, "registers"), (0, "direct"), (2, "direct")])
+def test_silu_of_the_tiled_product_keeps_float32(shape, path):
+    """Every kernel's epilogue, over all numbers whose e^-g lies in the float32 range: within two units of the last of 24
+    bits (one of the exponential, a half each of the sum and the quotient); past it the values of the full division."""
+    from sonicboom_amd import ops
+    g = torch.cat([torch.linspace(-88.7, 120.0, 20001), torch.logspace(-30, 38, 500), -torch.logspace(-30, 1.9, 500),
+                   torch.tensor([0.0, -88.8, -89.0, -1e3, -3e38, math.inf, -math.inf, math.nan, 1.0, 86.99, 87.0, -86.99, -87.0])])
+    x = torch.zeros(g.numel(), 64, dtype=BF16)
+    rest = g.clone()
+    for i in range(3):                           # three bfloat16 parts add up to the float32 number exactly
+        x[:, i] = torch.where(torch.isinf(g), torch.zeros_like(rest), rest).to(BF16)
+        rest = rest - x[:, i].float()
+    x[:, 3] = 1.0
+    x[:, 4] = torch.where(torch.isinf(g), torch.sign(g) * 1e10, torch.zeros_like(g)).to(BF16)    # an infinite product of finite numbers
+    w = torch.zeros(2, 64, dtype=BF16)
+    w[0, :3] = 1.0
+    w[0, 4] = 1e38
+    w[1, 3] = 1.0
+    with ops.gemm_tile_shape(shape, path):
+        got = ops.gemm_bf16(x.to(DEV), ops.pack_weight(w.to(DEV), True), None, None, F32, gated=True, packed_shape=(2, 64))
+    got = got.cpu()[:, 0].double()
+    finite = torch.isfinite(g)
+    z = torch.where(finite, x[:, :3].double().sum(1), torch.zeros(()).double())
+    assert ((z - g.double()).abs()[finite] <= 2.0 ** -23 * g.double().abs()[finite]).all()
+    want = z / (1.0 + torch.exp(-z))
+    ok = finite & (z >= -88.71)
+    assert ((got - want).abs()[ok] <= 2.5e-7 * want.abs()[ok]).all()
+    assert (got.abs()[finite & ~ok] <= 3e-37).all()
+    assert got[g == math.inf].item() == math.inf and torch.isnan(got[g.isnan() | (g == -math.inf)]).all()
+
+
 def test_gemm_bf16_blocks_that_go_from_tile_to_tile():
     """More 256 x 256 tiles than the GPU has CUs: the blocks of the kernel that loads straight into
     LDS go on to a second tile, whose first stage the first tile's last stage has loaded; in
