@@ -84,11 +84,16 @@ attention_plain_kernel(TA *__restrict__ out, const TA *__restrict__ q, int q_str
       const TC *vp = v_cache + (size_t(page) * heads_kv + kvh) * SB_PAGE * v_dim;
       const int j = c * SB_PAGE + lane;
       const bool visible = j >= lo && j <= pos;
+      // (keys outside the window are left out by their place, not by a weight of zero: what the
+      // cache holds there is anything)
+      const int j0 = max(lo - c * SB_PAGE, 0), j1 = min(pos - c * SB_PAGE, SB_PAGE - 1);
+      const auto seen = [&](int jg) { return 8 * jg <= j1 && 8 * jg + 7 >= j0; };      // some key of eight; uniform
       // the values of this lane's first dimension, asked for ahead of the keys
       float v[8][8];
       if (lane < v_dim) {
 #pragma unroll
-        for (int jg = 0; jg < 8; ++jg) ld_eight(vp + sb_value_index(lane, 8 * jg), v[jg]);
+        for (int jg = 0; jg < 8; ++jg)
+          if (seen(jg)) ld_eight(vp + sb_value_index(lane, 8 * jg), v[jg]);
       }
       float s = neg_inf;
       if (visible) {
@@ -117,17 +122,20 @@ attention_plain_kernel(TA *__restrict__ out, const TA *__restrict__ q, int q_str
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      // (keys outside the window are left out by their place, not by a weight of zero: what the
-      // cache holds there is anything)
-      const int j0 = max(lo - c * SB_PAGE, 0), j1 = min(pos - c * SB_PAGE, SB_PAGE - 1);
       for (int d = lane; d < v_dim; d += 64) {
         if (d >= 64) {
 #pragma unroll
-          for (int jg = 0; jg < 8; ++jg) ld_eight(vp + sb_value_index(d, 8 * jg), v[jg]);
+          for (int jg = 0; jg < 8; ++jg)
+            if (seen(jg)) ld_eight(vp + sb_value_index(d, 8 * jg), v[jg]);
         }
         float acc = 0.0f;
 #pragma unroll
-        for (int jj = 0; jj < SB_PAGE; ++jj) acc = fmaf(ps[wave][jj], jj >= j0 && jj <= j1 ? v[jj >> 3][jj & 7] : 0.0f, acc);
+        for (int jg = 0; jg < 8; ++jg) {
+          if (!seen(jg)) continue;
+#pragma unroll
+          for (int e = 0; e < 8; ++e)
+            acc = fmaf(ps[wave][8 * jg + e], 8 * jg + e >= j0 && 8 * jg + e <= j1 ? v[jg][e] : 0.0f, acc);
+        }
         part_o[wave][d] = acc;
       }
     } else if (lane == 0) {
@@ -162,16 +170,20 @@ attention_plain_kernel(TA *__restrict__ out, const TA *__restrict__ q, int q_str
   }
 }
 
-// Waves of a block: four, each a chunk of 64 keys at a time; eight where the blocks alone leave SIMDs idle.
+template <typename TA, typename TC, int WAVES, typename... A>
+void launch_waves(dim3 grid, int head_dim, hipStream_t s, A... a) {
+  if (head_dim % 8 == 0) attention_plain_kernel<TA, TC, WAVES, true><<<grid, 64 * WAVES, 0, s>>>(a...);
+  else attention_plain_kernel<TA, TC, WAVES, false><<<grid, 64 * WAVES, 0, s>>>(a...);
+}
+
+// Waves of a block: four, each a chunk of 64 keys at a time; eight where the blocks alone leave SIMDs idle; no more than
+// there are chunks that a row can see (`most`), since a wave without one only holds its block's place.
 template <typename TA, typename TC, typename... A>
-void launch_attention(dim3 grid, int head_dim, hipStream_t s, A... a) {
-  const bool few = (long long)grid.x * grid.y <= 512;
-  if (head_dim % 8 == 0) {
-    if (few) attention_plain_kernel<TA, TC, 8, true><<<grid, 512, 0, s>>>(a...);
-    else attention_plain_kernel<TA, TC, 4, true><<<grid, 256, 0, s>>>(a...);
-  } else {
-    attention_plain_kernel<TA, TC, 4, false><<<grid, 256, 0, s>>>(a...);
-  }
+void launch_attention(dim3 grid, int head_dim, int most, hipStream_t s, A... a) {
+  if (most <= 1) launch_waves<TA, TC, 1>(grid, head_dim, s, a...);
+  else if (most <= 2) launch_waves<TA, TC, 2>(grid, head_dim, s, a...);
+  else if (most <= 4 || (long long)grid.x * grid.y > 512) launch_waves<TA, TC, 4>(grid, head_dim, s, a...);
+  else launch_waves<TA, TC, 8>(grid, head_dim, s, a...);
 }
 
 }  // namespace
@@ -267,8 +279,10 @@ extern "C" int sb_attention_chunked(void *out, const void *q, int act_dtype, int
   if (n_rows == 0) return SB_OK;
   hipStream_t s = (hipStream_t)stream;
   dim3 grid(n_rows, heads_q);
+  const int reach = window > 0 ? window : chunk;             // keys from the first that a row sees to itself
+  const int most = reach > 0 ? min(max_pages, (reach - 1 + SB_PAGE - 1) / SB_PAGE + 1) : max_pages;
 #define SB_GO(TA, TC)                                                                           \
-  launch_attention<TA, TC>(grid, head_dim, s,                                                    \
+  launch_attention<TA, TC>(grid, head_dim, most, s,                                              \
       (TA *)out, (const TA *)q, q_stride, (const TC *)k_cache, (const TC *)v_cache, page_table,  \
       max_pages, n_pages_total, row_pos, row_seq, heads_q, heads_kv, head_dim, scale, window, v_dim,  \
       softcap, sink, sink_scores, gate, gate_stride, gate_per_head, chunk)

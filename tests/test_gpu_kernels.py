@@ -726,6 +726,27 @@ def test_attention_plain_kernel(hq, hkv, hd, dtype, window):
         close(got[r:r + 1], want, what=f"row {r} (seq {s}, pos {p})", **tol)
 
 
+@pytest.mark.parametrize("hq, hkv, hd", [(4, 2, 16), (3, 1, 20), (2, 1, 256)])
+@pytest.mark.parametrize("dtype", [F32, BF16])
+@pytest.mark.parametrize("window", [0, 1, 64, 65, 130])
+@pytest.mark.parametrize("keys", [50, 64, 100, 240, 600])
+def test_attention_plain_waves_of_a_block(hq, hkv, hd, dtype, window, keys):
+    """However many of a block's waves share a row's keys (the table's width and the window say how many there may be,
+    the count of rows how many the launcher likes), the bits are the same."""
+    from sonicboom_amd import ops
+    pages = (keys + 63) // 64
+    table = torch.randperm(pages, generator=torch.Generator().manual_seed(1)).int()[None]
+    kc, vc = (randn(pages, hkv, 64, hd, seed=2).to(dtype).to(DEV), randn(pages, hkv, hd, 64, seed=3).to(dtype).to(DEV))
+    rows = [0, 1, min(63, keys - 1), min(64, keys - 1), keys // 2, keys - 1]
+    outs = []
+    for extra, times in ((0, 1), (3, 1), (9, 1), (0, 200)):
+        t = torch.cat([table, torch.full((1, extra), -1, dtype=torch.int32)], 1).to(DEV)
+        q = randn(len(rows), hq * hd, seed=4).to(dtype).repeat(times, 1).to(DEV)
+        pos = torch.tensor(rows * times, dtype=torch.int32, device=DEV)
+        outs.append(ops.attention_plain(q, kc, vc, t, pos, torch.zeros_like(pos), hq, hkv, hd, hd ** -0.5, window))
+    assert all(torch.equal(outs[0], o[:len(rows)]) and torch.equal(o[-len(rows):], outs[0]) for o in outs)
+
+
 @pytest.mark.parametrize("dtype", [F32, BF16])
 @pytest.mark.parametrize("hd", [20, 64])
 @pytest.mark.parametrize("gone", [[64], [70], [64, 130], list(range(64, 128)), list(range(128, 140))])
