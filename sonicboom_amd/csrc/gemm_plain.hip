@@ -275,9 +275,100 @@ int launch_packed_tiles(const float *x, const float *w, const PlainArgs &a, int 
   return launch_packed<2, 1, G>(x, w, a, n_seg, s);
 }
 
-// Every type, any inner size and alignment: loads element by element.
+// The same sums with a chain a thread: 64 x 64 tiles staged in LDS, every element of X and W read once a tile.
+constexpr int kTile = 64;        // rows and columns of a block's tile
+constexpr int kStage = 16;       // k per stage; a segment is a whole number of stages
+constexpr int kTileThreads = 256;
+
+// Several segments' sums wait in LDS, a place a thread, but for a row of four: seven blocks then share a CU, with all in
+// registers five (2,048 rows against 3,584 x 3,584: 894 us), with all in LDS six (1,040).
+template <typename TX, typename TW, bool SEGMENTS>
+__global__ void __launch_bounds__(kTileThreads)
+gemm_tile_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a) {
+  __shared__ float xs[kStage][kTile + 4];
+  __shared__ float ws[kStage][kTile + 4];
+  __shared__ float total[SEGMENTS ? 12 : 1][kTileThreads];
+  const unsigned tiles_n = (a.n_out + kTile - 1) / kTile;
+  const int t0 = int(blockIdx.x / tiles_n) * kTile, n0 = int(blockIdx.x % tiles_n) * kTile;
+  const int tid = threadIdx.x, ty = tid / 16, tx = tid % 16;
+  float acc[4][4], last[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
+  for (int k0 = 0; k0 < a.n_in; k0 += kStage) {
+    if (SEGMENTS && k0 > 0 && k0 % kSegment == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (i < 3) total[4 * i + j][tid] = k0 > kSegment ? total[4 * i + j][tid] + acc[i][j] : acc[i][j];
+          else last[j] = last[j] + acc[i][j];
+          acc[i][j] = 0.0f;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int e = tid + i * kTileThreads;
+      const int r = e / kStage, k = e % kStage;
+      const int gk = k0 + k, gt = t0 + r, gn = n0 + r;
+      xs[k][r] = gt < a.n_rows && gk < a.n_in ? ld_f(x, size_t(gt) * a.n_in + gk) : 0.0f;
+      ws[k][r] = gn < a.n_out && gk < a.n_in ? ld_f(w, size_t(gn) * a.n_in + gk) : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kStage; ++k) {
+      float p[4], q[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) p[i] = xs[k][ty * 4 + i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) q[j] = ws[k][tx * 4 + j];
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(p[i], q[j], acc[i][j]);
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int t = t0 + ty * 4 + i;
+    if (t >= a.n_rows) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int n = n0 + tx * 4 + j;
+      if (n >= a.n_out) continue;
+      float v = !SEGMENTS ? acc[i][j] : i < 3 ? total[4 * i + j][tid] + acc[i][j] : last[j] + acc[i][j];
+      if (a.bias) v = v + ld_dyn(a.bias, a.bias_dtype, n);
+      const size_t idx = size_t(t) * a.n_out + n;
+      if (a.resid) v = v + a.resid[idx];
+      if (a.y_dtype == SB_F32) ((float *)a.y)[idx] = v;
+      else ((bf16_t *)a.y)[idx] = f32_to_bf16(v);
+    }
+  }
+}
+
+// Every type, any inner size and alignment: loads element by element.  The matrix-core form reads X and W once for every
+// 32 x 16 tile, an element a lane and load, 10 to 30 segments of such a tile a microsecond; the form above walks K at
+// 0.075 us a k with a tile or less a CU and 0.03 more for every tile a CU, and is ahead once there are many: float32,
+// 2,048 rows against 3,584 x 3,584 0.81 ms (matrix cores 4.07), bfloat16 0.72 (4.37), one row against 151,936 x 896 254 us
+// (436), 300 against 4,000 x 4,001 587 (814); behind with few: one row against 896 x 4,864 362 us (43), 64 against 4,096 x
+// 20,000 2,908 (822), 300 against 900 x 1,001 123 (44).
 template <typename TX, typename TW>
 int launch_any(const TX *x, const TW *w, const PlainArgs &a, int n_seg, hipStream_t s) {
+  const bool f32 = sizeof(TX) == 4 && sizeof(TW) == 4;
+  const double tiles = double((a.n_rows + kTile - 1) / kTile) * ((a.n_out + kTile - 1) / kTile);
+  const double segments = double((a.n_rows + 31) / 32) * ((a.n_out + 15) / 16) * (a.n_in / double(kSegment));
+  const double tile_us = a.n_in * (0.075 + 0.03 * tiles / 256.0);
+  const double mfma_us = segments / (!f32 ? 11.0 : a.n_rows <= 32 ? 30.0 : 17.0);
+  const double wave_us = (f32 ? 28.0 : 65.0) * (n_seg > 1 ? 1.0 : a.n_in / double(kSegment));      // one wave's segment
+  if (tile_us < (mfma_us > wave_us ? mfma_us : wave_us)) {
+    const long long blocks = (long long)tiles;
+    SB_SUPPORT(blocks <= 0x7fffffffLL, "sb_gemm: too many tiles");
+    if (n_seg == 1) gemm_tile_kernel<TX, TW, false><<<unsigned(blocks), kTileThreads, 0, s>>>(x, w, a);
+    else gemm_tile_kernel<TX, TW, true><<<unsigned(blocks), kTileThreads, 0, s>>>(x, w, a);
+    return sb::check_launch("sb_gemm");
+  }
   if (n_seg == 1) return launch_one<TX, TW, kAny, 2, 1, 1, 1>(x, w, a, s);
   return launch_one<TX, TW, kAny, 2, 1, 1, 8>(x, w, a, s);
 }

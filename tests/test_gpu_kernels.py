@@ -131,6 +131,20 @@ def test_gemm_plain_does_not_depend_on_the_batch():
         assert torch.equal(alone[0], whole[r])
 
 
+@pytest.mark.parametrize("t, n, k", [(2100, 520, 1100), (1030, 1100, 2060), (2048, 768, 64), (3, 33000, 2050)])
+@pytest.mark.parametrize("xd, wd", [(F32, F32), (BF16, BF16), (BF16, F32), (F32, BF16)])
+def test_gemm_plain_many_rows_give_the_bits_of_one(t, n, k, xd, wd):
+    """The form for many tiles and the form for few: the same bits of every element, over several segments of K."""
+    from sonicboom_amd import ops
+    x, w, bias, resid = randn(t, k).to(xd).to(DEV), randn(n, k, scale=0.05).to(wd).to(DEV), randn(n).to(DEV), randn(t, n).to(DEV)
+    whole = ops.gemm_plain(x, w, bias, resid, F32)
+    rows = [0, 1, t // 2, t - 1]
+    close(whole[rows], ref_gemm(x[rows].cpu(), w.cpu(), bias.cpu(), resid[rows].cpu()), atol=2e-5 * math.sqrt(k), rtol=1e-5)
+    for cols in (slice(0, 200), slice(n - 100, n)):
+        few = ops.gemm_plain(x[rows], w[cols].contiguous(), bias[cols].contiguous(), resid[rows][:, cols].contiguous(), F32)
+        assert torch.equal(whole[rows][:, cols], few)
+
+
 @pytest.mark.parametrize("t, n, k", [(1, 16, 16), (3, 70, 33), (16, 33, 1020), (17, 300, 1024), (33, 130, 1025), (64, 257, 2052),
                                      (65, 64, 4864), (2, 12300, 48), (700, 272, 9000)])
 def test_gemm_f32_packed_gives_the_bits_of_the_plain_product(t, n, k):
