@@ -54,14 +54,19 @@ class Linear:
             raise RuntimeError("this projection only keeps its packed weight")
         return self.weight
 
+    @staticmethod
+    def _bf16_rows(x: torch.Tensor) -> torch.Tensor:
+        """Rows as the matrix-core kernels take them: bfloat16, starting on 16 bytes."""
+        if x.dtype != torch.bfloat16:
+            return ops.cast(x, torch.bfloat16)
+        return x if x.data_ptr() % 16 == 0 else x.clone()
+
     def __call__(self, x: torch.Tensor, out_dtype: torch.dtype, resid: Optional[torch.Tensor] = None,
                  out: Optional[torch.Tensor] = None) -> torch.Tensor:
         if self.gated:
             return self.gated_product(x, out_dtype)
         if self.packed is not None:
-            if x.dtype != torch.bfloat16:
-                x = ops.cast(x, torch.bfloat16)
-            return ops.gemm_bf16(x, self.packed, self.bias, resid, out_dtype, out,
+            return ops.gemm_bf16(self._bf16_rows(x), self.packed, self.bias, resid, out_dtype, out,
                                  packed_shape=(self.rows, self.n_in))
         if self.packed_f32 is not None:
             return ops.gemm_f32(ops.cast(x, torch.float32), self.packed_f32, self.bias, resid, out_dtype,
@@ -106,7 +111,7 @@ class Linear:
     def joins(self, x: torch.Tensor, then_norm) -> bool:
         """Whether join() takes the call."""
         return self.packed is not None and not self.gated and x.dtype == torch.bfloat16 and x.shape[0] <= ops.SPLIT_MAX_ROWS \
-            and self.n_in % 8 == 0 and ops.launchers_choose() and getattr(then_norm, "fusable", False) and int(then_norm.groups) == 1
+            and x.data_ptr() % 16 == 0 and ops.launchers_choose() and getattr(then_norm, "fusable", False) and int(then_norm.groups) == 1
 
     def join(self, x: torch.Tensor, resid: torch.Tensor, then_norm) -> "ops.ScaledRows":
         """resid += x W^T (+ b); returns then_norm(resid) but for the rows' factors, for gated_product() to finish."""
@@ -132,9 +137,7 @@ class Linear:
         if isinstance(x, ops.ScaledRows):
             return ops.gemm_split_gated(x, self.packed, gated=self.activation, packed_shape=(self.rows, self.n_in))
         if self.packed is not None:
-            if x.dtype != torch.bfloat16:
-                x = ops.cast(x, torch.bfloat16)
-            return ops.gemm_bf16(x, self.packed, None, None, out_dtype, gated=self.activation,
+            return ops.gemm_bf16(self._bf16_rows(x), self.packed, None, None, out_dtype, gated=self.activation,
                                  packed_shape=(self.rows, self.n_in))
         if self.packed_f32 is not None:
             return ops.gemm_f32(ops.cast(x, torch.float32), self.packed_f32, None, None, out_dtype,

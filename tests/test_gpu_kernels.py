@@ -1209,6 +1209,27 @@ def test_the_norm_between_two_products_sums_in_double():
     assert ((got - torch.relu(g) * u).abs() <= (torch.relu(g) * u).abs() * 2.0 ** -8 + 1.2 * (sg * u.abs() + su * g.abs()) + 1e-5).all()
 
 
+def test_projections_of_rows_off_sixteen_bytes():
+    """Rows that start between two 16-byte lines: whole, gated, and joined to the stream with a norm to follow, where the
+    product that carries the norm stands back."""
+    from types import SimpleNamespace
+    from sonicboom_amd import ops
+    from sonicboom_amd.parts.linear import Linear
+    rows, n_in, width = 3, 96, 104
+    x, w = randn(rows, n_in).to(BF16).to(DEV), randn(width, n_in, scale=0.1, seed=1).to(BF16).to(DEV)
+    off = torch.empty(rows * n_in + 4, dtype=BF16, device=DEV)[4:].view(rows, n_in).copy_(x)
+    assert off.data_ptr() % 16 == 8
+    norm = SimpleNamespace(fusable=True, groups=1, weight=None, eps=1e-6)
+    lin = Linear(w, None)
+    assert lin.joins(x, norm) and not lin.joins(off, norm)
+    for rows_ in (x, off):
+        resid = torch.ones(rows, width, device=DEV)
+        lin.add_into(rows_, resid, norm, BF16)
+        close(resid, ref_gemm(x.cpu(), w.cpu()) + 1.0, atol=1e-4, rtol=1e-5, what="joined")
+    gated = Linear(w, None, gated=True)
+    assert torch.equal(gated(off, F32), gated(x, F32)) and torch.equal(lin(off, F32), lin(x, F32))
+
+
 FOLDED_SHAPES = [(4, 2, 16, 16), (3, 1, 32, 32), (5, 5, 48, 16), (6, 2, 80, 64), (28, 4, 128, 128), (16, 1, 64, 0),
                  (2, 1, 256, 256)]
 
