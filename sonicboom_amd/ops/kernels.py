@@ -642,6 +642,8 @@ def gemm_split_gated(x: ScaledRows, w: torch.Tensor, gated, packed_shape) -> tor
     rows, ssq = x.values, x.ssq
     _dev(rows, ssq, w)
     n, k, t = packed_shape[0] // 2, packed_shape[1], rows.shape[0]
+    if ssq.dtype != torch.float64 or ssq.dim() != 2 or ssq.shape[1] != t:
+        raise KernelLibraryError("the sums of squares must be float64 [parts, rows]")
     if w.dtype != torch.bfloat16 or rows.dim() != 2 or rows.shape[1] != k or packed_shape[0] % 2:
         raise KernelLibraryError(f"gemm shapes do not match: x {tuple(rows.shape)}, w {tuple(packed_shape)}")
     out = torch.empty((t, n), dtype=torch.bfloat16, device=rows.device)
@@ -662,8 +664,6 @@ def reduce_resid_norm(partial: torch.Tensor, bias: Optional[torch.Tensor], x: to
         raise KernelLibraryError("reduce_resid_norm needs float32 slices [s, rows, width] and a residual [rows, width]")
     s_, t, width = partial.shape
     if bias is not None and bias.numel() != width:
-    if ssq.dtype != torch.float64 or ssq.dim() != 2 or ssq.shape[1] != t:
-        raise KernelLibraryError("the sums of squares must be float64 [parts, rows]")
         raise KernelLibraryError("bias does not match the row width")
     if norm_weight is not None and norm_weight.numel() != width:
         raise KernelLibraryError("norm weight does not match the row width")
