@@ -606,6 +606,26 @@ STREAM_MIN_BLOCKS = 136
 
 # Rows of a decode step up to which the norm between attention and the feed-forward rides in the products around it
 SPLIT_MAX_ROWS = 8
+SPLIT_CUS = 256
+SPLIT_FULL = 0.87
+SPLIT_SMALL = 20 << 20
+
+
+def split_norm_pays(rows: int, width: int, inner: int) -> bool:
+    """Whether :func:`gemm_split_join` and :func:`gemm_split_gated` are ahead of the two products with the norm as a pass
+    between them.  A block of theirs owns sixteen features whole, so they want the blocks' rounds over the CUs nearly full
+    (the joining product: a single round, or up to four rows); a gated product of up to 20 M weights is so short that the pass
+    saved decides.  Measured, both products and the norm, replayed graphs with the weights cold, at 1 / 4 / 8 rows (us, before ->
+    after): 896 x 4,864 13.9 -> 11.8, 14.3 -> 12.0, 14.6 -> 12.2; 1,536 x 8,960 21.0 -> 19.8, 21.0 -> 20.3, 21.2 -> 21.0; 2,048 x
+    11,008 28.2 -> 26.3, 27.3 -> 26.3, 27.8 -> 27.2; 3,584 x 18,944 63.3 -> 58.2, 62.8 -> 57.6, 60.9 -> 59.9; 8,192 x 29,568 209
+    -> 199, 209 -> 202, and at eight rows, not taken, 201 -> 202.  Not taken either: 5,120 x 13,824 (320 blocks join, 864 gate)
+    68.7 -> 71.0, 68.4 -> 73.0, 65.7 -> 73.3; 4,608 x 8,960 46.8 -> 49.0, 47.0 -> 50.4, 47.4 -> 52.7; 3,072 x 13,824 42.0 -> 43.2,
+    42.1 -> 43.9, 40.7 -> 44.2; 3,072 x 8,960 34.0 -> 33.0, 32.6 -> 33.1, 32.8 -> 34.6; 7,168 x 18,944 at eight rows 117 -> 121."""
+    def full(features: int) -> bool:
+        rounds = -(-features // 16) / SPLIT_CUS
+        return rounds >= SPLIT_FULL * math.ceil(rounds)
+    return rows <= SPLIT_MAX_ROWS and (width <= 16 * SPLIT_CUS or (rows <= 4 and full(width))) \
+        and (width * inner <= SPLIT_SMALL or full(inner))
 
 
 class ScaledRows:

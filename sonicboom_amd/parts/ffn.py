@@ -67,7 +67,8 @@ class GatedDenseFFN(Part):
     def takes_unfinished(self, ctx) -> bool:
         """Whether forward() also takes what Linear.join() returns: in decode steps (what a prompt step launches is
         written down a second time for steps made in one call)."""
-        return ctx.is_decode and self.gate_up.packed is not None and self.rt.act_dtype == torch.bfloat16 and self.gate_up.n_in % 8 == 0
+        return ctx.is_decode and self.gate_up.packed is not None and self.rt.act_dtype == torch.bfloat16 \
+            and ops.split_norm_pays(ctx.n_rows, self.width, self.inner)
 
     def forward(self, h, x, ctx, then_norm=None):
         """x += out_scale * ffn(h).  Returns then_norm(x) when the down projection could apply the

@@ -1209,6 +1209,37 @@ def test_the_norm_between_two_products_sums_in_double():
     assert ((got - torch.relu(g) * u).abs() <= (torch.relu(g) * u).abs() * 2.0 ** -8 + 1.2 * (sg * u.abs() + su * g.abs()) + 1e-5).all()
 
 
+@pytest.mark.parametrize("width, heads, inner, rows", [(128, 2, 320, 9), (5120, 40, 320, 1), (8192, 64, 320, 4), (8192, 64, 320, 5)])
+def test_decode_steps_on_both_sides_of_the_rule_for_the_norm(width, heads, inner, rows):
+    """The norm rides in the products, or is a pass between them: the same logits but for the order of a norm's factor and of
+    sums, and the rule asks for what the sizes take."""
+    from sonicboom_amd import ops
+    from sonicboom_amd.engine import DecoderModel, Engine, StepEntry
+    from sonicboom_amd.ops import kernels
+    cfg = {"architectures": ["Qwen2ForCausalLM"], "num_hidden_layers": 2, "hidden_size": width, "num_attention_heads": heads,
+           "num_key_value_heads": 1, "intermediate_size": inner, "vocab_size": 300, "rope_theta": 10000.0, "rms_norm_eps": 1e-6,
+           "max_position_embeddings": 256, "tie_word_embeddings": True}
+    model = DecoderModel.from_random(cfg, 3, "bfloat16", DEV)
+    eng = Engine(model, 64 * rows, max_slots=rows)
+    joined = []
+    real = kernels.gemm_split_join
+    rides = ops.split_norm_pays(rows, width, inner)
+    assert rides == (rows <= 8 and (width <= 4096 or (width == 8192 and rows <= 4)))
+    out = []
+    for most in (kernels.SPLIT_MAX_ROWS, 0):
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setattr(ops, "gemm_split_join", lambda *a, **k: (joined.append(most), real(*a, **k))[1])
+            mp.setattr(kernels, "SPLIT_MAX_ROWS", most)
+            slots = [eng.alloc_slot() for _ in range(rows)]
+            eng.step([StepEntry(s, [5 + i, 7], ()) for i, s in enumerate(slots)])
+            out.append(eng.step([StepEntry(s, [11 + i], (0,)) for i, s in enumerate(slots)]).float().cpu())
+            for s in slots:
+                eng.free_slot(s)
+    assert joined == ([kernels.SPLIT_MAX_ROWS] * 2 if rides else [])
+    # a rounding of the normed rows to bfloat16 (2^-9) at another place in each of two layers
+    assert (out[0] - out[1]).abs().max() <= 0.05 * out[0].std()
+
+
 def test_projections_of_rows_off_sixteen_bytes():
     """Rows that start between two 16-byte lines: whole, gated, and joined to the stream with a norm to follow, where the
     product that carries the norm stands back."""
