@@ -198,7 +198,7 @@ class Engine:
         self.bindings = model.bindings(self.cache)
         self.use_graphs = True
         self._loop = None
-        # a model that is a run of like dense layers launches all of a short prompt step's layers in one call
+        # like dense layers are launched by one call each in a short prompt step
         self.one_call_layers = True
         # set to a callable (name, tensor) to receive a step's named intermediates, in the order of
         # the computation: "embedding", "entry<i>.after_mixer", "entry<i>.after_ffn", "logits"
@@ -317,17 +317,19 @@ class Engine:
         x = model.embedding.forward(ctx.ids, ctx)
         if tracer is not None:
             tracer("embedding", x)
+        run = None
         if tracer is None and self.one_call_layers and dense.takes_step(ctx):
             run = dense.DenseLayers.of(model, self.bindings)
-            if run is not None:
-                run(x, ctx)
-                return self._finish(x, ctx)
+            run = run if run is not None and run.pays(ctx.n_rows) else None
         h = None
         for junction in model.junctions:
             h = junction.begin(x, ctx)
         if not model.order or model.order[0].junction is None:
             h = None                           # (a block reads its own norm of x)
         for i, e in enumerate(model.order):
+            if run is not None and run.takes(i):
+                h = run.layer(i, x, ctx, h)
+                continue
             if e.junction is not None:
                 h = model.junctions[e.junction].forward(x, ctx, e.turn, h=h,
                                                         next_norm=getattr(model.blocks[e.block], "first_norm", None))

@@ -724,36 +724,47 @@ class _DenseStep(ctypes.Structure):
                                                "n_tiles", "tile_rows")])
 
 
-def dense_layers(x: torch.Tensor, h: torch.Tensor, layers, inner: int, heads_q: int, heads_kv: int, head_dim: int,
-                 page_table: torch.Tensor, n_pages: int, row_pos: torch.Tensor, row_seq: torch.Tensor, tiles: torch.Tensor,
-                 tile_rows: int) -> None:
-    """Decoder layers (a ctypes array of :class:`DenseLayer`) over a step's rows in one call of the library: ``x`` float32
-    [rows, width] in place, ``h`` bfloat16 the first layer's norm of it (overwritten)."""
-    _dev(x, h, page_table, row_pos, row_seq, tiles)
-    t, width = x.shape
-    if x.dtype != torch.float32 or h.dtype != torch.bfloat16 or tuple(h.shape) != (t, width):
-        raise KernelLibraryError("dense_layers takes the float32 stream and its first norm in bfloat16")
-    _check_rows(row_pos, row_seq, page_table, t)
-    if tiles.dtype != torch.int32 or tiles.dim() != 2 or tiles.shape[1] != 4:
-        raise KernelLibraryError("tiles must be int32 [n, 4]")
-    lib, attn = library.core(), library.attention_library(head_dim)
-    q_width = heads_q * head_dim
-    floats = lib.sb_dense_layers_floats(t, width, q_width + 2 * heads_kv * head_dim, q_width, inner)
-    # one allocation for what the layers hand from kernel to kernel, each part on 256 bytes
-    sizes = [4 * floats, 2 * t * q_width, 2 * t * q_width, 2 * t * inner]
-    offsets = [0]
-    for n in sizes:
-        offsets.append(offsets[-1] + (n + 255) // 256 * 256)
-    work = torch.empty((offsets[-1],), dtype=torch.uint8, device=x.device)
-    base = work.data_ptr()
-    step = _DenseStep(x=x.data_ptr(), h=h.data_ptr(), part=base, part_floats=floats, q=base + offsets[1], att=base + offsets[2],
-                      mid=base + offsets[3],
-                      attention=ctypes.cast(attn.sb_attn_prefill_bf16, ctypes.c_void_p),
-                      attention_error=ctypes.cast(attn.sb_attn_last_error, ctypes.c_void_p),
-                      row_pos=row_pos.data_ptr(), row_seq=row_seq.data_ptr(), page_table=page_table.data_ptr(), tiles=tiles.data_ptr(),
-                      n_rows=t, width=width, inner=inner, heads_q=heads_q, heads_kv=heads_kv, head_dim=head_dim,
-                      max_pages=page_table.shape[1], n_pages=n_pages, n_tiles=tiles.shape[0], tile_rows=int(tile_rows))
-    check(lib.sb_dense_layers(ctypes.addressof(step), ctypes.addressof(layers), len(layers), _stream()))
+class DenseStep:
+    """What the like decoder layers of a prompt step share: the stream ``x`` float32 [rows, width], the step's tables and a
+    workspace for what a layer hands from kernel to kernel.  Launches on the stream that is current when it is made."""
+
+    def __init__(self, x: torch.Tensor, inner: int, heads_q: int, heads_kv: int, head_dim: int, page_table: torch.Tensor, n_pages: int,
+                 row_pos: torch.Tensor, row_seq: torch.Tensor, tiles: torch.Tensor, tile_rows: int):
+        _dev(x, page_table, row_pos, row_seq, tiles)
+        t, width = x.shape
+        if x.dtype != torch.float32:
+            raise KernelLibraryError("the stream must be float32 [rows, width]")
+        _check_rows(row_pos, row_seq, page_table, t)
+        if tiles.dtype != torch.int32 or tiles.dim() != 2 or tiles.shape[1] != 4:
+            raise KernelLibraryError("tiles must be int32 [n, 4]")
+        self.lib, attn = library.core(), library.attention_library(head_dim)
+        q_width = heads_q * head_dim
+        floats = self.lib.sb_dense_layers_floats(t, width, q_width + 2 * heads_kv * head_dim, q_width, inner)
+        # one allocation, each part on 256 bytes
+        sizes = [4 * floats, 2 * t * q_width, 2 * t * q_width, 2 * t * inner]
+        offsets = [0]
+        for n in sizes:
+            offsets.append(offsets[-1] + (n + 255) // 256 * 256)
+        work = torch.empty((offsets[-1],), dtype=torch.uint8, device=x.device)
+        base = work.data_ptr()
+        self.kept = (x, page_table, row_pos, row_seq, tiles, work)
+        self.shape, self.stream = (t, width), _stream()
+        self.args = _DenseStep(x=x.data_ptr(), part=base, part_floats=floats, q=base + offsets[1], att=base + offsets[2],
+                               mid=base + offsets[3],
+                               attention=ctypes.cast(attn.sb_attn_prefill_bf16, ctypes.c_void_p),
+                               attention_error=ctypes.cast(attn.sb_attn_last_error, ctypes.c_void_p),
+                               row_pos=row_pos.data_ptr(), row_seq=row_seq.data_ptr(), page_table=page_table.data_ptr(), tiles=tiles.data_ptr(),
+                               n_rows=t, width=width, inner=inner, heads_q=heads_q, heads_kv=heads_kv, head_dim=head_dim,
+                               max_pages=page_table.shape[1], n_pages=n_pages, n_tiles=tiles.shape[0], tile_rows=int(tile_rows))
+
+    def run(self, layer: DenseLayer, h: torch.Tensor) -> None:
+        """A layer on the stream in place; ``h`` bfloat16 [rows, width] its norm of the stream, then the next norm, if the layer
+        names one."""
+        _dev(h)
+        if h.dtype != torch.bfloat16 or tuple(h.shape) != self.shape:
+            raise KernelLibraryError("the layer's norm of the stream must be bfloat16 [rows, width]")
+        self.args.h = h.data_ptr()
+        check(self.lib.sb_dense_layers(ctypes.addressof(self.args), ctypes.addressof(layer), 1, self.stream))
 
 
 def launchers_choose() -> bool:

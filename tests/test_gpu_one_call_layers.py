@@ -37,6 +37,41 @@ def test_one_call_gives_the_same_bits(cfg):
     assert DenseLayers.of(model, engines[0].bindings) is not None
 
 
+def same_bits(monkeypatch, cfg, steps, alter=None):
+    """Every step of more than single tokens takes one call a layer, whether it pays or not."""
+    from sonicboom_amd.engine import DecoderModel, Engine, StepEntry, dense
+    monkeypatch.setattr(dense.DenseLayers, "pays", lambda self, rows: True)
+    model = DecoderModel.from_random(cfg, 3, "bfloat16", "cuda:0")
+    if alter is not None:
+        alter(model)
+    engines = [Engine(model, 64 * 30, max_slots=4) for _ in range(2)]
+    engines[1].one_call_layers = False
+    rng = np.random.default_rng(5)
+    for lengths in steps:
+        tokens = [rng.integers(0, cfg["vocab_size"], size=n).tolist() for n in lengths]
+        slots = [[e.alloc_slot() for _ in lengths] for e in engines]
+        got, want = (e.step([StepEntry(s, t, (0, len(t) - 1)) for s, t in zip(ss, tokens)]) for e, ss in zip(engines, slots))
+        assert torch.equal(got, want), lengths
+        for e, ss in zip(engines, slots):
+            for s in ss:
+                e.free_slot(s)
+
+
+@pytest.mark.parametrize("other", [(0,), (1,), (2, 3), (1, 3)])
+def test_layers_that_differ_stand_between_those_that_do_not(monkeypatch, other):
+    """They run part by part, take the norm that the layer before has left and leave the next one's."""
+    def alter(model):
+        for i in other:
+            model.blocks[model.order[i].block].mixer.out_scale = 0.5
+    same_bits(monkeypatch, config(128, 2, 2, 320, layers=4), [[2, 3], [65], [7, 1, 200, 33]], alter)
+
+
+def test_long_steps_take_a_call_a_layer_too(monkeypatch):
+    """Sizes at which a call a layer would not pay."""
+    same_bits(monkeypatch, SIZES[1], [[700, 500], [1536]])
+    same_bits(monkeypatch, SIZES[3], [[129], [300, 41]])
+
+
 def test_other_models_and_choices_keep_their_parts():
     from sonicboom_amd import ops
     from sonicboom_amd.engine import DecoderModel, Engine, StepEntry
