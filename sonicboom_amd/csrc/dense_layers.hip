@@ -94,9 +94,13 @@ extern "C" size_t sb_dense_layers_floats(int n_rows, int width, int qkv_width, i
     const int s = raw_slices(n_rows, n_out, n_in);
     return size_t(s > 1 ? s : 1) * t * n_out;
   };
+  // (whole products of few rows cut K for themselves: the gated one, and those that join rows wider than one block norms)
+  const auto whole = [&](int n_out, int n_in, int gated) {
+    return n_rows <= kFewRows ? sb_gemm_skinny_scratch(n_rows, n_out, n_in, gated) : size_t(0);
+  };
   size_t most = sliced(qkv_width, width);
-  const size_t others[3] = {sliced(width, q_width), sliced(width, inner),
-                            n_rows <= kFewRows ? sb_gemm_skinny_scratch(n_rows, inner, width, 1) : 0};
+  const size_t others[5] = {sliced(width, q_width), sliced(width, inner), whole(inner, width, 1), whole(width, q_width, 0),
+                            whole(width, inner, 0)};
   for (size_t o : others) most = o > most ? o : most;
   return most;
 }

@@ -57,6 +57,11 @@ def same_bits(monkeypatch, cfg, steps, alter=None):
                 e.free_slot(s)
 
 
+def test_rows_wider_than_the_pass_that_adds_slices(monkeypatch):
+    """The products that join such rows are whole ones, whose own cuts of K need more of the workspace than any slices do."""
+    same_bits(monkeypatch, config(14464, 113, 1, 64, layers=1), [[3], [16], [2, 30], [70]])
+
+
 @pytest.mark.parametrize("other", [(0,), (1,), (2, 3), (1, 3)])
 def test_layers_that_differ_stand_between_those_that_do_not(monkeypatch, other):
     """They run part by part, take the norm that the layer before has left and leave the next one's."""
