@@ -189,6 +189,12 @@ def gemm_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], res
         out = torch.empty((t, n), dtype=out_dtype, device=x.device)
     elif out.dtype != out_dtype or tuple(out.shape) != (t, n):
         raise KernelLibraryError("gemm output buffer has the wrong shape or type")
+    if k > 256 and (k % 4 or x.data_ptr() % 16):
+        # Rows that cannot be read sixteen bytes at a time are copied, with zeros up to a multiple of four (the weight's blocks
+        # hold zeros there): the same sums.  Read a number at a time they took (us, copy and product in brackets) 21 (16) at
+        # 1 x 896 x 901, 387 (158) at 300 x 4,000 x 4,001, 1,977 (489) at 2,048 x 3,584 x 3,583; at 2,048 x 320 x 102 9 (17).
+        x = torch.nn.functional.pad(x, (0, -k % 4)) if k % 4 else x.clone()
+        k = x.shape[1]
     check(library.core().sb_gemm_f32_packed(_p(out), _dt(out), _p(x), _p(w), _p(bias), _dt(bias) if bias is not None else 0,
                                             _p(resid), t, n, k, gate, _stream()))
     return out

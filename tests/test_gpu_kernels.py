@@ -131,6 +131,19 @@ def test_gemm_plain_does_not_depend_on_the_batch():
         assert torch.equal(alone[0], whole[r])
 
 
+@pytest.mark.parametrize("t, n, k", [(3, 100, 255), (3, 100, 257), (300, 272, 1003), (70, 64, 1022), (2, 48, 4097)])
+def test_gemm_f32_of_rows_off_sixteen_bytes(t, n, k):
+    """Inner sizes that are no multiple of four, and rows that start between two lines of sixteen bytes: the bits of the plain
+    product, plain and gated."""
+    from sonicboom_amd import ops
+    x, w, bias = randn(t, k).to(DEV), randn(n, k, scale=0.05).to(DEV), randn(n).to(DEV)
+    off = torch.empty(t * k + 1, device=DEV)[1:].view(t, k).copy_(x)
+    want, both = ops.gemm_plain(x, w, bias, None, F32), ops.gemm_plain(x, w, None, None, F32)
+    for rows in (x, off):
+        assert torch.equal(ops.gemm_f32(rows, ops.pack_weight_f32(w), bias, None, F32, (n, k)), want)
+        assert torch.equal(ops.gemm_f32(rows, ops.pack_weight_f32(w, True), None, None, F32, (n, k), gated="silu"), ops.silu_mul(both, F32))
+
+
 @pytest.mark.parametrize("t, n, k", [(2100, 520, 1100), (1030, 1100, 2060), (2048, 768, 64), (3, 33000, 2050)])
 @pytest.mark.parametrize("xd, wd", [(F32, F32), (BF16, BF16), (BF16, F32), (F32, BF16)])
 def test_gemm_plain_many_rows_give_the_bits_of_one(t, n, k, xd, wd):
