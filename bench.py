@@ -173,14 +173,14 @@ class OpTimer:
     times are summed by (function, what it worked on)."""
 
     NAMES = ("embed", "rmsnorm", "gemm_bf16", "gemm_bf16_partial", "gemm_split_join", "gemm_split_gated", "reduce_resid_norm", "rope_kv_store",
-             "attention", "attention_decode_rope", "argmax", "gemm_plain", "silu_mul", "add_into", "cast")
+             "attention", "attention_decode_rope", "argmax", "gemm_plain", "gemm_f32", "silu_mul", "add_into", "cast")
 
     def __init__(self, m):
         self.m, self.records, self._saved = m, [], {}
 
     def _label(self, name, args, kw):
         m = self.m
-        if name.startswith(("gemm_bf16", "gemm_split")):
+        if name.startswith(("gemm_bf16", "gemm_split", "gemm_f32")):
             n, k = kw.get("packed_shape") or (args[1].shape[0], args[1].shape[-1])
             if kw.get("gated"):
                 return "gate_up"
@@ -890,7 +890,10 @@ def design_roofline(label, us, calls, rows, depth, batch, width, cfgs):
         n, k = (int(v) for v in label.split()[-1].split("x"))
         if n == cfgs["vocab"] and not decode:
             rows = 1                     # the head runs on the wanted rows only: the prompt's last
-        nbytes, flops = 2 * n * k + 2 * rows * k + 4 * rows * (n // (2 if "gated" in label else 1)), 2 * rows * n * k
+        size = 4 if label.startswith("gemm_f32") else 2          # bytes of a weight and of a row's number
+        nbytes, flops = size * (n * k + rows * k) + 4 * rows * (n // (2 if "gated" in label else 1)), 2 * rows * n * k
+        if size == 4:
+            peak_f = VECTOR_F32_FLOPS                            # (the float32 matrix cores' as well)
     elif label.startswith("rmsnorm") or label == "reduce_resid_norm":
         nbytes = rows * width * (4 + 2 + (8 if label == "reduce_resid_norm" else 0))
     elif label == "mingru_scan":

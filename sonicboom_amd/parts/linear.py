@@ -69,8 +69,8 @@ class Linear:
             return ops.gemm_bf16(self._bf16_rows(x), self.packed, self.bias, resid, out_dtype, out,
                                  packed_shape=(self.rows, self.n_in))
         if self.packed_f32 is not None:
-            return ops.gemm_f32(ops.cast(x, torch.float32), self.packed_f32, self.bias, resid, out_dtype,
-                                (self.rows, self.n_in), out)
+            return ops.gemm_f32(ops.cast(x, torch.float32), self.packed_f32, self.bias, resid, out_dtype, out=out,
+                                packed_shape=(self.rows, self.n_in))
         w = self._row_major()
         if w.dtype == torch.float32 and x.dtype != torch.float32:
             x = ops.cast(x, torch.float32)
@@ -140,8 +140,8 @@ class Linear:
             return ops.gemm_bf16(self._bf16_rows(x), self.packed, None, None, out_dtype, gated=self.activation,
                                  packed_shape=(self.rows, self.n_in))
         if self.packed_f32 is not None:
-            return ops.gemm_f32(ops.cast(x, torch.float32), self.packed_f32, None, None, out_dtype,
-                                (self.rows, self.n_in), gated=self.activation)
+            return ops.gemm_f32(ops.cast(x, torch.float32), self.packed_f32, None, None, out_dtype, gated=self.activation,
+                                packed_shape=(self.rows, self.n_in))
         w = self._row_major()
         if w.dtype == torch.float32 and x.dtype != torch.float32:
             x = ops.cast(x, torch.float32)
