@@ -441,6 +441,10 @@ def test_gemm_bf16_wide_matrix_with_few_rows(t):
     k = 64
     x = randn(t, k, dtype=BF16)
     edge = 4 * kernels.STREAM_MIN_BLOCKS
+    # (the library's choice does change there: 0 the stream kernel, 1 the one that splits K; both leave 65 rows and more of such sizes to the tiled one)
+    for gate, per in ((0, 32), (1, 16)):
+        took = [ops.library.core().sb_gemm_bf16_kernel(t, n, gate, 1) for n in (edge * per, edge * per - per)]
+        assert took == ([0, 1] if t <= 64 else [2, 2])
     for n in (edge * 32, edge * 32 - 32):
         w = randn(n, k, dtype=BF16, scale=0.05)
         got = ops.gemm_bf16(x.to(DEV), ops.pack_weight(w.to(DEV)), None, None, F32, packed_shape=(n, k))
