@@ -1,6 +1,7 @@
 // bf16 matrix product for many rows (prefill):  Y[t,n] = sum_k X[t,k] W[n,k]
 // on the matrix cores, with the model's epilogues fused: bias, float32
-// residual, gate activation, float32 or bfloat16 output.
+// residual, gate activation, float32 or bfloat16 output.  Three kernels: this one, of any inner size in
+// eights and weights of either layout, and two below it that load packed weights and rows straight into LDS.
 //
 // A block of 2 x NW waves owns a BM x BN tile of Y (128 x 128, 256 x 128 or
 // 256 x 256) and walks K in stages of BK.  Both operand tiles go
@@ -724,7 +725,8 @@ gemm_direct16_kernel(Args a) {
 // Measured, kernel above against this one: 3.6 % faster on the gate/up product of 2,048 x 37,888 x 3,584 (469 and 451 us),
 // 8 % on 6,398 x 2,048 x 11,008 (257 and 236), 3 % on 16,384 x 3,584 x 18,944 (1.87 and 1.81 ms), each by itself; in whole
 // prompt steps, back to back, 1 to 2.5 %.  What bounds it: with the loads left out 1.6 to 1.8 PFLOP/s, with the products left
-// out 0.55 of the time; the two together run at the clock that the chip's power allows.
+// out 0.55 of the time; why the two together reach 1.23 (2,048 x 37,888 x 3,584) is not settled: a library's product runs
+// 8,192 x 16,384 x 3,584 at 1.55 on the same card, so it is neither the clock nor the power alone.
 template <int GATED, bool PERSIST>
 __global__ void __launch_bounds__(512)
 gemm_pipe_kernel(Args a) {
@@ -1011,7 +1013,7 @@ constexpr Shape kShapes[6] = {{128, 128}, {256, 128}, {256, 256}, {128, 256}, {1
 // The tile shape for a problem: the one with the best product of three factors.  How fast the
 // shape's kernel runs on a full grid, relative to 128 x 128 (measured on MI355X at 2,048 to 16,384
 // rows of Qwen2.5-7B's four products: the 256 x 256 kernel, which loads straight into LDS, reaches
-// 1.19 to 1.31 PFLOP/s where the 128 x 128 one reaches 0.73 to 0.98; the same kernel with tiles of
+// 1.19 to 1.31 PFLOP/s (3 to 8 % more since it reads fragments ahead) where the 128 x 128 one reaches 0.73 to 0.98; the same kernel with tiles of
 // 192 rows takes 0.84 of the time for 0.75 of the outputs); the share of the tiles' rows
 // that are rows of Y; and the share of the last round of tiles over the CUs that is filled.
 // Some of what this decides at 2,048 rows: the output product (3,584 x 3,584) takes 256 x 128
