@@ -798,7 +798,7 @@ class AllOpsTimer:
     (function, what tells its calls apart: a product's matrix, the rows)."""
 
     SKIP = ("pack_weight", "read_bandwidth", "random_normal", "attention_row_tile", "attention_row_tiles",
-            "attention_tall_ok", "attention_tile_height", "launchers_choose", "pack_weight_f32", "attention_mfma_ok", "attention_decode_rope_ok", "gate_code", "reduce_resid_norm_ok",
+            "attention_tall_ok", "attention_tile_height", "attention_row_groups", "launchers_choose", "pack_weight_f32", "attention_mfma_ok", "attention_decode_rope_ok", "gate_code", "reduce_resid_norm_ok",
             "attention_decode_pages_per_wave", "attention_prefill_form", "gemm_tile_shape", "gemm_few_rows_kernel", "mingru_chunk_rows",
             "loaded_paths", "check", "latent_attention_mfma_ok", "capped_attention_mfma_ok", "moe_max_top", "moe_plan",
             "time_conv_max_taps", "state_scan_limits", "state_scan_chunk_rows", "shared_attention_mfma_ok", "decay_scan_max_side", "decay_scan_max_rank", "decay_chunk_rows",

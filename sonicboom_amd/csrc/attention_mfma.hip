@@ -1028,6 +1028,35 @@ attn_prefill_keys_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ q,
   }
 }
 
+// Whether that kernel is ahead of the form in which a block walks a tile's pages: a price for both, in us.  `blocks` of its
+// sixteen-row blocks are launched, of which `live` have rows; `most` pages are the longest walk, `mean` the mean over the
+// live blocks.  A block a CU is ahead for any walk.  Beyond, every head reads its pages for itself beside another block on the
+// CU, while the other form's time goes by the longest walk alone.  Fitted to both forms at 2,592 combinations of 15 head
+// layouts, 128 to 1,024 blocks and 1 to 12 pages, full tiles and tiles of nine rows, where the choice costs at most 1 % against
+// the walk; some of what it decides (walk, this kernel): heads of 64, 14 on 2: 672 blocks of 1 page 7.0 and 7.8, a prompt of
+// 1,000 rows 21.3 and 14.1; 16 on 16: 1,024 blocks of 1 page 5.6 and 8.7, of 16 causal pages 19.5 and 14.8; heads of 128, 28
+// on 4: 448 blocks of 1 page 9.2 and 9.5, of 4 13.1 and 11.9; heads of 96, 32 on 8: 512 blocks of 1 page 6.6 and 8.3, of 8 16.4
+// and 14.7.
+constexpr int kKeysMaxBlocks = HD <= 64 ? 1024 : 512;
+bool keys_ahead(int group, double blocks, double live, double most, double mean, bool window) {
+  if (blocks <= 256) return true;
+  if (blocks > kKeysMaxBlocks) return false;
+  const bool sparse = live * 4 <= blocks;        // tiles of 64 rows of which one group of sixteen is there
+  double keys, walk;
+  if (HD <= 32) {
+    keys = blocks <= 512 ? 5.0 + 0.25 * mean : 4.2 + blocks / 430 + mean * blocks / 2500;
+    walk = 4.2 + 0.62 * most;
+  } else if (HD <= 64) {
+    keys = sparse ? 5.2 + (blocks > 640 ? (blocks - 640) / 175 : 0.0) + 0.6 * mean
+           : blocks <= 512 ? 5.3 + 0.45 * mean : 6.0 + blocks / 480 + mean * blocks / 1024;
+    walk = (group >= 5 ? 5.9 + most : 4.7 + 0.92 * most) + (window ? 1.0 : 0.0);
+  } else {
+    keys = sparse ? 5.9 + (blocks > 384 ? (blocks - 384) / 110 : 0.0) + 0.6 * mean : 8.2 + mean * (0.75 + 0.2 * blocks / 512);
+    walk = group <= 4 ? 5.5 + 1.2 * most : group <= 6 ? 7.1 + 1.28 * most : 7.5 + 1.35 * most;
+  }
+  return keys < walk;
+}
+
 // ---------------------------------------------------------------------------------------------
 // Decode: one row per sequence.  Block (chunk, kv head x head tile, sequence); wave w of the
 // block takes page 4 * chunk + w; columns are the query heads of the kv head.
@@ -1921,14 +1950,31 @@ extern "C" int sb_attn_prefill_tile_rows(int heads_q, int heads_kv) {
   return group == 1 ? 64 : (group == 2 ? 32 : 16);
 }
 
+// Whether a step takes the kernel that cuts a tile's pages over a block's waves; the arguments as below.
+extern "C" int sb_attn_prefill_keys(int n_tiles, int tile_rows, int heads_q, int heads_kv, int max_pages, int window, int step_groups,
+                                    int step_pages) {
+  if (!kKeysOk || heads_kv <= 0 || heads_q % heads_kv) return 0;
+  const int group = heads_q / heads_kv;
+  const long long units = (long long)n_tiles * (tile_rows / 16) * heads_kv;
+  const double blocks = double((units + 7) / 8 * 8 * group);
+  const int seen = window > 0 ? (tile_rows + window - 2) / SB_PAGE + 2 : max_pages;      // pages that a tile sees at most
+  const double most = max_pages < seen ? max_pages : seen;
+  const double mean = step_groups > 0 && step_pages < most * step_groups ? double(step_pages) / step_groups : most;
+  const double live = step_groups > 0 ? double(step_groups) * heads_q : blocks;
+  return keys_ahead(group, blocks, live, most, mean, window > 0);
+}
+
 // q, out: bf16 [n_rows, heads_q * HD]; tiles int32 [n_tiles][4] = (first row, rows <= tile_rows,
 // sequence, 0), every tile inside one sequence and its rows at consecutive positions.  tile_rows:
 // 16, or what sb_attn_prefill_tile_rows gives for these heads.
+// step_groups, step_pages: the step's rows in groups of up to sixteen of a sequence, and the pages up to each group's last row
+// added up, for the choice between the kernels (0: not known).
 // form: 0, or a test's or a measurement's choice: 1 pages through the block one by one, 2 pages over the block's waves.
 extern "C" int sb_attn_prefill_bf16(void *out, const void *q, const void *k_cache, const void *v_cache,
                                     const int32_t *page_table, int max_pages, int n_pages_total,
                                     const int32_t *row_pos, const int32_t *tiles, int n_tiles, int heads_q,
-                                    int heads_kv, float scale, int window, int tile_rows, int form, void *stream) {
+                                    int heads_kv, float scale, int window, int tile_rows, int step_groups, int step_pages, int form,
+                                    void *stream) {
   int rc = check_common(out, q, k_cache, v_cache, page_table, row_pos, max_pages, n_pages_total, heads_q,
                         heads_kv, window, "sb_attn_prefill_bf16");
   if (rc != SB_OK) return rc;
@@ -1953,11 +1999,7 @@ extern "C" int sb_attn_prefill_bf16(void *out, const void *q, const void *k_cach
   if constexpr (kKeysOk) {
     const long long units = (long long)n_tiles * (tile_rows / 16) * heads_kv;
     const long long blocks = (units + 7) / 8 * 8 * group;
-    // Every head reads the pages for itself here, which pays while the blocks come in a round or two.  Two rounds at head
-    // sizes above 64: up to 512 blocks it is ahead or level (504: 14.2 -> 11.0 us; 24 sequences of 16 rows on 2,000 keys, 384
-    // blocks: 56.5 -> 55.1), at 560 behind (9.8 -> 12.0) or, with eight heads a kv head, still ahead (1,024: 32.3 -> 31.3).
-    // Up to 64 a page is half as long: 896 blocks 21.0 -> 13.8, 1,792 37.3 -> 34.4.
-    if (form == 2 || (form == 0 && blocks <= (HD <= 64 ? 1024 : 512))) {
+    if (form == 2 || (form == 0 && sb_attn_prefill_keys(n_tiles, tile_rows, heads_q, heads_kv, max_pages, window, step_groups, step_pages))) {
       SB_SUPPORT(blocks <= 0x7fffffffLL, "sb_attn_prefill_bf16: too many blocks");
       static bool raised_keys = false;
       if (kKeyLds > 48 * 1024 && !raised_keys) {

@@ -133,7 +133,7 @@ extern "C" int sb_dense_layers(const sb_dense_step *step, const sb_dense_layer *
                                   st.row_pos, st.row_seq, L.k_cache, L.v_cache, SB_BF16, st.page_table, st.max_pages, st.n_pages, t,
                                   st.heads_q, st.heads_kv, st.head_dim, st.head_dim, 1.0f, stream));
     const int rc = st.attention(st.att, st.q, L.k_cache, L.v_cache, st.page_table, st.max_pages, st.n_pages, st.row_pos, st.tiles,
-                                st.n_tiles, st.heads_q, st.heads_kv, L.scale, L.window, st.tile_rows, 0, stream);
+                                st.n_tiles, st.heads_q, st.heads_kv, L.scale, L.window, st.tile_rows, st.row_groups, st.group_pages, 0, stream);
     if (rc != SB_OK) return sb::fail(rc, "%s", st.attention_error());
     SB_TRY(join(st, st.att, L.out_w, q_width, L.norm_w, L.norm_dtype, L.norm_eps, stream));
     SB_TRY(whole_product(st.mid, SB_BF16, st.h, L.gate_up_w, nullptr, nullptr, t, st.inner, st.width, L.gate, st.part, st.part_floats,

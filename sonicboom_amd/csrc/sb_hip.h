@@ -678,10 +678,11 @@ typedef struct sb_dense_step {
   float *part;                              /* sb_dense_layers_floats(...) */
   size_t part_floats;
   int (*attention)(void *, const void *, const void *, const void *, const int32_t *, int, int, const int32_t *, const int32_t *, int,
-                   int, int, float, int, int, int, void *);       /* sb_attn_prefill_bf16 of the head size's library */
+                   int, int, float, int, int, int, int, int, void *);       /* sb_attn_prefill_bf16 of the head size's library */
   const char *(*attention_error)(void);
   const int32_t *row_pos, *row_seq, *page_table, *tiles;
   int n_rows, width, inner, heads_q, heads_kv, head_dim, max_pages, n_pages, n_tiles, tile_rows;
+  int row_groups, group_pages;              /* as the step_groups and step_pages of sb_attn_prefill_bf16 */
 } sb_dense_step;
 int sb_reduce_resid_norm_max_width(void);
 size_t sb_dense_layers_floats(int n_rows, int width, int qkv_width, int q_width, int inner);

@@ -116,6 +116,7 @@ class DenseLayers:
         if self.step is None:
             height = ops.attention_tile_height(ctx, m.heads_q, m.heads_kv, m.row_tile)
             self.step = ops.DenseStep(x, f.inner, m.heads_q, m.heads_kv, m.head_dim, ctx.page_table(bind.group), bind.k_cache.shape[0],
-                                      ctx.row_pos, ctx.row_seq, ctx.row_tiles(height), height)
+                                      ctx.row_pos, ctx.row_seq, ctx.row_tiles(height), height,
+                                      ops.attention_row_groups(ctx, height, m.heads_q))
         self.step.run(L, h)
         return h if follows else None

@@ -16,7 +16,7 @@ from typing import Optional, Sequence
 import numpy as np
 import torch
 
-from ..cache.paged import CacheError, PagedCache
+from ..cache.paged import PAGE, CacheError, PagedCache
 from . import dense
 from .model import DecoderModel
 
@@ -109,6 +109,17 @@ def row_runs(n_new: Sequence[int], cu, height: int) -> np.ndarray:
     return np.asarray(runs, dtype=np.int32).reshape(-1, 4)
 
 
+def group_pages(n_new: Sequence[int], before: Sequence[int], rows: int = 16):
+    """(groups, pages): the rows of a step in groups of up to ``rows`` consecutive rows of one sequence, and the pages
+    up to the last row of each added up."""
+    n, k = np.asarray(n_new, dtype=np.int64), np.asarray(before, dtype=np.int64)
+    groups = -(-n // rows)
+    first = np.cumsum(groups) - groups
+    seq = np.repeat(np.arange(len(n)), groups)
+    end = np.minimum((np.arange(len(seq)) - first[seq] + 1) * rows, n[seq])
+    return len(seq), int(((k[seq] + end - 1) // PAGE + 1).sum())
+
+
 class _Context:
     """What the parts read of a step's bookkeeping (see :class:`StepContext`)."""
 
@@ -180,6 +191,13 @@ class StepContext(_Context):
         self._host = host
         layout.bind(self, host.to(device, non_blocking=True))
         self.host_row_pos = row_pos
+        self._row_groups = None
+
+    def row_groups(self):
+        """:func:`group_pages` of the step."""
+        if self._row_groups is None:
+            self._row_groups = group_pages(self.n_new, self.lengths_before)
+        return self._row_groups
 
 
 class Engine:

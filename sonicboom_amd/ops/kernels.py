@@ -727,7 +727,7 @@ class _DenseStep(ctypes.Structure):
     _fields_ = ([(n, ctypes.c_void_p) for n in ("x", "h", "q", "att", "mid", "part")] + [("part_floats", ctypes.c_size_t)]
                 + [(n, ctypes.c_void_p) for n in ("attention", "attention_error", "row_pos", "row_seq", "page_table", "tiles")]
                 + [(n, ctypes.c_int) for n in ("n_rows", "width", "inner", "heads_q", "heads_kv", "head_dim", "max_pages", "n_pages",
-                                               "n_tiles", "tile_rows")])
+                                               "n_tiles", "tile_rows", "row_groups", "group_pages")])
 
 
 class DenseStep:
@@ -735,7 +735,7 @@ class DenseStep:
     workspace for what a layer hands from kernel to kernel.  Launches on the stream that is current when it is made."""
 
     def __init__(self, x: torch.Tensor, inner: int, heads_q: int, heads_kv: int, head_dim: int, page_table: torch.Tensor, n_pages: int,
-                 row_pos: torch.Tensor, row_seq: torch.Tensor, tiles: torch.Tensor, tile_rows: int):
+                 row_pos: torch.Tensor, row_seq: torch.Tensor, tiles: torch.Tensor, tile_rows: int, row_groups=(0, 0)):
         _dev(x, page_table, row_pos, row_seq, tiles)
         t, width = x.shape
         if x.dtype != torch.float32:
@@ -761,7 +761,8 @@ class DenseStep:
                                attention_error=ctypes.cast(attn.sb_attn_last_error, ctypes.c_void_p),
                                row_pos=row_pos.data_ptr(), row_seq=row_seq.data_ptr(), page_table=page_table.data_ptr(), tiles=tiles.data_ptr(),
                                n_rows=t, width=width, inner=inner, heads_q=heads_q, heads_kv=heads_kv, head_dim=head_dim,
-                               max_pages=page_table.shape[1], n_pages=n_pages, n_tiles=tiles.shape[0], tile_rows=int(tile_rows))
+                               max_pages=page_table.shape[1], n_pages=n_pages, n_tiles=tiles.shape[0], tile_rows=int(tile_rows),
+                               row_groups=row_groups[0], group_pages=row_groups[1])
 
     def run(self, layer: DenseLayer, h: torch.Tensor) -> None:
         """A layer on the stream in place; ``h`` bfloat16 [rows, width] its norm of the stream, then the next norm, if the layer
@@ -1040,10 +1041,11 @@ def attention_decode_pages_per_wave(head_dim: int, pages: int):
 
 
 def attention_prefill_mfma(q, k_cache, v_cache, page_table, row_pos, tiles, heads_q, heads_kv, head_dim, scale,
-                           window, tile_rows=16):
+                           window, tile_rows=16, row_groups=(0, 0)):
     """bf16 query rows over the cache; ``tiles`` int32 [n, 4] = (first row, rows <= tile_rows, sequence, 0)
     cuts the rows into runs of consecutive positions of one sequence.  ``tile_rows``: 16, or what
-    :func:`attention_row_tile` gives for these heads."""
+    :func:`attention_row_tile` gives for these heads.  ``row_groups``: what :func:`attention_row_groups` gives, for the choice
+    between the kernels."""
     _dev(q, k_cache, v_cache, page_table, row_pos, tiles)
     n = q.shape[0]
     if q.dim() != 2 or q.shape[1] != heads_q * head_dim or q.dtype != torch.bfloat16:
@@ -1058,7 +1060,7 @@ def attention_prefill_mfma(q, k_cache, v_cache, page_table, row_pos, tiles, head
     out = torch.empty_like(q)
     check(lib.sb_attn_prefill_bf16(_p(out), _p(q), _p(k_cache), _p(v_cache), _p(page_table), page_table.shape[1],
                                    k_cache.shape[0], _p(row_pos), _p(tiles), tiles.shape[0], heads_q, heads_kv,
-                                   float(scale), int(window), int(tile_rows), _hints.prefill_form, _stream()), lib,
+                                   float(scale), int(window), int(tile_rows), *row_groups, _hints.prefill_form, _stream()), lib,
           "sb_attn_last_error")
     return out
 
@@ -1123,6 +1125,13 @@ def attention_tile_height(ctx, heads_q: int, heads_kv: int, row_tile) -> int:
     return heights[0]
 
 
+def attention_row_groups(ctx, height: int, heads_q: int):
+    """(groups of up to sixteen rows, the pages they see added up) of a prompt step, where its attention chooses by them: the
+    kernel whose blocks take a group of one head each is ahead up to a block a CU whatever they see, and behind with many."""
+    blocks = ctx.row_tiles(height).shape[0] * (height // 16) * heads_q
+    return ctx.row_groups() if 192 < blocks <= 1024 and hasattr(ctx, "row_groups") else (0, 0)
+
+
 def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, page_table: torch.Tensor, ctx,
               heads_q: int, heads_kv: int, head_dim: int, scale: float, window: int,
               fast: bool = True, row_tile=ATTENTION_ROW_TILE) -> torch.Tensor:
@@ -1137,7 +1146,8 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pag
                                          head_dim, scale, window)
         height = attention_tile_height(ctx, heads_q, heads_kv, row_tile)
         return attention_prefill_mfma(q, k_cache, v_cache, page_table, ctx.row_pos, ctx.row_tiles(height),
-                                      heads_q, heads_kv, head_dim, scale, window, tile_rows=height)
+                                      heads_q, heads_kv, head_dim, scale, window, tile_rows=height,
+                                      row_groups=attention_row_groups(ctx, height, heads_q))
     return attention_plain(q, k_cache, v_cache, page_table, ctx.row_pos, ctx.row_seq, heads_q, heads_kv,
                            head_dim, scale, window)
 

@@ -6,7 +6,7 @@ import pytest
 import torch
 
 from sonicboom_amd.cache import GroupSpec, PagedCache
-from sonicboom_amd.engine.step import ContextLayout, Engine, StepContext, StepEntry, StepError, row_runs
+from sonicboom_amd.engine.step import ContextLayout, Engine, StepContext, StepEntry, StepError, group_pages, row_runs
 
 VOCAB = 50
 
@@ -101,6 +101,9 @@ def test_one_layout_for_both_kinds_of_context():
     assert ctx.row_pos.tolist() == list(range(70)) + [0, 1, 2] and ctx.cu_rows.tolist() == [0, 70, 73]
     assert ctx.row_tiles(16).tolist() == [[0, 16, 0, 0], [16, 16, 0, 0], [32, 16, 0, 0], [48, 16, 0, 0],
                                           [64, 6, 0, 0], [70, 3, 1, 0]]
+    assert ctx.row_groups() == (6, 4 * 1 + 2 + 1)              # (the fifth group's last row lies on the second page)
+    assert group_pages([1, 16, 17, 200], [64, 48, 47, 1000]) == (1 + 1 + 2 + 13, 2 + 1 + 1 + 1 + sum((min(1000 + 16 * j, 1200) - 1) // 64 + 1
+                                                                                                 for j in range(1, 14)))
     assert ctx.page_table(0).shape == (2, 2) and ctx.page_table(0)[1].tolist()[1] == -1
     with pytest.raises(StepError, match="row tiles of 8"):
         ctx.row_tiles(8)
