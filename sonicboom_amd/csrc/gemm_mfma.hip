@@ -1142,7 +1142,16 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
     const bool one_round = (blocks + kXcds - 1) / kXcds * kXcds <= sb::cu_count();
     if (variant == 0) rc = one_round ? launch_direct<4, 2, 64, 4, false>(a, blocks, 0, s) : launch_direct<4, 2, 64, 2, false>(a, blocks, 0, s);
     else if (variant == 1) rc = launch_direct<8, 2, 64, 2, false>(a, blocks, 0, s);
-    else if (variant == 2) rc = launch_pipe(a, blocks, path == 3, s);      // (path 3: a measurement's)
+    else if (variant == 2) {
+      // Which 256 x 256 kernel: the one that reads fragments ahead of the barrier for gated products (37,888 x 3,584, 2,048
+      // rows 461 -> 452 us, 512 rows 191 -> 181; 9,728 x 896, 12,000 rows 220 -> 209) and long K (3,584 x 18,944, 2,048 rows 399
+      // -> 371); otherwise, up to a round of tiles or with K below 8,192, the one a whole stage ahead, whose start and epilogue
+      // are shorter (4,608 x 3,584, 3,000 rows 85 for 81; 2,048 x 1,536, 6,400 rows 44 for 42; 3,584 x 3,584, 4,096 rows 88 for
+      // 83; 1,536 x 8,960, 2,048 rows 163 for 159, but at 12,000 rows 401 and 405).  The same bits.
+      const bool ahead = a.gated || n_in >= 16384 || (n_in >= 8192 && blocks > sb::cu_count());
+      if (ahead || path == 3) rc = launch_pipe(a, blocks, path == 3, s);      // (path 3: a measurement's)
+      else rc = launch_direct_one<8, 4, 64, 2, 0, true>(a, blocks, sb::cu_count(), s);
+    }
     else if (variant == 3) rc = launch_direct<4, 4, 64, 2, false>(a, blocks, 0, s);
     else if (variant == 4) rc = launch_direct<6, 4, 64, 2, true>(a, blocks, sb::cu_count(), s);
     else rc = one_round ? launch_direct<2, 2, 64, 4, false>(a, blocks, 0, s) : launch_direct<2, 2, 64, 2, false>(a, blocks, 0, s);

@@ -395,6 +395,26 @@ def test_gemm_bf16_blocks_that_go_from_tile_to_tile():
             close(got, g / (1.0 + torch.exp(-g)) * u, atol=1e-4 * math.sqrt(k), rtol=1e-4, what=f"gated {shape} {path}")
 
 
+@pytest.mark.parametrize("t, n, k", [(300, 520, 1024), (300, 520, 16448), (4400, 4200, 8128), (4400, 4200, 8192), (1000, 1800, 8192)])
+def test_gemm_bf16_both_kernels_of_the_largest_tiles_give_the_same_bits(t, n, k):
+    """256 x 256 tiles on either side of what chooses between the kernel that reads fragments ahead and the one a whole stage
+    ahead (the inner size, and more tiles than CUs), against the first with a block for every tile."""
+    from sonicboom_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(t, k, generator=gen, device=DEV).to(BF16)
+    w = ops.pack_weight((torch.randn(n, k, generator=gen, device=DEV) * 0.05).to(BF16))
+    resid = torch.randn(t, n, generator=gen, device=DEV)
+    got = {}
+    for path in ("direct", "direct, a block a tile"):
+        with ops.gemm_tile_shape(2, path):
+            got[path] = ops.gemm_bf16(x, w, None, resid, F32, packed_shape=(n, k))
+    assert torch.equal(*got.values())
+    with ops.gemm_tile_shape(0, "registers"):
+        other = ops.gemm_bf16(x, w, None, resid, F32, packed_shape=(n, k))
+    # (the sums in another order: k terms of size 0.05, 2^-24 each of sums of size sqrt(k) 0.05)
+    assert (got["direct"] - other).abs().max().item() <= 3e-5 * math.sqrt(k)
+
+
 def test_gemm_bf16_direct_path_refuses_what_it_cannot_take():
     from sonicboom_amd import ops
     x, w = randn(70, 96, dtype=BF16).to(DEV), randn(64, 96, dtype=BF16).to(DEV)
