@@ -78,7 +78,12 @@ struct PlainArgs {
   const float *resid;
   int n_rows, n_out, n_in;
   int gate;        // the activation (an sb_gate) of the gated form
+  bool vec4;       // n_out % 4 == 0, and Y and the residual start on 16 bytes
 };
+
+bool by_fours(const void *y, const float *resid, int n_out) {
+  return n_out % 4 == 0 && (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(resid)) % 16 == 0;
+}
 
 template <typename TX, typename TW, int FORM, int TT, int CT, int G, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
@@ -209,7 +214,8 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
     }
   }
 
-  // unit (tile (i, j), lane (g, r)): columns 16 i + 4 g + 0..3 of row 16 j + r
+  // unit (tile (i, j), lane (g, r)): columns 16 i + 4 g + 0..3 of row 16 j + r, stored together where they are aligned: a
+  // product of few k is bound here (4,096 x 64 onto a residual stream of 4,000 rows 105 us a number at a time, 56 the LDS tiles)
 #pragma unroll
   for (int u = 0; u < kUnits; ++u) {
     const int unit = tid + u * 64 * WAVES;
@@ -217,6 +223,22 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
     const int tile = unit >> 6, l = unit & 63;
     const int t = t0 + 16 * (tile % TT) + (l & 15), nb = n0 + 16 * (tile / TT) + 4 * (l >> 4);
     if (t >= a.n_rows) continue;
+    if (a.vec4) {
+      if (nb >= a.n_out) continue;
+      const size_t idx = size_t(t) * a.n_out + nb;
+      floatx4_t v = total[u][0];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (G == 2) v[e] = gate_act(v[e], a.gate) * total[u][G - 1][e];
+        if (a.bias) v[e] = v[e] + ld_dyn(a.bias, a.bias_dtype, nb + e);
+      }
+      if (a.resid) v = v + *reinterpret_cast<const floatx4_t *>(a.resid + idx);
+      if (a.y_dtype == SB_F32) *reinterpret_cast<floatx4_t *>((float *)a.y + idx) = v;
+      else
+        *reinterpret_cast<ushort4 *>((bf16_t *)a.y + idx) =
+            make_ushort4(f32_to_bf16(v[0]), f32_to_bf16(v[1]), f32_to_bf16(v[2]), f32_to_bf16(v[3]));
+      continue;
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int n = nb + e;
@@ -389,7 +411,7 @@ extern "C" int sb_gemm(void *y, int y_dtype, const void *x, int x_dtype, const v
   SB_SUPPORT((n_rows + 63) / 64 <= 65535, "sb_gemm: more than %d rows in one call", 65535 * 64);
   if (n_rows == 0) return SB_OK;
   hipStream_t s = (hipStream_t)stream;
-  const PlainArgs a{y, y_dtype, bias, bias_dtype, resid, n_rows, n_out, n_in, SB_GATE_NONE};
+  const PlainArgs a{y, y_dtype, bias, bias_dtype, resid, n_rows, n_out, n_in, SB_GATE_NONE, by_fours(y, resid, n_out)};
   const int n_seg = (n_in + kSegment - 1) / kSegment;
   if (x_dtype == SB_F32 && w_dtype == SB_F32) return launch_any((const float *)x, (const float *)w, a, n_seg, s);
   if (x_dtype == SB_F32) return launch_any((const float *)x, (const bf16_t *)w, a, n_seg, s);
@@ -413,7 +435,7 @@ extern "C" int sb_gemm_f32_packed(void *y, int y_dtype, const float *x, const fl
   SB_SUPPORT(reinterpret_cast<uintptr_t>(w) % 16 == 0, "sb_gemm_f32_packed: the packed weights must be 16-byte aligned");
   if (n_rows == 0) return SB_OK;
   hipStream_t s = (hipStream_t)stream;
-  const PlainArgs a{y, y_dtype, bias, bias_dtype, resid, n_rows, n_out, n_in, gated};
+  const PlainArgs a{y, y_dtype, bias, bias_dtype, resid, n_rows, n_out, n_in, gated, by_fours(y, resid, n_out)};
   const int n_seg = (n_in + kSegment - 1) / kSegment;
   // 16-byte loads need rows of X that start on 16 bytes; offsets inside a block's rows fit 31 bits
   const bool vec = n_in % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && size_t(n_in) * 64 * 4 < (size_t(1) << 31);

@@ -1189,6 +1189,35 @@ def test_attention_prefill_forms(hq, hkv, hd, window, form):
             test_attention_prefill_window_edge(hq, hkv, hd, window)
 
 
+@pytest.mark.parametrize("t, n, k", [(1, 4, 16), (3, 20, 40), (33, 100, 64), (70, 516, 1100), (40, 36, 2064)])
+@pytest.mark.parametrize("out_dtype", [F32, BF16])
+def test_float32_products_stored_by_fours(t, n, k, out_dtype):
+    """Four neighbouring outputs at a time where rows start on 16 bytes, and one by one where they do not: the same bits, with a
+    bias and a residual, in place, from packed and from row-major weights, and gated."""
+    from sonicboom_amd import ops
+    x, w, bias = randn(t, k).to(DEV), randn(n, k, seed=1).to(DEV), randn(n, seed=2).to(DEV)
+    resid = randn(t, n, seed=3)
+    off = torch.empty(t * n + 1, device=DEV)[1:].view(t, n)            # starts four bytes past sixteen
+    off_out = torch.empty(t * n + 1, dtype=out_dtype, device=DEV)[1:].view(t, n)
+    off.copy_(resid)
+    packed = ops.pack_weight_f32(w)
+    one = ops.gemm_f32(x, packed, bias, off, out_dtype, (n, k), out=off_out).clone()
+    four = ops.gemm_f32(x, packed, bias, resid.to(DEV), out_dtype, (n, k))
+    assert torch.equal(one, four)
+    assert torch.equal(four, ops.gemm_plain(x, w, bias, resid.to(DEV), out_dtype))
+    if out_dtype == F32:
+        place = resid.to(DEV)
+        assert torch.equal(ops.gemm_f32(x, packed, bias, place, F32, (n, k), out=place), four)
+        want = x.cpu().double() @ w.cpu().double().T + bias.cpu().double() + resid.double()
+        bound = (x.cpu().abs().double() @ w.cpu().abs().double().T + 4.0) * (k + 4) * 2.0 ** -24     # k roundings of the partial sums
+        assert ((four.cpu().double() - want).abs() <= bound).all()
+    h = n // 2
+    pair = ops.pack_weight_f32(w, True)
+    gated = ops.gemm_f32(x, pair, None, None, out_dtype, (n, k), gated="silu")
+    off_gated = torch.empty(t * h + 1, dtype=out_dtype, device=DEV)[1:].view(t, h)
+    assert torch.equal(gated, ops.gemm_f32(x, pair, None, None, out_dtype, (n, k), gated="silu", out=off_gated))
+
+
 # (heads, head size, tile height, [(cached, rows)], window, whether the pages are cut over a block's waves); both forms measured
 FORM_CHOICES = [
     (14, 2, 64, 16, [(0, 40)] * 16, 0, 0), (14, 2, 64, 16, [(0, 120)] * 8, 0, 0), (14, 2, 64, 16, [(200, 4)] * 64, 0, 0),
