@@ -22,8 +22,11 @@
 // It is bound by latency: a chunk is two dependent reads (the page's number, then its
 // keys and values).  The block's waves take a chunk each, and a wave asks for a chunk's values
 // before it reads its keys, sixteen bytes a load.  Measured with 14 heads of 64 in float32: one token of 3
-// sequences of 40 to 260 keys 37.7 us with one wave a row and head and an element a load, 10.7 now; their
-// prompts' 520 rows 116 and 74.
+// sequences of 40 to 260 keys 31.4 us with one wave a row and head and an element a load, 8.5 now; the
+// prompts of 40, 220 and 260 rows 145 and 59.  Behind it stay calls of a few rows on a few keys, which the longer code costs
+// (a prompt of 3 rows, 12 heads of 128: 7.2 and 9.0), and many rows of heads of 16 (1,000, a window of 100: 28 and 33).  Loads of
+// all eight groups of values, the hidden ones aimed at a visible one's place, cost more (32 prompts of 10 rows 12.4 and 19.5),
+// loads that leave the hidden ones out by a descriptor's end as much (13.7).
 #include "common.h"
 
 namespace {

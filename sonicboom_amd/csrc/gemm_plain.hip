@@ -24,9 +24,9 @@
 //
 // What bounds it: with few rows the read of W (each wave must have enough of it in flight) and the
 // chain's latency, with many the matrix cores.  Measured on MI355X at the 0.5B layer sizes, 3 rows, against the
-// kernel with one fmaf chain a thread that stood here before: 896 x 896 107 us then, 9.2 now; 896 x 4,864
-// 597 and 16.7; the gated 9,728 x 896 110 + 4.8 (its activation) and 16.2.  520 rows: the gated product 179 + 7 and
-// 150 (61 TFLOP/s), 896 x 4,864 666 and 78.  From row-major W with swaps the 3-row products took 13.6, 19.4 and 15 us.
+// kernel with one fmaf chain a thread that stood here before: 896 x 896 107 us then, 8.7 now; 896 x 4,864
+// 597 and 15.7; the gated 9,728 x 896 110 + 4.8 (its activation) and 14.1.  520 rows: the gated product 179 + 7 and
+// 138 (66 TFLOP/s), 896 x 4,864 666 and 76.  From row-major W with swaps the 3-row products took 13.6, 19.4 and 15 us.
 #include "mfma.h"
 
 namespace {
