@@ -214,17 +214,27 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
     }
   }
 
-  // unit (tile (i, j), lane (g, r)): columns 16 i + 4 g + 0..3 of row 16 j + r, stored together where they are aligned: a
-  // product of few k is bound here (4,096 x 64 onto a residual stream of 4,000 rows 105 us a number at a time, 56 the LDS tiles)
+  // unit (tile (i, j), lane (g, r)): columns 16 i + 4 g + 0..3 of row 16 j + r, stored together where they are aligned, and
+  // their residuals (which the stores may overwrite, each its own) asked for ahead of the first store: a product of few k is
+  // bound here (4,096 x 64 onto a residual stream of 4,000 rows 105 us a number at a time, 63 by fours, 57 so; 55 the LDS tiles)
+  const auto place = [&](int u, int &t, int &nb) {
+    const int unit = tid + u * 64 * WAVES, tile = unit >> 6, l = unit & 63;
+    t = t0 + 16 * (tile % TT) + (l & 15), nb = n0 + 16 * (tile / TT) + 4 * (l >> 4);
+    return unit < kTiles * 64 && t < a.n_rows && nb < a.n_out;
+  };
+  if (a.vec4) {
+    floatx4_t old[kUnits];
+    if (a.resid) {
 #pragma unroll
-  for (int u = 0; u < kUnits; ++u) {
-    const int unit = tid + u * 64 * WAVES;
-    if (unit >= kTiles * 64) continue;
-    const int tile = unit >> 6, l = unit & 63;
-    const int t = t0 + 16 * (tile % TT) + (l & 15), nb = n0 + 16 * (tile / TT) + 4 * (l >> 4);
-    if (t >= a.n_rows) continue;
-    if (a.vec4) {
-      if (nb >= a.n_out) continue;
+      for (int u = 0; u < kUnits; ++u) {
+        int t, nb;
+        if (place(u, t, nb)) old[u] = *reinterpret_cast<const floatx4_t *>(a.resid + size_t(t) * a.n_out + nb);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kUnits; ++u) {
+      int t, nb;
+      if (!place(u, t, nb)) continue;
       const size_t idx = size_t(t) * a.n_out + nb;
       floatx4_t v = total[u][0];
 #pragma unroll
@@ -232,13 +242,18 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
         if constexpr (G == 2) v[e] = gate_act(v[e], a.gate) * total[u][G - 1][e];
         if (a.bias) v[e] = v[e] + ld_dyn(a.bias, a.bias_dtype, nb + e);
       }
-      if (a.resid) v = v + *reinterpret_cast<const floatx4_t *>(a.resid + idx);
+      if (a.resid) v = v + old[u];
       if (a.y_dtype == SB_F32) *reinterpret_cast<floatx4_t *>((float *)a.y + idx) = v;
       else
         *reinterpret_cast<ushort4 *>((bf16_t *)a.y + idx) =
             make_ushort4(f32_to_bf16(v[0]), f32_to_bf16(v[1]), f32_to_bf16(v[2]), f32_to_bf16(v[3]));
-      continue;
     }
+    return;
+  }
+#pragma unroll
+  for (int u = 0; u < kUnits; ++u) {
+    int t, nb;
+    if (!place(u, t, nb)) continue;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int n = nb + e;
