@@ -714,25 +714,29 @@ gemm_direct16_kernel(Args a) {
 
 
 // ---------------------------------------------------------------------------------------------
-// The same, 256 x 256 tiles, in stages of 32 k through four buffers.  In the kernel above every wave
-// comes out of a stage's barrier with empty hands: it reads six fragments and waits for them before its first
-// product, both waves of a SIMD at once.  Here the barrier that ends stage s promises stage s + 2 (the wait
-// before it leaves only the newest stage's loads in flight), so the first fragments of stage s + 1 are read
-// in stage s, with its last tiles, and the products go on right behind the barrier.
-// A's rows are 64 bytes a stage: two 16-row tiles lie side by side in the 128-byte lines of LDS whose
-// swizzle the fragment reads take without conflicts.  The epilogue turns its rows through the one buffer that
-// holds nothing (swizzled instead of padded: it is exactly as large).
-// Measured, kernel above against this one: 3.6 % faster on the gate/up product of 2,048 x 37,888 x 3,584 (469 and 451 us),
-// 8 % on 6,398 x 2,048 x 11,008 (257 and 236), 3 % on 16,384 x 3,584 x 18,944 (1.87 and 1.81 ms), each by itself; in whole
-// prompt steps, back to back, 1 to 2.5 %.  What bounds it: with the loads left out 1.6 to 1.8 PFLOP/s, with the products left
-// out 0.55 of the time; why the two together reach 1.23 (2,048 x 37,888 x 3,584) is not settled: a library's product runs
-// 8,192 x 16,384 x 3,584 at 1.55 on the same card, so it is neither the clock nor the power alone.
+// The same, 256 x 256 tiles, in stages of 32 k, the two waves of a SIMD a turn apart: while waves 0 to 3 read their
+// fragments of a stage and send out loads, waves 4 to 7 keep the matrix cores busy with theirs, and at every meeting (a bare
+// barrier) they change places.  A wave comes to its products with all twelve fragments in registers.
+// X is loaded in whole lines of 128 bytes (64 k of a row, in three buffers), W, which lies in blocks, 32 k at a time through
+// four: all 160 KB of LDS.  The loads run two to three stages ahead; a meeting promises the stage that is read after it, for the
+// waves that read it next (which waited ahead of it for their own loads) and for the others.  A buffer's last readers were
+// through a turn before its next loads go out.  The epilogue turns its rows through the one buffer of X that holds nothing
+// (ungated: swizzled instead of padded, it is exactly as large), with both halves of the block at it.
+// What bounds it: the loads.  By themselves (no fragments read, no products) they take 0.83 of the kernel's time at 16,384 x
+// 3,584 x 18,944 and 0.71 at 16,384 x 37,888 x 3,584, products by themselves 0.67 and 0.70.  Half lines of X (64 bytes a row
+// and stage) made that 1.0 and 0.9: L2 answers as many requests a second of either size.  Measured against the kernel that had
+// one barrier a stage, both waves of a SIMD reading and multiplying at once, and half lines: 2,048 x 37,888 x 3,584 443 -> 415 us,
+// 16,384 rows 3.31 -> 3.13 ms (1.42 PFLOP/s), 16,384 x 3,584 x 18,944 1.89 -> 1.72, 6,398 x 22,016 x 2,048 475 -> 454 us; of that
+// the turns give 3 to 4 %.  Not kept: turns of 64 k (a wave's fragments then wait for W's loads, one stage ahead: 0.87 of
+// the speed), whole lines with one barrier a stage and no turns (3 to 4 % slower), loads between the products (2 to 5 %),
+// half of X's fragments read beside the products (6 to 10 %), s_setprio around the products (1 %).
 template <int GATED, bool PERSIST>
 __global__ void __launch_bounds__(512)
 gemm_pipe_kernel(Args a) {
-  constexpr int MT16 = 8, NW = 4, BM = 256, BN = 256, kWaves = 8, NBUF = 4;
-  constexpr int kLoads = 4;                          // of a wave and stage: two of A, two of W
-  constexpr int kBufChunks = (BM + BN) * 4;          // 16-byte chunks of a stage buffer: A, then W
+  constexpr int MT16 = 8, NW = 4, BM = 256, BN = 256, kWaves = 8;
+  constexpr int kRingA = 3, kRingW = 4;              // buffers of X (64 k each) and of W (32 k)
+  constexpr int kBufA = BM * 8, kBufW = BN * 4;      // 16-byte chunks of a buffer
+  constexpr int kFlight = 8;                         // loads that a wave has in flight across a meeting: two stages'
   extern __shared__ bf16x8_t lds[];
   typedef __attribute__((address_space(3))) bf16x8_t *lds_ptr_t;
 
@@ -747,37 +751,42 @@ gemm_pipe_kernel(Args a) {
       const_cast<bf16_t *>(a.x), 0, uint32_t(size_t(a.n_rows) * a.n_in * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<bf16_t *>(a.w), 0, uint32_t(w_rows_total * size_t(a.w_steps) * 64), 0x00020000);
-  // sources of the loads at stage 0 of tile (m, n): as in the kernel above but for A's lines: line l of a
-  // buffer holds, in the places p ^ (l / 2) % 8, chunks p % 4 of row l % 16 of tiles 2 (l / 16) (p < 4) and the next
-  uint32_t off[kLoads];
-  auto aim_at = [&](int m, int n) {
-    const int t0 = m * BM, n0 = n * (GATED ? BN / 2 : BN);
+  // sources of a wave's loads at k 0 of tile (m, n), as in the kernel above: four of X for 64 k, two of W for 32 k
+  uint32_t off_a[4], off_w[2];
+  auto aim_a = [&](int m) {
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) {
-      if (i < 2) {
-        const int place = (i * kWaves + wave) * 64 + lane;
-        const int line = place / 8, c8 = (place % 8) ^ ((line / 2) & 7);
-        const int row = (line / 16) * 32 + (c8 >> 2) * 16 + line % 16;
-        off[i] = uint32_t((size_t(t0 + row) * a.n_in + (c8 & 3) * 8) * 2);
-      } else {
-        const int rt = (i - 2) * kWaves + wave;
-        const int tile = GATED ? ((rt & 3) >> 1) * a.w_tiles + n0 / 16 + (rt >> 2) * 2 + (rt & 1) : n0 / 16 + rt;
-        off[i] = uint32_t((size_t(tile) * a.w_steps * 512 + size_t(lane) * 8) * 2);
-      }
+    for (int i = 0; i < 4; ++i) {
+      const int place = (i * kWaves + wave) * 64 + lane;
+      const int row = place / 8, c = (place % 8) ^ ((row / 2) & 7);
+      off_a[i] = uint32_t((size_t(m * BM + row) * a.n_in + c * 8) * 2);
     }
   };
-  auto issue_load = [&](int i, int kt, int buf) {
-    const bool is_a = i < 2;
-    const int chunk = buf * kBufChunks + (is_a ? (i * kWaves + wave) * 64 : BM * 4 + ((i - 2) * kWaves + wave) * 64);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(is_a ? rsrc_x : rsrc_w, (lds_ptr_t)(lds) + chunk, 16, int(off[i]),
-                                             is_a ? kt * 64 : kt * 1024, 0, 0);
+  auto aim_w = [&](int n) {
+    const int n0 = n * (GATED ? BN / 2 : BN);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int rt = i * kWaves + wave;
+      const int tile = GATED ? ((rt & 3) >> 1) * a.w_tiles + n0 / 16 + (rt >> 2) * 2 + (rt & 1) : n0 / 16 + rt;
+      off_w[i] = uint32_t((size_t(tile) * a.w_steps * 512 + size_t(lane) * 8) * 2);
+    }
   };
-  // everything but the loads of the newest stage has landed, for this wave and after the barrier for all
-  auto wait_and_meet = [&]() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kLoads) : "memory");
+  auto load_a = [&](int i, int k64, int buf) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_x, (lds_ptr_t)(lds) + buf * kBufA + (i * kWaves + wave) * 64, 16, int(off_a[i]),
+                                             k64 * 128, 0, 0);
+  };
+  auto load_w = [&](int kt, int buf) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (lds_ptr_t)(lds) + kRingA * kBufA + buf * kBufW + (i * kWaves + wave) * 64, 16,
+                                               int(off_w[i]), kt * 1024, 0, 0);
+  };
+  auto meet = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
   };
+  auto landed = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kFlight) : "memory"); };
 
   // stages of 32 k, an even count (the host: an inner size in 64s, slices of whole 64s)
   const int n_k_all = a.n_in / 32;
@@ -785,47 +794,79 @@ gemm_pipe_kernel(Args a) {
   const int n_k = a.partial ? min(kt_begin + a.stages_per_slice * 2, n_k_all) : n_k_all;
   // A stage past the end (of the last tile, when the block goes on) is the last stage once more, into a
   // buffer that nobody reads again, so that the count of loads in flight stays the same.
-  aim_at(tm, tn);
+  aim_a(tm);
+  aim_w(tn);
 #pragma unroll
-  for (int s = 0; s < NBUF - 1; ++s)
+  for (int i = 0; i < 4; ++i) load_a(i, kt_begin / 2, 0);
+  load_w(kt_begin, 0);
 #pragma unroll
-    for (int i = 0; i < kLoads; ++i) issue_load(i, min(kt_begin + s, n_k - 1), s);
-  wait_and_meet();
+  for (int h = 0; h < 2; ++h) {
+    load_a(2 * h, min(kt_begin / 2 + 1, n_k / 2 - 1), 1);
+    load_a(2 * h + 1, min(kt_begin / 2 + 1, n_k / 2 - 1), 1);
+    load_w(min(kt_begin + 1 + h, n_k - 1), 1 + h);
+  }
+  landed();
+  meet();
 
   const int fr = lane & 15, fg = lane >> 4;
-  int a_lane[2];
+  int a_lane[2];                  // the fragment's place in each half of a buffer of X
 #pragma unroll
-  for (int j = 0; j < 2; ++j) a_lane[j] = wm * (16 * MT16) * 4 + fr * 8 + ((4 * j + fg) ^ ((fr / 2) & 7));
-  auto a_at = [&](int i) { return a_lane[i & 1] + (i >> 1) * 128; };
-  const int b_lane = BM * 4 + wn * 4 * 64 + lane;
+  for (int j = 0; j < 2; ++j) a_lane[j] = (wm * (16 * MT16) + fr) * 8 + ((4 * j + fg) ^ ((fr / 2) & 7));
+  const int b_lane = kRingA * kBufA + wn * 4 * 64 + lane;
 
   floatx4_t acc[MT16][4];
-  bf16x8_t fa[4], fb[2][4];       // A in a ring of four tiles, W in a set for even and one for odd stages
-  auto stage = [&](auto PAR, int buf, int kt_load) {
-    constexpr int par = decltype(PAR)::value;
-    const bf16x8_t *ls = lds + buf * kBufChunks, *ls_next = lds + ((buf + 1) & (NBUF - 1)) * kBufChunks;
-    const int buf_load = (buf + NBUF - 1) & (NBUF - 1);
+  int tm_next = 0, tn_next = 0;
+  bool more = false;
+  int buf_a = 0, buf_w = 0;
+  // One stage, half HALF of 64 k: a wave's turn at the memories (its fragments, and its share of the loads two to three stages
+  // further on, into buffers whose last reader was through a turn ago), then its turn at the matrix cores.
+  auto stage = [&](auto HALF, int kt) {
+    constexpr int half = decltype(HALF)::value;
+    bf16x8_t fa[MT16], fb[4];
+    const bf16x8_t *ls_a = lds + buf_a * kBufA + a_lane[half], *ls_w = lds + (buf_w + half) * kBufW + b_lane;
 #pragma unroll
-    for (int i = 0; i < MT16; ++i) {
+    for (int f = 0; f < 4; ++f) fb[f] = ls_w[f * 64];
 #pragma unroll
-      for (int f = 0; f < 4; ++f) {
-        acc[i][f] = mfma16(fa[i & 3], fb[par][f], acc[i][f]);
-        // two tiles ahead; the next stage's first two with the last two of this one, its W with the last four
-        if (f == 0) fa[(i + 2) & 3] = i + 2 < MT16 ? ls[a_at(i + 2)] : ls_next[a_at(i + 2 - MT16)];
-        if (f == 1 && i >= MT16 - 4) fb[par ^ 1][i - (MT16 - 4)] = ls_next[b_lane + (i - (MT16 - 4)) * 64];
-        if (f >= 2 && i < 2) issue_load(i * 2 + f - 2, kt_load, buf_load);
-        __builtin_amdgcn_sched_barrier(0);       // keep this order (see above)
+    for (int i = 0; i < MT16; ++i) fa[i] = ls_a[i * 128];
+    int k64 = kt / 2 + 2, kw = kt + 3;
+    if (half == 0 ? kt + 4 >= n_k : kt + 3 >= n_k) {            // past the tile's end
+      if (!PERSIST || !more) {
+        k64 = n_k / 2 - 1;
+        kw = min(kw, n_k - 1);
+      } else {
+        k64 = k64 - n_k / 2 + kt_begin / 2;
+        if (half == 0) {
+          if (kt + 4 == n_k) aim_a(tm_next);                    // from here on X's loads are the next tile's,
+          if (kw >= n_k) kw = kw - n_k + kt_begin;
+        } else {
+          if (kt + 3 == n_k) aim_w(tn_next);                    // and from here on W's
+          kw = kw - n_k + kt_begin;
+        }
       }
     }
-    wait_and_meet();
+    const int to_a = buf_a == 0 ? 2 : buf_a - 1;
+    load_a(2 * half, k64, to_a);
+    load_a(2 * half + 1, k64, to_a);
+    load_w(kw, (buf_w + half + 3) & (kRingW - 1));
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (wm) landed();
+    meet();
+#pragma unroll
+    for (int i = 0; i < MT16; ++i)
+#pragma unroll
+      for (int f = 0; f < 4; ++f) acc[i][f] = mfma16(fa[i], fb[f], acc[i][f]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (!wm) landed();
+    meet();
   };
 
   constexpr int NC = GATED ? 32 : 64, kPitch = GATED ? NC + 4 : NC;
-  static_assert(kBufChunks * 16 >= kWaves * 16 * kPitch * 4, "the turning areas must fit a stage buffer");
-  auto epilogue = [&](int m, int n, int buf_free) {
+  static_assert(kBufA * 16 >= kWaves * 16 * kPitch * 4, "the turning areas must fit a buffer of X");
+  auto epilogue = [&](int m, int n, int a_free) {
     const bool far = silu_far<GATED, 8 * MT16>([&](int i) { return acc[i / 8][i % 8 / 4][i % 4]; });
     store_tile<MT16, 16, NW, NC, kPitch, !GATED>(
-        a, reinterpret_cast<float *>(lds + buf_free * kBufChunks), m * BM, n * (GATED ? BN / 2 : BN), !GATED,
+        a, reinterpret_cast<float *>(lds + a_free * kBufA), m * BM, n * (GATED ? BN / 2 : BN), !GATED,
         [&](int i, float *turn) {
           const auto fill = [&](auto FAR) {
 #pragma unroll
@@ -846,38 +887,27 @@ gemm_pipe_kernel(Args a) {
         });
   };
 
-  int buf = 0;
-#pragma unroll
-  for (int f = 0; f < 4; ++f) fb[0][f] = lds[b_lane + f * 64];
-  fa[0] = lds[a_at(0)];
-  fa[1] = lds[a_at(1)];
   for (;;) {
 #pragma unroll
     for (int i = 0; i < MT16; ++i)
 #pragma unroll
       for (int f = 0; f < 4; ++f) acc[i][f] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-    int tm_next = 0, tn_next = 0;
-    const bool more = PERSIST && tile_of_block(a, vblock + int(gridDim.x), tm_next, tn_next);
-    auto stage_to_load = [&](int kt) {
-      const int l = kt + NBUF - 1;
-      if (l < n_k) return l;
-      if (!PERSIST || !more) return n_k - 1;
-      if (l == n_k) aim_at(tm_next, tn_next);    // from here on the loads are the next tile's
-      return l - n_k + kt_begin;
-    };
+    more = PERSIST && tile_of_block(a, vblock + int(gridDim.x), tm_next, tn_next);
+    if (wm) meet();               // the second four waves are a turn behind the first
     for (int kt = kt_begin; kt < n_k; kt += 2) {
-      stage(std::integral_constant<int, 0>{}, buf, stage_to_load(kt));
-      buf = (buf + 1) & (NBUF - 1);
-      stage(std::integral_constant<int, 1>{}, buf, stage_to_load(kt + 1));
-      buf = (buf + 1) & (NBUF - 1);
+      stage(std::integral_constant<int, 0>{}, kt);
+      stage(std::integral_constant<int, 1>{}, kt + 1);
+      buf_a = buf_a == kRingA - 1 ? 0 : buf_a + 1;
+      buf_w ^= 2;
     }
+    if (!wm) meet();
     if (!PERSIST || !more) {
       // the last loads (of the last stage again) are still writing LDS
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
     }
-    epilogue(tm, tn, (buf + NBUF - 1) & (NBUF - 1));       // the other three hold the next tile's first stages
+    epilogue(tm, tn, buf_a == 0 ? 2 : buf_a - 1);       // the other buffers hold the next tile's first stages
     if (!PERSIST || !more) break;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -887,7 +917,6 @@ gemm_pipe_kernel(Args a) {
     tn = tn_next;
   }
 }
-
 
 template <int MT, int NW, int BK, int DEPTH, int GATED, bool PACKED, bool EVEN_K>
 int launch_one(const Args &a, long long blocks, hipStream_t s) {
@@ -972,7 +1001,7 @@ int launch_direct(const Args &a, long long blocks, int round_blocks, hipStream_t
 
 template <int GATED, bool PERSIST>
 int launch_pipe_one(const Args &a, long long blocks, hipStream_t s) {
-  constexpr int lds_bytes = 4 * (256 + 256) * 4 * 16;
+  constexpr int lds_bytes = 3 * 256 * 128 + 4 * 256 * 64;      // 160 KB: all that a CU has
   static bool raised = false;     // per instantiation; harmless if repeated
   if (!raised) {
     const hipError_t e = hipFuncSetAttribute((const void *)gemm_pipe_kernel<GATED, PERSIST>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -983,13 +1012,13 @@ int launch_pipe_one(const Args &a, long long blocks, hipStream_t s) {
   const int n_k = a.n_in / 64;
   const unsigned slices = a.partial ? unsigned((n_k + a.stages_per_slice - 1) / a.stages_per_slice) : 1u;
   long long grid = (blocks + kXcds - 1) / kXcds * kXcds;
-  if (PERSIST && grid > sb::cu_count()) grid = sb::cu_count();        // 128 KB of LDS: a block a CU
+  if (PERSIST && grid > sb::cu_count()) grid = sb::cu_count();        // a block a CU
   gemm_pipe_kernel<GATED, PERSIST><<<dim3(unsigned(grid), slices), 512, lds_bytes, s>>>(a);
   return SB_OK;
 }
 
 int launch_pipe(const Args &a, long long blocks, bool a_block_a_tile, hipStream_t s) {
-  // (going on to the next tile, whose first three stages are loaded in the last of this one, takes four stages)
+  // (going on to the next tile, whose first stages are loaded in the last 128 k of this one, takes 128 k)
   if (a_block_a_tile || a.n_in < 128) {
     switch (a.gated) {
       case 3: return launch_pipe_one<3, false>(a, blocks, s);
@@ -1012,9 +1041,8 @@ constexpr Shape kShapes[6] = {{128, 128}, {256, 128}, {256, 256}, {128, 256}, {1
 
 // The tile shape for a problem: the one with the best product of three factors.  How fast the
 // shape's kernel runs on a full grid, relative to 128 x 128 (measured on MI355X at 2,048 to 16,384
-// rows of Qwen2.5-7B's four products: the 256 x 256 kernel, which loads straight into LDS, reaches
-// 1.19 to 1.31 PFLOP/s (3 to 8 % more since it reads fragments ahead) where the 128 x 128 one reaches 0.73 to 0.98; the same kernel with tiles of
-// 192 rows takes 0.84 of the time for 0.75 of the outputs); the share of the tiles' rows
+// rows of Qwen2.5-7B's four products: the 256 x 256 kernel reaches 1.34 to 1.48 PFLOP/s on a full
+// grid where the 128 x 128 one reaches 0.73 to 0.98; tiles of 192 rows loaded straight into LDS 1.04 to 1.12); the share of the tiles' rows
 // that are rows of Y; and the share of the last round of tiles over the CUs that is filled.
 // Some of what this decides at 2,048 rows: the output product (3,584 x 3,584) takes 256 x 128
 // (224 tiles, one round: 65 us against 92 with 112 tiles of 256 x 256), the QKV product 192 x 256
@@ -1023,7 +1051,7 @@ constexpr Shape kShapes[6] = {{128, 128}, {256, 128}, {256, 256}, {128, 256}, {1
 // straight into LDS takes these operands (the 192 x 256 shape has no other).
 int pick_shape(int n_rows, int n_out, int n_in, int gated, bool direct_ok, double *score_out = nullptr) {
   (void)n_in;
-  const double speed[5] = {1.0, gated ? 1.0 : 1.05, gated ? 1.25 : 1.35, 0.0, (gated ? 1.25 : 1.35) * 0.89};
+  const double speed[5] = {1.0, gated ? 1.0 : 1.05, 1.45, 0.0, gated ? 1.11 : 1.2};
   double best = 0;
   int pick = 0;
   for (int v = 0; v < 5; ++v) {
@@ -1142,16 +1170,7 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
     const bool one_round = (blocks + kXcds - 1) / kXcds * kXcds <= sb::cu_count();
     if (variant == 0) rc = one_round ? launch_direct<4, 2, 64, 4, false>(a, blocks, 0, s) : launch_direct<4, 2, 64, 2, false>(a, blocks, 0, s);
     else if (variant == 1) rc = launch_direct<8, 2, 64, 2, false>(a, blocks, 0, s);
-    else if (variant == 2) {
-      // Which 256 x 256 kernel: the one that reads fragments ahead of the barrier for gated products (37,888 x 3,584, 2,048
-      // rows 461 -> 452 us, 512 rows 191 -> 181; 9,728 x 896, 12,000 rows 220 -> 209) and long K (3,584 x 18,944, 2,048 rows 399
-      // -> 371); otherwise, up to a round of tiles or with K below 8,192, the one a whole stage ahead, whose start and epilogue
-      // are shorter (4,608 x 3,584, 3,000 rows 85 for 81; 2,048 x 1,536, 6,400 rows 44 for 42; 3,584 x 3,584, 4,096 rows 88 for
-      // 83; 1,536 x 8,960, 2,048 rows 163 for 159, but at 12,000 rows 401 and 405).  The same bits.
-      const bool ahead = a.gated || n_in >= 16384 || (n_in >= 8192 && blocks > sb::cu_count());
-      if (ahead || path == 3) rc = launch_pipe(a, blocks, path == 3, s);      // (path 3: a measurement's)
-      else rc = launch_direct_one<8, 4, 64, 2, 0, true>(a, blocks, sb::cu_count(), s);
-    }
+    else if (variant == 2) rc = launch_pipe(a, blocks, path == 3, s);      // (path 3: a measurement's)
     else if (variant == 3) rc = launch_direct<4, 4, 64, 2, false>(a, blocks, 0, s);
     else if (variant == 4) rc = launch_direct<6, 4, 64, 2, true>(a, blocks, sb::cu_count(), s);
     else rc = one_round ? launch_direct<2, 2, 64, 4, false>(a, blocks, 0, s) : launch_direct<2, 2, 64, 2, false>(a, blocks, 0, s);
@@ -1203,7 +1222,7 @@ PartialPlan partial_plan(int n_rows, int n_out, int n_in, bool direct_ok) {
   const long long big_grid = (big + kXcds - 1) / kXcds * kXcds;       // the grid is padded to whole eights
   if (s == 1 && direct_ok && 2 * big_grid <= sb::cu_count()) {
     const double per_cu = 0.93e9 / 256.0;                                        // a CU's flops per microsecond at speed 1
-    const double speed[5] = {1.0, 1.05, 1.35, 0.0, 1.35 * 0.89};
+    const double speed[5] = {1.0, 1.05, 1.45, 0.0, 1.2};
     double t_whole = 0;
     for (int v = 0; v < 5; ++v) {
       if (v == 3) continue;

@@ -415,6 +415,26 @@ def test_gemm_bf16_both_kernels_of_the_largest_tiles_give_the_same_bits(t, n, k)
     assert (got["direct"] - other).abs().max().item() <= 3e-5 * math.sqrt(k)
 
 
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 384, 448, 512, 1088])
+@pytest.mark.parametrize("t, n", [(1, 5), (257, 300), (4400, 4200)])
+def test_gemm_bf16_largest_tiles_of_every_few_stages(t, n, k):
+    """256 x 256 tiles of one to eight 64s of k: shorter and longer than the rings of buffers that the loads run ahead in,
+    every position of the rings at a tile's end, in one tile, a few, and blocks that go on to a second one; gated too."""
+    from sonicboom_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(k)
+    x = torch.randn(t, k, generator=gen, device=DEV).to(BF16)
+    w = (torch.randn(n // 2 * 2, k, generator=gen, device=DEV) * 0.05).to(BF16)
+    want = x.double() @ w.double().T
+    for path in ("direct", "direct, a block a tile"):
+        with ops.gemm_tile_shape(2, path):
+            got = ops.gemm_bf16(x, ops.pack_weight(w), None, None, F32, packed_shape=tuple(w.shape))
+            # k terms of size 0.05, 2^-24 each of sums of size sqrt(k) 0.05
+            assert (got - want).abs().max().item() <= 3e-5 * math.sqrt(k), path
+            got = ops.gemm_bf16(x, ops.pack_weight(w, True), None, None, F32, gated=True, packed_shape=tuple(w.shape))
+            g, u = want.chunk(2, dim=1)
+            assert (got - g * torch.sigmoid(g) * u).abs().max().item() <= 1e-4 * math.sqrt(k), path
+
+
 def test_gemm_bf16_direct_path_refuses_what_it_cannot_take():
     from sonicboom_amd import ops
     x, w = randn(70, 96, dtype=BF16).to(DEV), randn(64, 96, dtype=BF16).to(DEV)
