@@ -22,11 +22,14 @@
 // The loads run kAhead steps of 16 k ahead in a ring of registers.  Gated (G = 2): a column tile
 // is a tile of W's first half and the same tile of the second, and Y = act(first) * second.
 //
-// What bounds it: with few rows the read of W (each wave must have enough of it in flight) and the
-// chain's latency, with many the matrix cores.  Measured on MI355X at the 0.5B layer sizes, 3 rows, against the
-// kernel with one fmaf chain a thread that stood here before: 896 x 896 107 us then, 8.7 now; 896 x 4,864
-// 597 and 15.7; the gated 9,728 x 896 110 + 4.8 (its activation) and 14.1.  520 rows: the gated product 179 + 7 and
-// 138 (66 TFLOP/s), 896 x 4,864 666 and 76.  From row-major W with swaps the 3-row products took 13.6, 19.4 and 15 us.
+// What bounds it: with few rows the chain of products (224 of them are 5 us of an 896-k product's 7.7) and, where several waves
+// share a SIMD or a CU streams much of W, those; with many the matrix cores.  The source keeps a step's loads behind its
+// products and turns X's fragments over a step ahead: left to itself the compiler turned a whole ring over at once and so
+// waited for the newest of its loads ahead of the round's first product.  Measured on MI355X at the 0.5B layer sizes, 3 rows,
+// left to itself and so: 896 x 896 8.2 and 7.7 us, the gated 9,728 x 896 16.1 and 13.5, 896 x 4,864 15.5 and 14.9, a block a
+// segment (sb_gemm_f32_packed_partial) 9.7; 520 rows: the gated product 140 and 105 us (86 TFLOP/s), 896 x 4,864 75 and 69.
+// Not kept for few rows: a wave for each half of the gated product (16 us), X's segment in LDS in the products' order with W's
+// loads twice as far ahead (12 to 17 us gated, 8.7 to 9.5 for 896 x 896: staging X costs what it saves).
 #include "mfma.h"
 
 namespace {
@@ -88,13 +91,13 @@ bool by_fours(const void *y, const float *resid, int n_out) {
 template <typename TX, typename TW, int FORM, int TT, int CT, int G, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a) {
-  constexpr int kStreams = CT * G, kTiles = TT * CT;
+  constexpr int kStreams = CT * G, kTiles = TT * CT, kThreads = 64 * WAVES;
   // steps in flight: as many as 192 registers hold (128 or less beside the accumulators of larger tiles
   // and the addresses of loads element by element)
   constexpr int kRegs = 4 * (kStreams + TT);
   constexpr int kAhead = FORM != kPacked ? 4 : kRegs == 8 ? 24 : kRegs <= 12 ? 16 : kRegs <= 16 ? 8 : 4;
-  constexpr int kUnits = (kTiles * 64 + 64 * WAVES - 1) / (64 * WAVES);   // groups of four outputs a thread
-  extern __shared__ floatx4_t part[];            // [WAVES][TT * kStreams][64]
+  constexpr int kUnits = (kTiles * 64 + kThreads - 1) / kThreads;   // groups of four outputs a thread
+  extern __shared__ floatx4_t part[];            // [WAVES][G][kTiles][64]
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -123,8 +126,10 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
   for (int u = 0; u < kUnits; ++u)
 #pragma unroll
     for (int q = 0; q < G; ++q) total[u][q] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-  const int n_seg = (a.n_in + kSegment - 1) / kSegment;
-  for (int s0 = 0; s0 < n_seg; s0 += WAVES) {
+  // a grid of as many layers as segments: each block one segment, whose raw sums are Y's plane of that number
+  const bool split = gridDim.y > 1;
+  const int n_seg = split ? int(blockIdx.y) + 1 : (a.n_in + kSegment - 1) / kSegment;
+  for (int s0 = blockIdx.y; s0 < n_seg; s0 += WAVES) {
     const int seg = s0 + wave;
     if (seg < n_seg) {                           // uniform over the wave
       const int k_end = min((seg + 1) * kSegment, a.n_in);
@@ -159,8 +164,14 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
           else rx[slot][j] = load4_any(x0 + x_at[j], k, k_end);
         }
       };
-      auto multiply = [&](int slot, auto then) {
-        float fw[kStreams][4], fx[TT][4];
+      // X's fragments are turned over a step ahead, beside the products of the step before
+      float fx[2][TT][4];
+      auto turn = [&](int slot, int set) {
+#pragma unroll
+        for (int j = 0; j < TT; ++j) by_step(rx[slot][j], fx[set][j]);
+      };
+      auto multiply = [&](int slot, int set) {
+        float fw[kStreams][4];
 #pragma unroll
         for (int i = 0; i < kStreams; ++i) {
           if constexpr (FORM == kAny) {
@@ -171,26 +182,34 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
           }
         }
 #pragma unroll
-        for (int j = 0; j < TT; ++j) by_step(rx[slot][j], fx[j]);
-        then();
-#pragma unroll
         for (int s = 0; s < 4; ++s)
 #pragma unroll
           for (int i = 0; i < kStreams; ++i)
 #pragma unroll
             for (int j = 0; j < TT; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[i][s], fx[j][s], acc[i][j], 0, 0, 0);
+              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[i][s], fx[set][j][s], acc[i][j], 0, 0, 0);
       };
+      static_assert(kAhead % 2 == 0, "the sets of turned fragments alternate");
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) ask(u, u);
+      turn(0, 0);
       int step = 0;
       for (; step + kAhead <= steps; step += kAhead) {       // whole rounds of the ring
 #pragma unroll
-        for (int u = 0; u < kAhead; ++u) multiply(u, [&]() { ask(u, step + kAhead + u); });
+        for (int u = 0; u < kAhead; ++u) {
+          turn((u + 1) % kAhead, (u + 1) & 1);
+          multiply(u, u & 1);
+          ask(u, step + kAhead + u);
+          // (left alone, the compiler turns a whole round over at once, waiting for the last of its loads ahead of the first product)
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
 #pragma unroll
       for (int u = 0; u < kAhead; ++u)
-        if (step + u < steps) multiply(u, []() {});
+        if (step + u < steps) {
+          if (u + 1 < kAhead) turn(u + 1, (u + 1) & 1);
+          multiply(u, u & 1);
+        }
 #pragma unroll
       for (int i = 0; i < kStreams; ++i)
 #pragma unroll
@@ -204,7 +223,7 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
       const int here = min(WAVES, n_seg - s0);
 #pragma unroll
       for (int u = 0; u < kUnits; ++u) {
-        const int unit = tid + u * 64 * WAVES;
+        const int unit = tid + u * kThreads;
         if (unit < kTiles * 64)
           for (int v = 0; v < here; ++v)
 #pragma unroll
@@ -218,10 +237,11 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
   // their residuals (which the stores may overwrite, each its own) asked for ahead of the first store: a product of few k is
   // bound here (4,096 x 64 onto a residual stream of 4,000 rows 105 us a number at a time, 63 by fours, 57 so; 55 the LDS tiles)
   const auto place = [&](int u, int &t, int &nb) {
-    const int unit = tid + u * 64 * WAVES, tile = unit >> 6, l = unit & 63;
+    const int unit = tid + u * kThreads, tile = unit >> 6, l = unit & 63;
     t = t0 + 16 * (tile % TT) + (l & 15), nb = n0 + 16 * (tile / TT) + 4 * (l >> 4);
     return unit < kTiles * 64 && t < a.n_rows && nb < a.n_out;
   };
+  if (split) a.y = (float *)a.y + size_t(blockIdx.y) * a.n_rows * a.n_out;
   if (a.vec4) {
     floatx4_t old[kUnits];
     if (a.resid) {
@@ -270,7 +290,7 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
 }
 
 template <typename TX, typename TW, int FORM, int TT, int CT, int G, int WAVES>
-int launch_one(const TX *x, const TW *w, const PlainArgs &a, hipStream_t s) {
+int launch_one(const TX *x, const TW *w, const PlainArgs &a, hipStream_t s, int layers = 1) {
   constexpr int lds_bytes = WAVES == 1 ? 0 : WAVES * TT * CT * G * 1024;
   auto kern = gemm_f32_kernel<TX, TW, FORM, TT, CT, G, WAVES>;
   static bool raised = false;     // per instantiation; harmless if repeated
@@ -281,7 +301,7 @@ int launch_one(const TX *x, const TW *w, const PlainArgs &a, hipStream_t s) {
   }
   const long long blocks = (long long)((a.n_out + 16 * CT - 1) / (16 * CT)) * ((a.n_rows + 16 * TT - 1) / (16 * TT));
   SB_SUPPORT(blocks <= 0x7fffffffLL, "sb_gemm: too many tiles");
-  kern<<<unsigned(blocks), 64 * WAVES, lds_bytes, s>>>(x, w, a);
+  kern<<<dim3(unsigned(blocks), layers), 64 * WAVES, lds_bytes, s>>>(x, w, a);
   return sb::check_launch("sb_gemm");
 }
 
@@ -293,9 +313,11 @@ int launch_packed(const float *x, const float *w, const PlainArgs &a, int n_seg,
   return launch_one<float, float, kPacked, TT, CT, G, 8>(x, w, a, s);
 }
 
-// The largest tile whose waves still give most of the 1,024 SIMDs one: larger tiles read X and W fewer
-// times (a wave of a 16 x 16 tile asks for 64 bytes a cycle and CU, what the cache gives; 64 x 64 for 16),
-// smaller ones leave no SIMD idle.
+// The tile for rows past sixteen.  One segment of K: the least price, rounds of waves over the SIMDs times a step's products and
+// nine tenths of its loads (tiles of both sides), so that a last round that is nearly empty counts; on a tie the larger tile.
+// 520 rows: gated 9,728 x 896 1,368 waves of 4 x 2 (tiles of both halves) 132 us, 2,736 of 4 x 1 105, 5,168 of 2 x 1 109; 1,152 x
+// 896 tiles of 2 x 2 22, 2 x 1 29, 4 x 2 38; 200 rows gated 66, 69 and 55.  Several segments: the largest tile whose waves give
+// most of the 1,024 SIMDs one (520 rows, 896 x 4,864: 4 x 2 71 us, 2 x 2 74, 2 x 1 108, 4 x 4 116).
 template <int G>
 int launch_packed_tiles(const float *x, const float *w, const PlainArgs &a, int n_seg, hipStream_t s) {
   const auto waves = [&](int tt, int ct) {
@@ -306,9 +328,24 @@ int launch_packed_tiles(const float *x, const float *w, const PlainArgs &a, int 
     if (G == 1 && waves(1, 2) >= 4 * kEnough) return launch_packed<1, 2, G>(x, w, a, n_seg, s);
     return launch_packed<1, 1, G>(x, w, a, n_seg, s);
   }
-  if (a.n_rows > 32 && waves(4, 4 / G) >= kEnough) return launch_packed<4, 4 / G, G>(x, w, a, n_seg, s);
-  if (a.n_rows > 32 && waves(4, 2 / G) >= kEnough) return launch_packed<4, 2 / G, G>(x, w, a, n_seg, s);
-  if (G == 1 && waves(2, 2) >= kEnough) return launch_packed<2, 2, G>(x, w, a, n_seg, s);
+  constexpr int kShapes[4][2] = {{4, 4 / G}, {4, 2 / G}, {2, 2 / G}, {2, 1}};      // (gated the last two are one)
+  int pick = 3;
+  if (n_seg == 1) {
+    double best = 0;
+    for (int v = 0; v < 4; ++v) {
+      const int tt = kShapes[v][0], ct = kShapes[v][1];
+      if (tt == 4 && a.n_rows <= 32) continue;
+      const double price = double((waves(tt, ct) + 1023) / 1024) * (tt * ct * G + 0.9 * (tt + ct * G));
+      if (best == 0 || price < best) best = price, pick = v;
+    }
+  } else {
+    if (a.n_rows > 32 && waves(4, 4 / G) >= kEnough) pick = 0;
+    else if (a.n_rows > 32 && waves(4, 2 / G) >= kEnough) pick = 1;
+    else if (G == 1 && waves(2, 2) >= kEnough) pick = 2;
+  }
+  if (pick == 0) return launch_packed<4, 4 / G, G>(x, w, a, n_seg, s);
+  if (pick == 1) return launch_packed<4, 2 / G, G>(x, w, a, n_seg, s);
+  if (pick == 2) return launch_packed<2, 2 / G, G>(x, w, a, n_seg, s);
   return launch_packed<2, 1, G>(x, w, a, n_seg, s);
 }
 
@@ -461,4 +498,25 @@ extern "C" int sb_gemm_f32_packed(void *y, int y_dtype, const float *x, const fl
                       : launch_one<float, float, kPackedAny, 2, 1, 1, 8>(x, w, a, s);
   }
   return gated ? launch_packed_tiles<2>(x, w, a, n_seg, s) : launch_packed_tiles<1>(x, w, a, n_seg, s);
+}
+
+// Segments of a row of K, the planes that sb_gemm_f32_packed_partial writes.
+extern "C" int sb_gemm_f32_segments(int n_in) { return (n_in + kSegment - 1) / kSegment; }
+
+// The raw product of float32 X and packed float32 W a segment at a time: partial float [segments][n_rows][n_out], which added
+// in ascending order are the bits of sb_gemm_f32_packed.  A block a segment and sixteen columns: with few rows the whole
+// product's blocks, whose waves take the segments between them, are a few dozen (3 rows against 896 x 4,864: 56 blocks and
+// 14.9 us, 280 and 9.7).
+extern "C" int sb_gemm_f32_packed_partial(float *partial, const float *x, const float *w, int n_rows, int n_out, int n_in, void *stream) {
+  SB_REQUIRE(partial && x && w, "sb_gemm_f32_packed_partial: null pointer");
+  SB_REQUIRE(n_rows >= 0 && n_out > 0 && n_in > 0, "sb_gemm_f32_packed_partial: bad sizes rows=%d out=%d in=%d", n_rows, n_out, n_in);
+  SB_SUPPORT(n_rows <= 16, "sb_gemm_f32_packed_partial: %d rows, at most 16", n_rows);
+  SB_SUPPORT(n_in % 4 == 0 && size_t(n_in) * 64 * 4 < (size_t(1) << 31), "sb_gemm_f32_packed_partial: inner size %d", n_in);
+  SB_SUPPORT((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w)) % 16 == 0,
+             "sb_gemm_f32_packed_partial: operands must be 16-byte aligned");
+  if (n_rows == 0) return SB_OK;
+  const int n_seg = sb_gemm_f32_segments(n_in);
+  SB_SUPPORT(n_seg >= 2 && n_seg <= 65535, "sb_gemm_f32_packed_partial: %d segments", n_seg);
+  const PlainArgs a{partial, SB_F32, nullptr, 0, nullptr, n_rows, n_out, n_in, SB_GATE_NONE, by_fours(partial, nullptr, n_out)};
+  return launch_one<float, float, kPacked, 1, 1, 1, 1>(x, w, a, (hipStream_t)stream, n_seg);
 }

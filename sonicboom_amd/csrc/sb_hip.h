@@ -120,6 +120,8 @@ int sb_gemm(void *y, int y_dtype, const void *x, int x_dtype, const void *w, int
  * halves of n_out rows, each packed by itself, and Y = act(X Wg^T) * (X Wu^T). */
 int sb_gemm_f32_packed(void *y, int y_dtype, const float *x, const float *w, const void *bias, int bias_dtype,
                        const float *resid, int n_rows, int n_out, int n_in, int gated, void *stream);
+int sb_gemm_f32_segments(int n_in);
+int sb_gemm_f32_packed_partial(float *partial, const float *x, const float *w, int n_rows, int n_out, int n_in, void *stream);
 
 /* bf16 products of up to 16 rows against packed weights whose blocks own their output features whole.
  * join: resid[t,n] += sum_k X[t,k] W[n,k] (+ bias[n]), resid f32 [n_rows][n_out] in place, and an RMS norm of it whose factor

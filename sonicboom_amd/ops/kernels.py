@@ -200,6 +200,28 @@ def gemm_f32(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], res
     return out
 
 
+F32_PARTIAL_MAX_ROWS = 16
+
+
+def gemm_f32_partial(x: torch.Tensor, w: torch.Tensor, packed_shape) -> Optional[torch.Tensor]:
+    """The product of few float32 rows in its segments of K, float32 [segments, rows, n], for :func:`reduce_resid_norm` to add
+    in order: the bits of :func:`gemm_f32`, from several times the blocks.  None for more rows, one segment or more than
+    that pass adds, and rows that cannot be read sixteen bytes at a time."""
+    _dev(x, w)
+    n, k = packed_shape
+    if x.dtype != torch.float32 or w.dtype != torch.float32 or x.dim() != 2 or x.shape[1] != k:
+        raise KernelLibraryError(f"gemm_f32_partial takes float32 rows of {k} and packed float32 weights, not {tuple(x.shape)} {x.dtype}")
+    if w.numel() != ((n + 15) // 16 * 16) * ((k + 15) // 16 * 16):
+        raise KernelLibraryError(f"{w.numel()} packed elements are not a weight of {packed_shape}")
+    t, lib = x.shape[0], library.core()
+    segments = lib.sb_gemm_f32_segments(k)
+    if not 0 < t <= F32_PARTIAL_MAX_ROWS or not 2 <= segments <= 8 or k % 4 or x.data_ptr() % 16 or not x.is_contiguous():
+        return None
+    part = torch.empty((segments, t, n), dtype=torch.float32, device=x.device)
+    check(lib.sb_gemm_f32_packed_partial(_p(part), _p(x), _p(w), t, n, k, _stream()))
+    return part
+
+
 GATES = {"silu": 1, "gelu_tanh": 2, "relu": 3}      # sb_gate of csrc/sb_hip.h
 
 

@@ -25,6 +25,8 @@ _CORE_SIGNATURES = {
     "sb_gemm_split_join_bf16": [_P, _P, _P, _P, _I, _P, _P, _P, _I, _I, _I, _I, _P],
     "sb_gemm_split_gated_bf16": [_P, _P, _P, _I, _F, _P, _I, _I, _I, _I, _P],
     "sb_gemm_f32_packed": [_P, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _P],
+    "sb_gemm_f32_segments": [_I],
+    "sb_gemm_f32_packed_partial": [_P, _P, _P, _I, _I, _I, _P],
     "sb_gemm_bf16_kernel": [_I, _I, _I, _I],
     "sb_dense_layers": [_P, _P, _I, _P],
     "sb_silu_mul": [_P, _I, _P, _I, _I, _I, _P],

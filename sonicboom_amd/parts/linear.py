@@ -97,6 +97,9 @@ class Linear:
         part = self.partial(x)
         fuse = then_norm is not None and getattr(then_norm, "fusable", False)
         groups = int(getattr(then_norm, "groups", 1)) if fuse else 1
+        if self.packed_f32 is not None and not self.gated and scale == 1.0 and groups == 1 and x.dtype == torch.float32 \
+                and resid.data_ptr() % 16 == 0 and ops.reduce_resid_norm_ok(self.n_out):
+            part = ops.gemm_f32_partial(x, self.packed_f32, (self.rows, self.n_in))
         if part is not None and ops.reduce_resid_norm_ok(self.n_out, scale, groups):
             return ops.reduce_resid_norm(part, self.bias, resid, then_norm.weight if fuse else None,
                                          then_norm.eps if fuse else 0.0, out_dtype if fuse else None,

@@ -179,6 +179,42 @@ def test_gemm_f32_packed_gives_the_bits_of_the_plain_product(t, n, k):
         assert torch.equal(gated, ops.silu_mul(both, F32))
 
 
+@pytest.mark.parametrize("t, n, k", [(18, 4880, 64), (64, 2100, 896), (200, 1216, 896), (520, 1152, 900), (1100, 272, 512), (1100, 1152, 896)])
+def test_gemm_f32_every_tile_of_one_segment_gives_the_same_bits(t, n, k):
+    """One segment of K: sizes on either side of what chooses among the tiles for more than sixteen rows, plain and gated."""
+    from sonicboom_amd import ops
+    x, w = randn(t, k).to(DEV), randn(n, k, scale=0.05).to(DEV)
+    want = ops.gemm_plain(x, w, None, None, F32)
+    assert torch.equal(ops.gemm_f32(x, ops.pack_weight_f32(w), None, None, F32, (n, k)), want)
+    gated = ops.gemm_f32(x, ops.pack_weight_f32(w, True), None, None, F32, (n, k), gated="silu")
+    assert torch.equal(gated, ops.silu_mul(want, F32))
+
+
+@pytest.mark.parametrize("t", [1, 3, 16])
+@pytest.mark.parametrize("n, k", [(896, 4864), (33, 1028), (300, 2048), (17, 8192)])
+def test_gemm_f32_segments_add_up_to_the_same_bits(t, n, k):
+    """The planes of K's segments, added in order, and through the pass that adds them to a residual and norms."""
+    from sonicboom_amd import ops
+    from sonicboom_amd.parts.linear import Linear
+    x, w, resid = randn(t, k).to(DEV), randn(n, k, scale=0.05).to(DEV), randn(t, n).to(DEV)
+    packed = ops.pack_weight_f32(w)
+    part = ops.gemm_f32_partial(x, packed, (n, k))
+    total = part[0].clone()
+    for plane in part[1:]:
+        total = total + plane
+    assert torch.equal(total, ops.gemm_f32(x, packed, None, None, F32, (n, k)))
+    want = ops.gemm_f32(x, packed, None, resid, F32, (n, k))
+    got = resid.clone()
+    Linear(w, None, fast=True).add_into(x, got)
+    assert torch.equal(got, want)
+    if n % 4 == 0:
+        assert torch.equal(ops.reduce_resid_norm(part, None, resid, torch.ones(n, device=DEV), 1e-6, F32),
+                           ops.rmsnorm(want, torch.ones(n, device=DEV), 1e-6, F32))
+    for rows, inner in ((17, k), (t, 1024), (t, 8196), (t, 1030)):     # more rows, one segment, nine, no whole fours
+        assert ops.gemm_f32_partial(torch.zeros(rows, inner, device=DEV), torch.zeros((n + 15) // 16 * 16 * ((inner + 15) // 16 * 16), device=DEV),
+                                    (n, inner)) is None
+
+
 @pytest.mark.parametrize("t", [1, 5, 16, 17, 33, 64, 65, 128, 300])
 @pytest.mark.parametrize("n, k", [(96, 64), (100, 96), (224, 200), (3584, 512), (1000, 3584), (72, 18944 // 8)])
 def test_gemm_bf16_matrix_cores(t, n, k):
@@ -444,6 +480,22 @@ def test_gemm_bf16_direct_path_refuses_what_it_cannot_take():
     with ops.gemm_tile_shape(3, "registers"):
         with pytest.raises(ops.KernelLibraryError, match="direct path only"):
             ops.gemm_bf16(x, ops.pack_weight(w), None, None, F32, packed_shape=(64, 96))
+
+
+@pytest.mark.parametrize("waves", [0, 2, 3])
+@pytest.mark.parametrize("t, n, k", [(1, 16, 32), (17, 100, 96), (40, 1000, 520), (65, 264, 2368), (128, 33, 264)])
+def test_gemm_bf16_stream_kernel_of_few_waves(t, waves, n, k):
+    """Two and three waves a block, which matrices of few tiles take: every count of row tiles, columns that end inside a
+    tile and inside a block, K inside a staged chunk; plain and gated."""
+    from sonicboom_amd import ops
+    x, w = randn(t, k, dtype=BF16), randn(2 * n, k, dtype=BF16, scale=0.05)
+    resid, wd = randn(t, n), w.to(DEV)
+    with ops.gemm_few_rows_kernel("stream", waves):
+        got = ops.gemm_bf16(x.to(DEV), ops.pack_weight(wd[:n].contiguous()), None, resid.to(DEV), F32, packed_shape=(n, k))
+        gated = ops.gemm_bf16(x.to(DEV), ops.pack_weight(wd, True), None, None, F32, gated=True, packed_shape=(2 * n, k))
+    close(got, ref_gemm(x, w[:n], None, resid), atol=3e-5 * math.sqrt(k), rtol=1e-5, what="plain")
+    g, u = ref_gemm(x, w, None, None).double().chunk(2, dim=1)
+    close(gated, g / (1.0 + torch.exp(-g)) * u, atol=1e-4 * math.sqrt(k), rtol=1e-4, what="gated")
 
 
 @pytest.mark.parametrize("t", [1, 16, 17, 40, 64, 65, 100, 128])
