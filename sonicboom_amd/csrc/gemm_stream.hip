@@ -136,18 +136,29 @@ gemm_stream_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, S
     const bool more = c + 1 < n_chunks;
     if (more) issue_x(c + 1);
     const uint4 *buf = xs_lds + (c & 1) * kBufUnits;
+    // Past sixteen rows the order is kept as written (a step's rows read a step ahead of its products, W's next load behind the
+    // products that free its registers).  Left alone, the compiler gathers a chunk's loads of W behind its last products: 41 rows,
+    // gated 17,920 x 1,536 19.2 us, so 17.0; 1,536 x 8,960 12.0 and 11.1; 100 rows, gated 28.0 and 24.1.  With up to sixteen rows, whose
+    // products take next to no time, a chunk's loads in one burst are the better way: 8 rows, 3,584 x 18,944 25.6 us and 27.5 in
+    // order, 152,064 x 3,584 197 and 211.
+    constexpr bool kOrdered = TT > 1;
+    uint4 b[2][TT];
+    auto read_x = [&](int u) {
+#pragma unroll
+      for (int j = 0; j < TT; ++j) b[u & 1][j] = buf[(j * 16 + r) * kRowStride + u * 4 + q];
+    };
+    read_x(0);
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) {
-      uint4 b[TT];
-#pragma unroll
-      for (int j = 0; j < TT; ++j) b[j] = buf[(j * 16 + r) * kRowStride + u * 4 + q];
+      if (u + 1 < kAhead) read_x(u + 1);
 #pragma unroll
       for (int f = 0; f < F; ++f) {
 #pragma unroll
-        for (int j = 0; j < TT; ++j) acc[f][j] = mfma16(as_bf16x8(ring[u][f]), as_bf16x8(b[j]), acc[f][j]);
+        for (int j = 0; j < TT; ++j) acc[f][j] = mfma16(as_bf16x8(ring[u][f]), as_bf16x8(b[u & 1][j]), acc[f][j]);
         ring[u][f] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[f], int(w_off), 0, 0));
       }
       w_off += 1024u;
+      if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);
     }
     if (more) store_x((c + 1) & 1);
     __syncthreads();
@@ -201,17 +212,18 @@ void launch_w(const bf16_t *x, const bf16_t *w, const StreamArgs &a, hipStream_t
 }
 
 // A call's hint (for tests and measurements; 0 = the launcher chooses): bits 0..7 the waves per
-// block (4..8), bits 8..15 the K slices the partial form aims at (1..8).
+// block (2..8; cutting K 4..8), bits 8..15 the K slices the partial form aims at (1..8).
 inline int hint_waves(int hint) { return hint & 0xff; }
 inline int hint_slices(int hint) { return (hint >> 8) & 0xff; }
 
-// Waves per block: the count whose blocks fill whole rounds over the CUs best; more waves on a tie.
+// Waves per block: the count whose blocks fill whole rounds over the CUs best; more waves on a tie.  Matrices of few tiles
+// take two or three (24 rows, gated 9,728 x 896: two 7.3 us, four 8.5; 48 rows, 22,016 x 2,048: three 22.6, four 23.1, five 25.2).
 int waves_for(int tiles, int r, int force_waves) {
-  if (force_waves >= 4 && force_waves <= 8) return force_waves;
+  if (force_waves >= 2 && force_waves <= 8) return force_waves;
   const int n_cu = sb::cu_count();
-  int best = 4;
+  int best = 2;
   long long best_cost = -1;
-  for (int w = 4; w <= 8; ++w) {
+  for (int w = 2; w <= 8; ++w) {
     const int blocks = (tiles + w * r - 1) / (w * r);
     const long long cost = (long long)((blocks + n_cu - 1) / n_cu) * w;
     if (best_cost < 0 || cost <= best_cost) best = w, best_cost = cost;
@@ -263,6 +275,8 @@ void launch_cut(const bf16_t *x, const bf16_t *w, const StreamArgs &a, int waves
 template <int TT, int G, int R>
 void launch(const bf16_t *x, const bf16_t *w, const StreamArgs &a, int hint, hipStream_t s) {
   switch (waves_for((a.n_out + 15) / 16, R, hint_waves(hint))) {
+    case 2: return launch_w<TT, G, R, 2>(x, w, a, s);
+    case 3: return launch_w<TT, G, R, 3>(x, w, a, s);
     case 4: return launch_w<TT, G, R, 4>(x, w, a, s);
     case 5: return launch_w<TT, G, R, 5>(x, w, a, s);
     case 6: return launch_w<TT, G, R, 6>(x, w, a, s);
