@@ -918,6 +918,189 @@ gemm_pipe_kernel(Args a) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The same in tiles of 256 x 128, a wave 64 x 64 of it, in stages of 64 k through three buffers of each side (144 KB), for
+// products whose 256 x 256 tiles would leave half the CUs idle.  A wave's turn at the matrix cores is 512 cycles, as above, its
+// turn at LDS sixteen fragments; the loads of a stage go out two stages ahead.  What bounds it: the loads, one and a half
+// times the tile above's for a product.  Measured against four waves of 128 x 64, one a SIMD, whose tiles went through registers:
+// 2,048 x 3,584 x 3,584 69 -> 57 us, 4,001 x 2,048 x 4,096 82 -> 70, 4,001 x 2,048 x 8,192 141 -> 123, 3,000 x 2,560 x 2,048 40 -> 35.
+template <int GATED, bool PERSIST>
+__global__ void __launch_bounds__(512)
+gemm_pipe_half_kernel(Args a) {
+  constexpr int MT16 = 4, NW = 2, BM = 256, BN = 128, kWaves = 8;
+  constexpr int kRing = 3;                           // buffers of X and of W, 64 k each
+  constexpr int kBufA = BM * 8, kBufW = BN * 8;      // 16-byte chunks of a buffer
+  constexpr int kFlight = 6;                         // loads that a wave has in flight across a meeting: a stage's
+  extern __shared__ bf16x8_t lds[];
+  typedef __attribute__((address_space(3))) bf16x8_t *lds_ptr_t;
+
+  int vblock = blockIdx.x, tm, tn;
+  if (!tile_of_block(a, vblock, tm, tn)) return;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / NW, wn = wave % NW;
+  const bool late = wave >= 4;                       // a turn behind the first four
+
+  const size_t w_rows_total = size_t(GATED ? 2 : 1) * size_t(a.w_tiles) * 16;
+  const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t *>(a.x), 0, uint32_t(size_t(a.n_rows) * a.n_in * 2), 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t *>(a.w), 0, uint32_t(w_rows_total * size_t(a.w_steps) * 64), 0x00020000);
+  // sources of a wave's loads at k 0 of tile (m, n), as in the kernel above: four of X, two of W
+  uint32_t off_a[4], off_w[2];
+  auto aim_a = [&](int m) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int place = (i * kWaves + wave) * 64 + lane;
+      const int row = place / 8, c = (place % 8) ^ ((row / 2) & 7);
+      off_a[i] = uint32_t((size_t(m * BM + row) * a.n_in + c * 8) * 2);
+    }
+  };
+  auto aim_w = [&](int n) {
+    const int n0 = n * (GATED ? BN / 2 : BN);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int blk = i * kWaves + wave, rt = blk / 2;
+      const int tile = GATED ? ((rt & 3) >> 1) * a.w_tiles + n0 / 16 + (rt >> 2) * 2 + (rt & 1) : n0 / 16 + rt;
+      off_w[i] = uint32_t(((size_t(tile) * a.w_steps + blk % 2) * 512 + size_t(lane) * 8) * 2);
+    }
+  };
+  auto load = [&](int kt, int buf) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_x, (lds_ptr_t)(lds) + buf * kBufA + (i * kWaves + wave) * 64, 16, int(off_a[i]),
+                                               kt * 128, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_w, (lds_ptr_t)(lds) + kRing * kBufA + buf * kBufW + (i * kWaves + wave) * 64, 16,
+                                               int(off_w[i]), kt * 2048, 0, 0);
+  };
+  auto meet = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto landed = [&]() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kFlight) : "memory"); };
+
+  // stages of 64 k
+  const int n_k_all = a.n_in / 64;
+  const int kt_begin = a.partial ? int(blockIdx.y) * a.stages_per_slice : 0;
+  const int n_k = a.partial ? min(kt_begin + a.stages_per_slice, n_k_all) : n_k_all;
+  // A stage past the end (of the last tile, when the block goes on) is the last stage once more, into a
+  // buffer that nobody reads again, so that the count of loads in flight stays the same.
+  aim_a(tm);
+  aim_w(tn);
+  load(kt_begin, 0);
+  load(min(kt_begin + 1, n_k - 1), 1);
+  landed();
+  meet();
+
+  const int fr = lane & 15, fg = lane >> 4;
+  int a_lane[2];                  // the fragment's place in each half of a buffer of X
+#pragma unroll
+  for (int j = 0; j < 2; ++j) a_lane[j] = (wm * (16 * MT16) + fr) * 8 + ((4 * j + fg) ^ ((fr / 2) & 7));
+  const int b_lane = kRing * kBufA + wn * 8 * 64 + lane;
+
+  floatx4_t acc[MT16][4];
+  int tm_next = 0, tn_next = 0;
+  bool more = false;
+  int buf = 0;
+  // One stage: a wave's turn at the memories (its fragments, and its share of the loads two stages further on, into the
+  // buffers whose last reader was through a turn ago), then its turn at the matrix cores.
+  auto stage = [&](int kt) {
+    bf16x8_t fa[2][MT16], fb[2][4];
+    const bf16x8_t *ls_a = lds + buf * kBufA, *ls_w = lds + buf * kBufW + b_lane;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int f = 0; f < 4; ++f) fb[j][f] = ls_w[(f * 2 + j) * 64];
+#pragma unroll
+      for (int i = 0; i < MT16; ++i) fa[j][i] = ls_a[a_lane[j] + i * 128];
+    }
+    int to = kt + 2;
+    if (to >= n_k) {                                            // past the tile's end
+      if (!PERSIST || !more) {
+        to = n_k - 1;
+      } else {
+        if (to == n_k) {                                        // from here on the loads are the next tile's
+          aim_a(tm_next);
+          aim_w(tn_next);
+        }
+        to = to - n_k + kt_begin;
+      }
+    }
+    load(to, buf == 0 ? kRing - 1 : buf - 1);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (late) landed();
+    meet();
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < MT16; ++i)
+#pragma unroll
+        for (int f = 0; f < 4; ++f) acc[i][f] = mfma16(fa[j][i], fb[j][f], acc[i][f]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (!late) landed();
+    meet();
+  };
+
+  constexpr int NC = GATED ? 32 : 64, kPitch = GATED ? NC + 4 : NC;
+  static_assert(kBufA * 16 >= kWaves * 16 * kPitch * 4, "the turning areas must fit a buffer of X");
+  auto epilogue = [&](int m, int n, int a_free) {
+    const bool far = silu_far<GATED, 8 * MT16>([&](int i) { return acc[i / 8][i % 8 / 4][i % 4]; });
+    store_tile<MT16, 16, NW, NC, kPitch, !GATED>(
+        a, reinterpret_cast<float *>(lds + a_free * kBufA), m * BM, n * (GATED ? BN / 2 : BN), !GATED,
+        [&](int i, float *turn) {
+          const auto fill = [&](auto FAR) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int row = 4 * fg + e;
+              if constexpr (GATED != 0) {
+#pragma unroll
+                for (int f = 0; f < 2; ++f)
+                  turn[row * kPitch + f * 16 + fr] = tile_gate<GATED, decltype(FAR)::value>(acc[i][f][e]) * acc[i][f + 2][e];
+              } else {
+#pragma unroll
+                for (int f = 0; f < 4; ++f) turn[row * kPitch + (f ^ fg) * 16 + fr] = acc[i][f][e];
+              }
+            }
+          };
+          if (GATED == SB_GATE_SILU && far) fill(std::true_type{});
+          else fill(std::false_type{});
+        });
+  };
+
+  for (;;) {
+#pragma unroll
+    for (int i = 0; i < MT16; ++i)
+#pragma unroll
+      for (int f = 0; f < 4; ++f) acc[i][f] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    more = PERSIST && tile_of_block(a, vblock + int(gridDim.x), tm_next, tn_next);
+    if (late) meet();
+    for (int kt = kt_begin; kt < n_k; ++kt) {
+      stage(kt);
+      buf = buf == kRing - 1 ? 0 : buf + 1;
+    }
+    if (!late) meet();
+    if (!PERSIST || !more) {
+      // the last loads (of the last stage again) are still writing LDS
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    epilogue(tm, tn, buf == 0 ? kRing - 1 : buf - 1);       // the other buffers hold the next tile's first stages
+    if (!PERSIST || !more) break;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    vblock += int(gridDim.x);
+    tm = tm_next;
+    tn = tn_next;
+  }
+}
+
 template <int MT, int NW, int BK, int DEPTH, int GATED, bool PACKED, bool EVEN_K>
 int launch_one(const Args &a, long long blocks, hipStream_t s) {
   constexpr int lds_bytes = 2 * (64 * MT + 64 * NW) * (BK / 8) * 16;
@@ -999,13 +1182,15 @@ int launch_direct(const Args &a, long long blocks, int round_blocks, hipStream_t
   }
 }
 
-template <int GATED, bool PERSIST>
+template <int GATED, bool PERSIST, bool HALF>
 int launch_pipe_one(const Args &a, long long blocks, hipStream_t s) {
-  constexpr int lds_bytes = 3 * 256 * 128 + 4 * 256 * 64;      // 160 KB: all that a CU has
+  // (256 x 256: all that a CU has)
+  constexpr int lds_bytes = HALF ? 3 * (256 + 128) * 128 : 3 * 256 * 128 + 4 * 256 * 64;
+  auto kern = gemm_pipe_kernel<GATED, PERSIST>;
+  if constexpr (HALF) kern = gemm_pipe_half_kernel<GATED, PERSIST>;
   static bool raised = false;     // per instantiation; harmless if repeated
   if (!raised) {
-    const hipError_t e = hipFuncSetAttribute((const void *)gemm_pipe_kernel<GATED, PERSIST>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             lds_bytes);
+    const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     SB_REQUIRE(e == hipSuccess, "sb_gemm_mfma_bf16: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
     raised = true;
   }
@@ -1013,25 +1198,26 @@ int launch_pipe_one(const Args &a, long long blocks, hipStream_t s) {
   const unsigned slices = a.partial ? unsigned((n_k + a.stages_per_slice - 1) / a.stages_per_slice) : 1u;
   long long grid = (blocks + kXcds - 1) / kXcds * kXcds;
   if (PERSIST && grid > sb::cu_count()) grid = sb::cu_count();        // a block a CU
-  gemm_pipe_kernel<GATED, PERSIST><<<dim3(unsigned(grid), slices), 512, lds_bytes, s>>>(a);
+  kern<<<dim3(unsigned(grid), slices), 512, lds_bytes, s>>>(a);
   return SB_OK;
 }
 
+template <bool HALF>
 int launch_pipe(const Args &a, long long blocks, bool a_block_a_tile, hipStream_t s) {
   // (going on to the next tile, whose first stages are loaded in the last 128 k of this one, takes 128 k)
   if (a_block_a_tile || a.n_in < 128) {
     switch (a.gated) {
-      case 3: return launch_pipe_one<3, false>(a, blocks, s);
-      case 2: return launch_pipe_one<2, false>(a, blocks, s);
-      case 1: return launch_pipe_one<1, false>(a, blocks, s);
-      default: return launch_pipe_one<0, false>(a, blocks, s);
+      case 3: return launch_pipe_one<3, false, HALF>(a, blocks, s);
+      case 2: return launch_pipe_one<2, false, HALF>(a, blocks, s);
+      case 1: return launch_pipe_one<1, false, HALF>(a, blocks, s);
+      default: return launch_pipe_one<0, false, HALF>(a, blocks, s);
     }
   }
   switch (a.gated) {
-    case 3: return launch_pipe_one<3, true>(a, blocks, s);
-    case 2: return launch_pipe_one<2, true>(a, blocks, s);
-    case 1: return launch_pipe_one<1, true>(a, blocks, s);
-    default: return launch_pipe_one<0, true>(a, blocks, s);
+    case 3: return launch_pipe_one<3, true, HALF>(a, blocks, s);
+    case 2: return launch_pipe_one<2, true, HALF>(a, blocks, s);
+    case 1: return launch_pipe_one<1, true, HALF>(a, blocks, s);
+    default: return launch_pipe_one<0, true, HALF>(a, blocks, s);
   }
 }
 
@@ -1042,16 +1228,18 @@ constexpr Shape kShapes[6] = {{128, 128}, {256, 128}, {256, 256}, {128, 256}, {1
 // The tile shape for a problem: the one with the best product of three factors.  How fast the
 // shape's kernel runs on a full grid, relative to 128 x 128 (measured on MI355X at 2,048 to 16,384
 // rows of Qwen2.5-7B's four products: the 256 x 256 kernel reaches 1.34 to 1.48 PFLOP/s on a full
-// grid where the 128 x 128 one reaches 0.73 to 0.98; tiles of 192 rows loaded straight into LDS 1.04 to 1.12); the share of the tiles' rows
+// grid where the 128 x 128 one reaches 0.73 to 0.98; tiles of 192 rows loaded straight into LDS 1.04 to 1.12, of 256 x 128 0.92 to 1.2); the share of the tiles' rows
 // that are rows of Y; and the share of the last round of tiles over the CUs that is filled.
 // Some of what this decides at 2,048 rows: the output product (3,584 x 3,584) takes 256 x 128
-// (224 tiles, one round: 65 us against 92 with 112 tiles of 256 x 256), the QKV product 192 x 256
-// (198 tiles: 63 us against 73 with 144 of 256 x 256), the down product 256 x 128 (274 against 403 us);
+// (224 tiles, one round: 57 us against 92 with 112 tiles of 256 x 256), the QKV product 192 x 256
+// (198 tiles: 63 us against 73 with 144 of 256 x 256, 93 with 288 of 256 x 128);
 // from 4,096 rows on nearly everything takes 256 x 256.  `direct_ok`: the kernel that loads
 // straight into LDS takes these operands (the 192 x 256 shape has no other).
 int pick_shape(int n_rows, int n_out, int n_in, int gated, bool direct_ok, double *score_out = nullptr) {
   (void)n_in;
-  const double speed[5] = {1.0, gated ? 1.0 : 1.05, 1.45, 0.0, gated ? 1.11 : 1.2};
+  // (256 x 128, gated: faster by itself, but no faster beside tiles of 128 x 128, several of which share a CU: 900 rows
+  // against 22,016 x 2,048 89 us and 79)
+  const double speed[5] = {1.0, gated ? 1.0 : direct_ok ? 1.24 : 1.05, 1.45, 0.0, gated ? 1.11 : 1.2};
   double best = 0;
   int pick = 0;
   for (int v = 0; v < 5; ++v) {
@@ -1159,18 +1347,18 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
   a.w_steps = (n_in + 31) / 32;
   int rc;
   SB_SUPPORT(path < 2 || direct_ok, "sb_gemm_mfma_bf16: the direct path takes packed weights and an inner size in 64s");
-  // left to themselves the shapes of 256 columns go straight into LDS; the smaller tiles' stages are too
+  // left to themselves the shapes of 192 and 256 rows go straight into LDS; the smaller tiles' stages are too
   // short for loads that run one stage ahead, and the register path, which runs two ahead, is
   // faster there unless the tiles make one round and LDS holds four stages of each
-  const bool direct = path >= 2 || (path == 0 && direct_ok && (variant == 2 || variant == 4));
+  const bool direct = path >= 2 || (path == 0 && direct_ok && (variant == 1 || variant == 2 || variant == 4));
   SB_SUPPORT(variant < 3 || direct, "sb_gemm_mfma_bf16: the shapes 128 x 256, 192 x 256 and 64 x 128 exist on the direct path only");
   if (direct) {
     // the shapes of four waves take as many buffers as the tiles' count leaves LDS for: four (a block a CU, three
     // stages in flight) in one round over the CUs, else two (two or three blocks a CU)
     const bool one_round = (blocks + kXcds - 1) / kXcds * kXcds <= sb::cu_count();
     if (variant == 0) rc = one_round ? launch_direct<4, 2, 64, 4, false>(a, blocks, 0, s) : launch_direct<4, 2, 64, 2, false>(a, blocks, 0, s);
-    else if (variant == 1) rc = launch_direct<8, 2, 64, 2, false>(a, blocks, 0, s);
-    else if (variant == 2) rc = launch_pipe(a, blocks, path == 3, s);      // (path 3: a measurement's)
+    else if (variant == 1) rc = launch_pipe<true>(a, blocks, path == 3, s);
+    else if (variant == 2) rc = launch_pipe<false>(a, blocks, path == 3, s);      // (path 3: a measurement's)
     else if (variant == 3) rc = launch_direct<4, 4, 64, 2, false>(a, blocks, 0, s);
     else if (variant == 4) rc = launch_direct<6, 4, 64, 2, true>(a, blocks, sb::cu_count(), s);
     else rc = one_round ? launch_direct<2, 2, 64, 4, false>(a, blocks, 0, s) : launch_direct<2, 2, 64, 2, false>(a, blocks, 0, s);
@@ -1197,7 +1385,8 @@ namespace {
 // blocks, rising to 1 at 256: the chip's clock follows its load); either kernel costs 14 us
 // beside its tiles; the consumer's pass over the additional slices moves (2 slices - 2) x the
 // result's bytes at 4 TB/s.  The cut is taken when it comes out under 0.9 of the best whole
-// product (at the 3B and 1.5B products of 2,048 rows, whose 128 x 128 tiles fill the GPU in one
+// product (256 x 128 whole is priced as it was through registers: by itself the down product of 2,048 rows takes 238 us so, 268 with
+// the cut, but in a whole prompt step of the 7B sizes the two are level, and the cut's sums are two shorter ones) (at the 3B and 1.5B products of 2,048 rows, whose 128 x 128 tiles fill the GPU in one
 // round as it is, a cut priced at 0.9 to 0.97 measured 0.99 to 1.04).  Measured, whole + norm against cut + the pass that adds the slices, the
 // residual and the norm: down (3,584 x 18,944) at 1,280 rows 237 against 152 us, at 2,048 rows 272
 // against 247; output (3,584 x 3,584) at 1,280 rows 69 against 52.
@@ -1308,7 +1497,7 @@ extern "C" int sb_gemm_mfma_partial_bf16(float *partial, const void *x, const vo
   a.vec4 = n_out % 4 == 0 && reinterpret_cast<uintptr_t>(partial) % 16 == 0;
   a.stages_per_slice = (n_k + slices - 1) / slices;
   hipStream_t st = (hipStream_t)stream;
-  const int rc = plan.tile == kBig         ? launch_pipe_one<0, false>(a, blocks, st)
+  const int rc = plan.tile == kBig         ? launch_pipe_one<0, false, false>(a, blocks, st)
                  : plan.tile == kDirect128 ? launch_direct_one<4, 2, 64, 4, 0, false>(a, blocks, 0, st)
                  : plan.tile == kDirect64  ? launch_direct_one<2, 2, 64, 4, 0, false>(a, blocks, 0, st)
                                            : launch<2, 2, 64, 2, true>(a, blocks, packed, st);

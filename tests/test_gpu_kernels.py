@@ -471,6 +471,27 @@ def test_gemm_bf16_largest_tiles_of_every_few_stages(t, n, k):
             assert (got - g * torch.sigmoid(g) * u).abs().max().item() <= 1e-4 * math.sqrt(k), path
 
 
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 448, 1088])
+@pytest.mark.parametrize("t, n", [(1, 5), (257, 300), (4400, 2200)])
+def test_gemm_bf16_tall_tiles_of_every_few_stages(t, n, k):
+    """256 x 128 tiles straight into LDS, likewise; with a bias and a residual in place."""
+    from sonicboom_amd import ops
+    gen = torch.Generator(device=DEV).manual_seed(k)
+    x = torch.randn(t, k, generator=gen, device=DEV).to(BF16)
+    w = (torch.randn(n // 2 * 2, k, generator=gen, device=DEV) * 0.05).to(BF16)
+    bias, resid = torch.randn(n // 2 * 2, generator=gen, device=DEV), torch.randn(t, n // 2 * 2, generator=gen, device=DEV)
+    want = x.double() @ w.double().T
+    for path in ("direct", "direct, a block a tile"):
+        with ops.gemm_tile_shape(1, path):
+            got = resid.clone()
+            ops.gemm_bf16(x, ops.pack_weight(w), bias, got, F32, out=got, packed_shape=tuple(w.shape))
+            # k terms of size 0.05, 2^-24 each of sums of size sqrt(k) 0.05
+            assert (got - (want + bias.double() + resid.double())).abs().max().item() <= 3e-5 * math.sqrt(k), path
+            got = ops.gemm_bf16(x, ops.pack_weight(w, True), None, None, F32, gated=True, packed_shape=tuple(w.shape))
+            g, u = want.chunk(2, dim=1)
+            assert (got - g * torch.sigmoid(g) * u).abs().max().item() <= 1e-4 * math.sqrt(k), path
+
+
 def test_gemm_bf16_direct_path_refuses_what_it_cannot_take():
     from sonicboom_amd import ops
     x, w = randn(70, 96, dtype=BF16).to(DEV), randn(64, 96, dtype=BF16).to(DEV)
