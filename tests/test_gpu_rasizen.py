@@ -566,6 +566,26 @@ def test_head_products_and_activation_alone(dtype, rows, heads, n_in, n_out):
     part_close(got, R.xielu(z.numpy(), float(p[0]), float(p[1])), dtype, "xielu")
 
 
+@pytest.mark.parametrize("rows", [1000, 2001])
+@pytest.mark.parametrize("n_in, n_out", [(8, 200), (72, 196), (136, 250), (512, 193)])
+def test_head_products_of_many_rows_have_the_bits_of_few(rows, n_in, n_out):
+    """Steps whose waves take 32 and 64 rows, against the same rows a few at a time: inner sizes of one stage, of one and a
+    bit, of several; outputs that end inside a tile; no gate, one a number (on 16 bytes and off them), one a head."""
+    from sonicboom_amd import ops
+    heads = 17
+    x, w = rand(rows, heads, n_in).to(torch.bfloat16).to(DEV), rand(heads, n_out, n_in, scale=0.3).to(torch.bfloat16).to(DEV)
+    gate = rand(rows, heads * n_out + 16, seed=4).to(DEV)
+    for g in (None, gate[:, 8:8 + heads * n_out], gate[:, 3:3 + heads * n_out], gate[:, :heads]):
+        whole = torch.zeros((rows, heads, n_out), dtype=torch.bfloat16, device=DEV)
+        parts = torch.zeros_like(whole)
+        each = g is not None and g.shape[1] == heads
+        ops.head_product(x, w, whole, gate=g, gate_per_head=each)
+        for first in range(0, rows, 61):
+            some = slice(first, min(rows, first + 61))
+            ops.head_product(x[some], w, parts[some], gate=None if g is None else g[some], gate_per_head=each)
+        assert torch.equal(whole, parts)
+
+
 @pytest.mark.parametrize("heads, dim, rot_dim, vdim, rank, window", [
     (4, 32, 16, 24, 64, 0), (20, 16, 8, 16, 40, 100), (3, 64, 32, 40, 256, 70), (2, 128, 64, 128, 512, 130)])
 def test_matrix_core_latent_attention_equals_the_plain_kernel(heads, dim, rot_dim, vdim, rank, window):
