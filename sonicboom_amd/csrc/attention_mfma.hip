@@ -50,6 +50,8 @@ constexpr int KS = (HD + 31) / 32;   // k-steps of the score product
 constexpr int DT = HD / 16;          // 16-row tiles of O^T
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kPagesPerChunk = 4;
+constexpr int kWholePages = 8;               // pages of a row that one block takes whole
+constexpr bool kWholeRows = HD <= 128;       // (its waves' sums meet in 64 KB of LDS at most)
 constexpr float kMaxSlack = 8.f;
 
 // A wave's running softmax for NC groups of 16 query columns that share positions (and so the
@@ -1090,6 +1092,7 @@ __device__ __forceinline__ DecodeBlock decode_block(int tiles, int n_seqs) {
 // The end of a decode block: the waves' running sums meet in LDS and are merged in wave order
 // (thread e owns (d, column), column fastest); the result goes to `out` when the row's keys lie
 // in this chunk alone, else to the chunk's place in the partial buffers.
+template <int WAVES>
 __device__ __forceinline__ void finish_decode_block(const WaveState<1> &st, float (*lds_o)[HD * 16], float (*lds_m)[16],
                                                     float (*lds_l)[16], bf16_t *__restrict__ out,
                                                     float *__restrict__ part_o, float *__restrict__ part_ml,
@@ -1109,18 +1112,18 @@ __device__ __forceinline__ void finish_decode_block(const WaveState<1> &st, floa
     lds_l[wave][r] = l;
   }
   __syncthreads();
-  // merge the four waves (pages in ascending order); thread e owns (d, col), column fastest
+  // merge the waves (pages in ascending order); thread e owns (d, col), column fastest
   float *po = part_o + (tile_index * n_chunks) * (HD * 16);
   float *pml = part_ml + (tile_index * n_chunks) * 32;
-  for (int e = threadIdx.x; e < HD * 16; e += 256) {
+  for (int e = threadIdx.x; e < HD * 16; e += 64 * WAVES) {
     const int c = e & 15, d = e >> 4;
     float m = -__builtin_inff();
 #pragma unroll
-    for (int w = 0; w < 4; ++w) m = fmaxf(m, lds_m[w][c]);
+    for (int w = 0; w < WAVES; ++w) m = fmaxf(m, lds_m[w][c]);
     const float m_use = m == -__builtin_inff() ? 0.f : m;
     float o = 0.f, lsum = 0.f;
 #pragma unroll
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       const float f = __builtin_amdgcn_exp2f(lds_m[w][c] - m_use);
       o += lds_o[w][e] * f;
       lsum += lds_l[w][c] * f;
@@ -1251,7 +1254,7 @@ struct RopeShared {
   uint4 q[16 * kQStride];
   uint4 k[HD / 8];      // the row's own key, rotated and rounded
   bf16_t v[HD];         // and its value
-  int page_of_wave[4];  // the page numbers the block's waves have looked up (kernels with a page a wave)
+  int page_of_wave[8];  // the page numbers the block's waves have looked up (kernels with a page a wave)
 };
 
 // Work item `it` of a block of the folded form: eight elements d0 .. d0+7 of one head of the qkv
@@ -1345,7 +1348,7 @@ __device__ __forceinline__ void rope_store(RopeShared &sh, const RopeItem &first
   if (half > 0 || first_page_of_block >= 0) __syncthreads();
   if (ra.store && mine && first_page_of_block >= 0) {
     const int w = lp - first_page_of_block;
-    page = (w >= 0 && w < 4 && lp < max_pages) ? sh.page_of_wave[w] : -1;
+    page = (w >= 0 && w < int(blockDim.x >> 6) && lp < max_pages) ? sh.page_of_wave[w] : -1;
     if (page >= n_pages_total) page = -1;
   }
   const int n_q = group * kPerHead;
@@ -1429,16 +1432,20 @@ __device__ __forceinline__ void staged_q(bf16x8_t (&qf)[KS], const RopeShared &s
   }
 }
 
-template <bool BOTH, bool FUSED>
-__global__ void __launch_bounds__(256)
+// WAVES: the pages of a block, four, or eight where a table has no more: a row is then one block's, and no second kernel
+// merges chunks.  What it is bound by stays the chain of look-ups, loads and sums; measured with the merging kernel and without: 14 heads
+// of 64 on 2, one row of 145 keys 6.1 -> 4.3 us, of 500 7.3 -> 5.3; 12 of 128 on 2, 500 keys 9.2 -> 7.5; 28 of 128 on 4, eight rows of 500
+// keys 11.0 -> 9.8, 24 rows 14.9 -> 13.8.  (Sixteen waves, heads of 64, up to sixteen pages: 900 keys 7.3 -> 8.0; not taken.)
+template <bool BOTH, bool FUSED, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
 attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml,
                    const bf16_t *__restrict__ q, const RopeArgs ra,
                    const bf16_t *k_cache, const bf16_t *v_cache,
                    const int32_t *__restrict__ page_table, int max_pages, int n_pages_total,
                    const int32_t *__restrict__ row_pos, int heads_q, int heads_kv, int n_chunks,
                    float scale_log2, int window, int n_seqs) {
-  __shared__ float lds_o[4][HD * 16];   // [wave][d][col]
-  __shared__ float lds_m[4][16], lds_l[4][16];
+  __shared__ float lds_o[WAVES][HD * 16];   // [wave][d][col]
+  __shared__ float lds_m[WAVES][16], lds_l[WAVES][16];
   __shared__ std::conditional_t<FUSED, RopeShared, int> rope_sh;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int group = heads_q / heads_kv;
@@ -1449,7 +1456,7 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
   const int kvh = blk.tile / head_tiles, ht = blk.tile - kvh * head_tiles;
   // the wave's page number does not depend on the position: both look-ups go out together, and
   // before everything else, since the page's loads wait for them
-  const int pg = chunk * kPagesPerChunk + wave;
+  const int pg = chunk * WAVES + wave;
   const int page_looked_up = page_table[size_t(seq) * max_pages + min(pg, max_pages - 1)];
   const int pos = row_pos[seq];
   // the folded form: this thread's share of the qkv row depends on the block's number only, so
@@ -1462,8 +1469,8 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
   }
   const float freq = FUSED ? rope_freq(ra) : 0.f;
   const int key_lo = (window > 0 && pos >= window) ? pos - window + 1 : 0;
-  const int first_chunk = key_lo / (SB_PAGE * kPagesPerChunk);
-  const int last_chunk = min(pos / (SB_PAGE * kPagesPerChunk), n_chunks - 1);
+  const int first_chunk = key_lo / (SB_PAGE * WAVES);
+  const int last_chunk = min(pos / (SB_PAGE * WAVES), n_chunks - 1);
   if (chunk < first_chunk || chunk > last_chunk) return;   // uniform over the block
 
   const int r = lane & 15, g = lane >> 4;
@@ -1500,7 +1507,7 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
     if (lane == 0) rope_sh.page_of_wave[wave] = page_looked_up;
     rope_store(rope_sh, first, freq, ra, seq, pos, kvh, group, heads_q, heads_kv, chunk == last_chunk, !kEarly,
                const_cast<bf16_t *>(k_cache), const_cast<bf16_t *>(v_cache), page_table, max_pages, n_pages_total,
-               chunk * kPagesPerChunk);
+               chunk * WAVES);
     staged_q(qf[0], rope_sh, hq, col_ok, lane);
     if (kEarly) {
       const int slot = pos % SB_PAGE;
@@ -1513,7 +1520,7 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
                            lane);
     }
   }
-  finish_decode_block(st, lds_o, lds_m, lds_l, out, part_o, part_ml, wave, lane, chunk, first_chunk == last_chunk,
+  finish_decode_block<WAVES>(st, lds_o, lds_m, lds_l, out, part_o, part_ml, wave, lane, chunk, first_chunk == last_chunk,
                       seq, kvh, ht, group, heads_q, n_chunks, size_t(seq) * tiles + blk.tile);
 }
 
@@ -1623,7 +1630,7 @@ attn_decode_long_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, fl
     attend(h0, pg * SB_PAGE, ok);
     attend(h1, pg * SB_PAGE + 32, ok);
   }
-  finish_decode_block(st, lds_o, lds_m, lds_l, out, part_o, part_ml, wave, lane, chunk, first_chunk == last_chunk,
+  finish_decode_block<4>(st, lds_o, lds_m, lds_l, out, part_o, part_ml, wave, lane, chunk, first_chunk == last_chunk,
                       seq, kvh, ht, group, heads_q, n_chunks, size_t(seq) * tiles + blk.tile);
 }
 
@@ -1840,25 +1847,33 @@ int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra,
   }
   // a test's or a measurement's choice (0: the launcher's own)
   if (pages_per_wave > 0 && (pages_per_wave == 1 || HD <= 128)) ppw = pages_per_wave;
-  const int pages_per_chunk = kPagesPerChunk * ppw;
+  // five to eight pages a row: a block of eight waves takes a row whole (with more rows than half the CUs the chunks fill the GPU as it is)
+  const bool whole_rows = kWholeRows && ppw == 1 && pages_per_wave == 0 && max_pages > kPagesPerChunk && max_pages <= kWholePages &&
+                          per_chunk <= 128;
+  const int pages_per_chunk = whole_rows ? kWholePages : kPagesPerChunk * ppw;
   const int n_chunks = (max_pages + pages_per_chunk - 1) / pages_per_chunk;
   SB_SUPPORT((long long)n_chunks * per_chunk <= 0x7fffffffLL, "%s: too many blocks", who);
   const unsigned grid = unsigned((long long)n_chunks * per_chunk);
 #define SB_ARGS                                                                                           \
   (bf16_t *)out, part_o, part_ml, (const bf16_t *)q, ra, (const bf16_t *)k_cache, (const bf16_t *)v_cache, \
       page_table, max_pages, n_pages_total, row_pos, heads_q, heads_kv, n_chunks, scale *kLog2e, window
-  if (ppw > 1) {
+  if (whole_rows) {
+    if constexpr (kWholeRows) {
+      if (fused) attn_decode_kernel<true, true, kWholePages><<<grid, 64 * kWholePages, 0, s>>>(SB_ARGS, n_seqs);
+      else attn_decode_kernel<true, false, kWholePages><<<grid, 64 * kWholePages, 0, s>>>(SB_ARGS, n_seqs);
+    }
+  } else if (ppw > 1) {
     // (only head sizes up to 128 get here, and only they hold this kernel)
     if constexpr (HD <= 128) {
       if (fused) attn_decode_long_kernel<true><<<grid, 256, 0, s>>>(SB_ARGS, ppw, n_seqs);
       else attn_decode_long_kernel<false><<<grid, 256, 0, s>>>(SB_ARGS, ppw, n_seqs);
     }
   } else if ((long long)n_chunks * per_chunk <= 1536) {
-    if (fused) attn_decode_kernel<true, true><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
-    else attn_decode_kernel<true, false><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
+    if (fused) attn_decode_kernel<true, true, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
+    else attn_decode_kernel<true, false, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
   } else {
-    if (fused) attn_decode_kernel<false, true><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
-    else attn_decode_kernel<false, false><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
+    if (fused) attn_decode_kernel<false, true, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
+    else attn_decode_kernel<false, false, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
   }
 #undef SB_ARGS
   int rc = sb::check_launch(who);

@@ -27,6 +27,7 @@ from ..cache.paged import CacheError, pages_for
 from .step import ContextLayout, StepError, _Context, row_runs
 
 WIDTH_STEP = 16      # page-table widths are rounded up to this many pages (1024 tokens)
+SHORT_WIDTH = 8      # ... but for sequences of up to 512 tokens
 CAPTURE_AFTER = 2    # kernel-by-kernel steps of a shape before its graph is captured
 MAX_GRAPHS = 24      # recorded shapes kept; the one unused for longest goes first
 EXACT_BATCHES = 8    # batches up to this size run as they are; larger ones are padded to a bucket
@@ -148,7 +149,8 @@ class DecodeLoop:
         cache = self.engine.cache
         need = max(pages_for(cache.length(s) + 1) for s in self.slots)
         batch = batch_bucket(len(self.slots)) if self.pad_batches else len(self.slots)
-        return batch, ((need + WIDTH_STEP - 1) // WIDTH_STEP) * WIDTH_STEP
+        # (up to eight pages a table of eight: the decode attention then takes rows whole, without a second kernel)
+        return batch, SHORT_WIDTH if need <= SHORT_WIDTH else ((need + WIDTH_STEP - 1) // WIDTH_STEP) * WIDTH_STEP
 
     def _choose(self, logits: torch.Tensor, ctx, choose) -> None:
         """The step's choice on the device, into ``ctx.next_ids``: the first maximum (``choose``

@@ -503,6 +503,19 @@ def test_gemm_bf16_direct_path_refuses_what_it_cannot_take():
             ops.gemm_bf16(x, ops.pack_weight(w), None, None, F32, packed_shape=(64, 96))
 
 
+@pytest.mark.parametrize("t", [1, 3, 8, 9])
+@pytest.mark.parametrize("n, k", [(16, 32), (33, 264), (352, 2048), (1000, 520)])
+@pytest.mark.parametrize("gate", ["silu", "gelu_tanh"])
+def test_gemm_bf16_gated_few_rows_of_small_matrices(t, n, k, gate):
+    """The kernel whose waves split K inside a block, for rows without an unfinished norm (up to eight), and the one past it."""
+    from sonicboom_amd import ops
+    x, w = randn(t, k, dtype=BF16), randn(2 * n, k, dtype=BF16, scale=0.05)
+    got = ops.gemm_bf16(x.to(DEV), ops.pack_weight(w.to(DEV), True), None, None, BF16, gated=gate, packed_shape=(2 * n, k))
+    g, u = ref_gemm(x, w, None, None).double().chunk(2, dim=1)
+    act = g / (1.0 + torch.exp(-g)) if gate == "silu" else torch.nn.functional.gelu(g, approximate="tanh")
+    close(got, act * u, atol=1e-4 * math.sqrt(k), rtol=8e-3, what=gate)      # one rounding to bfloat16
+
+
 @pytest.mark.parametrize("waves", [0, 2, 3])
 @pytest.mark.parametrize("t, n, k", [(1, 16, 32), (17, 100, 96), (40, 1000, 520), (65, 264, 2368), (128, 33, 264)])
 def test_gemm_bf16_stream_kernel_of_few_waves(t, waves, n, k):
@@ -1008,6 +1021,27 @@ def test_attention_decode_matrix_cores_long_rows_of_unequal_length(window, n_seq
     pos = torch.tensor([p for _, p in rows], dtype=torch.int32)
     got = ops.attention_decode_mfma(q.to(DEV), kc, vc, table.to(DEV), pos.to(DEV), hq, hkv, hd, scale, window)
     close(got, want, atol=1.5e-2, rtol=1e-2, what=f"decode, {n_seqs} rows up to {longest} keys")
+
+
+@pytest.mark.parametrize("hq, hkv, hd", [(4, 2, 16), (5, 5, 48), (14, 2, 64), (40, 2, 64), (6, 2, 80), (28, 4, 128)])
+@pytest.mark.parametrize("window", [0, 70])
+@pytest.mark.parametrize("longest", [257, 320, 448, 449, 512, 513])
+def test_attention_decode_of_rows_that_one_block_takes_whole(hq, hkv, hd, window, longest):
+    """Heads of up to 128 numbers, tables of five to eight pages (and of nine: chunks again): lengths around the edges of
+    pages and of the eight waves, page numbers outside the cache behind the window."""
+    from sonicboom_amd import ops
+    lens = [1, 64, 65, 256, 257, longest]
+    q, kc, vc, table, rows, scale, want = attention_case(hq, hkv, hd, lens, [[n - 1] for n in lens], window, seed=4)
+    pos = torch.tensor([p for _, p in rows], dtype=torch.int32)
+    if window:
+        table[-1, 0] = -1
+        table[-1, 1] = kc.shape[0] + 5
+    got = ops.attention_decode_mfma(q.to(DEV), kc, vc, table.to(DEV), pos.to(DEV), hq, hkv, hd, scale, window)
+    close(got, want, atol=1.5e-2, rtol=1e-2, what="decode, whole rows")
+    with ops.attention_decode_pages_per_wave(hd, 1):
+        chunks = ops.attention_decode_mfma(q.to(DEV), kc, vc, table.to(DEV), pos.to(DEV), hq, hkv, hd, scale, window)
+    # the same sums of float32 numbers in another order, then one rounding to bfloat16
+    close(got, chunks.float().cpu(), atol=2.0 ** -7, rtol=2.0 ** -7, what="against chunks of four pages")
 
 
 @pytest.mark.parametrize("hq, hkv, hd", [(4, 2, 16), (5, 5, 48), (6, 2, 80), (28, 4, 128), (40, 2, 64)])
