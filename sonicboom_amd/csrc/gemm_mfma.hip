@@ -1,7 +1,7 @@
 // bf16 matrix product for many rows (prefill):  Y[t,n] = sum_k X[t,k] W[n,k]
 // on the matrix cores, with the model's epilogues fused: bias, float32
-// residual, gate activation, float32 or bfloat16 output.  Three kernels: this one, of any inner size in
-// eights and weights of either layout, and two below it that load packed weights and rows straight into LDS.
+// residual, gate activation, float32 or bfloat16 output.  Four kernels: this one, of any inner size in
+// eights and weights of either layout, and three below it that load packed weights and rows straight into LDS.
 //
 // A block of 2 x NW waves owns a BM x BN tile of Y (128 x 128, 256 x 128 or
 // 256 x 256) and walks K in stages of BK.  Both operand tiles go
