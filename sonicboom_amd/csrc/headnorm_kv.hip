@@ -11,7 +11,8 @@
 //   before the mixing is written to v_out when that is given (the first mixing layer's);
 //   with gate_out the gate_n numbers behind the values are added up over the slices and written there;
 //   q goes out in the activation type, k and v into the page of the row's position.
-// One block a row; a wave a head at a time.
+// A row's blocks (one, or in steps of few rows a block for every four heads: blockIdx.y) share its heads, a wave a head at a time,
+// and its values.
 #include "common.h"
 
 namespace {
@@ -67,7 +68,7 @@ __global__ void __launch_bounds__(THREADS) headnorm_kv_store_kernel(Args a) {
     if (page >= a.n_pages) page = -1;
   }
   const int units = a.heads_q + (a.store ? a.heads_kv : 0);
-  for (int u = wave; u < units; u += THREADS / 64) {
+  for (int u = blockIdx.y * (THREADS / 64) + wave; u < units; u += gridDim.y * (THREADS / 64)) {
     const int col = u * a.dk;
     float v[kMaxHead / 64];
     double sq = 0.0;
@@ -101,9 +102,9 @@ __global__ void __launch_bounds__(THREADS) headnorm_kv_store_kernel(Args a) {
   const int v0 = (a.heads_q + a.heads_kv) * a.dk, nv = a.heads_kv * a.dv;
   const float lam = a.v_first ? ld_dyn(a.lam, a.lam_dtype, 0) : 0.0f;
   if (a.gate_out)
-    for (int e = threadIdx.x; e < a.gate_n; e += THREADS)
+    for (int e = blockIdx.y * THREADS + threadIdx.x; e < a.gate_n; e += gridDim.y * THREADS)
       a.gate_out[size_t(row) * a.gate_n + e] = sum_slices(src + v0 + nv + e, a.n_slices, a.slice_stride);
-  for (int e = threadIdx.x; e < nv; e += THREADS) {
+  for (int e = blockIdx.y * THREADS + threadIdx.x; e < nv; e += gridDim.y * THREADS) {
     float v = sum_slices(src + v0 + e, a.n_slices, a.slice_stride);
     if (a.v_out) a.v_out[size_t(row) * nv + e] = v;
     if (a.v_first) v = (1.0f - lam) * v + lam * a.v_first[size_t(row) * nv + e];
@@ -210,11 +211,14 @@ extern "C" int sb_headnorm_kv_store(void *q_out, int q_dtype, const float *qkv, 
                inv_freq, inv_freq ? rot_dims : 0, unit, gate_out, gate_n};
   hipStream_t s = (hipStream_t)stream;
   const bool qf = q_dtype == SB_F32, cf = !store || cache_dtype == SB_F32;
-  // (a wave a head: the sums do not depend on the block's size, so few rows may take more waves a row)
+  // (a wave a head: the sums do not depend on how a row's heads are shared out.  Few rows: a block for every four heads, so that no
+  // wave waits for a second head's slices; us, a block of sixteen waves a row and so: 3 rows of 16 + 4 heads of 128 in eight
+  // slices 7.5 and 5.7, one of 32 + 8 9.8 and 5.6, 64 of 16 + 4 in three 8.0 and 6.0)
+  const int units = heads_q + (store ? heads_kv : 0);
   if (qf && cf) headnorm_kv_store_kernel<float, float, 256><<<n_rows, 256, 0, s>>>(a);
   else if (qf) headnorm_kv_store_kernel<float, bf16_t, 256><<<n_rows, 256, 0, s>>>(a);
   else if (cf && store) headnorm_kv_store_kernel<bf16_t, float, 256><<<n_rows, 256, 0, s>>>(a);
-  else if (n_rows <= 64) headnorm_kv_store_kernel<bf16_t, bf16_t, 1024><<<n_rows, 1024, 0, s>>>(a);
+  else if (n_rows <= 64) headnorm_kv_store_kernel<bf16_t, bf16_t, 256><<<dim3(n_rows, (units + 3) / 4 < 64 ? (units + 3) / 4 : 64), 256, 0, s>>>(a);
   else if (n_rows >= 512 && n_slices == 1 && !gate_out && dk % 8 == 0 && (!inv_freq || rot_dims % 16 == 0) && row_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(qkv) & 15) == 0 &&
            (reinterpret_cast<uintptr_t>(q_out) & 15) == 0 && (!store || (reinterpret_cast<uintptr_t>(k_cache) & 15) == 0)) {
     if (dk <= 64) headnorm_kv_store_wide_kernel<8><<<n_rows, 256, 0, s>>>(a);

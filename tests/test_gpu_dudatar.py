@@ -544,6 +544,28 @@ def test_rotated_head_norms(dtype, rows, heads, kv_heads, dim, vdim, rot_dims):
     assert not keys[rows:].any(), "nothing is written past the step's rows"
 
 
+@pytest.mark.parametrize("heads, kv_heads, dim, vdim", [(1, 1, 16, 16), (5, 2, 32, 48), (16, 4, 128, 128), (40, 5, 24, 8)])
+def test_heads_of_few_rows_shared_out_give_the_bits_of_a_block_a_row(heads, kv_heads, dim, vdim):
+    """Up to 64 rows several blocks share a row's heads, and its values; past it a block has the row: the
+    same rows in a step of 65 and of 64 and one, in two slices."""
+    from sonicboom_amd import ops
+    rows, width, gate_n = 65, heads * dim + kv_heads * (dim + vdim), 12
+    qkv = rand(2, rows, width + gate_n).to(DEV)
+    t = lambda a: torch.tensor(np.asarray(a), dtype=torch.int32, device=DEV)
+    inv = torch.tensor([50.0 ** (-i / 4.0) for i in range(4)], dtype=F32, device=DEV)
+    got = []
+    for cuts in ((0, 65), (0, 64, 65)):
+        kc = torch.zeros(2, kv_heads, 64, dim, dtype=torch.bfloat16, device=DEV)
+        vc = torch.zeros(2, kv_heads, vdim, 64, dtype=torch.bfloat16, device=DEV)
+        q = []
+        for a, b in zip(cuts[:-1], cuts[1:]):
+            q.append(ops.headnorm_kv_store(qkv[:, a:b].contiguous(), torch.bfloat16, None, None, 0.3, t(np.arange(a, b)), t(np.zeros(b - a)),
+                                           kc, vc, t([[1, 0]]), heads, kv_heads, dim, vdim, inv_freq=inv, rot_dims=8, unit=True))
+        got.append((torch.cat(q), kc, vc))
+    assert all(torch.equal(x, y) for x, y in zip(*got))
+    assert got[0][1].any() and got[0][2].any()
+
+
 def part_from(spec, weights, dtype, fast=True):
     """A part on the GPU from a dict of arrays by tensor name, and the arrays as the part sees them."""
     from sonicboom_amd.parts import build_part
