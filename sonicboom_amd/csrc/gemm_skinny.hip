@@ -185,6 +185,108 @@ reduce_slices_kernel(const float *__restrict__ partial, Epilogue ep, int n_slice
   store_out(ep, t, n, ep.gated ? gate_act(g, ep.gated) * u : g);
 }
 
+// Gated products of few rows against packed matrices, whole in one launch: a block keeps all S slices of K of its sixteen features
+// to itself, so nothing goes through scratch and no second kernel adds and gates.  A wave takes of every slice the k-steps that
+// the wave of its number takes in the kernel above, a chain of products for each, the chains step by step side by side; they
+// meet in LDS and are added as there, waves within a slice and then slices: the same bits.  A ring of registers runs kAhead
+// steps of every chain ahead (chains one after the other, with their ends found as the steps run, kept no load in flight across a
+// step: 10.9 us for 6.8 at 4,096 x 2,048).  What bounds it: the read of W, and where blocks are few what one CU pulls.  Measured, three rows,
+// us, weights cold, with scratch and the second kernel and so: 11,264 x 2,048 14.9 -> 12.5, 16,384 x 2,048 17.2 -> 14.2, 8,192 x 1,024 8.8 -> 5.8,
+// 4,096 x 4,096 13.6 -> 10.5, 1,024 x 2,048 6.6 -> 4.6, 9,728 x 896 (a slice, one launch there too) 7.5 -> 6.5.
+template <int S>
+__global__ void __launch_bounds__(kThreads)
+gemm_skinny_gated_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, Epilogue ep, int n_in, int steps_per_slice) {
+  constexpr int kAhead = S == 1 ? 8 : S == 2 ? 4 : S == 3 ? 3 : 2;
+  __shared__ floatx4_t chains[S * kWaves * 2 * 64];          // [slice][wave][gate, up][lane]
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r = lane & 15, q = lane >> 4;
+  const int tile = blockIdx.x, tiles = (ep.n_out + 15) / 16;
+  const int n_steps = (n_in + kStepK - 1) / kStepK;
+  int begin[S], end[S], longest = 0;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    const int lo = min(s * steps_per_slice, n_steps), hi = min(lo + steps_per_slice, n_steps), per_wave = (hi - lo + kWaves - 1) / kWaves;
+    begin[s] = min(lo + wave * per_wave, hi);
+    end[s] = min(begin[s] + per_wave, hi);
+    longest = max(longest, end[s] - begin[s]);
+  }
+
+  __amdgpu_buffer_rsrc_t rsrc_w[2];
+#pragma unroll
+  for (int g = 0; g < 2; ++g)
+    rsrc_w[g] = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(w) + size_t(g * tiles + tile) * n_steps * 512, 0,
+                                                  uint32_t(n_steps) * 1024u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t *>(x), 0, uint32_t(size_t(ep.n_rows) * n_in * 2), 0x00020000);
+  constexpr uint32_t kOutside = 0x80000000u;     // past a descriptor's end: reads as zeros
+  const uint32_t x_off = r < ep.n_rows ? uint32_t((size_t(r) * n_in + 8 * q) * 2) : kOutside;
+
+  uint4 rw[kAhead][S][2], rx[kAhead][S];
+  const auto ask = [&](int slot, int s, int j) {             // (a step past the chain's end is zeros on both sides)
+    const bool in = begin[s] + j < end[s];
+    const int step = in ? begin[s] + j : n_steps;
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+      rw[slot][s][g] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[g], lane * 16 + step * 1024, 0, 0));
+    rx[slot][s] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
+        rsrc_x, int(in && step * kStepK + 8 * q < n_in ? x_off + uint32_t(step) * 64u : kOutside), 0, 0));    // (n_in is a multiple of 8)
+  };
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+    for (int s = 0; s < S; ++s) ask(u, s, u);
+  floatx4_t acc[S][2];
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int g = 0; g < 2; ++g) acc[s][g] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+  const auto multiply = [&](int slot, int s) {
+#pragma unroll
+    for (int g = 0; g < 2; ++g) acc[s][g] = mfma16(as_bf16x8(rw[slot][s][g]), as_bf16x8(rx[slot][s]), acc[s][g]);
+  };
+  int j = 0;
+  for (; j + kAhead < longest; j += kAhead)
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+      for (int s = 0; s < S; ++s) {
+        multiply(u, s);
+        ask(u, s, j + kAhead + u);
+      }
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+    for (int s = 0; s < S; ++s) multiply(u, s);
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int g = 0; g < 2; ++g) chains[((s * kWaves + wave) * 2 + g) * 64 + lane] = acc[s][g];
+  __syncthreads();
+
+  // a thread a number of the tile, element e of lane l
+  static_assert(kThreads == 256, "a thread a number of a tile of 16 x 16");
+  const int l = tid >> 2, e = tid & 3, t = l & 15, n = tile * 16 + 4 * (l >> 4) + e;
+  if (t >= ep.n_rows || n >= ep.n_out) return;
+  const float *at = reinterpret_cast<const float *>(chains) + tid;
+  float g = 0.f, u = 0.f;
+#pragma unroll
+  for (int s = 0; s < S; ++s) {
+    float gs = 0.f, us = 0.f;
+#pragma unroll
+    for (int wv = 0; wv < kWaves; ++wv) gs += at[(s * kWaves + wv) * 512], us += at[(s * kWaves + wv) * 512 + 256];
+    g += gs, u += us;
+  }
+  store_out(ep, t, n, gate_act(g, ep.gated) * u);
+}
+
+// Whether that kernel takes a gated product.
+constexpr int kWholeRows = 8;
+bool gated_whole(int n_rows, int n_in, int packed) {
+  return packed && n_rows <= kWholeRows && (unsigned long long)(n_rows + 1) * n_in * 2 < (1ull << 31) &&
+         (unsigned long long)n_in * 32 < (1ull << 31);          // 32-bit byte offsets into X and into a stream of W
+}
+
 template <int R, int TT, int G, bool PACKED>
 void launch(const bf16_t *x, const bf16_t *w, const Epilogue &ep, float *partial, int n_in,
             int n_slices, int steps_per_slice, hipStream_t s) {
@@ -288,6 +390,16 @@ extern "C" int sb_gemm_skinny_bf16(void *y, int y_dtype, const void *x, const vo
   Epilogue ep{y, y_dtype, bias, bias_dtype, resid, n_rows, n_out, gated};
   float *partial = p.n_slices > 1 ? scratch : nullptr;
   const bf16_t *xb = (const bf16_t *)x, *wb = (const bf16_t *)w;
+  if (gated && gated_whole(n_rows, n_in, packed)) {
+    switch (p.n_slices) {
+#define SB_CASE(n) \
+  case n: gemm_skinny_gated_kernel<n><<<(n_out + 15) / 16, kThreads, 0, s>>>(xb, wb, ep, n_in, p.steps_per_slice); break
+      SB_CASE(1); SB_CASE(2); SB_CASE(3); SB_CASE(4); SB_CASE(5); SB_CASE(6); SB_CASE(7);
+      default: SB_CASE(8);
+#undef SB_CASE
+    }
+    return sb::check_launch("sb_gemm_skinny_bf16");
+  }
   if (gated && packed) launch_rt<2, true>(p.R, p.TT, xb, wb, ep, partial, n_in, p.n_slices, p.steps_per_slice, s);
   else if (gated) launch_rt<2, false>(p.R, p.TT, xb, wb, ep, partial, n_in, p.n_slices, p.steps_per_slice, s);
   else if (packed) launch_rt<1, true>(p.R, p.TT, xb, wb, ep, partial, n_in, p.n_slices, p.steps_per_slice, s);

@@ -90,7 +90,7 @@ gemm_split_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, Sp
   if constexpr (GATED) {
     const int row = tid % kMaxRows, grp = tid / kMaxRows;
     double s = 0.0;
-    if (a.ssq && row < a.n_rows) {
+    if (row < a.n_rows) {
 #pragma unroll 4
       for (int p = grp; p < a.ssq_parts; p += kGroups) s += a.ssq[size_t(p) * a.n_rows + row];
     }
@@ -139,7 +139,7 @@ gemm_split_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, Sp
     double s = 0.0;
 #pragma unroll
     for (int k = 0; k < kGroups; ++k) s += row_part[k * kMaxRows + r];
-    const float inv = a.ssq ? 1.0f / sqrtf(float(s / double(a.n_in)) + a.eps) : 1.0f;      // (no sums: rows that are normed)
+    const float inv = 1.0f / sqrtf(float(s / double(a.n_in)) + a.eps);
     if (!unit_live) return;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -208,7 +208,7 @@ extern "C" int sb_gemm_split_gated_bf16(void *y, const void *x, const double *ss
                                         int n_rows, int n_out, int n_in, int gate, void *stream) {
   const int rc = check("sb_gemm_split_gated_bf16", x, w, n_rows, n_out, n_in);
   if (rc != SB_OK) return rc;
-  SB_REQUIRE(y && (!ssq || ssq_parts > 0), "sb_gemm_split_gated_bf16: null pointer");
+  SB_REQUIRE(y && ssq && ssq_parts > 0, "sb_gemm_split_gated_bf16: null pointer");
   SB_SUPPORT(gate > SB_GATE_NONE && gate <= SB_GATE_RELU, "sb_gemm_split_gated_bf16: unknown gate activation %d", gate);
   if (n_rows == 0) return SB_OK;
   SplitArgs a{};

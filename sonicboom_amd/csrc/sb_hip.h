@@ -130,7 +130,7 @@ int sb_gemm_f32_packed_partial(float *partial, const float *x, const float *w, i
 int sb_gemm_split_join_bf16(float *resid, void *xw, double *ssq, const void *norm_w, int norm_dtype, const void *x, const void *w,
                             const void *bias, int bias_dtype, int n_rows, int n_out, int n_in, void *stream);
 /* Y = act(f X Wg^T) * (f X Wu^T), bf16 [n_rows][n_out]: f[t] = 1 / sqrt(sum of ssq[.][t] / n_in + eps) the factor of such a
- * norm X, ssq f64 [ssq_parts][n_rows] (NULL: a factor of 1); gate: an sb_gate. */
+ * norm X, ssq f64 [ssq_parts][n_rows]; gate: an sb_gate. */
 int sb_gemm_split_gated_bf16(void *y, const void *x, const double *ssq, int ssq_parts, float eps, const void *w, int n_rows,
                              int n_out, int n_in, int gate, void *stream);
 

@@ -864,11 +864,6 @@ def gemm_bf16(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], re
     if t <= STREAM_MAX_ROWS and which == "stream" and packed:
         check(lib.sb_gemm_stream_bf16(_p(out), _dt(out), _p(x), _p(w), _p(bias), bdt, _p(resid), t, n, k,
                                       gate, _hints.stream, _stream()))
-    elif gate and packed and 0 < t <= SPLIT_MAX_ROWS and which == "skinny" and _hints.few_rows_kernel is None \
-            and out.dtype == torch.bfloat16 and bias is None and resid is None:
-        # a block's waves split K and meet in LDS: no slices, no pass that adds and gates them (3 rows, us, with them and without:
-        # 11,264 x 2,048 14.6 and 13.5, 8,192 x 1,024 8.8 and 6.5, 4,096 x 4,096 13.8 and 11.3, 512 x 2,048 6.1 and 4.9)
-        check(lib.sb_gemm_split_gated_bf16(_p(out), _p(x), None, 0, 0.0, _p(w), t, n, k, gate, _stream()))
     elif t <= SKINNY_MAX_ROWS and which != "tiled":
         need = lib.sb_gemm_skinny_scratch(t, n, k, gate)
         scratch = torch.empty((need,), dtype=torch.float32, device=x.device) if need else None

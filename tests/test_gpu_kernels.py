@@ -516,6 +516,26 @@ def test_gemm_bf16_gated_few_rows_of_small_matrices(t, n, k, gate):
     close(got, act * u, atol=1e-4 * math.sqrt(k), rtol=8e-3, what=gate)      # one rounding to bfloat16
 
 
+@pytest.mark.parametrize("t", [1, 3, 8])
+@pytest.mark.parametrize("n, k", [(5, 8), (33, 264), (100, 1032), (352, 1544), (200, 2048), (100, 2600), (77, 3080), (48, 3592), (130, 4096),
+                                  (5632, 2048), (8192, 1024), (64, 8200), (3080, 5128)])
+def test_gemm_bf16_gated_few_rows_have_the_bits_of_more(t, n, k):
+    """Up to eight rows take one launch whose blocks keep the slices of K to themselves, nine go through scratch and a second
+    kernel: one to eight slices, chains of unequal length and none, matrices on either side of the counts that cut K further."""
+    from sonicboom_amd import ops
+    x, w = randn(9, k, dtype=BF16).to(DEV), randn(2 * n, k, dtype=BF16, scale=0.05).to(DEV)
+    packed = ops.pack_weight(w, True)
+    for gate in ("silu", "gelu_tanh", "relu"):
+        for dtype in (BF16, F32):
+            with ops.gemm_few_rows_kernel("skinny"):
+                want = ops.gemm_bf16(x, packed, None, None, dtype, gated=gate, packed_shape=(2 * n, k))
+                got = ops.gemm_bf16(x[:t].clone(), packed, None, None, dtype, gated=gate, packed_shape=(2 * n, k))
+                rows = ops.gemm_bf16(x[:t].clone(), w, None, None, dtype, gated=gate)
+            assert torch.equal(got, want[:t]), (gate, dtype)
+            assert torch.equal(rows, want[:t]), (gate, dtype)
+            assert torch.equal(ops.gemm_bf16(x[:t].clone(), packed, None, None, dtype, gated=gate, packed_shape=(2 * n, k)), got)
+
+
 @pytest.mark.parametrize("waves", [0, 2, 3])
 @pytest.mark.parametrize("t, n, k", [(1, 16, 32), (17, 100, 96), (40, 1000, 520), (65, 264, 2368), (128, 33, 264)])
 def test_gemm_bf16_stream_kernel_of_few_waves(t, waves, n, k):

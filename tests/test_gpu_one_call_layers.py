@@ -64,6 +64,46 @@ def test_rows_wider_than_the_pass_that_adds_slices(monkeypatch):
     same_bits(monkeypatch, config(14464, 113, 1, 64, layers=1), [[3], [16], [2, 30], [70]])
 
 
+@pytest.mark.parametrize("cfg", [config(2048, 16, 2, 8192, layers=2), config(3072, 24, 4, 8192, layers=1), config(1024, 8, 2, 4096, layers=2),
+                                 config(2048, 16, 4, 5632, layers=1)], ids=lambda c: f"{c['hidden_size']}x{c['intermediate_size']}")
+def test_gated_products_that_cut_k_have_the_same_bits(cfg, monkeypatch):
+    """Two and three slices of K in the gated product of few rows: the feed-forward's own numbers, before what follows
+    rounds them again."""
+    from sonicboom_amd import ops
+    from sonicboom_amd.engine import DecoderModel, Engine, StepEntry, dense
+    monkeypatch.setattr(dense.DenseLayers, "pays", lambda self, rows: True)
+    model = DecoderModel.from_random(cfg, 3, "bfloat16", "cuda:0")
+    engines = [Engine(model, 64 * 30, max_slots=4) for _ in range(2)]
+    engines[1].one_call_layers = False
+    mids, run, product = ([], []), ops.DenseStep.run, ops.gemm_bf16
+
+    def watched_run(self, layer, h):
+        run(self, layer, h)
+        first = self.args.mid - self.args.part               # (`part` stands at the workspace's start)
+        mids[0].append(self.kept[-1][first:first + 2 * self.args.n_rows * self.args.inner].clone().view(torch.bfloat16))
+
+    def watched_product(x, w, *args, gated=False, **kw):
+        y = product(x, w, *args, gated=gated, **kw)
+        if gated:
+            mids[1].append(y.clone().reshape(-1))
+        return y
+    monkeypatch.setattr(ops.DenseStep, "run", watched_run)
+    monkeypatch.setattr(ops, "gemm_bf16", watched_product)
+    rng = np.random.default_rng(5)
+    for lengths in ([2], [3], [2, 6], [9], [16], [40]):
+        tokens = [rng.integers(0, cfg["vocab_size"], size=n).tolist() for n in lengths]
+        slots = [[e.alloc_slot() for _ in lengths] for e in engines]
+        got, want = (e.step([StepEntry(s, t, (0, len(t) - 1)) for s, t in zip(ss, tokens)]) for e, ss in zip(engines, slots))
+        assert len(mids[0]) == len(mids[1]) == cfg["num_hidden_layers"]
+        for i, (a, b) in enumerate(zip(*mids)):
+            assert torch.equal(a, b), (lengths, i)
+        assert torch.equal(got, want), lengths
+        mids[0].clear(), mids[1].clear()
+        for e, ss in zip(engines, slots):
+            for s in ss:
+                e.free_slot(s)
+
+
 @pytest.mark.parametrize("other", [(0,), (1,), (2, 3), (1, 3)])
 def test_layers_that_differ_stand_between_those_that_do_not(monkeypatch, other):
     """They run part by part, take the norm that the layer before has left and leave the next one's."""
