@@ -280,10 +280,19 @@ gemm_skinny_gated_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict_
   store_out(ep, t, n, gate_act(g, ep.gated) * u);
 }
 
-// Whether that kernel takes a gated product.
-constexpr int kWholeRows = 8;
-bool gated_whole(int n_rows, int n_in, int packed) {
-  return packed && n_rows <= kWholeRows && (unsigned long long)(n_rows + 1) * n_in * 2 < (1ull << 31) &&
+// Whether that kernel takes a gated product.  A block streams its share of W at what one CU pulls, whatever the count of blocks,
+// so few blocks of a long K are better spread over the GPU in slices, second launch and all.  Three and eight rows, us, in slices
+// and whole: 4,096 k, 16 blocks 7.7 and 7.0, 8.2 and 7.7; 32 blocks 8.9 and 8.4, 9.0 and 9.4; 128 blocks 14.0 and 11.6, 14.4 and 13.0;
+// 6,144 k, 64 blocks 11.9 and 12.3, 12.1 and 13.8; 128 blocks 16.6 and 15.4, 17.2 and 18.0; 192 blocks 21.0 and 17.9, 22.1 and 18.9;
+// 8,192 k, 16 blocks 9.8 and 13.3, 10.1 and 15.4; 128 blocks 21.4 and 19.1, 20.4 and 21.6; 192 blocks 25.6 and 22.1, 26.9 and 23.8;
+// 320 blocks 38.5 and 41.5, 40.2 and 44.1; 512 blocks 52.6 and 50.9, 53.9 and 54.2; 16,384 k, 64 blocks 22.1 and 27.2, 22.6 and 31.9;
+// 320 blocks 69.0 and 79.7, 70.1 and 86.4.
+constexpr int kWholeRows = 8, kWholeSteps = 128, kWholeBlocks = 192, kWholeStepsOfMany = 256;
+bool gated_whole(int n_rows, int n_out, int n_in, int n_slices, int packed) {
+  const int n_steps = (n_in + kStepK - 1) / kStepK, blocks = (n_out + 15) / 16;
+  return packed && n_rows <= kWholeRows &&
+         (n_steps <= kWholeSteps || (blocks >= kWholeBlocks && n_steps <= kWholeStepsOfMany) || n_slices == 1) &&
+         (unsigned long long)(n_rows + 1) * n_in * 2 < (1ull << 31) &&
          (unsigned long long)n_in * 32 < (1ull << 31);          // 32-bit byte offsets into X and into a stream of W
 }
 
@@ -390,7 +399,7 @@ extern "C" int sb_gemm_skinny_bf16(void *y, int y_dtype, const void *x, const vo
   Epilogue ep{y, y_dtype, bias, bias_dtype, resid, n_rows, n_out, gated};
   float *partial = p.n_slices > 1 ? scratch : nullptr;
   const bf16_t *xb = (const bf16_t *)x, *wb = (const bf16_t *)w;
-  if (gated && gated_whole(n_rows, n_in, packed)) {
+  if (gated && gated_whole(n_rows, n_out, n_in, p.n_slices, packed)) {
     switch (p.n_slices) {
 #define SB_CASE(n) \
   case n: gemm_skinny_gated_kernel<n><<<(n_out + 15) / 16, kThreads, 0, s>>>(xb, wb, ep, n_in, p.steps_per_slice); break

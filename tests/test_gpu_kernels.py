@@ -518,7 +518,8 @@ def test_gemm_bf16_gated_few_rows_of_small_matrices(t, n, k, gate):
 
 @pytest.mark.parametrize("t", [1, 3, 8])
 @pytest.mark.parametrize("n, k", [(5, 8), (33, 264), (100, 1032), (352, 1544), (200, 2048), (100, 2600), (77, 3080), (48, 3592), (130, 4096),
-                                  (5632, 2048), (8192, 1024), (64, 8200), (3080, 5128)])
+                                  (5632, 2048), (8192, 1024), (64, 4104), (3056, 4104), (3057, 4104), (3070, 8192),
+                                  (3070, 8200)])
 def test_gemm_bf16_gated_few_rows_have_the_bits_of_more(t, n, k):
     """Up to eight rows take one launch whose blocks keep the slices of K to themselves, nine go through scratch and a second
     kernel: one to eight slices, chains of unequal length and none, matrices on either side of the counts that cut K further."""
