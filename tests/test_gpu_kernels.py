@@ -1501,17 +1501,8 @@ FOLDED_SHAPES = [(4, 2, 16, 16), (3, 1, 32, 32), (5, 5, 48, 16), (6, 2, 80, 64),
                  (2, 1, 256, 256)]
 
 
-@pytest.mark.parametrize("hq, hkv, hd, rot, pages", [(*sh, p) for sh in FOLDED_SHAPES for p in (0, 1, 2, 8)
-                                                     if p <= 1 or sh[2] <= 128])     # several pages per wave: up to head size 128
-@pytest.mark.parametrize("window", [0, 70])
-def test_attention_decode_with_rotation_and_store_folded_in(hq, hkv, hd, rot, window, pages):
-    """A decode step's rotation, store and attention in one kernel against the two kernels one
-    after the other: the same output and the same cache, bit for bit.  The qkv rows come as one
-    array and as three K slices with a bias; rows stand at a page's first and last slot, on the
-    first token of a sequence, and behind a window; one row has no page at all (a row added to
-    fill a batch: nothing is stored, nothing seen)."""
+def folded_against_two_kernels(hq, hkv, hd, rot, window, pages, lens):
     from sonicboom_amd import ops
-    lens = [1, 64, 65, 128, 300, 700, 1]          # the row is the sequence's last token
     n_seq = len(lens)
     width_pages = max((n + 63) // 64 for n in lens)
     perm = torch.randperm(n_seq * width_pages + 3, generator=torch.Generator().manual_seed(5))
@@ -1559,6 +1550,28 @@ def test_attention_decode_with_rotation_and_store_folded_in(hq, hkv, hd, rot, wi
             assert torch.equal(got.view(torch.int16), want.view(torch.int16))
             assert torch.equal(kc3.view(torch.int16), kc1.view(torch.int16))
     assert not ops.attention_decode_rope_ok(arg, BF16, BF16, 34, 2, hd, rot)          # 17 heads per kv head
+
+
+@pytest.mark.parametrize("hq, hkv, hd, rot, pages", [(*sh, p) for sh in FOLDED_SHAPES for p in (0, 1, 2, 8)
+                                                     if p <= 1 or sh[2] <= 128])     # several pages per wave: up to head size 128
+@pytest.mark.parametrize("window", [0, 70])
+def test_attention_decode_with_rotation_and_store_folded_in(hq, hkv, hd, rot, window, pages):
+    """A decode step's rotation, store and attention in one kernel against the two kernels one
+    after the other: the same output and the same cache, bit for bit.  The qkv rows come as one
+    array and as three K slices with a bias; rows stand at a page's first and last slot, on the
+    first token of a sequence, and behind a window; one row has no page at all (a row added to
+    fill a batch: nothing is stored, nothing seen)."""
+    folded_against_two_kernels(hq, hkv, hd, rot, window, pages, [1, 64, 65, 128, 300, 700, 1])
+
+
+@pytest.mark.parametrize("hq, hkv, hd, rot", FOLDED_SHAPES)
+@pytest.mark.parametrize("window", [0, 70])
+@pytest.mark.parametrize("lens", [[1, 64, 256, 257, 320, 1], [100, 150, 350, 1], [400, 1], [1, 257, 320, 321, 384, 385, 448, 449, 512, 1]],
+                         ids=lambda n: f"to{max(n)}")
+def test_attention_decode_folded_in_where_one_block_takes_a_row(hq, hkv, hd, rot, window, lens):
+    """The same where a table has five to eight pages and eight waves take a row (heads of up to 128 numbers): the row's own
+    page with each of the eight waves, at its first and last slots and inside."""
+    folded_against_two_kernels(hq, hkv, hd, rot, window, 0, lens)
 
 
 @pytest.mark.parametrize("vocab", [5, 256, 1000, 152064])
