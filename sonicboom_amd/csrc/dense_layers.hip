@@ -17,7 +17,8 @@ constexpr int kStreamMaxRows = 128;
 // other kernel, which spreads K over the whole GPU, has more bytes to move than a block's share
 // takes: gate/up pairs of 8,960 x 1,536 (140 blocks) 13 to 18 us against 18 to 29 at up to 64 rows,
 // 11,008 x 2,048 (172 blocks) 19 to 25 against 25 to 34; 8,192 x 2,048 (128 blocks) 18 against 16,
-// and 4,864 x 896 (76 blocks) 4 % slower in a whole decode step.
+// and 4,864 x 896 (76 blocks) 4 % slower in a whole decode step.  (Measured with four waves a block and more; matrices of 544 to 768
+// tiles take three now, and are on this side of the line either way.)
 constexpr int kStreamMinBlocks = 136;
 constexpr int kStreamMinBlocksMoreRows = 192;        // for 65 to 128 rows
 

@@ -14,7 +14,7 @@
 //
 // A CU works through its blocks at a rate that co-resident blocks share, so the time
 // is set by the CU with the most work: 296 blocks of four waves on 256 CUs take 1.4
-// times as long as 256.  The launcher therefore picks the waves per block (4 to 8) so
+// times as long as 256.  The launcher therefore picks the waves per block (3 to 8, with K cut 4 to 8) so
 // that the blocks fill a whole number of rounds over the CUs as nearly as possible
 // (gate/up of 18,944 features: 237 blocks of five waves, 47 against 68 us at 64 rows).
 //
@@ -212,18 +212,18 @@ void launch_w(const bf16_t *x, const bf16_t *w, const StreamArgs &a, hipStream_t
 }
 
 // A call's hint (for tests and measurements; 0 = the launcher chooses): bits 0..7 the waves per
-// block (2..8; cutting K 4..8), bits 8..15 the K slices the partial form aims at (1..8).
+// block (3..8; cutting K 4..8), bits 8..15 the K slices the partial form aims at (1..8).
 inline int hint_waves(int hint) { return hint & 0xff; }
 inline int hint_slices(int hint) { return (hint >> 8) & 0xff; }
 
-// Waves per block: the count whose blocks fill whole rounds over the CUs best; more waves on a tie.  Matrices of few tiles
-// take two or three (24 rows, gated 9,728 x 896: two 7.3 us, four 8.5; 48 rows, 22,016 x 2,048: three 22.6, four 23.1, five 25.2).
+// Waves per block: the count whose blocks fill whole rounds over the CUs best; more waves on a tie.  Three where that is a single
+// round, 544 to 768 tiles (fewer are left to the kernel that cuts K): 48 rows, 22,016 x 2,048 three 22.6 us, four 23.1, five 25.2.
 int waves_for(int tiles, int r, int force_waves) {
-  if (force_waves >= 2 && force_waves <= 8) return force_waves;
+  if (force_waves >= 3 && force_waves <= 8) return force_waves;
   const int n_cu = sb::cu_count();
-  int best = 2;
+  int best = 3;
   long long best_cost = -1;
-  for (int w = 2; w <= 8; ++w) {
+  for (int w = 3; w <= 8; ++w) {
     const int blocks = (tiles + w * r - 1) / (w * r);
     const long long cost = (long long)((blocks + n_cu - 1) / n_cu) * w;
     if (best_cost < 0 || cost <= best_cost) best = w, best_cost = cost;
@@ -275,7 +275,6 @@ void launch_cut(const bf16_t *x, const bf16_t *w, const StreamArgs &a, int waves
 template <int TT, int G, int R>
 void launch(const bf16_t *x, const bf16_t *w, const StreamArgs &a, int hint, hipStream_t s) {
   switch (waves_for((a.n_out + 15) / 16, R, hint_waves(hint))) {
-    case 2: return launch_w<TT, G, R, 2>(x, w, a, s);
     case 3: return launch_w<TT, G, R, 3>(x, w, a, s);
     case 4: return launch_w<TT, G, R, 4>(x, w, a, s);
     case 5: return launch_w<TT, G, R, 5>(x, w, a, s);

@@ -938,7 +938,7 @@ def gemm_few_rows_kernel(which: Optional[str], waves: int = 0, slices: int = 0):
     """For tests and measurements: inside the block this thread's products of up to 64 rows,
     whole or in K slices, go to the kernel ``which`` ("stream", "skinny" or "tiled"; "stream"
     needs packed weights) whatever the sizes, and the stream kernel uses ``waves`` waves per block
-    (4 to 8) and aims at ``slices`` K slices (1 to 8); 0: its own choice."""
+    (3 to 8, with K cut 4 to 8) and aims at ``slices`` K slices (1 to 8); 0: its own choice."""
     if which not in (None, "stream", "skinny", "tiled"):
         raise ValueError(f"unknown kernel {which!r}")
     before = (_hints.few_rows_kernel, _hints.stream)

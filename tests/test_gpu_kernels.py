@@ -537,10 +537,10 @@ def test_gemm_bf16_gated_few_rows_have_the_bits_of_more(t, n, k):
             assert torch.equal(ops.gemm_bf16(x[:t].clone(), packed, None, None, dtype, gated=gate, packed_shape=(2 * n, k)), got)
 
 
-@pytest.mark.parametrize("waves", [0, 2, 3])
+@pytest.mark.parametrize("waves", [0, 3])
 @pytest.mark.parametrize("t, n, k", [(1, 16, 32), (17, 100, 96), (40, 1000, 520), (65, 264, 2368), (128, 33, 264)])
 def test_gemm_bf16_stream_kernel_of_few_waves(t, waves, n, k):
-    """Two and three waves a block, which matrices of few tiles take: every count of row tiles, columns that end inside a
+    """Three waves a block, which matrices of few tiles take: every count of row tiles, columns that end inside a
     tile and inside a block, K inside a staged chunk; plain and gated."""
     from sonicboom_amd import ops
     x, w = randn(t, k, dtype=BF16), randn(2 * n, k, dtype=BF16, scale=0.05)
