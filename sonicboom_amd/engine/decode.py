@@ -27,9 +27,10 @@ from ..cache.paged import CacheError, pages_for
 from .step import ContextLayout, StepError, _Context, row_runs
 
 WIDTH_STEP = 16      # page-table widths are rounded up to this many pages (1024 tokens)
-SHORT_WIDTH = 8      # ... but for sequences of up to 512 tokens
+SHORT_WIDTH = 8      # ... but for sequences of up to 512 tokens, a shape of their own
 CAPTURE_AFTER = 2    # kernel-by-kernel steps of a shape before its graph is captured
-MAX_GRAPHS = 24      # recorded shapes kept; the one unused for longest goes first
+MAX_GRAPHS = 40      # recorded shapes kept (some 25 MB each); the one unused for longest goes first.  (Batches that end one by
+                     # one from 48 pass through thirteen sizes, either side of 512 tokens.)
 EXACT_BATCHES = 8    # batches up to this size run as they are; larger ones are padded to a bucket
 
 
@@ -130,6 +131,7 @@ class DecodeLoop:
         self._ctx: Dict[Tuple[int, int], _StaticContext] = {}
         self._graphs: Dict[tuple, Tuple[torch.cuda.CUDAGraph, torch.Tensor]] = {}    # (batch, width, choice)
         self._uses: Dict[tuple, int] = {}
+        self._recorded = False
         self.slots: List[int] = []
         self.pending: List[int] = []
 
@@ -149,7 +151,9 @@ class DecodeLoop:
         cache = self.engine.cache
         need = max(pages_for(cache.length(s) + 1) for s in self.slots)
         batch = batch_bucket(len(self.slots)) if self.pad_batches else len(self.slots)
-        # (up to eight pages a table of eight: the decode attention then takes rows whole, without a second kernel)
+        # (Up to eight pages a table of eight: the decode attention then takes rows whole, without a second kernel.  0.5B sizes, one
+        # sequence: 0.055 ms less a step, against 4 ms once where a sequence grows past them: a first generation from 137 to 700
+        # tokens, recordings included, 592 ms with one width and 585 so (runs differ by 20), once recorded 537 and 517; from 480 to 560 132 and 136, 76 and 74.)
         return batch, SHORT_WIDTH if need <= SHORT_WIDTH else ((need + WIDTH_STEP - 1) // WIDTH_STEP) * WIDTH_STEP
 
     def _choose(self, logits: torch.Tensor, ctx, choose) -> None:
@@ -214,8 +218,12 @@ class DecodeLoop:
         # Python's collector must not run inside the capture: what it finalizes (the pinned
         # buffers of earlier steps' contexts, graphs of loops long gone, anything that waited in
         # a reference cycle) calls into the HIP runtime, which refuses such calls on a capturing
-        # stream, and the process aborts.  So it runs now, and not again until the capture ends.
-        gc.collect()
+        # stream, and the process aborts.  So it runs now, and not again until the capture ends:
+        # over everything for a loop's first recording, when other engines may just have gone,
+        # then over what is young.  (All of it takes 23 to 30 ms, the recording itself 2: a sequence
+        # that grows past 512 tokens changes its shape on the way.)
+        gc.collect(1 if self._recorded else 2)
+        self._recorded = True
         collecting = gc.isenabled()
         gc.disable()
         try:

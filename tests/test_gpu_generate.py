@@ -204,6 +204,33 @@ def test_the_collector_stays_out_of_graph_captures(model_folders):
     assert gc.isenabled()
 
 
+def test_a_sequence_that_outgrows_its_shape_pays_no_full_collection(monkeypatch):
+    """Past 512 tokens a step's page table gets wider, so a second shape is recorded in the middle of a generation: all of
+    Python's objects are looked over for a loop's first recording alone.  The tokens are those of steps kernel by kernel."""
+    import gc
+    from sonicboom_amd.engine import decode
+    from sonicboom_amd.engine import DecoderModel, Engine, generate
+    from sonicboom_amd.sampling import SamplingParams
+    model = DecoderModel.from_random(dict(TINY["A"], max_position_embeddings=2048), 3, "bfloat16", "cuda:0")
+    prompt = prompts_for("A", [503], seed=4)
+    collected = []
+
+    class Watched:
+        def __getattr__(self, name):
+            return getattr(gc, name)
+
+        def collect(self, generation=2):
+            collected.append(generation)
+            return gc.collect(generation)
+    monkeypatch.setattr(decode, "gc", Watched())
+    engines = [Engine(model, 64 * 12) for _ in range(2)]
+    engines[1].use_graphs = False
+    got, want = (generate(e, prompt, SamplingParams(max_tokens=24), stop_tokens=()) for e in engines)
+    assert got == want and len(got[0]) == 24
+    assert sorted(k[1] for k in engines[0].decode_loop()._graphs) == [8, 16]
+    assert collected == [2, 1]
+
+
 def test_batches_run_in_buckets_with_rows_that_do_nothing(model_folders):
     """The decode loop runs a batch of more than eight sequences at the next bucket's size (12,
     16, 24, ...): the rows it adds have no pages, store nothing and see no key.  A batch of 21
