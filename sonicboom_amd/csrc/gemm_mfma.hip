@@ -1380,16 +1380,21 @@ namespace {
 // still be faster with those tiles, loaded straight into LDS, and K cut so that the tiles and
 // slices together make one round over the CUs.  Both ways are priced in microseconds from
 // what was measured on MI355X with the 7B products at 768 to 2,304 rows: a shape's tile takes
-// 2 bm bn K flops at its kernel's rate on a full GPU (pick_shape's speeds, 1 standing for 0.93
+// 2 bm bn K flops at its kernel's rate on a full GPU (1 standing for 0.93
 // PFLOP/s over 256 CUs); a round that leaves CUs idle runs faster (0.72 of the time with up to 170
 // blocks, rising to 1 at 256: the chip's clock follows its load); either kernel costs 14 us
 // beside its tiles; the consumer's pass over the additional slices moves (2 slices - 2) x the
 // result's bytes at 4 TB/s.  The cut is taken when it comes out under 0.9 of the best whole
-// product (256 x 128 whole is priced as it was through registers: by itself the down product of 2,048 rows takes 238 us so, 268 with
-// the cut, but in a whole prompt step of the 7B sizes the two are level, and the cut's sums are two shorter ones) (at the 3B and 1.5B products of 2,048 rows, whose 128 x 128 tiles fill the GPU in one
-// round as it is, a cut priced at 0.9 to 0.97 measured 0.99 to 1.04).  Measured, whole + norm against cut + the pass that adds the slices, the
-// residual and the norm: down (3,584 x 18,944) at 1,280 rows 237 against 152 us, at 2,048 rows 272
-// against 247; output (3,584 x 3,584) at 1,280 rows 69 against 52.
+// product.  The 1.05 of tiles of 256 x 128 is not that kernel's speed (1.24, pick_shape) but what places this line: the pass
+// over a whole product's result is in neither price, and with 1.24 the down product of 1,536 rows and more would stay whole.
+// Measured one after the other with cold weights, whole + norm against the cut taken + the pass that adds the slices, the residual and
+// the norm, us: 3,584 x 18,944 at 1,024 rows 185 and 130, 1,280 226 and 157, 1,536 227 and 204, 1,792 241 and 220, 2,048 254 and 239,
+// 2,304 277 and 253; 2,560 x 9,728 at 1,792 130 and 96, 2,304 138 and 122; 3,072 x 8,192 at 1,536 109 and 87, 2,048 114 and 115; 4,096 x
+// 14,336 at 1,280 177 and 136, 2,048 210 and 203; 5,120 x 13,824 at 896 165 and 127, 1,536 200 and 190.  Left whole: 3,584 x 3,584 at 2,048 rows 69
+// (cut in two 71); and, where the cut would be ahead, 1,152 rows of 3,584 x 18,944 181 (three 151), 1,792 and 2,048 rows of 2,048 x
+// 11,008 109 and 111 (three 98 and 107), 896 rows of 4,096 x 14,336 138 (four 104).  Prices fitted to all of these (to 4 %) take those cuts as well; in
+// whole prompt steps that gave 4.5 % at 1,152 rows of the 7B sizes, nothing at 1,792 of the 3B ones, and cost 1 % at 2,048 of the
+// 3B sizes and at 1,800 and 2,300 of 2,048 wide layers of other designs: not taken.
 //
 // A few hundred rows: the same tiles of 128 x 128, or of 64 x 128, loaded straight into LDS with four
 // stages' buffers, a block a CU, where tiles x slices make one round over each die's 32 CUs.  A launch costs
@@ -1411,7 +1416,7 @@ PartialPlan partial_plan(int n_rows, int n_out, int n_in, bool direct_ok) {
   const long long big_grid = (big + kXcds - 1) / kXcds * kXcds;       // the grid is padded to whole eights
   if (s == 1 && direct_ok && 2 * big_grid <= sb::cu_count()) {
     const double per_cu = 0.93e9 / 256.0;                                        // a CU's flops per microsecond at speed 1
-    const double speed[5] = {1.0, 1.05, 1.45, 0.0, 1.2};
+    const double speed[5] = {1.0, 1.05, 1.45, 0.0, 1.2};                         // (256 x 128: see above)
     double t_whole = 0;
     for (int v = 0; v < 5; ++v) {
       if (v == 3) continue;
