@@ -431,10 +431,13 @@ def test_gemm_bf16_blocks_that_go_from_tile_to_tile():
             close(got, g / (1.0 + torch.exp(-g)) * u, atol=1e-4 * math.sqrt(k), rtol=1e-4, what=f"gated {shape} {path}")
 
 
-@pytest.mark.parametrize("t, n, k", [(300, 520, 1024), (300, 520, 16448), (4400, 4200, 8128), (4400, 4200, 8192), (1000, 1800, 8192)])
-def test_gemm_bf16_both_kernels_of_the_largest_tiles_give_the_same_bits(t, n, k):
-    """256 x 256 tiles on either side of what chooses between the kernel that reads fragments ahead and the one a whole stage
-    ahead (the inner size, and more tiles than CUs), against the first with a block for every tile."""
+@pytest.mark.parametrize("shape", [1, 2])
+@pytest.mark.parametrize("t, n, k", [(300, 520, 1024), (300, 520, 16448), (1000, 1800, 8192), (4400, 4200, 128), (4400, 4200, 192), (4400, 4200, 256),
+                                     (4400, 4200, 320), (4400, 4200, 1088), (4400, 4200, 8128), (4400, 4200, 8192)])
+def test_gemm_bf16_blocks_that_go_on_give_the_bits_of_a_block_a_tile(shape, t, n, k):
+    """Tiles of 256 x 128 and 256 x 256: blocks that go on to a second tile, whose first stages are loaded in the last ones of
+    the first (4,400 x 4,200: 594 and 306 tiles on 256 CUs), against a block for every tile, from the least inner size that
+    goes on; and few tiles, where no block does."""
     from sonicboom_amd import ops
     gen = torch.Generator(device=DEV).manual_seed(3)
     x = torch.randn(t, k, generator=gen, device=DEV).to(BF16)
@@ -442,7 +445,7 @@ def test_gemm_bf16_both_kernels_of_the_largest_tiles_give_the_same_bits(t, n, k)
     resid = torch.randn(t, n, generator=gen, device=DEV)
     got = {}
     for path in ("direct", "direct, a block a tile"):
-        with ops.gemm_tile_shape(2, path):
+        with ops.gemm_tile_shape(shape, path):
             got[path] = ops.gemm_bf16(x, w, None, resid, F32, packed_shape=(n, k))
     assert torch.equal(*got.values())
     with ops.gemm_tile_shape(0, "registers"):
