@@ -96,8 +96,10 @@ head_product_mfma_kernel(bf16_t *__restrict__ out, int out_stride, int out_hstri
 // The same for many rows: a wave takes 16 RT rows against its 64 outputs, so that a fragment of W feeds RT products and one
 // of the rows four (above: one and four, and W came in again for every 16 rows), 64 k a stage, the next stage's
 // fragments asked for ahead of this one's products.  The same bits.
-// Bound by the rows' reads and the outputs' writes from here on.  Measured, 16 heads, 4,001 rows, against the kernel above:
-// 128 to 512 numbers 83 -> 52 us, 512 to 128 with a gate 92 -> 55; 1,000 rows (RT 2) 128 to 512 23 -> 15.
+// What bounds it: the waves in flight.  With RT 4 a wave takes 348 registers, so a SIMD holds one and a CU one block, and nothing but
+// the stage asked for ahead covers a stage's loads (82 MB in 53 us is a third of a copy's rate).  Measured, 16 heads, rows of 16, 32 and
+// 64 a wave (the first the kernel above), us: 128 to 512 numbers, 4,001 rows 79.7, 58.6, 52.8, 1,000 rows 22.8, 17.5, 15.2, 500 rows 12.7, 9.9, 8.4;
+// 512 to 128 with a gate, 4,001 rows 92.7, 59.4, 55.8, 3,000 rows 69.6, 49.9, 52.3, 1,000 rows 26.5, 19.7, 27.4, 500 rows 15.5, 17.0, 24.1.
 template <bool GATED, int RT>
 __global__ void __launch_bounds__(kThreads)
 head_product_rows_kernel(bf16_t *__restrict__ out, int out_stride, int out_hstride, const bf16_t *__restrict__ in,
@@ -805,7 +807,8 @@ extern "C" int sb_head_product_gated_bf16(void *out, int out_stride, int out_hst
                                                                                  (const bf16_t *)in, in_stride, in_hstride,       \
                                                                                  (const bf16_t *)w, gate, gate_stride, n_rows,    \
                                                                                  n_in, n_out, gate_per_head)
-  // rows of a wave: the most (64, 32, 16) that leave two blocks a CU
+  // rows of a wave: the most (64, 32, 16) that give two blocks for every CU (a CU holds one of 64 rows a wave at a time, two of 32:
+  // see the kernel's figures; between one and two for every CU the larger is mostly ahead too, but for 3,000 rows of 512 to 128)
   const auto blocks = [&](int rows) { return (long long)((n_rows + rows - 1) / rows) * heads * out_tiles; };
   const int rt = blocks(256) >= 2 * sb::cu_count() ? 4 : blocks(128) >= 2 * sb::cu_count() ? 2 : 1;
   if (gate) {
