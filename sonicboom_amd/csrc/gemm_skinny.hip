@@ -228,7 +228,7 @@ gemm_skinny_gated_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict_
     const int step = in ? begin[s] + j : n_steps;
 #pragma unroll
     for (int g = 0; g < 2; ++g)
-      rw[slot][s][g] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[g], lane * 16 + step * 1024, 0, 0));
+      rw[slot][s][g] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[g], lane * 16 + step * 1024, 0, kReadOnce));
     rx[slot][s] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
         rsrc_x, int(in && step * kStepK + 8 * q < n_in ? x_off + uint32_t(step) * 64u : kOutside), 0, 0));    // (n_in is a multiple of 8)
   };

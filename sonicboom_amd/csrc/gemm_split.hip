@@ -75,7 +75,7 @@ gemm_split_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, Sp
   auto ask = [&](int slot, int step) {
 #pragma unroll
     for (int g = 0; g < G; ++g)
-      rw[slot][g] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[g], lane * 16 + step * 1024, 0, 0));
+      rw[slot][g] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[g], lane * 16 + step * 1024, 0, kReadOnce));
     const bool in = step < s1 && step * 32 + 8 * q < a.n_in;          // (n_in is a multiple of 8)
     rx[slot] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(
         rsrc_x, int(in ? x_off + uint32_t(step) * 64u : kOutside), 0, 0));

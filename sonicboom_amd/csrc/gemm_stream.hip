@@ -124,7 +124,7 @@ gemm_stream_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, S
   for (int u = 0; u < kAhead; ++u) {
 #pragma unroll
     for (int f = 0; f < F; ++f)
-      ring[u][f] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[f], int(w_off), 0, 0));
+      ring[u][f] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[f], int(w_off), 0, kReadOnce));
     w_off += 1024u;
   }
   issue_x(0);
@@ -155,7 +155,7 @@ gemm_stream_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, S
       for (int f = 0; f < F; ++f) {
 #pragma unroll
         for (int j = 0; j < TT; ++j) acc[f][j] = mfma16(as_bf16x8(ring[u][f]), as_bf16x8(b[u & 1][j]), acc[f][j]);
-        ring[u][f] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[f], int(w_off), 0, 0));
+        ring[u][f] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w[f], int(w_off), 0, kReadOnce));
       }
       w_off += 1024u;
       if constexpr (kOrdered) __builtin_amdgcn_sched_barrier(0);

@@ -29,6 +29,14 @@ __device__ __forceinline__ uint4 ld16(const void *p, bool ok) {
   return ok ? *reinterpret_cast<const uint4 *>(p) : make_uint4(0u, 0u, 0u, 0u);
 }
 
+// The cache policy of loads of what a launch reads once, as buffer loads take it (non-temporal): the weights of a product of
+// few rows, which no other block wants and no cache holds until the next step.  Measured, replayed graphs, weights cold, without
+// and with it (us): gated 18,944 x 3,584 of 8 rows 53.8 -> 48.7, 3,584 x 18,944 26.5 -> 25.2, gated 11,008 x 2,048 of 2 rows
+// 20.8 -> 19.6, gated 4,864 x 896 of one row 7.6 -> 7.2, 1,536 x 8,960 of 48 rows 11.0 -> 10.7; a plain read of 272 MB in the same
+// order of addresses 46.8 -> 41.9.  Only weights that one launch after another reads from L2 lose by it (8.7 MB again and again
+// 3.1 -> 4.5), which no model does.
+constexpr int kReadOnce = 2;
+
 // Two floats to two bf16 packed in 32 bits (low half first), round to nearest even: one
 // v_cvt_pk_bf16_f32.
 typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
