@@ -22,6 +22,7 @@
 // reads all of X).  The waves' sums meet in LDS and are added in wave order.
 //
 // MFMA roles: A = 16 rows of W, B = 16 rows of X, D[n][t]; a lane holds four consecutive n of one t.
+#include "gemm_rows.h"
 #include "mfma.h"
 
 namespace {
@@ -211,6 +212,8 @@ extern "C" int sb_gemm_split_gated_bf16(void *y, const void *x, const double *ss
   SB_REQUIRE(y && ssq && ssq_parts > 0, "sb_gemm_split_gated_bf16: null pointer");
   SB_SUPPORT(gate > SB_GATE_NONE && gate <= SB_GATE_RELU, "sb_gemm_split_gated_bf16: unknown gate activation %d", gate);
   if (n_rows == 0) return SB_OK;
+  if (sb::rows_whole(n_rows, n_out, n_in, 1))          // blocks that keep the rows in LDS, where these fit
+    return sb::rows_gated(y, x, ssq, ssq_parts, eps, w, n_rows, n_out, n_in, gate, stream);
   SplitArgs a{};
   a.n_rows = n_rows, a.n_out = n_out, a.n_in = n_in, a.ssq = ssq, a.ssq_parts = ssq_parts, a.eps = eps;
   a.y = (bf16_t *)y, a.gate = gate;

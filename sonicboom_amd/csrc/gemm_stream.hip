@@ -20,6 +20,7 @@
 //
 // MFMA roles: A = 16 rows of W, B = 16 rows of X, D[n][t]; a lane holds four
 // consecutive n of one t.
+#include "gemm_rows.h"
 #include "mfma.h"
 
 namespace {
@@ -313,6 +314,11 @@ extern "C" int sb_gemm_stream_bf16(void *y, int y_dtype, const void *x, const vo
   SB_SUPPORT(gated >= SB_GATE_NONE && gated <= SB_GATE_RELU, "sb_gemm_stream_bf16: unknown gate activation %d", gated);
   const StreamArgs a{y, y_dtype, bias, bias_dtype, resid, n_rows, n_out, n_in, nullptr, 0, gated};
   const bf16_t *xb = (const bf16_t *)x, *wb = (const bf16_t *)w;
+  // up to eight rows of large matrices: blocks that keep the rows
+  if (hint == 0 && gated && y_dtype == SB_BF16 && sb::rows_whole(n_rows, n_out, n_in, 1))
+    return sb::rows_gated(y, x, nullptr, 0, 0.f, w, n_rows, n_out, n_in, gated, stream);
+  if (hint == 0 && !gated && y_dtype == SB_F32 && !bias && !resid && sb::rows_whole(n_rows, n_out, n_in, 0))
+    return sb::rows_plain((float *)y, x, w, n_rows, n_out, n_in, stream);
   const int tt = row_tiles(n_rows);
   if (gated) {
     if (tt == 1) launch<1, 2, 1>(xb, wb, a, hint, s);
@@ -331,6 +337,7 @@ extern "C" int sb_gemm_stream_bf16(void *y, int y_dtype, const void *x, const vo
 // K slices sb_gemm_stream_partial_bf16 will produce for these sizes.
 extern "C" int sb_gemm_stream_slices(int n_rows, int n_out, int n_in, int hint) {
   if (n_rows <= 0 || n_out <= 0 || n_in <= 0) return 1;
+  if (const int s = hint ? 0 : sb::rows_slices(n_rows, n_out, n_in)) return s;
   return cut_for((n_out + 15) / 16, (n_in + kStepK - 1) / kStepK, row_tiles(n_rows), hint).slices;
 }
 
@@ -347,6 +354,7 @@ extern "C" int sb_gemm_stream_partial_bf16(float *partial, const void *x, const 
   SB_SUPPORT((unsigned long long)(n_rows + 1) * n_in * 2 < (1ull << 31) && (unsigned long long)n_in * 32 < (1ull << 31),
              "sb_gemm_stream_partial_bf16: inner size %d is too large", n_in);
   if (n_rows == 0) return SB_OK;
+  if (!hint && sb::rows_slices(n_rows, n_out, n_in)) return sb::rows_partial(partial, x, w, n_rows, n_out, n_in, stream);
   const Cut c = cut_for((n_out + 15) / 16, (n_in + kStepK - 1) / kStepK, row_tiles(n_rows), hint);
   const StreamArgs a{nullptr, SB_F32, nullptr, 0, nullptr, n_rows, n_out, n_in, partial, c.steps_per_slice, 0};
   const bf16_t *xb = (const bf16_t *)x, *wb = (const bf16_t *)w;

@@ -1424,6 +1424,46 @@ def test_products_that_carry_the_norm_between_them(rows, width, n_in, inner, gat
         assert ((got - ref).abs() <= ref.abs() * 2.0 ** -8 + 1.2 * (slack[:, :inner] * u.abs() + slack[:, inner:] * g.abs()) + 1e-5).all()
 
 
+# (rows, features, k): a tile of one feature, features and k that fill no tile, step or round, one block a tile and many, the most
+# rows and the first that stay with the other kernels, X that just fits beside the sums in LDS and X that does not
+ROWS_IN_LDS = [(1, 17, 512), (3, 40, 2560), (8, 264, 2568), (8, 4100, 1032), (5, 12300, 520), (8, 272, 7680), (8, 272, 7688), (9, 264, 1032)]
+
+
+@pytest.mark.parametrize("rows, inner, width", ROWS_IN_LDS)
+def test_gated_products_whose_blocks_keep_the_rows(rows, inner, width):
+    """Against 64 bits, with an unfinished norm's factor; a row of infinities stays its own."""
+    from sonicboom_amd import ops
+    x, wg = randn(rows, width).to(BF16), randn(2 * inner, width, scale=0.1, seed=1).to(BF16)
+    ssq = torch.rand((width + 15) // 16, rows, dtype=torch.float64, generator=torch.Generator().manual_seed(2)) * 16
+    h = ops.ScaledRows(x.to(DEV), ssq.to(DEV), 1e-6)
+    w = ops.pack_weight(wg.to(DEV), True)
+    got = ops.gemm_split_gated(h, w, "relu", packed_shape=(2 * inner, width)).cpu().double()
+    f = (ssq.sum(0) / width + 1e-6).rsqrt()[:, None]
+    e, m = f * (x.double() @ wg.double().T), f * (x.double().abs() @ wg.double().abs().T) * (width + 40) * 2.0 ** -24
+    g, u, mg, mu = torch.relu(e[:, :inner]), e[:, inner:], m[:, :inner], m[:, inner:]
+    assert ((got - g * u).abs() <= (g * u).abs() * 2.0 ** -8 + 1.2 * (mg * u.abs() + mu * g)).all()
+    if rows > 1:
+        h.values[1, 3] = float("inf")
+        again = ops.gemm_split_gated(h, w, "relu", packed_shape=(2 * inner, width)).cpu().double()
+        rest = [i for i in range(rows) if i != 1]
+        assert not torch.isfinite(again[1]).any()
+        assert torch.equal(again[rest], got[rest])
+
+
+@pytest.mark.parametrize("rows, n, k", [(1, 1000, 8184), (8, 8200, 520), (4, 2048, 2056), (8, 96, 61440), (8, 72, 70000), (9, 2048, 4096), (3, 20001, 136), (8, 17424, 7688)])
+def test_raw_and_plain_products_whose_blocks_keep_the_rows(rows, n, k):
+    """In K slices, and whole with float results where the matrix is wide, against 64 bits: cuts of K that the blocks' share of LDS
+    allows and some that it does not."""
+    from sonicboom_amd import ops
+    x, w = randn(rows, k).to(BF16), randn(n, k, scale=0.1, seed=1).to(BF16)
+    want, bound = x.double() @ w.double().T, (x.double().abs() @ w.double().abs().T) * (k + 8) * 2.0 ** -24
+    packed = ops.pack_weight(w.to(DEV))
+    part = ops.gemm_bf16_partial(x.to(DEV), packed, packed_shape=(n, k))
+    assert ((part.cpu().double().sum(0) - want).abs() <= bound).all()
+    whole = ops.gemm_bf16(x.to(DEV), packed, None, None, torch.float32, packed_shape=(n, k))
+    assert ((whole.cpu().double() - want).abs() <= bound).all()
+
+
 def test_the_norm_between_two_products_sums_in_double():
     """Rows whose squares are float numbers but whose sum of squares over the width is none, and rows of many small numbers
     beside a large one: the factor follows from the sum in double, as of every RMS norm."""
