@@ -53,6 +53,8 @@ constexpr int kPagesPerChunk = 4;
 constexpr int kWholePages = 8;               // pages of a row that one block takes whole
 constexpr bool kWholeRows = HD <= 128;       // (its waves' sums meet in 64 KB of LDS at most)
 constexpr float kMaxSlack = 8.f;
+constexpr int kWaveSlots = 2048;             // waves among which the pages of a batch are dealt out: two a SIMD
+constexpr int kDealtFrom = 256;              // (tables' eights of pages) x rows x head tiles
 
 // A wave's running softmax for NC groups of 16 query columns that share positions (and so the
 // mask): in decode one group, the heads of a kv head; in prefill up to four heads of one kv head
@@ -141,25 +143,48 @@ __device__ __forceinline__ void load_half(HalfPage &hp, const bf16_t *__restrict
   for (int dt = 0; dt < DT; ++dt) hp.v[dt] = ld16(vp + size_t(vat + 128 * dt) * 8, true);
 }
 
-// The same without a branch around any load (a branch makes the compiler wait for every load in
-// flight, which a loop that keeps the next half page's loads in flight cannot afford): a chunk
-// past the head size is read from the row's start and replaced by zeros afterwards.
-__device__ __forceinline__ void load_half_straight(HalfPage &hp, const bf16_t *__restrict__ kp,
-                                                   const bf16_t *__restrict__ vp, int half, int lane) {
+// The whole page through descriptors of its keys and values, without a branch around any load (a branch makes the compiler wait for
+// every load in flight) and with few registers for addresses: a chunk past the head size lies past the descriptor's end and reads
+// as zeros.  kp, vp: the same in every lane.
+constexpr int kPageBytes = SB_PAGE * HD * 2;
+__device__ __forceinline__ void load_keys_straight(HalfPage (&h)[2], const bf16_t *kp, int lane) {
   const int r = lane & 15, g = lane >> 4;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(kp), 0, kPageBytes, 0x00020000);
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const int d = ks * 32 + g * 8;
-    const int at = key_chunk(r, g, d < HD ? ks : 0);
+  for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const uint4 v = *reinterpret_cast<const uint4 *>(kp + size_t(at + (32 * half + 4 * t) * CPRK) * 8);
-      hp.k[t][ks] = ((ks + 1) * 32 <= HD || d < HD) ? v : make_uint4(0u, 0u, 0u, 0u);
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int at = ((ks + 1) * 32 <= HD || ks * 32 + g * 8 < HD) ? key_chunk(r, g, ks) * 16 : kPageBytes;
+        h[i].k[t][ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, at, (32 * i + 4 * t) * CPRK * 16, 0));
+      }
+}
+__device__ __forceinline__ void load_values_straight(HalfPage (&h)[2], const bf16_t *vp, int lane) {
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(vp), 0, kPageBytes, 0x00020000);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      h[i].v[dt] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, value_chunk(lane & 15, lane >> 4, i) * 16,
+                                                                                  128 * dt * 16, 0));
+}
+
+// Keys and values of one half of a page, the same way.
+__device__ __forceinline__ void load_half_straight(HalfPage &hp, const bf16_t *kp, const bf16_t *vp, int half, int lane) {
+  const int r = lane & 15, g = lane >> 4;
+  const __amdgpu_buffer_rsrc_t rsrc_k = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(kp), 0, kPageBytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_v = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(vp), 0, kPageBytes, 0x00020000);
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      const int at = ((ks + 1) * 32 <= HD || ks * 32 + g * 8 < HD) ? key_chunk(r, g, ks) * 16 : kPageBytes;
+      hp.k[t][ks] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_k, at + 32 * half * CPRK * 16, 4 * t * CPRK * 16, 0));
     }
-  }
-  const int vat = value_chunk(r, g, half);
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt) hp.v[dt] = *reinterpret_cast<const uint4 *>(vp + size_t(vat + 128 * dt) * 8);
+  for (int dt = 0; dt < DT; ++dt)
+    hp.v[dt] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_v, value_chunk(r, g, half) * 16, 128 * dt * 16, 0));
 }
 
 // 32 keys at absolute positions base .. base+31, their fragments in hp, for the wave's NC groups
@@ -230,18 +255,84 @@ __device__ __forceinline__ void attend_half(WaveState<NC> &st, const bf16x8_t (&
   }
 }
 
-// One page (64 keys at absolute positions page_pos .. page_pos+63).  With one column group and a
-// head size up to 128 both halves' fragments are requested before the first product, so a page
-// costs one round trip to memory (BOTH); otherwise half by half, to stay within the registers
-// (or, when there are many more blocks than the GPU holds at once, to let more of them in).
-template <int NC, bool BOTH = true>
+// A page, 64 keys at absolute positions base .. base+63 whose fragments are all in registers, for one group of columns: one
+// softmax step over the 64, keys tested one by one.  Arguments as above.
+template <bool MASKED, typename F>
+__device__ __forceinline__ void attend_whole_page(WaveState<1> &st, const bf16x8_t (&qf)[1][KS], HalfPage (&h)[2], int base, int col_pos,
+                                                  int col_lo, int key_lo, int key_hi, float scale_log2, int lane, F &&keys_done) {
+  const int g = lane >> 4;
+  floatx4_t s[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) s[i][t] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) s[i][t] = mfma16(as_bf16x8(h[i].k[t][ks]), qf[0][ks], s[i][t]);
+  keys_done();
+  // this lane: column lane % 16, keys base + 32 i + 8 g + e, e = 0..7 (s[i][0] holds e = 0..3, s[i][1] e = 4..7)
+  float sc[2][8];
+  float mx = -__builtin_inff();
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int j = base + 32 * i + 8 * g + e;
+      const bool vis = !MASKED || (j <= col_pos && j >= col_lo);
+      sc[i][e] = vis ? (e < 4 ? s[i][0][e] : s[i][1][e - 4]) * scale_log2 : -__builtin_inff();
+      mx = fmaxf(mx, sc[i][e]);
+    }
+  mx = max_over_lane_groups(mx);
+  const float m_new = fmaxf(st.m[0], mx);
+  // a column that has seen no key yet keeps m = -inf: give it a finite stand-in
+  const float m_use = m_new == -__builtin_inff() ? 0.f : m_new;
+  const float alpha = __builtin_amdgcn_exp2f(st.m[0] - m_use);   // m = -inf gives 0
+  uint4 pb[2];
+  float psum = 0.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    float p[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      p[e] = __builtin_amdgcn_exp2f(sc[i][e] - m_use);             // -inf gives 0
+      psum += p[e];
+    }
+    pb[i] = make_uint4(pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7]));
+  }
+  st.l[0] = st.l[0] * alpha + psum;
+  st.m[0] = m_new;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) {
+    floatx4_t acc = st.o[0][dt];
+    acc[0] *= alpha; acc[1] *= alpha; acc[2] *= alpha; acc[3] *= alpha;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      // values of keys outside [key_lo, key_hi] may be stale or never written: cut, as above
+      uint4 v = h[i].v[dt];
+      if (MASKED) {
+        const int k0 = base + 32 * i + 8 * g;
+        if (base + 63 > key_hi) v = keep_first(v, key_hi - k0 + 1);
+        if (base < key_lo) v = drop_first(v, key_lo - k0);
+      }
+      acc = mfma16(as_bf16x8(v), as_bf16x8(pb[i]), acc);
+    }
+    st.o[0][dt] = acc;
+  }
+}
+
+// One page (64 keys at absolute positions page_pos .. page_pos+63), half by half, to stay within the registers; with one column
+// group and a head size up to 128 both halves' fragments are requested before the first product.
+template <int NC>
 __device__ __forceinline__ void attend_page(WaveState<NC> &st, const bf16x8_t (&qf)[NC][KS],
                                             const bf16_t *__restrict__ kp, const bf16_t *__restrict__ vp,
                                             int page_pos, int col_pos, int col_lo, int key_lo, int key_hi,
                                             float scale_log2, int lane) {
   const bool use0 = !(page_pos > key_hi || page_pos + 31 < key_lo);
   const bool use1 = !(page_pos + 32 > key_hi || page_pos + 63 < key_lo);
-  if (BOTH && HD <= 128 && NC == 1) {
+  if (HD <= 128 && NC == 1) {
     HalfPage h0, h1;
     if (use0) load_half(h0, kp, vp, 0, lane);
     if (use1) load_half(h1, kp, vp, 1, lane);
@@ -1089,11 +1180,15 @@ __device__ __forceinline__ DecodeBlock decode_block(int tiles, int n_seqs) {
   return b;
 }
 
-// The end of a decode block: the waves' running sums meet in LDS and are merged in wave order
-// (thread e owns (d, column), column fastest); the result goes to `out` when the row's keys lie
-// in this chunk alone, else to the chunk's place in the partial buffers.
+// The end of a decode block: the waves' running sums meet in LDS and are merged in wave order; the result goes to `out` when the
+// row's keys lie in this chunk alone, else to the chunk's place in the partial buffers: part_o [chunk][column][d], part_ml
+// [chunk][16 maxima, 16 sums].  A lane's four d of a column are sixteen bytes in LDS, the columns' groups of four d permuted so
+// that the sixteen columns a wave writes at once lie in distinct banks; a thread merges four d of a column that has a head.
+constexpr int kFours = HD / 4;
+constexpr int kFourMask = kFours % 16 == 0 ? 15 : (kFours % 8 == 0 ? 7 : 3);
+__device__ __forceinline__ int four_slot(int col, int d4) { return col * kFours + (d4 ^ (col & kFourMask)); }
 template <int WAVES>
-__device__ __forceinline__ void finish_decode_block(const WaveState<1> &st, float (*lds_o)[HD * 16], float (*lds_m)[16],
+__device__ __forceinline__ void finish_decode_block(const WaveState<1> &st, floatx4_t (*lds_o)[kFours * 16], float (*lds_m)[16],
                                                     float (*lds_l)[16], bf16_t *__restrict__ out,
                                                     float *__restrict__ part_o, float *__restrict__ part_ml,
                                                     int wave, int lane, int chunk, bool alone, int seq, int kvh,
@@ -1104,39 +1199,41 @@ __device__ __forceinline__ void finish_decode_block(const WaveState<1> &st, floa
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
 #pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) lds_o[wave][(dt * 16 + 4 * g + i) * 16 + r] = st.o[0][dt][i];
+  for (int dt = 0; dt < DT; ++dt) lds_o[wave][four_slot(r, dt * 4 + g)] = st.o[0][dt];
   if (g == 0) {
     lds_m[wave][r] = st.m[0];
     lds_l[wave][r] = l;
   }
   __syncthreads();
-  // merge the waves (pages in ascending order); thread e owns (d, col), column fastest
-  float *po = part_o + (tile_index * n_chunks) * (HD * 16);
-  float *pml = part_ml + (tile_index * n_chunks) * 32;
-  for (int e = threadIdx.x; e < HD * 16; e += 64 * WAVES) {
-    const int c = e & 15, d = e >> 4;
+  // merge the waves (pages in ascending order)
+  float *po = part_o + (tile_index * n_chunks + chunk) * (HD * 16);
+  float *pml = part_ml + (tile_index * n_chunks + chunk) * 32;
+  const int columns = min(group - ht * 16, 16);
+  for (int e = threadIdx.x; e < columns * kFours; e += 64 * WAVES) {
+    const int c = e / kFours, d4 = e - c * kFours;
     float m = -__builtin_inff();
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) m = fmaxf(m, lds_m[w][c]);
     const float m_use = m == -__builtin_inff() ? 0.f : m;
-    float o = 0.f, lsum = 0.f;
+    floatx4_t o = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    float lsum = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
       const float f = __builtin_amdgcn_exp2f(lds_m[w][c] - m_use);
-      o += lds_o[w][e] * f;
+      o = o + lds_o[w][four_slot(c, d4)] * f;
       lsum += lds_l[w][c] * f;
     }
     if (alone) {
-      const int hh = ht * 16 + c;
-      if (hh < group)
-        out[(size_t(seq) * heads_q + kvh * group + hh) * HD + d] = f32_to_bf16(lsum > 0.f ? o / lsum : 0.f);
-    } else if (ht * 16 + c < group) {
-      po[size_t(chunk) * (HD * 16) + e] = o;
-      if (d == 0) {
-        pml[size_t(chunk) * 32 + c] = m;
-        pml[size_t(chunk) * 32 + 16 + c] = lsum;
+      bf16_t *to = out + (size_t(seq) * heads_q + kvh * group + ht * 16 + c) * HD + 4 * d4;
+      float v[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = lsum > 0.f ? o[i] / lsum : 0.f;
+      *reinterpret_cast<ushort4 *>(to) = make_ushort4(f32_to_bf16(v[0]), f32_to_bf16(v[1]), f32_to_bf16(v[2]), f32_to_bf16(v[3]));
+    } else {
+      *reinterpret_cast<floatx4_t *>(po + c * HD + 4 * d4) = o;
+      if (d4 == 0) {
+        pml[c] = m;
+        pml[16 + c] = lsum;
       }
     }
   }
@@ -1436,7 +1533,7 @@ __device__ __forceinline__ void staged_q(bf16x8_t (&qf)[KS], const RopeShared &s
 // merges chunks.  What it is bound by stays the chain of look-ups, loads and sums; measured with the merging kernel and without: 14 heads
 // of 64 on 2, one row of 145 keys 6.1 -> 4.3 us, of 500 7.3 -> 5.3; 12 of 128 on 2, 500 keys 9.2 -> 7.5; 28 of 128 on 4, eight rows of 500
 // keys 11.0 -> 9.8, 24 rows 14.9 -> 13.8.  (Sixteen waves, heads of 64, up to sixteen pages: 900 keys 7.3 -> 8.0; not taken.)
-template <bool BOTH, bool FUSED, int WAVES>
+template <bool FUSED, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
 attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml,
                    const bf16_t *__restrict__ q, const RopeArgs ra,
@@ -1444,10 +1541,11 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
                    const int32_t *__restrict__ page_table, int max_pages, int n_pages_total,
                    const int32_t *__restrict__ row_pos, int heads_q, int heads_kv, int n_chunks,
                    float scale_log2, int window, int n_seqs) {
-  __shared__ float lds_o[WAVES][HD * 16];   // [wave][d][col]
+  __shared__ floatx4_t lds_o[WAVES][kFours * 16];
   __shared__ float lds_m[WAVES][16], lds_l[WAVES][16];
   __shared__ std::conditional_t<FUSED, RopeShared, int> rope_sh;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int group = heads_q / heads_kv;
   const int head_tiles = (group + 15) / 16;
   const int tiles = heads_kv * head_tiles;
@@ -1484,61 +1582,137 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
   bf16x8_t qf[1][KS];
   WaveState<1> st;
   init_state<1>(st);
+  const int page_pos = pg * SB_PAGE;
+  // Head sizes up to 128: the whole page is asked for at once, one round trip to memory, and ahead of the queries that the folded
+  // form builds; or the half of it that holds a visible key (one row of 145 keys 6.0 us, 6.4 with the last page whole).  The page
+  // that receives the row's own key and value is read like the others, before they are stored, and its fragments are patched from
+  // LDS afterwards.
+  constexpr bool kWhole = HD <= 128;
+  const bool use0 = have_page && !(page_pos > pos || page_pos + 31 < key_lo);
+  const bool use1 = have_page && !(page_pos + 32 > pos || page_pos + 63 < key_lo);
+  const bool both = use0 && use1;
+  HalfPage h[2], &one = h[0];       // one: the only half
+  const int half = use0 ? 0 : 1;
+  if constexpr (kWhole) {
+    if (both) {
+      load_keys_straight(h, k_cache + off, lane);
+      load_values_straight(h, v_cache + off, lane);
+    } else if (use0 || use1) {
+      load_half_straight(one, k_cache + off, v_cache + off, half, lane);
+    }
+  }
   if constexpr (!FUSED) {
     load_q(qf[0], q + (size_t(seq) * heads_q + head) * HD, col_ok, lane);
-    if (have_page)
-      attend_page<1, BOTH>(st, qf, k_cache + off, v_cache + off, pg * SB_PAGE, col_pos, key_lo, key_lo, pos, scale_log2,
-                           lane);
   } else {
-    // The page's keys and values do not depend on the queries: their loads go out first and are
-    // in flight while the block builds its queries.  The page that receives the row's own key
-    // and value is read like the others, before they are stored, and its fragments are patched
-    // from LDS afterwards.
-    const int page_pos = pg * SB_PAGE;
-    const bool use0 = have_page && !(page_pos > pos || page_pos + 31 < key_lo);
-    const bool use1 = have_page && !(page_pos + 32 > pos || page_pos + 63 < key_lo);
-    const bool own_page = ra.store && have_page && pg == pos / SB_PAGE;
-    constexpr bool kEarly = BOTH && HD <= 128;
-    HalfPage h0, h1;
-    if (kEarly) {
-      if (use0) load_half(h0, k_cache + off, v_cache + off, 0, lane);
-      if (use1) load_half(h1, k_cache + off, v_cache + off, 1, lane);
-    }
     if (lane == 0) rope_sh.page_of_wave[wave] = page_looked_up;
-    rope_store(rope_sh, first, freq, ra, seq, pos, kvh, group, heads_q, heads_kv, chunk == last_chunk, !kEarly,
+    rope_store(rope_sh, first, freq, ra, seq, pos, kvh, group, heads_q, heads_kv, chunk == last_chunk, !kWhole,
                const_cast<bf16_t *>(k_cache), const_cast<bf16_t *>(v_cache), page_table, max_pages, n_pages_total,
                chunk * WAVES);
     staged_q(qf[0], rope_sh, hq, col_ok, lane);
-    if (kEarly) {
-      const int slot = pos % SB_PAGE;
-      if (own_page && slot < 32 && use0) patch_half(h0, rope_sh, 0, slot, lane);
-      if (own_page && slot >= 32 && use1) patch_half(h1, rope_sh, 1, slot, lane);
-      if (use0) attend_half<1>(st, qf, h0, page_pos, col_pos, key_lo, key_lo, pos, scale_log2, lane);
-      if (use1) attend_half<1>(st, qf, h1, page_pos + 32, col_pos, key_lo, key_lo, pos, scale_log2, lane);
-    } else if (have_page) {
-      attend_page<1, BOTH>(st, qf, k_cache + off, v_cache + off, page_pos, col_pos, key_lo, key_lo, pos, scale_log2,
-                           lane);
+    if constexpr (kWhole) {
+      if (ra.store && have_page && pg == pos / SB_PAGE) {
+        const int slot = pos % SB_PAGE;       // (in the last half that is read)
+        if (both) patch_half(h[1], rope_sh, 1, slot, lane);
+        else patch_half(one, rope_sh, half, slot, lane);
+      }
     }
+  }
+  if (have_page) {
+    if constexpr (kWhole) {
+      if (both)
+        attend_whole_page<true>(st, qf, h, page_pos, col_pos, key_lo, key_lo, pos, scale_log2, lane, [] {});
+      else if (use0 || use1)
+        attend_half<1>(st, qf, one, page_pos + 32 * half, col_pos, key_lo, key_lo, pos, scale_log2, lane);
+    } else
+      attend_page<1>(st, qf, k_cache + off, v_cache + off, page_pos, col_pos, key_lo, key_lo, pos, scale_log2, lane);
   }
   finish_decode_block<WAVES>(st, lds_o, lds_m, lds_l, out, part_o, part_ml, wave, lane, chunk, first_chunk == last_chunk,
                       seq, kvh, ht, group, heads_q, n_chunks, size_t(seq) * tiles + blk.tile);
 }
 
-// Decode with many more blocks than the GPU holds at once (long contexts, large batches): a wave
-// takes `ppw` consecutive pages instead of one and keeps the next half page's keys and values in
-// flight while it multiplies the current one, so that a block lives long enough to stream and the
-// fixed costs of a block (look-ups, queries, the merge through LDS, the partial results) are paid
-// once per 4 * ppw pages.  Block (chunk of 4 * ppw pages, kv head x head tile, sequence); wave w
-// takes pages chunk * 4 * ppw + w * ppw + 0 .. ppw-1.  Head sizes up to 128.
+// Decode over many rows, long ones or rows of unequal length: the pages of the whole batch are dealt out to the GPU's waves by the
+// kernel itself, from the rows' positions.  A launch is recorded once and replayed as rows grow and end, so its grid cannot know
+// the lengths; a grid over (row, chunk of the widest table) leaves most blocks without work where lengths differ and gives the
+// rest rows of pages to walk.  Here block b finds the b-th chunk that exists: the pages of all rows, times tiles, over the
+// waves that the GPU holds are a wave's share, at least a page; a row has as many chunks of four shares as it fills, cut evenly.
+// What bounds it: the read of keys and values (5.3 to 5.8 TB/s at 2,048 waves with a page in flight each; non-temporal loads,
+// 64 bytes of a line at a time, are slower), and 5 us of look-ups, sums and merges.  Measured with the merging kernel, us, a grid over rows
+// and chunks and so (28 heads of 128 on 4 unless said): 48 rows of 8 to 4,000 keys 61.4 -> 23.0; 64 rows of 60 to 4,000 66.4 -> 39.6; 16 rows
+// of 100 to 16,000 73.9 -> 44.3; 12 heads on 2, 41 rows of 60 to 3,000 24.3 -> 17.5; 16 on 2, 96 rows of 60 to 4,000 63.0 -> 30.1; 32 on 32,
+// 16 rows of 100 to 4,000 93.9 -> 67.8; rows of one length: 32 rows of 8,000 110.5 -> 109.3, 64 of 2,048 53.3 -> 56.4, 128 of 1,000
+// 53.2 -> 54.2, one of 131,000 57.1 -> 55.3.
+struct DecodePlan {
+  int share;        // pages of a wave at most; a chunk is four shares
+  int pages0;       // of row `lane`
+};
+
+__device__ __forceinline__ int first_key(int pos, int window) { return (window > 0 && pos >= window) ? pos - window + 1 : 0; }
+// Pages that a row at `pos` sees (a row without a page of its own counts as one)
+__device__ __forceinline__ int row_pages(int pos, int window, int max_pages) {
+  return max(min(pos / SB_PAGE, max_pages - 1) - first_key(pos, window) / SB_PAGE + 1, 1);
+}
+// (a last quarter of a chunk goes to the others: no chunk is smaller than half of the largest by much)
+__device__ __forceinline__ int row_chunks(int pages, int share) {
+  return max((pages + (kPagesPerChunk - 1) * share) / (kPagesPerChunk * share), 1);
+}
+
+// The sums of v over lanes 0 .. l, in lane l: shifts inside rows of 16 lanes, then the rows' last lanes handed on.
+__device__ __forceinline__ int scan_wave(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);      // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);      // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);      // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);      // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);      // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);      // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+// The largest v of the wave (v >= 0), in lane 63.
+__device__ __forceinline__ int max_wave(int v) {
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+  v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+  return v;
+}
+
+// Rows that give half of the GPU's places a block each and are of like length (the longest at most one and a half times the mean)
+// stay whole: 64 rows of 2,048 keys, 28 heads of 128 on 4, 56 us whole and 62 in two chunks.
+// fixed_share: a test's or a measurement's choice, 0: from the batch.
+__device__ __forceinline__ DecodePlan decode_plan(const int32_t *row_pos, int n_seqs, int tiles, int max_pages, int window,
+                                                  int wave_slots, int fixed_share, int lane) {
+  DecodePlan plan;
+  plan.pages0 = lane < n_seqs ? row_pages(row_pos[lane], window, max_pages) : 0;
+  if (fixed_share > 0) {
+    plan.share = fixed_share;
+    return plan;
+  }
+  int mine = plan.pages0, most = plan.pages0;
+  for (int s = lane + 64; s < n_seqs; s += 64) {
+    const int pages = row_pages(row_pos[s], window, max_pages);
+    mine += pages;
+    most = max(most, pages);
+  }
+  const long long all = __builtin_amdgcn_readlane(scan_wave(mine), 63), longest = __builtin_amdgcn_readlane(max_wave(most), 63);
+  if (n_seqs * tiles * 2 * kPagesPerChunk >= wave_slots && 2 * longest * n_seqs <= 3 * all)
+    plan.share = max(int((longest + kPagesPerChunk - 1) / kPagesPerChunk), 1);
+  else
+    plan.share = max(int((all * tiles + wave_slots - 1) / wave_slots), 1);
+  return plan;
+}
+
+// Grid: a block for every chunk that there can be (decode_launch); block size 256.  Head sizes up to 128.
 template <bool FUSED>
 __global__ void __launch_bounds__(256, 2)
-attn_decode_long_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml,
-                        const bf16_t *__restrict__ q, const RopeArgs ra,
-                        const bf16_t *k_cache, const bf16_t *v_cache,
-                        const int32_t *__restrict__ page_table, int max_pages, int n_pages_total,
-                        const int32_t *__restrict__ row_pos, int heads_q, int heads_kv, int n_chunks,
-                        float scale_log2, int window, int ppw, int n_seqs) {
-  __shared__ float lds_o[4][HD * 16];   // [wave][d][col]
+attn_decode_dealt_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml,
+                         const bf16_t *__restrict__ q, const RopeArgs ra,
+                         const bf16_t *k_cache, const bf16_t *v_cache,
+                         const int32_t *__restrict__ page_table, int max_pages, int n_pages_total,
+                         const int32_t *__restrict__ row_pos, int heads_q, int heads_kv, int n_chunks,
+                         float scale_log2, int window, int n_seqs, int wave_slots, int fixed_share) {
+  __shared__ floatx4_t lds_o[4][kFours * 16];
   __shared__ float lds_m[4][16], lds_l[4][16];
   __shared__ std::conditional_t<FUSED, RopeShared, int> rope_sh;
   const int lane = threadIdx.x & 63;
@@ -1546,10 +1720,30 @@ attn_decode_long_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, fl
   const int group = heads_q / heads_kv;
   const int head_tiles = (group + 15) / 16;
   const int tiles = heads_kv * head_tiles;
-  const DecodeBlock blk = decode_block(tiles, n_seqs);
-  const int chunk = blk.chunk, seq = blk.seq;
-  const int kvh = blk.tile / head_tiles, ht = blk.tile - kvh * head_tiles;
+
+  // the block's chunk: every wave looks for it, no barrier is needed
+  const DecodePlan plan = decode_plan(row_pos, n_seqs, tiles, max_pages, window, wave_slots, fixed_share, lane);
+  const int tile = int(blockIdx.x) % tiles;
+  int wanted = int(blockIdx.x) / tiles, seq = -1, chunk = 0, pages = 0;
+  for (int base = 0; base < n_seqs; base += 64) {
+    const int here = base == 0 ? plan.pages0 : base + lane < n_seqs ? row_pages(row_pos[base + lane], window, max_pages) : 0;
+    const int chunks = here > 0 ? row_chunks(here, plan.share) : 0;
+    const int upto = scan_wave(chunks);
+    const int all = __builtin_amdgcn_readlane(upto, 63);
+    if (wanted < all) {
+      const unsigned long long past = __ballot(upto > wanted);
+      const int at = __builtin_ctzll(past);
+      seq = base + at;
+      pages = __builtin_amdgcn_readlane(here, at);
+      chunk = wanted - (__builtin_amdgcn_readlane(upto, at) - __builtin_amdgcn_readlane(chunks, at));
+      break;
+    }
+    wanted -= all;
+  }
+  if (seq < 0) return;                        // uniform over the block: fewer chunks than blocks
+  const int kvh = tile / head_tiles, ht = tile - kvh * head_tiles;
   const int pos = row_pos[seq];
+  const int chunks = row_chunks(pages, plan.share);
   RopeItem first;       // the folded form: see attn_decode_kernel
   if constexpr (FUSED) {
     const int n_q = group * kPerHead, n_all = n_q + (ra.store ? 2 * kPerHead : 0);
@@ -1557,11 +1751,7 @@ attn_decode_long_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, fl
       fetch_item(first, ra, seq, threadIdx.x, n_q, kvh, group, heads_q, heads_kv, ra.inv_freq ? ra.rot_dims / 2 : 0);
   }
   const float freq = FUSED ? rope_freq(ra) : 0.f;
-  const int pages_per_chunk = kPagesPerChunk * ppw;
-  const int key_lo = (window > 0 && pos >= window) ? pos - window + 1 : 0;
-  const int first_chunk = key_lo / (SB_PAGE * pages_per_chunk);
-  const int last_chunk = min(pos / (SB_PAGE * pages_per_chunk), n_chunks - 1);
-  if (chunk < first_chunk || chunk > last_chunk) return;   // uniform over the block
+  const int key_lo = first_key(pos, window);
 
   const int r = lane & 15;
   const int hq = ht * 16 + r;                 // query head within the group
@@ -1571,67 +1761,92 @@ attn_decode_long_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, fl
   WaveState<1> st;
   init_state<1>(st);
 
+  // the row's pages cut evenly into chunks and a chunk's into the waves' shares
   const int32_t *pt = page_table + size_t(seq) * max_pages;
-  const int pg_begin = max(chunk * pages_per_chunk + wave * ppw, key_lo / SB_PAGE);
-  const int pg_end = min(min(chunk * pages_per_chunk + (wave + 1) * ppw, pos / SB_PAGE + 1), max_pages);
+  const int page_lo = key_lo / SB_PAGE;
+  const int from = int((long long)pages * chunk / chunks), to = int((long long)pages * (chunk + 1) / chunks);
+  const int pg_begin = min(page_lo + from + (to - from) * wave / 4, max_pages);
+  const int pg_end = min(page_lo + from + (to - from) * (wave + 1) / 4, max_pages);
   const size_t page_elems = size_t(heads_kv) * SB_PAGE * HD;
   const size_t head_off = size_t(kvh) * SB_PAGE * HD;
   // a page number outside the cache: read page 0 and see none of its keys
-  auto page_of = [&](int pg, bool &ok) {
-    const int page = pt[pg];
+  auto place_of = [&](int page, bool &ok) {
     ok = page >= 0 && page < n_pages_total;
     return size_t(ok ? page : 0) * page_elems + head_off;
   };
-  HalfPage h0, h1;
+  HalfPage h[2];
   bool ok = false;
   size_t off = 0;
-  // The folded form: the first half page's loads go out before the block builds its queries.  The
-  // page that receives the row's own key and value is read like the others (before or after they
-  // are stored: the stores are not waited for) and its fragments are patched from LDS.
+  int next_page = 0;
+  // The folded form: the first page's loads go out before the block builds its queries.  The page that receives the row's own
+  // key and value is read like the others (before or after they are stored: the stores are not waited for) and its fragments
+  // are patched from LDS.
   if (pg_begin < pg_end) {
-    off = page_of(pg_begin, ok);
-    load_half_straight(h0, k_cache + off, v_cache + off, 0, lane);
+    off = place_of(pt[pg_begin], ok);
+    load_keys_straight(h, k_cache + off, lane);
+    load_values_straight(h, v_cache + off, lane);
+    next_page = pt[min(pg_begin + 1, max_pages - 1)];
   }
   if constexpr (FUSED) {
-    rope_store(rope_sh, first, freq, ra, seq, pos, kvh, group, heads_q, heads_kv, chunk == last_chunk, false,
+    rope_store(rope_sh, first, freq, ra, seq, pos, kvh, group, heads_q, heads_kv, chunk == chunks - 1, false,
                const_cast<bf16_t *>(k_cache), const_cast<bf16_t *>(v_cache), page_table, max_pages, n_pages_total);
     staged_q(qf[0], rope_sh, hq, col_ok, lane);
   } else {
     load_q(qf[0], q + (size_t(seq) * heads_q + head) * HD, col_ok, lane);
   }
   if (pg_begin < pg_end) {
-    // 32 keys from `base` on: all visible and written (the common case), or tested one by one
-    const int own_base = (FUSED && ra.store) ? (pos / 32) * 32 : -1;     // the half page of the row's own slot
-    auto attend = [&](HalfPage &h, int base, bool ok) {
-      if constexpr (FUSED) {
-        if (ok && base == own_base) patch_half(h, rope_sh, (base >> 5) & 1, pos % SB_PAGE, lane);
-      }
-      if (ok && base >= key_lo && base + 31 <= pos) {
-        attend_half<1, false>(st, qf, h, base, pos, key_lo, key_lo, pos, scale_log2, lane);
-      } else {
-        // hi < lo for a page that is not there: every value is cut, no key seen
-        attend_half<1, true>(st, qf, h, base, (ok && col_ok) ? pos : -1, key_lo, key_lo, ok ? pos : -1, scale_log2,
-                             lane);
-      }
+    // a page whose keys are tested one by one; hi < lo for a page that is not there: every value is cut, no key seen
+    const auto attend_tested = [&](int pg) {
+      attend_whole_page<true>(st, qf, h, pg * SB_PAGE, (ok && col_ok) ? pos : -1, key_lo, key_lo, ok ? pos : -1, scale_log2, lane, [] {});
     };
     int pg = pg_begin;
-    // every page but the last: the loads of the next half page go out before this half's
-    // products, with no branch between a load and its use
+    if (pg + 1 < pg_end && pg * SB_PAGE < key_lo) {      // a window that starts inside the first page
+      attend_tested(pg);
+      off = place_of(next_page, ok);
+      next_page = pt[min(pg + 2, max_pages - 1)];
+      load_keys_straight(h, k_cache + off, lane);
+      load_values_straight(h, v_cache + off, lane);
+      ++pg;
+    }
+    // every page but the last, all of whose keys are visible and written: its keys' registers take the next page's as soon as the
+    // scores are there, its values' behind the second product, and the page after it is looked up meanwhile
     for (; pg + 1 < pg_end; ++pg) {
-      load_half_straight(h1, k_cache + off, v_cache + off, 1, lane);
-      attend(h0, pg * SB_PAGE, ok);
       bool ok_next;
-      off = page_of(pg + 1, ok_next);
-      load_half_straight(h0, k_cache + off, v_cache + off, 0, lane);
-      attend(h1, pg * SB_PAGE + 32, ok);
+      off = place_of(next_page, ok_next);
+      next_page = pt[min(pg + 2, max_pages - 1)];
+      if (ok)
+        attend_whole_page<false>(st, qf, h, 0, 0, 0, 0, 0, scale_log2, lane, [&] { load_keys_straight(h, k_cache + off, lane); });
+      else
+        load_keys_straight(h, k_cache + off, lane);
+      load_values_straight(h, v_cache + off, lane);
       ok = ok_next;
     }
-    load_half_straight(h1, k_cache + off, v_cache + off, 1, lane);
-    attend(h0, pg * SB_PAGE, ok);
-    attend(h1, pg * SB_PAGE + 32, ok);
+    if constexpr (FUSED) {
+      if (ra.store && ok && pg == pos / SB_PAGE) {
+        const int slot = pos % SB_PAGE;
+        if (slot < 32) patch_half(h[0], rope_sh, 0, slot, lane);
+        else patch_half(h[1], rope_sh, 1, slot, lane);
+      }
+    }
+    attend_tested(pg);
   }
-  finish_decode_block<4>(st, lds_o, lds_m, lds_l, out, part_o, part_ml, wave, lane, chunk, first_chunk == last_chunk,
-                      seq, kvh, ht, group, heads_q, n_chunks, size_t(seq) * tiles + blk.tile);
+  finish_decode_block<4>(st, lds_o, lds_m, lds_l, out, part_o, part_ml, wave, lane, chunk, chunks == 1,
+                         seq, kvh, ht, group, heads_q, n_chunks, size_t(seq) * tiles + tile);
+}
+
+// The chunks of a row that hold partial results: [first, last].
+struct ChunkRange {
+  int first, last;
+};
+// wave_slots > 0: of the kernel above; else of the kernels whose chunks are pages_per_chunk pages of the table.
+__device__ __forceinline__ ChunkRange chunk_range(const int32_t *row_pos, int seq, int n_seqs, int tiles, int max_pages, int n_chunks,
+                                                  int window, int pages_per_chunk, int wave_slots, int fixed_share, int lane) {
+  const int pos = row_pos[seq];
+  if (wave_slots > 0) {
+    const DecodePlan plan = decode_plan(row_pos, n_seqs, tiles, max_pages, window, wave_slots, fixed_share, lane);
+    return ChunkRange{0, row_chunks(row_pages(pos, window, max_pages), plan.share) - 1};
+  }
+  return ChunkRange{first_key(pos, window) / (SB_PAGE * pages_per_chunk), min(pos / (SB_PAGE * pages_per_chunk), n_chunks - 1)};
 }
 
 // Merge the chunks of a (sequence, tile), at most kAtOnce of them, in ascending order: one thread
@@ -1639,37 +1854,44 @@ attn_decode_long_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, fl
 __global__ void __launch_bounds__(256)
 attn_decode_merge_kernel(bf16_t *__restrict__ out, const float *__restrict__ part_o,
                          const float *__restrict__ part_ml, const int32_t *__restrict__ row_pos,
-                         int heads_q, int heads_kv, int n_chunks, int window, int pages_per_chunk) {
+                         int heads_q, int heads_kv, int n_chunks, int window, int pages_per_chunk, int max_pages, int wave_slots,
+                         int fixed_share) {
   const int seq = blockIdx.z;
   const int group = heads_q / heads_kv;
   const int head_tiles = (group + 15) / 16;
   const int kvh = blockIdx.y / head_tiles, ht = blockIdx.y - kvh * head_tiles;
-  const int pos = row_pos[seq];
-  const int e = blockIdx.x * 256 + threadIdx.x;
+  const int e = blockIdx.x * 256 + threadIdx.x, c = min(e / HD, 15);      // (past the last column: the last once more, not stored)
   const size_t tile_index = size_t(seq) * gridDim.y + blockIdx.y;
   const float *po = part_o + (tile_index * n_chunks) * (HD * 16), *pml = part_ml + (tile_index * n_chunks) * 32;
   // Up to kAtOnce chunks: the partial results of all of them are asked for together with the
   // position, which says which of them count (a chunk past the last is the last once more);
   // waiting for the position first costs this short kernel a trip to memory of its two.
   constexpr int kAtOnce = 16;
-  float mv[kAtOnce], lv[kAtOnce], ov[kAtOnce];
-  {
-    const int c = e & 15;
-#pragma unroll
-    for (int ch = 0; ch < kAtOnce; ++ch) {
-      const size_t cc = size_t(min(ch, n_chunks - 1));
-      mv[ch] = pml[cc * 32 + c];
-      lv[ch] = pml[cc * 32 + 16 + c];
-      ov[ch] = po[cc * (HD * 16) + e];
-    }
+  const auto range_of = [&] {
+    return chunk_range(row_pos, seq, gridDim.z, gridDim.y, max_pages, n_chunks, window, pages_per_chunk, wave_slots, fixed_share,
+                       threadIdx.x & 63);
+  };
+  ChunkRange range{0, 1};
+  // (rows that fill the GPU by themselves hardly ever come in chunks: looked at first, so that nothing is read in vain)
+  const bool look_first = wave_slots > 0 && gridDim.y * gridDim.z * 4 >= unsigned(wave_slots);
+  if (look_first) {
+    range = range_of();
+    if (range.first == range.last) return;
   }
-  const int key_lo = (window > 0 && pos >= window) ? pos - window + 1 : 0;
-  const int first = key_lo / (SB_PAGE * pages_per_chunk), last = min(pos / (SB_PAGE * pages_per_chunk), n_chunks - 1);
+  float mv[kAtOnce], lv[kAtOnce], ov[kAtOnce];
+#pragma unroll
+  for (int ch = 0; ch < kAtOnce; ++ch) {
+    const size_t cc = size_t(min(ch, n_chunks - 1));
+    mv[ch] = pml[cc * 32 + c];
+    lv[ch] = pml[cc * 32 + 16 + c];
+    ov[ch] = po[cc * (HD * 16) + min(e, HD * 16 - 1)];
+  }
+  if (!look_first) range = range_of();
+  const int first = range.first, last = range.last;
   if (first == last) return;      // the decode kernel has written the result itself
   // rescaled to the common maximum and added in ascending chunk order
-  const int c = e & 15, d = e >> 4;
-  const int hh = ht * 16 + c;
-  if (hh >= group) return;
+  const int hh = ht * 16 + e / HD;
+  if (e >= HD * 16 || hh >= group) return;
   float m = -__builtin_inff();
 #pragma unroll
   for (int ch = 0; ch < kAtOnce; ++ch) m = (ch >= first && ch <= last) ? fmaxf(m, mv[ch]) : m;
@@ -1682,26 +1904,28 @@ attn_decode_merge_kernel(bf16_t *__restrict__ out, const float *__restrict__ par
     o = use ? o + ov[ch] * f : o;
     l = use ? l + lv[ch] * f : l;
   }
-  out[(size_t(seq) * heads_q + kvh * group + hh) * HD + d] = f32_to_bf16(l > 0.f ? o / l : 0.f);
+  out[(size_t(seq) * heads_q + kvh * group + hh) * HD + e % HD] = f32_to_bf16(l > 0.f ? o / l : 0.f);
 }
 
-// The same for rows of many chunks: a block takes 64 elements, its four waves every fourth
+constexpr int kMergeWaves = 8;
+// The same for rows of many chunks: a block takes 64 elements, its eight waves every eighth
 // chunk each, eight chunks' partial results in flight at a time (one thread walking all chunks
 // waits for memory once per few chunks: 128 chunks took it longer than the decode kernel took to
-// read the keys).  A wave keeps a running maximum of its own; the four meet in LDS and are folded
-// in wave order.  Grid (HD * 16 / 64, tiles, sequences).
-__global__ void __launch_bounds__(256)
+// read the keys).  A wave keeps a running maximum of its own; the eight meet in LDS and are folded
+// in wave order.  Grid (columns * HD / 64, tiles, sequences).
+__global__ void __launch_bounds__(64 * kMergeWaves)
 attn_decode_merge_many_kernel(bf16_t *__restrict__ out, const float *__restrict__ part_o,
                               const float *__restrict__ part_ml, const int32_t *__restrict__ row_pos,
-                              int heads_q, int heads_kv, int n_chunks, int window, int pages_per_chunk) {
-  __shared__ float lds_m[4][64], lds_l[4][64], lds_o[4][64];
+                              int heads_q, int heads_kv, int n_chunks, int window, int pages_per_chunk, int max_pages, int wave_slots,
+                              int fixed_share) {
+  __shared__ float lds_m[kMergeWaves][64], lds_l[kMergeWaves][64], lds_o[kMergeWaves][64];
   const int seq = blockIdx.z;
   const int group = heads_q / heads_kv;
   const int head_tiles = (group + 15) / 16;
   const int kvh = blockIdx.y / head_tiles, ht = blockIdx.y - kvh * head_tiles;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int e = blockIdx.x * 64 + lane;                 // < HD * 16: 64 divides it
-  const int c = e & 15, d = e >> 4;
+  const int c = e / HD, d = e % HD;
   const size_t tile_index = size_t(seq) * gridDim.y + blockIdx.y;
   const float *po = part_o + (tile_index * n_chunks) * (HD * 16), *pml = part_ml + (tile_index * n_chunks) * 32;
   constexpr int kAtOnce = 8;
@@ -1709,7 +1933,7 @@ attn_decode_merge_many_kernel(bf16_t *__restrict__ out, const float *__restrict_
   auto ask = [&](int base) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kAtOnce; ++i) {
-      const size_t cc = size_t(min(base + 4 * i, n_chunks - 1));   // (past the end: the last once more, not used)
+      const size_t cc = size_t(min(base + kMergeWaves * i, n_chunks - 1));   // (past the end: the last once more, not used)
       mv[i] = pml[cc * 32 + c];
       lv[i] = pml[cc * 32 + 16 + c];
       ov[i] = po[cc * (HD * 16) + e];
@@ -1717,16 +1941,16 @@ attn_decode_merge_many_kernel(bf16_t *__restrict__ out, const float *__restrict_
   };
   // the first round goes out together with the position, which says which chunks count
   ask(wave);
-  const int pos = row_pos[seq];
-  const int key_lo = (window > 0 && pos >= window) ? pos - window + 1 : 0;
-  const int first = key_lo / (SB_PAGE * pages_per_chunk), last = min(pos / (SB_PAGE * pages_per_chunk), n_chunks - 1);
+  const ChunkRange range = chunk_range(row_pos, seq, gridDim.z, gridDim.y, max_pages, n_chunks, window, pages_per_chunk, wave_slots,
+                                       fixed_share, lane);
+  const int first = range.first, last = range.last;
   if (first == last) return;      // the decode kernel has written the result itself
   float m = -__builtin_inff(), o = 0.f, l = 0.f;
-  for (int base = wave;; base += 4 * kAtOnce) {
-    if (base + 4 * (kAtOnce - 1) >= first) {
+  for (int base = wave;; base += kMergeWaves * kAtOnce) {
+    if (base + kMergeWaves * (kAtOnce - 1) >= first) {
 #pragma unroll
       for (int i = 0; i < kAtOnce; ++i) {
-        const int ch = base + 4 * i;
+        const int ch = base + kMergeWaves * i;
         const bool use = ch >= first && ch <= last;
         const float m_new = use ? fmaxf(m, mv[i]) : m;
         const float m_use = m_new == -__builtin_inff() ? 0.f : m_new;
@@ -1736,8 +1960,8 @@ attn_decode_merge_many_kernel(bf16_t *__restrict__ out, const float *__restrict_
         m = m_new;
       }
     }
-    if (base + 4 * kAtOnce > last) break;
-    ask(base + 4 * kAtOnce);
+    if (base + kMergeWaves * kAtOnce > last) break;
+    ask(base + kMergeWaves * kAtOnce);
   }
   lds_m[wave][lane] = m;
   lds_l[wave][lane] = l;
@@ -1746,11 +1970,13 @@ attn_decode_merge_many_kernel(bf16_t *__restrict__ out, const float *__restrict_
   if (wave != 0) return;
   const int hh = ht * 16 + c;
   if (hh >= group) return;
-  float m_all = fmaxf(fmaxf(lds_m[0][lane], lds_m[1][lane]), fmaxf(lds_m[2][lane], lds_m[3][lane]));
+  float m_all = lds_m[0][lane];
+#pragma unroll
+  for (int w = 1; w < kMergeWaves; ++w) m_all = fmaxf(m_all, lds_m[w][lane]);
   if (m_all == -__builtin_inff()) m_all = 0.f;
   float o_all = 0.f, l_all = 0.f;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < kMergeWaves; ++w) {
     const float f = __builtin_amdgcn_exp2f(lds_m[w][lane] - m_all);
     o_all += lds_o[w][lane] * f;
     l_all += lds_l[w][lane] * f;
@@ -1804,53 +2030,15 @@ int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra,
   const int head_tiles = (group + 15) / 16;
   hipStream_t s = (hipStream_t)stream;
   SB_SUPPORT(heads_kv * head_tiles <= 65535, "%s: too many heads", who);
-  // A wave takes one page and asks for all of it at once (one round trip to memory), or, when
-  // two pages per wave still leave a block for every CU, several pages in a row with half a page
-  // in flight while the half before it is multiplied.
+  // A wave takes one page and asks for all of it at once (one round trip to memory).  Where the widest row's chunks for every row
+  // would be blocks for most of the GPU, the chunks are dealt out by what the rows hold.
   const long long per_chunk = (long long)heads_kv * head_tiles * n_seqs;
-  int ppw = 1;
-  if (HD <= 128 && (long long)((max_pages + 7) / 8) * per_chunk >= 256) {
-    // How many pages in a row: the count with the least estimated time, in microseconds, from
-    // what was measured (MI355X, cold caches).  A wave gets through a page in about 3.3 us
-    // whatever the head size (two round trips to memory); a CU streams about 27 GB/s, all of
-    // them together 5.3 TB/s; a block costs about 2 us besides (fitted: with 4 the choices lost 42 us over
-    // 29 measured cases of 1 to 128 sequences and 2,000 to 131,000 keys, with 2 they lose 5); more than one chunk costs the
-    // partial results and the second kernel, about 8 us.  The table's width is taken for the rows' length less half of the 16
-    // pages it is rounded up by.  One chunk (a quarter of the width per wave) is among the
-    // candidates: it wins when sequences x kv heads alone fill most of the GPU.
-    const double page_bytes = 2.0 * SB_PAGE * HD * 2;
-    const int pages = max_pages > 8 ? max_pages - 8 : 1;
-    const int whole = (max_pages + kPagesPerChunk - 1) / kPagesPerChunk;
-    const int candidates[5] = {2, 4, 8, 16, whole < 2 ? 2 : whole};
-    double best = -1.0;
-    for (int c : candidates) {
-      const int chunks = (max_pages + 4 * c - 1) / (4 * c);
-      const int full = pages / (4 * c) > 1 ? pages / (4 * c) : 1;
-      const double busy = double(per_chunk) * full < 256.0 ? double(per_chunk) * full : 256.0;
-      const double rate = busy * 27e3 < 5.3e6 ? busy * 27e3 : 5.3e6;            // bytes per us
-      const int run = c < pages ? c : pages;
-      // a block spends about 2 us on what is not streaming (look-ups, queries, the merge)
-      // blocks that a CU holds together share its rate, so the CU with the most blocks sets the
-      // time: 260 equal blocks take as long as 512 (measured: 65 sequences x 4 kv heads x 2,048
-      // keys 77 us in one chunk against 45 for 64 sequences, 63 in chunks of eight pages)
-      const long long n_busy = per_chunk * full;
-      // (blocks of few pages in a row pay less of it, the CU's second block being short: 260
-      // blocks of two pages a wave took 22.7 us where 130 of four took 25.7)
-      const double rounds = n_busy > 256 ? double((n_busy + 255) / 256) * 256.0 / double(n_busy) : 1.0;
-      const double uneven = 1.0 + (rounds - 1.0) * (run < 8 ? run / 8.0 : 1.0);
-      const double stream_us =
-          double(per_chunk) * pages * page_bytes / rate * (1.0 + 2.0 / (run * 3.3)) * uneven;
-      const double in_a_row = run * 3.3 + 2.0;
-      const double t = (stream_us > in_a_row ? stream_us : in_a_row) + (chunks > 1 ? 8.0 : 0.0);
-      if (best < 0.0 || t < best) best = t, ppw = c;
-    }
-  }
-  // a test's or a measurement's choice (0: the launcher's own)
-  if (pages_per_wave > 0 && (pages_per_wave == 1 || HD <= 128)) ppw = pages_per_wave;
+  // a test's or a measurement's choice (0: the launcher's own): pages of a wave
+  const bool dealt = HD <= 128 && (pages_per_wave > 1 || (pages_per_wave == 0 && (long long)((max_pages + 7) / 8) * per_chunk >= kDealtFrom));
   // five to eight pages a row: a block of eight waves takes a row whole (with more rows than half the CUs the chunks fill the GPU as it is)
-  const bool whole_rows = kWholeRows && ppw == 1 && pages_per_wave == 0 && max_pages > kPagesPerChunk && max_pages <= kWholePages &&
+  const bool whole_rows = kWholeRows && !dealt && pages_per_wave == 0 && max_pages > kPagesPerChunk && max_pages <= kWholePages &&
                           per_chunk <= 128;
-  const int pages_per_chunk = whole_rows ? kWholePages : kPagesPerChunk * ppw;
+  const int pages_per_chunk = whole_rows ? kWholePages : kPagesPerChunk;
   const int n_chunks = (max_pages + pages_per_chunk - 1) / pages_per_chunk;
   SB_SUPPORT((long long)n_chunks * per_chunk <= 0x7fffffffLL, "%s: too many blocks", who);
   const unsigned grid = unsigned((long long)n_chunks * per_chunk);
@@ -1859,31 +2047,32 @@ int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra,
       page_table, max_pages, n_pages_total, row_pos, heads_q, heads_kv, n_chunks, scale *kLog2e, window
   if (whole_rows) {
     if constexpr (kWholeRows) {
-      if (fused) attn_decode_kernel<true, true, kWholePages><<<grid, 64 * kWholePages, 0, s>>>(SB_ARGS, n_seqs);
-      else attn_decode_kernel<true, false, kWholePages><<<grid, 64 * kWholePages, 0, s>>>(SB_ARGS, n_seqs);
+      if (fused) attn_decode_kernel<true, kWholePages><<<grid, 64 * kWholePages, 0, s>>>(SB_ARGS, n_seqs);
+      else attn_decode_kernel<false, kWholePages><<<grid, 64 * kWholePages, 0, s>>>(SB_ARGS, n_seqs);
     }
-  } else if (ppw > 1) {
+  } else if (dealt) {
+    // a chunk for every row and tile, and as many as the waves' shares fill; no more than there are
+    const long long most = per_chunk + (pages_per_wave > 1 ? per_chunk * n_chunks : kWaveSlots / kPagesPerChunk);
+    const unsigned blocks = unsigned(most < (long long)grid ? most : (long long)grid);
     // (only head sizes up to 128 get here, and only they hold this kernel)
     if constexpr (HD <= 128) {
-      if (fused) attn_decode_long_kernel<true><<<grid, 256, 0, s>>>(SB_ARGS, ppw, n_seqs);
-      else attn_decode_long_kernel<false><<<grid, 256, 0, s>>>(SB_ARGS, ppw, n_seqs);
+      if (fused) attn_decode_dealt_kernel<true><<<blocks, 256, 0, s>>>(SB_ARGS, n_seqs, kWaveSlots, pages_per_wave);
+      else attn_decode_dealt_kernel<false><<<blocks, 256, 0, s>>>(SB_ARGS, n_seqs, kWaveSlots, pages_per_wave);
     }
-  } else if ((long long)n_chunks * per_chunk <= 1536) {
-    if (fused) attn_decode_kernel<true, true, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
-    else attn_decode_kernel<true, false, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
   } else {
-    if (fused) attn_decode_kernel<false, true, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
-    else attn_decode_kernel<false, false, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
+    if (fused) attn_decode_kernel<true, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
+    else attn_decode_kernel<false, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
   }
 #undef SB_ARGS
   int rc = sb::check_launch(who);
   if (rc != SB_OK || n_chunks == 1) return rc;
+  const int elements = (group < 16 ? group : 16) * HD;      // of a tile: its columns that have a head
   if (n_chunks <= 16)
-    attn_decode_merge_kernel<<<dim3((HD * 16 + 255) / 256, heads_kv * head_tiles, n_seqs), 256, 0, s>>>(
-        (bf16_t *)out, part_o, part_ml, row_pos, heads_q, heads_kv, n_chunks, window, pages_per_chunk);
+    attn_decode_merge_kernel<<<dim3((elements + 255) / 256, heads_kv * head_tiles, n_seqs), 256, 0, s>>>(
+        (bf16_t *)out, part_o, part_ml, row_pos, heads_q, heads_kv, n_chunks, window, pages_per_chunk, max_pages, dealt ? kWaveSlots : 0, pages_per_wave);
   else
-    attn_decode_merge_many_kernel<<<dim3(HD * 16 / 64, heads_kv * head_tiles, n_seqs), 256, 0, s>>>(
-        (bf16_t *)out, part_o, part_ml, row_pos, heads_q, heads_kv, n_chunks, window, pages_per_chunk);
+    attn_decode_merge_many_kernel<<<dim3((elements + 63) / 64, heads_kv * head_tiles, n_seqs), 64 * kMergeWaves, 0, s>>>(
+        (bf16_t *)out, part_o, part_ml, row_pos, heads_q, heads_kv, n_chunks, window, pages_per_chunk, max_pages, dealt ? kWaveSlots : 0, pages_per_wave);
   return sb::check_launch(who);
 }
 

@@ -1617,6 +1617,44 @@ def test_attention_decode_folded_in_where_one_block_takes_a_row(hq, hkv, hd, rot
     folded_against_two_kernels(hq, hkv, hd, rot, window, 0, lens)
 
 
+# (heads, kv heads, head size, the rows' numbers of keys): rows past the 64 that a wave looks at at once, two tiles of heads a kv head, a
+# wave's share of one page and of several, rows that stay whole, one long row among short ones, one page a row
+DEALT = [(4, 2, 16, [1 + 31 * i % 2100 for i in range(130)]), (20, 1, 64, [64 * (1 + 7 * i % 23) for i in range(70)]),
+         (28, 4, 32, [2000 + 97 * i for i in range(33)]), (28, 4, 128, [640 - i % 3 for i in range(64)]), (14, 2, 64, [20000] + [5] * 40),
+         (8, 8, 48, [30 + i for i in range(33)])]
+
+
+@pytest.mark.parametrize("hq, hkv, hd, lens", DEALT, ids=lambda v: f"{len(v)}rows" if isinstance(v, list) else str(v))
+@pytest.mark.parametrize("window", [0, 70, 1000])
+def test_attention_decode_deals_pages_out(hq, hkv, hd, lens, window):
+    """Many rows of unequal length, whose pages the kernel deals out to its blocks, against blocks of four pages of a row each: the
+    same sums of float32 numbers in another order, then one rounding to bfloat16.  Every ninth row has no page."""
+    from sonicboom_amd import ops
+    width = max(-(-n // 64) for n in lens)
+    assert -(-width // 8) * len(lens) * hkv * -(-(hq // hkv) // 16) >= 256
+    table = torch.full((len(lens), width), -1, dtype=torch.int32)
+    n_pages = sum(-(-n // 64) for n in lens) + 3
+    pages = iter(torch.randperm(n_pages, generator=torch.Generator().manual_seed(1)).tolist())
+    for i, n in enumerate(lens):
+        for pg in range(-(-n // 64)):
+            table[i, pg] = next(pages)
+        if window:
+            table[i, :max(n - window, 0) // 64] = -1         # the cache gives pages behind a window back
+        if i % 9 == 5:
+            table[i] = -1
+    kc, vc = (randn(*shape, seed=2).to(BF16).to(DEV) for shape in ((n_pages, hkv, 64, hd), (n_pages, hkv, hd, 64)))
+    q, pos = randn(len(lens), hq * hd, seed=3).to(BF16).to(DEV), torch.tensor([n - 1 for n in lens], dtype=torch.int32).to(DEV)
+    run = lambda: ops.attention_decode_mfma(q, kc, vc, table.to(DEV), pos, hq, hkv, hd, hd ** -0.5, window).float()
+    got, again = run(), run()
+    with ops.attention_decode_pages_per_wave(hd, 1):
+        want = run()
+    assert torch.equal(got, again)
+    assert (got[5::9] == 0).all() and want.abs().max() > 0.1
+    # probabilities are rounded to bfloat16 (2^-9 of each) relative to another maximum, as keys meet in other steps: the sums' part
+    # in that is at most 2^-8 of the values' largest, and half of one rounding of each result
+    assert ((got - want).abs() <= 2.0 ** -8 * vc.float().abs().max() * 0.5 + want.abs() * 2.0 ** -8).all()
+
+
 @pytest.mark.parametrize("vocab", [5, 256, 1000, 152064])
 def test_argmax_first_maximum(vocab):
     from sonicboom_amd import ops
