@@ -1312,14 +1312,21 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
   a.vec4 = n_out % 4 == 0 && (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(resid)) % 16 == 0;
   const bool direct_ok = packed && n_in % 64 == 0;
   int variant = pick_shape(n_rows, n_out, n_in, a.gated, direct_ok);
-  // Gated products of a few hundred rows (K cannot be cut over the grid): 128 x 128 tiles straight into LDS
-  // where they make one round over the CUs (288 rows against 9,728 x 896: 14.2 us, through registers 15.1); a
-  // little over one round, 64 x 128 tiles, three to a CU (183 rows against 17,920 x 1,536, 280 tiles of 128: 26.4 and 31.5).
+  // Tiles that make one round over the CUs go straight into LDS with four stages' buffers, a block a CU: a stage of 64 k then takes
+  // 0.33 us in tiles of 64 x 128 and 0.55 in 128 x 128, through registers 0.65 (600 rows against 2,560 x 2,048 15.9, 21.4 and 22.6
+  // us; 400 against 4,608 x 3,584 25.2, 30.0 and 33.8, 600 there, 360 tiles of 64, 46.5, 34.7 and 38.0; gated, 183 against 9,728 x 896 10.8, 13.3 and
+  // 14.6, 288 there 18.1, 13.3 and 15.1).  Gated, a little over one round: 64 x 128 tiles, three to a CU (183 rows against 17,920 x
+  // 1,536, 280 tiles of 128: 26.4 and 31.5).
   int path = 0;
-  if (gated && direct_ok && variant == 0 && n_rows <= 384) {
-    const long long tiles = (long long)((n_rows + 127) / 128) * ((n_out + 63) / 64);
-    if (tiles <= sb::cu_count()) path = 2;
-    else if (tiles <= sb::cu_count() * 3 / 2 && (n_rows + 63) / 64 * 64 < (n_rows + 127) / 128 * 128) variant = 5, path = 2;
+  if (direct_ok && variant == 0) {
+    const int bn = gated ? 64 : 128;
+    const long long across = (n_out + bn - 1) / bn;
+    const auto one_round = [&](long long tiles) { return (tiles + kXcds - 1) / kXcds * kXcds <= sb::cu_count(); };
+    const long long tiles = (long long)((n_rows + 127) / 128) * across;
+    if (one_round((long long)((n_rows + 63) / 64) * across)) variant = 5, path = 2;
+    else if (one_round(tiles)) path = 2;
+    else if (gated && n_rows <= 384 && tiles <= sb::cu_count() * 3 / 2 && (n_rows + 63) / 64 * 64 < (n_rows + 127) / 128 * 128)
+      variant = 5, path = 2;
   }
   // a test's or a measurement's choice: the shape (0..5) + 16 * the path (0: the launcher's, 1:
   // through registers, 2: straight into LDS)
@@ -1349,7 +1356,7 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
   SB_SUPPORT(path < 2 || direct_ok, "sb_gemm_mfma_bf16: the direct path takes packed weights and an inner size in 64s");
   // left to themselves the shapes of 192 and 256 rows go straight into LDS; the smaller tiles' stages are too
   // short for loads that run one stage ahead, and the register path, which runs two ahead, is
-  // faster there unless the tiles make one round and LDS holds four stages of each
+  // faster there unless the tiles make one round and LDS holds four stages of each (above)
   const bool direct = path >= 2 || (path == 0 && direct_ok && (variant == 1 || variant == 2 || variant == 4));
   SB_SUPPORT(variant < 3 || direct, "sb_gemm_mfma_bf16: the shapes 128 x 256, 192 x 256 and 64 x 128 exist on the direct path only");
   if (direct) {
