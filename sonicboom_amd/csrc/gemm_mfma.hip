@@ -1403,12 +1403,15 @@ namespace {
 // whole prompt steps that gave 4.5 % at 1,152 rows of the 7B sizes, nothing at 1,792 of the 3B ones, and cost 1 % at 2,048 of the
 // 3B sizes and at 1,800 and 2,300 of 2,048 wide layers of other designs: not taken.
 //
-// A few hundred rows: the same tiles of 128 x 128, or of 64 x 128, loaded straight into LDS with four
+// Some hundred rows: the same tiles of 128 x 128, or of 64 x 128, loaded straight into LDS with four
 // stages' buffers, a block a CU, where tiles x slices make one round over each die's 32 CUs.  A launch costs
-// 3.5 us and a stage of 64 k, measured at 183 to 500 rows of the 0.5B to 7B products, 0.33 us (64 rows), 0.55 (128 rows)
-// and 0.65 (128 x 128 through registers); the consumer reads and the product writes a slice at 4 TB/s.
-// 183 rows against 1,536 x 1,536: 8.5 us through registers, 6.2; 288 against 896 x 4,864: 14.9 and 9.8; 183 against
-// 3,584 x 18,944: 50.9 and 45.5.
+// 3.5 us and a stage of 64 k 0.33 us (64 rows), 0.55 (128 rows) and 0.75 (128 x 128 through registers); a slice is written and
+// read, and the stream and its norm cost two and a half times as much, at 2.9 TB/s (up to 640 rows 4).  183 rows against 1,536 x 1,536: 8.5 us through
+// registers, 6.2; 288 against 896 x 4,864: 14.9 and 9.8; with the pass that adds and norms, 700 against 2,048 x 1,536 26.0 and 19.8, 900
+// against 1,536 x 1,536 26.0 and 20.0, 520 against 896 x 4,864 26.6 and 18.5.  A whole product whose tiles make one round is as fast a
+// stage, and its residual and norm move three and a half planes in 4 us more: taken where that is less (1,300 rows against 1,536 x 8,960 81
+// and 60 us, 896 x 896 20.7 and 16.1, 2,048 x 1,536 31.3 and 27.4; 700 rows against 1,536 x 1,536 19.4 in slices and 20.2), and
+// past 1,200 rows where only tiles through registers are left (1,600 against 2,048 x 11,008 109 and 98, 2,560 x 2,048 48 and 42).
 enum PartialTile { kRegisters128, kBig, kDirect128, kDirect64 };
 struct PartialPlan { int slices; PartialTile tile; };
 double load_factor(long long blocks) { return blocks <= 170 ? 0.72 : 0.72 + 0.28 * double(blocks - 170) / 86.0; }
@@ -1446,20 +1449,25 @@ PartialPlan partial_plan(int n_rows, int n_out, int n_in, bool direct_ok) {
       return {(n_k + per - 1) / per, kBig};
     }
   }
-  if (s > 1 && direct_ok && n_rows <= 512) {
+  if (s > 1 && direct_ok) {
+    const double plane = n_rows * double(n_out) * 4.0 / (n_rows <= 640 ? 4e6 : 2.9e6);      // us that a slice takes to write or read
     const auto cost = [&](double stage_us, long long slices) {
-      return stage_us * double((n_k + slices - 1) / slices) + 2.0 * slices * n_rows * double(n_out) * 4.0 / 4e6;
+      return stage_us * double((n_k + slices - 1) / slices) + (2.0 * slices + 2.5) * plane;
     };
-    double best = cost(0.65, s);
+    const auto one_round = [&](long long n_tiles) { return (n_tiles + kXcds - 1) / kXcds <= sb::cu_count() / kXcds; };
+    const auto tiles_of = [&](int bm) { return (long long)((n_rows + bm - 1) / bm) * ((n_out + 127) / 128); };
+    double best = cost(0.75, s);
     PartialTile tile = kRegisters128;
     for (int half = 0; half < 2; ++half) {
-      const int bm = half ? 64 : 128;
-      const long long n_tiles = (long long)((n_rows + bm - 1) / bm) * ((n_out + 127) / 128);
+      const long long n_tiles = tiles_of(half ? 64 : 128);
       for (long long s2 = 2; s2 <= 8 && (n_tiles + kXcds - 1) / kXcds * s2 <= sb::cu_count() / kXcds && s2 * 3 <= n_k; ++s2) {
         const double t = cost(half ? 0.33 : 0.55, s2);
         if (t < best) best = t, tile = half ? kDirect64 : kDirect128, s = s2;
       }
     }
+    const double stage_whole = one_round(tiles_of(64)) ? 0.33 : one_round(tiles_of(128)) ? 0.45 : 0.0;
+    if ((tile == kRegisters128 && n_rows > 1200) || (stage_whole > 0.0 && stage_whole * n_k + 3.5 * plane + 4.0 < best))
+      return {1, kRegisters128};
     const int per = int((n_k + s - 1) / s);
     return {(n_k + per - 1) / per, tile};
   }
