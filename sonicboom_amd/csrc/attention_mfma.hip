@@ -1040,6 +1040,9 @@ attn_prefill_tall_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ q,
 //   238 -> 52.  4 on 4, size 64 (tiles of 64 rows): 8.4 -> 5.2, 19.1 -> 7.3, 78 -> 18, 258 -> 64.
 constexpr bool kKeysOk = HD <= 128;      // (beyond, a page's fragments no longer fit the registers at once)
 constexpr int kKeyWaves = 8;
+// Waves of several pages keep one in flight: 12 heads of 128 on 2, 183 rows on 461 to 961 keys, 15.3 -> 14.0 us in a step.  Smaller heads
+// would lose a CU's second block to the registers it takes (heads of 64: 336 blocks of short prompts 5.5 and 7.2 us).
+constexpr bool kKeysInFlight = HD > 64;
 constexpr int kKeyStride = HD + 4;       // floats of a column's sums in LDS: lanes of a store four banks apart
 constexpr int kKeyLds = (kKeyWaves * 16 * kKeyStride + kKeyWaves * 32) * 4;
 
@@ -1079,12 +1082,53 @@ attn_prefill_keys_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ q,
     WaveState<1> st;
     init_state<1>(st);
     const int32_t *pt = page_table + size_t(seq) * max_pages;
-    const int pg_hi = min(key_hi / SB_PAGE, max_pages - 1);
-    for (int pg = key_lo / SB_PAGE + wave; pg <= pg_hi; pg += kKeyWaves) {
-      const int page = pt[pg];
-      if (page < 0 || page >= n_pages_total) continue;
-      const size_t off = (size_t(page) * heads_kv + kvh) * SB_PAGE * HD;
-      attend_page<1>(st, qf, k_cache + off, v_cache + off, pg * SB_PAGE, col_pos, col_lo, key_lo, key_hi, scale_log2, lane);
+    const int pg_end = min(key_hi / SB_PAGE, max_pages - 1) + 1;
+    int pg = key_lo / SB_PAGE + wave;
+    const size_t page_elems = size_t(heads_kv) * SB_PAGE * HD, head_off = size_t(kvh) * SB_PAGE * HD;
+    const auto place_of = [&](int page, bool &ok) {
+      ok = page >= 0 && page < n_pages_total;
+      return size_t(ok ? page : 0) * page_elems + head_off;
+    };
+    if (!kKeysInFlight || pg + kKeyWaves >= pg_end) {      // page by page, of a page the half that holds a visible key, or both
+      for (; pg < pg_end; pg += kKeyWaves) {
+        bool ok;
+        const size_t off = place_of(pt[pg], ok);
+        if (ok) attend_page<1>(st, qf, k_cache + off, v_cache + off, pg * SB_PAGE, col_pos, col_lo, key_lo, key_hi, scale_log2, lane);
+      }
+    } else if constexpr (kKeysInFlight) {
+      // Several, a page in flight throughout: the fragments' registers take the next page's keys as soon as the scores are there,
+      // its values behind the second product, and the page after it is looked up meanwhile.  Rows follow one another, so a key
+      // is hidden from some of them in the last two pages alone, and behind a window's edge in the first two: the waves' last
+      // and first ones, whose keys are tested one by one.
+      HalfPage h[2];
+      bool ok;
+      size_t off = place_of(pt[pg], ok);
+      const auto ask_keys = [&] { load_keys_straight(h, k_cache + off, lane); };
+      const auto ask_values = [&] { load_values_straight(h, v_cache + off, lane); };
+      const auto tested = [&] {       // hi < lo for a page that is not there: every value is cut, no key seen
+        attend_whole_page<true>(st, qf, h, pg * SB_PAGE, ok ? col_pos : -1, col_lo, key_lo, ok ? key_hi : -1, scale_log2, lane, [] {});
+      };
+      ask_keys();
+      ask_values();
+      int next_page = pt[pg + kKeyWaves];
+      if (pg * SB_PAGE < (window > 0 ? key_hi - window + 1 : 0)) {       // (the first key that every row sees)
+        tested();
+        off = place_of(next_page, ok);
+        next_page = pt[min(pg + 2 * kKeyWaves, max_pages - 1)];
+        ask_keys();
+        ask_values();
+        pg += kKeyWaves;
+      }
+      for (; pg + kKeyWaves < pg_end; pg += kKeyWaves) {
+        bool ok_next;
+        off = place_of(next_page, ok_next);
+        next_page = pt[min(pg + 2 * kKeyWaves, max_pages - 1)];
+        if (ok) attend_whole_page<false>(st, qf, h, 0, 0, 0, 0, 0, scale_log2, lane, ask_keys);
+        else ask_keys();
+        ask_values();
+        ok = ok_next;
+      }
+      tested();
     }
     float l = st.l[0];
     l += __shfl_xor(l, 16, 64);
@@ -1155,7 +1199,7 @@ bool keys_ahead(int group, double blocks, double live, double most, double mean,
 // block takes page 4 * chunk + w; columns are the query heads of the kv head.
 //
 // Partial results, when a row's keys span several chunks, go to
-//   part_o  float [seqs][tiles][n_chunks][HD][16]   (unnormalised sums, column fastest)
+//   part_o  float [seqs][tiles][n_chunks][16][HD]   (unnormalised sums, a column's d together)
 //   part_ml float [seqs][tiles][n_chunks][2][16]    (maximum, sum)
 // and are merged by attn_decode_merge_kernel (up to 16 chunks, in ascending order) or
 // attn_decode_merge_many_kernel.  (Merging in the block
