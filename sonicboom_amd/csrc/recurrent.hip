@@ -26,8 +26,17 @@ struct Gate {
   float a, b, silu_g;
 };
 
-__device__ __forceinline__ Gate mingru_gate(const float *__restrict__ row, int width, int ch) {
-  const float zp = row[ch], up = row[width + ch], gp = row[2 * size_t(width) + ch];
+// A row's three numbers of a channel (OUT: the output's gate among them).
+struct Row {
+  float z, u, g;
+};
+template <bool OUT>
+__device__ __forceinline__ Row mingru_row(const float *__restrict__ row, int width, int ch) {
+  return Row{row[ch], row[width + ch], OUT ? row[2 * size_t(width) + ch] : 0.0f};
+}
+
+__device__ __forceinline__ Gate mingru_gate(const Row &row) {
+  const float zp = row.z, up = row.u, gp = row.g;
   const float z = sigmoid_f(zp);
   const float cand = up >= 0.0f ? up + 0.5f : sigmoid_f(up);
   Gate g;
@@ -48,11 +57,32 @@ mingru_serial_kernel(TO *__restrict__ out, const float *__restrict__ p, float *_
   float *sp = state + size_t(slots[seq]) * width + ch;
   float s = *sp;
   for (int r = r0; r < r1; ++r) {
-    const Gate g = mingru_gate(p + size_t(r) * 3 * width, width, ch);
+    const Gate g = mingru_gate(mingru_row<true>(p + size_t(r) * 3 * width, width, ch));
     s = g.a * s + g.b;
     st_f(out, size_t(r) * width + ch, s * g.silu_g);
   }
   if (r1 > r0) *sp = s;
+}
+
+// The rows [r0, r0 + n) of a channel in order, the next kRows of them asked for ahead of these rows' arithmetic (a row at a time
+// a thread waits for memory once a row: 4,001 rows of 4,096 channels, folding 52 us and 36 so, walking 65 and WALK_NOW).
+constexpr int kRows = 4;
+template <bool OUT, typename F>
+__device__ __forceinline__ void mingru_rows(const float *__restrict__ p, int r0, int n, int width, int ch, F &&each) {
+  Row at[kRows], next[kRows];
+  const auto ask = [&](Row (&to)[kRows], int from) {
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) to[i] = mingru_row<OUT>(p + size_t(r0 + min(from + i, n - 1)) * 3 * width, width, ch);
+  };
+  ask(at, 0);
+  for (int done = 0; done < n; done += kRows) {
+    ask(next, done + kRows);                     // (past the end: the last row once more, not used)
+#pragma unroll
+    for (int i = 0; i < kRows; ++i)
+      if (done + i < n) each(r0 + done + i, mingru_gate(at[i]));
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) at[i] = next[i];
+  }
 }
 
 // chunk c of the launch: rows [first, first + n) of sequence seq, as int32 [n_chunks, 4] =
@@ -65,11 +95,11 @@ mingru_fold_kernel(float2 *__restrict__ folded, const float *__restrict__ p, con
   if (ch >= width) return;
   const int r0 = chunks[4 * c], n = chunks[4 * c + 1];
   float a = 1.0f, b = 0.0f;
-  for (int r = r0; r < r0 + n; ++r) {
-    const Gate g = mingru_gate(p + size_t(r) * 3 * width, width, ch);
-    a = g.a * a;
-    b = g.a * b + g.b;
-  }
+  if (n > 0)
+    mingru_rows<false>(p, r0, n, width, ch, [&](int, const Gate &g) {
+      a = g.a * a;
+      b = g.a * b + g.b;
+    });
   folded[size_t(c) * width + ch] = make_float2(a, b);
 }
 
@@ -90,13 +120,27 @@ mingru_carry_kernel(float2 *__restrict__ folded, float *__restrict__ state, cons
   }
   float *sp = state + size_t(slots[seq]) * width + ch;
   float s = *sp;
-  int c = lo;
-  for (; c < n_chunks && chunks[4 * c + 2] == seq; ++c) {
-    const float2 f = folded[size_t(c) * width + ch];
-    folded[size_t(c) * width + ch].x = s;
-    s = f.x * s + f.y;
+  // ... and one past its last, so that the pairs of kAtOnce chunks can be asked for together (a pair at a time a sequence of 63
+  // chunks took 27 us, 10 so)
+  int end = lo, past = n_chunks;
+  while (end < past) {
+    const int mid = (end + past) >> 1;
+    if (chunks[4 * mid + 2] <= seq) end = mid + 1;
+    else past = mid;
   }
-  if (c > lo) *sp = s;
+  constexpr int kAtOnce = 8;
+  for (int c = lo; c < end; c += kAtOnce) {
+    float2 f[kAtOnce];
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i) f[i] = folded[size_t(min(c + i, end - 1)) * width + ch];
+#pragma unroll
+    for (int i = 0; i < kAtOnce; ++i)
+      if (c + i < end) {
+        folded[size_t(c + i) * width + ch].x = s;
+        s = f[i].x * s + f[i].y;
+      }
+  }
+  if (end > lo) *sp = s;
 }
 
 template <typename TO>
@@ -108,11 +152,11 @@ mingru_walk_kernel(TO *__restrict__ out, const float *__restrict__ p, const floa
   if (ch >= width) return;
   const int r0 = chunks[4 * c], n = chunks[4 * c + 1];
   float s = folded[size_t(c) * width + ch].x;
-  for (int r = r0; r < r0 + n; ++r) {
-    const Gate g = mingru_gate(p + size_t(r) * 3 * width, width, ch);
-    s = g.a * s + g.b;
-    st_f(out, size_t(r) * width + ch, s * g.silu_g);
-  }
+  if (n > 0)
+    mingru_rows<true>(p, r0, n, width, ch, [&](int r, const Gate &g) {
+      s = g.a * s + g.b;
+      st_f(out, size_t(r) * width + ch, s * g.silu_g);
+    });
 }
 
 }  // namespace
