@@ -96,41 +96,55 @@ head_product_mfma_kernel(bf16_t *__restrict__ out, int out_stride, int out_hstri
 // The same for many rows: a wave takes 16 RT rows against its 64 outputs, so that a fragment of W feeds RT products and one
 // of the rows four (above: one and four, and W came in again for every 16 rows), 64 k a stage, the next stage's
 // fragments asked for ahead of this one's products.  The same bits.
-// What bounds it: the waves in flight.  With RT 4 a wave takes 348 registers, so a SIMD holds one and a CU one block, and nothing but
-// the stage asked for ahead covers a stage's loads (82 MB in 53 us is a third of a copy's rate).  Measured, 16 heads, rows of 16, 32 and
-// 64 a wave (the first the kernel above), us: 128 to 512 numbers, 4,001 rows 79.7, 58.6, 52.8, 1,000 rows 22.8, 17.5, 15.2, 500 rows 12.7, 9.9, 8.4;
-// 512 to 128 with a gate, 4,001 rows 92.7, 59.4, 55.8, 3,000 rows 69.6, 49.9, 52.3, 1,000 rows 26.5, 19.7, 27.4, 500 rows 15.5, 17.0, 24.1.
+// What bounds it: the waves in flight (82 MB in 44 us are 0.4 of a copy's rate).  With RT 4 a stage is 32 k, so that with the next
+// one's fragments a wave stays at 208 registers and a SIMD holds two; with 64 k a stage and its loads behind branches it took 348, one
+// a SIMD.  Measured, 16 heads, rows of 16, 32 and 64 a wave (the first the kernel above), us: 128 to 512 numbers, 4,001 rows 79.7, 58.6, 43.8 (348
+// registers: 51.4), 1,000 rows 22.8, 14.3, 14.0, 500 rows 12.7, 10.5, 8.4; 512 to 128 with a gate, 4,001 rows 92.7, 59.4, 44.7 (54.8),
+// 3,000 rows 69.6, 48.9, 42.9, 2,000 rows with 32 31.3, with 64 27.3, 1,000 rows 26.5, 19.4, 27.4, 500 rows 15.5, 17.0, 24.1.
 template <bool GATED, int RT>
-__global__ void __launch_bounds__(kThreads)
+__global__ void __launch_bounds__(kThreads, 2)
 head_product_rows_kernel(bf16_t *__restrict__ out, int out_stride, int out_hstride, const bf16_t *__restrict__ in,
                          int in_stride, int in_hstride, const bf16_t *__restrict__ w, const float *__restrict__ gate,
                          int gate_stride, int n_rows, int n_in, int n_out, int gate_per_head) {
-  constexpr int kSteps = 2;                  // of 32 k a stage
+  constexpr int kSteps = RT == 4 ? 1 : 2;    // of 32 k a stage
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int a = blockIdx.y, o0 = blockIdx.z * 64, g = lane >> 4;
   const int t0 = (blockIdx.x * 4 + wave) * (16 * RT) + (lane & 15);
   if ((blockIdx.x * 4 + wave) * (16 * RT) >= n_rows) return;      // uniform over the wave; no barrier in this kernel
-  const bf16_t *xin[RT], *wa[4];
+  // Through descriptors (of the block's rows of this head, and of the head's W) rows, outputs and k past the last read as zeros on both
+  // sides without a branch, and a load's address is one register.
+  const int row0 = blockIdx.x * 4 * (16 * RT), rows_here = min(n_rows - row0, 4 * 16 * RT);
+  const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t *>(in) + size_t(row0) * in_stride + size_t(a) * in_hstride, 0,
+      (uint32_t(rows_here - 1) * uint32_t(in_stride) + uint32_t(n_in)) * 2u, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(w) + size_t(a) * n_out * n_in, 0,
+                                                                          uint32_t(n_out) * uint32_t(n_in) * 2u, 0x00020000);
+  constexpr uint32_t kOutside = 0x80000000u;
+  uint32_t x_at[RT], w_at[4];
 #pragma unroll
-  for (int i = 0; i < RT; ++i) xin[i] = in + size_t(min(t0 + 16 * i, n_rows - 1)) * in_stride + size_t(a) * in_hstride;
+  for (int i = 0; i < RT; ++i) x_at[i] = t0 + 16 * i < n_rows ? (uint32_t(t0 + 16 * i - row0) * uint32_t(in_stride) + 8u * g) * 2u : kOutside;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) wa[j] = w + (size_t(a) * n_out + min(o0 + 16 * j + (lane & 15), n_out - 1)) * n_in;
+  for (int j = 0; j < 4; ++j) {
+    const int o = o0 + 16 * j + (lane & 15);
+    w_at[j] = o < n_out ? (uint32_t(o) * uint32_t(n_in) + 8u * g) * 2u : kOutside;
+  }
   floatx4_t acc[RT][4];
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int j = 0; j < 4; ++j) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-  // (rows and outputs past the last are the last again, not stored; k past the end are zeros on both sides)
   uint4 fx[2][kSteps][RT], fw[2][kSteps][4];
   auto ask = [&](int set, int k0) {
 #pragma unroll
     for (int u = 0; u < kSteps; ++u) {
-      const int k = k0 + 32 * u + 8 * g;
-      const bool kin = k < n_in;             // n_in is a multiple of 8
+      const int k = k0 + 32 * u;
+      const bool kin = k + 8 * g < n_in;     // n_in is a multiple of 8
 #pragma unroll
-      for (int i = 0; i < RT; ++i) fx[set][u][i] = ld16(xin[i] + (kin ? k : 0), kin);
+      for (int i = 0; i < RT; ++i)
+        fx[set][u][i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_x, int(kin ? x_at[i] + 2u * k : kOutside), 0, 0));
 #pragma unroll
-      for (int j = 0; j < 4; ++j) fw[set][u][j] = ld16(wa[j] + (kin ? k : 0), kin);
+      for (int j = 0; j < 4; ++j)
+        fw[set][u][j] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, int(kin ? w_at[j] + 2u * k : kOutside), 0, 0));
     }
   };
   auto multiply = [&](int set) {
@@ -807,10 +821,11 @@ extern "C" int sb_head_product_gated_bf16(void *out, int out_stride, int out_hst
                                                                                  (const bf16_t *)in, in_stride, in_hstride,       \
                                                                                  (const bf16_t *)w, gate, gate_stride, n_rows,    \
                                                                                  n_in, n_out, gate_per_head)
-  // rows of a wave: the most (64, 32, 16) that give two blocks for every CU (a CU holds one of 64 rows a wave at a time, two of 32:
-  // see the kernel's figures; between one and two for every CU the larger is mostly ahead too, but for 3,000 rows of 512 to 128)
+  // rows of a wave: the most (64, 32, 16) that give a block for every CU (see the kernel's figures)
   const auto blocks = [&](int rows) { return (long long)((n_rows + rows - 1) / rows) * heads * out_tiles; };
-  const int rt = blocks(256) >= 2 * sb::cu_count() ? 4 : blocks(128) >= 2 * sb::cu_count() ? 2 : 1;
+  // (those kernels address a block's rows and a head's W with 32-bit byte offsets)
+  const bool reach = (long long)in_stride * 256 * 2 < (1ll << 31) && (long long)n_out * n_in * 2 < (1ll << 31);
+  const int rt = !reach ? 1 : blocks(256) >= sb::cu_count() ? 4 : blocks(128) >= sb::cu_count() ? 2 : 1;
   if (gate) {
     if (rt == 4) SB_HEAD_PRODUCT((head_product_rows_kernel<true, 4>), 256);
     else if (rt == 2) SB_HEAD_PRODUCT((head_product_rows_kernel<true, 2>), 128);
