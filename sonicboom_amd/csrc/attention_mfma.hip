@@ -23,7 +23,9 @@
 //
 // Order of summation: keys are visited in ascending order, 32 at a time, within
 // a wave; decode merges waves (pages) and then blocks (chunks of 4 pages) in
-// ascending order.  It depends on positions only, not on the batch.
+// ascending order, and where chunks are merged by a second kernel its waves take
+// every eighth each.  In prefill it depends on positions only; in decode which pages
+// are a wave's also on the rows beside it (`decode_plan`).
 #include <type_traits>
 
 #include "mfma.h"

@@ -1,6 +1,7 @@
 // bf16 matrix product for up to 128 rows against a packed matrix (decode steps and
 // short prompts: the gate/up product, the head; qkv, output and down with K cut
-// over the grid):  Y[t,n] = sum_k X[t,k] W[n,k].
+// over the grid):  Y[t,n] = sum_k X[t,k] W[n,k].  (Up to eight rows most of these
+// go on to gemm_rows.hip, whose blocks keep the rows: rows_gated, rows_plain, rows_partial.)
 //
 // Like the few-row kernel it is bound by reading W once, and every wave loads its
 // W fragments straight from global memory into MFMA operands.  With this many rows

@@ -65,7 +65,7 @@ mingru_serial_kernel(TO *__restrict__ out, const float *__restrict__ p, float *_
 }
 
 // The rows [r0, r0 + n) of a channel in order, the next kRows of them asked for ahead of these rows' arithmetic (a row at a time
-// a thread waits for memory once a row: 4,001 rows of 4,096 channels, folding 52 us and 36 so, walking 65 and WALK_NOW).
+// a thread waits for memory once a row: 4,001 rows of 4,096 channels, folding 52 us and 36 so, walking 65 and 57).
 constexpr int kRows = 4;
 template <bool OUT, typename F>
 __device__ __forceinline__ void mingru_rows(const float *__restrict__ p, int r0, int n, int width, int ch, F &&each) {
@@ -121,7 +121,7 @@ mingru_carry_kernel(float2 *__restrict__ folded, float *__restrict__ state, cons
   float *sp = state + size_t(slots[seq]) * width + ch;
   float s = *sp;
   // ... and one past its last, so that the pairs of kAtOnce chunks can be asked for together (a pair at a time a sequence of 63
-  // chunks took 27 us, 10 so)
+  // chunks took 27 us, and 10 so)
   int end = lo, past = n_chunks;
   while (end < past) {
     const int mid = (end + past) >> 1;
