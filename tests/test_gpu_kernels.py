@@ -1464,6 +1464,67 @@ def test_raw_and_plain_products_whose_blocks_keep_the_rows(rows, n, k):
     assert ((whole.cpu().double() - want).abs() <= bound).all()
 
 
+# (rows, features, k): 64- and 128-row tiles that make one round over the CUs, exactly and but for one, inner sizes of one to many
+# stages, rows and features that end inside a tile, gated widths a little over a round, and the first that leave the rule
+@pytest.mark.parametrize("rows, n, k", [(129, 2560, 2048), (400, 4608, 3584), (512, 4096, 64), (513, 4100, 192), (600, 4608, 640),
+                                        (1300, 896, 896), (1301, 3072, 128), (183, 9728, 896), (183, 17920, 320)])
+def test_tiled_products_of_one_round(rows, n, k):
+    """The launcher's own choice, plain, gated and (where it cuts K) in slices, against 64 bits."""
+    from sonicboom_amd import ops
+    x, w = randn(rows, k).to(BF16), randn(n, k, scale=0.1, seed=1).to(BF16)
+    want = (x.double() @ w.double().T)
+    bound = (x.double().abs() @ w.double().abs().T) * (k + 8) * 2.0 ** -24
+    packed = ops.pack_weight(w.to(DEV))
+    got = ops.gemm_bf16(x.to(DEV), packed, None, None, F32, packed_shape=(n, k))
+    assert ((got.cpu().double() - want).abs() <= bound).all()
+    part = ops.gemm_bf16_partial(x.to(DEV), packed, packed_shape=(n, k))
+    assert part is None or ((part.cpu().double().sum(0) - want).abs() <= bound).all()
+    half = n // 2
+    got = ops.gemm_bf16(x.to(DEV), ops.pack_weight(w.to(DEV), True), None, None, F32, gated="relu", packed_shape=(n, k)).cpu().double()
+    g, u, mg, mu = torch.relu(want[:, :half]), want[:, half:], bound[:, :half], bound[:, half:]
+    assert ((got - g * u).abs() <= (g * u).abs() * 2.0 ** -22 + 1.1 * (mg * u.abs() + mu * g) + mg * mu).all()
+
+
+# (width, groups, offset): lengths that a wave's four registers of four just hold and just do not, parts that no four divides, a row
+# off 16 bytes, groups that leave waves idle, more groups than waves
+@pytest.mark.parametrize("width, groups, offset", [(4096, 2, 0), (4104, 2, 0), (4096, 4, 0), (4112, 4, 0), (2048, 2, 4), (3072, 3, 0), (3084, 3, 0), (4095, 5, 0),
+                                                   (4100, 5, 0), (60, 5, 0), (64, 16, 0), (8, 2, 0), (90, 9, 0)])
+@pytest.mark.parametrize("out_dtype, w_dtype", [(F32, F32), (BF16, BF16), (F32, None)])
+def test_norms_in_groups(width, groups, offset, out_dtype, w_dtype):
+    """Against 64 bits: a sum in double, and four float roundings behind it (the factor's two, by the row, by the weight)."""
+    from sonicboom_amd import ops
+    rows = 5
+    w = None if w_dtype is None else (1.0 + randn(width, scale=0.1)).to(w_dtype)
+    x = torch.empty(rows * width + 4, device=DEV)[offset // 4:][:rows * width].view(rows, width).copy_(randn(rows, width, scale=3.0))
+    pick = torch.tensor([4, 0, 4], dtype=torch.int32, device=DEV)
+    f = x.cpu().double().view(rows, groups, -1)
+    want = (f / (f.square().mean(-1, keepdim=True) + 1e-6).sqrt()).view(rows, width) * (1.0 if w is None else w.double())
+    for index in (None, pick):
+        got = ops.rmsnorm(x, None if w is None else w.to(DEV), 1e-6, out_dtype, index, groups).cpu().double()
+        ref = want if index is None else want[index.cpu().long()]
+        assert ((got - ref).abs() <= ref.abs() * (2.0 ** -21 + (2.0 ** -8 if out_dtype == BF16 else 0.0))).all()
+
+
+# sequences of less than four rows and of remainders, of one chunk, of eight, of more than eight and of none of their own
+def test_gated_recurrence_in_chunks_of_every_remainder():
+    """In chunks against the walk of the same kernel's rows: the states meet through products of at most one, so both are within the
+    roundings of a sum as long as the sequence."""
+    from sonicboom_amd import ops
+    from sonicboom_amd.engine.step import row_runs
+    step = ops.mingru_chunk_rows()
+    lengths, width = [1, 3, 4, 5, step - 1, step, step + 1, 7 * step, 8 * step, 8 * step + 2, 9 * step - 3, 2], 70
+    cu = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    slots = np.arange(len(lengths), dtype=np.int32)[::-1].copy()
+    p, state = randn(int(cu[-1]), 3 * width, scale=2.0).to(DEV), randn(len(lengths), width, seed=1).to(DEV)
+    dev = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.int32).to(DEV)
+    walked, chunked = state.clone(), state.clone()
+    want = ops.mingru_scan(p, walked, dev(cu), dev(slots), len(lengths), F32)
+    got = ops.mingru_scan(p, chunked, dev(cu), dev(slots), len(lengths), F32, dev(row_runs(lengths, cu, step)))
+    # |state| stays below the largest start or candidate, about 10: some hundred rows' roundings of 2^-24 of that, decayed
+    close(chunked, walked.cpu(), atol=1e-5, rtol=1e-5, what="states")
+    close(got, want.cpu(), atol=1e-5, rtol=1e-5, what="rows")
+
+
 def test_the_norm_between_two_products_sums_in_double():
     """Rows whose squares are float numbers but whose sum of squares over the width is none, and rows of many small numbers
     beside a large one: the factor follows from the sum in double, as of every RMS norm."""
