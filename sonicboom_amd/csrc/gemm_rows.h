@@ -19,4 +19,9 @@ int rows_plain(float *y, const void *x, const void *w, int n_rows, int n_out, in
 int rows_gated(void *y, const void *x, const double *ssq, int ssq_parts, float eps, const void *w, int n_rows, int n_out, int n_in,
                int gate, void *stream);
 
+// The same from blocks that take a tile of features each and read X's fragments beside W's (gemm_skinny.hip), and where that is ahead.
+bool tile_gated_pays(int n_rows, int n_out, int n_in);
+int tile_gated(void *y, const void *x, const double *ssq, int ssq_parts, float eps, const void *w, int n_rows, int n_out, int n_in,
+               int gate, void *stream);
+
 }  // namespace sb

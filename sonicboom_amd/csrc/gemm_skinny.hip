@@ -13,6 +13,7 @@
 //
 // MFMA roles: A = 16 rows of W, B = 16 rows of X, D[n][t]; a lane then holds
 // four consecutive n of one t, a 16-byte store.
+#include "gemm_rows.h"
 #include "mfma.h"
 
 namespace {
@@ -193,11 +194,17 @@ reduce_slices_kernel(const float *__restrict__ partial, Epilogue ep, int n_slice
 // step: 10.9 us for 6.8 at 4,096 x 2,048).  What bounds it: the read of W, and where blocks are few what one CU pulls.  Measured, three rows,
 // us, weights cold, with scratch and the second kernel and so: 11,264 x 2,048 14.9 -> 12.5, 16,384 x 2,048 17.2 -> 14.2, 8,192 x 1,024 8.8 -> 5.8,
 // 4,096 x 4,096 13.6 -> 10.5, 1,024 x 2,048 6.6 -> 4.6, 9,728 x 896 (a slice, one launch there too) 7.5 -> 6.5.
-template <int S>
+// SCALED: a row's factor that follows from its sums of squares ssq [ssq_parts][n_rows] (an unfinished norm) goes into both halves;
+// they are asked for ahead of the ring and added up behind it, in the time that W's first loads take (left to the end, and by one
+// wave in four, they cost 2 us at 4,096 k).
+template <int S, bool SCALED>
 __global__ void __launch_bounds__(kThreads)
-gemm_skinny_gated_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, Epilogue ep, int n_in, int steps_per_slice) {
+gemm_skinny_gated_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict__ w, Epilogue ep, int n_in, int steps_per_slice,
+                         const double *__restrict__ ssq, int ssq_parts, float eps) {
   constexpr int kAhead = S == 1 ? 8 : S == 2 ? 4 : S == 3 ? 3 : 2;
+  constexpr int kGroups = kThreads / 8, kParts = 8;          // threads a row (of eight) that add its sums of squares; asked for ahead
   __shared__ floatx4_t chains[S * kWaves * 2 * 64];          // [slice][wave][gate, up][lane]
+  __shared__ double row_part[SCALED ? kWaves * 8 : 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, q = lane >> 4;
@@ -222,6 +229,21 @@ gemm_skinny_gated_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict_
   constexpr uint32_t kOutside = 0x80000000u;     // past a descriptor's end: reads as zeros
   const uint32_t x_off = r < ep.n_rows ? uint32_t((size_t(r) * n_in + 8 * q) * 2) : kOutside;
 
+  const int sq_row = tid & 7, sq_group = tid >> 3;
+  double parts[SCALED ? kParts : 1];
+  if constexpr (SCALED) {
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    const __amdgpu_buffer_rsrc_t rsrc_s = __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(ssq), 0,
+                                                                            uint32_t(ssq_parts) * uint32_t(ep.n_rows) * 8u, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < kParts; ++i) {
+      const uint32_t at = uint32_t(sq_group + i * kGroups) * uint32_t(ep.n_rows) + sq_row;
+      parts[i] = __builtin_bit_cast(double, __builtin_bit_cast(u32x2_t, __builtin_amdgcn_raw_buffer_load_b64(
+          rsrc_s, int(sq_row < ep.n_rows ? at * 8u : kOutside), 0, 0)));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
   uint4 rw[kAhead][S][2], rx[kAhead][S];
   const auto ask = [&](int slot, int s, int j) {             // (a step past the chain's end is zeros on both sides)
     const bool in = begin[s] + j < end[s];
@@ -236,6 +258,25 @@ gemm_skinny_gated_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict_
   for (int u = 0; u < kAhead; ++u)
 #pragma unroll
     for (int s = 0; s < S; ++s) ask(u, s, u);
+  float factor = 1.0f;
+  if constexpr (SCALED) {
+    __builtin_amdgcn_sched_barrier(0);
+    double sum = 0.0;
+#pragma unroll
+    for (int i = 0; i < kParts; ++i) sum += parts[i];
+    if (sq_row < ep.n_rows)
+      for (int p = sq_group + kParts * kGroups; p < ssq_parts; p += kGroups) sum += ssq[size_t(p) * ep.n_rows + sq_row];
+    sum += __shfl_xor(sum, 8, 64);
+    sum += __shfl_xor(sum, 16, 64);
+    sum += __shfl_xor(sum, 32, 64);
+    if (lane < 8) row_part[wave * 8 + lane] = sum;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (a barrier for what is in LDS alone: the ring stays in flight)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const int row = (tid >> 2) & 7;                          // of this thread's number of the tile
+    sum = (row_part[row] + row_part[8 + row]) + (row_part[16 + row] + row_part[24 + row]);
+    factor = 1.0f / sqrtf(float(sum / double(n_in)) + eps);
+  }
   floatx4_t acc[S][2];
 #pragma unroll
   for (int s = 0; s < S; ++s)
@@ -277,6 +318,7 @@ gemm_skinny_gated_kernel(const bf16_t *__restrict__ x, const bf16_t *__restrict_
     for (int wv = 0; wv < kWaves; ++wv) gs += at[(s * kWaves + wv) * 512], us += at[(s * kWaves + wv) * 512 + 256];
     g += gs, u += us;
   }
+  if constexpr (SCALED) g *= factor, u *= factor;
   store_out(ep, t, n, gate_act(g, ep.gated) * u);
 }
 
@@ -364,7 +406,45 @@ Plan plan_for(int n_rows, int n_out, int n_in, int gated) {
   p.n_slices = (n_steps + p.steps_per_slice - 1) / p.steps_per_slice;
   return p;
 }
+
+template <bool SCALED>
+void launch_gated(const Plan &p, const bf16_t *x, const bf16_t *w, const Epilogue &ep, int n_in, const double *ssq, int ssq_parts,
+                  float eps, hipStream_t s) {
+  switch (p.n_slices) {
+#define SB_CASE(n)                                                                                                                   \
+  case n: gemm_skinny_gated_kernel<n, SCALED><<<(ep.n_out + 15) / 16, kThreads, 0, s>>>(x, w, ep, n_in, p.steps_per_slice, ssq,      \
+                                                                                        ssq_parts, eps); break
+    SB_CASE(1); SB_CASE(2); SB_CASE(3); SB_CASE(4); SB_CASE(5); SB_CASE(6); SB_CASE(7);
+    default: SB_CASE(8);
+#undef SB_CASE
+  }
+}
 }  // namespace
+
+namespace sb {
+// A block a tile, or blocks that keep the rows (rows_gated)?  Without a staged X the first is ahead by its shorter start up to 4,096 k,
+// but for more than four rows against matrices that take long or are few tiles of long k, where X's fragments from L2 cost more than
+// that.  Scaled, us, weights cold, blocks that keep the rows and so, one and eight rows: 1,024 x 1,024 5.1 -> 4.1, 5.2 -> 4.2; 4,864 x 896
+// 7.2 -> 6.4, 7.2 -> 6.4; 8,960 x 1,536 13.7 -> 13.2, 14.2 -> 13.9; 5,632 x 2,048 11.9 -> 11.8, 11.3 and 11.6; 11,008 x 2,048 18.1 -> 17.2, 17.6
+// -> 17.2; 9,728 x 2,560 21.0 -> 20.9, 26.6 -> 21.3; 4,096 x 4,096 14.0 -> 13.8, 14.0 -> 13.3; 2,048 x 4,096 10.3 and 10.5, 10.5 and 11.3; 18,944 x
+// 3,584 45.8 -> 45.0, 43.6 and 44.2.  Not scaled: 4,864 x 896 7.3 -> 5.7, 7.4 -> 6.0; 18,944 x 1,024 15.9 -> 13.5, 16.0 -> 13.8; 8,960 x 1,536
+// 13.2 -> 12.4, 13.5 and 13.6; 11,008 x 2,048 18.0 -> 16.7, 17.4 -> 16.9; 14,336 x 4,096 40.5 -> 39.9, 40.4 and 41.9.
+bool tile_gated_pays(int n_rows, int n_out, int n_in) {
+  constexpr long long kLong = 26ll << 20;
+  return n_rows > 0 && n_rows <= kWholeRows && n_out > 0 && n_in >= 512 && n_in <= kWholeSteps * kStepK && n_in % 8 == 0 &&
+         (n_rows <= 4 || ((long long)n_out * n_in <= kLong && (n_in <= 2048 || n_out > 2048))) &&
+         gated_whole(n_rows, n_out, n_in, plan_for(n_rows, n_out, n_in, 1).n_slices, 1);
+}
+int tile_gated(void *y, const void *x, const double *ssq, int ssq_parts, float eps, const void *w, int n_rows, int n_out, int n_in,
+               int gate, void *stream) {
+  SB_REQUIRE(tile_gated_pays(n_rows, n_out, n_in), "tile_gated: sizes that it does not take");
+  const Plan p = plan_for(n_rows, n_out, n_in, 1);
+  const Epilogue ep{y, SB_BF16, nullptr, 0, nullptr, n_rows, n_out, gate};
+  if (ssq) launch_gated<true>(p, (const bf16_t *)x, (const bf16_t *)w, ep, n_in, ssq, ssq_parts, eps, (hipStream_t)stream);
+  else launch_gated<false>(p, (const bf16_t *)x, (const bf16_t *)w, ep, n_in, nullptr, 0, 0.f, (hipStream_t)stream);
+  return sb::check_launch("tile_gated");
+}
+}  // namespace sb
 
 extern "C" size_t sb_gemm_skinny_scratch(int n_rows, int n_out, int n_in, int gated) {
   if (n_rows <= 0 || n_out <= 0 || n_in <= 0) return 0;
@@ -400,13 +480,7 @@ extern "C" int sb_gemm_skinny_bf16(void *y, int y_dtype, const void *x, const vo
   float *partial = p.n_slices > 1 ? scratch : nullptr;
   const bf16_t *xb = (const bf16_t *)x, *wb = (const bf16_t *)w;
   if (gated && gated_whole(n_rows, n_out, n_in, p.n_slices, packed)) {
-    switch (p.n_slices) {
-#define SB_CASE(n) \
-  case n: gemm_skinny_gated_kernel<n><<<(n_out + 15) / 16, kThreads, 0, s>>>(xb, wb, ep, n_in, p.steps_per_slice); break
-      SB_CASE(1); SB_CASE(2); SB_CASE(3); SB_CASE(4); SB_CASE(5); SB_CASE(6); SB_CASE(7);
-      default: SB_CASE(8);
-#undef SB_CASE
-    }
+    launch_gated<false>(p, xb, wb, ep, n_in, nullptr, 0, 0.f, s);
     return sb::check_launch("sb_gemm_skinny_bf16");
   }
   if (gated && packed) launch_rt<2, true>(p.R, p.TT, xb, wb, ep, partial, n_in, p.n_slices, p.steps_per_slice, s);

@@ -15,8 +15,9 @@
 // the pass, width 896 6.2 -> 3.7 and 6.6 -> 4.0, 1,536 7.4 -> 4.6 and 7.8 -> 5.1, 2,048 8.6 -> 6.1 and 8.9 -> 6.5, 3,584
 // 11.1 -> 8.1 and 11.5 -> 8.4; the gated one against the kernel that streams weights, 9,728 x 896 7.3 -> 7.6 and 7.7 -> 7.8,
 // 17,920 x 1,536 14.3 -> 15.5 and 14.3 -> 16.2, 22,016 x 2,048 20.9 -> 21.0 and 20.8 -> 22.0, 37,888 x 3,584 52.1 -> 49.9 and
-// 51.6 -> 52.8.  With more rows the gated one falls behind by more than the other gains.  Of eight rows and fewer and sizes that
-// `rows_whole` takes, the gated product is gemm_rows.hip's by now, which holds the rows in LDS; its figures stand there.
+// 51.6 -> 52.8.  With more rows the gated one falls behind by more than the other gains.  The gated product of up to eight rows
+// goes on to gemm_skinny.hip or gemm_rows.hip where these take the sizes (gemm_rows.h); here stay less than 512 k and rows that
+// do not fit LDS.
 //
 // W is packed (16 x 32 tiles of 1 KB in fragment order, the tiles of a row block consecutive in k), so
 // a wave reads one contiguous stream, a ring of registers ahead; X's fragments come from L2 (every block
@@ -213,6 +214,8 @@ extern "C" int sb_gemm_split_gated_bf16(void *y, const void *x, const double *ss
   SB_REQUIRE(y && ssq && ssq_parts > 0, "sb_gemm_split_gated_bf16: null pointer");
   SB_SUPPORT(gate > SB_GATE_NONE && gate <= SB_GATE_RELU, "sb_gemm_split_gated_bf16: unknown gate activation %d", gate);
   if (n_rows == 0) return SB_OK;
+  if (sb::tile_gated_pays(n_rows, n_out, n_in))
+    return sb::tile_gated(y, x, ssq, ssq_parts, eps, w, n_rows, n_out, n_in, gate, stream);
   if (sb::rows_whole(n_rows, n_out, n_in, 1))          // blocks that keep the rows in LDS, where these fit
     return sb::rows_gated(y, x, ssq, ssq_parts, eps, w, n_rows, n_out, n_in, gate, stream);
   SplitArgs a{};

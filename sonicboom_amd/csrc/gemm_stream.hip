@@ -1,7 +1,7 @@
 // bf16 matrix product for up to 128 rows against a packed matrix (decode steps and
 // short prompts: the gate/up product, the head; qkv, output and down with K cut
 // over the grid):  Y[t,n] = sum_k X[t,k] W[n,k].  (Up to eight rows most of these
-// go on to gemm_rows.hip, whose blocks keep the rows: rows_gated, rows_plain, rows_partial.)
+// go on to gemm_rows.hip, whose blocks keep the rows, or gated to gemm_skinny.hip: see gemm_rows.h.)
 //
 // Like the few-row kernel it is bound by reading W once, and every wave loads its
 // W fragments straight from global memory into MFMA operands.  With this many rows
@@ -315,7 +315,9 @@ extern "C" int sb_gemm_stream_bf16(void *y, int y_dtype, const void *x, const vo
   SB_SUPPORT(gated >= SB_GATE_NONE && gated <= SB_GATE_RELU, "sb_gemm_stream_bf16: unknown gate activation %d", gated);
   const StreamArgs a{y, y_dtype, bias, bias_dtype, resid, n_rows, n_out, n_in, nullptr, 0, gated};
   const bf16_t *xb = (const bf16_t *)x, *wb = (const bf16_t *)w;
-  // up to eight rows of large matrices: blocks that keep the rows
+  // up to eight rows of large matrices: blocks that take a tile each, or that keep the rows
+  if (hint == 0 && gated && y_dtype == SB_BF16 && sb::tile_gated_pays(n_rows, n_out, n_in))
+    return sb::tile_gated(y, x, nullptr, 0, 0.f, w, n_rows, n_out, n_in, gated, stream);
   if (hint == 0 && gated && y_dtype == SB_BF16 && sb::rows_whole(n_rows, n_out, n_in, 1))
     return sb::rows_gated(y, x, nullptr, 0, 0.f, w, n_rows, n_out, n_in, gated, stream);
   if (hint == 0 && !gated && y_dtype == SB_F32 && !bias && !resid && sb::rows_whole(n_rows, n_out, n_in, 0))

@@ -1426,7 +1426,11 @@ def test_products_that_carry_the_norm_between_them(rows, width, n_in, inner, gat
 
 # (rows, features, k): a tile of one feature, features and k that fill no tile, step or round, one block a tile and many, the most
 # rows and the first that stay with the other kernels, X that just fits beside the sums in LDS and X that does not
-ROWS_IN_LDS = [(1, 17, 512), (3, 40, 2560), (8, 264, 2568), (8, 4100, 1032), (5, 12300, 520), (8, 272, 7680), (8, 272, 7688), (9, 264, 1032)]
+ROWS_IN_LDS = [(1, 17, 512), (3, 40, 2560), (8, 264, 2568), (8, 4100, 1032), (5, 12300, 520), (8, 272, 7680), (8, 272, 7688), (9, 264, 1032),
+               # as above where blocks that take a tile each stay behind: more than four rows of long products, long k
+               (8, 13700, 2056), (5, 9000, 3200), (1, 40, 4104), (4, 264, 7680),
+               # ... and where they do not: one slice of k to eight, a step a wave and remainders, many sums of squares a row
+               (4, 13700, 2056), (8, 2064, 4096), (8, 2048, 4096), (2, 3000, 4088), (7, 9000, 904), (8, 1032, 1544)]
 
 
 @pytest.mark.parametrize("rows, inner, width", ROWS_IN_LDS)
