@@ -21,11 +21,13 @@
 // 16 bytes per lane) and so do V fragments, because the cache keeps values
 // transposed ([d][key]).  No LDS is used in the main loops.
 //
-// Order of summation: keys are visited in ascending order, 32 at a time, within
-// a wave; decode merges waves (pages) and then blocks (chunks of 4 pages) in
-// ascending order, and where chunks are merged by a second kernel its waves take
-// every eighth each.  In prefill it depends on positions only; in decode which pages
-// are a wave's also on the rows beside it (`decode_plan`).
+// Order of summation: a wave visits its keys in ascending order, 32 a softmax step, or 64
+// where a page's fragments are all in its registers.  Decode merges waves (runs of pages)
+// and then blocks (chunks of a row) in ascending order, and where many chunks are merged by
+// a second kernel its waves take every eighth each.  Which pages are a wave's depends on
+// positions, in prefill also on the form that the step's sizes choose (`keys_ahead`), in
+// decode on the count of rows and the table's width, and where pages are dealt out on the
+// lengths of the rows beside (`decode_plan`).
 #include <type_traits>
 
 #include "mfma.h"
@@ -1688,19 +1690,24 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
 // 16 rows of 100 to 4,000 93.9 -> 67.8; rows of one length: 32 rows of 8,000 110.5 -> 109.3, 64 of 2,048 53.3 -> 56.4, 128 of 1,000
 // 53.2 -> 54.2, one of 131,000 57.1 -> 55.3.
 struct DecodePlan {
-  int share;        // pages of a wave at most; a chunk is four shares
+  int share;        // pages of a wave, in kShareParts of a page: whole pages would leave a third of the places empty just past one
+  int up;           // what row_chunks rounds with
   int pages0;       // of row `lane`
 };
+constexpr int kShareParts = 64;
 
 __device__ __forceinline__ int first_key(int pos, int window) { return (window > 0 && pos >= window) ? pos - window + 1 : 0; }
 // Pages that a row at `pos` sees (a row without a page of its own counts as one)
 __device__ __forceinline__ int row_pages(int pos, int window, int max_pages) {
   return max(min(pos / SB_PAGE, max_pages - 1) - first_key(pos, window) / SB_PAGE + 1, 1);
 }
-// (a last quarter of a chunk goes to the others: no chunk is smaller than half of the largest by much)
-__device__ __forceinline__ int row_chunks(int pages, int share) {
-  return max((pages + (kPagesPerChunk - 1) * share) / (kPagesPerChunk * share), 1);
+// A row's chunks: its pages over four shares, rounded as the plan says.  The row's pages are cut evenly into them, so that a chunk
+// may hold more than four shares: up to seven where one and three quarters are rounded to one.
+__device__ __forceinline__ int row_chunks(int pages, const DecodePlan &plan) {
+  return max((pages * kShareParts + plan.up) / (kPagesPerChunk * plan.share), 1);
 }
+// The same where every row of a batch comes in `cut` chunks: no more than it has fours of pages.
+__device__ __forceinline__ int cut_chunks(int pages, int cut) { return min(cut, (pages + kPagesPerChunk - 1) / kPagesPerChunk); }
 
 // The sums of v over lanes 0 .. l, in lane l: shifts inside rows of 16 lanes, then the rows' last lanes handed on.
 __device__ __forceinline__ int scan_wave(int v) {
@@ -1726,13 +1733,17 @@ __device__ __forceinline__ int max_wave(int v) {
 
 // Rows that give half of the GPU's places a block each and are of like length (the longest at most one and a half times the mean)
 // stay whole: 64 rows of 2,048 keys, 28 heads of 128 on 4, 56 us whole and 62 in two chunks.
-// fixed_share: a test's or a measurement's choice, 0: from the batch.
+// fixed_share: a test's or a measurement's choice of pages of a wave, 0: from the batch.
+// Rounding: where the batch fits a page a wave, up (a wave with a second page would take twice as long).  Else a last quarter of
+// a chunk makes one more where rows x tiles are many, as rows that stay whole then wait for the longest, and three quarters where they are
+// few: 512 chunks are what the GPU holds, and past them a block waits for a place (24 rows of 4,100 keys 58.1 and 50.9 us, 41 of 60 to 3,000,
+// 12 heads on 2, 28.2 and 24.3; 16 rows x 32 tiles of 100 to 4,000 99 and 115).
 __device__ __forceinline__ DecodePlan decode_plan(const int32_t *row_pos, int n_seqs, int tiles, int max_pages, int window,
                                                   int wave_slots, int fixed_share, int lane) {
   DecodePlan plan;
   plan.pages0 = lane < n_seqs ? row_pages(row_pos[lane], window, max_pages) : 0;
   if (fixed_share > 0) {
-    plan.share = fixed_share;
+    plan.share = fixed_share * kShareParts, plan.up = kPagesPerChunk * plan.share - 1;
     return plan;
   }
   int mine = plan.pages0, most = plan.pages0;
@@ -1742,14 +1753,18 @@ __device__ __forceinline__ DecodePlan decode_plan(const int32_t *row_pos, int n_
     most = max(most, pages);
   }
   const long long all = __builtin_amdgcn_readlane(scan_wave(mine), 63), longest = __builtin_amdgcn_readlane(max_wave(most), 63);
-  if (n_seqs * tiles * 2 * kPagesPerChunk >= wave_slots && 2 * longest * n_seqs <= 3 * all)
-    plan.share = max(int((longest + kPagesPerChunk - 1) / kPagesPerChunk), 1);
-  else
-    plan.share = max(int((all * tiles + wave_slots - 1) / wave_slots), 1);
+  const int half_places = n_seqs * tiles * 2 * kPagesPerChunk;
+  if (half_places >= wave_slots && 2 * longest * n_seqs <= 3 * all) {
+    plan.share = int(longest * kShareParts + kPagesPerChunk - 1) / kPagesPerChunk, plan.up = kPagesPerChunk * plan.share - 1;
+    return plan;
+  }
+  plan.share = max(int((all * tiles * kShareParts + wave_slots - 1) / wave_slots), kShareParts);
+  plan.up = plan.share == kShareParts ? kPagesPerChunk * plan.share - 1 : half_places <= wave_slots ? plan.share : (kPagesPerChunk - 1) * plan.share;
   return plan;
 }
 
 // Grid: a block for every chunk that there can be (decode_launch); block size 256.  Head sizes up to 128.
+// fixed_share below 0: every row in -fixed_share chunks, without a plan (like_cut).
 template <bool FUSED>
 __global__ void __launch_bounds__(256, 2)
 attn_decode_dealt_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *__restrict__ part_ml,
@@ -1768,28 +1783,35 @@ attn_decode_dealt_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, f
   const int tiles = heads_kv * head_tiles;
 
   // the block's chunk: every wave looks for it, no barrier is needed
-  const DecodePlan plan = decode_plan(row_pos, n_seqs, tiles, max_pages, window, wave_slots, fixed_share, lane);
   const int tile = int(blockIdx.x) % tiles;
-  int wanted = int(blockIdx.x) / tiles, seq = -1, chunk = 0, pages = 0;
-  for (int base = 0; base < n_seqs; base += 64) {
-    const int here = base == 0 ? plan.pages0 : base + lane < n_seqs ? row_pages(row_pos[base + lane], window, max_pages) : 0;
-    const int chunks = here > 0 ? row_chunks(here, plan.share) : 0;
-    const int upto = scan_wave(chunks);
-    const int all = __builtin_amdgcn_readlane(upto, 63);
-    if (wanted < all) {
-      const unsigned long long past = __ballot(upto > wanted);
-      const int at = __builtin_ctzll(past);
-      seq = base + at;
-      pages = __builtin_amdgcn_readlane(here, at);
-      chunk = wanted - (__builtin_amdgcn_readlane(upto, at) - __builtin_amdgcn_readlane(chunks, at));
-      break;
+  int wanted = int(blockIdx.x) / tiles, seq = -1, chunk = 0, chunks = 0, pages = 0;
+  if (fixed_share < 0) {
+    seq = wanted % n_seqs, chunk = wanted / n_seqs;
+    pages = row_pages(row_pos[seq], window, max_pages);
+    chunks = cut_chunks(pages, -fixed_share);
+    if (chunk >= chunks) seq = -1;
+  } else {
+    const DecodePlan plan = decode_plan(row_pos, n_seqs, tiles, max_pages, window, wave_slots, fixed_share, lane);
+    for (int base = 0; base < n_seqs; base += 64) {
+      const int here = base == 0 ? plan.pages0 : base + lane < n_seqs ? row_pages(row_pos[base + lane], window, max_pages) : 0;
+      const int counts = here > 0 ? row_chunks(here, plan) : 0;
+      const int upto = scan_wave(counts);
+      const int all = __builtin_amdgcn_readlane(upto, 63);
+      if (wanted < all) {
+        const unsigned long long past = __ballot(upto > wanted);
+        const int at = __builtin_ctzll(past);
+        seq = base + at;
+        pages = __builtin_amdgcn_readlane(here, at);
+        chunks = __builtin_amdgcn_readlane(counts, at);
+        chunk = wanted - (__builtin_amdgcn_readlane(upto, at) - chunks);
+        break;
+      }
+      wanted -= all;
     }
-    wanted -= all;
   }
   if (seq < 0) return;                        // uniform over the block: fewer chunks than blocks
   const int kvh = tile / head_tiles, ht = tile - kvh * head_tiles;
   const int pos = row_pos[seq];
-  const int chunks = row_chunks(pages, plan.share);
   RopeItem first;       // the folded form: see attn_decode_kernel
   if constexpr (FUSED) {
     const int n_q = group * kPerHead, n_all = n_q + (ra.store ? 2 * kPerHead : 0);
@@ -1888,11 +1910,20 @@ struct ChunkRange {
 __device__ __forceinline__ ChunkRange chunk_range(const int32_t *row_pos, int seq, int n_seqs, int tiles, int max_pages, int n_chunks,
                                                   int window, int pages_per_chunk, int wave_slots, int fixed_share, int lane) {
   const int pos = row_pos[seq];
+  if (fixed_share < 0) return ChunkRange{0, cut_chunks(row_pages(pos, window, max_pages), -fixed_share) - 1};
   if (wave_slots > 0) {
     const DecodePlan plan = decode_plan(row_pos, n_seqs, tiles, max_pages, window, wave_slots, fixed_share, lane);
-    return ChunkRange{0, row_chunks(row_pages(pos, window, max_pages), plan.share) - 1};
+    return ChunkRange{0, row_chunks(row_pages(pos, window, max_pages), plan) - 1};
   }
   return ChunkRange{first_key(pos, window) / (SB_PAGE * pages_per_chunk), min(pos / (SB_PAGE * pages_per_chunk), n_chunks - 1)};
+}
+
+// Places for partial results (rows x tiles x the table's chunks) past which the merging kernels look first how many of them hold one:
+// dealt out, most don't, and reading them in vain takes longer (32 rows of 8,200 keys, 28 heads of 128 on 4, the merge 10.7 us and
+// 5; 64 of 2,048, whole, all in all 64.3 and 60.7).
+constexpr unsigned kLookFirst = 512;
+__device__ __forceinline__ bool look_first(int rows_tiles, int n_chunks, int wave_slots, int fixed_share) {
+  return wave_slots > 0 && fixed_share >= 0 && unsigned(rows_tiles) * unsigned(min(n_chunks, 64)) > kLookFirst;
 }
 
 // Merge the chunks of a (sequence, tile), at most kAtOnce of them, in ascending order: one thread
@@ -1918,9 +1949,8 @@ attn_decode_merge_kernel(bf16_t *__restrict__ out, const float *__restrict__ par
                        threadIdx.x & 63);
   };
   ChunkRange range{0, 1};
-  // (rows that fill the GPU by themselves hardly ever come in chunks: looked at first, so that nothing is read in vain)
-  const bool look_first = wave_slots > 0 && gridDim.y * gridDim.z * 4 >= unsigned(wave_slots);
-  if (look_first) {
+  const bool looked = look_first(gridDim.y * gridDim.z, n_chunks, wave_slots, fixed_share);
+  if (looked) {
     range = range_of();
     if (range.first == range.last) return;
   }
@@ -1932,7 +1962,7 @@ attn_decode_merge_kernel(bf16_t *__restrict__ out, const float *__restrict__ par
     lv[ch] = pml[cc * 32 + 16 + c];
     ov[ch] = po[cc * (HD * 16) + min(e, HD * 16 - 1)];
   }
-  if (!look_first) range = range_of();
+  if (!looked) range = range_of();
   const int first = range.first, last = range.last;
   if (first == last) return;      // the decode kernel has written the result itself
   // rescaled to the common maximum and added in ascending chunk order
@@ -1976,10 +2006,19 @@ attn_decode_merge_many_kernel(bf16_t *__restrict__ out, const float *__restrict_
   const float *po = part_o + (tile_index * n_chunks) * (HD * 16), *pml = part_ml + (tile_index * n_chunks) * 32;
   constexpr int kAtOnce = 8;
   float mv[kAtOnce], lv[kAtOnce], ov[kAtOnce];
+  const auto range_of = [&] {
+    return chunk_range(row_pos, seq, gridDim.z, gridDim.y, max_pages, n_chunks, window, pages_per_chunk, wave_slots, fixed_share, lane);
+  };
+  ChunkRange range{0, n_chunks - 1};
+  const bool looked = look_first(gridDim.y * gridDim.z, n_chunks, wave_slots, fixed_share);
+  if (looked) {
+    range = range_of();
+    if (range.first == range.last) return;
+  }
   auto ask = [&](int base) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < kAtOnce; ++i) {
-      const size_t cc = size_t(min(base + kMergeWaves * i, n_chunks - 1));   // (past the end: the last once more, not used)
+      const size_t cc = size_t(min(base + kMergeWaves * i, range.last));   // (past the end: the last once more, not used)
       mv[i] = pml[cc * 32 + c];
       lv[i] = pml[cc * 32 + 16 + c];
       ov[i] = po[cc * (HD * 16) + e];
@@ -1987,8 +2026,7 @@ attn_decode_merge_many_kernel(bf16_t *__restrict__ out, const float *__restrict_
   };
   // the first round goes out together with the position, which says which chunks count
   ask(wave);
-  const ChunkRange range = chunk_range(row_pos, seq, gridDim.z, gridDim.y, max_pages, n_chunks, window, pages_per_chunk, wave_slots,
-                                       fixed_share, lane);
+  if (!looked) range = range_of();
   const int first = range.first, last = range.last;
   if (first == last) return;      // the decode kernel has written the result itself
   float m = -__builtin_inff(), o = 0.f, l = 0.f;
@@ -2052,6 +2090,8 @@ extern "C" int sb_attn_decode_chunks(int max_pages) {
   return (max_pages + kPagesPerChunk - 1) / kPagesPerChunk;
 }
 
+extern "C" int sb_attn_decode_cut(int n_seqs, int heads_q, int heads_kv, int max_pages);
+
 // Floats of part_o and of part_ml that sb_attn_decode_bf16 needs for these sizes.
 extern "C" size_t sb_attn_decode_part_o(int n_seqs, int heads_q, int heads_kv, int max_pages) {
   const int tiles = heads_kv * ((heads_q / heads_kv + 15) / 16);
@@ -2063,6 +2103,32 @@ extern "C" size_t sb_attn_decode_part_ml(int n_seqs, int heads_q, int heads_kv, 
 }
 
 namespace {
+
+// Rows of like length, as the caller knows: every row in so many chunks (1 to 16) that the GPU's blocks finish together, which needs no
+// look at the other rows and, in one chunk, no merging kernel.  The count with the least estimated time (MI355X, cold caches): a CU
+// streams some 27 GB/s whatever the count of its blocks, all of them 5.3 TB/s; a wave gets through a page in 3.3 us at least; a second
+// kernel costs 5 us.  The table's width is taken for the rows' length less half of the 16 pages it is rounded up by.
+// Measured with the merging kernel, us, dealt out and so (28 heads of 128 on 4): 8 rows of 4,096 keys 25.1 -> 22.7, of 8,200 36.5 -> 33.9, of 16,390
+// 60.6 -> 58.0; 16 of 4,100 39.0 -> 34.9; 32 of 8,200 115 -> 104; 48 of 2,048 55.7 -> 45.3; 64 of 2,048 60.9 -> 58.1, of 1,500 to 2,500 64.8 -> 61.8,
+// of 4,100 113 -> 103; 65 of 2,048 83.5 -> 70.7; 128 of 2,048 113 -> 108; 14 heads of 64 on 2, 128 of 2,048 35.4 -> 32.6.  Less than 32
+// rows x tiles would need more chunks than a block merges at once (3 rows of 10,000: 19.8 and 21.0).
+constexpr int kLikeFrom = 32, kMostCuts = 16;
+int like_cut(long long rows_tiles, int max_pages) {
+  const double page_us = 2.0 * SB_PAGE * HD * 2 / 27e3, pages = max_pages > 8 ? max_pages - 8 : 1;
+  const double stream_us = double(rows_tiles) * pages * page_us * 27e3 / 5.3e6;
+  int cut = 0;
+  double best = 0.0;
+  for (int c = 1; c <= kMostCuts && c <= sb_attn_decode_chunks(max_pages); ++c) {
+    const double cu_us = double((rows_tiles * c + 255) / 256) * pages / c * page_us, in_a_row = pages / c / kPagesPerChunk * 3.3 + 2.0;
+    double t = cu_us > stream_us ? cu_us : stream_us;
+    t = (t > in_a_row ? t : in_a_row) + (c > 1 ? 5.0 : 0.0);
+    if (!cut || t < best * 0.99) best = t, cut = c;
+  }
+  return cut;
+}
+
+// Whether the pages of a step's rows are dealt out: where the widest row's chunks for every row would be blocks for most of the GPU.
+bool deals(long long rows_tiles, int max_pages) { return HD <= 128 && (long long)((max_pages + 7) / 8) * rows_tiles >= kDealtFrom; }
 
 // The decode launch, for queries that are given (q) or still to be built (ra.qkv).
 int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra, const void *k_cache,
@@ -2076,16 +2142,17 @@ int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra,
   const int head_tiles = (group + 15) / 16;
   hipStream_t s = (hipStream_t)stream;
   SB_SUPPORT(heads_kv * head_tiles <= 65535, "%s: too many heads", who);
-  // A wave takes one page and asks for all of it at once (one round trip to memory).  Where the widest row's chunks for every row
-  // would be blocks for most of the GPU, the chunks are dealt out by what the rows hold.
+  // A wave takes one page and asks for all of it at once (one round trip to memory), or the chunks are dealt out by what the rows hold.
   const long long per_chunk = (long long)heads_kv * head_tiles * n_seqs;
-  // a test's or a measurement's choice (0: the launcher's own): pages of a wave
-  const bool dealt = HD <= 128 && (pages_per_wave > 1 || (pages_per_wave == 0 && (long long)((max_pages + 7) / 8) * per_chunk >= kDealtFrom));
+  // pages_per_wave: a test's or a measurement's choice of pages of a wave, 0 the launcher's own, -1 too, with rows of like length
+  const bool dealt = HD <= 128 && (pages_per_wave > 1 || (pages_per_wave <= 0 && deals(per_chunk, max_pages)));
+  const int cut = pages_per_wave < 0 ? sb_attn_decode_cut(n_seqs, heads_q, heads_kv, max_pages) : 0;
+  const int fixed_share = cut ? -cut : pages_per_wave > 0 ? pages_per_wave : 0;
   // five to eight pages a row: a block of eight waves takes a row whole (with more rows than half the CUs the chunks fill the GPU as it is)
-  const bool whole_rows = kWholeRows && !dealt && pages_per_wave == 0 && max_pages > kPagesPerChunk && max_pages <= kWholePages &&
+  const bool whole_rows = kWholeRows && !dealt && pages_per_wave <= 0 && max_pages > kPagesPerChunk && max_pages <= kWholePages &&
                           per_chunk <= 128;
   const int pages_per_chunk = whole_rows ? kWholePages : kPagesPerChunk;
-  const int n_chunks = (max_pages + pages_per_chunk - 1) / pages_per_chunk;
+  const int n_chunks = cut ? cut : (max_pages + pages_per_chunk - 1) / pages_per_chunk;
   SB_SUPPORT((long long)n_chunks * per_chunk <= 0x7fffffffLL, "%s: too many blocks", who);
   const unsigned grid = unsigned((long long)n_chunks * per_chunk);
 #define SB_ARGS                                                                                           \
@@ -2098,12 +2165,12 @@ int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra,
     }
   } else if (dealt) {
     // a chunk for every row and tile, and as many as the waves' shares fill; no more than there are
-    const long long most = per_chunk + (pages_per_wave > 1 ? per_chunk * n_chunks : kWaveSlots / kPagesPerChunk);
+    const long long most = per_chunk + (fixed_share ? per_chunk * n_chunks : kWaveSlots / kPagesPerChunk);
     const unsigned blocks = unsigned(most < (long long)grid ? most : (long long)grid);
     // (only head sizes up to 128 get here, and only they hold this kernel)
     if constexpr (HD <= 128) {
-      if (fused) attn_decode_dealt_kernel<true><<<blocks, 256, 0, s>>>(SB_ARGS, n_seqs, kWaveSlots, pages_per_wave);
-      else attn_decode_dealt_kernel<false><<<blocks, 256, 0, s>>>(SB_ARGS, n_seqs, kWaveSlots, pages_per_wave);
+      if (fused) attn_decode_dealt_kernel<true><<<blocks, 256, 0, s>>>(SB_ARGS, n_seqs, kWaveSlots, fixed_share);
+      else attn_decode_dealt_kernel<false><<<blocks, 256, 0, s>>>(SB_ARGS, n_seqs, kWaveSlots, fixed_share);
     }
   } else {
     if (fused) attn_decode_kernel<true, 4><<<grid, 256, 0, s>>>(SB_ARGS, n_seqs);
@@ -2115,19 +2182,28 @@ int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra,
   const int elements = (group < 16 ? group : 16) * HD;      // of a tile: its columns that have a head
   if (n_chunks <= 16)
     attn_decode_merge_kernel<<<dim3((elements + 255) / 256, heads_kv * head_tiles, n_seqs), 256, 0, s>>>(
-        (bf16_t *)out, part_o, part_ml, row_pos, heads_q, heads_kv, n_chunks, window, pages_per_chunk, max_pages, dealt ? kWaveSlots : 0, pages_per_wave);
+        (bf16_t *)out, part_o, part_ml, row_pos, heads_q, heads_kv, n_chunks, window, pages_per_chunk, max_pages, dealt ? kWaveSlots : 0, fixed_share);
   else
     attn_decode_merge_many_kernel<<<dim3((elements + 63) / 64, heads_kv * head_tiles, n_seqs), 64 * kMergeWaves, 0, s>>>(
-        (bf16_t *)out, part_o, part_ml, row_pos, heads_q, heads_kv, n_chunks, window, pages_per_chunk, max_pages, dealt ? kWaveSlots : 0, pages_per_wave);
+        (bf16_t *)out, part_o, part_ml, row_pos, heads_q, heads_kv, n_chunks, window, pages_per_chunk, max_pages, dealt ? kWaveSlots : 0, fixed_share);
   return sb::check_launch(who);
 }
 
 }  // namespace
 
+// Chunks that every row of a step comes in when its rows are said to be of like length (pages_per_wave -1 below), 0 where the word
+// makes no difference.
+extern "C" int sb_attn_decode_cut(int n_seqs, int heads_q, int heads_kv, int max_pages) {
+  if (n_seqs <= 0 || heads_kv <= 0 || heads_q % heads_kv || max_pages <= 0) return 0;
+  const long long rows_tiles = (long long)n_seqs * heads_kv * ((heads_q / heads_kv + 15) / 16);
+  return deals(rows_tiles, max_pages) && rows_tiles >= kLikeFrom ? like_cut(rows_tiles, max_pages) : 0;
+}
+
 // q, out: bf16 [n_seqs, heads_q * HD], one row per sequence; k_cache bf16 [pages][heads_kv][64][HD],
 // v_cache bf16 [pages][heads_kv][HD][64].  part_o / part_ml: float buffers of the sizes the two
-// functions above give (may be NULL when max_pages fits one chunk).  pages_per_wave: 0, or a
-// test's or a measurement's choice of how many pages in a row a wave takes.
+// functions above give (may be NULL when max_pages fits one chunk).  pages_per_wave: 0; -1 where the rows are known to be of like
+// length (the longest at most one and a half times the mean; wrong results do not follow from a wrong word, only time lost); or a
+// test's or a measurement's choice of how many pages in a row a wave takes at most.
 extern "C" int sb_attn_decode_bf16(void *out, const void *q, const void *k_cache, const void *v_cache,
                                    const int32_t *page_table, int max_pages, int n_pages_total,
                                    const int32_t *row_pos, float *part_o, float *part_ml, int n_seqs,

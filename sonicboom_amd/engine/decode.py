@@ -6,7 +6,8 @@ therefore keeps the step's bookkeeping (token ids, positions, page tables) in
 fixed device buffers, runs the step once or twice kernel by kernel, then
 captures exactly the same launches into a HIP graph per (batch size, page
 table width) and replays it, refreshing the buffers with one small copy per
-step.  Graph and kernel-by-kernel steps run the same kernels on the same
+step (a step whose sequences are of like length and which gains by the word is a
+recording of its own).  Graph and kernel-by-kernel steps run the same kernels on the same
 shapes, so they give the same bits; the graph is only a way of launching.
 Nothing in the graph clears memory with a memset node.
 
@@ -71,6 +72,8 @@ class _StaticContext(_Context):
         self.dev = torch.zeros(layout.total, dtype=torch.int32, device=dev)
         self.next_ids = torch.zeros(batch, dtype=torch.int32, device=dev)
         layout.bind(self, self.dev)
+        mixers = [m for b in engine.model.blocks if hasattr(m := getattr(b, "mixer", None), "alike_pays")]
+        self.alike_pays = any(m.alike_pays(batch, width) for m in mixers)
         # the parts that never change for a decode step of this batch size: a row a sequence,
         # every row wanted, and whatever the height a run is that one row
         ar = np.arange(batch, dtype=np.int32)
@@ -107,6 +110,7 @@ class _StaticContext(_Context):
             table[:live] = cache.page_table(g, slots, min_width=self.width)
             table[live:] = -1
         self.max_len_after = int(lengths.max()) + 1
+        self.alike = self.alike_pays and ops.rows_alike([int(n) + 1 for n in lengths[:live]])
         # the host's view of the step, as StepContext has it
         self.slot_list = list(slots) + [slots[0]] * (self.batch - live)
         self.lengths_before = lengths.tolist()
@@ -129,7 +133,7 @@ class DecodeLoop:
         # added rows would run a mixer's per-sequence state of some live slot: no padding then
         self.pad_batches = not engine.cache.state
         self._ctx: Dict[Tuple[int, int], _StaticContext] = {}
-        self._graphs: Dict[tuple, Tuple[torch.cuda.CUDAGraph, torch.Tensor]] = {}    # (batch, width, choice)
+        self._graphs: Dict[tuple, Tuple[torch.cuda.CUDAGraph, torch.Tensor]] = {}    # (batch, width, choice, alike)
         self._uses: Dict[tuple, int] = {}
         self._recorded = False
         self.slots: List[int] = []
@@ -192,7 +196,7 @@ class DecodeLoop:
                 self._forget(next(iter(self._ctx)))      # its pinned buffers and its recordings
         self._ctx[key] = ctx                             # most recently used last
         ctx.refresh(cache, self.slots, tokens)
-        gkey = (*key, choose)
+        gkey = (*key, choose, ctx.alike)
         entry = self._graphs.pop(gkey, None)
         if entry is not None:
             self._graphs[gkey] = entry          # most recently used last

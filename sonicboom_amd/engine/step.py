@@ -16,6 +16,7 @@ from typing import Optional, Sequence
 import numpy as np
 import torch
 
+from .. import ops
 from ..cache.paged import PAGE, CacheError, PagedCache
 from . import dense
 from .model import DecoderModel
@@ -124,6 +125,7 @@ class _Context:
     """What the parts read of a step's bookkeeping (see :class:`StepContext`)."""
 
     trace = None            # set by the engine while a tracer listens
+    alike = False           # one token a sequence, of sequences of like length (``ops.rows_alike``)
     shared = None           # a step's own scratch: what a part leaves for a later part of the same step
 
     def page_table(self, group: int) -> torch.Tensor:
@@ -161,6 +163,7 @@ class StepContext(_Context):
         self.lengths_before = [cache.length(s) for s in self.slot_list]
         self.n_rows = sum(self.n_new)
         self.is_decode = all(n == 1 for n in self.n_new)
+        self.alike = self.is_decode and ops.rows_alike([n + 1 for n in self.lengths_before])
         self.max_new = max(self.n_new)
         self.max_len_after = max(l + n for l, n in zip(self.lengths_before, self.n_new))
         cu = np.zeros(self.n_seqs + 1, dtype=np.int32)

@@ -14,7 +14,7 @@ import ctypes
 import math
 import threading
 
-from typing import Optional
+from typing import Optional, Sequence
 
 import torch
 
@@ -960,9 +960,10 @@ def attention_mfma_ok(q_dtype, cache_dtype, head_dim: int) -> bool:
             and 16 <= head_dim <= MFMA_MAX_HEAD_DIM)
 
 
-def attention_decode_mfma(q, k_cache, v_cache, page_table, seq_pos, heads_q, heads_kv, head_dim, scale, window):
+def attention_decode_mfma(q, k_cache, v_cache, page_table, seq_pos, heads_q, heads_kv, head_dim, scale, window, alike=False):
     """One bf16 query row per sequence (row i belongs to row i of ``page_table``) at position
-    ``seq_pos[i]``, over the cache; keys are split over blocks and merged in ascending order."""
+    ``seq_pos[i]``, over the cache; keys are split over blocks and merged in ascending order.
+    ``alike``: the caller knows the rows to be of like length (:func:`rows_alike`), and the kernel need not look."""
     _dev(q, k_cache, v_cache, page_table, seq_pos)
     n = q.shape[0]
     if q.dim() != 2 or q.shape[1] != heads_q * head_dim or q.dtype != torch.bfloat16:
@@ -983,7 +984,7 @@ def attention_decode_mfma(q, k_cache, v_cache, page_table, seq_pos, heads_q, hea
                               device=q.device)
     check(lib.sb_attn_decode_bf16(_p(out), _p(q), _p(k_cache), _p(v_cache), _p(page_table), max_pages,
                                   k_cache.shape[0], _p(seq_pos), _p(part_o), _p(part_ml), n, heads_q,
-                                  heads_kv, float(scale), int(window), _hints.decode_pages, _stream()),
+                                  heads_kv, float(scale), int(window), _hints.decode_pages or -int(alike), _stream()),
           lib, "sb_attn_last_error")
     return out
 
@@ -1001,13 +1002,13 @@ def attention_decode_rope_ok(qkv: torch.Tensor, q_dtype, cache_dtype, heads_q: i
 def attention_decode_rope(qkv: torch.Tensor, inv_freq: Optional[torch.Tensor], freq_factors: Optional[torch.Tensor],
                           rot_dims: int, k_cache: torch.Tensor, v_cache: torch.Tensor, page_table: torch.Tensor,
                           seq_pos: torch.Tensor, heads_q: int, heads_kv: int, head_dim: int, scale: float, window: int,
-                          bias: Optional[torch.Tensor] = None, store: bool = True) -> torch.Tensor:
+                          bias: Optional[torch.Tensor] = None, store: bool = True, alike: bool = False) -> torch.Tensor:
     """A decode step's rotation, store and attention in one kernel: ``qkv`` float32 [n, width] or
     [slices, n, width] (partial sums of the projection, added in ascending order, then ``bias``),
     one row per sequence at position ``seq_pos[i]``.  Queries and keys are rotated as
     :func:`rope_kv_store` rotates them, the row's key and value go into the cache (``store``), and the
-    row attends over its sequence's keys, its own among them.  Returns the attention output in
-    bfloat16 [n, heads_q * head_dim]: the bits of the two kernels one after the other."""
+    row attends over its sequence's keys, its own among them.  ``alike``: as in :func:`attention_decode_mfma`.  Returns the
+    attention output in bfloat16 [n, heads_q * head_dim]: the bits of the two kernels one after the other."""
     _dev(qkv, inv_freq, freq_factors, k_cache, v_cache, page_table, seq_pos, bias)
     n_slices = 1
     if qkv.dim() == 3:
@@ -1044,15 +1045,26 @@ def attention_decode_rope(qkv: torch.Tensor, inv_freq: Optional[torch.Tensor], f
                                        _p(freq_factors), int(rot_dims) if inv_freq is not None else 0,
                                        1 if store else 0, _p(k_cache), _p(v_cache), _p(page_table), max_pages,
                                        k_cache.shape[0], _p(seq_pos), _p(part_o), _p(part_ml), n, heads_q, heads_kv,
-                                       float(scale), int(window), _hints.decode_pages, _stream()),
+                                       float(scale), int(window), _hints.decode_pages or -int(alike), _stream()),
           lib, "sb_attn_last_error")
     return out
 
 
+def attention_decode_alike_pays(rows: int, heads_q: int, heads_kv: int, head_dim: int, pages: int) -> bool:
+    """Whether a decode step of ``rows`` rows and page tables of ``pages`` runs otherwise when its rows are said to be alike."""
+    return library.attention_library(head_dim).sb_attn_decode_cut(rows, heads_q, heads_kv, pages) > 0
+
+
+def rows_alike(lengths: Sequence[int]) -> bool:
+    """Whether sequences of these lengths are of like length, as the decode attention takes the word: the longest at most one and
+    a half times the mean."""
+    return 2 * max(lengths) * len(lengths) <= 3 * sum(lengths)
+
+
 @contextlib.contextmanager
 def attention_decode_pages_per_wave(head_dim: int, pages: int):
-    """For tests and measurements: inside the block this thread's decode attention gives every
-    wave ``pages`` pages (1, 2, 4 or 8; more than one only up to head size 128) instead of
+    """For tests and measurements: inside the block this thread's decode attention gives a wave up to
+    ``pages`` pages (1, 2, 4 or 8; more than one only up to head size 128) instead of
     choosing from the sizes; 0: the launcher's choice."""
     before = _hints.decode_pages
     _hints.decode_pages = int(pages)
@@ -1165,7 +1177,7 @@ def attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pag
     if fast and attention_mfma_ok(q.dtype, k_cache.dtype, head_dim):
         if ctx.is_decode:
             return attention_decode_mfma(q, k_cache, v_cache, page_table, ctx.row_pos, heads_q, heads_kv,
-                                         head_dim, scale, window)
+                                         head_dim, scale, window, alike=getattr(ctx, "alike", False))
         height = attention_tile_height(ctx, heads_q, heads_kv, row_tile)
         return attention_prefill_mfma(q, k_cache, v_cache, page_table, ctx.row_pos, ctx.row_tiles(height),
                                       heads_q, heads_kv, head_dim, scale, window, tile_rows=height,

@@ -162,6 +162,7 @@ _ATTN_SIGNATURES = {
                                  _I, _I, _P],
     "sb_attn_decode_rope_ok": [_I, _I, _I, _I],
     "sb_attn_decode_chunks": [_I],
+    "sb_attn_decode_cut": [_I, _I, _I, _I],
     "sb_attn_head_dim": [],
 }
 

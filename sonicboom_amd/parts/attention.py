@@ -227,6 +227,13 @@ class Attention(Mixer):
             return self._attend_rotating(None, ctx, binding, rows)
         return self._attend_extended(None, ctx, binding, rows)
 
+    def alike_pays(self, rows: int, pages: int) -> bool:
+        """Whether a decode step of these sizes runs otherwise when its sequences are of like length."""
+        rt = self.rt
+        return self.plain_scores and (not self.extended or self.row_norm) and rt.fast_kernels \
+            and ops.attention_mfma_ok(rt.act_dtype, rt.cache_dtype, self.head_dim) \
+            and ops.attention_decode_alike_pays(rows, self.heads_q, self.heads_kv, self.head_dim, pages)
+
     def takes_slices(self, ctx) -> bool:
         """Whether from_rows() adds a product's K slices itself."""
         return self.head_norm_path or self.row_norm
@@ -361,7 +368,8 @@ class Attention(Mixer):
             # one token per sequence: rotation, store and attention in one kernel
             return ops.attention_decode_rope(qkv, inv_freq, freq_factors, rot_dims, binding.k_cache, binding.v_cache,
                                              page_table, ctx.row_pos, self.heads_q, self.heads_kv, self.head_dim,
-                                             self.scale, self.window, bias=bias, store=writes)
+                                             self.scale, self.window, bias=bias, store=writes,
+                                             alike=getattr(ctx, "alike", False))
         q = ops.rope_kv_store(
             qkv, rt.act_dtype, inv_freq, freq_factors, rot_dims, ctx.row_pos, ctx.row_seq,
             binding.k_cache if writes else None, binding.v_cache if writes else None,

@@ -1609,7 +1609,7 @@ FOLDED_SHAPES = [(4, 2, 16, 16), (3, 1, 32, 32), (5, 5, 48, 16), (6, 2, 80, 64),
                  (2, 1, 256, 256)]
 
 
-def folded_against_two_kernels(hq, hkv, hd, rot, window, pages, lens):
+def folded_against_two_kernels(hq, hkv, hd, rot, window, pages, lens, alike=False):
     from sonicboom_amd import ops
     n_seq = len(lens)
     width_pages = max((n + 63) // 64 for n in lens)
@@ -1640,12 +1640,12 @@ def folded_against_two_kernels(hq, hkv, hd, rot, window, pages, lens):
         q = ops.rope_kv_store(arg, BF16, inv, ff, rot, pos.to(DEV), seq.to(DEV), kc1, vc1, table.to(DEV), hq, hkv, hd,
                               bias=bias)
         with ops.attention_decode_pages_per_wave(hd, pages):
-            want = ops.attention_decode_mfma(q, kc1, vc1, table.to(DEV), pos.to(DEV), hq, hkv, hd, scale, window)
+            want = ops.attention_decode_mfma(q, kc1, vc1, table.to(DEV), pos.to(DEV), hq, hkv, hd, scale, window, alike=alike)
             # one kernel
             kc2, vc2 = kc0.clone().to(DEV), vc0.clone().to(DEV)
             assert ops.attention_decode_rope_ok(arg, BF16, BF16, hq, hkv, hd, rot)
             got = ops.attention_decode_rope(arg, inv, ff, rot, kc2, vc2, table.to(DEV), pos.to(DEV), hq, hkv, hd, scale,
-                                            window, bias=bias)
+                                            window, bias=bias, alike=alike)
             assert torch.equal(got.view(torch.int16), want.view(torch.int16)), f"slices {n_slices}"
             assert torch.equal(kc2.view(torch.int16), kc1.view(torch.int16))
             assert torch.equal(vc2.view(torch.int16), vc1.view(torch.int16))
@@ -1654,7 +1654,7 @@ def folded_against_two_kernels(hq, hkv, hd, rot, window, pages, lens):
             kc3, vc3 = kc1.clone(), vc1.clone()
             only_q = arg[..., : hq * hd].contiguous()
             got = ops.attention_decode_rope(only_q, inv, ff, rot, kc3, vc3, table.to(DEV), pos.to(DEV), hq, hkv, hd,
-                                            scale, window, bias=bias, store=False)
+                                            scale, window, bias=bias, store=False, alike=alike)
             assert torch.equal(got.view(torch.int16), want.view(torch.int16))
             assert torch.equal(kc3.view(torch.int16), kc1.view(torch.int16))
     assert not ops.attention_decode_rope_ok(arg, BF16, BF16, 34, 2, hd, rot)          # 17 heads per kv head
@@ -1689,11 +1689,38 @@ DEALT = [(4, 2, 16, [1 + 31 * i % 2100 for i in range(130)]), (20, 1, 64, [64 * 
          (8, 8, 48, [30 + i for i in range(33)])]
 
 
+def attention_64(q, k, v, seen, scale):
+    """Rows q [n, heads, d] over keys k and values v [m, kv heads, d] in 64 bits, `seen` bool [n, m]: the weights [heads, n, m], the results
+    [n, heads, d], and how far a kernel may be off them.  It rounds every weight to bfloat16, by up to 2^-9 of it and so by 0.58 of that
+    in the root mean square: 2^-7 sqrt(sum p^2 v^2) is seven times what these roundings add up to.  The result is rounded once more."""
+    group = q.shape[1] // k.shape[1]
+    k, v = (t.double().repeat_interleave(group, 1).transpose(0, 1) for t in (k, v))
+    s = q.double().transpose(0, 1) @ k.transpose(1, 2) * scale
+    p = torch.softmax(s.masked_fill(~seen, -math.inf), -1).nan_to_num(0.0)
+    out, spread = p @ v, ((p * p) @ (v * v)).sqrt()
+    return p, out.transpose(0, 1), (2.0 ** -7 * spread + 2.0 ** -8 * out.abs() + 1e-6).transpose(0, 1)
+
+
+def a_page_left_out_shows(p, v, out, slack, hq):
+    """Whether every page of which a row (n = 1) sees half or more would be missed: results without it lie outside of what two kernels within
+    the slack can differ by."""
+    v = v.double().repeat_interleave(hq // v.shape[1], 1)
+    for lo in range(0, p.shape[2], 64):
+        w = p[:, :, lo:lo + 64]
+        if int((w[0] > 0).sum()) < 32 or float(w.sum(-1).max()) > 1 - 1e-9:
+            continue
+        without = (out - (w @ v[lo:lo + 64].transpose(0, 1)).transpose(0, 1)) / (1 - w.sum(-1)).T[:, :, None]
+        if not ((without - out).abs() > 2 * slack).any():
+            return False
+    return True
+
+
 @pytest.mark.parametrize("hq, hkv, hd, lens", DEALT, ids=lambda v: f"{len(v)}rows" if isinstance(v, list) else str(v))
 @pytest.mark.parametrize("window", [0, 70, 1000])
 def test_attention_decode_deals_pages_out(hq, hkv, hd, lens, window):
-    """Many rows of unequal length, whose pages the kernel deals out to its blocks, against blocks of four pages of a row each: the
-    same sums of float32 numbers in another order, then one rounding to bfloat16.  Every ninth row has no page."""
+    """Many rows of unequal length, whose pages the kernel deals out to its blocks or, told that they are alike, cuts into as many chunks
+    each: against 64 bits, and against blocks of four pages of a row each, the same sums of float32 numbers in another order, then one
+    rounding to bfloat16.  Every ninth row has no page."""
     from sonicboom_amd import ops
     width = max(-(-n // 64) for n in lens)
     assert -(-width // 8) * len(lens) * hkv * -(-(hq // hkv) // 16) >= 256
@@ -1709,7 +1736,7 @@ def test_attention_decode_deals_pages_out(hq, hkv, hd, lens, window):
             table[i] = -1
     kc, vc = (randn(*shape, seed=2).to(BF16).to(DEV) for shape in ((n_pages, hkv, 64, hd), (n_pages, hkv, hd, 64)))
     q, pos = randn(len(lens), hq * hd, seed=3).to(BF16).to(DEV), torch.tensor([n - 1 for n in lens], dtype=torch.int32).to(DEV)
-    run = lambda: ops.attention_decode_mfma(q, kc, vc, table.to(DEV), pos, hq, hkv, hd, hd ** -0.5, window).float()
+    run = lambda **how: ops.attention_decode_mfma(q, kc, vc, table.to(DEV), pos, hq, hkv, hd, hd ** -0.5, window, **how).float()
     got, again = run(), run()
     with ops.attention_decode_pages_per_wave(hd, 1):
         want = run()
@@ -1718,6 +1745,44 @@ def test_attention_decode_deals_pages_out(hq, hkv, hd, lens, window):
     # probabilities are rounded to bfloat16 (2^-9 of each) relative to another maximum, as keys meet in other steps: the sums' part
     # in that is at most 2^-8 of the values' largest, and half of one rounding of each result
     assert ((got - want).abs() <= 2.0 ** -8 * vc.float().abs().max() * 0.5 + want.abs() * 2.0 ** -8).all()
+    assert ops.attention_decode_alike_pays(len(lens), hq, hkv, hd, width)
+    alike = run(alike=True)
+    k_all, v_all = layout.keys_in_order(kc.cpu()), layout.values_in_order(vc.cpu())
+    longest = max((i for i in range(len(lens)) if i % 9 != 5), key=lambda i: lens[i])
+    for i, n in enumerate(lens):
+        if i % 9 == 5:
+            assert (alike[i] == 0).all()
+            continue
+        own = table[i, :-(-n // 64)].long().clamp(min=0)     # (pages behind the window: whatever is there, not seen)
+        k = k_all[own].permute(0, 2, 1, 3).reshape(-1, hkv, hd)[:n]
+        v = v_all[own].permute(0, 3, 1, 2).reshape(-1, hkv, hd)[:n]
+        seen = (torch.arange(n) > n - 1 - window) if window else torch.ones(n, dtype=torch.bool)
+        p, ref, slack = attention_64(q[i:i + 1].cpu().view(1, hq, hd), k, v, seen[None, :], hd ** -0.5)
+        for name, out in (("dealt out", got), ("alike", alike)):
+            off = (out[i].cpu().double().view(1, hq, hd) - ref).abs()
+            assert (off <= slack).all(), f"{name}, row {i} of {n} keys: off by {off.max():.3g}, {(off / slack).max():.3g} of the slack"
+        if i == longest:
+            assert a_page_left_out_shows(p, v, ref, slack, hq)
+
+
+# (heads, kv heads, head size, rotary width): more rows than a wave looks at at once, of lengths from one key on
+@pytest.mark.parametrize("hq, hkv, hd, rot, lens", [(14, 2, 64, 64, [1 + 37 * i % 1500 for i in range(130)]), (28, 4, 128, 128, [60 + 131 * i % 1400 for i in range(70)]),
+                                                    (16, 1, 128, 64, [30 + 211 * i % 6000 for i in range(65)]), (8, 8, 80, 0, [64 * (1 + 5 * i % 40) for i in range(20)])],
+                         ids=lambda v: f"{len(v)}rows" if isinstance(v, list) else str(v))
+@pytest.mark.parametrize("window, alike", [(0, False), (0, True), (300, False), (300, True)])
+def test_attention_decode_folded_in_where_pages_are_dealt_out(hq, hkv, hd, rot, lens, window, alike):
+    assert -(-max(lens) // 64 // 8) * len(lens) * hkv >= 256
+    folded_against_two_kernels(hq, hkv, hd, rot, window, 0, lens, alike)
+
+
+def test_attention_decode_of_like_rows_needs_no_second_kernel():
+    """Where rows of like length fill the GPU by themselves every row is one chunk, and chunks a row grow as rows get fewer."""
+    from sonicboom_amd.ops import library
+    cut = library.attention_library(128).sb_attn_decode_cut
+    assert [cut(n, 28, 4, 48) for n in (48, 64, 128)] == [1, 1, 1]
+    assert 1 < cut(16, 28, 4, 80) <= cut(8, 28, 4, 144) <= 16
+    assert cut(2, 28, 4, 512) == 0 and cut(64, 28, 4, 4) == 1 and cut(8, 28, 4, 8) == 0        # few rows, short tables: the word is not heard
+    assert library.attention_library(256).sb_attn_decode_cut(64, 28, 4, 48) == 0
 
 
 @pytest.mark.parametrize("vocab", [5, 256, 1000, 152064])
