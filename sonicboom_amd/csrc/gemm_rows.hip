@@ -211,18 +211,25 @@ bool reach(int n_rows, int n_out, int n_in) {
 // eight), eight where it has more (4,096 k: 40.4 and 39.0 of 14,336 pairs, 3,072: 20.0 and 19.5 of 8,192).
 constexpr int kFewSteps = 80;
 
+// LDS of a block besides X's share: where the waves' sums meet, and the parts of the rows' sums of squares.
+constexpr size_t own_bytes(bool gated, int w) {
+  return sizeof(floatx4_t) * 2 * w * (gated ? 2 : 1) * 64 + sizeof(double) * (gated ? 64 * w : 1);
+}
+
 template <bool GATED, int W, int BATCH>
-void launch(const void *x, const void *w, RowsArgs a, int blocks, int slices, hipStream_t s) {
+int launch(const char *who, const void *x, const void *w, RowsArgs a, int blocks, int slices, hipStream_t s) {
   a.rounds = rounds_of(a.steps_per_slice, W);
   const size_t lds = x_bytes(a.n_rows, a.steps_per_slice, W);
   const auto kern = gemm_rows_kernel<GATED, W, BATCH>;
-  static bool raised = false;      // once per instantiation: allow more than the default dynamic LDS
-  if (lds > 48 * 1024 && !raised) {
-    (void)hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(kLds - sizeof(floatx4_t) * 2 * W * (GATED ? 2 : 1) * 64 -
-                                                                                                    (GATED ? 64 * W * sizeof(double) : sizeof(double))));
+  constexpr int kMost = int(kLds - own_bytes(GATED, W));
+  static bool raised = false;      // once per instantiation: X's share and the block's own LDS may be more than the default allows
+  if (!raised) {
+    const hipError_t e = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, kMost);
+    SB_REQUIRE(e == hipSuccess, "%s: cannot reserve %d bytes of LDS: %s", who, kMost, hipGetErrorString(e));
     raised = true;
   }
   kern<<<dim3(blocks, slices), 64 * W, lds, s>>>((const bf16_t *)x, (const bf16_t *)w, a);
+  return sb::check_launch(who);
 }
 
 // K cut over the grid: slices, and blocks that each slice's tiles are dealt out to.
@@ -273,9 +280,8 @@ int rows_partial(float *partial, const void *x, const void *w, int n_rows, int n
   SB_REQUIRE(c.slices > 0 && reach(n_rows, n_out, n_in), "rows_partial: sizes that it does not take");
   RowsArgs a{};
   a.n_rows = n_rows, a.n_out = n_out, a.n_in = n_in, a.steps_per_slice = c.steps_per_slice, a.y = partial;
-  if (n_rows <= 4) launch<false, 8, 2>(x, w, a, c.blocks, c.slices, (hipStream_t)stream);
-  else launch<false, 8, 4>(x, w, a, c.blocks, c.slices, (hipStream_t)stream);
-  return sb::check_launch("rows_partial");
+  return n_rows <= 4 ? launch<false, 8, 2>("rows_partial", x, w, a, c.blocks, c.slices, (hipStream_t)stream)
+                     : launch<false, 8, 4>("rows_partial", x, w, a, c.blocks, c.slices, (hipStream_t)stream);
 }
 
 // (Gated ones from 512 k: 9,001 pairs of 40 k 4.5 us in the kernel whose waves split the features and 6.0 here.)
@@ -293,9 +299,8 @@ int rows_gated(void *y, const void *x, const double *ssq, int ssq_parts, float e
   a.n_rows = n_rows, a.n_out = n_out, a.n_in = n_in, a.steps_per_slice = (n_in + 31) / 32;
   a.ssq = ssq, a.ssq_parts = ssq_parts, a.eps = eps, a.gate = gate, a.y = y;
   const int tiles = (n_out + kTile - 1) / kTile, n_cu = sb::cu_count();
-  if (a.steps_per_slice <= kFewSteps) launch<true, 4, 8>(x, w, a, tiles < 3 * n_cu ? tiles : 3 * n_cu, 1, (hipStream_t)stream);
-  else launch<true, 8, 8>(x, w, a, tiles < n_cu ? tiles : n_cu, 1, (hipStream_t)stream);
-  return sb::check_launch("rows_gated");
+  return a.steps_per_slice <= kFewSteps ? launch<true, 4, 8>("rows_gated", x, w, a, tiles < 3 * n_cu ? tiles : 3 * n_cu, 1, (hipStream_t)stream)
+                                        : launch<true, 8, 8>("rows_gated", x, w, a, tiles < n_cu ? tiles : n_cu, 1, (hipStream_t)stream);
 }
 
 int rows_plain(float *y, const void *x, const void *w, int n_rows, int n_out, int n_in, void *stream) {
@@ -303,9 +308,8 @@ int rows_plain(float *y, const void *x, const void *w, int n_rows, int n_out, in
   RowsArgs a{};
   a.n_rows = n_rows, a.n_out = n_out, a.n_in = n_in, a.steps_per_slice = (n_in + 31) / 32, a.y = y;
   const int tiles = (n_out + kTile - 1) / kTile, n_cu = sb::cu_count();
-  if (a.steps_per_slice <= kFewSteps) launch<false, 4, 8>(x, w, a, tiles < 3 * n_cu ? tiles : 3 * n_cu, 1, (hipStream_t)stream);
-  else launch<false, 8, 8>(x, w, a, tiles < 2 * n_cu ? tiles : 2 * n_cu, 1, (hipStream_t)stream);
-  return sb::check_launch("rows_plain");
+  return a.steps_per_slice <= kFewSteps ? launch<false, 4, 8>("rows_plain", x, w, a, tiles < 3 * n_cu ? tiles : 3 * n_cu, 1, (hipStream_t)stream)
+                                        : launch<false, 8, 8>("rows_plain", x, w, a, tiles < 2 * n_cu ? tiles : 2 * n_cu, 1, (hipStream_t)stream);
 }
 
 }  // namespace sb

@@ -1430,7 +1430,9 @@ ROWS_IN_LDS = [(1, 17, 512), (3, 40, 2560), (8, 264, 2568), (8, 4100, 1032), (5,
                # as above where blocks that take a tile each stay behind: more than four rows of long products, long k
                (8, 13700, 2056), (5, 9000, 3200), (1, 40, 4104), (4, 264, 7680),
                # ... and where they do not: one slice of k to eight, a step a wave and remainders, many sums of squares a row
-               (4, 13700, 2056), (8, 2064, 4096), (8, 2048, 4096), (2, 3000, 4088), (7, 9000, 904), (8, 1032, 1544)]
+               (4, 13700, 2056), (8, 2064, 4096), (8, 2048, 4096), (2, 3000, 4088), (7, 9000, 904), (8, 1032, 1544),
+               # X's share below 48 KB and past 64 KB with the block's own LDS, the most rows that this holds for, and the first past it
+               (5, 264, 3584), (5, 272, 4096), (6, 264, 3584)]
 
 
 @pytest.mark.parametrize("rows, inner, width", ROWS_IN_LDS)
