@@ -216,6 +216,16 @@ constexpr size_t own_bytes(bool gated, int w) {
   return sizeof(floatx4_t) * 2 * w * (gated ? 2 : 1) * 64 + sizeof(double) * (gated ? 64 * w : 1);
 }
 
+// Blocks of a whole form: at most `each` a CU, and no more than its LDS holds: one that waits for a place stages X when the others are
+// done, and its share runs by itself.  Eight rows, us, three a CU where two fit and so: gated 13,824 x 2,560 28.7 -> 27.0, 20,480 x 2,560
+// 39.2 -> 35.7, 27,648 x 2,560 49.6 -> 47.0; two where one fits: plain 40,000 x 3,584 48.5 -> 46.8, 152,064 x 3,584 175.3 -> 173.7, 32,000 x
+// 4,096 45.1 -> 43.7, but 128,256 x 4,096 166.4 and 166.6.
+int blocks_for(const RowsArgs &a, bool gated, int w, int each) {
+  const int tiles = (a.n_out + kTile - 1) / kTile, fit = int(kLds / (x_bytes(a.n_rows, a.steps_per_slice, w) + own_bytes(gated, w)));
+  const int most = (each < fit ? each : fit) * sb::cu_count();
+  return tiles < most ? tiles : most;
+}
+
 template <bool GATED, int W, int BATCH>
 int launch(const char *who, const void *x, const void *w, RowsArgs a, int blocks, int slices, hipStream_t s) {
   a.rounds = rounds_of(a.steps_per_slice, W);
@@ -298,18 +308,16 @@ int rows_gated(void *y, const void *x, const double *ssq, int ssq_parts, float e
   RowsArgs a{};
   a.n_rows = n_rows, a.n_out = n_out, a.n_in = n_in, a.steps_per_slice = (n_in + 31) / 32;
   a.ssq = ssq, a.ssq_parts = ssq_parts, a.eps = eps, a.gate = gate, a.y = y;
-  const int tiles = (n_out + kTile - 1) / kTile, n_cu = sb::cu_count();
-  return a.steps_per_slice <= kFewSteps ? launch<true, 4, 8>("rows_gated", x, w, a, tiles < 3 * n_cu ? tiles : 3 * n_cu, 1, (hipStream_t)stream)
-                                        : launch<true, 8, 8>("rows_gated", x, w, a, tiles < n_cu ? tiles : n_cu, 1, (hipStream_t)stream);
+  return a.steps_per_slice <= kFewSteps ? launch<true, 4, 8>("rows_gated", x, w, a, blocks_for(a, true, 4, 3), 1, (hipStream_t)stream)
+                                        : launch<true, 8, 8>("rows_gated", x, w, a, blocks_for(a, true, 8, 1), 1, (hipStream_t)stream);
 }
 
 int rows_plain(float *y, const void *x, const void *w, int n_rows, int n_out, int n_in, void *stream) {
   SB_REQUIRE(rows_whole(n_rows, n_out, n_in, 0), "rows_plain: sizes that it does not take");
   RowsArgs a{};
   a.n_rows = n_rows, a.n_out = n_out, a.n_in = n_in, a.steps_per_slice = (n_in + 31) / 32, a.y = y;
-  const int tiles = (n_out + kTile - 1) / kTile, n_cu = sb::cu_count();
-  return a.steps_per_slice <= kFewSteps ? launch<false, 4, 8>("rows_plain", x, w, a, tiles < 3 * n_cu ? tiles : 3 * n_cu, 1, (hipStream_t)stream)
-                                        : launch<false, 8, 8>("rows_plain", x, w, a, tiles < 2 * n_cu ? tiles : 2 * n_cu, 1, (hipStream_t)stream);
+  return a.steps_per_slice <= kFewSteps ? launch<false, 4, 8>("rows_plain", x, w, a, blocks_for(a, false, 4, 3), 1, (hipStream_t)stream)
+                                        : launch<false, 8, 8>("rows_plain", x, w, a, blocks_for(a, false, 8, 2), 1, (hipStream_t)stream);
 }
 
 }  // namespace sb

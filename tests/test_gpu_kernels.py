@@ -1432,7 +1432,9 @@ ROWS_IN_LDS = [(1, 17, 512), (3, 40, 2560), (8, 264, 2568), (8, 4100, 1032), (5,
                # ... and where they do not: one slice of k to eight, a step a wave and remainders, many sums of squares a row
                (4, 13700, 2056), (8, 2064, 4096), (8, 2048, 4096), (2, 3000, 4088), (7, 9000, 904), (8, 1032, 1544),
                # X's share below 48 KB and past 64 KB with the block's own LDS, the most rows that this holds for, and the first past it
-               (5, 264, 3584), (5, 272, 4096), (6, 264, 3584)]
+               (5, 264, 3584), (5, 272, 4096), (6, 264, 3584),
+               # blocks of which a CU holds two, not three, and tiles for more than one round of either
+               (8, 12304, 2560), (6, 12289, 2552)]
 
 
 @pytest.mark.parametrize("rows, inner, width", ROWS_IN_LDS)
@@ -1456,7 +1458,9 @@ def test_gated_products_whose_blocks_keep_the_rows(rows, inner, width):
         assert torch.equal(again[rest], got[rest])
 
 
-@pytest.mark.parametrize("rows, n, k", [(1, 1000, 8184), (8, 8200, 520), (4, 2048, 2056), (8, 96, 61440), (8, 72, 70000), (9, 2048, 4096), (3, 20001, 136), (8, 17424, 7688)])
+@pytest.mark.parametrize("rows, n, k", [(1, 1000, 8184), (8, 8200, 520), (4, 2048, 2056), (8, 96, 61440), (8, 72, 70000), (9, 2048, 4096), (3, 20001, 136), (8, 17424, 7688),
+                                        # one block a CU, and tiles that fill a round of one and not of two
+                                        (8, 4112, 3584), (8, 8208, 4096)])
 def test_raw_and_plain_products_whose_blocks_keep_the_rows(rows, n, k):
     """In K slices, and whole with float results where the matrix is wide, against 64 bits: cuts of K that the blocks' share of LDS
     allows and some that it does not."""
