@@ -636,24 +636,21 @@ STREAM_MIN_BLOCKS = 136
 SPLIT_MAX_ROWS = 8
 SPLIT_CUS = 256
 SPLIT_FULL = 0.87
-SPLIT_SMALL = 20 << 20
 
 
 def split_norm_pays(rows: int, width: int, inner: int) -> bool:
     """Whether :func:`gemm_split_join` and :func:`gemm_split_gated` are ahead of the two products with the norm as a pass
-    between them.  A block of theirs owns sixteen features whole, so they want the blocks' rounds over the CUs nearly full
-    (the joining product: a single round, or up to four rows); a gated product of up to 20 M weights is so short that the pass
-    saved decides.  Measured, both products and the norm, replayed graphs with the weights cold, at 1 / 4 / 8 rows (us, before ->
-    after): 896 x 4,864 13.9 -> 11.8, 14.3 -> 12.0, 14.6 -> 12.2; 1,536 x 8,960 21.0 -> 19.8, 21.0 -> 20.3, 21.2 -> 21.0; 2,048 x
-    11,008 28.2 -> 26.3, 27.3 -> 26.3, 27.8 -> 27.2; 3,584 x 18,944 63.3 -> 58.2, 62.8 -> 57.6, 60.9 -> 59.9; 8,192 x 29,568 209
-    -> 199, 209 -> 202, and at eight rows, not taken, 201 -> 202.  Not taken either: 5,120 x 13,824 (320 blocks join, 864 gate)
-    68.7 -> 71.0, 68.4 -> 73.0, 65.7 -> 73.3; 4,608 x 8,960 46.8 -> 49.0, 47.0 -> 50.4, 47.4 -> 52.7; 3,072 x 13,824 42.0 -> 43.2,
-    42.1 -> 43.9, 40.7 -> 44.2; 3,072 x 8,960 34.0 -> 33.0, 32.6 -> 33.1, 32.8 -> 34.6; 7,168 x 18,944 at eight rows 117 -> 121."""
-    def full(features: int) -> bool:
-        rounds = -(-features // 16) / SPLIT_CUS
-        return rounds >= SPLIT_FULL * math.ceil(rounds)
-    return rows <= SPLIT_MAX_ROWS and (width <= 16 * SPLIT_CUS or (rows <= 4 and full(width))) \
-        and (width * inner <= SPLIT_SMALL or full(inner))
+    between them.  The gated product runs in the same kernels either way, whatever its ``inner`` size; a block of the joining one owns
+    sixteen features whole, so it wants a single round over the CUs, or up to four rows in rounds that are nearly full.  Measured, both
+    products and the norm, replayed graphs with the weights cold, at 1 / 4 / 8 rows (us, with the pass -> without): 896 x 4,864 11.5 ->
+    9.6, 11.9 -> 9.7, 12.4 -> 10.0; 1,536 x 8,960 19.1 -> 17.3, 19.7 -> 17.7, 20.5 -> 18.4; 2,048 x 11,008 23.9 -> 22.3, 23.7 -> 22.0, 24.7 ->
+    22.9; 2,560 x 9,728 26.5 -> 25.2, 27.6 -> 26.0, 29.9 -> 27.8; 3,072 x 8,960 30.7 -> 28.5, 31.7 -> 29.1, 31.8 -> 29.0; 3,072 x 13,824 38.2
+    -> 36.4, 39.5 -> 37.0, 39.6 -> 36.8; 3,584 x 18,944 54.0 -> 51.6, 52.6 -> 50.1, 53.8 -> 51.3; 4,096 x 11,008 40.8 -> 39.7, 39.9 -> 38.4,
+    41.5 -> 39.5; 7,168 x 18,944 109.4 -> 104.3, 105.6 -> 103.9; 8,192 x 29,568 186.3 -> 182.2, 184.9 -> 183.0.  Not taken: 7,168 and 8,192 wide at
+    eight rows 107.3 -> 107.2 and 173.8 -> 181.4; 4,608 x 8,960 (288 blocks) 44.1 -> 45.2, 44.8 -> 45.8, 46.7 -> 47.7; 5,120 x 13,824 64.1 ->
+    64.7, 64.6 -> 65.3, 63.6 -> 65.1; 6,144 x 16,384 82.3 -> 84.4, 80.7 -> 82.4, 84.9 -> 84.5."""
+    rounds = -(-width // 16) / SPLIT_CUS
+    return rows <= SPLIT_MAX_ROWS and (rounds <= 1 or (rows <= 4 and rounds >= SPLIT_FULL * math.ceil(rounds)))
 
 
 class ScaledRows:

@@ -1559,7 +1559,8 @@ def test_the_norm_between_two_products_sums_in_double():
     assert ((got - torch.relu(g) * u).abs() <= (torch.relu(g) * u).abs() * 2.0 ** -8 + 1.2 * (sg * u.abs() + su * g.abs()) + 1e-5).all()
 
 
-@pytest.mark.parametrize("width, heads, inner, rows", [(128, 2, 320, 9), (5120, 40, 320, 1), (8192, 64, 320, 4), (8192, 64, 320, 5)])
+@pytest.mark.parametrize("width, heads, inner, rows", [(128, 2, 320, 9), (5120, 40, 320, 1), (8192, 64, 320, 4), (8192, 64, 320, 5),
+                                                        (3072, 24, 8960, 2)])
 def test_decode_steps_on_both_sides_of_the_rule_for_the_norm(width, heads, inner, rows):
     """The norm rides in the products, or is a pass between them: the same logits but for the order of a norm's factor and of
     sums, and the rule asks for what the sizes take."""
