@@ -1332,12 +1332,60 @@ def test_attention_prefill_window_edge(hq, hkv, hd, window):
 @pytest.mark.parametrize("form", [1, 2])
 def test_attention_prefill_forms(hq, hkv, hd, window, form):
     """Pages one by one through a block and pages cut over a block's waves, whichever the sizes would choose: whole
-    prompts and a continuation in tiles of every height, and the edges of a window over more pages than a block has waves."""
+    prompts and a continuation in tiles of every height, and the edges of a window, up to six pages of which a block sees."""
     from sonicboom_amd import ops
     with ops.attention_prefill_form(form):
         test_attention_prefill_matrix_cores(hq, hkv, hd, min(window, 70))
         if window:
             test_attention_prefill_window_edge(hq, hkv, hd, window)
+
+
+@pytest.mark.parametrize("hq, hkv, hd", [(4, 1, 64), (2, 1, 96), (5, 1, 112), (6, 2, 128)])
+@pytest.mark.parametrize("window", [0, 577, 1000, 1024])
+@pytest.mark.parametrize("missing", [(), (3, 10)])
+def test_attention_prefill_waves_of_several_pages(hq, hkv, hd, window, missing):
+    """Pages cut over a block's eight waves, ten to 28 of them, against 64 bits: waves with one, two and more pages, a window that starts
+    in a wave's first page, on a page's first key and in the page after it, pages behind the window that are not in the table, keys that no
+    row sees that are not numbers, and pages outside the cache as a wave's first and as a later one.  One key more or less at the
+    window's edge, and every page, would show."""
+    from sonicboom_amd import ops
+    n, first = 1730, 1660                       # rows first .. n - 1
+    rows = n - first
+    width = -(-n // 64)
+    lo_all = max(first - window + 1, 0) if window else 0
+    table = torch.randperm(width + 3, generator=torch.Generator().manual_seed(5))[:width].to(torch.int32)[None, :]
+    kc, vc = (randn(*shape, seed=2 + i).to(BF16) for i, shape in enumerate(((width + 3, hkv, 64, hd), (width + 3, hkv, hd, 64))))
+    own = table[0].long()
+    for p in range(lo_all - 1, lo_all + rows) if window else ():       # (large values where the rows' windows start)
+        layout.put_value(vc, int(own[p // 64]), p % 64, 4.0 * layout.get_value(vc, int(own[p // 64]), p % 64).float())
+    k = layout.keys_in_order(kc)[own].permute(0, 2, 1, 3).reshape(-1, hkv, hd)[:n]
+    v = layout.values_in_order(vc)[own].permute(0, 3, 1, 2).reshape(-1, hkv, hd)[:n]
+    none = torch.full((hkv, hd), float("nan"))
+    for p in [*range(lo_all // 64 * 64, lo_all), *range(n, width * 64)]:
+        layout.put_key(kc, int(table[0, p // 64]), p % 64, none)
+        layout.put_value(vc, int(table[0, p // 64]), p % 64, none)
+    first_page = lo_all // 64
+    table[0, :first_page] = -1
+    pos, key = torch.arange(first, n)[:, None], torch.arange(n)[None, :]
+    seen = (key <= pos) & (key > pos - window if window else key >= 0)
+    for i, page in enumerate(missing):
+        table[0, first_page + page] = (-1, width + 3)[i]
+        seen[:, (first_page + page) * 64:(first_page + page + 1) * 64] = False
+    q = randn(rows, hq * hd, seed=7).to(BF16)
+    views = q.view(rows, hq, hd)
+    p, want, slack = attention_64(views, k, v, seen, hd ** -0.5)
+    assert a_page_left_out_shows(p[:, :1], v, want[:1], slack[:1], hq)
+    if window and not missing:
+        for shift in (-1, 1):
+            off = attention_64(views, k, v, (key <= pos) & (key > pos - window - shift), hd ** -0.5)[1]
+            assert ((off - want).abs() > 2 * slack).any(2).any(1).all()
+    for height in (16, 32) if ops.attention_tall_ok(hq, hkv, hd) else (16,):
+        tiles = torch.tensor([(r, min(height, rows - r), 0, 0) for r in range(0, rows, height)], dtype=torch.int32)
+        with ops.attention_prefill_form(2):
+            got = ops.attention_prefill_mfma(q.to(DEV), kc.to(DEV), vc.to(DEV), table.to(DEV), pos[:, 0].to(torch.int32).to(DEV),
+                                             tiles.to(DEV), hq, hkv, hd, hd ** -0.5, window, tile_rows=height)
+        off = (got.cpu().double().view(rows, hq, hd) - want).abs()
+        assert (off <= slack).all(), f"tiles of {height}: off by {off.nan_to_num(math.inf).max():.3g}"
 
 
 @pytest.mark.parametrize("t, n, k", [(1, 4, 16), (3, 20, 40), (33, 100, 64), (70, 516, 1100), (40, 36, 2064)])
