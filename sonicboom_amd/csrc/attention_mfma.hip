@@ -1635,14 +1635,22 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
   // form builds; or the half of it that holds a visible key (one row of 145 keys 6.0 us, 6.4 with the last page whole).  The page
   // that receives the row's own key and value is read like the others, before they are stored, and its fragments are patched from
   // LDS afterwards.
-  constexpr bool kWhole = HD <= 128;
+  // Chunks of four pages take a page in one softmax step.  Rows taken whole take it half by half: the first half's step runs while the
+  // second half's loads are on their way, and the registers are fewer.  us, a page a step and so, 16 heads of 128 on 2: 140 keys, one row
+  // 8.30 -> 7.81, 24 rows 9.01 -> 8.70; 500 keys 10.07 -> 9.62, eight rows 10.53 -> 10.23, but 24 rows 12.9 -> 13.3; 14 heads of 64 on 2, 140
+  // keys 6.68 -> 6.46, 24 rows 7.31 -> 7.12, 500 keys 7.25 -> 7.11, but 24 rows 8.25 -> 8.40.  (A kernel of both forms, by the row's length,
+  // needs more registers: in chunks, 24 rows of 2,000 keys 20.1 -> 24.3.)
+  constexpr bool kWhole = HD <= 128, kHalves = WAVES > kPagesPerChunk;
   const bool use0 = have_page && !(page_pos > pos || page_pos + 31 < key_lo);
   const bool use1 = have_page && !(page_pos + 32 > pos || page_pos + 63 < key_lo);
   const bool both = use0 && use1;
   HalfPage h[2], &one = h[0];       // one: the only half
   const int half = use0 ? 0 : 1;
   if constexpr (kWhole) {
-    if (both) {
+    if constexpr (kHalves) {
+      if (use0) load_half_straight(h[0], k_cache + off, v_cache + off, 0, lane);
+      if (use1) load_half_straight(h[1], k_cache + off, v_cache + off, 1, lane);
+    } else if (both) {
       load_keys_straight(h, k_cache + off, lane);
       load_values_straight(h, v_cache + off, lane);
     } else if (use0 || use1) {
@@ -1660,14 +1668,20 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
     if constexpr (kWhole) {
       if (ra.store && have_page && pg == pos / SB_PAGE) {
         const int slot = pos % SB_PAGE;       // (in the last half that is read)
-        if (both) patch_half(h[1], rope_sh, 1, slot, lane);
+        if constexpr (kHalves) {
+          if (slot < 32) patch_half(h[0], rope_sh, 0, slot, lane);
+          else patch_half(h[1], rope_sh, 1, slot, lane);
+        } else if (both) patch_half(h[1], rope_sh, 1, slot, lane);
         else patch_half(one, rope_sh, half, slot, lane);
       }
     }
   }
   if (have_page) {
     if constexpr (kWhole) {
-      if (both)
+      if constexpr (kHalves) {
+        if (use0) attend_half<1>(st, qf, h[0], page_pos, col_pos, key_lo, key_lo, pos, scale_log2, lane);
+        if (use1) attend_half<1>(st, qf, h[1], page_pos + 32, col_pos, key_lo, key_lo, pos, scale_log2, lane);
+      } else if (both)
         attend_whole_page<true>(st, qf, h, page_pos, col_pos, key_lo, key_lo, pos, scale_log2, lane, [] {});
       else if (use0 || use1)
         attend_half<1>(st, qf, one, page_pos + 32 * half, col_pos, key_lo, key_lo, pos, scale_log2, lane);
