@@ -2118,7 +2118,7 @@ extern "C" size_t sb_attn_decode_part_ml(int n_seqs, int heads_q, int heads_kv, 
 
 namespace {
 
-// Rows of like length, as the caller knows: every row in so many chunks (1 to 16) that the GPU's blocks finish together, which needs no
+// Rows of like length, as the caller knows, or of whatever length on short tables (equal_chunks): every row in so many chunks (1 to 16) that the GPU's blocks finish together, which needs no
 // look at the other rows and, in one chunk, no merging kernel.  The count with the least estimated time (MI355X, cold caches): a CU
 // streams some 27 GB/s whatever the count of its blocks, all of them 5.3 TB/s; a wave gets through a page in 3.3 us at least; a second
 // kernel costs 5 us.  The table's width is taken for the rows' length less half of the 16 pages it is rounded up by.
@@ -2144,6 +2144,16 @@ int like_cut(long long rows_tiles, int max_pages) {
 // Whether the pages of a step's rows are dealt out: where the widest row's chunks for every row would be blocks for most of the GPU.
 bool deals(long long rows_tiles, int max_pages) { return HD <= 128 && (long long)((max_pages + 7) / 8) * rows_tiles >= kDealtFrom; }
 
+// Whether rows come in equal chunks whatever their lengths: where the table is short beside the count of rows, the longest row cannot hold up
+// the others by more than dealing out and merging cost (less so with larger heads, whose pages take longer).  Lengths spread from 8
+// keys to what fills the table, us, dealt out and so: 28 heads of 128 on 4, 64 rows on 8 pages 19.4 -> 15.1, on 16 19.4 -> 17.7, on 24 22.3 and 25.8;
+// 128 rows on 8 28.6 -> 19.0, on 16 32.4 -> 25.0, on 24 35.2 -> 30.9, on 32 39.4 -> 39.0, on 48 46.5 and 53.0; 16 on 2, 96 rows on 16 18.3 -> 17.7, on
+// 24 19.7 and 22.5; 14 heads of 64 on 2, 64 rows on 16 12.1 -> 11.4, on 24 12.4 and 14.1, 128 on 8 14.9 -> 10.4, on 16 14.7 -> 12.2, on 24 15.9 ->
+// 14.6, on 48 19.4 and 23.4.
+bool equal_chunks(long long rows_tiles, int max_pages) {
+  return deals(rows_tiles, max_pages) && (long long)max_pages * (HD + 64) <= 12 * (rows_tiles + 64);
+}
+
 // The decode launch, for queries that are given (q) or still to be built (ra.qkv).
 int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra, const void *k_cache,
                   const void *v_cache, const int32_t *page_table, int max_pages, int n_pages_total,
@@ -2160,7 +2170,8 @@ int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra,
   const long long per_chunk = (long long)heads_kv * head_tiles * n_seqs;
   // pages_per_wave: a test's or a measurement's choice of pages of a wave, 0 the launcher's own, -1 too, with rows of like length
   const bool dealt = HD <= 128 && (pages_per_wave > 1 || (pages_per_wave <= 0 && deals(per_chunk, max_pages)));
-  const int cut = pages_per_wave < 0 ? sb_attn_decode_cut(n_seqs, heads_q, heads_kv, max_pages) : 0;
+  const int cut = pages_per_wave <= 0 && equal_chunks(per_chunk, max_pages) ? like_cut(per_chunk, max_pages)
+                  : pages_per_wave < 0 ? sb_attn_decode_cut(n_seqs, heads_q, heads_kv, max_pages) : 0;
   const int fixed_share = cut ? -cut : pages_per_wave > 0 ? pages_per_wave : 0;
   // five to eight pages a row: a block of eight waves takes a row whole (with more rows than half the CUs the chunks fill the GPU as it is)
   const bool whole_rows = kWholeRows && !dealt && pages_per_wave <= 0 && max_pages > kPagesPerChunk && max_pages <= kWholePages &&
@@ -2210,7 +2221,7 @@ int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra,
 extern "C" int sb_attn_decode_cut(int n_seqs, int heads_q, int heads_kv, int max_pages) {
   if (n_seqs <= 0 || heads_kv <= 0 || heads_q % heads_kv || max_pages <= 0) return 0;
   const long long rows_tiles = (long long)n_seqs * heads_kv * ((heads_q / heads_kv + 15) / 16);
-  return deals(rows_tiles, max_pages) && rows_tiles >= kLikeFrom ? like_cut(rows_tiles, max_pages) : 0;
+  return deals(rows_tiles, max_pages) && !equal_chunks(rows_tiles, max_pages) && rows_tiles >= kLikeFrom ? like_cut(rows_tiles, max_pages) : 0;
 }
 
 // q, out: bf16 [n_seqs, heads_q * HD], one row per sequence; k_cache bf16 [pages][heads_kv][64][HD],

@@ -268,25 +268,25 @@ def test_batches_run_in_buckets_with_rows_that_do_nothing(model_folders):
 
 
 def test_steps_of_like_sequences_are_recordings_of_their_own():
-    """128 sequences on two key/value heads fill the GPU by themselves: a step of sequences of like length runs their attention without
-    a look at the lengths and a merging kernel, as a recording beside the one for unequal lengths, and gives the tokens of kernel by kernel."""
+    """Many sequences on long tables: a step of sequences of like length runs their attention without a look at the lengths, as a recording
+    beside the one for unequal lengths, and gives the tokens of kernel by kernel.  On short tables the lengths make no difference."""
     from sonicboom_amd.engine import DecoderModel, Engine, generate
     from sonicboom_amd.sampling import SamplingParams
-    model = DecoderModel.from_random(dict(TINY["A"]), 3, "bfloat16", "cuda:0")
-    n = 128
-    engines = [Engine(model, 64 * 4 * n, max_slots=n) for _ in range(2)]
+    model = DecoderModel.from_random(dict(TINY["A"], max_position_embeddings=4096), 3, "bfloat16", "cuda:0")
+    n = 33
+    engines = [Engine(model, 64 * 33 * n, max_slots=n) for _ in range(2)]
     engines[1].use_graphs = False
-    for lengths, steps in (([9 + i % 3 for i in range(n)], 8), ([60 + 5 * (i == 7) for i in range(n)], 8), ([100 if i < 8 else 2 for i in range(n)], 8)):
+    for lengths, steps in (([1540 + i % 3 for i in range(n)], 8), ([1600] + [9] * (n - 1), 8)):
         prompts = prompts_for("A", lengths, seed=5)
         got, want = (generate(e, prompts, SamplingParams(max_tokens=steps), stop_tokens=(), max_batch=n) for e in engines)
         assert got == want and all(len(o) == steps for o in got)
-    assert {k[0] for k in engines[0].decode_loop()._graphs} == {n}
     assert [k[3] for k in engines[0].decode_loop()._graphs] == [True, False]
-    # few sequences: the lengths make no difference, and one recording serves both
-    assert not engines[0].decode_loop()._graphs.clear()
-    generate(engines[0], prompts_for("A", [9, 9, 9], seed=6), SamplingParams(max_tokens=8), stop_tokens=())
-    generate(engines[0], prompts_for("A", [90, 9, 9], seed=6), SamplingParams(max_tokens=8), stop_tokens=())
-    assert [k[0::3] for k in engines[0].decode_loop()._graphs] == [(3, False)]
+    # short tables: one recording serves both, with many sequences, which come in equal chunks, and with few
+    for n, lengths in ((128, [9 + i % 3 for i in range(128)]), (128, [100 if i < 8 else 2 for i in range(128)]), (3, [9, 9, 9]), (3, [90, 9, 9])):
+        engine = engines[0] if n == 3 else Engine(model, 64 * 4 * n, max_slots=n)
+        assert not engine.decode_loop()._graphs.clear()
+        generate(engine, prompts_for("A", lengths, seed=6), SamplingParams(max_tokens=8), stop_tokens=(), max_batch=n)
+        assert [k[0::3] for k in engine.decode_loop()._graphs] == [(n, False)]
 
 
 def test_graph_replay_when_the_page_table_grows(tmp_path):
