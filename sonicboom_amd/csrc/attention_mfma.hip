@@ -55,6 +55,7 @@ constexpr int DT = HD / 16;          // 16-row tiles of O^T
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kPagesPerChunk = 4;
 constexpr int kWholePages = 8;               // pages of a row that one block takes whole
+constexpr int kWholeMost = 128;              // ... of rows x head tiles
 constexpr bool kWholeRows = HD <= 128;       // (its waves' sums meet in 64 KB of LDS at most)
 constexpr float kMaxSlack = 8.f;
 constexpr int kWaveSlots = 2048;             // waves among which the pages of a batch are dealt out: two a SIMD
@@ -2149,9 +2150,10 @@ bool deals(long long rows_tiles, int max_pages) { return HD <= 128 && (long long
 // keys to what fills the table, us, dealt out and so: 28 heads of 128 on 4, 64 rows on 8 pages 19.4 -> 15.1, on 16 19.4 -> 17.7, on 24 22.3 and 25.8;
 // 128 rows on 8 28.6 -> 19.0, on 16 32.4 -> 25.0, on 24 35.2 -> 30.9, on 32 39.4 -> 39.0, on 48 46.5 and 53.0; 16 on 2, 96 rows on 16 18.3 -> 17.7, on
 // 24 19.7 and 22.5; 14 heads of 64 on 2, 64 rows on 16 12.1 -> 11.4, on 24 12.4 and 14.1, 128 on 8 14.9 -> 10.4, on 16 14.7 -> 12.2, on 24 15.9 ->
-// 14.6, on 48 19.4 and 23.4.
+// 14.6, on 48 19.4 and 23.4.  From five to eight pages also with fewer rows, where a row is not taken whole by eight waves: against chunks
+// of four pages and a merging kernel, 28 on 4, 48 rows of 140 keys 13.5 -> 11.0, of 500 22.2 -> 17.1; 14 of 64 on 2, 96 rows 10.4 -> 7.8 and 15.6 -> 11.4.
 bool equal_chunks(long long rows_tiles, int max_pages) {
-  return deals(rows_tiles, max_pages) && (long long)max_pages * (HD + 64) <= 12 * (rows_tiles + 64);
+  return HD <= 128 && (deals(rows_tiles, max_pages) || (rows_tiles > kWholeMost && max_pages > kPagesPerChunk)) && (long long)max_pages * (HD + 64) <= 12 * (rows_tiles + 64);
 }
 
 // The decode launch, for queries that are given (q) or still to be built (ra.qkv).
@@ -2169,13 +2171,13 @@ int decode_launch(const char *who, void *out, const void *q, const RopeArgs &ra,
   // A wave takes one page and asks for all of it at once (one round trip to memory), or the chunks are dealt out by what the rows hold.
   const long long per_chunk = (long long)heads_kv * head_tiles * n_seqs;
   // pages_per_wave: a test's or a measurement's choice of pages of a wave, 0 the launcher's own, -1 too, with rows of like length
-  const bool dealt = HD <= 128 && (pages_per_wave > 1 || (pages_per_wave <= 0 && deals(per_chunk, max_pages)));
+  const bool dealt = HD <= 128 && (pages_per_wave > 1 || (pages_per_wave <= 0 && (deals(per_chunk, max_pages) || equal_chunks(per_chunk, max_pages))));
   const int cut = pages_per_wave <= 0 && equal_chunks(per_chunk, max_pages) ? like_cut(per_chunk, max_pages)
                   : pages_per_wave < 0 ? sb_attn_decode_cut(n_seqs, heads_q, heads_kv, max_pages) : 0;
   const int fixed_share = cut ? -cut : pages_per_wave > 0 ? pages_per_wave : 0;
   // five to eight pages a row: a block of eight waves takes a row whole (with more rows than half the CUs the chunks fill the GPU as it is)
   const bool whole_rows = kWholeRows && !dealt && pages_per_wave <= 0 && max_pages > kPagesPerChunk && max_pages <= kWholePages &&
-                          per_chunk <= 128;
+                          per_chunk <= kWholeMost;
   const int pages_per_chunk = whole_rows ? kWholePages : kPagesPerChunk;
   const int n_chunks = cut ? cut : (max_pages + pages_per_chunk - 1) / pages_per_chunk;
   SB_SUPPORT((long long)n_chunks * per_chunk <= 0x7fffffffLL, "%s: too many blocks", who);

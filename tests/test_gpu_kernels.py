@@ -1826,11 +1826,11 @@ def test_attention_decode_deals_pages_out(hq, hkv, hd, lens, window):
 # (heads, kv heads, head size, rotary width): more rows than a wave looks at at once, of lengths from one key on
 @pytest.mark.parametrize("hq, hkv, hd, rot, lens", [(14, 2, 64, 64, [1 + 37 * i % 1500 for i in range(130)]), (28, 4, 128, 128, [60 + 131 * i % 1400 for i in range(70)]),
                                                     (16, 1, 128, 64, [30 + 211 * i % 6000 for i in range(65)]), (8, 8, 80, 0, [64 * (1 + 5 * i % 40) for i in range(20)]),
-                                                    (14, 2, 64, 64, [1 + 37 * i % 2400 for i in range(130)])],
+                                                    (14, 2, 64, 64, [1 + 37 * i % 2400 for i in range(130)]), (28, 4, 128, 128, [1 + 97 * i % 500 for i in range(40)])],
                          ids=lambda v: f"{len(v)}rows" if isinstance(v, list) else str(v))
 @pytest.mark.parametrize("window, alike", [(0, False), (0, True), (300, False), (300, True)])
 def test_attention_decode_folded_in_where_pages_are_dealt_out(hq, hkv, hd, rot, lens, window, alike):
-    assert -(-max(lens) // 64 // 8) * len(lens) * hkv >= 256
+    assert -(-max(lens) // 64 // 8) * len(lens) * hkv >= 256 or (len(lens) * hkv > 128 and max(lens) > 4 * 64)
     folded_against_two_kernels(hq, hkv, hd, rot, window, 0, lens, alike)
 
 
