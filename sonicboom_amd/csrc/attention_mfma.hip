@@ -1636,12 +1636,13 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
   // form builds; or the half of it that holds a visible key (one row of 145 keys 6.0 us, 6.4 with the last page whole).  The page
   // that receives the row's own key and value is read like the others, before they are stored, and its fragments are patched from
   // LDS afterwards.
-  // Chunks of four pages take a page in one softmax step.  Rows taken whole take it half by half: the first half's step runs while the
-  // second half's loads are on their way, and the registers are fewer.  us, a page a step and so, 16 heads of 128 on 2: 140 keys, one row
-  // 8.30 -> 7.81, 24 rows 9.01 -> 8.70; 500 keys 10.07 -> 9.62, eight rows 10.53 -> 10.23, but 24 rows 12.9 -> 13.3; 14 heads of 64 on 2, 140
-  // keys 6.68 -> 6.46, 24 rows 7.31 -> 7.12, 500 keys 7.25 -> 7.11, but 24 rows 8.25 -> 8.40.  (A kernel of both forms, by the row's length,
-  // needs more registers: in chunks, 24 rows of 2,000 keys 20.1 -> 24.3.)
-  constexpr bool kWhole = HD <= 128, kHalves = WAVES > kPagesPerChunk;
+  // A page is one softmax step.  Only heads of more than 64 in rows taken whole step half by half: the first half's step runs while the
+  // second half's loads are on their way.  us, a page a step and so, 16 heads of 128 on 2: 140 keys, one row 8.30 -> 7.81, 24 rows 9.01 ->
+  // 8.70; 500 keys 10.07 -> 9.62, eight rows 10.53 -> 10.23, but 24 rows 12.9 -> 13.3; in decode steps of the 1.5B sizes one row of 440 keys
+  // 1,312 -> 1,298, eight of 115 1,337 -> 1,325.  14 heads of 64 on 2 gain alone (6.68 -> 6.46 and 7.25 -> 7.11) and not in a step (0.5B sizes,
+  // one row of 137 keys 745 and 749, 24 of 440 1,169 and 1,178).  (A kernel of both forms, by the row's length, needs more registers: in
+  // chunks, 24 rows of 2,000 keys 20.1 -> 24.3.)
+  constexpr bool kWhole = HD <= 128, kHalves = WAVES > kPagesPerChunk && HD > 64;
   const bool use0 = have_page && !(page_pos > pos || page_pos + 31 < key_lo);
   const bool use1 = have_page && !(page_pos + 32 > pos || page_pos + 63 < key_lo);
   const bool both = use0 && use1;
