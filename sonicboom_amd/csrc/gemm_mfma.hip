@@ -1404,14 +1404,16 @@ namespace {
 // 3B sizes and at 1,800 and 2,300 of 2,048 wide layers of other designs: not taken.
 //
 // Some hundred rows: the same tiles of 128 x 128, or of 64 x 128, loaded straight into LDS with four
-// stages' buffers, a block a CU, where tiles x slices make one round over each die's 32 CUs.  A launch costs
-// 3.5 us and a stage of 64 k 0.33 us (64 rows), 0.55 (128 rows) and 0.75 (128 x 128 through registers); a slice is written and
-// read, and the stream and its norm cost two and a half times as much, at 2.9 TB/s (up to 640 rows 4).  183 rows against 1,536 x 1,536: 8.5 us through
-// registers, 6.2; 288 against 896 x 4,864: 14.9 and 9.8; with the pass that adds and norms, 700 against 2,048 x 1,536 26.0 and 19.8, 900
-// against 1,536 x 1,536 26.0 and 20.0, 520 against 896 x 4,864 26.6 and 18.5.  A whole product whose tiles make one round is as fast a
-// stage, and its residual and norm move three and a half planes in 4 us more: taken where that is less (1,300 rows against 1,536 x 8,960 81
-// and 60 us, 896 x 896 20.7 and 16.1, 2,048 x 1,536 31.3 and 27.4; 700 rows against 1,536 x 1,536 19.4 in slices and 20.2), and
-// past 1,200 rows where only tiles through registers are left (1,600 against 2,048 x 11,008 109 and 98, 2,560 x 2,048 48 and 42).
+// stages' buffers, a block a CU, where tiles x slices make one round over each die's 32 CUs, or a whole product whose tiles make one.
+// Prices in microseconds, fitted to 292 sizes of 96 to 3,500 rows in all their cuts (slices and the pass that adds them, the stream and its
+// norm, against the whole product and the norm; replayed graphs, weights cold): a stage of 64 k 0.29 (64 rows), 0.41 (128 rows; in a whole
+// product 0.525) and 0.8 (128 x 128 through registers); a slice is written and read at 3.1 TB/s, past 32 MB (what
+// the dies' L2 hold) at 2.8, the stream and its norm take two and a half times as much, and a whole product one plane and 2.6 us more; past
+// 1,150 rows slices through registers are never ahead.  The choice is 2.2 % behind the best on the mean (3.6 with the prices before), most where
+// a whole product takes larger tiles than the price knows: 700 x 3,584 x 18,944 (rows, out, in) 120 us whole, 154 in slices.  us, the best cut / the
+// choice with prices of 183 to 900 rows that changed their rate at 640 / this one: 288 x 4,096 x 14,336 60.6 / 82.3 / 60.6; 400 x 3,072 x
+// 8,192 38.9 / 50.2 / 38.9; 520 x 2,560 x 9,728 46.4 / 59.9 / 46.4; 640 x 1,536 x 8,960 35.6 / 39.1 / 35.6; 1,000 x 1,152 x 896 15.0 / 19.1 / 15.0; 1,200 x
+// 896 x 896 14.7 / 19.4 / 14.8; but 600 x 2,560 x 2,048 21.4 / 21.4 / 22.6.
 enum PartialTile { kRegisters128, kBig, kDirect128, kDirect64 };
 struct PartialPlan { int slices; PartialTile tile; };
 double load_factor(long long blocks) { return blocks <= 170 ? 0.72 : 0.72 + 0.28 * double(blocks - 170) / 86.0; }
@@ -1450,23 +1452,24 @@ PartialPlan partial_plan(int n_rows, int n_out, int n_in, bool direct_ok) {
     }
   }
   if (s > 1 && direct_ok) {
-    const double plane = n_rows * double(n_out) * 4.0 / (n_rows <= 640 ? 4e6 : 2.9e6);      // us that a slice takes to write or read
+    const double plane_mb = n_rows * double(n_out) * 4e-6;
+    const auto pass_us = [](double mb) { return mb <= 32.0 ? 0.325 * mb : 0.325 * 32.0 + 0.36 * (mb - 32.0); };      // to write or read
     const auto cost = [&](double stage_us, long long slices) {
-      return stage_us * double((n_k + slices - 1) / slices) + (2.0 * slices + 2.5) * plane;
+      return stage_us * double((n_k + slices - 1) / slices) + 2.0 * pass_us(slices * plane_mb) + 2.5 * pass_us(plane_mb);
     };
     const auto one_round = [&](long long n_tiles) { return (n_tiles + kXcds - 1) / kXcds <= sb::cu_count() / kXcds; };
     const auto tiles_of = [&](int bm) { return (long long)((n_rows + bm - 1) / bm) * ((n_out + 127) / 128); };
-    double best = cost(0.75, s);
+    double best = cost(0.8, s);
     PartialTile tile = kRegisters128;
     for (int half = 0; half < 2; ++half) {
       const long long n_tiles = tiles_of(half ? 64 : 128);
       for (long long s2 = 2; s2 <= 8 && (n_tiles + kXcds - 1) / kXcds * s2 <= sb::cu_count() / kXcds && s2 * 3 <= n_k; ++s2) {
-        const double t = cost(half ? 0.33 : 0.55, s2);
+        const double t = cost(half ? 0.29 : 0.41, s2);
         if (t < best) best = t, tile = half ? kDirect64 : kDirect128, s = s2;
       }
     }
-    const double stage_whole = one_round(tiles_of(64)) ? 0.33 : one_round(tiles_of(128)) ? 0.45 : 0.0;
-    if ((tile == kRegisters128 && n_rows > 1200) || (stage_whole > 0.0 && stage_whole * n_k + 3.5 * plane + 4.0 < best))
+    const double stage_whole = one_round(tiles_of(64)) ? 0.29 : one_round(tiles_of(128)) ? 0.525 : 0.0;
+    if ((tile == kRegisters128 && n_rows > 1150) || (stage_whole > 0.0 && stage_whole * n_k + 3.5 * pass_us(plane_mb) + 2.6 < best))
       return {1, kRegisters128};
     const int per = int((n_k + s - 1) / s);
     return {(n_k + per - 1) / per, tile};

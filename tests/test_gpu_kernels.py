@@ -359,6 +359,14 @@ def test_gemm_bf16_k_slices_of_tiled_products(t, n, k):
     close(got, ref_gemm(x, w, None, None), atol=3e-5 * math.sqrt(k), rtol=1e-5, what="slices")
 
 
+def test_k_slices_of_prompts_of_some_hundred_rows():
+    """How a prompt's product is cut over K: in fewer slices as rows grow, and whole where slices cost more to write and read than they save."""
+    from sonicboom_amd import ops
+    slices = ops.library.core().sb_gemm_mfma_slices
+    assert [slices(t, 896, 896, 1) for t in (183, 400, 1200)] == [3, 2, 1]
+    assert [slices(t, 4096, 14336, 1) for t in (183, 288, 400)] == [4, 2, 2] and slices(640, 1536, 8960, 1) == 4
+
+
 def test_silu_of_the_tiled_product_over_its_range():
     """A product that hands the gate its numbers as they are, over the float32 range: against 64-bit arithmetic to
     two units of the last of 24 bits, and where e^-g runs out of the range to what is as good as zero."""
