@@ -101,6 +101,7 @@ head_product_mfma_kernel(bf16_t *__restrict__ out, int out_stride, int out_hstri
 // a SIMD.  Measured, 16 heads, rows of 16, 32 and 64 a wave (the first the kernel above), us: 128 to 512 numbers, 4,001 rows 79.7, 58.6, 43.8 (348
 // registers: 51.4), 1,000 rows 22.8, 14.3, 14.0, 500 rows 12.7, 10.5, 8.4; 512 to 128 with a gate, 4,001 rows 92.7, 59.4, 44.7 (54.8),
 // 3,000 rows 69.6, 48.9, 42.9, 2,000 rows with 32 31.3, with 64 27.3, 1,000 rows 26.5, 19.4, 27.4, 500 rows 15.5, 17.0, 24.1.
+// (Alone, operands cold.  In a prompt of 4,001 rows, traced, 63 -> 54.9 and 54.7.)
 template <bool GATED, int RT>
 __global__ void __launch_bounds__(kThreads, 2)
 head_product_rows_kernel(bf16_t *__restrict__ out, int out_stride, int out_hstride, const bf16_t *__restrict__ in,

@@ -1703,8 +1703,8 @@ attn_decode_kernel(bf16_t *__restrict__ out, float *__restrict__ part_o, float *
 // 64 bytes of a line at a time, are slower), and 5 us of look-ups, sums and merges.  Measured with the merging kernel, us, a grid over rows
 // and chunks and so (28 heads of 128 on 4 unless said): 48 rows of 8 to 4,000 keys 61.4 -> 23.0; 64 rows of 60 to 4,000 66.4 -> 39.6; 16 rows
 // of 100 to 16,000 73.9 -> 44.3; 12 heads on 2, 41 rows of 60 to 3,000 24.3 -> 17.5; 16 on 2, 96 rows of 60 to 4,000 63.0 -> 30.1; 32 on 32,
-// 16 rows of 100 to 4,000 93.9 -> 67.8; rows of one length: 32 rows of 8,000 110.5 -> 109.3, 64 of 2,048 53.3 -> 56.4, 128 of 1,000
-// 53.2 -> 54.2, one of 131,000 57.1 -> 55.3.
+// 16 rows of 100 to 4,000 93.9 -> 67.8; one row of 131,000 57.1 -> 55.3.  Many rows of one length gain nothing by being dealt out (64 of 2,048
+// 53.3 -> 57.4): they come in equal chunks, where the caller says so (like_cut) or the table is short (equal_chunks).
 struct DecodePlan {
   int share;        // pages of a wave, in kShareParts of a page: whole pages would leave a third of the places empty just past one
   int up;           // what row_chunks rounds with

@@ -33,8 +33,11 @@ __device__ __forceinline__ uint4 ld16(const void *p, bool ok) {
 // few rows, which no other block wants and no cache holds until the next step.  Measured, replayed graphs, weights cold, without
 // and with it (us): gated 18,944 x 3,584 of 8 rows 53.8 -> 48.7, 3,584 x 18,944 26.5 -> 25.2, gated 11,008 x 2,048 of 2 rows
 // 20.8 -> 19.6, gated 4,864 x 896 of one row 7.6 -> 7.2, 1,536 x 8,960 of 48 rows 11.0 -> 10.7; a plain read of 272 MB in the same
-// order of addresses 46.8 -> 41.9.  Only weights that one launch after another reads from L2 lose by it (8.7 MB again and again
-// 3.1 -> 4.5), which no model does.
+// order of addresses 46.8 -> 41.9.  Weights that stay in a cache from one step to the next lose by it, 8.7 MB read again and again by one
+// product 3.1 -> 4.5.  Whole decode steps, us, at 1, 8 and 24 rows: models of 42 MB 198 -> 190, 217 -> 208, 281 -> 283; 84 MB 337 -> 332, 367 ->
+// 372, 468 -> 481; 176 MB 353 -> 358, 380 -> 389, 495 -> 507; 251 MB 460 -> 447, 509 -> 497, 674 -> 649; 459 MB 736 -> 657, 772 -> 718, 1,033 ->
+// 991; 988 MB 832 -> 748, 883 -> 840, 1,126 -> 1,133.  What loses is not told by a matrix (those of 176 and 251 MB are the same, in other
+// numbers), so the policy is one for all.
 constexpr int kReadOnce = 2;
 
 // Two floats to two bf16 packed in 32 bits (low half first), round to nearest even: one
