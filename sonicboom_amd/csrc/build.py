@@ -39,7 +39,7 @@ FLAGS = [
 CORE_SOURCES = [
     "status.hip", "embed_norm.hip", "elementwise.hip", "gemm_plain.hip", "rope_kv.hip",
     "attention_plain.hip", "sampling.hip", "gemm_skinny.hip", "gemm_stream.hip", "gemm_split.hip", "gemm_rows.hip", "gemm_mfma.hip",
-    "random_fill.hip", "recurrent.hip", "attention_latent.hip", "attention_latent_mfma.hip",
+    "random_fill.hip", "recurrent.hip", "attention_latent.hip", "attention_latent_mfma.hip", "attention_built.hip",
     "outnorm.hip", "headnorm_kv.hip", "moe.hip", "moe_mfma.hip", "timeconv.hip", "state_space.hip",
     "attention_mixed.hip", "join.hip", "decay_scan.hip", "decay_chunks.hip", "streams.hip", "rownorm.hip", "gated_lru.hip",
     "dense_layers.hip",

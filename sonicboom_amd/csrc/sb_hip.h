@@ -249,6 +249,24 @@ int sb_latent_attention_bf16(void *out, const void *q, const void *cache, const 
                              int n_tiles, int heads, int rank, int rot_dim, float scale, int window,
                              int tile_rows, int n_splits, float *part_o, float *part_ml, int n_rows, void *stream);
 
+/* Attention of prompts over built keys and values (csrc/attention_built.hip), everything bfloat16.
+ * sb_built_gather: pages int32 [n_pages, 4] = (sequence, page of the sequence, first key, end of the keys) -> out
+ *   [n_pages * SB_PAGE][rank], the first rank numbers of the cached rows; keys outside [first, end) and pages that
+ *   are not there are zeros.
+ * sb_built_attention: built [keys][built_stride], the key of head a at a * dim, its value at heads * dim + a * vdim;
+ *   rotated key parts behind the first rank numbers of the cached rows; q_plain [n_rows, heads, dim], q_rot: row r,
+ *   head a at (r * heads + a) * q_rot_stride; tiles int32 [n_tiles, 8] = (first row, rows <= sb_built_tile_rows(),
+ *   sequence, the built row that the sequence's key 0 would have, position of the first row, 0, 0, 0); out [n_rows, heads, vdim], times sigmoid(gate) as in
+ *   sb_head_product_gated_bf16 unless gate is NULL. */
+int sb_built_attention_ok(int dim, int rot_dim, int vdim, int rank);
+int sb_built_tile_rows(void);
+int sb_built_gather(void *out, const void *cache, const int32_t *page_table, int max_pages, int n_pages_total,
+                    const int32_t *pages, int n_pages, int rank, int rot_dim, void *stream);
+int sb_built_attention(void *out, const void *q_plain, const void *q_rot, int q_rot_stride, const void *built, int built_stride,
+                       const void *cache, const int32_t *page_table, int max_pages, int n_pages_total,
+                       const int32_t *tiles, int n_tiles, int heads, int dim, int rot_dim, int vdim, int rank, float scale,
+                       int window, const float *gate, int gate_stride, int gate_per_head, void *stream);
+
 /* ---- norms on what a sublayer gives back, an embedding with positions (csrc/outnorm.hip) --------
  * un(v) = v / sqrt(mean(v^2) + eps) * (offset + w): offset 1 for weights kept as multiplier minus one.
  * sb_offset_norm: y[r,:] = un(x[rows ? rows[r] : r,:]).

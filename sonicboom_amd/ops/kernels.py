@@ -16,6 +16,7 @@ import threading
 
 from typing import Optional, Sequence
 
+import numpy as np
 import torch
 
 from . import library
@@ -1336,6 +1337,13 @@ LATENT_SPLIT_BLOCKS = 512       # blocks a step of few rows aims at by sharing o
 LATENT_SPLIT_KEYS = 128         # keys a share has at least (64: 45 us, 128: 41, 256: 50 for 8 rows over 2,049 keys of 576 numbers)
 
 
+def latent_splits(blocks: int, max_keys: int) -> int:
+    """Shares of every run's keys in a launch of ``blocks`` blocks whose rows see at most ``max_keys``."""
+    if max_keys > LATENT_SPLIT_KEYS and 0 < blocks < LATENT_SPLIT_BLOCKS:
+        return max(1, min(-(-LATENT_SPLIT_BLOCKS // blocks), max_keys // LATENT_SPLIT_KEYS))
+    return 1
+
+
 def latent_attention_mfma(q: torch.Tensor, cache: torch.Tensor, page_table: torch.Tensor, row_pos: torch.Tensor,
                           tiles: torch.Tensor, rank: int, scale: float, window: int, single_rows: bool,
                           max_keys: int = 0) -> torch.Tensor:
@@ -1354,9 +1362,7 @@ def latent_attention_mfma(q: torch.Tensor, cache: torch.Tensor, page_table: torc
         raise KernelLibraryError("the page table must be int32 [sequences, pages]")
     out = torch.empty((n, heads, rank), dtype=q.dtype, device=q.device)
     blocks = tiles.shape[0] * -(-heads // (64 if single_rows else 4))
-    splits = 1
-    if max_keys > LATENT_SPLIT_KEYS and 0 < blocks < LATENT_SPLIT_BLOCKS:
-        splits = max(1, min(-(-LATENT_SPLIT_BLOCKS // blocks), max_keys // LATENT_SPLIT_KEYS))
+    splits = latent_splits(blocks, max_keys)
     part_o = part_ml = None
     if splits > 1:
         part_o = torch.empty((splits, n, heads, rank), dtype=torch.float32, device=q.device)
@@ -1379,6 +1385,106 @@ def latent_attention(q: torch.Tensor, cache: torch.Tensor, page_table: torch.Ten
                                      window, single_rows=bool(ctx.is_decode),
                                      max_keys=min(keys, window) if window > 0 else keys)
     return latent_attention_plain(q, cache, page_table, ctx.row_pos, ctx.row_seq, rank, scale, window)
+
+
+BUILT_ROW_TILE = 128        # rows of a run that a block of the kernel over built keys takes (sb_built_tile_rows)
+BUILT_LEAST_HEADS = 4       # fewer gain 7 to 17 us a layer (2 heads, 330 rows 40.6 -> 28.5) and stay with the roundings of their decode steps
+BUILT_MOST_BYTES = 2 << 30  # of built keys and values (and the latents they are built from) that a step's layer may hold
+
+
+def latent_built_ok(act_dtype, cache_dtype, dim: int, rot_dim: int, vdim: int, rank: int) -> bool:
+    """Whether prompts of these heads may build keys and values (:func:`latent_built_attention`)."""
+    return act_dtype == torch.bfloat16 and cache_dtype == torch.bfloat16 \
+        and bool(library.core().sb_built_attention_ok(int(dim), int(rot_dim), int(vdim), int(rank)))
+
+
+def latent_built_pays(n_new, before, window: int, heads: int, dim: int, rot_dim: int, vdim: int, rank: int) -> bool:
+    """Whether a step of ``n_new[i]`` rows behind ``before[i]`` cached ones is faster with every head's keys and values built
+    than in the latent's space: a price of both in microseconds.  Built: three launches, the longest run's pages at 1.25 us (two a
+    turn) or all pages at 1.5 us a page, run and CU, and the product that builds.  In the latent's space: three launches, the
+    arithmetic of the pairs or the longest share's pages, the per-head products and, where keys are shared out, the partial
+    results' way through memory (:func:`latent_attention_mfma`).  Measured on heads of 128 + 64 and 128 of a latent of 512, 6, 16 and
+    32 heads, 2 to 1,500 rows behind 0 to 12,000 (latent's space / built, us, 16 heads): 40 rows 31.9 / 23.0, behind 400 42.3 / 31.6,
+    behind 1,200 48.9 / 60.5; 250 43.7 / 28.7, behind 1,200 78.1 / 69.4, behind 3,500 104 / 122; 600 110 / 42, behind 3,500 214 / 141;
+    12 x 60 rows behind 150 63.1 / 47.2, 12 x 3 there 31.7 / 46.2; 4,001 rows 490 / 159.  Over 186 such steps the choice is 0.5 %
+    behind the better side on the mean."""
+    n, k = np.asarray(n_new, dtype=np.int64), np.asarray(before, dtype=np.int64)
+    first = np.maximum(k - window + 1, 0) if window > 0 else np.zeros_like(k)
+    pages = (k + n - 1) // PAGE - first // PAGE + 1
+    keys = int(pages.sum()) * PAGE
+    per_key = heads * (dim + vdim)
+    if heads < BUILT_LEAST_HEADS or keys * (per_key + rank) * 2 > BUILT_MOST_BYTES:
+        return False
+    seen = (k + 1 + k + n) / 2.0                                    # by a row, on the mean
+    most = k + n
+    if window > 0:
+        seen, most = np.minimum(seen, window), np.minimum(most, window)
+    pairs, rows, longest = float((n * seen).sum()), int(n.sum()), int(most.max())
+    runs = -(-n // BUILT_ROW_TILE)
+    tile_pages = float((runs * (seen / PAGE + 1.0)).sum())
+    product = 2.0 * (dim + vdim) * rank * heads
+    built = 19.5 + max(1.25 * (longest / PAGE + 1), 1.5 * tile_pages * heads / SPLIT_CUS) + keys * product / 5.5e8
+    blocks = int((-(-n // LATENT_ROW_TILE)).sum()) * -(-heads // 4)
+    splits = latent_splits(blocks, longest)
+    plain = 25.0 + max(1.8 * (longest / PAGE / splits), pairs * heads * 2.0 * (2 * rank + rot_dim) / 6.5e8) + rows * product / 3.5e8
+    if splits > 1:
+        plain += 9.0 + splits * rows * heads * rank * 8.0 / 4e6
+    return bool(built < plain)
+
+
+def latent_built_plan(n_new, before, window: int):
+    """(tiles int32 [n, 8], pages int32 [m, 4]) of :func:`latent_built_attention` as NumPy arrays: the pages that a step's rows
+    see, sequence after sequence, and the rows in runs of up to BUILT_ROW_TILE, longest first."""
+    tiles, pages, work, row0 = [], [], [], 0
+    for i, (n, k) in enumerate(zip(n_new, before)):
+        lo = max(k - window + 1, 0) if window > 0 else 0
+        p0, p1 = lo // PAGE, (k + n - 1) // PAGE
+        key0 = (len(pages) - p0) * PAGE
+        pages += [(i, p, max(lo - p * PAGE, 0), min(k + n - p * PAGE, PAGE)) for p in range(p0, p1 + 1)]
+        for r in range(0, n, BUILT_ROW_TILE):
+            rows = min(BUILT_ROW_TILE, n - r)
+            tiles.append((row0 + r, rows, i, key0, k + r, 0, 0, 0))
+            a = max(k + r - window + 1, 0) if window > 0 else 0
+            work.append((k + r + rows - 1) // PAGE - a // PAGE + 1)
+        row0 += n
+    order = sorted(range(len(tiles)), key=lambda t: -work[t])
+    return np.asarray([tiles[t] for t in order], dtype=np.int32).reshape(-1, 8), np.asarray(pages, dtype=np.int32).reshape(-1, 4)
+
+
+def latent_built_attention(q_plain: torch.Tensor, q_latent: torch.Tensor, build, cache: torch.Tensor, page_table: torch.Tensor,
+                           tiles: torch.Tensor, pages: torch.Tensor, rank: int, vdim: int, scale: float, window: int,
+                           gate: Optional[torch.Tensor] = None, gate_per_head: bool = False) -> torch.Tensor:
+    """Latent attention of a prompt's rows with keys and values built: ``q_plain`` [rows, heads, dim], ``q_latent`` [rows, heads,
+    rank + rot_dim] of which the rotated parts count, ``build``: the product from latents to [all heads' keys | all heads'
+    values]; ``tiles`` and ``pages`` as :func:`latent_built_plan` lays them out.  Returns [rows, heads, vdim], times the
+    sigmoid of the gate."""
+    _dev(q_plain, q_latent, cache, page_table, tiles, pages)
+    _on_gpu(gate)
+    n, heads, dim = q_plain.shape
+    latent = q_latent.shape[2]
+    if cache.dim() != 3 or cache.shape[1] != PAGE or cache.shape[2] != latent or tuple(q_latent.shape[:2]) != (n, heads):
+        raise KernelLibraryError("latent attention takes q [rows, heads, latent] and a cache [pages, PAGE, latent]")
+    for t, columns in ((tiles, 8), (pages, 4)):
+        if t.dtype != torch.int32 or t.dim() != 2 or t.shape[1] != columns:
+            raise KernelLibraryError("runs of rows must be int32 [n, 8], pages int32 [n, 4]")
+    if page_table.dtype != torch.int32 or page_table.dim() != 2:
+        raise KernelLibraryError("the page table must be int32 [sequences, pages]")
+    if gate is not None and (gate.dtype != torch.float32 or gate.dim() != 2 or gate.shape[0] != n or gate.stride(1) != 1
+                             or gate.shape[1] < (heads if gate_per_head else heads * vdim)):
+        raise KernelLibraryError("the gate must be float32 [rows, heads * out] (or [rows, heads], a number a head)")
+    lib = library.core()
+    c = torch.empty((pages.shape[0] * PAGE, rank), dtype=cache.dtype, device=cache.device)
+    check(lib.sb_built_gather(_p(c), _p(cache), _p(page_table), page_table.shape[1], cache.shape[0], _p(pages), pages.shape[0],
+                              rank, latent - rank, _stream()))
+    built = build(c)
+    if built.dtype != torch.bfloat16 or built.dim() != 2 or built.shape[0] != c.shape[0] or not built.is_contiguous():
+        raise KernelLibraryError("the built keys and values must be bfloat16 [keys, heads * (dim + vdim)]")
+    out = torch.empty((n, heads, vdim), dtype=q_plain.dtype, device=q_plain.device)
+    check(lib.sb_built_attention(_p(out), _p(q_plain), q_latent.data_ptr() + 2 * rank, latent, _p(built), built.shape[1], _p(cache),
+                                 _p(page_table), page_table.shape[1], cache.shape[0], _p(tiles), tiles.shape[0], heads, dim,
+                                 latent - rank, vdim, rank, float(scale), int(window), _p(gate), 0 if gate is None else gate.stride(0),
+                                 1 if gate_per_head else 0, _stream()))
+    return out
 
 
 # --------------------------------------------------------------------------

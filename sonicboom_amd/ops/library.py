@@ -59,6 +59,10 @@ _CORE_SIGNATURES = {
     "sb_head_product_bf16": [_P, _I, _I, _P, _I, _I, _P, _P, _I, _I, _I, _I, _I, _P],
     "sb_latent_attention_tile_rows": [],
     "sb_latent_attention_bf16_ok": [_I, _I],
+    "sb_built_attention_ok": [_I, _I, _I, _I],
+    "sb_built_tile_rows": [],
+    "sb_built_gather": [_P, _P, _P, _I, _I, _P, _I, _I, _I, _P],
+    "sb_built_attention": [_P, _P, _P, _I, _P, _I, _P, _P, _I, _I, _P, _I, _I, _I, _I, _I, _I, _F, _I, _P, _I, _I, _P],
     "sb_offset_norm": [_P, _I, _P, _P, _I, _P, _I, _I, _F, _F, _P],
     "sb_norm_add": [_P, _P, _I, _P, _I, _Z, _Z, _P, _I, _P, _P, _I, _P, _I, _I, _I, _F, _F, _I, _P],
     "sb_scale": [_P, _F, _Z, _P],

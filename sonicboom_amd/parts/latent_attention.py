@@ -10,7 +10,8 @@
 The cache holds the row [c | r] per token (a cache of rows, one "head" for all query heads), and
 the kernels work in that space: W_uk,a carries head a's plain query part into the latent space,
 attention runs over the cached rows, and W_uv,a (with the output gate) brings the result back
-(csrc/attention_latent.hip).  The input projections (queries, output gate, and the latent's
+(csrc/attention_latent.hip).  Steps that bring many rows a key they see build the heads' keys and
+values of those keys instead, for the layer (csrc/attention_built.hip).  The input projections (queries, output gate, and the latent's
 projection when the layer has one) are one stacked matrix.  A layer may read the rows another
 layer stores (an order entry that does not write its cache): it then has no W_dkv, and its own
 queries, W_uk, W_uv, window and scale.  The rotation is a nested position part of a rotary kind;
@@ -24,6 +25,7 @@ from __future__ import annotations
 
 from typing import Optional
 
+import numpy as np
 import torch
 
 from .. import ops
@@ -108,6 +110,10 @@ class LatentAttention(Mixer):
         wdt = rt.act_dtype
         self.uk = tensors["uk_weight"].to(wdt).reshape(H, self.dim, self.rank).transpose(1, 2).contiguous()
         self.uv = tensors["uv_weight"].to(wdt).reshape(H, self.vdim, self.rank).contiguous()
+        # for steps that build keys and values: both matrices stacked, a product's operand
+        self.ukv = None
+        if rt.fast_kernels and ops.latent_built_ok(wdt, rt.cache_dtype, self.dim, self.rot_dim, self.vdim, self.rank):
+            self.ukv = Linear(torch.cat([tensors["uk_weight"], tensors["uv_weight"]], dim=0).to(wdt), None, True)
         # the matrix-core attention kernel takes a prompt step's rows in runs of this many
         if rt.fast_kernels and ops.latent_attention_mfma_ok(rt.act_dtype, rt.cache_dtype, self.rank, self.rot_dim):
             self.row_tile = ops.LATENT_ROW_TILE
@@ -136,9 +142,31 @@ class LatentAttention(Mixer):
             bool(self.position.interleaved), ctx.row_pos, ctx.row_seq, cache if writes else None,
             table if writes else None, self.heads, self.dim, self.rot_dim, self.rank, kv_rows=kv_rows,
             magnitude=self.magnitude)
+        gate = pre[:, self.g_off:self.g_off + self.gate_cols]
+        plan = self._built_plan(ctx)
+        if plan is not None:
+            a = ops.latent_built_attention(q_plain, q_lat, lambda c: self.ukv(c, rt.act_dtype), cache, table, *plan[:2],
+                                           self.rank, self.vdim, self.scale, self.window, gate, self.gate_per_head)
+            return self.out.add_into(a.view(a.shape[0], -1), x, then_norm, rt.act_dtype, scale=self.out_scale)
         ops.head_product(q_plain, self.uk, q_lat, fast=rt.fast_kernels)     # the first rank numbers of every head's query
         a_lat = ops.latent_attention(q_lat, cache, table, ctx, self.rank, self.scale, self.window, fast=rt.fast_kernels)
         a = torch.empty((a_lat.shape[0], self.heads, self.vdim), dtype=rt.act_dtype, device=a_lat.device)
-        gate = pre[:, self.g_off:self.g_off + self.gate_cols]
         ops.head_product(a_lat, self.uv, a, gate=gate, fast=rt.fast_kernels, gate_per_head=self.gate_per_head)
         return self.out.add_into(a.view(a.shape[0], -1), x, then_norm, rt.act_dtype, scale=self.out_scale)
+
+    def _built_plan(self, ctx):
+        """(runs of rows, pages, their host copies) on the device when the step is faster with keys and values built, else None.
+        Layers of one window share a step's plan."""
+        if self.ukv is None or ctx.is_decode:
+            return None
+        shared = ctx.shared if ctx.shared is not None else {}
+        key = ("latent_built", self.window, self.heads, self.dim, self.rot_dim, self.vdim, self.rank)
+        if key not in shared:
+            shared[key] = None
+            if ops.latent_built_pays(ctx.n_new, ctx.lengths_before, self.window, self.heads, self.dim, self.rot_dim, self.vdim, self.rank):
+                tiles, pages = ops.latent_built_plan(ctx.n_new, ctx.lengths_before, self.window)
+                host = torch.empty(tiles.size + pages.size, dtype=torch.int32, pin_memory=True)
+                host.numpy()[...] = np.concatenate([tiles.ravel(), pages.ravel()])
+                dev = host.to(ctx.row_pos.device, non_blocking=True)
+                shared[key] = (dev[:tiles.size].view(-1, 8), dev[tiles.size:].view(-1, 4), host)
+        return shared[key]
