@@ -1,0 +1,30 @@
+"""Float32 products in chains of 256 k, gated products whose weights pass through registers, xIELU as a pass and on a product's way out."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV, F32, BF16 = "cuda:0", torch.float32, torch.bfloat16
+
+
+def randn(*shape, seed=0, scale=1.0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)) * scale
+
+
+@pytest.mark.parametrize("t", [1, 16, 20, 70])
+@pytest.mark.parametrize("n, k", [(40, 256), (40, 260), (33, 768), (33, 1024), (48, 1280), (16, 2304)])
+def test_float32_chains_end_inside_and_between_segments(t, n, k):
+    """One to nine chains of 256 k in up to three segments: the same bits from every kernel, within a chain's roundings of 64 bits."""
+    from sonicboom_amd import ops
+    x, w = randn(t, k, seed=t), randn(n, k, seed=k, scale=0.05)
+    want = ops.gemm_plain(x.to(DEV), w.to(DEV), None, None, F32)
+    got = ops.gemm_f32(x.to(DEV), ops.pack_weight_f32(w.to(DEV)), None, None, F32, (n, k))
+    assert torch.equal(got, want)
+    # each of at most 256 + 4 + 3 roundings is half a unit of a running sum that the terms' absolute values bound
+    bound = (256 + 4 + 3) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    assert ((got.cpu().double() - x.double() @ w.double().T).abs() <= bound).all()
+    if n % 2 == 0:
+        gated = ops.gemm_f32(x.to(DEV), ops.pack_weight_f32(w.to(DEV), True), None, None, F32, (n, k), gated="silu")
+        assert torch.equal(gated, ops.silu_mul(want, F32))
