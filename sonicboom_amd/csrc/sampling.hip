@@ -162,8 +162,22 @@ __device__ __forceinline__ uint64_t select_kth(const uint64_t (&mine)[PER], int 
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const uint64_t key = mine[j];
-      if (pass == 7 || (key >> (shift + 8)) == (prefix >> (shift + 8)))
-        atomicAdd(&sh.hist[wave][(key >> shift) & 0xffu], 1u);
+      const uint32_t bucket = uint32_t(key >> shift) & 0xffu;
+      bool counts = pass == 7 || (key >> (shift + 8)) == (prefix >> (shift + 8));
+      // Logits agree in sign and mostly in the exponent: lanes that add to one counter do so one after the other, so up to two
+      // buckets of a wave's keys are counted by a vote first.  (With the ranks below, the second stage of three rows of 32,768
+      // logits takes 14.0 us for 25.4.)
+#pragma unroll
+      for (int vote = 0; vote < 2; ++vote) {
+        const uint64_t left = __ballot(counts);
+        if (left == 0) break;
+        const int leader = __ffsll((unsigned long long)left) - 1;
+        const uint32_t its = __builtin_amdgcn_readlane(bucket, leader);
+        const uint64_t same = __ballot(counts && bucket == its);
+        if (lane == leader) atomicAdd(&sh.hist[wave][its], uint32_t(__popcll(same)));
+        counts = counts && bucket != its;
+      }
+      if (counts) atomicAdd(&sh.hist[wave][bucket], 1u);
     }
     __syncthreads();
     // thread b < 256 owns bucket b: its count, and by a suffix sum over the wave and the waves
@@ -236,7 +250,7 @@ top_candidates_kernel(int32_t *__restrict__ cand_id, float *__restrict__ cand_z,
                       const float *__restrict__ logits, const uint64_t *__restrict__ part_keys, int n_keys,
                       int vocab, int k, float temperature) {
   __shared__ SelectShared sh;
-  __shared__ uint64_t sel[kMaxCand];
+  __shared__ uint64_t sel[kMaxCand], ordered[kMaxCand];
   __shared__ int count_s;
   const float *x = logits + size_t(blockIdx.x) * vocab;
   const uint64_t *pk = part_keys + size_t(blockIdx.x) * n_keys;
@@ -260,24 +274,22 @@ top_candidates_kernel(int32_t *__restrict__ cand_id, float *__restrict__ cand_z,
     }
   __syncthreads();
 
-  // Bitonic sort of 256 keys, descending; empty slots (0) sink to the end.
-  for (int size = 2; size <= kMaxCand; size <<= 1) {
-    for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      if (tid < kMaxCand / 2) {
-        const int lo = ((tid / stride) * stride * 2) + (tid % stride);
-        const int hi = lo + stride;
-        const bool descending = ((lo & size) == 0);
-        const uint64_t a = sel[lo], b = sel[hi];
-        if (descending ? (a < b) : (a > b)) {
-          sel[lo] = b;
-          sel[hi] = a;
-        }
-      }
-      __syncthreads();
-    }
+  // Descending order: a key's place is the count of larger ones (no two are equal), four threads a key, each a quarter of the
+  // keys (sorting them in steps of compare and exchange took 36 barriers of the whole block).
+  static_assert(kSelThreads == 4 * kMaxCand, "four threads a key");
+  {
+    const uint64_t own = sel[tid >> 2];
+    const int quarter = tid & 3;
+    int larger = 0;
+#pragma unroll 16
+    for (int i = 0; i < kMaxCand / 4; ++i) larger += int(sel[4 * i + quarter] > own);
+    larger += __shfl_xor(larger, 1, 64);
+    larger += __shfl_xor(larger, 2, 64);
+    if (quarter == 0 && own != 0) ordered[larger] = own;
   }
+  __syncthreads();
   for (int i = tid; i < k; i += kSelThreads) {
-    const uint64_t key = sel[i];
+    const uint64_t key = ordered[i];
     const bool real = i < want;
     cand_id[size_t(blockIdx.x) * k + i] = real ? int32_t(0xffffffffu - uint32_t(key)) : -1;
     cand_z[size_t(blockIdx.x) * k + i] = real ? key_float(uint32_t(key >> 32)) : 0.0f;
@@ -314,8 +326,6 @@ __global__ void __launch_bounds__(64)
 draw_kernel(int32_t *__restrict__ token, const int32_t *__restrict__ cand_id, const float *__restrict__ cand_z,
             const POS *__restrict__ position, int64_t position_offset, int k, int top_k, int use_min_p,
             float log_min_p, int use_top_p, double top_p, uint64_t seed) {
-  __shared__ double e_of[kMaxCand];
-  __shared__ int n_keep_sh;
   const int row = blockIdx.x, lane = threadIdx.x;
   const int32_t *ids = cand_id + size_t(row) * k;
   const float *zs = cand_z + size_t(row) * k;
@@ -340,30 +350,33 @@ draw_kernel(int32_t *__restrict__ token, const int32_t *__restrict__ cand_id, co
     keep = kept;
   }
   if (use_top_p && keep > 0) {
+    // running sums in order, by all lanes alike; a lane keeps those of its own candidates and looks at all of them at once (one lane
+    // that added, divided and compared in turn: 11.3 us for 7.8 at 50 candidates)
+    double e[kDrawPerLane], upto[kDrawPerLane], total = 0.0;
 #pragma unroll
     for (int j = 0; j < kDrawPerLane; ++j) {
-      const int c = lane + 64 * j;
-      if (c < keep) e_of[c] = exp(double(z[j]) - double(m));
+      e[j] = lane + 64 * j < keep ? exp(double(z[j]) - double(m)) : 0.0;
+      upto[j] = 0.0;
     }
-    __syncthreads();
-    if (lane == 0) {
-      double total = 0.0;
-      for (int c = 0; c < keep; ++c) total += e_of[c];
-      int n = keep;
-      if (total > 0.0) {
-        double acc = 0.0;
-        for (int c = 0; c < keep; ++c) {
-          acc += e_of[c];
-          if (acc / total >= top_p) {
-            n = c + 1;
-            break;
-          }
-        }
+#pragma unroll
+    for (int j = 0; j < kDrawPerLane; ++j) {
+      const int here = min(keep - 64 * j, 64);
+      const uint64_t bits = __builtin_bit_cast(uint64_t, e[j]);
+      for (int c = 0; c < here; ++c) {
+        const uint32_t lo = __builtin_amdgcn_readlane(uint32_t(bits), c), hi = __builtin_amdgcn_readlane(uint32_t(bits >> 32), c);
+        total += __builtin_bit_cast(double, uint64_t(hi) << 32 | lo);
+        if (lane == c) upto[j] = total;
       }
-      n_keep_sh = n;
     }
-    __syncthreads();
-    keep = n_keep_sh;
+    if (total > 0.0) {
+      int n = keep;
+#pragma unroll
+      for (int j = kDrawPerLane - 1; j >= 0; --j) {
+        const uint64_t reached = __ballot(lane + 64 * j < keep && upto[j] / total >= top_p);
+        if (reached) n = 64 * j + __ffsll((unsigned long long)reached);
+      }
+      keep = n;
+    }
   }
   double best = -__builtin_inf();
   int best_id = 0x7fffffff;
