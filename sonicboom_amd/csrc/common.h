@@ -97,6 +97,35 @@ __device__ __forceinline__ float sum_slices(const float *p, int n_slices, size_t
   return v;
 }
 
+__device__ __forceinline__ float softplus_f(float a) { return a > 20.0f ? a : log1pf(expf(a)); }
+
+// exp(z) - 1 - z for z <= 0: near zero the series z^2 (1/2! + z/3! + ..), whose terms from z^12 on are below the last digit, without
+// the digits that expm1(z) - z loses there; further down the exponential itself, the smaller part of the result.
+__device__ __forceinline__ float exp_rest(float z) {
+  float p = 1.0f / 39916800.0f;
+  p = fmaf(p, z, 1.0f / 3628800.0f);
+  p = fmaf(p, z, 1.0f / 362880.0f);
+  p = fmaf(p, z, 1.0f / 40320.0f);
+  p = fmaf(p, z, 1.0f / 5040.0f);
+  p = fmaf(p, z, 1.0f / 720.0f);
+  p = fmaf(p, z, 1.0f / 120.0f);
+  p = fmaf(p, z, 1.0f / 24.0f);
+  p = fmaf(p, z, 1.0f / 6.0f);
+  p = fmaf(p, z, 0.5f);
+  const float far = (__builtin_amdgcn_exp2f(z * 1.4426950408889634f) - 1.0f) - z;
+  return z > -1.0f ? p * z * z : far;
+}
+
+// xIELU with the two numbers (p, q) of a layer: for z > 0 softplus(p) z^2 + z/2, else
+// (1/2 + softplus(q)) (exp(z) - 1 - z) + z/2.
+__device__ __forceinline__ float xielu(float z, float rise, float bend) {
+  return z > 0.0f ? rise * z * z + 0.5f * z : bend * exp_rest(z) + 0.5f * z;
+}
+__device__ __forceinline__ void xielu_numbers(const void *params, int dtype, float &rise, float &bend) {
+  rise = softplus_f(ld_dyn(params, dtype, 0));
+  bend = 0.5f + softplus_f(ld_dyn(params, dtype, 1));
+}
+
 // ---- wave (64 lanes) reductions with a fixed butterfly order -----------------
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -28,3 +28,23 @@ def test_float32_chains_end_inside_and_between_segments(t, n, k):
     if n % 2 == 0:
         gated = ops.gemm_f32(x.to(DEV), ops.pack_weight_f32(w.to(DEV), True), None, None, F32, (n, k), gated="silu")
         assert torch.equal(gated, ops.silu_mul(want, F32))
+
+
+def xielu(z, p, q):
+    z = z.double().numpy()
+    rise, bend = np.log1p(np.exp(p)), 0.5 + np.log1p(np.exp(q))
+    return np.where(z > 0, rise * z * z + z / 2, bend * (np.expm1(np.minimum(z, 0.0)) - np.minimum(z, 0.0)) + z / 2)
+
+
+@pytest.mark.parametrize("n", [3, 4096, (1 << 23) + 5])
+def test_xielu_against_64_bits(n):
+    """One group of four a thread and several, a tail; numbers around the two borders of its exponential."""
+    from sonicboom_amd import ops
+    z = randn(n, seed=n, scale=3.0)
+    z[:3] = torch.tensor([-1.0, -1e-3, -0.99999994])
+    z[n // 2:] *= 0.02
+    p = torch.tensor([0.4, -0.3])
+    got = ops.activate(z.to(DEV), F32, "xielu", p.to(DEV)).cpu().numpy().astype(np.float64)
+    want = xielu(z, 0.4, -0.3)
+    # some eight roundings of terms that the result and z / 2 bound
+    assert (np.abs(got - want) <= 8 * 2.0 ** -23 * (np.abs(want) + np.abs(z.numpy()))).all()
