@@ -1101,6 +1101,154 @@ gemm_pipe_half_kernel(Args a) {
   }
 }
 
+// ---------------------------------------------------------------------------------------------
+// The gated product of up to two hundred rows, whose weights are most of what there is to read.  What bounds it in the forms above
+// is how much of W a CU has on its way (three stages in LDS, beside X's): memory answers in some 2 us, and 48 KB in that time are
+// 24 GB/s a CU.  Here W never passes through LDS: a wave owns 16 columns of either half, whose packed blocks are the matrix
+// instruction's fragments as they lie, and keeps kDeep stages of 64 k of them in registers on their way.  Rows of X, which the block's four such
+// waves share, are brought into LDS by two waves that do nothing else: loads return in order, so that waiting for a stage of X
+// would also wait for the weights that were asked for before it.  One barrier a stage.
+// us, the form taken before and this one (rows x 2 halves of W x k): 183 x 17,920 x 1,536 26.0 and 22.4 (a read of W alone 11),
+// 96 rows 20.4 and 17.7, 192 x 22,016 x 2,048 32.7 and 28.4, 260 x 11,008 x 2,048 31.4 and 23.0, 288 x 9,728 x 896 12.6 and 9.2; prompts
+// of 288 rows of the 0.5B sizes 1,519 -> 1,454, 183 rows of the 1.5B ones 2,614 -> 2,514.  Tiles of 96 and 192 rows straight into LDS as
+// above were ahead by themselves (10.7 and 25.5) and not in whole steps.
+// RT: tiles of 16 rows of a block.  The weights are the first operand, so that a lane ends up with four neighbouring
+// columns of a row.
+template <int RT, int GATED>
+__global__ void __launch_bounds__(384)
+gemm_ahead_kernel(Args a) {
+  constexpr int kRows = 16 * RT, kBuf = kRows * 8, NB = 4, kDeep = 6;
+  static_assert(GATED != 0 && (NB - 2) * RT < 64, "the memory counter has six bits");
+  extern __shared__ bf16x8_t lds[];                    // [NB][row][8 chunks of 16 bytes, turned by the row]
+  typedef __attribute__((address_space(3))) bf16x8_t *lds_ptr_t;
+  int tm, tn;
+  if (!tile_of_block(a, int(blockIdx.x), tm, tn)) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n_k = a.n_in / 64, t0 = tm * kRows;
+  if (wave >= 4) {
+    const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<bf16_t *>(a.x), 0, uint32_t(size_t(a.n_rows) * a.n_in * 2), 0x00020000);
+    uint32_t off[RT];                                  // rows past the last lie past the descriptor's end: zeros
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      const int place = (2 * i + wave - 4) * 64 + lane, row = place / 8, c = (place % 8) ^ ((row / 2) & 7);
+      off[i] = uint32_t((size_t(t0 + row) * a.n_in + c * 8) * 2);
+    }
+    const auto bring = [&](int kt) {                   // (past the end: the last stage again, into a buffer that nobody reads)
+      const int from = min(kt, n_k - 1) * 128;
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_x, (lds_ptr_t)(lds) + (kt % NB) * kBuf + (2 * i + wave - 4) * 64, 16, int(off[i]),
+                                                 from, 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < NB - 1; ++s) bring(s);
+    for (int kt = 0; kt < n_k; ++kt) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * RT) : "memory");
+      __builtin_amdgcn_s_barrier();                    // stage kt is there, and stage kt - 1 has been read
+      asm volatile("" ::: "memory");
+      bring(kt + NB - 1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    return;
+  }
+  const int n_first = tn * 64 + 16 * wave;             // this wave's columns
+  const __amdgpu_buffer_rsrc_t rsrc_w = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<bf16_t *>(a.w), 0, uint32_t(size_t(2) * a.w_tiles * 16 * size_t(a.w_steps) * 64), 0x00020000);
+  uint32_t w_off[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) w_off[h] = uint32_t((size_t(h * a.w_tiles + n_first / 16) * a.w_steps * 512 + size_t(lane) * 8) * 2);
+  bf16x8_t w[kDeep][2][2];                             // [stage][32 k][half]
+  const auto ask = [&](int slot, int kt) __attribute__((always_inline)) {
+    const int from = min(kt, n_k - 1) * 2048;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        w[slot][j][h] = __builtin_bit_cast(bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(rsrc_w, int(w_off[h]), from + 1024 * j, 0));
+  };
+  floatx4_t acc[RT][2];
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) acc[i][h] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int s = 0; s < kDeep; ++s) {
+    ask(s, s);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  const int fr = lane & 15, fg = lane >> 4;
+  const int x_lane[2] = {fr * 8 + (fg ^ (fr / 2)), fr * 8 + ((4 + fg) ^ (fr / 2))};
+  const auto stage = [&](int u, int kt) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const bf16x8_t *ls = lds + (kt % NB) * kBuf;
+    bf16x8_t x[4];                                     // three tiles on their way out of LDS
+#pragma unroll
+    for (int i = 0; i < 3; ++i) x[i] = ls[x_lane[0] + i * 128];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 2 * RT; ++i) {
+      if (i + 3 < 2 * RT) x[(i + 3) & 3] = ls[x_lane[(i + 3) / RT] + (i + 3) % RT * 128];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) acc[i % RT][h] = mfma16(w[u][i / RT][h], x[i & 3], acc[i % RT][h]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  int kt = 0;
+  for (; kt + kDeep <= n_k; kt += kDeep) {
+#pragma unroll
+    for (int u = 0; u < kDeep; ++u) {
+      stage(u, kt + u);
+      ask(u, kt + kDeep + u);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kDeep; ++u)
+    if (kt + u < n_k) stage(u, kt + u);
+  // acc[i][h][e]: column n_first + 4 fg + e of row 16 i + fr
+  const bool far = silu_far<GATED, 4 * RT>([&](int i) { return acc[i / 4][0][i % 4]; });
+  const int n = n_first + 4 * fg;
+  const auto store = [&](auto FAR) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      const int t = t0 + 16 * i + fr;
+      if (t >= a.n_rows || n >= a.n_out) continue;
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = tile_gate<GATED, decltype(FAR)::value>(acc[i][0][e]) * acc[i][1][e];
+      const size_t at = size_t(t) * a.n_out + n;
+      if (a.y_dtype == SB_F32) *reinterpret_cast<floatx4_t *>((float *)a.y + at) = floatx4_t{v[0], v[1], v[2], v[3]};
+      else *reinterpret_cast<uint2 *>((bf16_t *)a.y + at) = make_uint2(pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3]));
+    }
+  };
+  if (GATED == SB_GATE_SILU && far) store(std::true_type{});
+  else store(std::false_type{});
+}
+
+template <int RT, int GATED>
+int launch_ahead_one(const Args &a, long long blocks, hipStream_t s) {
+  constexpr int lds_bytes = 4 * 16 * RT * 128;
+  static bool raised = false;     // per instantiation; harmless if repeated
+  if (lds_bytes > 48 * 1024 && !raised) {
+    const hipError_t e = hipFuncSetAttribute((const void *)gemm_ahead_kernel<RT, GATED>, hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
+    SB_REQUIRE(e == hipSuccess, "sb_gemm_mfma_bf16: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    raised = true;
+  }
+  gemm_ahead_kernel<RT, GATED><<<unsigned((blocks + kXcds - 1) / kXcds * kXcds), 384, lds_bytes, s>>>(a);
+  return SB_OK;
+}
+template <int RT>
+int launch_ahead(const Args &a, long long blocks, hipStream_t s) {
+  switch (a.gated) {
+    case 3: return launch_ahead_one<RT, 3>(a, blocks, s);
+    case 2: return launch_ahead_one<RT, 2>(a, blocks, s);
+    default: return launch_ahead_one<RT, 1>(a, blocks, s);
+  }
+}
+
 template <int MT, int NW, int BK, int DEPTH, int GATED, bool PACKED, bool EVEN_K>
 int launch_one(const Args &a, long long blocks, hipStream_t s) {
   constexpr int lds_bytes = 2 * (64 * MT + 64 * NW) * (BK / 8) * 16;
@@ -1223,7 +1371,8 @@ int launch_pipe(const Args &a, long long blocks, bool a_block_a_tile, hipStream_
 
 // Tile shapes the launcher chooses from: rows x columns of Y per block.
 struct Shape { int bm, bn; };
-constexpr Shape kShapes[6] = {{128, 128}, {256, 128}, {256, 256}, {128, 256}, {192, 256}, {64, 128}};
+constexpr Shape kShapes[9] = {{128, 128}, {256, 128}, {256, 256}, {128, 256}, {192, 256}, {64, 128},
+                              {96, 128}, {128, 128}, {192, 128}};      // (the last three: gated, weights through registers)
 
 // The tile shape for a problem: the one with the best product of three factors.  How fast the
 // shape's kernel runs on a full grid, relative to 128 x 128 (measured on MI355X at 2,048 to 16,384
@@ -1316,7 +1465,9 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
   // 0.33 us in tiles of 64 x 128 and 0.55 in 128 x 128, through registers 0.65 (600 rows against 2,560 x 2,048 15.9, 21.4 and 22.6
   // us; 400 against 4,608 x 3,584 25.2, 30.0 and 33.8, 600 there, 360 tiles of 64, 46.5, 34.7 and 38.0; gated, 183 against 9,728 x 896 10.8, 13.3 and
   // 14.6, 288 there 18.1, 13.3 and 15.1).  Gated, a little over one round: 64 x 128 tiles, three to a CU (183 rows against 17,920 x
-  // 1,536, 280 tiles of 128: 26.4 and 31.5).
+  // 1,536, 280 tiles of 128: 26.4 and 31.5).  Gated, past one round of tiles of 64 rows: the lowest of the tiles of 96, 128 and 192 whose
+  // weights pass through registers that makes one round (figures at gemm_ahead_kernel; 66 to 120 rows against 11,008 x 2,048, in one round of 64 x
+  // 128, 16.5 to 19.0 and 19.4 to 22.5 so).
   int path = 0;
   if (direct_ok && variant == 0) {
     const int bn = gated ? 64 : 128;
@@ -1324,6 +1475,9 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
     const auto one_round = [&](long long tiles) { return (tiles + kXcds - 1) / kXcds * kXcds <= sb::cu_count(); };
     const long long tiles = (long long)((n_rows + 127) / 128) * across;
     if (one_round((long long)((n_rows + 63) / 64) * across)) variant = 5, path = 2;
+    else if (gated && a.vec4 && one_round((long long)((n_rows + 95) / 96) * across)) variant = 6, path = 2;
+    else if (gated && a.vec4 && one_round(tiles)) variant = 7, path = 2;
+    else if (gated && a.vec4 && one_round((long long)((n_rows + 191) / 192) * across)) variant = 8, path = 2;
     else if (one_round(tiles)) path = 2;
     else if (gated && n_rows <= 384 && tiles <= sb::cu_count() * 3 / 2 && (n_rows + 63) / 64 * 64 < (n_rows + 127) / 128 * 128)
       variant = 5, path = 2;
@@ -1331,7 +1485,7 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
   // a test's or a measurement's choice: the shape (0..5) + 16 * the path (0: the launcher's, 1:
   // through registers, 2: straight into LDS)
   if (tile_shape >= 0) {
-    SB_REQUIRE((tile_shape & 15) < 6 && (tile_shape >> 4) < 4, "sb_gemm_mfma_bf16: unknown tile shape %d", tile_shape);
+    SB_REQUIRE((tile_shape & 15) < 9 && (tile_shape >> 4) < 4, "sb_gemm_mfma_bf16: unknown tile shape %d", tile_shape);
     variant = tile_shape & 15;
     path = tile_shape >> 4;
   }
@@ -1358,7 +1512,8 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
   // short for loads that run one stage ahead, and the register path, which runs two ahead, is
   // faster there unless the tiles make one round and LDS holds four stages of each (above)
   const bool direct = path >= 2 || (path == 0 && direct_ok && (variant == 1 || variant == 2 || variant == 4));
-  SB_SUPPORT(variant < 3 || direct, "sb_gemm_mfma_bf16: the shapes 128 x 256, 192 x 256 and 64 x 128 exist on the direct path only");
+  SB_SUPPORT(variant < 6 || (gated && a.vec4 && direct), "sb_gemm_mfma_bf16: the shapes whose weights pass through registers are gated ones");
+  SB_SUPPORT(variant < 3 || direct, "sb_gemm_mfma_bf16: the shapes from 128 x 256 on exist on the direct path only");
   if (direct) {
     // the shapes of four waves take as many buffers as the tiles' count leaves LDS for: four (a block a CU, three
     // stages in flight) in one round over the CUs, else two (two or three blocks a CU)
@@ -1368,6 +1523,9 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
     else if (variant == 2) rc = launch_pipe<false>(a, blocks, path == 3, s);      // (path 3: a measurement's)
     else if (variant == 3) rc = launch_direct<4, 4, 64, 2, false>(a, blocks, 0, s);
     else if (variant == 4) rc = launch_direct<6, 4, 64, 2, true>(a, blocks, sb::cu_count(), s);
+    else if (variant == 6) rc = launch_ahead<6>(a, blocks, s);
+    else if (variant == 7) rc = launch_ahead<8>(a, blocks, s);
+    else if (variant == 8) rc = launch_ahead<12>(a, blocks, s);
     else rc = one_round ? launch_direct<2, 2, 64, 4, false>(a, blocks, 0, s) : launch_direct<2, 2, 64, 2, false>(a, blocks, 0, s);
   } else {
     if (variant == 0) rc = launch<2, 2, 64, 2, true>(a, blocks, packed, s);

@@ -915,9 +915,9 @@ def gemm_bf16_activated(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.T
 def gemm_tile_shape(shape: Optional[int], path: Optional[str] = None):
     """For tests and measurements: inside the block the tiled products of this thread use tile
     shape ``shape`` (0: 128 x 128, 1: 256 x 128, 2: 256 x 256, 3: 128 x 256, 4: 192 x 256, 5: 64 x 128 outputs per
-    block) instead of choosing one, and with ``path`` the kernel that stages tiles through
-    "registers" or the one that loads them "direct" into LDS (packed weights, inner size in 64s;
-    the only one with shapes 3, 4 and 5)."""
+    block; 6, 7, 8: 96, 128 and 192 x 128 of a gated product whose weights pass through registers) instead of choosing one, and with
+    ``path`` the kernel that stages tiles through "registers" or the one that loads them "direct" into LDS (packed weights, inner
+    size in 64s; the only one with the shapes from 3 on)."""
     paths = {None: 0, "registers": 1, "direct": 2, "direct, a block a tile": 3}
     if path not in paths:
         raise ValueError(f"unknown path {path!r}")

@@ -30,6 +30,24 @@ def test_float32_chains_end_inside_and_between_segments(t, n, k):
         assert torch.equal(gated, ops.silu_mul(want, F32))
 
 
+@pytest.mark.parametrize("shape", [6, 7, 8])
+@pytest.mark.parametrize("t, inner, k", [(65, 64, 64), (96, 72, 320), (97, 132, 384), (129, 20, 448), (193, 260, 896), (400, 64, 192)])
+def test_gated_products_with_weights_through_registers(shape, t, inner, k):
+    """Rows and columns that end inside a tile, stage counts on either side of the ring of six."""
+    from sonicboom_amd import ops
+    x, w = randn(t, k, seed=t).to(BF16), randn(2 * inner, k, seed=k, scale=0.05).to(BF16)
+    gu = x.double() @ w.double().T
+    g, u = gu[:, :inner], gu[:, inner:]
+    packed = ops.pack_weight(w.to(DEV), True)
+    for act, want in (("silu", g / (1.0 + torch.exp(-g)) * u), ("relu", torch.relu(g) * u),
+                      ("gelu_tanh", 0.5 * g * (1 + torch.tanh(0.7978845608028654 * g * (1 + 0.044715 * g * g))) * u)):
+        with ops.gemm_tile_shape(shape, "direct"):
+            got = ops.gemm_bf16(x.to(DEV), packed, None, None, F32, gated=act, packed_shape=(2 * inner, k))
+            half = ops.gemm_bf16(x.to(DEV), packed, None, None, BF16, gated=act, packed_shape=(2 * inner, k))
+        assert ((got.cpu().double() - want).abs() <= 1e-4 * math.sqrt(k) + 1e-4 * want.abs()).all(), act
+        assert torch.equal(half, got.to(BF16)), act
+
+
 def xielu(z, p, q):
     z = z.double().numpy()
     rise, bend = np.log1p(np.exp(p)), 0.5 + np.log1p(np.exp(q))
