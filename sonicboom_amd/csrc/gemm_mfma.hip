@@ -77,6 +77,7 @@ struct Args {
   float resid_scale;   // Y = resid_scale * (X W^T + bias) + resid  (1 unless a branch has a multiplier)
   int n_rows, n_out, n_in;
   int relu_sq;     // 1: Y = max(X W^T + bias, 0)^2 (no residual, whole products)
+  const void *act_params; int act_dtype;      // xIELU's two numbers (kernels built for it)
   int gated;       // an sb_gate; not 0: W is [2*n_out, n_in], rows n (gate) and n_out + n (up)
   int tiles_m, tiles_n;
   int w_tiles;     // packed W: 16-row tiles of one half (ceil(n_out / 16))
@@ -730,7 +731,7 @@ gemm_direct16_kernel(Args a) {
 // the turns give 3 to 4 %.  Not kept: turns of 64 k (a wave's fragments then wait for W's loads, one stage ahead: 0.87 of
 // the speed), whole lines with one barrier a stage and no turns (3 to 4 % slower), loads between the products (2 to 5 %),
 // half of X's fragments read beside the products (6 to 10 %), s_setprio around the products (1 %).
-template <int GATED, bool PERSIST>
+template <int GATED, bool PERSIST, bool XIELU = false>
 __global__ void __launch_bounds__(512)
 gemm_pipe_kernel(Args a) {
   constexpr int MT16 = 8, NW = 4, BM = 256, BN = 256, kWaves = 8;
@@ -865,6 +866,8 @@ gemm_pipe_kernel(Args a) {
   static_assert(kBufA * 16 >= kWaves * 16 * kPitch * 4, "the turning areas must fit a buffer of X");
   auto epilogue = [&](int m, int n, int a_free) {
     const bool far = silu_far<GATED, 8 * MT16>([&](int i) { return acc[i / 8][i % 8 / 4][i % 4]; });
+    float rise = 0.0f, bend = 0.0f;
+    if constexpr (XIELU) xielu_numbers(a.act_params, a.act_dtype, rise, bend);
     store_tile<MT16, 16, NW, NC, kPitch, !GATED>(
         a, reinterpret_cast<float *>(lds + a_free * kBufA), m * BM, n * (GATED ? BN / 2 : BN), !GATED,
         [&](int i, float *turn) {
@@ -878,7 +881,7 @@ gemm_pipe_kernel(Args a) {
                   turn[row * kPitch + f * 16 + fr] = tile_gate<GATED, decltype(FAR)::value>(acc[i][f][e]) * acc[i][f + 2][e];
               } else {
 #pragma unroll
-                for (int f = 0; f < 4; ++f) turn[row * kPitch + (f ^ fg) * 16 + fr] = acc[i][f][e];
+                for (int f = 0; f < 4; ++f) turn[row * kPitch + (f ^ fg) * 16 + fr] = XIELU ? xielu(acc[i][f][e], rise, bend) : acc[i][f][e];
               }
             }
           };
@@ -1330,11 +1333,11 @@ int launch_direct(const Args &a, long long blocks, int round_blocks, hipStream_t
   }
 }
 
-template <int GATED, bool PERSIST, bool HALF>
+template <int GATED, bool PERSIST, bool HALF, bool XIELU = false>
 int launch_pipe_one(const Args &a, long long blocks, hipStream_t s) {
   // (256 x 256: all that a CU has)
   constexpr int lds_bytes = HALF ? 3 * (256 + 128) * 128 : 3 * 256 * 128 + 4 * 256 * 64;
-  auto kern = gemm_pipe_kernel<GATED, PERSIST>;
+  auto kern = gemm_pipe_kernel<GATED, PERSIST, XIELU>;
   if constexpr (HALF) kern = gemm_pipe_half_kernel<GATED, PERSIST>;
   static bool raised = false;     // per instantiation; harmless if repeated
   if (!raised) {
@@ -1353,6 +1356,7 @@ int launch_pipe_one(const Args &a, long long blocks, hipStream_t s) {
 template <bool HALF>
 int launch_pipe(const Args &a, long long blocks, bool a_block_a_tile, hipStream_t s) {
   // (going on to the next tile, whose first stages are loaded in the last 128 k of this one, takes 128 k)
+  if (!HALF && a.act_params) return launch_pipe_one<0, true, false, true>(a, blocks, s);      // (128 k and more)
   if (a_block_a_tile || a.n_in < 128) {
     switch (a.gated) {
       case 3: return launch_pipe_one<3, false, HALF>(a, blocks, s);
@@ -1414,7 +1418,8 @@ extern "C" int sb_gemm_mfma_scaled_bf16(void *y, int y_dtype, const void *x, con
 
 namespace {
 int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *bias, int bias_dtype, const float *resid, float resid_scale,
-               int n_rows, int n_out, int n_in, int gated, int relu_sq, int packed, int tile_shape, void *stream);
+               int n_rows, int n_out, int n_in, int gated, int relu_sq, int packed, int tile_shape, void *stream,
+               const void *act_params = nullptr, int act_dtype = 0);
 }
 
 // The product with an activation of an ungated feed-forward on its way out: SB_ACT_RELU_SQ, max(z, 0)^2 of z = X W^T + bias.
@@ -1422,6 +1427,20 @@ extern "C" int sb_gemm_mfma_act_bf16(void *y, int y_dtype, const void *x, const 
                                      int n_out, int n_in, int act, int packed, int tile_shape, void *stream) {
   SB_SUPPORT(act == SB_ACT_RELU_SQ, "sb_gemm_mfma_act_bf16: activation %d is not the square of max(z, 0)", act);
   return gemm_whole(y, y_dtype, x, w, bias, bias_dtype, nullptr, 1.0f, n_rows, n_out, n_in, 0, 1, packed, tile_shape, stream);
+}
+
+// xIELU on a product's way out: in tiles of 256 x 256, whose kernel is built for it (asked for at run time it slows every product),
+// of packed weights whose product would stay whole.
+// 4,001 rows against 8,192 x 2,048: 117 us and a pass of 49, together 147.
+extern "C" int sb_gemm_mfma_xielu_ok(int n_rows, int n_out, int n_in) {
+  return n_rows > 0 && n_out > 0 && n_in >= 128 && n_in % 64 == 0 && pick_shape(n_rows, n_out, n_in, 0, true) == 2 &&
+         sb_gemm_mfma_slices(n_rows, n_out, n_in, 1) == 1;
+}
+extern "C" int sb_gemm_mfma_xielu_bf16(void *y, int y_dtype, const void *x, const void *w, int n_rows, int n_out, int n_in,
+                                       const void *params, int params_dtype, void *stream) {
+  SB_SUPPORT(sb_gemm_mfma_xielu_ok(n_rows, n_out, n_in), "sb_gemm_mfma_xielu_bf16: rows=%d out=%d in=%d are not taken", n_rows, n_out, n_in);
+  SB_REQUIRE(params && sb::valid_dtype(params_dtype), "sb_gemm_mfma_xielu_bf16: xIELU takes two numbers");
+  return gemm_whole(y, y_dtype, x, w, nullptr, 0, nullptr, 1.0f, n_rows, n_out, n_in, 0, 0, 1, -1, stream, params, params_dtype);
 }
 
 extern "C" int sb_gemm_mfma_bf16(void *y, int y_dtype, const void *x, const void *w, const void *bias,
@@ -1441,7 +1460,8 @@ extern "C" int sb_gemm_mfma_scaled_bf16(void *y, int y_dtype, const void *x, con
 
 namespace {
 int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *bias, int bias_dtype, const float *resid, float resid_scale,
-               int n_rows, int n_out, int n_in, int gated, int relu_sq, int packed, int tile_shape, void *stream) {
+               int n_rows, int n_out, int n_in, int gated, int relu_sq, int packed, int tile_shape, void *stream, const void *act_params,
+               int act_dtype) {
   SB_REQUIRE(y && x && w, "sb_gemm_mfma_bf16: null pointer");
   SB_REQUIRE(n_rows >= 0 && n_out > 0 && n_in > 0, "sb_gemm_mfma_bf16: bad sizes rows=%d out=%d in=%d",
              n_rows, n_out, n_in);
@@ -1457,6 +1477,7 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
   a.y = y; a.y_dtype = y_dtype; a.x = (const bf16_t *)x; a.w = (const bf16_t *)w;
   a.bias = bias; a.bias_dtype = bias_dtype; a.resid = resid; a.resid_scale = resid_scale;
   a.n_rows = n_rows; a.n_out = n_out; a.n_in = n_in; a.gated = gated; a.relu_sq = relu_sq;
+  a.act_params = act_params; a.act_dtype = act_dtype;
   a.partial = nullptr; a.stages_per_slice = 0;
   a.vec4 = n_out % 4 == 0 && (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(resid)) % 16 == 0;
   const bool direct_ok = packed && n_in % 64 == 0;
@@ -1657,7 +1678,7 @@ extern "C" int sb_gemm_mfma_partial_bf16(float *partial, const void *x, const vo
   Args a;
   a.y = nullptr; a.y_dtype = SB_F32; a.x = (const bf16_t *)x; a.w = (const bf16_t *)w;
   a.bias = nullptr; a.bias_dtype = 0; a.resid = nullptr; a.resid_scale = 1.0f;
-  a.n_rows = n_rows; a.n_out = n_out; a.n_in = n_in; a.gated = 0; a.relu_sq = 0;
+  a.n_rows = n_rows; a.n_out = n_out; a.n_in = n_in; a.gated = 0; a.relu_sq = 0; a.act_params = nullptr; a.act_dtype = 0;
   const PartialPlan plan = partial_plan(n_rows, n_out, n_in, packed && n_in % 64 == 0);
   const int bm = plan.tile == kBig ? 256 : plan.tile == kDirect64 ? 64 : 128, bn = plan.tile == kBig ? 256 : 128;
   a.tiles_m = (n_rows + bm - 1) / bm;

@@ -893,11 +893,11 @@ def gemm_bf16_add_scaled(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.
 
 
 def gemm_bf16_activated(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out_dtype: torch.dtype, activation: str,
-                        packed_shape) -> Optional[torch.Tensor]:
+                        packed_shape, params: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
     """act(x w^T (+ bias)) in the tiled product's own epilogue; None when the activation or the sizes are not its own (few
     rows go to the weight-streaming kernels): the caller then activates in a pass of its own."""
     _dev(x, w, bias)
-    if activation != "relu_sq" or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or packed_shape is None or x.dim() != 2:
+    if activation not in ("relu_sq", "xielu") or x.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or packed_shape is None or x.dim() != 2:
         return None
     n, k = packed_shape
     t = x.shape[0]
@@ -905,6 +905,14 @@ def gemm_bf16_activated(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.T
         return None
     if bias is not None and bias.numel() != n:
         raise KernelLibraryError(f"bias has {bias.numel()} elements, the product has {n} columns")
+    if activation == "xielu":
+        # (a measurement's choice of a tile keeps the pass of its own)
+        if bias is not None or params is None or params.numel() != 2 or _hints.tile_shape >= 0 or not library.core().sb_gemm_mfma_xielu_ok(t, n, k):
+            return None
+        _dev(params)
+        y = torch.empty((t, n), dtype=out_dtype, device=x.device)
+        check(library.core().sb_gemm_mfma_xielu_bf16(_p(y), _dt(y), _p(x), _p(w), t, n, k, _p(params), _dt(params), _stream()))
+        return y
     y = torch.empty((t, n), dtype=out_dtype, device=x.device)
     check(library.core().sb_gemm_mfma_act_bf16(_p(y), _dt(y), _p(x), _p(w), _p(bias), _dt(bias) if bias is not None else 0, t, n, k,
                                                ACTIVATIONS[activation], 1, _hints.tile_shape, _stream()))

@@ -126,7 +126,7 @@ class Linear:
         slices where there are any; else in a pass of its own over the float32 product."""
         if self.packed is not None and x.dtype == torch.bfloat16:
             y = ops.gemm_bf16_activated(x, self.packed, self.bias, out_dtype, activation,
-                                        packed_shape=(self.rows, self.n_in))
+                                        packed_shape=(self.rows, self.n_in), params=params)
             if y is not None:
                 return y
             part = self.partial(x) if self.n_out % 4 == 0 else None

@@ -66,3 +66,18 @@ def test_xielu_against_64_bits(n):
     want = xielu(z, 0.4, -0.3)
     # some eight roundings of terms that the result and z / 2 bound
     assert (np.abs(got - want) <= 8 * 2.0 ** -23 * (np.abs(want) + np.abs(z.numpy()))).all()
+
+
+@pytest.mark.parametrize("t, n, k", [(4001, 4096, 128), (4096, 4094, 192), (4001, 8192, 320)])
+def test_xielu_on_a_products_way_out(t, n, k):
+    """The bits of the product followed by the pass."""
+    from sonicboom_amd import ops
+    x, w, p = randn(t, k, seed=1).to(BF16).to(DEV), randn(n, k, seed=2, scale=0.1).to(BF16).to(DEV), torch.tensor([0.4, -0.3], device=DEV)
+    packed = ops.pack_weight(w)
+    with ops.gemm_tile_shape(2, "direct"):
+        z = ops.gemm_bf16(x, packed, None, None, F32, packed_shape=(n, k))
+    for dtype in (BF16, F32):
+        got = ops.gemm_bf16_activated(x, packed, None, dtype, "xielu", (n, k), params=p)
+        assert got is not None and torch.equal(got, ops.activate(z, dtype, "xielu", p))
+    assert ops.gemm_bf16_activated(x, packed, torch.zeros(n, device=DEV), BF16, "xielu", (n, k), params=p) is None
+    assert ops.gemm_bf16_activated(x[:100], packed, None, BF16, "xielu", (n, k), params=p) is None
