@@ -4,17 +4,17 @@
 // It runs on the float32 matrix cores.  v_mfma_f32_16x16x4_f32 adds its four products to the
 // accumulator one after the other in ascending k, each with one rounding: the bits of a chain of
 // fmaf (checked against fmaf over 1,000 k, denormals among them).  An element is the sum of its
-// segments of kSegment k, a segment the sum of its chains of kChain k, each from zero, both added in ascending order: a function
-// of k alone, so its value does not depend on how many rows share the launch, on the tile or on the
-// waves that made it.  The same (row, column) gives the same bits in a whole prompt, in a
+// chains, each from zero, added in ascending order: chains of kChain k where there are up to kSegment of them, of a segment of
+// kSegment k where there are more.  That is a function of k alone, so its value does not depend on how many rows share the
+// launch, on the tile or on the waves that made it.  The same (row, column) gives the same bits in a whole prompt, in a
 // single-token step and in any batch.  W is [out, in] row-major, the memory of a
 // projection weight (/root/reference/core/include/sonicboom/quant/quantized_matmul.h:74-77);
 // the bias is added after the product and the residual after the bias
 // (/root/reference/core/src/model/emit.cpp:260-261, :447).
 //
 // A block owns 16 CT columns of 16 TT rows.  Its WAVES waves take the segments of K between them
-// (segment s goes to wave s % WAVES), or, where there are few blocks, the chains, straight from memory and without a barrier on the way; the
-// sums meet in LDS.  A lane loads four consecutive k of one row, the four lane groups of
+// (segment s goes to wave s % WAVES), or, where there is one and there are few blocks, its chains, straight from memory and without a
+// barrier on the way; the sums meet in LDS.  A lane loads four consecutive k of one row, the four lane groups of
 // a row 64 bytes side by side; four lane swaps turn the 4 x 4 of lane groups and registers over,
 // after which register s holds k = 4 s + lane group, what step s of the matrix instruction takes.
 // W that a projection keeps is packed (FORM kPacked): blocks of 16 rows x 16 k in the order that
@@ -23,9 +23,13 @@
 // is a tile of W's first half and the same tile of the second, and Y = act(first) * second.
 //
 // What bounds it: with few rows a chain of products (64 of them are 1.3 us) behind the first loads and, where a CU streams much of W (the
-// gated product: 304 blocks of 115 KB on 256 CUs), that; with many rows the matrix cores.  Chains of a whole segment in a wave each took
-// longer: 3 rows against 896 x 896 7.6 us and 5.1 with a wave a chain, 1,152 x 896 7.7 and 5.2, 50 rows 12.3 and 8.4, the planes of 896 x
-// 4,864 9.4 and 8.4; and the error against 64 bits is half of what it was (2.8e-7 of the result instead of 5.4e-7).  The source keeps a step's loads behind its
+// gated product: 304 blocks of 115 KB on 256 CUs), that; with many rows the matrix cores.  With one chain of up to 1,024 k few rows took
+// longer: 3 rows against 896 x 896 8.1 us and 5.7 with a wave a chain, 1,152 x 896 8.1 and 5.7, 50 rows 12.9 and 9.1, 16 against 16,384 x
+// 256 8.0 and 7.0; 130 rows against 1,152 x 896 14.1 and 14.5; and the error against 64 bits is half of what it was.  Longer products keep
+// chains of a segment.  Shorter ones gave few rows 2,048 x 2,048 9.7 -> 9.0 us, but their sums cost registers or loads in flight: 3 rows
+// against 3,584 x 18,944 54.8 -> 68.6, gated 17,920 x 1,536 26.2 -> 31.3, 520 rows against gated 37,888 x 3,584 1,372 -> 1,562 (with the
+// registers bounded and the sums joined between products 1,454).
+// The source keeps a step's loads behind its
 // products and turns X's fragments over a step ahead: left to itself the compiler turned a whole ring over at once and so
 // waited for the newest of its loads ahead of the round's first product.  Measured on MI355X at the 0.5B layer sizes, 3 rows,
 // left to itself and so, a wave a segment: 896 x 896 8.2 and 7.7 us, the gated 9,728 x 896 16.1 and 13.5, 896 x 4,864 15.5 and 14.9, a block a
@@ -36,10 +40,9 @@
 
 namespace {
 
-constexpr int kSegment = 1024;          // k of a segment, and of one chain: part of what the result's bits are
-constexpr int kChain = 256;
+constexpr int kSegment = 1024;          // k of a segment, the chain of products with more k: part of what the result's bits are
+constexpr int kChain = 256;             // k of a chain of products with no more than a segment: likewise
 constexpr int kChains = kSegment / kChain;
-constexpr int kSteps = kSegment / 16;   // loads of a row in a segment
 constexpr int kChainSteps = kChain / 16;
 
 enum Form { kAny, kPacked, kPackedAny };   // W row-major; W packed, X by 16-byte loads; W packed, X element by element
@@ -93,16 +96,19 @@ bool by_fours(const void *y, const float *resid, int n_out) {
   return n_out % 4 == 0 && (reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(resid)) % 16 == 0;
 }
 
-// CHAINS: a wave's share is a chain (wave w of a block takes every WAVES-th), else a segment.
-template <typename TX, typename TW, int FORM, int TT, int CT, int G, int WAVES, bool CHAINS>
+// CHAINS: kWhole: a wave's share is a segment, one chain (more than one segment); kInTurn: the one segment, its chains one after the
+// other; kApart: a wave a chain of it.
+enum Chains { kWhole, kInTurn, kApart };
+template <typename TX, typename TW, int FORM, int TT, int CT, int G, int WAVES, Chains CHAINS>
 __global__ void __launch_bounds__(64 * WAVES)
 gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a) {
   constexpr int kStreams = CT * G, kTiles = TT * CT, kThreads = 64 * WAVES;
-  // steps in flight: as many as 192 registers hold (128 or less beside the accumulators of larger tiles
+  // steps in flight: as many as 192 registers hold, and a chain ends with a round of them (128 or less beside the accumulators of larger tiles
   // and the addresses of loads element by element)
   constexpr int kRegs = 4 * (kStreams + TT);
-  constexpr int kAhead = FORM != kPacked ? 4 : kRegs <= 12 ? 16 : kRegs <= 16 ? 8 : 4;
-  static_assert(kChainSteps % kAhead == 0 && (!CHAINS || WAVES % kChains == 0), "chains end with a round of the ring");
+  constexpr int kAhead = FORM != kPacked ? 4 : kRegs == 8 && CHAINS == kWhole ? 24 : kRegs <= 12 ? 16 : kRegs <= 16 ? 8 : 4;
+  static_assert(CHAINS == kWhole || kChainSteps % kAhead == 0, "chains end with a round of the ring");
+  static_assert(CHAINS == kWhole || WAVES == (CHAINS == kApart ? kChains : 1), "a block has the segment's chains");
   constexpr int kPolicy = TT == 1 ? kReadOnce : 0;                  // up to sixteen rows: no other block reads this share of W (prompts and
                                                                     // eight tokens of the 0.5B sizes 19.7 -> 19.2 ms)
   constexpr int kUnits = (kTiles * 64 + kThreads - 1) / kThreads;   // groups of four outputs a thread
@@ -138,11 +144,12 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
   // a grid of as many layers as segments: each block one segment, whose raw sums are Y's plane of that number
   const bool split = gridDim.y > 1;
   const int n_seg = split ? int(blockIdx.y) + 1 : (a.n_in + kSegment - 1) / kSegment;
+  constexpr int kShare = CHAINS == kApart ? kChain : kSegment;
   const int k_all = min(n_seg * kSegment, a.n_in);
-  for (int s0 = blockIdx.y; s0 < n_seg; s0 += CHAINS ? WAVES / kChains : WAVES) {
-    const int k0 = s0 * kSegment + wave * (CHAINS ? kChain : kSegment);
+  for (int s0 = blockIdx.y; s0 < n_seg; s0 += WAVES) {
+    const int k0 = s0 * kSegment + wave * kShare;
     if (k0 < k_all) {                            // uniform over the wave
-      const int k_end = min(k0 + (CHAINS ? kChain : kSegment), a.n_in);
+      const int k_end = min(k0 + kShare, a.n_in);
       const int steps = (k_end - k0 + 15) / 16;
       // packed: a descriptor a stream, of its tile's blocks up to the segment's end
       __amdgpu_buffer_rsrc_t rsrc_w[kStreams];
@@ -200,19 +207,14 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
               acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[i][s], fx[set][j][s], acc[i][j], 0, 0, 0);
       };
       static_assert(kAhead % 2 == 0, "the sets of turned fragments alternate");
-      // a chain's end: its sums join the segment's, in registers or in this lane's own places in LDS
-      auto fold = [&](bool first, bool more) {
+      // a chain's end: its sums join the total, or wait in this lane's own places in LDS
+      auto fold = [&](bool more) {
 #pragma unroll
         for (int i = 0; i < kStreams; ++i)
 #pragma unroll
           for (int j = 0; j < TT; ++j) {
-            if constexpr (WAVES == 1) {
-              total[(i / G) * TT + j][i % G] = total[(i / G) * TT + j][i % G] + acc[i][j];
-            } else {
-              floatx4_t &at = part[((wave * G + i % G) * kTiles + (i / G) * TT + j) * 64 + lane];
-              if (CHAINS || first) at = acc[i][j];
-              else at = at + acc[i][j];
-            }
+            if constexpr (WAVES == 1) total[(i / G) * TT + j][i % G] = total[(i / G) * TT + j][i % G] + acc[i][j];
+            else part[((wave * G + i % G) * kTiles + (i / G) * TT + j) * 64 + lane] = acc[i][j];
             if (more) acc[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
           }
       };
@@ -229,9 +231,9 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
           // (left alone, the compiler turns a whole round over at once, waiting for the last of its loads ahead of the first product)
           __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (!CHAINS) {
+        if constexpr (CHAINS == kInTurn) {
           const int done = step + kAhead;
-          if (done % kChainSteps == 0 && done < steps) fold(done == kChainSteps, true);
+          if (done % kChainSteps == 0 && done < steps) fold(true);
         }
       }
 #pragma unroll
@@ -240,32 +242,18 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
           if (u + 1 < kAhead) turn(u + 1, (u + 1) & 1);
           multiply(u, u & 1);
         }
-      fold(steps <= kChainSteps, false);
+      fold(false);
     }
     if constexpr (WAVES > 1) {
       __syncthreads();
-      const int here = CHAINS ? min(WAVES, (k_all - s0 * kSegment + kChain - 1) / kChain) : min(WAVES, n_seg - s0);
+      const int here = min(WAVES, (k_all - s0 * kSegment + kShare - 1) / kShare);
 #pragma unroll
       for (int u = 0; u < kUnits; ++u) {
         const int unit = tid + u * kThreads;
-        if (unit < kTiles * 64) {
+        if (unit < kTiles * 64)
+          for (int v = 0; v < here; ++v)
 #pragma unroll
-          for (int q = 0; q < G; ++q) {
-            if constexpr (CHAINS) {
-#pragma unroll
-              for (int v = 0; v < WAVES; v += kChains) {
-                if (v >= here) break;
-                floatx4_t sum = part[(v * G + q) * kTiles * 64 + unit];
-#pragma unroll
-                for (int c = 1; c < kChains; ++c)
-                  if (v + c < here) sum = sum + part[((v + c) * G + q) * kTiles * 64 + unit];
-                total[u][q] = total[u][q] + sum;
-              }
-            } else {
-              for (int v = 0; v < here; ++v) total[u][q] = total[u][q] + part[(v * G + q) * kTiles * 64 + unit];
-            }
-          }
-        }
+            for (int q = 0; q < G; ++q) total[u][q] = total[u][q] + part[(v * G + q) * kTiles * 64 + unit];
       }
       __syncthreads();
     }
@@ -327,7 +315,7 @@ gemm_f32_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a)
   }
 }
 
-template <typename TX, typename TW, int FORM, int TT, int CT, int G, int WAVES, bool CHAINS = false>
+template <typename TX, typename TW, int FORM, int TT, int CT, int G, int WAVES, Chains CHAINS = kWhole>
 int launch_one(const TX *x, const TW *w, const PlainArgs &a, hipStream_t s, int layers = 1) {
   constexpr int lds_bytes = WAVES == 1 ? 0 : WAVES * TT * CT * G * 1024;
   auto kern = gemm_f32_kernel<TX, TW, FORM, TT, CT, G, WAVES, CHAINS>;
@@ -345,7 +333,7 @@ int launch_one(const TX *x, const TW *w, const PlainArgs &a, hipStream_t s, int 
 
 template <int TT, int CT, int G>
 int launch_packed(const float *x, const float *w, const PlainArgs &a, int n_seg, hipStream_t s) {
-  if (n_seg == 1) return launch_one<float, float, kPacked, TT, CT, G, 1>(x, w, a, s);
+  if (n_seg == 1) return launch_one<float, float, kPacked, TT, CT, G, 1, kInTurn>(x, w, a, s);
   if (n_seg == 2) return launch_one<float, float, kPacked, TT, CT, G, 2>(x, w, a, s);
   if (n_seg <= 4) return launch_one<float, float, kPacked, TT, CT, G, 4>(x, w, a, s);
   return launch_one<float, float, kPacked, TT, CT, G, 8>(x, w, a, s);
@@ -366,9 +354,8 @@ int launch_packed_tiles(const float *x, const float *w, const PlainArgs &a, int 
   if (a.n_rows <= 16) {
     if (G == 1 && waves(1, 2) >= 4 * kEnough) return launch_packed<1, 2, G>(x, w, a, n_seg, s);
     // a wave a chain while there is a CU a block (gated, 304 blocks, it would be 13.6 us for 13.2)
-    if (tiles(1, 1) > 256) return launch_packed<1, 1, G>(x, w, a, n_seg, s);
-    if (n_seg == 1) return launch_one<float, float, kPacked, 1, 1, G, 4, true>(x, w, a, s);
-    return launch_one<float, float, kPacked, 1, 1, G, 8, true>(x, w, a, s);
+    if (n_seg == 1 && tiles(1, 1) <= sb::cu_count()) return launch_one<float, float, kPacked, 1, 1, G, kChains, kApart>(x, w, a, s);
+    return launch_packed<1, 1, G>(x, w, a, n_seg, s);
   }
   constexpr int kShapes[4][2] = {{4, 4 / G}, {4, 2 / G}, {2, 2 / G}, {2, 1}};      // (gated the last two are one)
   int pick = 3;
@@ -388,8 +375,10 @@ int launch_packed_tiles(const float *x, const float *w, const PlainArgs &a, int 
   if (pick == 0) return launch_packed<4, 4 / G, G>(x, w, a, n_seg, s);
   if (pick == 1) return launch_packed<4, 2 / G, G>(x, w, a, n_seg, s);
   if (pick == 2) return launch_packed<2, 2 / G, G>(x, w, a, n_seg, s);
-  // (288 blocks 12.2 -> 8.6 us; gated, 304, 20.4 and 21.0; a wave a chain of several segments 25.7 and 30.5 at 20 rows against 896 x 4,864)
-  if (n_seg == 1 && tiles(2, 1) <= (G == 1 ? 512 : 256)) return launch_one<float, float, kPacked, 2, 1, G, 4, true>(x, w, a, s);
+  // a wave a chain, of three or four (50 rows against 1,152 x 896, 144 blocks, 12.9 -> 9.1 us; gated, 304 and more, 20.4 and 21.0; two
+  // chains, 20 rows against 6,144 x 512, 384 blocks, 9.8 and 11.1)
+  if (n_seg == 1 && a.n_in > 2 * kChain && tiles(2, 1) <= (G == 1 ? 2 : 1) * sb::cu_count())
+    return launch_one<float, float, kPacked, 2, 1, G, kChains, kApart>(x, w, a, s);
   return launch_packed<2, 1, G>(x, w, a, n_seg, s);
 }
 
@@ -398,9 +387,11 @@ constexpr int kTile = 64;        // rows and columns of a block's tile
 constexpr int kStage = 16;       // k per stage; a segment is a whole number of stages
 constexpr int kTileThreads = 256;
 
-// A segment's sums are in registers; several segments' wait in LDS, a place a thread, but for a row of four.  The next stage is
-// asked for ahead of a stage's products: loaded and waited for in turn, the sums of the chains (sixteen registers more) cost the
-// waves that hid it (2,048 rows against 3,584 x 3,584, float32, 803 us without chains, 1,177 with, 749 so; bfloat16 724, 1,041 and 682).
+// The sums of chains are in registers; several segments' wait in LDS, a place a thread, but for a row of four.  The next stage is
+// asked for ahead of a stage's products, at addresses that are the block's plus one number a thread: 58 registers, eight waves a SIMD (with
+// an address for each load 96 and five).  Us, one chain of up to 1,024 k and no stage ahead, with an address each, so: 2,048 rows against
+// 3,584 x 3,584 float32 796, 748, 698, bfloat16 714, 684, 636; 3,584 x 896 207, 206, 195 and 179, 193, 181; 4,000 rows against 2,000 x
+// 1,024 246, 268, 248 and 231, 245, 228.
 template <typename TX, typename TW, bool SEGMENTS>
 __global__ void __launch_bounds__(kTileThreads)
 gemm_tile_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a) {
@@ -410,32 +401,34 @@ gemm_tile_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a
   const unsigned tiles_n = (a.n_out + kTile - 1) / kTile;
   const int t0 = int(blockIdx.x / tiles_n) * kTile, n0 = int(blockIdx.x % tiles_n) * kTile;
   const int tid = threadIdx.x, ty = tid / 16, tx = tid % 16;
-  float acc[4][4], seg[4][4], last[4];
+  float acc[4][4], sum[4][4];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = seg[i][j] = last[j] = 0.0f;
+    for (int j = 0; j < 4; ++j) acc[i][j] = sum[i][j] = 0.0f;
   // a stage on its way: asked for ahead of the products of the stage before
+  constexpr int kRowsApart = kTileThreads / kStage;
+  const int row = tid / kStage, k_of = tid % kStage;
+  const unsigned off = unsigned(row) * unsigned(a.n_in) + unsigned(k_of);      // (beside addresses that are the block's)
   TX nx[4];
   TW nw[4];
   const auto ask = [&](int k0) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int e = tid + i * kTileThreads;
-      const int gk = k0 + e % kStage, gt = t0 + e / kStage, gn = n0 + e / kStage;
-      nx[i] = gt < a.n_rows && gk < a.n_in ? x[size_t(gt) * a.n_in + gk] : TX(0);
-      nw[i] = gn < a.n_out && gk < a.n_in ? w[size_t(gn) * a.n_in + gk] : TW(0);
+      const int t = t0 + i * kRowsApart, n = n0 + i * kRowsApart;
+      nx[i] = t + row < a.n_rows && k0 + k_of < a.n_in ? (x + size_t(t) * a.n_in + k0)[off] : TX(0);
+      nw[i] = n + row < a.n_out && k0 + k_of < a.n_in ? (w + size_t(n) * a.n_in + k0)[off] : TW(0);
     }
   };
   ask(0);
-  for (int c0 = 0; c0 < a.n_in; c0 += kChain) {
-    const int c_end = min(c0 + kChain, a.n_in);
+  constexpr int kLength = SEGMENTS ? kSegment : kChain;
+  for (int c0 = 0; c0 < a.n_in; c0 += kLength) {
+    const int c_end = min(c0 + kLength, a.n_in);
     for (int k0 = c0; k0 < c_end; k0 += kStage) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int e = tid + i * kTileThreads;
-        xs[e % kStage][e / kStage] = ld_f(&nx[i], 0);
-        ws[e % kStage][e / kStage] = ld_f(&nw[i], 0);
+        xs[k_of][row + i * kRowsApart] = ld_f(&nx[i], 0);
+        ws[k_of][row + i * kRowsApart] = ld_f(&nw[i], 0);
       }
       __syncthreads();
       ask(k0 + kStage);
@@ -453,18 +446,13 @@ gemm_tile_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a
       }
       __syncthreads();
     }
-    const bool ends = SEGMENTS && (c_end == a.n_in || c_end % kSegment == 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        seg[i][j] = seg[i][j] + acc[i][j];
+        if (SEGMENTS && i < 3) total[4 * i + j][tid] = c0 > 0 ? total[4 * i + j][tid] + acc[i][j] : acc[i][j];
+        else sum[i][j] = sum[i][j] + acc[i][j];
         acc[i][j] = 0.0f;
-        if (ends) {
-          if (i < 3) total[4 * i + j][tid] = c0 < kSegment ? seg[i][j] : total[4 * i + j][tid] + seg[i][j];
-          else last[j] = last[j] + seg[i][j];
-          seg[i][j] = 0.0f;
-        }
       }
   }
 #pragma unroll
@@ -475,7 +463,7 @@ gemm_tile_kernel(const TX *__restrict__ x, const TW *__restrict__ w, PlainArgs a
     for (int j = 0; j < 4; ++j) {
       const int n = n0 + tx * 4 + j;
       if (n >= a.n_out) continue;
-      float v = !SEGMENTS ? seg[i][j] : i < 3 ? total[4 * i + j][tid] : last[j];
+      float v = SEGMENTS && i < 3 ? total[4 * i + j][tid] : sum[i][j];
       if (a.bias) v = v + ld_dyn(a.bias, a.bias_dtype, n);
       const size_t idx = size_t(t) * a.n_out + n;
       if (a.resid) v = v + a.resid[idx];
@@ -506,7 +494,7 @@ int launch_any(const TX *x, const TW *w, const PlainArgs &a, int n_seg, hipStrea
     else gemm_tile_kernel<TX, TW, true><<<unsigned(blocks), kTileThreads, 0, s>>>(x, w, a);
     return sb::check_launch("sb_gemm");
   }
-  if (n_seg == 1) return launch_one<TX, TW, kAny, 2, 1, 1, 1>(x, w, a, s);
+  if (n_seg == 1) return launch_one<TX, TW, kAny, 2, 1, 1, 1, kInTurn>(x, w, a, s);
   return launch_one<TX, TW, kAny, 2, 1, 1, 8>(x, w, a, s);
 }
 
@@ -555,9 +543,9 @@ extern "C" int sb_gemm_f32_packed(void *y, int y_dtype, const float *x, const fl
   // 16-byte loads need rows of X that start on 16 bytes; offsets inside a block's rows fit 31 bits
   const bool vec = n_in % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && size_t(n_in) * 64 * 4 < (size_t(1) << 31);
   if (!vec) {
-    if (gated) return n_seg == 1 ? launch_one<float, float, kPackedAny, 2, 1, 2, 1>(x, w, a, s)
+    if (gated) return n_seg == 1 ? launch_one<float, float, kPackedAny, 2, 1, 2, 1, kInTurn>(x, w, a, s)
                                  : launch_one<float, float, kPackedAny, 2, 1, 2, 8>(x, w, a, s);
-    return n_seg == 1 ? launch_one<float, float, kPackedAny, 2, 1, 1, 1>(x, w, a, s)
+    return n_seg == 1 ? launch_one<float, float, kPackedAny, 2, 1, 1, 1, kInTurn>(x, w, a, s)
                       : launch_one<float, float, kPackedAny, 2, 1, 1, 8>(x, w, a, s);
   }
   return gated ? launch_packed_tiles<2>(x, w, a, n_seg, s) : launch_packed_tiles<1>(x, w, a, n_seg, s);
@@ -569,7 +557,7 @@ extern "C" int sb_gemm_f32_segments(int n_in) { return (n_in + kSegment - 1) / k
 // The raw product of float32 X and packed float32 W a segment at a time: partial float [segments][n_rows][n_out], which added
 // in ascending order are the bits of sb_gemm_f32_packed.  A block a segment and sixteen columns: with few rows the whole
 // product's blocks, whose waves take the segments between them, are a few dozen (3 rows against 896 x 4,864: 56 blocks and
-// 14.9 us, 280 and 9.4, with four waves a segment, a chain each, 8.4).
+// 15.8 us, 280 and 9.8).
 extern "C" int sb_gemm_f32_packed_partial(float *partial, const float *x, const float *w, int n_rows, int n_out, int n_in, void *stream) {
   SB_REQUIRE(partial && x && w, "sb_gemm_f32_packed_partial: null pointer");
   SB_REQUIRE(n_rows >= 0 && n_out > 0 && n_in > 0, "sb_gemm_f32_packed_partial: bad sizes rows=%d out=%d in=%d", n_rows, n_out, n_in);
@@ -581,5 +569,5 @@ extern "C" int sb_gemm_f32_packed_partial(float *partial, const float *x, const 
   const int n_seg = sb_gemm_f32_segments(n_in);
   SB_SUPPORT(n_seg >= 2 && n_seg <= 65535, "sb_gemm_f32_packed_partial: %d segments", n_seg);
   const PlainArgs a{partial, SB_F32, nullptr, 0, nullptr, n_rows, n_out, n_in, SB_GATE_NONE, by_fours(partial, nullptr, n_out)};
-  return launch_one<float, float, kPacked, 1, 1, 1, 4, true>(x, w, a, (hipStream_t)stream, n_seg);
+  return launch_one<float, float, kPacked, 1, 1, 1, 1>(x, w, a, (hipStream_t)stream, n_seg);
 }

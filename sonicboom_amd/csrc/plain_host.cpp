@@ -75,22 +75,19 @@ int sbp_reduce_resid_norm(float *y, float *x, const float *partial, int n_slices
   return do_norm ? sbp_rmsnorm(y, x, w, nullptr, n_rows, width, eps) : 0;
 }
 
-// Y[t,n] = sum_k X[t,k] W[n,k] (+ bias[n]) (+ resid[t,n]) in the plain kernel's order (so the two agree to the bit): chains
-// of 256 k, one fused multiply-add per k in ascending order from zero, added into segments of 1,024 k, and those into the sum.
+// Y[t,n] = sum_k X[t,k] W[n,k] (+ bias[n]) (+ resid[t,n]) in the plain kernel's order (so the two agree to the bit): chains of
+// 256 k, of 1,024 where there are more k than that, one fused multiply-add per k in ascending order from zero, added in order.
 int sbp_gemm(float *y, const float *x, const float *w, const float *bias, const float *resid, int n_rows,
              int n_out, int n_in) {
   if (!y || !x || !w || n_rows < 0 || n_out <= 0 || n_in <= 0) return 1;
   for (int t = 0; t < n_rows; ++t)
     for (int n = 0; n < n_out; ++n) {
       float acc = 0.0f;
-      for (int s = 0; s < n_in; s += 1024) {
-        float segment = 0.0f;
-        for (int c = s; c < n_in && c < s + 1024; c += 256) {
-          float chain = 0.0f;
-          for (int k = c; k < n_in && k < c + 256; ++k) chain = std::fmaf(x[size_t(t) * n_in + k], w[size_t(n) * n_in + k], chain);
-          segment = segment + chain;
-        }
-        acc = acc + segment;
+      const int length = n_in > 1024 ? 1024 : 256;
+      for (int c = 0; c < n_in; c += length) {
+        float chain = 0.0f;
+        for (int k = c; k < n_in && k < c + length; ++k) chain = std::fmaf(x[size_t(t) * n_in + k], w[size_t(n) * n_in + k], chain);
+        acc = acc + chain;
       }
       if (bias) acc = acc + bias[n];
       if (resid) acc = acc + resid[size_t(t) * n_out + n];

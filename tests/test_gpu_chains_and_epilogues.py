@@ -1,4 +1,4 @@
-"""Float32 products in chains of 256 k, gated products whose weights pass through registers, xIELU as a pass and on a product's way out."""
+"""Float32 products in their chains, gated products whose weights pass through registers, xIELU as a pass and on a product's way out."""
 import math
 
 import numpy as np
@@ -16,18 +16,28 @@ def randn(*shape, seed=0, scale=1.0):
 @pytest.mark.parametrize("t", [1, 16, 20, 70])
 @pytest.mark.parametrize("n, k", [(40, 256), (40, 260), (33, 768), (33, 1024), (48, 1280), (16, 2304)])
 def test_float32_chains_end_inside_and_between_segments(t, n, k):
-    """One to nine chains of 256 k in up to three segments: the same bits from every kernel, within a chain's roundings of 64 bits."""
+    """One to four chains of 256 k, two and three of 1,024: the same bits from every kernel, within a chain's roundings of 64 bits."""
     from sonicboom_amd import ops
     x, w = randn(t, k, seed=t), randn(n, k, seed=k, scale=0.05)
     want = ops.gemm_plain(x.to(DEV), w.to(DEV), None, None, F32)
     got = ops.gemm_f32(x.to(DEV), ops.pack_weight_f32(w.to(DEV)), None, None, F32, (n, k))
     assert torch.equal(got, want)
-    # each of at most 256 + 4 + 3 roundings is half a unit of a running sum that the terms' absolute values bound
-    bound = (256 + 4 + 3) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+    # each of at most a chain's and four more roundings is half a unit of a running sum that the terms' absolute values bound
+    bound = ((1024 if k > 1024 else 256) + 4) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
     assert ((got.cpu().double() - x.double() @ w.double().T).abs() <= bound).all()
     if n % 2 == 0:
         gated = ops.gemm_f32(x.to(DEV), ops.pack_weight_f32(w.to(DEV), True), None, None, F32, (n, k), gated="silu")
         assert torch.equal(gated, ops.silu_mul(want, F32))
+
+
+@pytest.mark.parametrize("t, n, k", [(515, 3001, 901), (515, 3001, 1029), (4033, 700, 272), (129, 9000, 2300)])
+def test_row_major_products_of_many_tiles_have_the_bits_of_packed_ones(t, n, k):
+    """Rows, columns and k that end inside a tile and a stage, one chain to four, two and three of 1,024."""
+    from sonicboom_amd import ops
+    for dtype in (F32, BF16):
+        x, w = randn(t, k, seed=t).to(DEV, dtype), randn(n, k, seed=k, scale=0.05).to(DEV, dtype)
+        want = ops.gemm_f32(x.float(), ops.pack_weight_f32(w.float()), None, None, F32, (n, k))
+        assert torch.equal(ops.gemm_plain(x, w, None, None, F32), want)
 
 
 @pytest.mark.parametrize("shape", [6, 7, 8])
