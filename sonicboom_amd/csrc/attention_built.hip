@@ -376,6 +376,7 @@ extern "C" int sb_built_attention(void *out, const void *q_plain, const void *q_
                                   int window, const float *gate, int gate_stride, int gate_per_head, void *stream) {
   SB_REQUIRE(out && q_plain && q_rot && built && cache && page_table && tiles, "sb_built_attention: null pointer");
   SB_REQUIRE(n_tiles >= 0 && heads > 0 && max_pages > 0 && n_pages_total > 0 && window >= 0, "sb_built_attention: bad sizes");
+  SB_SUPPORT(scale > 0.0f, "sb_built_attention: a scale of %g is not taken", double(scale));
   SB_SUPPORT(sb_built_attention_ok(dim, rot_dim, vdim, rank), "sb_built_attention: heads of %d + %d numbers and %d values are not taken", dim,
              rot_dim, vdim);
   SB_SUPPORT((reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(q_plain) | reinterpret_cast<uintptr_t>(q_rot) |

@@ -257,7 +257,7 @@ int sb_latent_attention_bf16(void *out, const void *q, const void *cache, const 
  *   rotated key parts behind the first rank numbers of the cached rows; q_plain [n_rows, heads, dim], q_rot: row r,
  *   head a at (r * heads + a) * q_rot_stride; tiles int32 [n_tiles, 8] = (first row, rows <= sb_built_tile_rows(),
  *   sequence, the built row that the sequence's key 0 would have, position of the first row, 0, 0, 0); out [n_rows, heads, vdim], times sigmoid(gate) as in
- *   sb_head_product_gated_bf16 unless gate is NULL. */
+ *   sb_head_product_gated_bf16 unless gate is NULL.  scale > 0. */
 int sb_built_attention_ok(int dim, int rot_dim, int vdim, int rank);
 int sb_built_tile_rows(void);
 int sb_built_gather(void *out, const void *cache, const int32_t *page_table, int max_pages, int n_pages_total,
