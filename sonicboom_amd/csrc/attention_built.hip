@@ -46,6 +46,13 @@ __device__ __forceinline__ constexpr int value_turned(int key) {
   return CH == 16 ? (key & 3) << 2 : ((key >> 1) & 1) << 2;
 }
 
+// Whether eight bfloat16 numbers are finite: one to the lowest bit of an exponent of ones carries into the sign's place.
+__device__ __forceinline__ bool finite(bf16x8_t v) {
+  const uint4 w = __builtin_bit_cast(uint4, v);
+  const auto past = [](uint32_t u) { return (u & 0x7f807f80u) + 0x00800080u; };
+  return ((past(w.x) | past(w.y) | past(w.z) | past(w.w)) & 0x80008000u) == 0;
+}
+
 struct BuiltArgs {
   bf16_t *out;                      // [rows][heads][VD]
   const bf16_t *q_plain;            // [rows][heads][DP]
@@ -99,6 +106,7 @@ built_attention_kernel(BuiltArgs a) {
   // a tile's rows are consecutive positions
   const int pos_first = a.tiles[8 * tile + 4], pos_last = pos_first + n_tile - 1;
   const int lo_of_first = (a.window > 0 && pos_first >= a.window) ? pos_first - a.window + 1 : 0;
+  const int lo_of_last = (a.window > 0 && pos_last >= a.window) ? pos_last - a.window + 1 : 0;      // the first key that every row sees
   const int wave_first = pos_first + 32 * wave, wave_last = wave_first + n_wave - 1;
   const int wave_lo = (a.window > 0 && wave_first >= a.window) ? wave_first - a.window + 1 : 0;
   const int wave_lo_last = (a.window > 0 && wave_last >= a.window) ? wave_last - a.window + 1 : 0;
@@ -173,13 +181,19 @@ built_attention_kernel(BuiltArgs a) {
     if (have_next) bring(pg + 2, buf ^ 1);
     const int page_pos = pg * SB_PAGE;
     bf16x8_t *page = lds_built + (2 * half + buf) * kBuf;
-    if ((pg0 + 2) * SB_PAGE - 1 > pos_last || pg0 * SB_PAGE < lo_of_first) {
-      // (the pages on the diagonal and at a window's edge) values of keys that no row of the tile sees go to zero: a
-      // weight of zero does not keep a NaN out of the sums
+    if ((pg0 + 2) * SB_PAGE - 1 > pos_first || pg0 * SB_PAGE < lo_of_last) {
+      // (the pages on the diagonal and at a window's edge) a weight of zero does not keep a NaN or an infinity out of the sums.
+      // Values of keys that no row of the tile sees go to zero; so do those of a key that some rows see and that hold a number that is not
+      // finite, and the key becomes a NaN, which the weights of the rows that see it take on.
       const bf16x8_t zero = as_bf16x8(make_uint4(0u, 0u, 0u, 0u));
-      for (int i = threadIdx.x & 255; i < kV; i += 256) {
-        const int j = page_pos + i / CV;
-        if (j > pos_last || j < lo_of_first) page[kK + kR + i] = zero;
+      for (int i = threadIdx.x & 255; have && i < kV; i += 256) {
+        const int key = i / CV, j = page_pos + key;
+        if (j > pos_last || j < lo_of_first) {
+          page[kK + kR + i] = zero;
+        } else if ((j > pos_first || j < lo_of_last) && !finite(page[kK + kR + i])) {
+          page[kK + kR + i] = zero;
+          page[key * CK] = as_bf16x8(make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u));
+        }
       }
       __syncthreads();
     }

@@ -76,6 +76,36 @@ def test_built_attention_equals_64_bits(heads, rank, gates, window):
     assert bool(((got - torch.cat(want)).abs() <= torch.cat(bound) + 1e-6).all())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("number", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("window", [0, 64, 130])
+def test_a_number_that_is_not_finite_reaches_the_rows_that_see_it(window, number):
+    """A latent with such a number among the keys of a prompt's own tiles: the rows that do not see it keep their bits, the others
+    have nothing else."""
+    from sonicboom_amd import ops
+    from sonicboom_amd.parts.linear import Linear
+    heads, rank, cached, n = 2, 64, 70, 300
+    table = torch.randperm(6, generator=torch.Generator().manual_seed(1)).int()[None]
+    cache = rand(6, 64, rank + ROT, seed=3).to(BF16)
+    q_plain, q_latent = rand(n, heads, DIM, seed=4).to(BF16).to(DEV), rand(n, heads, rank + ROT, seed=5).to(BF16).to(DEV)
+    build = Linear(rand(2 * heads * DIM, rank, seed=6, scale=rank ** -0.5).to(BF16).to(DEV), None, True)
+    tiles, pages = (torch.from_numpy(t).to(DEV) for t in ops.latent_built_plan([n], [cached], window))
+    run = lambda c: ops.latent_built_attention(q_plain, q_latent, lambda x: build(x, BF16), c.to(DEV), table.to(DEV), tiles, pages, rank, VDIM,
+                                               0.07, window)
+    clean = run(cache)
+    assert torch.isfinite(clean.float()).all()
+    at = torch.arange(cached, cached + n)
+    for key in (3, 69, 70, 100, 127, 128, 197, 198, 250, 319, 369):
+        for number_of_row in (5, rank + 7):                       # of c, of the rotated part
+            if number_of_row >= rank and number != number or number_of_row < rank:
+                held = cache.clone()
+                held[table[0, key // 64].long(), key % 64, number_of_row] = number
+                got = run(held)
+                sees = ((at >= key) & ((at - key < window) if window else (at >= 0))).to(DEV)
+                assert torch.equal(got[~sees], clean[~sees]), (key, number_of_row)
+                assert not torch.isfinite(got[sees].float()).any(), (key, number_of_row)
+
+
 @pytest.mark.parametrize("window", [0, 64, 200])
 def test_plan_covers_every_row_and_every_key_it_sees(window):
     from sonicboom_amd.ops import kernels as K
