@@ -115,6 +115,7 @@ class LatentAttention(Mixer):
         self.ukv = None
         if rt.fast_kernels and self.scale > 0.0 and ops.latent_built_ok(wdt, rt.cache_dtype, self.dim, self.rot_dim, self.vdim, self.rank):
             self.ukv = Linear(torch.cat([tensors["uk_weight"], tensors["uv_weight"]], dim=0).to(wdt), None, True)
+        self.built_key = ("latent_built", self.window, self.heads, self.dim, self.rot_dim, self.vdim, self.rank)
         # the matrix-core attention kernel takes a prompt step's rows in runs of this many
         if rt.fast_kernels and ops.latent_attention_mfma_ok(rt.act_dtype, rt.cache_dtype, self.rank, self.rot_dim):
             self.row_tile = ops.LATENT_ROW_TILE
@@ -144,10 +145,8 @@ class LatentAttention(Mixer):
             table if writes else None, self.heads, self.dim, self.rot_dim, self.rank, kv_rows=kv_rows,
             magnitude=self.magnitude)
         gate = pre[:, self.g_off:self.g_off + self.gate_cols]
-        plan = self._built_plan(ctx)
-        if plan is not None:
-            a = ops.latent_built_attention(q_plain, q_lat, lambda c: self.ukv(c, rt.act_dtype), cache, table, *plan[:2],
-                                           self.rank, self.vdim, self.scale, self.window, gate, self.gate_per_head)
+        a = self._over_built(ctx, q_plain, q_lat, cache, table, gate)
+        if a is not None:
             return self.out.add_into(a.view(a.shape[0], -1), x, then_norm, rt.act_dtype, scale=self.out_scale)
         ops.head_product(q_plain, self.uk, q_lat, fast=rt.fast_kernels)     # the first rank numbers of every head's query
         a_lat = ops.latent_attention(q_lat, cache, table, ctx, self.rank, self.scale, self.window, fast=rt.fast_kernels)
@@ -155,13 +154,26 @@ class LatentAttention(Mixer):
         ops.head_product(a_lat, self.uv, a, gate=gate, fast=rt.fast_kernels, gate_per_head=self.gate_per_head)
         return self.out.add_into(a.view(a.shape[0], -1), x, then_norm, rt.act_dtype, scale=self.out_scale)
 
-    def _built_plan(self, ctx):
+    def _over_built(self, ctx, q_plain, q_lat, cache, table, gate):
+        """Attention's result with keys and values built, or None where the step stays in the latent's space: where that is faster, or
+        where memory does not hold them (the step's later layers then do not ask for it again)."""
+        shared = ctx.shared if ctx.shared is not None else {}
+        plan = self._built_plan(ctx, shared)
+        if plan is None:
+            return None
+        try:
+            return ops.latent_built_attention(q_plain, q_lat, lambda c: self.ukv(c, self.rt.act_dtype), cache, table, *plan[:2],
+                                              self.rank, self.vdim, self.scale, self.window, gate, self.gate_per_head)
+        except torch.OutOfMemoryError:
+            shared[self.built_key] = None
+        return None
+
+    def _built_plan(self, ctx, shared):
         """(runs of rows, pages, their host copies) on the device when the step is faster with keys and values built, else None.
         Layers of one window share a step's plan."""
         if self.ukv is None or ctx.is_decode:
             return None
-        shared = ctx.shared if ctx.shared is not None else {}
-        key = ("latent_built", self.window, self.heads, self.dim, self.rot_dim, self.vdim, self.rank)
+        key = self.built_key
         if key not in shared:
             shared[key] = None
             if ops.latent_built_pays(ctx.n_new, ctx.lengths_before, self.window, self.heads, self.dim, self.rot_dim, self.vdim, self.rank):

@@ -31,3 +31,60 @@ def test_a_scale_that_is_not_positive(scale):
         mixer, _, rt = layer(4, scale=scale, fast=fast)
         outs.append(mixer_harness(mixer, rt)(h, [330], WIDTH))
     part_close(outs[0], outs[1].cpu().numpy(), "bfloat16", f"scale {scale}")
+
+
+class Fed:
+    """A cache for one layer alone: sequences filled with anything, and steps over them."""
+
+    def __init__(self, mixer, rt, tokens, slots=4):
+        from sonicboom_amd.cache import PagedCache, group_entries
+        self.mixer, self.rt = mixer, rt
+        self.cache = PagedCache(group_entries({0: mixer.cache_spec().key()}), tokens, rt.cache_dtype, rt.device, None, max_slots=slots)
+        self.rows, v, group = self.cache.entry_views(0)
+        from sonicboom_amd.engine.model import LayerBinding
+        self.binding = LayerBinding(0, group, self.rows, v, True, None)
+
+    def fill(self, n):
+        """A sequence of n cached positions."""
+        slot = self.cache.alloc_slot()
+        if n:
+            self.cache.reserve([slot], [n])
+            self.cache.advance([slot], [n])
+        return slot
+
+    def step(self, slots, h, n_new, built=None, advance=True):
+        """(the layer's output for these rows, whether keys and values were built); built: False keeps them out."""
+        from sonicboom_amd.engine.step import StepContext, StepEntry
+        self.cache.reserve(slots, n_new)
+        ctx = StepContext(self.cache, [StepEntry(s, [0] * n, ()) for s, n in zip(slots, n_new)], self.rt.device, (self.mixer.row_tile,))
+        ctx.shared = {self.mixer.built_key: None} if built is False else {}
+        x = torch.zeros((sum(n_new), WIDTH), dtype=torch.float32, device=DEV)
+        self.mixer.forward(h.to(DEV).contiguous(), x, ctx, self.binding)
+        if advance:
+            self.cache.advance(slots, n_new)
+        else:
+            self.cache.trim(slots)
+        return x, ctx.shared.get(self.mixer.built_key) is not None
+
+
+def test_memory_that_does_not_hold_the_built_keys(monkeypatch):
+    """Under a limit that the built keys of 120,000 positions (370 MB) do not fit, the step stays in the latent's space."""
+    from sonicboom_amd import ops
+    monkeypatch.setattr(ops, "latent_built_pays", lambda *a: True)
+    mixer, _, rt = layer(4)
+    fed = Fed(mixer, rt, 120_064)
+    fed.rows.normal_()
+    slot, h = fed.fill(119_936), rand(64, WIDTH).to(BF16)
+    want, _ = fed.step([slot], h, [64], built=False, advance=False)
+    over, built = fed.step([slot], h, [64], advance=False)
+    assert built
+    part_close(over, want.cpu().numpy(), "bfloat16", "built against the latent's space")
+    del over
+    torch.cuda.empty_cache()
+    most = torch.cuda.memory_reserved() + (200 << 20)
+    torch.cuda.set_per_process_memory_fraction(most / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        got, built = fed.step([slot], h, [64], advance=False)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert not built and torch.equal(got, want)
