@@ -110,10 +110,9 @@ class LatentAttention(Mixer):
         wdt = rt.act_dtype
         self.uk = tensors["uk_weight"].to(wdt).reshape(H, self.dim, self.rank).transpose(1, 2).contiguous()
         self.uv = tensors["uv_weight"].to(wdt).reshape(H, self.vdim, self.rank).contiguous()
-        # for steps that build keys and values: both matrices stacked, a product's operand (the kernel hides a key by a score of
-        # minus infinity ahead of the scale, which then has to be positive)
+        # for steps that build keys and values: both matrices stacked, a product's operand
         self.ukv = None
-        if rt.fast_kernels and self.scale > 0.0 and ops.latent_built_ok(wdt, rt.cache_dtype, self.dim, self.rot_dim, self.vdim, self.rank):
+        if rt.fast_kernels and ops.latent_built_ok(wdt, rt.cache_dtype, self.dim, self.rot_dim, self.vdim, self.rank, self.scale):
             self.ukv = Linear(torch.cat([tensors["uk_weight"], tensors["uv_weight"]], dim=0).to(wdt), None, True)
         self.built_key = ("latent_built", self.window, self.heads, self.dim, self.rot_dim, self.vdim, self.rank)
         # the matrix-core attention kernel takes a prompt step's rows in runs of this many

@@ -22,13 +22,14 @@ def layer(heads, rank=512, window=0, scale=0.05, fast=True, **more):
     return build_part(spec, dev, rt), ref, rt
 
 
-@pytest.mark.parametrize("scale", [-0.05, 0.0])
-def test_a_scale_that_is_not_positive(scale):
-    """Scores times a negative number, and all alike: the layer's result is the plain kernels'."""
+@pytest.mark.parametrize("scale", [-0.05, 0.0, 0.109])
+def test_scales_that_stay_in_the_latents_space(scale):
+    """Scores times a negative number, all alike, and peaked: the layer's result is the plain kernels'."""
     h = rand(330, WIDTH).to(BF16)
     outs = []
     for fast in (True, False):
         mixer, _, rt = layer(4, scale=scale, fast=fast)
+        assert mixer.ukv is None
         outs.append(mixer_harness(mixer, rt)(h, [330], WIDTH))
     part_close(outs[0], outs[1].cpu().numpy(), "bfloat16", f"scale {scale}")
 
