@@ -4,9 +4,13 @@ import numpy as np
 import pytest
 import torch
 
-from test_gpu_rasizen import BF16, DEV, mixer_harness, part_close, part_tensors, rand
+import test_gpu_fitatar as fitatar
+from plain import fitatar_plain as P
+from plain import rasizen_plain as R
+from test_gpu_rasizen import BF16, DEV, close, config, latent, mixer_harness, part_close, part_tensors, rand, run_cuts
 
 DIM, ROT, VDIM, WIDTH = 128, 64, 128, 64
+EPS = 1e-5
 
 pytestmark = pytest.mark.gpu
 
@@ -16,10 +20,109 @@ def layer(heads, rank=512, window=0, scale=0.05, fast=True, **more):
     from sonicboom_amd.parts import Runtime, build_part
     from sonicboom_amd.parts.latent_attention import latent_attention_spec
     from sonicboom_amd.parts.position import rope_interleaved_spec
-    spec = latent_attention_spec("a.", WIDTH, heads, DIM, ROT, VDIM, rank, scale, rope_interleaved_spec(ROT, 1e4), window=window, eps=1e-5, **more)
+    spec = latent_attention_spec("a.", WIDTH, heads, DIM, ROT, VDIM, rank, scale, rope_interleaved_spec(ROT, 1e4), window=window, eps=EPS, **more)
     dev, ref = part_tensors(spec, "bfloat16", scale=0.2)
     rt = Runtime(torch.device(DEV), BF16, fast)
     return build_part(spec, dev, rt), ref, rt
+
+
+def in_64_bits(ref, h, heads, rank, window, scale):
+    mx = {"heads": heads, "dim": DIM, "rot_dim": ROT, "vdim": VDIM, "kv_rank": rank, "scale": scale, "rot": {"base": 1e4, "dims": ROT},
+          "mask": {"size": window}}
+    hn, at = h.float().numpy(), np.arange(len(h))
+    return R.latent_attention_mixer(hn, at, ref, "a.", mx, EPS, R.latent_kv(hn, at, ref, "a.", mx, EPS))
+
+
+def off(got, want):
+    return float(np.linalg.norm(got.double().cpu().numpy() - want) / np.linalg.norm(want))
+
+
+@pytest.mark.parametrize("heads, rank", [(1, 512), (2, 512), (4, 64), (16, 512)])
+@pytest.mark.parametrize("window", [0, 130])
+def test_a_layer_whole_and_in_portions(heads, rank, window):
+    """A prompt in one step, in two, and in five with single rows between them, whose windows have left pages behind; and how far the
+    built form and the latent's space are from 64 bits."""
+    mixer, ref, rt = layer(heads, rank, window)
+    h = rand(470, WIDTH).to(BF16)
+    want = in_64_bits(ref, h, heads, rank, window, 0.05)
+    error = {}
+    for cuts in ([470], [300, 170], [260, 64, 1, 1, 144]):
+        for form in (None, False):
+            fed = Fed(mixer, rt, 1024)
+            slot, at, outs, built = fed.fill(0), 0, [], []
+            for n in cuts:
+                out, b = fed.step([slot], h[at:at + n], [n], built=form)
+                outs.append(out)
+                built.append(b)
+                at += n
+            if window:
+                assert fed.cache.page_table(0, [slot])[0, 0] == -1
+            got = torch.cat(outs)
+            part_close(got, want, "bfloat16", f"cuts {cuts}, built {built}")
+            assert built[0] == (form is None) and not any(b for b, n in zip(built, cuts) if n == 1)
+            error[form] = max(error.get(form, 0.0), off(got, want))
+    # both round four times on the way (queries or keys, weights, latent results or values, results): the attention alone is between 0.94 and 1.06
+    # of the other's error, and all the layer's other roundings are the same
+    assert error[None] <= 1.1 * error[False], error
+
+
+def test_a_step_of_prompts_and_single_rows():
+    """A prompt, a sequence that goes on by 40 rows and one by a single row in one step: each has the result that it has alone."""
+    heads, rank = 4, 512
+    mixer, ref, rt = layer(heads, rank)
+    fed = Fed(mixer, rt, 4096)
+    rows, before = (300, 40, 1), (0, 77, 200)
+    h = [rand(k + n, WIDTH, seed=i).to(BF16) for i, (k, n) in enumerate(zip(before, rows))]
+    slots = [fed.fill(0) for _ in rows]
+    for s, k, x in zip(slots, before, h):
+        if k:
+            fed.step([s], x[:k], [k])
+    got, built = fed.step(slots, torch.cat([x[k:] for x, k in zip(h, before)]), list(rows))
+    assert built
+    for part, x, k in zip(got.split(rows), h, before):
+        part_close(part, in_64_bits(ref, x, heads, rank, 0, 0.05)[k:], "bfloat16", f"{len(x) - k} rows behind {k}")
+
+
+def test_queries_of_a_latent_a_gate_a_head_and_a_reader(monkeypatch):
+    """Stretched frequencies and a gate a head; and a second layer, with W_uk and W_uv of its own, that reads the first one's rows."""
+    from sonicboom_amd import ops
+    rank, q_rank, n = 512, 24, 330
+    scale = 3.0 / (0.3 * np.sqrt(q_rank * rank * (DIM + ROT)))
+    mixer, rt, ref, mx = fitatar.latent_mixer("bfloat16", 4, DIM, ROT, VDIM, rank, q_rank, scale, (4.0, 64, 16.0, 1.0))
+    reader, _, ref2, mx2 = fitatar.latent_mixer("bfloat16", 6, DIM, ROT, VDIM, rank, q_rank, scale, (4.0, 64, 16.0, 1.0), seed=50, own=False)
+    calls, whole = [], ops.latent_built_attention
+    monkeypatch.setattr(ops, "latent_built_attention", lambda *a, **kw: calls.append(a[0].shape[:2]) or whole(*a, **kw))
+    h, h2 = rand(n, WIDTH).to(BF16), rand(n, WIDTH, seed=9).to(BF16)
+    kept = P.latent_rows(mx, EPS, ref, "a.", h.float().numpy(), np.arange(n))
+    part_close(fitatar.mixer_harness(mixer, rt, WIDTH)(h, [n]), P.latent_attention(mx, EPS, ref, "a.", h.float().numpy(), kept), "bfloat16", "own rows")
+    both = fitatar.mixer_harness(mixer, rt, WIDTH, reader=reader)
+    want = P.latent_attention(mx2, EPS, ref2, "a.", h2.float().numpy(), kept)
+    for cuts in ([n], [200, 129, 1]):
+        part_close(both(h, cuts, reader_rows=h2), want, "bfloat16", f"a reader, cuts {cuts}")
+    assert calls[:3] == [(n, 4), (n, 4), (n, 6)] and calls.count((200, 6)) == 1
+
+
+def test_a_model_of_two_windows(monkeypatch, tmp_path):
+    """Layers without a window and with one, and a reader with another, in one step: whole, in portions and in portions that the engine cuts."""
+    import json
+    from safetensors.torch import load_file
+    from sonicboom_amd import ops
+    from sonicboom_amd.engine import DecoderModel, Engine
+    from sonicboom_amd.weights import write_random_model
+    cfg = config(160, 96, [latent(4, DIM, ROT, VDIM, 64, 0.07, 70, mlp=64), latent(2, DIM, ROT, VDIM, 64, 0.07, 0, kv_from=0),
+                           latent(4, DIM, ROT, VDIM, 40, 0.07, 0), latent(4, DIM, ROT, VDIM, 40, 0.07, 150, kv_from=2, mlp=64)], groups=2)
+    write_random_model(str(tmp_path), json.loads(json.dumps(cfg)), seed=5, dtype="bfloat16", device=None)
+    plain = {k: v.float().numpy().astype(np.float64) for k, v in load_file(str(tmp_path / "model.safetensors")).items()}
+    calls, whole = [], ops.latent_built_attention
+    monkeypatch.setattr(ops, "latent_built_attention", lambda *a, **kw: calls.append((a[0].shape[0], a[10])) or whole(*a, **kw))
+    tokens = [int(t) for t in np.random.default_rng(3).integers(0, 160, size=400)]
+    want = R.forward(cfg, plain, tokens)
+    model = DecoderModel.from_folder(str(tmp_path), "bfloat16")
+    eng = Engine(model, 64 * 20)
+    for cuts in ([400], [170, 1, 229]):
+        close(run_cuts(eng, tokens, cuts), want, "bfloat16", f"cuts {cuts}")
+    assert calls[:4] == [(400, 70), (400, 0), (400, 0), (400, 150)]
+    close(run_cuts(Engine(model, 64 * 20, max_step_rows=150), tokens, [400]), want, "bfloat16", "portions")
 
 
 @pytest.mark.parametrize("scale", [-0.05, 0.0, 0.109])
