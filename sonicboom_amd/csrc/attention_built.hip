@@ -8,7 +8,8 @@
 //   sb_built_attention  softmax attention of the queries' plain and rotated parts over [built key | r of the cached row]
 //                       and the built values, times the sigmoid of the output gate.
 // Nothing of it is kept after the step's layer.  Measured, 16 heads, 4,001 rows (us): per-head products and attention in the latent's space
-// 524, here 159 (gathering 6, building 28, attention 125); a prompt of 4,001 rows of the second design 5,490 -> 4,236.
+// 455, here 165 (gathering 8, building 29, attention 118), 2,048 rows 203 and 79, 300 rows 60.7 and 29.3; a prompt of 4,001 rows of the
+// second design 5,490 -> 4,236.
 #include "mfma.h"
 
 namespace {
@@ -39,12 +40,9 @@ built_gather_kernel(bf16_t *__restrict__ out, const bf16_t *__restrict__ cache, 
 // keys at one chunk, which meet every bank once; a value chunk four keys at four neighbouring ones (ds_read_b64_tr_b16).
 template <int CH>
 __device__ __forceinline__ constexpr int key_turned(int key) {
-  return CH == 16 ? key & 15 : CH == 8 ? (key >> 1) & 7 : (key >> 2) & 3;
+  return CH == 16 ? key & 15 : (key >> 1) & 7;
 }
-template <int CH>
-__device__ __forceinline__ constexpr int value_turned(int key) {
-  return CH == 16 ? (key & 3) << 2 : ((key >> 1) & 1) << 2;
-}
+__device__ __forceinline__ constexpr int value_turned(int key) { return (key & 3) << 2; }
 
 // Whether eight bfloat16 numbers are finite: one to the lowest bit of an exponent of ones carries into the sign's place.
 __device__ __forceinline__ bool finite(bf16x8_t v) {
@@ -79,8 +77,9 @@ struct BuiltArgs {
 // rows of a key each, are read turned.
 // What bounds it: a turn of two pages takes 2.6 to 2.9 us, its products 1.2 of them; fragments from LDS (320 KB a turn) and the
 // exponentials fall between the products of the waves that share a SIMD instead of beside them, and a block costs some 8 us beside
-// its turns.  4,001 rows of 16 heads 125 us (655 TFLOP/s), 2,048 rows 54, 300 rows 15.5, 8,000 rows of 32 heads 640 (1,035).  Blocks of
-// four waves that take every page, two a CU: 142, 75, 18.5 and 621, as a long run's pages come one after the other.
+// its turns.  4,001 rows of 16 heads 118 us (695 TFLOP/s), 2,048 rows 55, 300 rows 15.4 (14.6 without the look at values on the diagonal), 8,000
+// rows of 32 heads 750 (875).  Blocks of four waves that take every page, two a CU: 142, 75, 18.5 and 621 where these took 125, 54, 15.5 and
+// 640, as a long run's pages come one after the other.
 // Which blocks: the block number counts heads fastest, so that a multiple of eight heads has a head's blocks on one die, whose
 // L2 then holds its keys and values.
 template <int DP, int RD, int VD>
@@ -93,7 +92,7 @@ built_attention_kernel(BuiltArgs a) {
   constexpr int kK = SB_PAGE * CK, kR = SB_PAGE * CR, kV = SB_PAGE * CV, kBuf = kK + kR + kV;
   constexpr int kSteps = (DP + RD) / 16, DT = VD / 32;
   static_assert(DT % 2 == 0 && (DT * 8 + 2) * 2 * 256 * 4 <= 4 * kBuf * 16, "halves to exchange, and room for them");
-  static_assert((CK == 8 || CK == 16) && (CR == 4 || CR == 8) && (CV == 8 || CV == 16), "sizes that the orders in LDS know");
+  static_assert((CK == 8 || CK == 16) && (CR == 8 || CR == 16) && CV == 16, "sizes that the orders in LDS know");
   extern __shared__ bf16x8_t lds_built[];                        // [2 halves of the waves][2][keys | rotated parts | values]
   const int lane = threadIdx.x & 63, wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = wave8 >> 2, wave = wave8 & 3;
@@ -143,7 +142,7 @@ built_attention_kernel(BuiltArgs a) {
     const int kk = wave * (64 / CK) + lane / CK, kr = wave * (64 / CR) + lane / CR, kv = wave * (64 / CV) + lane / CV;
     off_k = uint32_t(kk) * row_bytes + uint32_t((lane % CK) ^ key_turned<CK>(kk)) * 16 + uint32_t(head * DP) * 2;
     off_r = uint32_t(kr) * latent_bytes + uint32_t((lane % CR) ^ key_turned<CR>(kr)) * 16 + uint32_t(a.rank) * 2;
-    off_v = uint32_t(kv) * row_bytes + uint32_t((lane % CV) ^ value_turned<CV>(kv)) * 16 + uint32_t(a.heads * DP + head * VD) * 2;
+    off_v = uint32_t(kv) * row_bytes + uint32_t((lane % CV) ^ value_turned(kv)) * 16 + uint32_t(a.heads * DP + head * VD) * 2;
   }
   auto bring = [&](int pg, int buf) __attribute__((always_inline)) {
     const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc(
@@ -169,7 +168,7 @@ built_attention_kernel(BuiltArgs a) {
   // where this lane reads: key n of a score tile, chunk 2 s + h; keys 4 h + .. of a value quartet, in units of 8 bytes
   const int at_k = n * CK + (h ^ key_turned<CK>(n)), at_r = kK + n * CR + (h ^ key_turned<CR>(n));
   const int key_v = 4 * h + ((lane >> 2) & 3);
-  const int at_v = 2 * (kK + kR + key_v * CV + ((2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) ^ value_turned<CV>(key_v))) + (lane & 1);
+  const int at_v = 2 * (kK + kR + key_v * CV + ((2 * ((lane >> 4) & 1) + ((lane >> 1) & 1)) ^ value_turned(key_v))) + (lane & 1);
 
   int buf = 0;
   bool have = there(pg_lo + half);
@@ -354,10 +353,12 @@ built_attention_kernel(BuiltArgs a) {
 template <int DP, int RD, int VD>
 int launch_built(const BuiltArgs &a, int n_tiles, hipStream_t s) {
   constexpr int lds_bytes = 4 * SB_PAGE * (DP + RD + VD) * 2;
-  if (lds_bytes > 48 * 1024) {
+  static bool raised = false;     // per instantiation; harmless if repeated
+  if (!raised) {
     const hipError_t e = hipFuncSetAttribute((const void *)built_attention_kernel<DP, RD, VD>,
                                              hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes);
     SB_REQUIRE(e == hipSuccess, "sb_built_attention: cannot reserve %d bytes of LDS: %s", lds_bytes, hipGetErrorString(e));
+    raised = true;
   }
   built_attention_kernel<DP, RD, VD><<<unsigned(n_tiles) * unsigned(a.heads), 512, lds_bytes, s>>>(a);
   return sb::check_launch("sb_built_attention");

@@ -1420,7 +1420,7 @@ def latent_built_pays(n_new, before, window: int, heads: int, dim: int, rot_dim:
     results' way through memory (:func:`latent_attention_mfma`).  Measured on heads of 128 + 64 and 128 of a latent of 512, 6, 16 and
     32 heads, 2 to 1,500 rows behind 0 to 12,000 (latent's space / built, us, 16 heads): 40 rows 31.9 / 23.0, behind 400 42.3 / 31.6,
     behind 1,200 48.9 / 60.5; 250 43.7 / 28.7, behind 1,200 78.1 / 69.4, behind 3,500 104 / 122; 600 110 / 42, behind 3,500 214 / 141;
-    12 x 60 rows behind 150 63.1 / 47.2, 12 x 3 there 31.7 / 46.2; 4,001 rows 490 / 159.  Over 186 such steps the choice is 0.5 %
+    12 x 60 rows behind 150 63.1 / 47.2, 12 x 3 there 31.7 / 46.2; 4,001 rows 455 / 165.  Over 186 such steps the choice is 0.5 %
     behind the better side on the mean.  Over 104 steps each of whole layers with 1, 2, 3, 4, 8 and 16 heads, 2 to 4,000 rows behind 0 to
     12,000, without a window and with one of 512, it is 3.5, 0.7, 0.0, 0.1, 0.1 and 0.4 % behind (never to build: 8.3, 10.3, 15.9,
     17.5, 30.4 and 39.7; us, the layer in the latent's space / built: one head, 40 rows behind 400 53.1 / 47.2, 12 x 200 behind 150

@@ -35,7 +35,9 @@ def test_built_attention_equals_64_bits(heads, rank, gates, window):
     """Runs of one row, of whole tiles, one more and one less; rows that start and end on a page's first and last slot, an odd and an
     even count of pages; a page that is not there; slots that no row sees hold anything, a NaN among it."""
     from sonicboom_amd import ops
+    from sonicboom_amd.ops import kernels, library
     from sonicboom_amd.parts.linear import Linear
+    assert library.core().sb_built_tile_rows() == kernels.BUILT_ROW_TILE          # the plan lays out what a block takes
     latent, scale = rank + ROT, (DIM + ROT) ** -0.5
     seqs = [(0, 1), (0, 64), (63, 17), (190, 66), (511, 129), (0, 128), (300, 127)]           # (cached keys, rows)
     n_pages = [(k + n + 63) // 64 for k, n in seqs]
@@ -74,6 +76,65 @@ def test_built_attention_equals_64_bits(heads, rank, gates, window):
     got = ops.latent_built_attention(q_plain.to(DEV), q_latent.to(DEV), lambda c: build(c, BF16), dev[0], dev[1], dev[2], dev[3], rank, VDIM,
                                      scale, window, g, per_head).double().cpu()
     assert bool(((got - torch.cat(want)).abs() <= torch.cat(bound) + 1e-6).all())
+
+
+def finite_moves(s, at, window):
+    """How often the kernel's running maximum (in powers of two; a half of the waves takes every second page of a tile of 128 rows) moves from
+    a finite number, for scores s [rows, keys] of rows at positions ``at``."""
+    moves = 0
+    for t0 in range(0, len(at), 128):
+        lo = max(int(at[t0]) - window + 1, 0) if window else 0
+        last = int(at[min(t0 + 127, len(at) - 1)]) // 64
+        for half in range(2):
+            m = torch.full((min(128, len(at) - t0),), float("-inf"), dtype=torch.float64)
+            for page in range(lo // 64 + half, last + 1, 2):
+                mx = s[t0:t0 + 128, 64 * page:64 * page + 64].amax(-1) * 1.4426950408889634
+                move = mx > m + 8
+                moves += int((move & torch.isfinite(m)).sum())
+                m = torch.where(move, mx, m)
+    return moves
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("window", [0, 200])
+def test_built_attention_of_peaked_scores(window):
+    """Scores that climb by twelve powers of two a page for some rows, fall for others and stay for others still; and, a head on, keys
+    that stand out in every second page alone: maxima that move from a finite number, in some lanes of a wave and not in others, and
+    halves of a block whose maxima are far apart."""
+    from sonicboom_amd import ops
+    from sonicboom_amd.parts.linear import Linear
+    heads, rank, cached, n, scale = 3, 64, 190, 330, 0.07
+    keys = cached + n
+    pages_n = (keys + 63) // 64
+    cache = rand(pages_n * 64, rank + ROT, seed=3, scale=0.5)
+    page, step = torch.arange(pages_n * 64) // 64, 12 * np.log(2) / scale
+    cache[:, rank] = step / 16 * page.float()
+    cache[:, rank + 1], cache[:, rank + 2] = (page % 2).float() * step / 4, (page % 2 == 0).float() * step / 4
+    cache = cache.to(BF16).reshape(pages_n, 64, rank + ROT)
+    q_plain, q_latent = rand(n, heads, DIM, seed=4).to(BF16), rand(n, heads, rank + ROT, seed=5)
+    row = torch.arange(n)
+    q_latent[:, :, rank:rank + 3] = 0.0
+    q_latent[:, 0, rank] = torch.tensor([16.0, -16.0, 0.0])[row % 3]
+    q_latent[:, 1, rank + 1], q_latent[:, 1, rank + 2] = (row % 2) * 16.0, (row % 4 == 0) * 16.0
+    q_latent[:, 2, rank], q_latent[:, 2, rank + 1] = (row % 5 == 0) * 8.0, (row % 3 == 0) * -16.0
+    q_latent = q_latent.to(BF16)
+    uk, uv = rand(heads * DIM, rank, seed=6, scale=rank ** -0.5).to(BF16), rand(heads * VDIM, rank, seed=7, scale=rank ** -0.5).to(BF16)
+    rows = cache.reshape(-1, rank + ROT)[:keys]
+    want, bound = reference(q_plain, q_latent[:, :, rank:], rows, uk, uv, cached, window, scale, None)
+    # a score is 192 products added in float32, each rounding half a unit of what their absolute values add up to
+    k = (rows[:, :rank].float() @ uk.float().T).to(BF16).double().reshape(keys, heads, DIM)
+    terms = torch.einsum("tad,sad->ats", q_plain.double().abs(), k.abs()) + torch.einsum("tar,sr->ats", q_latent[:, :, rank:].double().abs(), rows[:, rank:].double().abs())
+    bound = bound * (1.0 + 2.0 ** 8 * 2 * 192 * 2.0 ** -24 * float(terms.max()) * scale)
+    s = (torch.einsum("tad,sad->ats", q_plain.double(), k) + torch.einsum("tar,sr->ats", q_latent[:, :, rank:].double(), rows[:, rank:].double())) * scale
+    at, j = torch.arange(cached, keys), torch.arange(keys)
+    seen = (j[None] <= at[:, None]) & ((at[:, None] - j[None] < window) if window else torch.ones(n, keys, dtype=torch.bool))
+    moves = [finite_moves(s[a].masked_fill(~seen, float("-inf")), at, window) for a in range(heads)]
+    assert moves[0] > 30 and moves[2] > 30, moves            # (head 1: a half of the waves has the pages that stand out)
+    tiles, pages = (torch.from_numpy(t).to(DEV) for t in ops.latent_built_plan([n], [cached], window))
+    build = Linear(torch.cat([uk, uv]).to(DEV), None, True)
+    got = ops.latent_built_attention(q_plain.to(DEV), q_latent.to(DEV), lambda c: build(c, BF16), cache.to(DEV), torch.arange(pages_n, device=DEV).int()[None],
+                                     tiles, pages, rank, VDIM, scale, window).double().cpu()
+    assert bool(((got - want).abs() <= bound + 1e-6).all())
 
 
 @pytest.mark.gpu
