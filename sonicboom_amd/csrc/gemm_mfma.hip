@@ -1,7 +1,8 @@
 // bf16 matrix product for many rows (prefill):  Y[t,n] = sum_k X[t,k] W[n,k]
 // on the matrix cores, with the model's epilogues fused: bias, float32
-// residual, gate activation, float32 or bfloat16 output.  Four kernels: this one, of any inner size in
-// eights and weights of either layout, and three below it that load packed weights and rows straight into LDS.
+// residual, gate activation, float32 or bfloat16 output.  Five kernels: this one, of any inner size in
+// eights and weights of either layout, three below it that load packed weights and rows straight into LDS, and one of gated products
+// that loads rows so and keeps weights in registers.
 //
 // A block of 2 x NW waves owns a BM x BN tile of Y (128 x 128, 256 x 128 or
 // 256 x 256) and walks K in stages of BK.  Both operand tiles go
@@ -1105,15 +1106,16 @@ gemm_pipe_half_kernel(Args a) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// The gated product of up to two hundred rows, whose weights are most of what there is to read.  What bounds it in the forms above
-// is how much of W a CU has on its way (three stages in LDS, beside X's): memory answers in some 2 us, and 48 KB in that time are
+// The gated product whose tiles of 96, 128 or 192 rows make one round over the CUs: some hundred rows of wide matrices, whose weights
+// are most of what there is to read, up to some thousand of narrow ones.  What bounds it in the forms above is how much of W a CU has on its way (three stages in LDS, beside X's): memory answers in some 2 us, and 48 KB in that time are
 // 24 GB/s a CU.  Here W never passes through LDS: a wave owns 16 columns of either half, whose packed blocks are the matrix
 // instruction's fragments as they lie, and keeps kDeep stages of 64 k of them in registers on their way.  Rows of X, which the block's four such
 // waves share, are brought into LDS by two waves that do nothing else: loads return in order, so that waiting for a stage of X
 // would also wait for the weights that were asked for before it.  One barrier a stage.
 // us, the form taken before and this one (rows x 2 halves of W x k): 183 x 17,920 x 1,536 26.0 and 22.4 (a read of W alone 11),
 // 96 rows 20.4 and 17.7, 192 x 22,016 x 2,048 32.7 and 28.4, 260 x 11,008 x 2,048 31.4 and 23.0, 288 x 9,728 x 896 12.6 and 9.2; prompts
-// of 288 rows of the 0.5B sizes 1,519 -> 1,454, 183 rows of the 1.5B ones 2,614 -> 2,514.  Tiles of 96 and 192 rows straight into LDS as
+// of 288 rows of the 0.5B sizes 1,519 -> 1,454, 183 rows of the 1.5B ones 2,614 -> 2,514; narrow matrices (2 x 512 x 2,048) 1,040 rows
+// 19.2 and 14.1, 2,048 20.9 and 18.3, 3,072 35.6 and 24.5, (2 x 128 x 512) 8,208 10.4 and 7.4, 288 rows x 11,008 x 512 11.6 and 10.7.  Tiles of 96 and 192 rows straight into LDS as
 // above were ahead by themselves (10.7 and 25.5) and not in whole steps.
 // RT: tiles of 16 rows of a block.  The weights are the first operand, so that a lane ends up with four neighbouring
 // columns of a row.
@@ -1503,7 +1505,7 @@ int gemm_whole(void *y, int y_dtype, const void *x, const void *w, const void *b
     else if (gated && n_rows <= 384 && tiles <= sb::cu_count() * 3 / 2 && (n_rows + 63) / 64 * 64 < (n_rows + 127) / 128 * 128)
       variant = 5, path = 2;
   }
-  // a test's or a measurement's choice: the shape (0..5) + 16 * the path (0: the launcher's, 1:
+  // a test's or a measurement's choice: the shape (0..8) + 16 * the path (0: the launcher's, 1:
   // through registers, 2: straight into LDS)
   if (tile_shape >= 0) {
     SB_REQUIRE((tile_shape & 15) < 9 && (tile_shape >> 4) < 4, "sb_gemm_mfma_bf16: unknown tile shape %d", tile_shape);

@@ -241,7 +241,7 @@ top_part_kernel(uint64_t *__restrict__ part_keys, const float *__restrict__ logi
 
 // Stage 2, or the only stage of a short row: one block per row finds the k largest keys among the
 // row's (FROM_KEYS: among the n_keys that stage 1 left in part_keys, at most kRowKeys * 1024; else
-// among the keys of its vocab <= kRowKeys * 1024 logits), sorts them (bitonic, in shared memory)
+// among the keys of its vocab <= kRowKeys * 1024 logits), puts them in order by counting larger ones
 // and writes ids and z.
 constexpr int kRowKeys = 16;
 template <bool FROM_KEYS>

@@ -65,7 +65,7 @@ def latent_attention_spec(prefix: str, width: int, heads: int, dim: int, rot_dim
 @register_part("mixer", "latent_attention")
 class LatentAttention(Mixer):
     fuses_norm = True
-    graph_safe = True     # its launches depend on device buffers only
+    graph_safe = True     # launches of single-token steps depend on device buffers only (those of prompts follow a plan of the host's)
 
     def __init__(self, spec, tensors, parts, rt):
         super().__init__(spec, tensors, parts, rt)

@@ -58,6 +58,21 @@ def test_gated_products_with_weights_through_registers(shape, t, inner, k):
         assert torch.equal(half, got.to(BF16)), act
 
 
+@pytest.mark.parametrize("inner, rows", [(1024, (1024, 1536, 2048, 3072)), (64, (16384,)), (11008, (65, 96))])
+def test_gated_products_on_either_side_of_a_round_of_tiles(inner, rows):
+    """The launcher's own choice where 64, 96, 128 and 192 rows a tile cease to make one round over 256 CUs, many rows of narrow weights
+    among it: the bits of the kernel that stages tiles through registers."""
+    from sonicboom_amd import ops
+    k = 448
+    packed = ops.pack_weight(randn(2 * inner, k, seed=k, scale=0.05).to(DEV, BF16), True)
+    for t in sorted({n + d for n in rows for d in (0, 1)}):
+        x = randn(t, k, seed=t).to(DEV, BF16)
+        got = ops.gemm_bf16(x, packed, None, None, F32, gated="silu", packed_shape=(2 * inner, k))
+        with ops.gemm_tile_shape(0, "registers"):
+            want = ops.gemm_bf16(x, packed, None, None, F32, gated="silu", packed_shape=(2 * inner, k))
+        assert torch.equal(got, want), t
+
+
 def xielu(z, p, q):
     z = z.double().numpy()
     rise, bend = np.log1p(np.exp(p)), 0.5 + np.log1p(np.exp(q))
@@ -76,6 +91,19 @@ def test_xielu_against_64_bits(n):
     want = xielu(z, 0.4, -0.3)
     # some eight roundings of terms that the result and z / 2 bound
     assert (np.abs(got - want) <= 8 * 2.0 ** -23 * (np.abs(want) + np.abs(z.numpy()))).all()
+
+
+@pytest.mark.parametrize("n", [12, (1 << 23) + 4])
+def test_xielu_of_numbers_that_are_not_finite(n):
+    """NaN and minus infinity give a NaN (infinity less infinity), infinity stays, zeros of either sign give zero, and the smallest and the
+    largest numbers below zero what 64 bits give."""
+    from sonicboom_amd import ops
+    z = torch.zeros(n)
+    z[:9] = torch.tensor([float("nan"), float("inf"), float("-inf"), -0.0, 0.0, -1.0e-38, -1.0e-20, -200.0, -1.0e30])
+    got = ops.activate(z.to(DEV), F32, "xielu", torch.tensor([0.4, -0.3], device=DEV)).cpu()
+    assert torch.isnan(got[0]) and got[1] == float("inf") and torch.isnan(got[2]) and (got[3:5] == 0).all() and (got[9:] == 0).all()
+    want = torch.from_numpy(xielu(z[5:9], 0.4, -0.3))
+    assert ((got[5:9].double() - want).abs() <= 8 * 2.0 ** -23 * (want.abs() + z[5:9].abs())).all()
 
 
 @pytest.mark.parametrize("t, n, k", [(4001, 4096, 128), (4096, 4094, 192), (4001, 8192, 320)])
