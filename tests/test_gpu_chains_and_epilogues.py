@@ -73,6 +73,27 @@ def test_gated_products_on_either_side_of_a_round_of_tiles(inner, rows):
         assert torch.equal(got, want), t
 
 
+@pytest.mark.parametrize("count", [1, 2, 15, 16, 17, 32, 33, 64, 65, 255, 256])
+def test_top_p_that_ends_on_either_side_of_a_run(count):
+    """Shares that the first, the last and the candidates around every sixteenth reach exactly, just not, and just."""
+    from plain import sampling_plain as SP
+    from sonicboom_amd import ops
+    z = (-0.02 * np.arange(count)).astype(np.float32)
+    ids = np.random.default_rng(count).permutation(5000)[:count].astype(np.int32)
+    e = np.exp(z.astype(np.float64) - float(z[0]))
+    shares = np.cumsum(e) / np.cumsum(e)[-1]
+    seed, positions = 99, [3, 4000, 77]
+    on_gpu = [torch.from_numpy(np.repeat(a[None], 3, 0).copy()).to(DEV) for a in (ids, z)]
+    for c in sorted({i for i in (0, 14, 15, 16, 17, 31, 32, 63, 64, count - 2, count - 1) if 0 <= i < count}):
+        for share in (shares[c], np.nextafter(shares[c], 0.0), np.nextafter(shares[c], 1.0)):
+            top_p = float(np.float32(share))
+            if not 0.0 < top_p < 1.0:
+                continue
+            kept = SP.filter_candidates(list(zip(ids.tolist(), z.tolist())), 0, top_p, 0.0)
+            got = ops.draw(*on_gpu, positions, 0, None, top_p, seed).tolist()
+            assert got == [SP.draw(kept, seed, p) for p in positions], (c, top_p)
+
+
 def xielu(z, p, q):
     z = z.double().numpy()
     rise, bend = np.log1p(np.exp(p)), 0.5 + np.log1p(np.exp(q))
