@@ -138,6 +138,8 @@ __device__ __forceinline__ uint64_t cand_key(float logit, float temperature, int
 // equal z at the cut.  A key of 0 stands for "nothing" and lies below every real key; `want` must
 // not exceed the number of real keys.  Every thread of the block calls it and gets the same key:
 // exactly `want` of the real keys are greater or equal.
+// ADAPT: a wave whose keys are spread over many buckets stops voting (stage 1, where many rows fill the chip with blocks: 256 rows of
+// 151,936 logits, spread over four orders, 182 us without votes, 206 with all of them, 187 so; masked rows, all alike, 1,157, 352, 340).
 struct SelectShared {
   uint32_t hist[kSelWaves][256];
   uint32_t wave_total[4];
@@ -145,7 +147,7 @@ struct SelectShared {
   int remaining;
 };
 
-template <int PER>
+template <int PER, bool ADAPT>
 __device__ __forceinline__ uint64_t select_kth(const uint64_t (&mine)[PER], int want, SelectShared &sh) {
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   if (tid == 0) {
@@ -159,23 +161,29 @@ __device__ __forceinline__ uint64_t select_kth(const uint64_t (&mine)[PER], int 
     const uint64_t prefix = sh.prefix;
     const uint32_t remaining = uint32_t(sh.remaining);
     if (remaining == 0) break;          // (uniform) the cut is found
+    bool voting = true;
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const uint64_t key = mine[j];
       const uint32_t bucket = uint32_t(key >> shift) & 0xffu;
       bool counts = pass == 7 || (key >> (shift + 8)) == (prefix >> (shift + 8));
       // Logits agree in sign and mostly in the exponent: lanes that add to one counter do so one after the other, so up to two
-      // buckets of a wave's keys are counted by a vote first.  (With the ranks below, the second stage of three rows of 32,768
-      // logits takes 14.0 us for 25.4.)
+      // buckets of a wave's keys are counted by a vote first.  (With the ranks below, three rows of 32,768 logits take 21.6 us for
+      // 32.6.)
+      if (voting) {
+        uint64_t left = __ballot(counts);
+        const int all = __popcll(left);
 #pragma unroll
-      for (int vote = 0; vote < 2; ++vote) {
-        const uint64_t left = __ballot(counts);
-        if (left == 0) break;
-        const int leader = __ffsll((unsigned long long)left) - 1;
-        const uint32_t its = __builtin_amdgcn_readlane(bucket, leader);
-        const uint64_t same = __ballot(counts && bucket == its);
-        if (lane == leader) atomicAdd(&sh.hist[wave][its], uint32_t(__popcll(same)));
-        counts = counts && bucket != its;
+        for (int vote = 0; vote < 2; ++vote) {
+          if (left == 0) break;
+          const int leader = __ffsll((unsigned long long)left) - 1;
+          const uint32_t its = __builtin_amdgcn_readlane(bucket, leader);
+          const uint64_t same = __ballot(counts && bucket == its);
+          if (lane == leader) atomicAdd(&sh.hist[wave][its], uint32_t(__popcll(same)));
+          counts = counts && bucket != its;
+          left &= ~same;
+        }
+        if (ADAPT) voting = 4 * __popcll(left) <= all;
       }
       if (counts) atomicAdd(&sh.hist[wave][bucket], 1u);
     }
@@ -230,7 +238,7 @@ top_part_kernel(uint64_t *__restrict__ part_keys, const float *__restrict__ logi
   if (tid < kMaxCand) out[tid] = 0;
   if (tid == 0) count_s = 0;
   const int real = min(kPartElems, vocab - first);
-  const uint64_t kth = select_kth<PER>(mine, min(kMaxCand, real), sh);   // syncs inside
+  const uint64_t kth = select_kth<PER, true>(mine, min(kMaxCand, real), sh);   // syncs inside
 #pragma unroll
   for (int j = 0; j < PER; ++j)
     if (mine[j] >= kth && mine[j] != 0) {
@@ -265,7 +273,7 @@ top_candidates_kernel(int32_t *__restrict__ cand_id, float *__restrict__ cand_z,
   }
   if (tid == 0) count_s = 0;
   for (int i = tid; i < kMaxCand; i += kSelThreads) sel[i] = 0;
-  const uint64_t kth = select_kth<kRowKeys>(mine, want, sh);              // syncs inside
+  const uint64_t kth = select_kth<kRowKeys, false>(mine, want, sh);              // syncs inside
 #pragma unroll
   for (int j = 0; j < kRowKeys; ++j)
     if (mine[j] >= kth && mine[j] != 0) {

@@ -94,6 +94,20 @@ def test_top_p_that_ends_on_either_side_of_a_run(count):
             assert got == [SP.draw(kept, seed, p) for p in positions], (c, top_p)
 
 
+@pytest.mark.parametrize("vocab", [900, 16384, 40003])
+def test_candidates_of_rows_alike_spread_and_masked(vocab):
+    """Logits of a few values, over many orders, and all but a few of them masked: waves that count by votes and waves that stop."""
+    from plain import sampling_plain as SP
+    from sonicboom_amd import ops
+    g = np.random.default_rng(vocab)
+    rows = np.stack([np.zeros(vocab), g.integers(0, 3, vocab) * 0.5, g.standard_normal(vocab) * 10.0 ** g.integers(-6, 5, vocab),
+                     np.where(g.random(vocab) < 0.01, g.standard_normal(vocab), -1.0e30), g.standard_normal(vocab)]).astype(np.float32)
+    ids, z = ops.top_candidates(torch.from_numpy(rows).to(DEV), 0.7, 256)
+    for r, row in enumerate(rows):
+        want = SP.select_candidates(row, 0.7)
+        assert [c[0] for c in want] == ids[r].tolist() and [np.float32(c[1]) for c in want] == z[r].tolist(), r
+
+
 def xielu(z, p, q):
     z = z.double().numpy()
     rise, bend = np.log1p(np.exp(p)), 0.5 + np.log1p(np.exp(q))
