@@ -1420,11 +1420,11 @@ def latent_built_pays(n_new, before, window: int, heads: int, dim: int, rot_dim:
     results' way through memory (:func:`latent_attention_mfma`).  Measured on heads of 128 + 64 and 128 of a latent of 512, 6, 16 and
     32 heads, 2 to 1,500 rows behind 0 to 12,000 (latent's space / built, us, 16 heads): 40 rows 31.9 / 23.0, behind 400 42.3 / 31.6,
     behind 1,200 48.9 / 60.5; 250 43.7 / 28.7, behind 1,200 78.1 / 69.4, behind 3,500 104 / 122; 600 110 / 42, behind 3,500 214 / 141;
-    12 x 60 rows behind 150 63.1 / 47.2, 12 x 3 there 31.7 / 46.2; 4,001 rows 455 / 165.  Over 186 such steps the choice is 0.5 %
-    behind the better side on the mean.  Over 104 steps each of whole layers with 1, 2, 3, 4, 8 and 16 heads, 2 to 4,000 rows behind 0 to
-    12,000, without a window and with one of 512, it is 3.5, 0.7, 0.0, 0.1, 0.1 and 0.4 % behind (never to build: 8.3, 10.3, 15.9,
-    17.5, 30.4 and 39.7; us, the layer in the latent's space / built: one head, 40 rows behind 400 53.1 / 47.2, 12 x 200 behind 150
-    87.2 / 65.8, 250 behind 1,200 in the window 53.9 / 58.8; two heads, 330 rows 62 / 50)."""
+    12 x 60 rows behind 150 63.1 / 47.2, 12 x 3 there 31.7 / 46.2; 4,001 rows 455 / 165.  Over 104 steps each of whole layers with 1,
+    2, 3, 4, 8 and 16 heads, 2 to 4,000 rows behind 0 to 12,000, without a window and with one of 512, the choice is 3.5, 0.8, 0.4,
+    0.2, 0.1 and 0.2 % behind the better side on the mean (never to build: 8.3, 10.3, 15.9, 17.5, 30.4 and 39.7), and no step of three
+    heads or more is more than 2.5 % slower for it (us, the layer in the latent's space / built: one head, 40 rows behind 400 53.1 /
+    47.2, 12 x 200 behind 150 87.2 / 65.8, 250 behind 1,200 in the window 53.9 / 58.8; two heads, 330 rows 62 / 50)."""
     n, k = np.asarray(n_new, dtype=np.int64), np.asarray(before, dtype=np.int64)
     first = np.maximum(k - window + 1, 0) if window > 0 else np.zeros_like(k)
     pages = (k + n - 1) // PAGE - first // PAGE + 1
@@ -1433,14 +1433,15 @@ def latent_built_pays(n_new, before, window: int, heads: int, dim: int, rot_dim:
     if keys * (per_key + rank) * 2 > BUILT_MOST_BYTES:
         return False
     seen = (k + 1 + k + n) / 2.0                                    # by a row, on the mean
-    most = k + n
+    most, of_tile = k + n, k + n                                    # keys that a row sees at most, and a tile of rows
     if window > 0:
         seen, most = np.minimum(seen, window), np.minimum(most, window)
+        of_tile = np.minimum(of_tile, window + np.minimum(n, BUILT_ROW_TILE) - 1)
     pairs, rows, longest = float((n * seen).sum()), int(n.sum()), int(most.max())
     runs = -(-n // BUILT_ROW_TILE)
     tile_pages = float((runs * (seen / PAGE + 1.0)).sum())
     product = 2.0 * (dim + vdim) * rank * heads
-    built = 19.5 + max(1.25 * (longest / PAGE + 1), 1.5 * tile_pages * heads / SPLIT_CUS) + keys * product / 5.5e8
+    built = 22.5 + max(1.25 * (int(of_tile.max()) / PAGE + 1), 1.5 * tile_pages * heads / SPLIT_CUS) + keys * product / 5.5e8
     blocks = int((-(-n // LATENT_ROW_TILE)).sum()) * -(-heads // 4)
     splits = latent_splits(blocks, longest)
     plain = 25.0 + max(1.8 * (longest / PAGE / splits), pairs * heads * 2.0 * (2 * rank + rot_dim) / 6.5e8) + rows * product / 3.5e8

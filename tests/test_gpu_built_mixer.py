@@ -15,6 +15,13 @@ EPS = 1e-5
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def every_prompt_builds(monkeypatch):
+    """Whatever the price says of a step."""
+    from sonicboom_amd import ops
+    monkeypatch.setattr(ops, "latent_built_pays", lambda *a: True)
+
+
 def layer(heads, rank=512, window=0, scale=0.05, fast=True, **more):
     """(the mixer, its tensors in float64, its runtime)."""
     from sonicboom_amd.parts import Runtime, build_part
@@ -64,6 +71,19 @@ def test_a_layer_whole_and_in_portions(heads, rank, window):
     # both round four times on the way (queries or keys, weights, latent results or values, results): the attention alone is between 0.94 and 1.06
     # of the other's error, and all the layer's other roundings are the same
     assert error[None] <= 1.1 * error[False], error
+
+
+def test_the_price_leads_a_step(monkeypatch):
+    """A prompt's rows over few keys go over built keys, few rows behind many do not."""
+    from sonicboom_amd import ops
+    from sonicboom_amd.ops import kernels
+    asked = []
+    monkeypatch.setattr(ops, "latent_built_pays", lambda *a: asked.append(a) or kernels.latent_built_pays(*a))
+    mixer, _, rt = layer(2)
+    fed = Fed(mixer, rt, 20_000)
+    fed.rows.normal_()
+    assert fed.step([fed.fill(0)], rand(300, WIDTH).to(BF16), [300])[1] and not fed.step([fed.fill(12_000)], rand(3, WIDTH).to(BF16), [3])[1]
+    assert [a[:3] for a in asked] == [([300], [0], 0), ([3], [12_000], 0)]
 
 
 def test_a_step_of_prompts_and_single_rows():
@@ -171,10 +191,8 @@ class Fed:
         return x, ctx.shared.get(self.mixer.built_key) is not None
 
 
-def test_memory_that_does_not_hold_the_built_keys(monkeypatch):
+def test_memory_that_does_not_hold_the_built_keys():
     """Under a limit that the built keys of 120,000 positions (370 MB) do not fit, the step stays in the latent's space."""
-    from sonicboom_amd import ops
-    monkeypatch.setattr(ops, "latent_built_pays", lambda *a: True)
     mixer, _, rt = layer(4)
     fed = Fed(mixer, rt, 120_064)
     fed.rows.normal_()
