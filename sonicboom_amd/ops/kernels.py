@@ -1398,6 +1398,7 @@ def latent_attention(q: torch.Tensor, cache: torch.Tensor, page_table: torch.Ten
 BUILT_ROW_TILE = 128        # rows of a run that a block of the kernel over built keys takes (sb_built_tile_rows)
 BUILT_MOST_BYTES = 2 << 30  # of built keys and values (and the latents they are built from) that a step's layer may hold
 BUILT_MOST_SCALE = 1.5      # of the scores, times the square root of a key's numbers
+BUILT_LEAST_RANK = 256      # of the latents
 
 
 def latent_built_ok(act_dtype, cache_dtype, dim: int, rot_dim: int, vdim: int, rank: int, scale: float) -> bool:
@@ -1406,25 +1407,24 @@ def latent_built_ok(act_dtype, cache_dtype, dim: int, rot_dim: int, vdim: int, r
     space queries and results are, and where a row's weight lies on few keys these roundings tell more: the result's error against 64 bits
     over the latent space's, normal queries and keys, 2 and 16 heads, 200 to 2,000 rows, scales of 0.5, 1, 1.5, 2, 3 and 6 over the root of
     a key's numbers: 0.96 to 1.02, 0.94 to 1.01, 0.98 to 1.00, 1.00 to 1.04, 1.00 to 1.07, 1.02 to 1.06.  Larger scales stay in
-    the latent's space."""
+    the latent's space, and so do smaller latents, which cost little more there than built keys (latents of 64 and 128 numbers: built
+    where the price below has it, a layer of 16 heads is 1.04 and 0.96 of the latent's space's time, of 4 heads 1.13 and 1.09)."""
     return act_dtype == torch.bfloat16 and cache_dtype == torch.bfloat16 \
-        and 0.0 < scale <= BUILT_MOST_SCALE / (dim + rot_dim) ** 0.5 \
+        and rank >= BUILT_LEAST_RANK and 0.0 < scale <= BUILT_MOST_SCALE / (dim + rot_dim) ** 0.5 \
         and bool(library.core().sb_built_attention_ok(int(dim), int(rot_dim), int(vdim), int(rank)))
 
 
 def latent_built_pays(n_new, before, window: int, heads: int, dim: int, rot_dim: int, vdim: int, rank: int) -> bool:
     """Whether a step of ``n_new[i]`` rows behind ``before[i]`` cached ones is faster with every head's keys and values built
-    than in the latent's space: a price of both in microseconds.  Built: three launches, the longest run's pages at 1.25 us (two a
-    turn) or all pages at 1.5 us a page, run and CU, and the product that builds.  In the latent's space: three launches, the
+    than in the latent's space: a price of both in microseconds.  Built: three launches, the longest run's pages (two a
+    turn) or all pages at 1.52 us a page, run and CU, and the product that builds.  In the latent's space: three launches, the
     arithmetic of the pairs or the longest share's pages, the per-head products and, where keys are shared out, the partial
-    results' way through memory (:func:`latent_attention_mfma`).  Measured on heads of 128 + 64 and 128 of a latent of 512, 6, 16 and
-    32 heads, 2 to 1,500 rows behind 0 to 12,000 (latent's space / built, us, 16 heads): 40 rows 31.9 / 23.0, behind 400 42.3 / 31.6,
-    behind 1,200 48.9 / 60.5; 250 43.7 / 28.7, behind 1,200 78.1 / 69.4, behind 3,500 104 / 122; 600 110 / 42, behind 3,500 214 / 141;
-    12 x 60 rows behind 150 63.1 / 47.2, 12 x 3 there 31.7 / 46.2; 4,001 rows 455 / 165.  Over 104 steps each of whole layers with 1,
-    2, 3, 4, 8 and 16 heads, 2 to 4,000 rows behind 0 to 12,000, without a window and with one of 512, the choice is 3.5, 0.8, 0.4,
-    0.2, 0.1 and 0.2 % behind the better side on the mean (never to build: 8.3, 10.3, 15.9, 17.5, 30.4 and 39.7), and no step of three
-    heads or more is more than 2.5 % slower for it (us, the layer in the latent's space / built: one head, 40 rows behind 400 53.1 /
-    47.2, 12 x 200 behind 150 87.2 / 65.8, 250 behind 1,200 in the window 53.9 / 58.8; two heads, 330 rows 62 / 50)."""
+    results' way through memory (:func:`latent_attention_mfma`).  Fitted to whole layers of 1 to 16 heads of 128 + 64 and 128 numbers
+    and latents of 256 and 512, 104 steps each of 2 to 4,000 rows behind 0 to 12,000, without a window and with one of 512, and looked
+    at with 4 to 32 heads of 256, 384 and 512: no step is more than 1.5 % slower for the choice, and on the mean it is 0.3 to 2.0 % behind
+    the better side (never to build: 2.0 % with 2 heads of 256, 10.3 of 512, with 16 18.4 and 39.7).  Us, the layer in the latent's
+    space / built, a latent of 512: 16 heads, 40 rows 54.1 / 46.1, 250 behind 1,200 103.9 / 95.0, 4,001 rows 455 / 165 (attention and
+    its products alone); one head, 40 rows behind 400 53.1 / 47.2; two heads, 330 rows 62 / 50."""
     n, k = np.asarray(n_new, dtype=np.int64), np.asarray(before, dtype=np.int64)
     first = np.maximum(k - window + 1, 0) if window > 0 else np.zeros_like(k)
     pages = (k + n - 1) // PAGE - first // PAGE + 1
@@ -1441,12 +1441,13 @@ def latent_built_pays(n_new, before, window: int, heads: int, dim: int, rot_dim:
     runs = -(-n // BUILT_ROW_TILE)
     tile_pages = float((runs * (seen / PAGE + 1.0)).sum())
     product = 2.0 * (dim + vdim) * rank * heads
-    built = 22.5 + max(1.25 * (int(of_tile.max()) / PAGE + 1), 1.5 * tile_pages * heads / SPLIT_CUS) + keys * product / 5.5e8
+    built = 24.0 + max(1.08 * (int(of_tile.max()) / PAGE + 1), 1.52 * tile_pages * heads / SPLIT_CUS) + keys * product / 4.76e8
     blocks = int((-(-n // LATENT_ROW_TILE)).sum()) * -(-heads // 4)
     splits = latent_splits(blocks, longest)
-    plain = 25.0 + max(1.8 * (longest / PAGE / splits), pairs * heads * 2.0 * (2 * rank + rot_dim) / 6.5e8) + rows * product / 3.5e8
+    plain = 18.3 + 0.0143 * rank + max((0.81 + 0.0041 * rank) * (longest / PAGE / splits),
+                                       pairs * heads * 2.0 * (2 * rank + rot_dim) / 5.88e8) + rows * product / 3.23e8
     if splits > 1:
-        plain += 9.0 + splits * rows * heads * rank * 8.0 / 4e6
+        plain += 2.0 + splits * rows * heads * rank * 8.0 / 4.14e6
     return bool(built < plain)
 
 

@@ -44,7 +44,7 @@ def off(got, want):
     return float(np.linalg.norm(got.double().cpu().numpy() - want) / np.linalg.norm(want))
 
 
-@pytest.mark.parametrize("heads, rank", [(1, 512), (2, 512), (4, 64), (16, 512)])
+@pytest.mark.parametrize("heads, rank", [(1, 512), (2, 512), (4, 256), (16, 512)])
 @pytest.mark.parametrize("window", [0, 130])
 def test_a_layer_whole_and_in_portions(heads, rank, window):
     """A prompt in one step, in two, and in five with single rows between them, whose windows have left pages behind; and how far the
@@ -129,8 +129,8 @@ def test_a_model_of_two_windows(monkeypatch, tmp_path):
     from sonicboom_amd import ops
     from sonicboom_amd.engine import DecoderModel, Engine
     from sonicboom_amd.weights import write_random_model
-    cfg = config(160, 96, [latent(4, DIM, ROT, VDIM, 64, 0.07, 70, mlp=64), latent(2, DIM, ROT, VDIM, 64, 0.07, 0, kv_from=0),
-                           latent(4, DIM, ROT, VDIM, 40, 0.07, 0), latent(4, DIM, ROT, VDIM, 40, 0.07, 150, kv_from=2, mlp=64)], groups=2)
+    cfg = config(160, 96, [latent(4, DIM, ROT, VDIM, 256, 0.07, 70, mlp=64), latent(2, DIM, ROT, VDIM, 256, 0.07, 0, kv_from=0),
+                           latent(4, DIM, ROT, VDIM, 264, 0.07, 0), latent(4, DIM, ROT, VDIM, 264, 0.07, 150, kv_from=2, mlp=64)], groups=2)
     write_random_model(str(tmp_path), json.loads(json.dumps(cfg)), seed=5, dtype="bfloat16", device=None)
     plain = {k: v.float().numpy().astype(np.float64) for k, v in load_file(str(tmp_path / "model.safetensors")).items()}
     calls, whole = [], ops.latent_built_attention
@@ -145,13 +145,13 @@ def test_a_model_of_two_windows(monkeypatch, tmp_path):
     close(run_cuts(Engine(model, 64 * 20, max_step_rows=150), tokens, [400]), want, "bfloat16", "portions")
 
 
-@pytest.mark.parametrize("scale", [-0.05, 0.0, 0.109])
-def test_scales_that_stay_in_the_latents_space(scale):
-    """Scores times a negative number, all alike, and peaked: the layer's result is the plain kernels'."""
+@pytest.mark.parametrize("scale, rank", [(-0.05, 512), (0.0, 512), (0.109, 512), (0.05, 248)])
+def test_layers_that_stay_in_the_latents_space(scale, rank):
+    """Scores times a negative number, all alike, and peaked, and latents of few numbers: the layer's result is the plain kernels'."""
     h = rand(330, WIDTH).to(BF16)
     outs = []
     for fast in (True, False):
-        mixer, _, rt = layer(4, scale=scale, fast=fast)
+        mixer, _, rt = layer(4, rank, scale=scale, fast=fast)
         assert mixer.ukv is None
         outs.append(mixer_harness(mixer, rt)(h, [330], WIDTH))
     part_close(outs[0], outs[1].cpu().numpy(), "bfloat16", f"scale {scale}")
